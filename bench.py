@@ -421,19 +421,17 @@ def main() -> int:
 
     def class_kernel(name):
         N_, K_ = shapes[name]
+        if B >= (9 if bits == 4 else 6):
+            return "gemm_wide_kernel"
         if name in ("qkv", "gate_up", "lm_head"):
             if fold_on:
                 xk = T.X_F16_FOLDED
-            elif bits == 4 and B > 1 and lib.ti_gemm_packed_rows_for(bits, B, N_, K_):
-                xk = T.X_F16_PACKED
             elif lib.ti_gemm_max_rows(bits, T.X_F32_RMSNORM, N_, K_) < B:
                 xk = T.X_F16
             else:
                 xk = T.X_F32_RMSNORM
-        elif name == "o" and B == 1:
-            xk = T.X_ATTN_SPLITS
         else:
-            xk = T.X_F16_PACKED if bits == 4 and lib.ti_gemm_packed_rows(bits, B) else T.X_F16
+            xk = T.X_ATTN_SPLITS if name == "o" and B == 1 else T.X_F16
         return T.gemm_kernel_name(bits, xk, B, N_, K_)
 
     # In-step timing: the replay step graph captured with per-workgroup

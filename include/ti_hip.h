@@ -255,10 +255,9 @@ int ti_gemm_packed_rows(int bits, int M);
 /* The same for one M x N x K call: 0 also where 17..64 int4 rows of a wide output take the tile
  * GEMM (rows x N >= TI_GEMM_TILE_WIDE_MN, env, default 850000), which needs TI_X_F16 rows. */
 int ti_gemm_packed_rows_for(int bits, int M, int N, int K);
-/* The tile GEMM's plan for an int4 (bits 4 or 4 | TI_BITS_G32) M x N x K call with a split-K
- * workspace of ws_bytes (0 = none): row-waves, weight tiles per wave and k-slices (1 = no split;
- * K is split only where one slice per column block would leave most CUs idle, TI_GEMM_SPLITK=0
- * never).  TI_ERR_UNSUPPORTED when the call would not take the tile kernel. */
+/* The many-rows GEMM's plan for an int4 (bits 4 or 4 | TI_BITS_G32) M x N x K call with a split-K
+ * workspace of ws_bytes (0 = none), for eight waves (one workgroup or two): row-waves, weight tiles
+ * per wave and k-slices (1 = no split, TI_GEMM_SPLITK=0 never).  TI_ERR_UNSUPPORTED when the call would not take the tile kernel. */
 int ti_gemm_tile_plan(int bits, int M, int N, int K, int64_t ws_bytes, int* wmr, int* tpw, int* n_ks);
 /* y[m][0:K] = fp16(rms_norm(x[m][0:K]) * w), tensor_engine.cpp:1452-1508 (the batched path's
  * activation prep; the same arithmetic as the fused TI_X_F32_RMSNORM prologue). */
@@ -274,6 +273,14 @@ int ti_gemm_grid(int M, int N, int K);
  * rows): the fold_ss partials per row its TI_EPI_RESID_F32 fold epilogue writes (0 = the call
  * does not take the batched-rows kernel). */
 int ti_gemm_fold_partials(int bits, int M, int N, int K);
+/* y = x W^T for 1 .. TI_GEMM_MAX_ROWS rows of row-major fp16 x (16-byte aligned rows, ldx % 8 == 0) and weights of
+ * every format (bits as ti_gemm_wq_a16, TI_BITS_G32 / TI_BITS_AFF included), any epilogue kind with row-major
+ * outputs; splits K with epi->splitk_ws.  ss_in / n_ss: x holds fp16(h * nw), outputs divided by the row's rms
+ * (M <= TI_FOLD_SS_ROWS).  TI_EPI_RESID_F32 with fold_x: also the next call's folded input, rows of ldo, and
+ * fold_ss[b * TI_FOLD_SS_ROWS + m], b < ti_gemm_rows_fold_partials(same call and workspace). */
+int ti_gemm_rows(const void* tiles, const uint16_t* scales, int bits, const void* x, int ldx, float eps, int M, int N, int K,
+                 const ti_epilogue* epi, ti_stream_t s);
+int ti_gemm_rows_fold_partials(int bits, int M, int N, int K, int64_t ws_bytes);
 /* One-time kernel attribute setup; call before capturing ti_gemm_wq_a16 into a graph. */
 int ti_gemm_prepare(void);
 
@@ -364,7 +371,7 @@ int ti_attn_prefill(const float* q, const uint16_t* k_cache, const uint16_t* v_c
 int ti_attn_prefill_set_kernel(int mode);
 
 /* The kernel ti_gemm_wq_a16 launches for plain (not group-32) weights of this shape, e.g.
- * "gemv_wq_kernel<4,4>", "gemm_rows_kernel", "gemm_tile_kernel" (bench / profile labels). */
+ * "gemv_wq_kernel<4,4>", "gemm_rows_kernel", "gemm_wide_kernel" (bench / profile labels). */
 int ti_gemm_kernel_name(int bits, int x_kind, int M, int N, int K, char* buf, int len);
 
 /* Same-run HBM calibration (bench lines): best-of-`reps` read GB/s of a `bytes` buffer streamed

@@ -1,0 +1,208 @@
+"""The many-rows GEMM (ti_gemm_rows, gemm_wide.hip): row-major fp16 rows against packed weights of every format,
+against the weights' exact values in float64 (test_gpu_kernels.py's bound: fp32 summation order)."""
+from __future__ import annotations
+
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from test_gpu_g32 import g32_weight, pack_g32
+from test_gpu_kernels import assert_close_dot, deq, dev
+
+pytestmark = pytest.mark.gpu
+f16, f32 = np.float16, np.float32
+G32, WS = 32, 64 << 20
+
+
+@pytest.fixture(scope="module")
+def ws(ti):
+    b = ti.DeviceBuffer(WS)
+    b.zero()
+    return b
+
+
+def weight(ti, oracle, bits, K, N, rng):
+    """(device tiles, device scales, the weight's exact values [K][N])."""
+    if bits & G32:
+        q, d, w = g32_weight(rng, K, N, bits & 15)
+        t, s = pack_g32(ti, q, d, bits & 15)
+        return t, s, w.astype(f32)
+    w = (rng.standard_normal((K, N)) * 0.03).astype(f32)
+    t, s = ti.wpack_host(w, bits)
+    return dev(ti, t), dev(ti, s), w.astype(f16).astype(f32) if bits == 16 else deq(oracle, w, bits)
+
+
+def rows(ti, bits, td, sd, xd, M, N, K, ep, ldx=None, ws=None):
+    if ws is not None:
+        ep.splitk_ws, ep.splitk_bytes = ws.ptr, ws.nbytes
+    rc = ti.lib().ti_gemm_rows(td.ptr, sd.ptr, bits, xd.ptr, ldx or K, 1e-5, M, N, K, C.byref(ep), None)
+    ti.check(rc)
+    ti.sync()
+    if ws is not None:
+        assert not ws.download(np.int32, (65536,)).any(), "split-K tickets not re-armed"
+
+
+# rows at the edges of the 16-, 32- and 64-row blocks, ragged column tiles, one k-group, odd numbers of them, narrow
+# outputs whose K is split, wide ones in several rounds
+@pytest.mark.parametrize("M,K,N", [(1, 128, 16), (16, 384, 80), (17, 1152, 4000), (32, 4096, 4096 + 48), (33, 128, 64),
+                                   (64, 1152, 6208), (65, 2048, 2560), (129, 384, 400), (333, 5632, 2048), (1000, 640, 11264),
+                                   (1024, 256, 1040), (100, 14336, 512)])
+@pytest.mark.parametrize("bits", [4, 8, 16, 4 | G32, 8 | G32])
+def test_rows_store(ti, oracle, ws, bits, M, K, N):
+    rng = np.random.RandomState(M * 7 + K + N + bits)
+    td, sd, w = weight(ti, oracle, bits, K, N, rng)
+    ldx = K + 8 * (M % 3)
+    x = rng.standard_normal((M, ldx)).astype(f16)
+    xd, yd = dev(ti, x), ti.DeviceBuffer(M * N * 4)
+    xa = x[:, :K].astype(f32)
+    ref = xa.astype(np.float64) @ w.astype(np.float64)
+    for k in (None, ws):
+        yd.zero()
+        ep = ti.Epilogue()
+        ep.kind, ep.ldo, ep.out = ti.EPI_STORE_F32, N, yd.ptr
+        rows(ti, bits, td, sd, xd, M, N, K, ep, ldx, k)
+        assert_close_dot(yd.download(f32, (M, N)), ref, xa, w)
+
+
+def test_rows_affine_blocks(ti, oracle, ws):
+    """Q4_1 blocks (4 | 32 | 64): the offset term through the block's sum of x."""
+    from test_gpu_g32 import pack_q1
+    for M, K, N in [(24, 384, 96), (100, 1152, 1040), (700, 2048, 512)]:
+        rng = np.random.RandomState(M)
+        q = rng.randint(0, 16, (K, N)).astype(np.uint8)
+        d = (rng.uniform(0.5, 1.5, (K // 32, N)) * 0.01).astype(f16)
+        m = (rng.standard_normal((K // 32, N)) * 0.05).astype(f16)
+        td, sd = pack_q1(ti, q, d, m)
+        w = np.repeat(d.astype(np.float64), 32, 0) * q + np.repeat(m.astype(np.float64), 32, 0)
+        parts = np.repeat(np.abs(d.astype(np.float64)), 32, 0) * 16 + np.repeat(np.abs(m.astype(np.float64)), 32, 0)
+        x = rng.standard_normal((M, K)).astype(f16)
+        yd = ti.DeviceBuffer(M * N * 4)
+        ep = ti.Epilogue()
+        ep.kind, ep.ldo, ep.out = ti.EPI_STORE_F32, N, yd.ptr
+        rows(ti, 4 | G32 | 64, td, sd, dev(ti, x), M, N, K, ep, ws=ws)
+        # fp32 sums of d (q - 8) x and (8 d + m) x: the bound is on the parts' magnitudes
+        assert np.all(np.abs(yd.download(f32, (M, N)) - x.astype(np.float64) @ w) <= 2e-5 * (np.abs(x.astype(np.float64)) @ parts) + 1e-6)
+
+
+@pytest.mark.parametrize("bits", [4, 8, 16])
+@pytest.mark.parametrize("M", [5, 30, 57, 150])
+def test_rows_epilogues(ti, oracle, ws, bits, M):
+    """fp16 store, residual add, SiLU * up and logits + argmax; rows of an odd pitch take the per-element form."""
+    K, N = 1152, 1056
+    rng = np.random.RandomState(M + bits)
+    td, sd, w = weight(ti, oracle, bits, K, N, rng)
+    x = rng.standard_normal((M, K)).astype(f16)
+    xd, xa = dev(ti, x), x.astype(np.float64)
+    ref = xa @ w.astype(np.float64)
+    for ldo in (N, N + 3):
+        r = rng.standard_normal((M, ldo)).astype(f32)
+        rd = dev(ti, r)
+        ep = ti.Epilogue()
+        ep.kind, ep.ldo, ep.out = ti.EPI_RESID_F32, ldo, rd.ptr
+        rows(ti, bits, td, sd, xd, M, N, K, ep, ws=ws)
+        got = rd.download(f32, (M, ldo))
+        assert_close_dot(got[:, :N] - r[:, :N], ref, x.astype(f32), w, rel=5e-5)
+        np.testing.assert_array_equal(got[:, N:], r[:, N:])
+        sil = ref.reshape(M, N // 16, 2, 8)
+        sil = (sil[:, :, 1] * (sil[:, :, 0] / (1 + np.exp(-sil[:, :, 0])))).reshape(M, N // 2)
+        hd = ti.DeviceBuffer(M * ldo * 2)
+        ep = ti.Epilogue()
+        ep.kind, ep.ldo, ep.out = ti.EPI_SILU_MUL_F16, ldo, hd.ptr
+        rows(ti, bits, td, sd, xd, M, N, K, ep, ws=ws)
+        np.testing.assert_allclose(hd.download(f16, (M, ldo))[:, : N // 2].astype(np.float64), sil, rtol=3e-3, atol=2e-3)
+        ep.kind = ti.EPI_STORE_F16
+        rows(ti, bits, td, sd, xd, M, N, K, ep, ws=ws)
+        np.testing.assert_allclose(hd.download(f16, (M, ldo))[:, :N].astype(np.float64), ref, rtol=2e-3, atol=1e-4)
+    ld, am = ti.DeviceBuffer(M * N * 4), ti.DeviceBuffer(M * ti.ARGMAX_SLOTS * 8)
+    am.zero()
+    ep = ti.Epilogue()
+    ep.kind, ep.ldo, ep.out, ep.argmax = ti.EPI_LOGITS_ARGMAX, N, ld.ptr, am.ptr
+    rows(ti, bits, td, sd, xd, M, N, K, ep, ws=ws)
+    lg = ld.download(f32, (M, N))
+    keys = am.download(np.uint64, (M, ti.ARGMAX_SLOTS)).max(axis=1)
+    np.testing.assert_array_equal((0xFFFFFFFF - (keys & 0xFFFFFFFF)).astype(np.int64), np.argmax(lg, axis=1))
+    np.testing.assert_allclose(lg, ref, rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("hd,M", [(64, 21), (128, 70)])
+def test_rows_qkv(ti, oracle, ws, hd, M):
+    """RoPE + KV append against the fused kernel's epilogue on the same products (int8, 16-row calls)."""
+    heads, kvh, K, S = 4, 2, 512, 96
+    qd, kd = heads * hd, kvh * hd
+    N = qd + 2 * kd
+    rng = np.random.RandomState(hd)
+    td, sd, _ = weight(ti, oracle, 8, K, N, rng)
+    xd = dev(ti, rng.standard_normal((M, K)).astype(f16))
+    pos = rng.permutation(S)[:M].astype(np.int32)
+    pd = dev(ti, pos)
+    cs = dev(ti, ti.rope_table(np.arange(S), hd, 10000.0))
+    outs = []
+    for wide in (True, False):
+        q, k, v = ti.DeviceBuffer(M * qd * 4), ti.DeviceBuffer(kvh * S * hd * 2), ti.DeviceBuffer(kvh * S * hd * 2)
+        for b in (k, v):
+            b.zero()
+        ep = ti.Epilogue()
+        ep.kind, ep.ldo, ep.out, ep.q_dim, ep.kv_dim, ep.head_dim, ep.max_seq = ti.EPI_QKV_ROPE_KV, qd, q.ptr, qd, kd, hd, S
+        ep.pos, ep.rope_cs, ep.k_cache, ep.v_cache, ep.kv_stream_stride = pd.ptr, cs.ptr, k.ptr, v.ptr, 0
+        if wide:
+            rows(ti, 8, td, sd, xd, M, N, K, ep, ws=ws)
+        else:
+            for m in range(0, M, 16):
+                ep.out, ep.pos = q.ptr + m * qd * 4, pd.ptr + 4 * m
+                ti.check(ti.lib().ti_gemm_wq_a16(td.ptr, sd.ptr, 8, xd.ptr + m * K * 2, ti.X_F16, K, None, 1e-5, min(16, M - m), N, K,
+                                                 C.byref(ep), None))
+            ti.sync()
+        outs.append([q.download(f32, (M, qd)), k.download(f16, (kvh, S, hd)).astype(f32), v.download(f16, (kvh, S, hd)).astype(f32)])
+    for a, b in zip(*outs):
+        np.testing.assert_allclose(a, b, rtol=2e-3, atol=2e-3)
+
+
+@pytest.mark.parametrize("bits", [4, 8, 16, 4 | G32])
+@pytest.mark.parametrize("M", [3, 16, 17, 45, 64])
+def test_rows_fold(ti, oracle, ws, bits, M):
+    """The batched fold: residual epilogue writes fp16(h * w) and sums of h^2, the next call divides by the rms."""
+    L, K, H, N = ti.lib(), 1152, 1024, 768
+    rng = np.random.RandomState(M + bits)
+    to, so, wo = weight(ti, oracle, bits, K, H, rng)
+    t2, s2, w2 = weight(ti, oracle, bits, H, N, rng)
+    act = rng.standard_normal((M, K)).astype(f16)
+    h0 = rng.standard_normal((M, H)).astype(f32)
+    nw = (1 + 0.1 * rng.standard_normal(H)).astype(f32)
+    n_ss = L.ti_gemm_rows_fold_partials(bits, M, H, K, WS)
+    assert 1 <= n_ss <= 4096
+    bits_out = []
+    for _ in range(2):
+        hd, fx, ss, yd = dev(ti, h0), ti.DeviceBuffer(M * H * 2), ti.DeviceBuffer(n_ss * 64 * 4), ti.DeviceBuffer(M * N * 4)
+        nwd = dev(ti, nw)
+        ep = ti.Epilogue()
+        ep.kind, ep.ldo, ep.out = ti.EPI_RESID_F32, H, hd.ptr
+        ep.fold_w, ep.fold_x, ep.fold_ss = nwd.ptr, fx.ptr, ss.ptr
+        rows(ti, bits, to, so, dev(ti, act), M, H, K, ep, ws=ws)
+        h1 = hd.download(f32, (M, H))
+        assert_close_dot(h1 - h0, act.astype(np.float64) @ wo.astype(np.float64), act.astype(f32), wo, rel=5e-5)
+        np.testing.assert_array_equal(fx.download(np.uint16, (M, H)), (h1 * nw).astype(f16).view(np.uint16))
+        np.testing.assert_allclose(ss.download(f32, (n_ss, 64))[:, :M].sum(axis=0), (h1.astype(np.float64) ** 2).sum(axis=1), rtol=1e-5)
+        ep = ti.Epilogue()
+        ep.kind, ep.ldo, ep.out, ep.ss_in, ep.n_ss = ti.EPI_STORE_F32, N, yd.ptr, ss.ptr, n_ss
+        rows(ti, bits, t2, s2, fx, M, N, H, ep, ws=ws)
+        y = yd.download(f32, (M, N))
+        bits_out.append(y.view(np.uint32))
+    rms = np.sqrt((h1.astype(np.float64) ** 2).mean(axis=1) + 1e-5)
+    xf = (h1 * nw).astype(f16).astype(np.float64) / rms[:, None]
+    assert_close_dot(y, xf @ w2.astype(np.float64), xf.astype(f32), w2, rel=5e-5)
+    np.testing.assert_array_equal(*bits_out)   # fixed-order sums
+
+
+def test_rows_refusals(ti):
+    L = ti.lib()
+    b = ti.DeviceBuffer(1 << 20)
+    ep = ti.Epilogue()
+    ep.kind, ep.ldo, ep.out = ti.EPI_STORE_F32, 64, b.ptr
+    ok = (b.ptr, b.ptr, 8, b.ptr, 256, 1e-5, 4, 64, 256)
+    for i, v in [(2, 5), (2, 16 | G32), (3, b.ptr + 2), (4, 260), (4, 128), (6, 0), (6, 2000), (7, 60), (8, 200)]:
+        a = list(ok)
+        a[i] = v
+        assert L.ti_gemm_rows(*a, C.byref(ep), None) != 0, (i, v)
+    ep.kind, ep.fold_x = ti.EPI_RESID_F32, b.ptr
+    assert L.ti_gemm_rows(*ok, C.byref(ep), None) != 0

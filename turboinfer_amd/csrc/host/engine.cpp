@@ -98,15 +98,16 @@ struct ti_engine {
   float* ws = nullptr;
   uint16_t* attn = nullptr;
   uint16_t* act = nullptr;
-  uint16_t* xn = nullptr;      // fp16 rms_norm rows for the batched-rows GEMM [R][hidden]
+  uint16_t* xn = nullptr;      // fp16 rms_norm rows for the many-rows GEMM [R][hidden]
+  bool wide_ok = false;        // every weight within the many-rows GEMM's offsets
   // single-stream steps with the rms_norm folded behind the GEMM (ti_hip.h TI_X_F16_FOLDED):
   // the epilogue that writes h also writes fx = fp16(h * next norm weight) and its workgroups'
   // sums of h^2 (ss); the next projection stages fx and divides its outputs by the rms
   bool fold_on = true;         // TI_FOLD=0 / ti_engine_set_fold
   uint16_t* fx = nullptr;      // [hidden]
   float* ss = nullptr;         // [256]
-  // batched fold (17..64 int4 rows): the producers' (O, down) epilogues write xn = fp16(h * next
-  // norm weight) and per-column-group sums of h^2 per row [n_cg][TI_FOLD_SS_ROWS]
+  // batched fold (up to 64 rows): the producers' (O, down) epilogues write xn = fp16(h * next
+  // norm weight) and per-column-block sums of h^2 per row [n_cb][TI_FOLD_SS_ROWS]
   float* ss_rows = nullptr;
   // single-stream attention leaves its split merge to the O projection (ti_attn_decode_partials
   // + TI_X_ATTN_SPLITS): no arrival-ticket hand-off at the end of the attention launch
@@ -124,7 +125,7 @@ struct ti_engine {
   float* draws = nullptr;      // [max_batch][draw_cap] uniform draws, per new token
   float* lps = nullptr;        // [max_batch][draw_cap] log p of the sampled tokens
   int draw_cap = 0;
-  void* splitk_ws = nullptr;   // tile GEMM split-K workspace (ti_epilogue.splitk_ws), int4 engines
+  void* splitk_ws = nullptr;   // the many-rows GEMM's split-K workspace (ti_epilogue.splitk_ws)
   size_t splitk_bytes = 0;
   void* samp_ws = nullptr;     // ti_sample_step_ws workspace (top_k > TI_SAMPLE_MAX_K)
   size_t samp_ws_bytes = 0;
@@ -277,30 +278,32 @@ int validate(const ti_engine_config& c) {
 // Rows of the batched-rows kernel (int4, M > 16) take their fp16 operands in fragment order
 // (TI_X_F16_PACKED): the rms_norm prep, the attention output and the SiLU*up output are written
 // that way, so every operand load of the kernel is one contiguous KiB per wave.
-bool packed_rows(const ti_engine* e, int M) { return ti_gemm_packed_rows(e->c.bits, M) != 0; }
+// Rows whose projections run on the many-rows kernel (ti_gemm_rows).  From the rows where a layer's four launches
+// take less there, the rms_norm folded into them, than the fused kernel's (int8 / fp16: its rms_norm prologue and, from
+// 8 rows on, several launches for a long K) or the 3..16-row int4 kernel's beside two rms_norm launches.  Measured at
+// 4 / 8 / 16 rows, us per layer: int8 2048 x 5632 30.6 / 30.5 / 30.6 against 30.3 / 33 / 35, fp16 35 / 35 / 35 against
+// 37 / 40 / 45, int4 4096 x 11008 50 / 50 / 50 against 42 / 46 / 55.
+bool rows_wide(const ti_engine* e, int M) {
+  return e->wide_ok && M >= ((e->c.bits & ~TI_BITS_G32) == 4 ? 9 : 6);
+}
 
-// One projection for rows [0, M): the fused kernel in chunks of the rows its LDS image
-// holds, or -- int4, when the rows do not fit -- rms_norm into fp16 rows once (e->xn) and
-// the batched-rows kernel in chunks of TI_GEMM_MAX_ROWS.  Graph-capturable.
+// One projection for rows [0, M): the many-rows kernel, fp32 rows normalised into fp16 first (e->xn); or the fused
+// kernel in chunks of the rows its LDS image holds (int4 rows that do not fit: the batched kernel behind the same
+// rms_norm).  Graph-capturable.
 int gemm_rows(ti_engine* e, const DevLinear& W, int M, const void* x, int x_kind, int ldx, const float* nw,
               const ti_epilogue& epi, size_t out_elem, bool last_gets_ctr) {
   const ti_engine_config& c = e->c;
-  int rows = ti_gemm_max_rows(c.bits, x_kind, W.N, W.K);
-  if (x_kind == TI_X_F32_RMSNORM && ti_gemm_packed_rows_for(c.bits, M, W.N, W.K) && e->xn) {
-    TI_TRY(ti_rmsnorm_f16_packed(static_cast<const float*>(x), ldx, nw, c.eps, e->xn, M, W.K, e->s));
-    x = e->xn;
-    x_kind = TI_X_F16_PACKED;
-    ldx = W.K;
-    rows = ti_gemm_max_rows(c.bits, x_kind, W.N, W.K);
-  } else if (x_kind == TI_X_F32_RMSNORM && rows < M && (c.bits & ~TI_BITS_G32) == 4 && e->xn) {
+  const bool wide = rows_wide(e, M);
+  int rows = wide ? TI_GEMM_MAX_ROWS : ti_gemm_max_rows(c.bits, x_kind, W.N, W.K);
+  if (x_kind == TI_X_F32_RMSNORM && e->xn && (wide || (rows < M && (c.bits & ~TI_BITS_G32) == 4))) {
     TI_TRY(ti_rmsnorm_f16(static_cast<const float*>(x), ldx, nw, c.eps, e->xn, W.K, M, W.K, e->s));
     x = e->xn;
     x_kind = TI_X_F16;
     ldx = W.K;
-    rows = ti_gemm_max_rows(c.bits, x_kind, W.N, W.K);
+    if (!wide) rows = ti_gemm_max_rows(c.bits, x_kind, W.N, W.K);
   }
   if (rows < 1) return ti_set_error(TI_ERR_UNSUPPORTED, "engine: no GEMM kernel for N=%d K=%d", W.N, W.K);
-  const size_t x_elem = x_kind == TI_X_F16 || x_kind == TI_X_F16_FOLDED || x_kind == TI_X_F16_PACKED ? 2 : 4;
+  const size_t x_elem = x_kind == TI_X_F16 || x_kind == TI_X_F16_FOLDED ? 2 : 4;
   for (int m0 = 0; m0 < M; m0 += rows) {
     const int mm = std::min(rows, M - m0);
     ti_epilogue ep = epi;
@@ -313,7 +316,8 @@ int gemm_rows(ti_engine* e, const DevLinear& W, int M, const void* x, int x_kind
     ep.splitk_ws = e->splitk_ws;
     ep.splitk_bytes = (int64_t)e->splitk_bytes;
     const void* xm = static_cast<const char*>(x) + (size_t)m0 * ldx * x_elem;
-    TI_TRY(ti_gemm_wq_a16(W.tiles, W.scales, c.bits, xm, x_kind, ldx, nw, c.eps, mm, W.N, W.K, &ep, e->s));
+    if (wide) TI_TRY(ti_gemm_rows(W.tiles, W.scales, c.bits, xm, ldx, c.eps, mm, W.N, W.K, &ep, e->s));
+    else TI_TRY(ti_gemm_wq_a16(W.tiles, W.scales, c.bits, xm, x_kind, ldx, nw, c.eps, mm, W.N, W.K, &ep, e->s));
   }
   return TI_OK;
 }
@@ -342,13 +346,13 @@ bool fold_usable(ti_engine* e, int M) {
   return g_o > 0 && g_o <= 256 && g_d > 0 && g_d <= 256 && ti_gemm_max_rows(c.bits, TI_X_F16, H, qd) >= 1;
 }
 
-// The batched fold: 17..64 int4 rows on the batched-rows kernels (packed operands), the O / down
-// producers' column groups within the partial buffer.
+// The batched fold: up to 64 rows on the many-rows kernel, the O / down producers' column blocks within the partial
+// buffer.
 bool bfold_usable(ti_engine* e, int M) {
   const ti_engine_config& c = e->c;
-  if (!e->fold_on || c.compat || c.bits != 4 || M <= 16 || M > TI_FOLD_SS_ROWS || !packed_rows(e, M) || !e->ss_rows)
-    return false;
-  const int po = ti_gemm_fold_partials(c.bits, M, c.hidden, e->qd()), pd = ti_gemm_fold_partials(c.bits, M, c.hidden, c.inter);
+  if (!e->fold_on || c.compat || M > TI_FOLD_SS_ROWS || !rows_wide(e, M) || !e->ss_rows) return false;
+  const int po = ti_gemm_rows_fold_partials(c.bits, M, c.hidden, e->qd(), (int64_t)e->splitk_bytes);
+  const int pd = ti_gemm_rows_fold_partials(c.bits, M, c.hidden, c.inter, (int64_t)e->splitk_bytes);
   return po >= 1 && po <= 4096 && pd >= 1 && pd <= 4096;
 }
 
@@ -479,13 +483,12 @@ int enqueue_step(ti_engine* e, int M, int advance) {
   }
   const int H = c.hidden, qd = e->qd(), kvd = e->kvd(), I = c.inter, V = c.vocab;
   // fold (M == 1): every rms_norm input is handed over as fx + ss partials by its producer
-  const bool fold = fold_usable(e, M), part = part_usable(e, M), pk = packed_rows(e, M), qa = qa_usable(e, M);
-  // batched fold (17..64 rows): O / down write xn = fp16(h * next norm weight) and per-row sums of
-  // h^2; QKV (after layer 0), gate/up and the lm_head normalise behind their GEMM (ti_hip.h)
+  const bool fold = fold_usable(e, M), part = part_usable(e, M), qa = qa_usable(e, M);
+  // batched fold (many-rows kernel, up to 64 rows): O / down write xn = fp16(h * next norm weight) and per-row
+  // sums of h^2; QKV (after layer 0), gate/up and the lm_head normalise behind their GEMM (ti_hip.h)
   const bool bfold = !fold && bfold_usable(e, M);
   int bn_ss = 0;   // partials per row the last batched producer wrote (0: none yet, rms_norm prep)
   auto next_norm = [&](int l) -> const float* { return l < c.layers ? e->layer[l].attn_norm : e->out_norm; };
-  auto next_n = [&](int l) -> int { return l < c.layers ? e->layer[l].qkv.N : e->lm.N; };
   if (fold) {
     sa.fold_w = next_norm(0);
     sa.fold_x = e->fx;
@@ -494,8 +497,7 @@ int enqueue_step(ti_engine* e, int M, int advance) {
   stamp_tag(TI_STAMP_TAG_BEGIN);
   TI_TRY(ti_step_begin(&sa, e->s));
   int n_ss = 1;   // partials the last producer wrote (step_begin: one)
-  // producer side (RESID epilogue); n_next: output width of the call that consumes the fold
-  auto fold_into = [&](ti_epilogue& ep, const float* w, int n_next) {
+  auto fold_into = [&](ti_epilogue& ep, const float* w) {   // producer side (RESID epilogue)
     if (fold) {
       ep.fold_w = w;
       ep.fold_x = e->fx;
@@ -504,10 +506,9 @@ int enqueue_step(ti_engine* e, int M, int advance) {
       ep.fold_w = w;
       ep.fold_x = e->xn;
       ep.fold_ss = e->ss_rows;
-      ep.fold_packed = ti_gemm_packed_rows_for(c.bits, M, n_next, H);
     }
   };
-  auto norm_in = [&](const void*& x, int& xk, int& ldx, const float*& nw, ti_epilogue& ep, int n) {   // consumer side
+  auto norm_in = [&](const void*& x, int& xk, int& ldx, const float*& nw, ti_epilogue& ep) {   // consumer side
     if (fold) {
       x = e->fx;
       xk = TI_X_F16_FOLDED;
@@ -517,7 +518,7 @@ int enqueue_step(ti_engine* e, int M, int advance) {
       ep.n_ss = n_ss;
     } else if (bfold && bn_ss > 0) {
       x = e->xn;
-      xk = ti_gemm_packed_rows_for(c.bits, M, n, H) ? TI_X_F16_PACKED : TI_X_F16;
+      xk = TI_X_F16;
       ldx = H;
       nw = nullptr;
       ep.ss_in = e->ss_rows;
@@ -527,10 +528,10 @@ int enqueue_step(ti_engine* e, int M, int advance) {
 
   auto gemm = [&](const DevLinear& W, const void* x, int x_kind, int ldx, size_t /*x_elem*/, const float* nw,
                   ti_epilogue epi, size_t out_elem, bool last_gets_ctr) -> int {
-    if (x_kind == TI_X_F32_RMSNORM) norm_in(x, x_kind, ldx, nw, epi, W.N);
+    if (x_kind == TI_X_F32_RMSNORM) norm_in(x, x_kind, ldx, nw, epi);
     TI_TRY(gemm_rows(e, W, M, x, x_kind, ldx, nw, epi, out_elem, last_gets_ctr));
     if (epi.fold_x && fold) n_ss = ti_gemm_grid(M, W.N, W.K);
-    if (epi.fold_x && bfold) bn_ss = ti_gemm_fold_partials(c.bits, M, W.N, W.K);
+    if (epi.fold_x && bfold) bn_ss = ti_gemm_rows_fold_partials(c.bits, M, W.N, W.K, (int64_t)e->splitk_bytes);
     return TI_OK;
   };
 
@@ -553,7 +554,7 @@ int enqueue_step(ti_engine* e, int M, int advance) {
     eo.kind = TI_EPI_RESID_F32;
     eo.ldo = H;
     eo.out = e->h;
-    fold_into(eo, L.ffn_norm, L.gu.N);
+    fold_into(eo, L.ffn_norm);
     if (qa) {   // QKV + attention in one launch; O merges the splits
       stamp_tag(TI_STAMP_TAG_QKV);
       const int S = e->splits_for(M);
@@ -580,18 +581,16 @@ int enqueue_step(ti_engine* e, int M, int advance) {
       stamp_tag(TI_STAMP_TAG_QKV);
       TI_TRY(gemm(L.qkv, e->h, TI_X_F32_RMSNORM, H, 4, L.attn_norm, ep, 4, false));
       stamp_tag(TI_STAMP_TAG_ATTN);
-      TI_TRY((pk ? ti_attn_decode_packed : ti_attn_decode)(e->q, L.kc, L.vc, e->kv_stride, c.max_seq, e->pos, M,
-                                                           c.heads, c.kv_heads, c.head_dim, e->splits_for(M), e->ws,
-                                                           e->attn, e->s));
+      TI_TRY(ti_attn_decode(e->q, L.kc, L.vc, e->kv_stride, c.max_seq, e->pos, M, c.heads, c.kv_heads, c.head_dim,
+                            e->splits_for(M), e->ws, e->attn, e->s));
       stamp_tag(TI_STAMP_TAG_O);
-      TI_TRY(gemm(L.o, e->attn, pk ? TI_X_F16_PACKED : TI_X_F16, qd, 2, nullptr, eo, 4, false));
+      TI_TRY(gemm(L.o, e->attn, TI_X_F16, qd, 2, nullptr, eo, 4, false));
     }
 
     ti_epilogue eg{};
     eg.kind = TI_EPI_SILU_MUL_F16;
     eg.ldo = I;
     eg.out = e->act;
-    eg.out_packed = pk;
     stamp_tag(TI_STAMP_TAG_GATE_UP);
     TI_TRY(gemm(L.gu, e->h, TI_X_F32_RMSNORM, H, 4, L.ffn_norm, eg, 2, false));
 
@@ -599,9 +598,9 @@ int enqueue_step(ti_engine* e, int M, int advance) {
     ed.kind = TI_EPI_RESID_F32;
     ed.ldo = H;
     ed.out = e->h;
-    fold_into(ed, next_norm(l + 1), next_n(l + 1));
+    fold_into(ed, next_norm(l + 1));
     stamp_tag(TI_STAMP_TAG_DOWN);
-    TI_TRY(gemm(L.down, e->act, pk ? TI_X_F16_PACKED : TI_X_F16, I, 2, nullptr, ed, 4, false));
+    TI_TRY(gemm(L.down, e->act, TI_X_F16, I, 2, nullptr, ed, 4, false));
   }
   ti_epilogue el{};
   el.kind = TI_EPI_LOGITS_ARGMAX;
@@ -629,11 +628,11 @@ int enqueue_step(ti_engine* e, int M, int advance) {
 static bool prefill_attn_on();
 
 // Decode-attention workspace: the largest need over the row counts that run the split kernel --
-// decode batches up to max_batch and prompt chunks of up to 64 rows (ti_gemm_packed_rows; longer
-// chunks run ti_attn_prefill, no workspace), all chunk sizes when TI_ATTN_PREFILL=0.
+// decode batches up to max_batch (prompt chunks run ti_attn_prefill, no workspace), all chunk sizes when
+// TI_ATTN_PREFILL=0.
 size_t ws_bytes(const ti_engine* e) {
   const ti_engine_config& c = e->c;
-  const int R = prefill_attn_on() ? std::min(e->rows_cap, std::max(c.max_batch, 64)) : e->rows_cap;
+  const int R = prefill_attn_on() ? c.max_batch : e->rows_cap;
   size_t b = 0;
   for (int M = 1; M <= R; ++M) b = std::max(b, ti_attn_workspace_bytes(M, c.heads, c.head_dim, e->splits_for(M)));
   return b;
@@ -717,29 +716,26 @@ int enqueue_prefill(ti_engine* e, int m, int t0, int rows, int base, float* laye
     ep.v_cache = vc;
     ep.kv_stream_stride = 0;
     TI_TRY(gemm_rows(e, L.qkv, rows, e->h, TI_X_F32_RMSNORM, H, L.attn_norm, ep, 4, false));
-    const bool pk = packed_rows(e, rows);
-    if (!pk && prefill_attn_on())   // row-major chunk: one pass over the prefix per 16 rows (MFMA)
+    if (prefill_attn_on())   // one pass over the prefix per 16 rows (MFMA)
       TI_TRY(ti_attn_prefill(e->q, kc, vc, c.max_seq, e->pos, rows, c.heads, c.kv_heads, c.head_dim, e->attn, e->s));
     else
-      TI_TRY((pk ? ti_attn_decode_packed : ti_attn_decode)(e->q, kc, vc, 0, c.max_seq, e->pos, rows, c.heads,
-                                                           c.kv_heads, c.head_dim, e->splits_for(rows), e->ws,
-                                                           e->attn, e->s));
+      TI_TRY(ti_attn_decode(e->q, kc, vc, 0, c.max_seq, e->pos, rows, c.heads, c.kv_heads, c.head_dim, e->splits_for(rows),
+                            e->ws, e->attn, e->s));
     ti_epilogue eo{};
     eo.kind = TI_EPI_RESID_F32;
     eo.ldo = H;
     eo.out = e->h;
-    TI_TRY(gemm_rows(e, L.o, rows, e->attn, pk ? TI_X_F16_PACKED : TI_X_F16, qd, nullptr, eo, 4, false));
+    TI_TRY(gemm_rows(e, L.o, rows, e->attn, TI_X_F16, qd, nullptr, eo, 4, false));
     ti_epilogue eg{};
     eg.kind = TI_EPI_SILU_MUL_F16;
     eg.ldo = I;
     eg.out = e->act;
-    eg.out_packed = pk;
     TI_TRY(gemm_rows(e, L.gu, rows, e->h, TI_X_F32_RMSNORM, H, L.ffn_norm, eg, 2, false));
     ti_epilogue ed{};
     ed.kind = TI_EPI_RESID_F32;
     ed.ldo = H;
     ed.out = e->h;
-    TI_TRY(gemm_rows(e, L.down, rows, e->act, pk ? TI_X_F16_PACKED : TI_X_F16, I, nullptr, ed, 4, false));
+    TI_TRY(gemm_rows(e, L.down, rows, e->act, TI_X_F16, I, nullptr, ed, 4, false));
   }
   return TI_OK;
 }
@@ -850,13 +846,16 @@ int ti_engine_create(const ti_engine_config* cfg, ti_engine** out) {
     if ((rc = ti_memcpy_h2d(e->rope_cs, cs.data(), cs.size() * 4, e->s))) return fail(rc);
     if (const char* env = getenv("TI_ATTN_PART")) e->part_on = atoi(env) != 0;
     e->splits_max = e->splits_for(1);
-    e->pf_rows = (c.bits & ~TI_BITS_G32) == 4 ? TI_GEMM_MAX_ROWS : 16;   // int4 (also group-32): the tile GEMM
-    // (affine group-32 runs the fused kernel only: prompt chunks of its 16 rows)
+    // the many-rows kernel's byte offsets into a weight are 32 bits; wider ones keep the fused kernel's 16-row pieces
+    e->wide_ok = true;
+    for (const DevLinear* w : {&e->layer[0].qkv, &e->layer[0].o, &e->layer[0].gu, &e->layer[0].down, &e->lm})
+      e->wide_ok = e->wide_ok && ti_gemm_rows_fold_partials(c.bits, TI_FOLD_SS_ROWS, w->N, w->K, 0) > 0;
+    e->pf_rows = !e->wide_ok && (c.bits & ~TI_BITS_G32) != 4 ? 16 : TI_GEMM_MAX_ROWS;
+    if ((c.bits & ~TI_BITS_G32) != 4) e->pf_rows = std::min(e->pf_rows, std::max(16, c.max_seq));
     e->rows_cap = std::max(B, e->pf_rows);
     const int R = e->rows_cap;
-    const int Rp = (R + 15) / 16 * 16;   // packed operands hold whole 16-row blocks
-    if ((rc = e->alloc_t(&e->q, (size_t)R * qd)) || (rc = e->alloc_t(&e->attn, (size_t)Rp * qd)) ||
-        (rc = e->alloc_t(&e->act, (size_t)Rp * I)) || (rc = e->alloc_t(&e->xn, (size_t)Rp * std::max(H, I))) ||
+    if ((rc = e->alloc_t(&e->q, (size_t)R * qd)) || (rc = e->alloc_t(&e->attn, (size_t)R * qd)) ||
+        (rc = e->alloc_t(&e->act, (size_t)R * I)) || (rc = e->alloc_t(&e->xn, (size_t)R * std::max(H, I))) ||
         (rc = e->alloc(reinterpret_cast<void**>(&e->ws), ws_bytes(e))) ||
         (rc = e->alloc_t(&e->pf_ones, (size_t)e->pf_rows)) || (rc = e->alloc_t(&e->pf_zero, (size_t)1)) ||
         (rc = e->alloc_t(&e->pf_base, (size_t)e->pf_rows)) || (rc = e->alloc_t(&e->fx, (size_t)H)) ||
@@ -867,7 +866,7 @@ int ti_engine_create(const ti_engine_config* cfg, ti_engine** out) {
       return fail(rc);
     if (const char* env = getenv("TI_FOLD")) e->fold_on = atoi(env) != 0;
     if (const char* env = getenv("TI_QKV_ATTN")) e->qa_on = atoi(env) != 0;
-    if ((c.bits & ~TI_BITS_G32) == 4) {   // batched rows and prompt chunks: split-K tile GEMM (TI_SPLITK_MB, 0 = off)
+    {   // batched rows and prompt chunks: the many-rows GEMM's split-K (TI_SPLITK_MB, 0 = off)
       const char* env = getenv("TI_SPLITK_MB");
       const size_t mb = env ? (size_t)std::max(0, atoi(env)) : 64;
       if (mb && (rc = e->alloc(&e->splitk_ws, mb << 20))) return fail(rc);
@@ -1888,7 +1887,6 @@ int ti_engine_time_kernel(ti_engine* e, int which, int n, int kv_len, int reps, 
         ep.fold_w = L.ffn_norm;
         ep.fold_x = e->xn;
         ep.fold_ss = e->ss_rows;
-        ep.fold_packed = ti_gemm_packed_rows_for(c.bits, n, which == 1 ? L.gu.N : L.qkv.N, H);
       }
       if (which == 1 && part) {   // O merges the attention's split partials
         x = e->part_o;
@@ -1898,8 +1896,6 @@ int ti_engine_time_kernel(ti_engine* e, int which, int n, int kv_len, int reps, 
         ep.head_dim = c.head_dim;
       }
     }
-    if (packed_rows(e, n) && (which == 1 || which == 3)) xk = TI_X_F16_PACKED;   // enqueue_step's operands
-    if (packed_rows(e, n) && which == 2) ep.out_packed = 1;
     if (fold && xk == TI_X_F32_RMSNORM) {   // the step's consumer form (enqueue_step)
       x = e->fx;
       xk = TI_X_F16_FOLDED;
@@ -1908,10 +1904,11 @@ int ti_engine_time_kernel(ti_engine* e, int which, int n, int kv_len, int reps, 
       ep.n_ss = ti_gemm_grid(1, H, which == 2 ? qd : I);
     } else if (bfold && xk == TI_X_F32_RMSNORM) {   // the batched fold's consumer form
       x = e->xn;
-      xk = ti_gemm_packed_rows_for(c.bits, n, W->N, H) ? TI_X_F16_PACKED : TI_X_F16;
+      xk = TI_X_F16;
+      ldx = H;
       nw = nullptr;
       ep.ss_in = e->ss_rows;
-      ep.n_ss = ti_gemm_fold_partials(c.bits, n, H, which == 2 ? qd : I);
+      ep.n_ss = ti_gemm_rows_fold_partials(c.bits, n, H, which == 2 ? qd : I, (int64_t)e->splitk_bytes);
     }
     return TI_OK;
   };
@@ -1936,9 +1933,8 @@ int ti_engine_time_kernel(ti_engine* e, int which, int n, int kv_len, int reps, 
       return ti_attn_decode_partials(e->q, L.kc, L.vc, e->kv_stride, c.max_seq, e->pos, n, c.heads, c.kv_heads,
                                      c.head_dim, e->splits_for(n), e->part_o, e->part_ml, e->s);
     if (which == 5)
-      return (packed_rows(e, n) ? ti_attn_decode_packed : ti_attn_decode)(e->q, L.kc, L.vc, e->kv_stride, c.max_seq,
-                                                                           e->pos, n, c.heads, c.kv_heads, c.head_dim,
-                                                                           e->splits_for(n), e->ws, e->attn, e->s);
+      return ti_attn_decode(e->q, L.kc, L.vc, e->kv_stride, c.max_seq, e->pos, n, c.heads, c.kv_heads, c.head_dim,
+                            e->splits_for(n), e->ws, e->attn, e->s);
     return gemm_rows(e, *W, n, x, xk, ldx, nw, ep, which == 2 ? 2 : 4, false);
   };
   // The `reps` launches are captured once into a graph and the graph is replayed `rounds`

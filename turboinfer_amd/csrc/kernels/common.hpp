@@ -231,7 +231,8 @@ __device__ __forceinline__ void stamp_end(unsigned long long* st, unsigned long 
     const unsigned wave = threadIdx.x >> 6;
     const size_t wg = blockIdx.x + (size_t)gridDim.x * (blockIdx.y + (size_t)gridDim.y * blockIdx.z);
     unsigned long long* p = st + wg * kStampWords;
-    if (wave < 8) p[1 + wave] = stamp_now();
+    const unsigned waves = (blockDim.x + 63) >> 6;   // (fewer than 8: the last words repeat)
+    for (unsigned w = wave; w < 8; w += waves) p[1 + w] = stamp_now();
     if (TI_STAMP_PHASES && wave < 8) p[16 + wave] = wave_mark;
     if (wave == 0) {
       p[0] = t_entry;

@@ -27,13 +27,11 @@
 #include <atomic>
 #include <stdlib.h>
 
-#include "common.hpp"
 #include "attention_body.hpp"
-#include "dequant.hpp"
+#include "gemm_common.hpp"
+#include "gemm_wide.hpp"
 
 namespace ti {
-
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 #ifndef TI_GEMV_RING_VGPRS
 // VGPRs per lane of packed weights in flight.  Deeper is slower: a CU accepts a bounded
@@ -46,9 +44,6 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 #endif
 #ifndef TI_GEMV_RING_DELAY
 #define TI_GEMV_RING_DELAY 0
-#endif
-#ifndef TI_GEMV_EXP
-#define TI_GEMV_EXP 0   // product build; tools/probe_gemv.hip compiles diagnostic variants
 #endif
 #if TI_GEMV_EXP & 4   // diagnostic: per-workgroup phase timestamps (s_memrealtime, 100 MHz)
 __device__ unsigned long long g_gemv_ts[4096 * 8];
@@ -68,37 +63,6 @@ __device__ unsigned long long g_rows_ts[4096 * 8 * 8];   // [wg][wave][phase] (g
 #define GEMV_TS(k) do { } while (0)
 #define ROWS_TS(k) do { } while (0)
 #endif
-
-constexpr int kGemvWaves = 8;
-constexpr int kGemvThreads = kGemvWaves * kWave;
-
-struct GemvArgs {
-  const u32x4* tiles;
-  const uint16_t* scales;
-  const void* x;
-  const float* norm_w;
-  float eps;
-  int32_t x_kind, ldx, M, N, K;
-  ti_epilogue epi;
-  unsigned long long* stamp;   // in-step launch stamps (common.hpp stamp_end), NULL in product launches
-};
-
-__host__ __device__ constexpr int align16(int b) { return (b + 15) & ~15; }
-
-// The GEMM's two remaining A/B knobs, read once per process (thread-safe static init).
-struct GemmKnobs {
-  bool splitk = true;       // TI_GEMM_SPLITK=0: no split-K for under-filled tile grids
-  bool rows_split = true;   // TI_GEMM_ROWS_SPLIT=0: all rows in one batched-rows workgroup
-};
-__host__ inline const GemmKnobs& gemm_knobs() {
-  static const GemmKnobs k = [] {
-    GemmKnobs v;
-    if (const char* e = getenv("TI_GEMM_SPLITK")) v.splitk = atoi(e) != 0;
-    if (const char* e = getenv("TI_GEMM_ROWS_SPLIT")) v.rows_split = atoi(e) != 0;
-    return v;
-  }();
-  return k;
-}
 
 // Workgroups per launch: one 8-wave workgroup per CU (a second workgroup per CU measured slower,
 // DESIGN 4.1), never more than there are 16-row tiles.
@@ -288,18 +252,6 @@ __device__ __forceinline__ void epilogue(const GemvArgs& a, int nt, int tl, int 
   }
 }
 
-// Weight stream load: read once per launch, so non-temporal where that pays (TI_GEMV_NT).
-#ifndef TI_GEMV_NT
-#define TI_GEMV_NT 1
-#endif
-__device__ __forceinline__ u32x4 ld_w(const u32x4* p) {
-#if TI_GEMV_NT || (TI_GEMV_EXP & 16)
-  return __builtin_nontemporal_load(p);
-#else
-  return *p;
-#endif
-}
-
 // Offset-folded int4 input prep of one staged x piece (deq_int4_raw): the high-nibble slots scaled
 // by 1/16 (exact in fp16) and the piece's share of corr[g][m] = 1032 * sum_lo x + 1152 * sum_hi x.
 __device__ __forceinline__ float int4_x_prep(f16x8& h) {
@@ -311,14 +263,6 @@ __device__ __forceinline__ float int4_x_prep(f16x8& h) {
 }
 
 // --------------------------------------------------------------------- kernel
-// LDS barrier that leaves the wave's outstanding global loads in flight (a plain
-// __syncthreads() may drain vmcnt): LDS writes retired, then s_barrier.
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
 // The fields on the prologue's critical path come first as separate arguments: gfx950 can
 // preload leading kernel arguments into SGPRs before the waves start (compiled with
 // -mllvm -amdgpu-kernarg-preload-count, see Makefile), so the first x / weight / epilogue-input
@@ -855,255 +799,9 @@ __global__ __launch_bounds__(kGemvThreads, 1) void gemv_wq_kernel(const u32x4* p
 }
 
 // ================================================================= batched rows
-// gemv_mb_kernel<MB, NTL>: int4 weights x fp16 activations for M <= 16*MB rows (MB <= 2):
-// the batched decode of generate_batch (inference_engine.cpp:804-828), and
-// long-K projections whose activation rows no longer fit gemv_wq_kernel's LDS image.
-// Weights are still read once per launch, straight into registers; the activations are
-// staged in k-chunks of 1024 (8 k-tiles, one per wave):
-//   * a chunk of all rows is copied by LDS-DMA (global_load_lds_dwordx4: every wave
-//     instruction one contiguous KiB of a row) into one of two LDS buffers, one chunk ahead;
-//   * item order per wave: chunk c (k-tile 8c + wave) x tile tl; the NTL tiles' weights of
-//     chunk c + 1 are loaded into the other register buffer while chunk c computes (the chunk
-//     loop unrolled by two), and one barrier per chunk hands the x buffers over;
-//   * per 32-k step one dequantized weight fragment feeds MB MFMAs (one per 16-row block);
-//     nibble offsets are removed in the dequant (x is used as staged);
-//   * k-tiles past K (the last chunk) and the dummy tile of workgroups with NTL - 1 tiles use
-//     clamped addresses and a zero scale.
-// After the stream the waves' blocks are summed in a fixed order through LDS (the x buffers
-// are reused) and the same epilogue kinds run, their inputs read from global.
-constexpr int kMbChunkK = 1024;
-constexpr int kMbXs = kMbChunkK + 8;   // LDS row (halfs): 516 dwords = 4 mod 64 banks, conflict-free A reads
-
-__host__ __device__ inline int mb_xbuf_bytes(int MB) { return align16(2 * 16 * MB * kMbXs * 2); }
-__host__ __device__ inline int mb_lds_bytes(int MB, int ntl, int K) {
-  const int x = mb_xbuf_bytes(MB), slab = align16(ntl * MB * kGemvWaves * kWave * 16);
-  return (x > slab ? x : slab) + align16(ntl * (K >> 7) * 32);
-}
-
-__device__ __forceinline__ f16x8 deq_int4_signed(uint32_t w, uint32_t magic) {
-  const f16x8 r = deq_int4_raw(w, magic);   // lanes (1024 + n) and (1024 + 16 n)
-  const f16x2 lo_off = {(f16)-1032.0f, (f16)-1032.0f}, hi_mul = {(f16)0.0625f, (f16)0.0625f},
-              hi_off = {(f16)-72.0f, (f16)-72.0f};
-  // (1024 + 16 n) / 16 - 72 = n - 8 exactly: one v_pk_fma_f16 (the build's -ffp-contract=off
-  // would otherwise split it into a multiply and an add)
-  const f16x2 a = (f16x2){r[0], r[1]} + lo_off, b = __builtin_elementwise_fma((f16x2){r[2], r[3]}, hi_mul, hi_off);
-  const f16x2 c = (f16x2){r[4], r[5]} + lo_off, d = __builtin_elementwise_fma((f16x2){r[6], r[7]}, hi_mul, hi_off);
-  return (f16x8){a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
-}
-
-// Epilogue of one output y[m][nt*16 + n]; the inputs gemv_wq_kernel stages in LDS are read
-// from global.  Shuffle partners (n ^ 1, n + 8) are lanes of the same 16-lane group.
-__device__ __forceinline__ void epilogue_mb(const GemvArgs& a, int nt, int m, int n, float v, bool live) {
-  const ti_epilogue& e = a.epi;
-  const int ng = nt * 16 + n;
-  switch (e.kind) {
-    case TI_EPI_STORE_F32:
-      if (live) ((float*)e.out)[(size_t)m * e.ldo + ng] = v;
-      break;
-    case TI_EPI_STORE_F16:
-      if (live)
-        ((uint16_t*)e.out)[e.out_packed ? TI_PACKED_INDEX(m, ng, e.ldo >> 7) : (size_t)m * e.ldo + ng] = f2h(v);
-      break;
-    case TI_EPI_RESID_F32:
-      if (live) {
-        float* o = (float*)e.out + (size_t)m * e.ldo + ng;
-        *o = *o + v;
-      }
-      break;
-    case TI_EPI_SILU_MUL_F16: {
-      const float up = __shfl_down(v, 8, kWave);
-      if (live && n < 8) {
-        const float s = v / (1.0f + expf(-v));
-        const int j = nt * 8 + n;
-        ((uint16_t*)e.out)[e.out_packed ? TI_PACKED_INDEX(m, j, e.ldo >> 7) : (size_t)m * e.ldo + j] = f2h(up * s);
-      }
-      break;
-    }
-    case TI_EPI_QKV_ROPE_KV: {
-      const float partner = __shfl_xor(v, 1, kWave);
-      if (!live) break;
-      const int hd = e.head_dim, p = e.pos[m];
-      if (ng < e.q_dim + e.kv_dim) {
-        const int base = ng < e.q_dim ? 0 : e.q_dim;
-        const int d = (ng - base) % hd;
-        const float2 cs = *(const float2*)(e.rope_cs + (size_t)p * hd + (d & ~1));
-        const float r = (d & 1) == 0 ? fmaf(-partner, cs.y, v * cs.x) : fmaf(v, cs.x, partner * cs.y);
-        if (ng < e.q_dim) {
-          ((float*)e.out)[(size_t)m * e.ldo + ng] = r;
-        } else {
-          const int kvh = (ng - e.q_dim) / hd;
-          e.k_cache[(size_t)m * e.kv_stream_stride + ((size_t)kvh * e.max_seq + p) * hd + d] = f2h(r);
-        }
-      } else {
-        const int c = ng - e.q_dim - e.kv_dim;
-        const int kvh = c / hd, d = c - kvh * hd;
-        e.v_cache[(size_t)m * e.kv_stream_stride + ((size_t)kvh * e.max_seq + p) * hd + d] = f2h(v);
-      }
-      break;
-    }
-    case TI_EPI_LOGITS_ARGMAX: {
-      unsigned long long key = 0ull;
-      if (live) {
-        ((float*)e.out)[(size_t)m * e.ldo + ng] = v;
-        key = ((unsigned long long)float_order_key(v) << 32) | (unsigned long long)(0xFFFFFFFFu - (uint32_t)ng);
-      }
-#pragma unroll
-      for (int o = 1; o < 16; o <<= 1) {
-        const unsigned long long other = __shfl_xor(key, o, kWave);
-        key = other > key ? other : key;
-      }
-      if (n == 0 && key) atomicMax(e.argmax + (size_t)m * TI_ARGMAX_SLOTS + (blockIdx.x & (TI_ARGMAX_SLOTS - 1)), key);
-      break;
-    }
-    default:
-      break;
-  }
-}
-
-__device__ __forceinline__ void dma_1k(const void* src_lane, void* lds_wave) {   // 64 lanes x 16 B -> LDS
-  __builtin_amdgcn_global_load_lds(src_lane, lds_wave, 16, 0, 0);
-}
-
-template <int MB, int NTL>
-__device__ __forceinline__ void gemv_mb_body(const GemvArgs a, int grid);
-template <int MB, int NTL>
-__global__ __launch_bounds__(kGemvThreads, 1) void gemv_mb_kernel(const GemvArgs a, int grid) {
-  const unsigned long long t_entry = stamp_now();
-  gemv_mb_body<MB, NTL>(a, grid);
-  stamp_end(a.stamp, t_entry);
-}
-template <int MB, int NTL>
-__device__ __forceinline__ void gemv_mb_body(const GemvArgs a, int grid) {
-  constexpr int XDMA = 2 * 16 * MB / kGemvWaves;   // x-chunk DMA instructions per wave (2 per row)
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  const int KT = a.K >> 7, NT = a.N >> 4, NC = (KT + kGemvWaves - 1) / kGemvWaves;
-  const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, kq = lane >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int t0 = (int)(blockIdx.x * (unsigned)NT / (unsigned)grid);
-  const int t1 = (int)((blockIdx.x + 1) * (unsigned)NT / (unsigned)grid);
-  const int ntl = t1 - t0;                           // NTL or NTL - 1
-  f16* xb = (f16*)smem;                              // [2][16 MB][kMbXs]
-  const int xslab = mb_xbuf_bytes(MB) > align16(NTL * MB * kGemvWaves * kWave * 16)
-                        ? mb_xbuf_bytes(MB) : align16(NTL * MB * kGemvWaves * kWave * 16);
-  f32x4* slab = (f32x4*)smem;                        // after the stream: [NTL][MB][8][64]
-  uint16_t* sl = (uint16_t*)(smem + xslab);          // [ntl][KT][16]
-
-  // scales of our tiles first (two pieces per thread cover ntl * KT <= 512 groups)
-  const int n_sc = ntl * KT * 2;
-  const u32x4* sg = (const u32x4*)(a.scales + (size_t)t0 * KT * 16);
-  const u32x4 sc0 = ld_w(sg + (tid < n_sc ? tid : 0));
-  const u32x4 sc1 = ld_w(sg + (tid + kGemvThreads < n_sc ? tid + kGemvThreads : 0));
-
-  const f16* xg = (const f16*)a.x;
-  auto issue_x = [&](int c) {   // chunk c of every row into buffer c & 1 (rows >= M repeat row M-1)
-#pragma unroll
-    for (int q = 0; q < XDMA; ++q) {
-      const int piece = wave * XDMA + q, row = piece >> 1, half = piece & 1;
-      const int m = row < a.M ? row : a.M - 1;
-      int k = c * kMbChunkK + half * 512 + lane * 8;
-      k = k < a.K ? k : a.K - 8;
-#if TI_GEMV_EXP & 8   // diagnostic: no activation traffic (the first chunk only)
-      if (c > 0) continue;
-#endif
-      dma_1k(xg + (size_t)m * a.ldx + k, xb + ((c & 1) * 16 * MB + row) * kMbXs + half * 512);
-    }
-  };
-  const u32x4* tb = a.tiles + lane;
-  auto load = [&](u32x4 (&w)[NTL], int c) {
-#if TI_GEMV_EXP & 32  // diagnostic: no weight traffic (the first chunk's weights re-used)
-    c = 0;
-#endif
-    const int kt = min(c * kGemvWaves + wave, KT - 1);
-#pragma unroll
-    for (int tl = 0; tl < NTL; ++tl) w[tl] = ld_w(tb + ((size_t)(t0 + min(tl, ntl - 1)) * KT + kt) * kWave);
-  };
-  u32x4 B0[NTL], B1[NTL];
-  issue_x(0);
-  load(B0, 0);
-  if (tid < n_sc) ((u32x4*)sl)[tid] = sc0;
-  if (tid + kGemvThreads < n_sc) ((u32x4*)sl)[tid + kGemvThreads] = sc1;
-  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(NTL) : "memory");   // x chunk 0 landed (B0 may fly)
-  lds_barrier();
-
-  f32x4 acc[NTL][MB];
-#pragma unroll
-  for (int t = 0; t < NTL; ++t)
-#pragma unroll
-    for (int b = 0; b < MB; ++b) acc[t][b] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-  uint32_t magic;
-  asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(magic));
-  auto compute = [&](const u32x4 (&w)[NTL], int c) {
-    const int kt = c * kGemvWaves + wave;
-    const bool kvalid = kt < KT;
-    const f16* xr = xb + ((c & 1) * 16 * MB + r) * kMbXs + wave * 128 + kq * 32;   // the tile's k order
-    f16x8 xf[MB][4];
-#pragma unroll
-    for (int b = 0; b < MB; ++b)
-#pragma unroll
-      for (int s4 = 0; s4 < 4; ++s4) xf[b][s4] = *(const f16x8*)(xr + b * 16 * kMbXs + s4 * 8);
-#pragma unroll
-    for (int tl = 0; tl < NTL; ++tl) {
-      f32x4 t[MB];
-#pragma unroll
-      for (int b = 0; b < MB; ++b) t[b] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int s4 = 0; s4 < 4; ++s4) {
-        const f16x8 bf = deq_int4_signed(w[tl][s4], magic);
-#pragma unroll
-        for (int b = 0; b < MB; ++b) t[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[b][s4], bf, t[b], 0, 0, 0);
-      }
-      const float sc = kvalid ? h2f(sl[(min(tl, ntl - 1) * KT + kt) * 16 + r]) : 0.0f;
-#pragma unroll
-      for (int b = 0; b < MB; ++b) {
-        acc[tl][b][0] = fmaf(sc, t[b][0], acc[tl][b][0]);
-        acc[tl][b][1] = fmaf(sc, t[b][1], acc[tl][b][1]);
-        acc[tl][b][2] = fmaf(sc, t[b][2], acc[tl][b][2]);
-        acc[tl][b][3] = fmaf(sc, t[b][3], acc[tl][b][3]);
-      }
-    }
-  };
-  // Per chunk: DMA the next x chunk into the other buffer, load the next weights, compute,
-  // wait for our DMA (the NTL weight loads after it may still fly), barrier.  Reloads past the
-  // end are clamped and harmless; the tail computes load nothing.
-  int c = 0;
-  for (; c + 1 < NC; c += 2) {
-    issue_x(c + 1);
-    load(B1, c + 1);
-    compute(B0, c);
-    asm volatile("s_waitcnt vmcnt(%0)" :: "n"(NTL) : "memory");
-    lds_barrier();
-    issue_x(c + 2 < NC ? c + 2 : NC - 1);
-    load(B0, c + 2 < NC ? c + 2 : NC - 1);
-    compute(B1, c + 1);
-    asm volatile("s_waitcnt vmcnt(%0)" :: "n"(NTL) : "memory");
-    lds_barrier();
-  }
-  if (c < NC) compute(B0, c);
-
-  // ---- sum the 8 waves' blocks in a fixed order, then the epilogue
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // clamped reloads / DMA done before the slab reuses LDS
-  lds_barrier();
-#pragma unroll
-  for (int tl = 0; tl < NTL; ++tl)
-#pragma unroll
-    for (int b = 0; b < MB; ++b) slab[((tl * MB + b) * kGemvWaves + wave) * kWave + lane] = acc[tl][b];
-  lds_barrier();
-  const int n = lane & 15, nblk = ntl * MB * 4;
-  const int nblk_pad = (nblk + kGemvWaves - 1) / kGemvWaves * kGemvWaves;
-  for (int cb = wave; cb < nblk_pad; cb += kGemvWaves) {   // wave-uniform trip count (shuffles inside)
-    const bool ok = cb < nblk;
-    const int cbc = ok ? cb : 0, tl = cbc / (MB * 4), b = (cbc >> 2) % MB, i = cbc & 3;
-    const float* sp = (const float*)(slab + (tl * MB + b) * kGemvWaves * kWave + lane) + i;
-    float v = 0.0f;
-#pragma unroll
-    for (int w = 0; w < kGemvWaves; ++w) v += sp[w * kWave * 4];
-    const int m = b * 16 + 4 * (lane >> 4) + i;
-    epilogue_mb(a, t0 + tl, m, n, v, ok && m < a.M);
-  }
-  if (a.epi.kind == TI_EPI_LOGITS_ARGMAX && a.epi.step_ctr && blockIdx.x == 0 && tid == 0)
-    *a.epi.step_ctr += a.epi.advance;
-}
-
+// gemv_mbr_kernel<MB, NTL>: int4 weights x 3..16 fp16 rows (a batch of a few streams, and long-K projections whose
+// rows no longer fit gemv_wq_kernel's LDS image).  Weights are read once per launch, straight into registers, in
+// chunks of 1024 k (8 k-tiles, one per wave), one chunk ahead.
 __host__ __device__ inline int mbr_slab_bytes(int MB, int ntl) { return align16(ntl * MB * kGemvWaves * kWave * 16); }
 __host__ __device__ inline int mbr_lds_bytes(int MB, int ntl, int K) {
   return mbr_slab_bytes(MB, ntl) + align16(ntl * (K >> 7) * 32);
@@ -1115,7 +813,7 @@ struct MbrChunk {       // one chunk's operands of one wave
   f16x8 x[MB][4];      // A fragments: rows 16 b + (lane & 15), k = kt*128 + 32 (lane >> 4) + 8 s4
 };
 
-// Register-fragment variant (one 16-row block): each wave loads the A fragments of its own
+// Each wave loads the A fragments of its own
 // k-tile straight into registers, one chunk ahead, so no barrier is needed until the end;
 // at <= 16 rows this beats the LDS-staged kernel (bench.py --batch 8/16).
 template <int MB, int NTL>
@@ -1248,58 +946,27 @@ __host__ __device__ inline int rows_slab_bytes(int mb_total, int ntl) {
 // batched fold (ti_hip.h TI_FOLD_SS_ROWS): per-thread partial sums [512] | 1 / rms per row [64] |
 // per-tile sums of h^2 per row [4][64], behind the slab and the scales
 constexpr int kFoldLdsBytes = 4096;
-__host__ __device__ inline int rows_fold_offset(int mb_total, int ntl, int K, bool g32 = false) {
-  return rows_slab_bytes(mb_total, ntl) + align16(ntl * (K >> 7) * 32 * (g32 ? 4 : 1));
+__host__ __device__ inline int rows_fold_offset(int mb_total, int ntl, int K) {
+  return rows_slab_bytes(mb_total, ntl) + align16(ntl * (K >> 7) * 32);
 }
-__host__ __device__ inline int rows_lds_bytes(int mb_total, int ntl, int K, bool g32 = false) {
-  return rows_fold_offset(mb_total, ntl, K, g32) + kFoldLdsBytes;
-}
-
-// Batched fold, consumer side: this thread's share of row `row`'s partial sums of h^2 (rows
-// of R per workgroup, 512 / R threads per row taking partials part, part + P, ...; loads issued
-// 8 at a time, summed in partial order).  fold_rms_finish turns the shares into rms per row.
-__device__ __forceinline__ float fold_share(const GemvArgs& a, int m, int part, int P) {
-  float t = 0.0f;
-  if (m >= a.M) return t;
-  const float* ss = a.epi.ss_in + m;
-  for (int b0 = part; b0 < a.epi.n_ss; b0 += 8 * P) {
-    float v[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = b0 + j * P < a.epi.n_ss ? ss[(size_t)(b0 + j * P) * TI_FOLD_SS_ROWS] : 0.0f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) t += v[j];
-  }
-  return t;
-}
-// part[512] holds every thread's share (thread = part * R + row); rms[row] = sqrt(sum / K + eps)
-// (the M == 1 fold's formula, gemv_wq_kernel XM_F16F).  Call between two workgroup barriers.
-__device__ __forceinline__ void fold_rms_finish(const GemvArgs& a, const float* part, float* rms, int R, int tid) {
-  if (tid < R) {
-    float t = 0.0f;
-    for (int p = 0; p < kGemvThreads / R; ++p) t += part[p * R + tid];
-    rms[tid] = sqrtf(t / (float)a.K + a.eps);
-  }
+__host__ __device__ inline int rows_lds_bytes(int mb_total, int ntl, int K) {
+  return rows_fold_offset(mb_total, ntl, K) + kFoldLdsBytes;
 }
 
 // Workgroups: n_cg column groups x n_rb row blocks of 16 RG MB rows (narrow outputs split the
 // rows: a workgroup's activation bytes shrink with its rows, and its column group's weights are
 // re-read by the other row blocks from the same XCD's L2 -- blockIdx % 8 is the column group's
 // low bits, a speed placement only).
-// G32: group-32 int4 tiles (GGUF Q4_0 blocks, TI_BITS_G32; row-major x only): MFMA step s4 of a
-// k-tile reads k-chunk 32 s4 + 8 kq and is scaled by its own block's scale (4 per tile row and
-// k-tile), as in the fused and tile kernels.
-template <int MB, int NTL, int RG, bool XP, bool G32>
+template <int MB, int NTL, int RG, bool XP>
 __device__ __forceinline__ void gemm_rows_body(const GemvArgs a, int n_cg, int n_rb);
-template <int MB, int NTL, int RG, bool XP, bool G32 = false>
+template <int MB, int NTL, int RG, bool XP>
 __global__ __launch_bounds__(kGemvThreads, 1) void gemm_rows_kernel(const GemvArgs a, int n_cg, int n_rb) {
   const unsigned long long t_entry = stamp_now();
-  gemm_rows_body<MB, NTL, RG, XP, G32>(a, n_cg, n_rb);
+  gemm_rows_body<MB, NTL, RG, XP>(a, n_cg, n_rb);
   stamp_end(a.stamp, t_entry);
 }
-template <int MB, int NTL, int RG, bool XP, bool G32>
+template <int MB, int NTL, int RG, bool XP>
 __device__ __forceinline__ void gemm_rows_body(const GemvArgs a, int n_cg, int n_rb) {
-  static_assert(!(XP && G32), "group-32 rows take row-major activations");
-  constexpr int SG = G32 ? 4 : 1;   // scales per tile row and k-tile
   constexpr int GW = RowsCfg<MB, NTL, RG>::kGroupWaves, WD = RowsCfg<MB, NTL, RG>::kWD;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int KT = a.K >> 7, NT = a.N >> 4;
@@ -1315,23 +982,14 @@ __device__ __forceinline__ void gemm_rows_body(const GemvArgs a, int n_cg, int n
   const int NI = (KT + GW - 1) / GW, NIP = (NI + WD - 1) / WD * WD;
   ROWS_TS(0);
   f32x4* slab = (f32x4*)smem;                        // after the stream: [NTL][RG * MB][8][64]
-  uint16_t* sl = (uint16_t*)(smem + rows_slab_bytes(RG * MB, NTL));   // [ntl][KT][SG][16]
+  uint16_t* sl = (uint16_t*)(smem + rows_slab_bytes(RG * MB, NTL));   // [ntl][KT][16]
 
-  // the workgroup's group scales (ntl * KT * SG <= 512: 2 SG 16-byte pieces per thread), first
-  const int n_sc = ntl * KT * 2 * SG;
-  const u32x4* sg = (const u32x4*)(a.scales + (size_t)t0 * KT * 16 * SG);
+  // the workgroup's group scales (ntl * KT <= 512: two 16-byte pieces per thread), first
+  const int n_sc = ntl * KT * 2;
+  const u32x4* sg = (const u32x4*)(a.scales + (size_t)t0 * KT * 16);
   u32x4 scr[2];
-  if constexpr (G32) {   // transposed to [ntl][KT][16 rows][4 blocks]: one 8-byte LDS read per tile and item
-    for (int i = tid; i < n_sc; i += kGemvThreads) {
-      const u32x4 v = ld_w(sg + i);
-      const int rr0 = (i & 1) * 8, s4 = (i >> 1) & 3, tk = i >> 3;   // piece: 8 rows of block s4 of (tile, kt)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) sl[(tk * 16 + rr0 + e) * 4 + s4] = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
-    }
-  } else {
-#pragma unroll
-    for (int j = 0; j < 2; ++j) scr[j] = ld_w(sg + (tid + j * kGemvThreads < n_sc ? tid + j * kGemvThreads : 0));
-  }
+  for (int j = 0; j < 2; ++j) scr[j] = ld_w(sg + (tid + j * kGemvThreads < n_sc ? tid + j * kGemvThreads : 0));
 
   const f16* xg = (const f16*)a.x;
   const u32x4* tb = a.tiles + lane;
@@ -1358,10 +1016,10 @@ __device__ __forceinline__ void gemm_rows_body(const GemvArgs a, int n_cg, int n
         for (int s4 = 0; s4 < 4; ++s4) x[b][s4] = *(const f16x8*)(xp + s4 * 512);
       } else {
         const int m = min((b0 + grp * MB + b) * 16 + r, a.M - 1);
-        // the tile's k order (A fragments): k = 128 kt + 32 kq + 8 s4 (+ e), group-32 32 s4 + 8 kq
-        const f16* xr = xg + (size_t)m * a.ldx + kt * 128 + kq * (G32 ? 8 : 32);
+        // the tile's k order (A fragments): k = 128 kt + 32 kq + 8 s4 (+ e)
+        const f16* xr = xg + (size_t)m * a.ldx + kt * 128 + kq * 32;
 #pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) x[b][s4] = *(const f16x8*)(xr + s4 * (G32 ? 32 : 8));
+        for (int s4 = 0; s4 < 4; ++s4) x[b][s4] = *(const f16x8*)(xr + s4 * 8);
       }
     }
   };
@@ -1375,14 +1033,12 @@ __device__ __forceinline__ void gemm_rows_body(const GemvArgs a, int n_cg, int n
   // batched fold: the consumer's per-row rms shares (after the first ring loads: their wait
   // costs nothing the first item would not wait for), the producer's per-tile h^2 sums
   constexpr int R = 16 * RG * MB;
-  float* fold_l = (float*)(smem + rows_fold_offset(RG * MB, NTL, a.K, G32));
+  float* fold_l = (float*)(smem + rows_fold_offset(RG * MB, NTL, a.K));
   const bool fold_in = a.epi.ss_in != nullptr, fold_out = a.epi.kind == TI_EPI_RESID_F32 && a.epi.fold_x != nullptr;
   const float share = fold_in ? fold_share(a, b0 * 16 + tid % R, tid / R, kGemvThreads / R) : 0.0f;
-  if constexpr (!G32) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-      if (tid + j * kGemvThreads < n_sc) ((u32x4*)sl)[tid + j * kGemvThreads] = scr[j];
-  }
+  for (int j = 0; j < 2; ++j)
+    if (tid + j * kGemvThreads < n_sc) ((u32x4*)sl)[tid + j * kGemvThreads] = scr[j];
   lds_barrier();
   ROWS_TS(1);
 
@@ -1399,27 +1055,6 @@ __device__ __forceinline__ void gemm_rows_body(const GemvArgs a, int n_cg, int n
     const int ktc = kvalid ? kt : KT - 1;
 #pragma unroll
     for (int tl = 0; tl < NTL; ++tl) {
-      if constexpr (G32) {   // one scale per 32-k block: each MFMA step scaled on its own
-        const uint2 s4p = *(const uint2*)(sl + ((min(tl, ntl - 1) * KT + ktc) * 16 + r) * 4);
-#pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) {
-          const f16x8 bf = deq_int4_signed(w[tl][s4], magic);
-          f32x4 t[MB];
-#pragma unroll
-          for (int b = 0; b < MB; ++b)
-            t[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[b][s4], bf, (f32x4){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-          const uint32_t sp = s4 < 2 ? s4p.x : s4p.y;
-          const float sc = kvalid ? h2f((uint16_t)(sp >> (16 * (s4 & 1)))) : 0.0f;
-#pragma unroll
-          for (int b = 0; b < MB; ++b) {
-            acc[tl][b][0] = fmaf(sc, t[b][0], acc[tl][b][0]);
-            acc[tl][b][1] = fmaf(sc, t[b][1], acc[tl][b][1]);
-            acc[tl][b][2] = fmaf(sc, t[b][2], acc[tl][b][2]);
-            acc[tl][b][3] = fmaf(sc, t[b][3], acc[tl][b][3]);
-          }
-        }
-        continue;
-      }
       f32x4 t[MB];
 #pragma unroll
       for (int b = 0; b < MB; ++b) t[b] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
@@ -1503,708 +1138,7 @@ __device__ __forceinline__ void gemm_rows_body(const GemvArgs a, int n_cg, int n
     *a.epi.step_ctr += a.epi.advance;
 }
 
-// ------------------------------------------------------------- tile kernel (>= 128 rows)
-// Prefill (forward_pass over a prompt chunk, inference_engine.cpp:1429-1491) and very large
-// batches: a classic LDS-tiled MFMA GEMM, compute-bound at these row counts.  One workgroup
-// computes a 128-row x 128-column block; its 8 waves form 2 (rows) x 4 (columns) and each owns
-// 64 rows x 2 weight tiles.  Per 128-k group: the activation block (128 rows x 128 k fp16,
-// 32 KiB) arrives in LDS by LDS-DMA one group ahead (double buffer) -- each DMA instruction
-// fetches 4 contiguous 256-byte row segments, its lanes' 16-byte chunks XOR-swizzled by row so
-// the A-fragment reads are bank-conflict free -- and the waves' packed weights come straight
-// into VGPRs from a ring three groups ahead.  Group scales of the workgroup's tiles sit in LDS.
-// Per group and wave: 2 tiles dequantized (offset-free int4 -> fp16), 16 A fragments read,
-// 32 v_mfma_f32_16x16x32_f16, then the fp32 group-scale FMA.  The workgroup grid is ordered so
-// that the row blocks sharing a column block run on one XCD (blockIdx % 8), where its L2
-// serves their common weight stream.
-// WMR: row-waves per workgroup (2: 128 rows x 4 column-waves; 1: 64 rows x 8 column-waves, half
-// the activation block and no weight tile loaded twice)
-// XB: activation-block buffers (2: double buffer; 4: issued three groups ahead, when the LDS holds them)
-// RB: 16-row blocks per row-wave (4: 64-row waves; 2: 32-row waves for calls of at most 32 rows,
-// half the activation block per group)
-__host__ __device__ inline int tile_lds_bytes(int K, int tpw, bool g32 = false, int wmr = 2, int xb = 2, int rb = 4) {
-  const int n = xb * 16 * rb * wmr * 256 + align16((8 / wmr) * tpw * (K >> 7) * 32 * (g32 ? 4 : 1));
-  // >= the epilogue's staging blocks (tile_epi_lds_bytes) + the batched fold's rms per row
-  return n > 8 * 64 * 20 * 4 + 512 ? n : 8 * 64 * 20 * 4 + 512;
-}
-
-// TPW: weight tiles per wave (2: 128 columns per workgroup; 1: 64 columns, twice the workgroups
-// for the narrow N = 4096 projections, which otherwise fill only 64 of 256 CUs at 256 rows;
-// 4: 256 columns, half the activation bytes per MFMA, when the rows give enough workgroups;
-// 3: 192 columns, e.g. the 7B QKV's 768 tiles at 64 rows as exactly 256 workgroups).
-// G32: group-32 int4 tiles (TI_BITS_G32): MFMA step s4 of a group reads k-chunk 4 s4 + kq and
-// carries its own scale (one per 32-k block), so each step's product is scaled separately.
-#ifndef TI_TILE_ASM
-// 1: both operand streams of the k-loop issued from inline asm (the activation block's LDS-DMA,
-// the weight tiles' VGPR loads) with hand-counted waits.  Beside a builtin LDS-DMA hipcc's waitcnt
-// pass cannot count the VGPR weight loads and drains vmcnt(0) before every group
-// (cdna_hip_programming.md section 5, "Three .s-level traps" (b)); with only the DMA hidden its
-// weight waits count the DMAs as older loads and cut the lookahead; with both hidden every group's
-// loads stay in flight across the barrier as deep as the rings allow.
-#define TI_TILE_ASM 1
-#endif
-#ifndef TI_TILE_WNT
-#define TI_TILE_WNT 0   // weight tiles are re-read by the row blocks of a column block (L2): default policy
-#endif
-// A 16-byte VGPR load hipcc does not count (beside the asm DMA it could not count its own loads
-// exactly either): the caller waits with a counted s_waitcnt and ties the destination ("+v")
-// before any use (cdna_hip_programming.md 5.7, item 1, form ii).
-__device__ __forceinline__ u32x4 ld_w_asm(const u32x4* p) {
-  u32x4 v;
-#if TI_TILE_WNT
-  asm volatile("global_load_dwordx4 %0, %1, off nt" : "=v"(v) : "v"(p) : "memory");
-#else
-  asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(v) : "v"(p) : "memory");
-#endif
-  return v;
-}
-
-#if TI_GEMV_EXP & 16384   // diagnostic (tools/probe_tile.hip): per-wave cycles by loop phase
-__device__ unsigned long long g_tile_cy[4096 * 8 * 8];   // [workgroup][wave][phase]
-#define TILE_CY_DECL()                                \
-  unsigned long long cy_acc[6] = {0, 0, 0, 0, 0, 0}; \
-  unsigned long long cy_t = __builtin_readcyclecounter()
-#define TILE_CY(i)                                           \
-  do {                                                       \
-    const unsigned long long t_ = __builtin_readcyclecounter(); \
-    cy_acc[i] += t_ - cy_t;                                  \
-    cy_t = t_;                                               \
-  } while (0)
-#define TILE_CY_STORE()                                                                          \
-  do {                                                                                           \
-    if (lane == 0)                                                                               \
-      for (int i_ = 0; i_ < 6; ++i_) g_tile_cy[((size_t)blockIdx.x * 8 + wave) * 8 + i_] = cy_acc[i_]; \
-  } while (0)
-#else
-#define TILE_CY_DECL() do { } while (0)
-#define TILE_CY(i) do { } while (0)
-#define TILE_CY_STORE() do { } while (0)
-#endif
-
-// Split-K merge of one wave's block (n_ks > 1): every k-slice's wave stores its fp32 partial
-// block write-through into the workspace and adds to the block's ticket after its stores have
-// drained; the last arriver reads the other slices back (sc1 loads, CH slices per round trip),
-// sums the n_ks slices in slice order (deterministic whatever the arrival order), re-arms the
-// ticket and runs the epilogue.  Workspace: ti_epilogue.splitk_ws (include/ti_hip.h).
-template <int TPW>
-__device__ __forceinline__ bool splitk_merge(const GemvArgs& a, f32x4 (&acc)[TPW][4], int wave_id, int n_waves, int ks,
-                                             int n_ks, int lane) {
-  char* ws = (char*)a.epi.splitk_ws;
-  int32_t* ticket = (int32_t*)ws + wave_id;
-  const __amdgpu_buffer_rsrc_t rs = sc1_rsrc(ws + TI_SPLITK_TICKET_BYTES);
-  constexpr int kSlab = TPW * 4 * kWave * 16;   // bytes per wave and slice
-  auto off = [&](int sl, int t, int b) {
-    return (uint32_t)(((size_t)sl * n_waves + wave_id) * kSlab + (size_t)((t * 4 + b) * kWave + lane) * 16);
-  };
-#pragma unroll
-  for (int t = 0; t < TPW; ++t)
-#pragma unroll
-    for (int b = 0; b < 4; ++b) __builtin_amdgcn_raw_buffer_store_b128(acc[t][b], rs, off(ks, t, b), 0, kAuxSc1Load);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  int arrived = 0;
-  if (lane == 0) arrived = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  arrived = __builtin_amdgcn_readfirstlane(arrived);
-  if (arrived != n_ks - 1) return false;
-#if TI_GEMV_EXP & 1024   // diagnostic: no read-back (the last arriver keeps its own slice)
-  if (lane == 0) __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return true;
-#endif
-  constexpr int CH = TPW >= 4 ? 1 : 4 / TPW;   // slices per round trip (VGPR budget)
-  f32x4 sum[TPW][4];
-#pragma unroll
-  for (int t = 0; t < TPW; ++t)
-#pragma unroll
-    for (int b = 0; b < 4; ++b) sum[t][b] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-  for (int s0 = 0; s0 < n_ks; s0 += CH) {
-    f32x4 ld[CH][TPW][4];
-#pragma unroll
-    for (int c = 0; c < CH; ++c)
-#pragma unroll
-      for (int t = 0; t < TPW; ++t)
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-          ld[c][t][b] = __builtin_bit_cast(
-              f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off(min(s0 + c, n_ks - 1), t, b), 0, kAuxSc1Load));
-#pragma unroll
-    for (int c = 0; c < CH; ++c)
-      if (s0 + c < n_ks)
-#pragma unroll
-        for (int t = 0; t < TPW; ++t)
-#pragma unroll
-          for (int b = 0; b < 4; ++b) sum[t][b] += s0 + c == ks ? acc[t][b] : ld[c][t][b];
-  }
-#pragma unroll
-  for (int t = 0; t < TPW; ++t)
-#pragma unroll
-    for (int b = 0; b < 4; ++b) acc[t][b] = sum[t][b];
-  if (lane == 0) __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // re-arm
-  return true;
-}
-
-#ifndef TI_TILE_PAIR
-// asm pipeline with 4 activation buffers and one weight tile per wave: one barrier per pair of
-// groups (0: per group).  tools/probe_tile: TPW 1 (O, down at 512 rows) 6-9 % fewer cycles,
-// TPW 2-3 5 % more (the barrier's share stays, its per-pair wait doubles), so wider shapes keep
-// one barrier per group.
-#define TI_TILE_PAIR 1
-#endif
-#ifndef TI_TILE_EPI_LDS
-#define TI_TILE_EPI_LDS 1   // 0: every epilogue per element from the MFMA layout (A/B knob)
-#endif
-#ifndef TI_TILE_HALVES
-// 1: the asm loops compute each group as two halves (compute_half: k-steps 0-1, then 2-3, half the A
-// fragments live at a time); 3-5 % less time than the whole group at once (compute) on TPW 2-4 at
-// 256-1024 rows (profiles/r5_tile_halves_ab.txt).  0: compute (A/B knob)
-#define TI_TILE_HALVES 1
-#endif
-constexpr int kTileEpiStride = 20;   // floats per row of a wave's 64 x 16 staging block (padded: no bank conflicts)
-__host__ __device__ constexpr int tile_epi_lds_bytes() { return kGemvWaves * 64 * kTileEpiStride * 4; }
-
-// Epilogue of weight tile tn (16 outputs) for rows mb .. mb + 63 of one wave, from its LDS block
-// stg[row][col] (row stride kTileEpiStride).  Same arithmetic as epilogue_mb, element for element.
-//   STORE_F32 / RESID_F32 / QKV_ROPE_KV: lane l owns columns 4 (l & 3) .. + 3 of rows 16 it + l / 4
-//   SILU_MUL_F16: lane l owns outputs 4 (l & 1) .. + 3 (gate columns, up = column + 8) of rows 32 it + l / 2
-template <int RB = 4>   // the wave's rows: 16 RB
-__device__ __forceinline__ void tile_epilogue_lds(const GemvArgs& a, int tn, int mb, const float* stg, int lane) {
-  const ti_epilogue& e = a.epi;
-  if (e.kind == TI_EPI_SILU_MUL_F16) {
-    const int h = 4 * (lane & 1);
-#pragma unroll
-    for (int it = 0; it < RB / 2; ++it) {
-      const int row = 32 * it + (lane >> 1), m = mb + row;
-      const float4 g = *(const float4*)(stg + row * kTileEpiStride + h);
-      const float4 u = *(const float4*)(stg + row * kTileEpiStride + 8 + h);
-      if (m >= a.M) continue;
-      auto sm = [](float v, float up) { return f2h(up * (v / (1.0f + expf(-v)))); };
-      const uint32_t lo = sm(g.x, u.x) | ((uint32_t)sm(g.y, u.y) << 16), hi = sm(g.z, u.z) | ((uint32_t)sm(g.w, u.w) << 16);
-      *(uint2*)((uint16_t*)e.out + (size_t)m * e.ldo + tn * 8 + h) = make_uint2(lo, hi);
-    }
-    return;
-  }
-  const int c4 = 4 * (lane & 3), ng = tn * 16 + c4;
-  // QKV: the tile lies in one of q / k / v and one head (head_dim % 16 == 0)
-  const int hd = e.head_dim;
-  const bool in_q = ng < e.q_dim, in_k = !in_q && ng < e.q_dim + e.kv_dim;
-  const int c = in_q ? ng : in_k ? ng - e.q_dim : ng - e.q_dim - e.kv_dim;
-  const int kvh = e.kind == TI_EPI_QKV_ROPE_KV ? c / hd : 0, d = c - kvh * hd;
-#pragma unroll
-  for (int it = 0; it < RB; ++it) {
-    const int row = 16 * it + (lane >> 2), m = mb + row;
-    const float4 v = *(const float4*)(stg + row * kTileEpiStride + c4);
-    if (m >= a.M) continue;
-    if (e.kind == TI_EPI_STORE_F32) {
-      *(float4*)((float*)e.out + (size_t)m * e.ldo + ng) = v;
-    } else if (e.kind == TI_EPI_RESID_F32) {
-      float4* o = (float4*)((float*)e.out + (size_t)m * e.ldo + ng);
-      const float4 h = *o;
-      *o = make_float4(h.x + v.x, h.y + v.y, h.z + v.z, h.w + v.w);
-    } else {   // TI_EPI_QKV_ROPE_KV
-      const int p = e.pos[m];
-      if (in_q || in_k) {
-        // (cos, sin) of pairs d / 2 and d / 2 + 1: even output fmaf(-odd, sin, even * cos), odd
-        // output fmaf(odd, cos, even * sin) (epilogue_mb with partner = the other of the pair)
-        const float4 cs = *(const float4*)(e.rope_cs + (size_t)p * hd + d);
-        const float r0 = fmaf(-v.y, cs.y, v.x * cs.x), r1 = fmaf(v.y, cs.x, v.x * cs.y);
-        const float r2 = fmaf(-v.w, cs.w, v.z * cs.z), r3 = fmaf(v.w, cs.z, v.z * cs.w);
-        if (in_q) {
-          *(float4*)((float*)e.out + (size_t)m * e.ldo + ng) = make_float4(r0, r1, r2, r3);
-        } else {
-          *(uint2*)(e.k_cache + (size_t)m * e.kv_stream_stride + ((size_t)kvh * e.max_seq + p) * hd + d) =
-              make_uint2(f2h(r0) | ((uint32_t)f2h(r1) << 16), f2h(r2) | ((uint32_t)f2h(r3) << 16));
-        }
-      } else {
-        *(uint2*)(e.v_cache + (size_t)m * e.kv_stream_stride + ((size_t)kvh * e.max_seq + p) * hd + d) =
-            make_uint2(f2h(v.x) | ((uint32_t)f2h(v.y) << 16), f2h(v.z) | ((uint32_t)f2h(v.w) << 16));
-      }
-    }
-  }
-}
-
-// Physical 16-byte chunk of logical chunk c in activation row `row` of the tile kernel's LDS image:
-// c ^ tile_swz(row).  An A-fragment read (ds_read_b128, lane l: row l & 15, chunk 4 (l >> 4) + s, or
-// 4 s + (l >> 4) with group-32 weights) is serviced in the lane groups {0-3,12-15,20-27},
-// {4-11,16-19,28-31}, {32-35,44-47,52-59}, {36-43,48-51,60-63} (MI355X_MICROARCH.md, LDS); each
-// holds the 16 rows once, rows {0-3,12-15} at one chunk column and rows {4-11} at the next.  With
-// (row + 4) & 15 the first set lands in chunks 0-7 and the second in 8-15 of a row, so the 16 lanes
-// of a group hit 16 different chunks (64 banks): conflict-free.  (row & 15 put both sets on the
-// same 8 chunks: 2-way conflicts in every group, SQ_LDS_BANK_CONFLICT 3.3 cycles per read.)
-#ifndef TI_TILE_SWZ4
-#define TI_TILE_SWZ4 1
-#endif
-__device__ __forceinline__ int tile_swz(int row) { return TI_TILE_SWZ4 ? (row + 4) & 15 : row & 15; }
-
-template <int TPW, bool G32, int WMR, int XB, int RB>
-__device__ __forceinline__ void gemm_tile_body(const GemvArgs a, int n_cb, int n_rb, int n_ks);
-template <int TPW, bool G32 = false, int WMR = 2, int XB = 2, int RB = 4>
-__global__ __launch_bounds__(kGemvThreads, 1) void gemm_tile_kernel(const GemvArgs a, int n_cb, int n_rb, int n_ks) {
-  const unsigned long long t_entry = stamp_now();
-  gemm_tile_body<TPW, G32, WMR, XB, RB>(a, n_cb, n_rb, n_ks);
-  stamp_end(a.stamp, t_entry);
-}
-template <int TPW, bool G32, int WMR, int XB, int RB>
-__device__ __forceinline__ void gemm_tile_body(const GemvArgs a, int n_cb, int n_rb, int n_ks) {
-  constexpr int WCOL = kGemvWaves / WMR, BM = 16 * RB * WMR;   // column-waves, rows per workgroup
-  constexpr int ND = BM / 32;                                  // activation DMA instructions per wave and group
-  static_assert(RB == 4 || (RB == 2 && WMR == 1), "32-row waves: one row-wave per workgroup");
-  static_assert(XB == 2 || (XB == 4 && TI_TILE_ASM), "deep activation ring: asm-issued DMA only");
-  constexpr int XL = XB - 1;                               // groups of activations issued ahead
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  const int KT = a.K >> 7, NT = a.N >> 4;
-  const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, kq = lane >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave / WCOL, wn = wave % WCOL;
-  // blockIdx -> (row block, k-slice, column block): the n_rb row blocks and n_ks k-slices of a
-  // column block share an XCD; k-slice ks covers groups [kb, kb + nk)
-  const int b8 = blockIdx.x & 7, rest = blockIdx.x >> 3;
-  const int rb = rest % n_rb, r2 = rest / n_rb, ks = r2 % n_ks, cb = (r2 / n_ks) * 8 + b8;
-  if (cb >= n_cb) return;
-  const int kb = ks * KT / n_ks, nk = (ks + 1) * KT / n_ks - kb;
-  const int m0 = rb * BM, t0 = cb * WCOL * TPW;
-  f16* xb = (f16*)smem;                                       // [2][BM rows][128 k] swizzled
-  constexpr int SG = G32 ? 4 : 1;                             // scales per tile row and group
-  uint16_t* sl = (uint16_t*)(smem + XB * BM * 256);           // [WCOL TPW tiles][KT][SG][16]
-  const int n_sc = WCOL * TPW * nk * 2 * SG;                  // 16-byte pieces of this k-slice
-  const u32x4* sg = (const u32x4*)(a.scales + (size_t)t0 * KT * 16 * SG);
-  const int ntile_ok = min(WCOL * TPW, NT - t0);
-  // batched fold (decode rows, ti_hip.h TI_FOLD_SS_ROWS): this thread's share of its row's rms
-  // (TPW 4, already short of registers: after the stream)
-  const bool fold_in = a.epi.ss_in != nullptr;
-  float share = fold_in && TPW < 4 ? fold_share(a, m0 + tid % BM, tid / BM, kGemvThreads / BM) : 0.0f;
-  for (int i = tid; i < n_sc; i += kGemvThreads) {
-    const int j = i / (nk * 2 * SG), p = (j * KT + kb) * 2 * SG + (i - j * nk * 2 * SG);   // tile j, piece in slice
-    ((u32x4*)sl)[p] = j < ntile_ok ? ld_w(sg + p) : (u32x4){0u, 0u, 0u, 0u};
-  }
-
-  const f16* xg = (const f16*)a.x;
-  const uint32_t xb_lds = (uint32_t)(uintptr_t)xb;   // LDS byte address of the staging buffers
-  auto issue_x = [&](int kg) __attribute__((always_inline)) {   // BM / 4 DMA instructions per group
-    f16* dst = xb + (kg & (XB - 1)) * BM * 128;
-#pragma unroll
-    for (int q = 0; q < ND; ++q) {
-      const int j = wave * ND + q, row = 4 * j + (lane >> 4), p = lane & 15, c = p ^ tile_swz(row);
-      const int m = min(m0 + row, a.M - 1);
-      if constexpr (TI_TILE_ASM)
-        dma_1k_asm(xg + (size_t)m * a.ldx + kg * 128 + c * 8,
-                   __builtin_amdgcn_readfirstlane(xb_lds + (uint32_t)(((kg & (XB - 1)) * BM * 128 + j * 512) * 2)));
-      else
-        dma_1k(xg + (size_t)m * a.ldx + kg * 128 + c * 8, dst + j * 512);
-    }
-  };
-#ifndef TI_TILE_XREG
-#define TI_TILE_XREG 0   // 1: the activation block through VGPRs + ds_write instead of LDS-DMA
-#endif
-  u32x4 xreg[ND];
-  auto load_xr = [&](int kg) __attribute__((always_inline)) {
-#pragma unroll
-    for (int q = 0; q < ND; ++q) {
-      const int j = wave * ND + q, row = 4 * j + (lane >> 4), c = (lane & 15) ^ tile_swz(row);
-      xreg[q] = *(const u32x4*)(xg + (size_t)min(m0 + row, a.M - 1) * a.ldx + kg * 128 + c * 8);
-    }
-  };
-  auto store_xr = [&](int kg) __attribute__((always_inline)) {
-#pragma unroll
-    for (int q = 0; q < ND; ++q)
-      *(u32x4*)(xb + (kg & 1) * BM * 128 + (wave * ND + q) * 512 + lane * 8) = xreg[q];
-  };
-  const u32x4* tb = a.tiles + lane;
-  auto load_w = [&](u32x4 (&w)[TPW], int kg) __attribute__((always_inline)) {
-    kg = min(kg, KT - 1);
-#pragma unroll
-    for (int t = 0; t < TPW; ++t) {
-      const u32x4* src = tb + ((size_t)min(t0 + wn * TPW + t, NT - 1) * KT + kg) * kWave;
-      if constexpr (TI_TILE_ASM) w[t] = ld_w_asm(src);
-      else w[t] = ld_w(src);
-    }
-  };
-  // weight ring: 4 groups deep (2 at TPW 4, whose 4-deep ring hipcc keeps in scratch); the asm
-  // pipeline keeps 3 (the covering wait then retires W(kg) together with x(kg), see below)
-  constexpr int kTileWR = TI_TILE_ASM ? 3 : (TPW == 4 ? 2 : 4);
-  u32x4 W[kTileWR][TPW];
-  if constexpr (!TI_TILE_ASM) {   // (the asm pipeline issues its first loads inside its loop)
-    if constexpr (TI_TILE_XREG) load_xr(kb);
-    else issue_x(kb);
-#pragma unroll
-    for (int u = 0; u < kTileWR - 1; ++u) load_w(W[u], kb + min(u, nk - 1));
-  }
-  f32x4 acc[TPW][RB];
-#pragma unroll
-  for (int t = 0; t < TPW; ++t)
-#pragma unroll
-    for (int b = 0; b < RB; ++b) acc[t][b] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-  uint32_t magic;
-  asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(magic));
-  auto compute = [&](const u32x4 (&w)[TPW], int kg) __attribute__((always_inline)) {
-    const f16* xr = xb + (kg & (XB - 1)) * BM * 128 + (wm * 16 * RB + r) * 128;
-    f16x8 xf[RB][4];
-#pragma unroll
-    for (int b = 0; b < RB; ++b)
-#pragma unroll
-      for (int s4 = 0; s4 < 4; ++s4)
-        xf[b][s4] = *(const f16x8*)(xr + b * 16 * 128 + (((G32 ? s4 * 4 + kq : kq * 4 + s4) ^ tile_swz(r)) * 8));
-#pragma unroll
-    for (int t = 0; t < TPW; ++t) {
-      if constexpr (G32) {
-#pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) {
-          const f16x8 bf = deq_int4_signed(w[t][s4], magic);
-          f32x4 tmp[RB];
-#pragma unroll
-          for (int b = 0; b < RB; ++b)
-            tmp[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[b][s4], bf, (f32x4){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-          const float sc = h2f(sl[(((wn * TPW + t) * KT + kg) * 4 + s4) * 16 + r]);
-#pragma unroll
-          for (int b = 0; b < RB; ++b) {
-            acc[t][b][0] = fmaf(sc, tmp[b][0], acc[t][b][0]);
-            acc[t][b][1] = fmaf(sc, tmp[b][1], acc[t][b][1]);
-            acc[t][b][2] = fmaf(sc, tmp[b][2], acc[t][b][2]);
-            acc[t][b][3] = fmaf(sc, tmp[b][3], acc[t][b][3]);
-          }
-        }
-        continue;
-      }
-      f32x4 tmp[RB];
-#pragma unroll
-      for (int b = 0; b < RB; ++b) tmp[b] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int s4 = 0; s4 < 4; ++s4) {
-        const f16x8 bf = deq_int4_signed(w[t][s4], magic);
-#pragma unroll
-        for (int b = 0; b < RB; ++b) tmp[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[b][s4], bf, tmp[b], 0, 0, 0);
-      }
-      const float sc = h2f(sl[((wn * TPW + t) * KT + kg) * 16 + r]);
-#pragma unroll
-      for (int b = 0; b < RB; ++b) acc[t][b] = fma_scale4(sc, tmp[b], acc[t][b]);
-    }
-  };
-  // The same group in two halves (k-steps 0-1 / 2-3; the MFMA partials tmpS carried between them):
-  // the same products and sums in the same order as compute.
-  f32x4 tmpS[TPW][RB];
-  auto compute_half = [&](const u32x4 (&w)[TPW], int kg, auto hc) __attribute__((always_inline)) {
-    constexpr int H = decltype(hc)::value;
-    const f16* xr = xb + (kg & (XB - 1)) * BM * 128 + (wm * 16 * RB + r) * 128;
-    f16x8 xf[RB][2];
-#pragma unroll
-    for (int b = 0; b < RB; ++b)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) xf[b][j] = *(const f16x8*)(xr + b * 16 * 128 + (((kq * 4 + 2 * H + j) ^ tile_swz(r)) * 8));
-#pragma unroll
-    for (int t = 0; t < TPW; ++t) {
-      if constexpr (H == 0)
-#pragma unroll
-        for (int b = 0; b < RB; ++b) tmpS[t][b] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const f16x8 bf = deq_int4_signed(w[t][2 * H + j], magic);
-#pragma unroll
-        for (int b = 0; b < RB; ++b) tmpS[t][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[b][j], bf, tmpS[t][b], 0, 0, 0);
-      }
-      if constexpr (H == 1) {
-        const float sc = h2f(sl[((wn * TPW + t) * KT + kg) * 16 + r]);
-#pragma unroll
-        for (int b = 0; b < RB; ++b) acc[t][b] = fma_scale4(sc, tmpS[t][b], acc[t][b]);
-      }
-    }
-  };
-  // Per group kg: x(kg) and W(kg) were issued earlier; issue x(kg + 1) and W(kg + WR - 1),
-  // wait until only those weight loads are younger than x(kg + 1)... (see below), compute kg.
-  const int KTP = (nk + kTileWR - 1) / kTileWR * kTileWR;
-  TILE_CY_DECL();
-  if constexpr (TI_TILE_ASM) {
-    // Every group issues, in order, x(kg + XL) (2 WMR DMA instructions into buffer
-    // (kg + XL) % XB, read last in group kg - 1) and W(kg + 2) (TPW loads into ring slot
-    // (kg + 2) % 3), both clamped into [0, KT): the same count in every group, so the waits are
-    // constants.  The loop starts at group -3 with the compute off, which also makes the first
-    // loads the loop's own code (no prologue whose registers hipcc could shuffle in flight).
-    //   x(kg): younger loads at the top of group kg are W(kg + 3 - XL) and XL - 1 whole groups
-    //          -> vmcnt(NX), then the barrier makes every wave's part visible;
-    //   W(kg): after group kg's own issue, two whole groups are younger -> vmcnt(NWT), then the
-    //          slot's registers are tied ("+v") so nothing reads them earlier.
-    constexpr int NX = (XL - 1) * (ND + TPW) + TPW, NWT = 2 * (ND + TPW);
-    if constexpr (TI_TILE_PAIR && XB == 4 && TPW == 1) {
-      // Pairs of groups per barrier (half the barriers): at the top of pair (kg, kg + 1), kg even,
-      // x(kg) and x(kg + 1) have landed in every wave and every wave is done with pair kg - 2, whose
-      // two buffers then take x(kg + 2) and x(kg + 3); W(kg + 2) goes out every group as before.
-      // Issue order: [pair top: 2 x 2 WMR DMAs, TPW weight loads] [odd group: TPW weight loads], so
-      //   x(kg + 1) at the pair top: the two groups' weight loads are younger -> vmcnt(2 TPW);
-      //   W(kg) after the group's own issue: one pair's worth -> vmcnt(4 WMR + 2 TPW).
-      // Slots: the loop runs in steps of 6 from -6 (k0 = 0 mod 2 and mod 3: static pair and slot
-      // positions); groups before -2 issue nothing (their waits pass at once).
-      constexpr int NX2 = 2 * TPW, NWT2 = 2 * ND + 2 * TPW;
-      for (int k0 = -6; k0 < nk; k0 += 6) {
-#pragma unroll
-        for (int u = 0; u < 6; ++u) {
-          const int kg = k0 + u, su = u % 3;
-          __builtin_amdgcn_sched_barrier(0);   // no interleaving across groups (register pressure)
-          if ((u & 1) == 0) {
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NX2) : "memory");   // x(kg), x(kg + 1)
-            TILE_CY(0);
-            lds_barrier();
-            TILE_CY(1);
-            if (kg >= -2) {
-              issue_x(kb + max(0, min(kg + 2, nk - 1)));
-              issue_x(kb + max(0, min(kg + 3, nk - 1)));
-            }
-          }
-          if (kg >= -2) load_w(W[(su + 2) % 3], kb + max(0, min(kg + 2, nk - 1)));
-          TILE_CY(2);
-          asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NWT2) : "memory");   // W(kg)
-#pragma unroll
-          for (int t = 0; t < TPW; ++t) asm volatile("" : "+v"(W[su][t]));
-          TILE_CY(3);
-          if (kg >= 0 && kg < nk) {
-            if constexpr (TI_TILE_HALVES && !G32) {
-              compute_half(W[su], kb + kg, std::integral_constant<int, 0>());
-              compute_half(W[su], kb + kg, std::integral_constant<int, 1>());
-            } else {
-              compute(W[su], kb + kg);
-            }
-          }
-          TILE_CY(4);
-        }
-      }
-    } else
-    for (int k0 = -kTileWR; k0 < nk; k0 += kTileWR) {   // kg: group of this k-slice
-#pragma unroll
-      for (int u = 0; u < kTileWR; ++u) {
-        const int kg = k0 + u;
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NX) : "memory");   // x(kg): this wave's DMA
-        TILE_CY(0);
-        lds_barrier();
-        TILE_CY(1);
-#if TI_GEMV_EXP & 4096   // diagnostic: the weight stream replaced by re-reads of the first group (L2)
-        issue_x(kb + max(0, min(kg + XL, nk - 1)));
-        load_w(W[(u + 2) % kTileWR], kb);
-#elif TI_GEMV_EXP & 8192   // diagnostic: the activation stream replaced by re-reads of the first group
-        issue_x(kb);
-        load_w(W[(u + 2) % kTileWR], kb + max(0, min(kg + 2, nk - 1)));
-#else
-        issue_x(kb + max(0, min(kg + XL, nk - 1)));
-        load_w(W[(u + 2) % kTileWR], kb + max(0, min(kg + 2, nk - 1)));
-#endif
-        // (also in the groups without compute: a slot's load is always consumed by its tie, so
-        // hipcc never hands its registers to anything else while the load is in flight)
-        TILE_CY(2);
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NWT) : "memory");   // W(kg)
-#pragma unroll
-        for (int t = 0; t < TPW; ++t) asm volatile("" : "+v"(W[u][t]));
-        TILE_CY(3);
-#if TI_GEMV_EXP & 2048   // diagnostic (tools/tile_diag.sh): operand streams only, no dequant / MFMA
-        if (kg >= 0 && kg < nk && lane == 64) compute(W[u], kb + kg);
-#else
-        if (kg >= 0 && kg < nk) {
-          if constexpr (TI_TILE_HALVES && !G32) {
-            compute_half(W[u], kb + kg, std::integral_constant<int, 0>());
-            compute_half(W[u], kb + kg, std::integral_constant<int, 1>());
-          } else {
-            compute(W[u], kb + kg);
-          }
-        }
-#endif
-        TILE_CY(4);
-      }
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the clamped loads past the end
-#pragma unroll
-    for (int u = 0; u < kTileWR; ++u)
-#pragma unroll
-      for (int t = 0; t < TPW; ++t) asm volatile("" : "+v"(W[u][t]));
-  } else {
-  for (int k0 = 0; k0 < KTP; k0 += kTileWR) {
-#pragma unroll
-    for (int u = 0; u < kTileWR; ++u) {
-      const int kg = k0 + u;
-      // x(kg) landed (the loads younger than it: W(kg + WR - 2), TPW instructions) and every
-      // wave is past compute(kg - 1), so buffer (kg + 1) & 1 is free
-      if constexpr (TI_TILE_XREG) {
-        if (kg < nk) store_xr(kb + kg);
-      }
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(TPW) : "memory");
-      lds_barrier();
-      if (kg < nk) {
-        if (kg + 1 < nk) {
-          if constexpr (TI_TILE_XREG) load_xr(kb + kg + 1);
-          else issue_x(kb + kg + 1);
-        }
-        load_w(W[(u + kTileWR - 1) % kTileWR], kb + min(kg + kTileWR - 1, nk - 1));
-        compute(W[u], kb + kg);
-      }
-    }
-  }
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  // every wave is past its last read of the x / scale images (and every DMA into them has
-  // landed): the epilogue may stage through that LDS
-  lds_barrier();
-  const float* rmsv = (const float*)(smem + tile_epi_lds_bytes());   // batched fold: rms per row
-  if (fold_in) {
-    if constexpr (TPW == 4) share = fold_share(a, m0 + tid % BM, tid / BM, kGemvThreads / BM);
-    ((float*)smem)[tid] = share;
-    lds_barrier();
-    fold_rms_finish(a, (const float*)smem, (float*)rmsv, BM, tid);
-    lds_barrier();
-  }
-#if TI_GEMV_EXP & 512   // diagnostic: no split-K merge at all (every slice runs the epilogue)
-  const bool merged = true;
-#else
-  bool merged = n_ks == 1;   // (32-row waves never split: tile_plan)
-  if constexpr (RB == 4)
-    merged = merged || splitk_merge<TPW>(a, acc, (cb * n_rb + rb) * kGemvWaves + wave, n_cb * n_rb * kGemvWaves, ks,
-                                         n_ks, lane);
-#endif
-  // Epilogue, one weight tile at a time (the loop stays rolled: 64 inlined epilogues are too large
-  // to unroll, so the tile's accumulators are picked by static selects and acc stays in
-  // registers).  Kinds with row-contiguous outputs go through the wave's own LDS block
-  // (tile_epilogue_lds: a lane then owns 4 consecutive outputs of a row, 8- / 16-byte accesses
-  // instead of 16 scattered 2- / 4-byte ones per tile); the rest per element from the MFMA layout.
-  const int ek = a.epi.kind;
-  const bool via_lds = TI_TILE_EPI_LDS && (ek == TI_EPI_STORE_F32 || ek == TI_EPI_RESID_F32 || ek == TI_EPI_QKV_ROPE_KV ||
-                                           (ek == TI_EPI_SILU_MUL_F16 && !a.epi.out_packed));
-  float* stg = (float*)smem + wave * (64 * kTileEpiStride);
-#pragma unroll 1
-  for (int t = 0; t < (merged ? TPW : 0); ++t) {
-    const int tn = t0 + wn * TPW + t;
-    f32x4 av[RB];
-#pragma unroll
-    for (int tt = 0; tt < TPW; ++tt)
-      if (tt == t)
-#pragma unroll
-        for (int b = 0; b < RB; ++b) av[b] = acc[tt][b];
-    if (fold_in)
-#pragma unroll
-      for (int b = 0; b < RB; ++b)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) av[b][i] = av[b][i] / rmsv[wm * 16 * RB + b * 16 + 4 * (lane >> 4) + i];
-    if (via_lds) {
-      // lane (r, kq) holds rows b*16 + 4 kq + i of column r; LDS program order within the wave
-      // makes the reads below see these writes, and the next tile's writes follow the reads
-#pragma unroll
-      for (int b = 0; b < RB; ++b)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) stg[(b * 16 + 4 * (lane >> 4) + i) * kTileEpiStride + r] = av[b][i];
-      if (tn < NT) tile_epilogue_lds<RB>(a, tn, m0 + wm * 16 * RB, stg, lane);
-      continue;
-    }
-#pragma unroll
-    for (int b = 0; b < RB; ++b)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int m = m0 + wm * 16 * RB + b * 16 + 4 * (lane >> 4) + i;
-        epilogue_mb(a, tn < NT ? tn : NT - 1, m, r, av[b][i], tn < NT && m < a.M);
-      }
-  }
-  if (a.epi.kind == TI_EPI_LOGITS_ARGMAX && a.epi.step_ctr && blockIdx.x == 0 && tid == 0)
-    *a.epi.step_ctr += a.epi.advance;
-#if TI_GEMV_EXP & 16384
-  if constexpr (TI_TILE_ASM) {
-    TILE_CY(5);
-    TILE_CY_STORE();
-  }
-#endif
-}
-
 static std::atomic<int> g_num_cus{0};   // (a racing first query stores the same value)
-
-// Tile kernel shape by a per-CU byte model: a CU streams a bounded number of bytes per
-// microsecond, a workgroup moves its activation block plus its weight tiles per
-// 128-k group, and the launch takes ceil(workgroups / CUs) rounds; the cheapest shape wins
-// (TI_TILE_NARROW / TI_TILE_WIDE / TI_TILE_WMR1 drop TPW 1 / TPW 4 / 64-row shapes, A/B knobs).
-#if TI_TILE_ASM
-#define TI_TILE_XB4 4
-#else
-#define TI_TILE_XB4 2
-#endif
-#define TI_TILE_FNS_XB(XB)                                                                                     \
-  (const void*)gemm_tile_kernel<1, false, 2, XB>, (const void*)gemm_tile_kernel<2, false, 2, XB>,              \
-      (const void*)gemm_tile_kernel<4, false, 2, XB>, (const void*)gemm_tile_kernel<1, true, 2, XB>,           \
-      (const void*)gemm_tile_kernel<2, true, 2, XB>, (const void*)gemm_tile_kernel<4, true, 2, XB>,            \
-      (const void*)gemm_tile_kernel<1, false, 1, XB>, (const void*)gemm_tile_kernel<2, false, 1, XB>,          \
-      (const void*)gemm_tile_kernel<4, false, 1, XB>, (const void*)gemm_tile_kernel<1, true, 1, XB>,           \
-      (const void*)gemm_tile_kernel<2, true, 1, XB>, (const void*)gemm_tile_kernel<4, true, 1, XB>,             \
-      (const void*)gemm_tile_kernel<3, false, 2, XB>, (const void*)gemm_tile_kernel<3, true, 2, XB>,           \
-      (const void*)gemm_tile_kernel<3, false, 1, XB>, (const void*)gemm_tile_kernel<3, true, 1, XB>
-// 32-row waves (RB 2): one row-wave, the deep activation ring only
-#define TI_TILE_FNS_RB2                                                                                          \
-  (const void*)gemm_tile_kernel<1, false, 1, TI_TILE_XB4, 2>, (const void*)gemm_tile_kernel<2, false, 1, TI_TILE_XB4, 2>, \
-      (const void*)gemm_tile_kernel<3, false, 1, TI_TILE_XB4, 2>, (const void*)gemm_tile_kernel<4, false, 1, TI_TILE_XB4, 2>, \
-      (const void*)gemm_tile_kernel<1, true, 1, TI_TILE_XB4, 2>, (const void*)gemm_tile_kernel<2, true, 1, TI_TILE_XB4, 2>,  \
-      (const void*)gemm_tile_kernel<3, true, 1, TI_TILE_XB4, 2>
-#define TI_TILE_FNS TI_TILE_FNS_XB(2), TI_TILE_FNS_XB(TI_TILE_XB4), TI_TILE_FNS_RB2
-__host__ inline const void* tile_fn(int tpw, bool g32, int wmr, int xb, int rb = 4) {
-  static const void* const fns[] = {TI_TILE_FNS};
-  if (rb == 2) return fns[32 + (g32 ? 4 : 0) + tpw - 1];   // (group-32 at TPW 4: never planned)
-  const int base = xb == 4 ? 16 : 0;
-  if (tpw == 3) return fns[base + 12 + (wmr == 1 ? 2 : 0) + (g32 ? 1 : 0)];
-  return fns[base + (wmr == 1 ? 6 : 0) + (g32 ? 3 : 0) + (tpw == 1 ? 0 : tpw == 2 ? 1 : 2)];
-}
-// the deep activation ring when it fits the LDS
-__host__ inline int tile_xb(int K, int tpw, bool g32, int wmr, int rb = 4) {
-  if (TI_TILE_XB4 != 4) return 2;
-  return tile_lds_bytes(K, tpw, g32, wmr, 4, rb) <= 160 * 1024 ? 4 : 2;
-}
-
-// 32-row waves (they need the deep activation ring)
-__host__ inline bool tile_rb2_on() { return TI_TILE_XB4 == 4; }
-
-// Shapes considered: (row-waves WMR, 16-row blocks per row-wave RB, tiles per wave TPW); a
-// workgroup moves 4 RB WMR KiB of activations and WMR x (8 / WMR) TPW KiB of weights per group.
-// 32-row waves (WMR 1, RB 2) only for calls of at most 32 rows: the 64-row block's activation DMA
-// would move half padding (TI_TILE_RB2=0: A/B knob).  TI_TILE_WMR1=0 keeps 128-row workgroups
-// (A/B knob).  Returns 32 * (RB == 2) + 8 * WMR + TPW.
-__host__ inline int tile_shape(int M, int N, int K, bool g32, int cus) {
-  // 32-row waves only up to 32 rows: at 33-64 rows their second row block re-reads every weight
-  // tile (7-8 % slower on the wide outputs, profiles/r3c_tile_rb2_64rows.txt)
-  constexpr int rb2_rows = 32;
-  const int NT = N >> 4;
-  int best = 8 * 2 + 2;
-  long best_cost = -1;
-  for (int wr : {8, 4, 2}) {   // row-wave shape: 4 RB WMR (2 x 4, 1 x 4, 1 x 2)
-    const int wmr = wr == 8 ? 2 : 1, rb = wr == 2 ? 2 : 4;
-    if (rb == 2 && (!tile_rb2_on() || M > rb2_rows)) continue;
-    for (int tpw : {2, 1, 4, 3}) {
-      // (group-32 at TPW 4 spills to scratch: kept out, its asm-loaded weight ring must stay in VGPRs)
-      if ((tpw == 4 && g32 && TI_TILE_ASM) ||
-          tile_lds_bytes(K, tpw, g32, wmr, 2, rb) > 160 * 1024 || (rb == 2 && tile_xb(K, tpw, g32, wmr, rb) != 4))
-        continue;
-      const int cols = (8 / wmr) * tpw, bm = 16 * rb * wmr;
-      // rounds as launched: ceil(column blocks / 8) x row blocks workgroups on each XCD's CUs
-      const long per_xcd = (long)((NT + cols - 1) / cols + 7) / 8 * ((M + bm - 1) / bm);
-      const long cost = (per_xcd + cus / 8 - 1) / (cus / 8) * (4 * rb * wmr + 8 * tpw);
-      if (best_cost < 0 || cost < best_cost) {
-        best = (rb == 2 ? 32 : 0) + 8 * wmr + tpw;
-        best_cost = cost;
-      }
-    }
-  }
-  return best;
-}
-
-// Tile GEMM plan with split-K (ti_epilogue.splitk_ws).  A split costs ≈ 5–14 µs of seam
-// (write-through partial stores, the ticket, the last arriver's read-back: tools/splitk_diag.sh)
-// and a tile workgroup carries ≈ 7 µs of fixed pipeline cost, so K is split only where the
-// one-slice grid would leave most of the chip idle: at most a quarter of the CUs busy, each
-// slice still at least 8 groups deep, the slices filling at most one round of workgroups.
-// (17..64 decode rows stay on the batched-rows kernel: split there measured slower, 5–14 µs of
-// seam against 12–50 µs launches.)  TI_GEMM_SPLITK=0 turns splitting off (A/B knob).
-__host__ inline bool splitk_on() { return gemm_knobs().splitk; }
-__host__ inline size_t splitk_slab_bytes(int n_ks, int n_cb, int n_rb, int tpw) {
-  return (size_t)n_ks * n_cb * n_rb * kGemvWaves * tpw * 4 * kWave * 16;
-}
-__host__ inline void tile_plan(int M, int N, int K, bool g32, int cus, int64_t ws_bytes, int* wmr_o, int* tpw_o,
-                               int* ks_o, int* rb_o = nullptr) {
-  const int shape = tile_shape(M, N, K, g32, cus);   // the one-slice choice (knobs applied there)
-  const int wmr = (shape >> 3) & 3, tpw = shape & 7, rb = shape & 32 ? 2 : 4;
-  *wmr_o = wmr;
-  *tpw_o = tpw;
-  *ks_o = 1;
-  if (rb_o) *rb_o = rb;
-  if (rb == 2 || !splitk_on() || ws_bytes <= TI_SPLITK_TICKET_BYTES) return;   // (32-row waves never split)
-  const int NT = N >> 4, KT = K >> 7, cols = (8 / wmr) * tpw;
-  const int n_cb = (NT + cols - 1) / cols, n_rb = (M + 64 * wmr - 1) / (64 * wmr);
-  const long wgs = (long)n_cb * n_rb, grid1 = (long)(n_cb + 7) / 8 * 8 * n_rb;   // (launched: whole XCD rows)
-  if (wgs * 4 > cus || (size_t)wgs * kGemvWaves * 4 > TI_SPLITK_TICKET_BYTES) return;
-  int S = (int)(cus / grid1);
-  while (S > 1 && ((KT + S - 1) / S < 8 || splitk_slab_bytes(S, n_cb, n_rb, tpw) + TI_SPLITK_TICKET_BYTES > (size_t)ws_bytes))
-    --S;
-  *ks_o = S;
-}
 
 __host__ inline int gemv_xmode(int x_kind, int M, int K) {
   if (x_kind == TI_X_F16) return XM_F16;
@@ -2286,56 +1220,28 @@ __host__ inline int mb_grid(int MB, int N, int K, int num_cus, int* ntl_out) {
   return grid;
 }
 
-// One 16-row block: the register-fragment kernel; two: the LDS-DMA one.
-static bool mb_use_lds(int MB) { return MB == 2; }
-template <int MB, int NTL>
-static int launch_mb_t(const GemvArgs& a, int grid, int lds, hipStream_t s) {
-  if constexpr (MB == 1) {
-    if (!mb_use_lds(MB)) {
-      hipLaunchKernelGGL((gemv_mbr_kernel<MB, NTL>), dim3(grid), dim3(kGemvThreads), lds, s, a, grid);
-      TI_LAUNCH_CHECK("gemv_mbr_kernel");
-      return TI_OK;
-    }
+static int launch_mb(const GemvArgs& a, int grid, int ntl, int lds, hipStream_t s) {
+#define TI_MB_CASE(n) \
+  case n: hipLaunchKernelGGL((gemv_mbr_kernel<1, n>), dim3(grid), dim3(kGemvThreads), lds, s, a, grid); break
+  switch (ntl) {
+    TI_MB_CASE(1); TI_MB_CASE(2); TI_MB_CASE(3); TI_MB_CASE(4); TI_MB_CASE(5); TI_MB_CASE(6); TI_MB_CASE(7);
+    default: hipLaunchKernelGGL((gemv_mbr_kernel<1, 8>), dim3(grid), dim3(kGemvThreads), lds, s, a, grid);
   }
-  hipLaunchKernelGGL((gemv_mb_kernel<MB, NTL>), dim3(grid), dim3(kGemvThreads), lds, s, a, grid);
-  TI_LAUNCH_CHECK("gemv_mb_kernel");
+#undef TI_MB_CASE
+  TI_LAUNCH_CHECK("gemv_mbr_kernel");
   return TI_OK;
 }
-static int launch_mb(const GemvArgs& a, int MB, int grid, int ntl, int lds, hipStream_t s) {
-  if (MB == 2) {
-    switch (ntl) {
-      case 1: return launch_mb_t<2, 1>(a, grid, lds, s);
-      case 2: return launch_mb_t<2, 2>(a, grid, lds, s);
-      case 3: return launch_mb_t<2, 3>(a, grid, lds, s);
-      case 4: return launch_mb_t<2, 4>(a, grid, lds, s);
-      case 5: return launch_mb_t<2, 5>(a, grid, lds, s);
-      default: return launch_mb_t<2, 6>(a, grid, lds, s);
-    }
-  }
-  switch (ntl) {
-    case 1: return launch_mb_t<1, 1>(a, grid, lds, s);
-    case 2: return launch_mb_t<1, 2>(a, grid, lds, s);
-    case 3: return launch_mb_t<1, 3>(a, grid, lds, s);
-    case 4: return launch_mb_t<1, 4>(a, grid, lds, s);
-    case 5: return launch_mb_t<1, 5>(a, grid, lds, s);
-    case 6: return launch_mb_t<1, 6>(a, grid, lds, s);
-    case 7: return launch_mb_t<1, 7>(a, grid, lds, s);
-    default: return launch_mb_t<1, 8>(a, grid, lds, s);
-  }
-}
 // Rows kernel (M > 16): RG row groups x MB blocks per group, NTL tiles per workgroup.
-static bool rows_on() { return true; }
 __host__ inline void rows_shape(int M, int* MB, int* RG) {
   const int rg = M > 32 ? 2 : 1;   // 64 rows: two groups of 32
   const int mb = (M + 16 * rg - 1) / (16 * rg);
   *MB = mb;
   *RG = rg;
 }
-__host__ inline bool g32_rows_on() { return true; }
 // Tile kernel from this many rows on (the rows kernel takes at most 64 rows).
 static int tile_rows() { return 65; }
-__host__ inline int rows_tiles_cap(int MB, int K, bool g32 = false) {
-  const int lim = MB >= 2 ? 3 : 4, cap = 512 / ((K >> 7) * (g32 ? 4 : 1));   // VGPR budget / scale pieces
+__host__ inline int rows_tiles_cap(int MB, int K) {
+  const int lim = MB >= 2 ? 3 : 4, cap = 512 / (K >> 7);   // VGPR budget / scale pieces
   return cap < 1 ? 1 : (cap > lim ? lim : cap);
 }
 // Column groups for row blocks of MB blocks per group (one round of workgroups where the VGPR
@@ -2343,8 +1249,8 @@ __host__ inline int rows_tiles_cap(int MB, int K, bool g32 = false) {
 // The launch is ceil(n_cg / 8) * 8 * n_rb workgroups spread round-robin over the 8 XCDs, so with
 // row blocks the column groups per block are a multiple of 8 (3 row blocks x 85 groups = 264
 // workgroups put 33 on an XCD of 32 CUs: a second round, 1.7x the time, tools/rows_m_sweep.py).
-__host__ inline int rows_grid(int MB, int N, int K, int num_cus, int* ntl_out, int n_rb = 1, bool g32 = false) {
-  const int NT = N >> 4, cap = rows_tiles_cap(MB, K, g32);
+__host__ inline int rows_grid(int MB, int N, int K, int num_cus, int* ntl_out, int n_rb = 1) {
+  const int NT = N >> 4, cap = rows_tiles_cap(MB, K);
   const int per = n_rb > 1 ? (num_cus / n_rb / 8 * 8 > 0 ? num_cus / n_rb / 8 * 8 : 8) : num_cus;
   int n_cg = NT < per ? NT : per;
   if ((NT + n_cg - 1) / n_cg > cap) n_cg = (NT + cap - 1) / cap;
@@ -2355,11 +1261,10 @@ __host__ inline int rows_grid(int MB, int N, int K, int num_cus, int* ntl_out, i
 // launch's rounds -- a workgroup streams its rows' activations (R K 2 bytes, L2) and its tiles'
 // weights (ntl 8 K bytes); narrow outputs (O, down) take 16-row blocks, wide ones all the rows.
 // TI_GEMM_ROWS_SPLIT=0 keeps all rows in one workgroup (A/B knob).
-__host__ inline void rows_plan(int M, int N, int K, int cus, int* MB, int* RG, int* n_rb, int* n_cg, int* ntl,
-                               bool g32 = false) {
+__host__ inline void rows_plan(int M, int N, int K, int cus, int* MB, int* RG, int* n_rb, int* n_cg, int* ntl) {
   rows_shape(M, MB, RG);   // all rows in one workgroup
   *n_rb = 1;
-  *n_cg = rows_grid(*MB, N, K, cus, ntl, 1, g32);
+  *n_cg = rows_grid(*MB, N, K, cus, ntl, 1);
   if (!gemm_knobs().rows_split) return;
   const int NT = N >> 4;
   auto cost = [&](int mb, int rg, int nrb, int ncg, int nt) {
@@ -2373,7 +1278,7 @@ __host__ inline void rows_plan(int M, int N, int K, int cus, int* MB, int* RG, i
     if (rows >= M) continue;
     const int nrb = (M + rows - 1) / rows;
     int nt = 0;
-    const int ncg = rows_grid(mb, N, K, cus, &nt, nrb, g32);
+    const int ncg = rows_grid(mb, N, K, cus, &nt, nrb);
     const long c = cost(mb, rg, nrb, ncg, nt);
     if (c * 20 < best * 17 && nt <= NT) {   // a clear (15 %) win only: the model ignores round overlap
       best = c;
@@ -2385,44 +1290,39 @@ __host__ inline void rows_plan(int M, int N, int K, int cus, int* MB, int* RG, i
     }
   }
 }
-template <int MB, int RG, bool XP, bool G32>
+template <int MB, int RG, bool XP>
 static int launch_rows_t(const GemvArgs& a, int ntl, int n_cg, int n_rb, int lds, hipStream_t s) {
   const dim3 grid((unsigned)((n_cg + 7) / 8 * 8 * n_rb));
-  if (ntl == 1) hipLaunchKernelGGL((gemm_rows_kernel<MB, 1, RG, XP, G32>), grid, dim3(kGemvThreads), lds, s, a, n_cg, n_rb);
-  else if (ntl == 2) hipLaunchKernelGGL((gemm_rows_kernel<MB, 2, RG, XP, G32>), grid, dim3(kGemvThreads), lds, s, a, n_cg, n_rb);
-  else if (ntl == 3) hipLaunchKernelGGL((gemm_rows_kernel<MB, 3, RG, XP, G32>), grid, dim3(kGemvThreads), lds, s, a, n_cg, n_rb);
-  else if constexpr (MB < 2) hipLaunchKernelGGL((gemm_rows_kernel<MB, 4, RG, XP, G32>), grid, dim3(kGemvThreads), lds, s, a, n_cg, n_rb);
+  if (ntl == 1) hipLaunchKernelGGL((gemm_rows_kernel<MB, 1, RG, XP>), grid, dim3(kGemvThreads), lds, s, a, n_cg, n_rb);
+  else if (ntl == 2) hipLaunchKernelGGL((gemm_rows_kernel<MB, 2, RG, XP>), grid, dim3(kGemvThreads), lds, s, a, n_cg, n_rb);
+  else if (ntl == 3) hipLaunchKernelGGL((gemm_rows_kernel<MB, 3, RG, XP>), grid, dim3(kGemvThreads), lds, s, a, n_cg, n_rb);
+  else if constexpr (MB < 2) hipLaunchKernelGGL((gemm_rows_kernel<MB, 4, RG, XP>), grid, dim3(kGemvThreads), lds, s, a, n_cg, n_rb);
   else return ti_set_error(TI_ERR_ARG, "gemm_rows_kernel: %d tiles per workgroup at MB %d", ntl, MB);
   TI_LAUNCH_CHECK("gemm_rows_kernel");
   return TI_OK;
 }
-template <bool XP, bool G32 = false>
+template <bool XP>
 static int launch_rows_x(const GemvArgs& a, int MB, int RG, int ntl, int n_cg, int n_rb, int lds, hipStream_t s) {
   if (RG == 2)
-    return MB == 1 ? launch_rows_t<1, 2, XP, G32>(a, ntl, n_cg, n_rb, lds, s) : launch_rows_t<2, 2, XP, G32>(a, ntl, n_cg, n_rb, lds, s);
-  return MB == 1 ? launch_rows_t<1, 1, XP, G32>(a, ntl, n_cg, n_rb, lds, s) : launch_rows_t<2, 1, XP, G32>(a, ntl, n_cg, n_rb, lds, s);
+    return MB == 1 ? launch_rows_t<1, 2, XP>(a, ntl, n_cg, n_rb, lds, s) : launch_rows_t<2, 2, XP>(a, ntl, n_cg, n_rb, lds, s);
+  return MB == 1 ? launch_rows_t<1, 1, XP>(a, ntl, n_cg, n_rb, lds, s) : launch_rows_t<2, 1, XP>(a, ntl, n_cg, n_rb, lds, s);
 }
-static int launch_rows(const GemvArgs& a, int MB, int RG, int ntl, int n_cg, int n_rb, int lds, hipStream_t s,
-                       bool g32 = false) {
-  if (g32) return launch_rows_x<false, true>(a, MB, RG, ntl, n_cg, n_rb, lds, s);
+static int launch_rows(const GemvArgs& a, int MB, int RG, int ntl, int n_cg, int n_rb, int lds, hipStream_t s) {
   return a.x_kind == TI_X_F16_PACKED ? launch_rows_x<true>(a, MB, RG, ntl, n_cg, n_rb, lds, s)
                                      : launch_rows_x<false>(a, MB, RG, ntl, n_cg, n_rb, lds, s);
 }
-#define TI_ROWS_FNS1(MB, RG, XP, G)                                                                       \
-  (const void*)gemm_rows_kernel<MB, 1, RG, XP, G>, (const void*)gemm_rows_kernel<MB, 2, RG, XP, G>,          \
-      (const void*)gemm_rows_kernel<MB, 3, RG, XP, G>
-#define TI_ROWS_FNS2(XP, G)                                                                              \
-  TI_ROWS_FNS1(1, 1, XP, G), TI_ROWS_FNS1(2, 1, XP, G), TI_ROWS_FNS1(1, 2, XP, G), TI_ROWS_FNS1(2, 2, XP, G), \
-      (const void*)gemm_rows_kernel<1, 4, 1, XP, G>, (const void*)gemm_rows_kernel<1, 4, 2, XP, G>
-#define TI_ROWS_FNS TI_ROWS_FNS2(false, false), TI_ROWS_FNS2(true, false), TI_ROWS_FNS2(false, true)
+#define TI_ROWS_FNS1(MB, RG, XP)                                                                      \
+  (const void*)gemm_rows_kernel<MB, 1, RG, XP>, (const void*)gemm_rows_kernel<MB, 2, RG, XP>,            \
+      (const void*)gemm_rows_kernel<MB, 3, RG, XP>
+#define TI_ROWS_FNS2(XP)                                                                              \
+  TI_ROWS_FNS1(1, 1, XP), TI_ROWS_FNS1(2, 1, XP), TI_ROWS_FNS1(1, 2, XP), TI_ROWS_FNS1(2, 2, XP),        \
+      (const void*)gemm_rows_kernel<1, 4, 1, XP>, (const void*)gemm_rows_kernel<1, 4, 2, XP>
+#define TI_ROWS_FNS TI_ROWS_FNS2(false), TI_ROWS_FNS2(true)
 
 #define TI_MB_FNS1(K)                                                                                \
   (const void*)K<1, 1>, (const void*)K<1, 2>, (const void*)K<1, 3>, (const void*)K<1, 4>, (const void*)K<1, 5>, \
       (const void*)K<1, 6>, (const void*)K<1, 7>, (const void*)K<1, 8>
-#define TI_MB_FNS                                                                                      \
-  TI_MB_FNS1(gemv_mb_kernel), TI_MB_FNS1(gemv_mbr_kernel), (const void*)gemv_mb_kernel<2, 1>,           \
-      (const void*)gemv_mb_kernel<2, 2>, (const void*)gemv_mb_kernel<2, 3>, (const void*)gemv_mb_kernel<2, 4>, \
-      (const void*)gemv_mb_kernel<2, 5>, (const void*)gemv_mb_kernel<2, 6>
+#define TI_MB_FNS TI_MB_FNS1(gemv_mbr_kernel)
 
 // devices (bit per ordinal) whose attributes are set; engines may be driven from several threads
 // (test_gpu_threads.py): fetch_or, and a repeated setup by a racing first call is harmless
@@ -2443,6 +1343,8 @@ static int query_cus() {
   return n;
 }
 
+int ti::gemm_cus() { return query_cus(); }
+
 extern "C" int ti_gemm_prepare(void) {
   using namespace ti;
   query_cus();
@@ -2459,11 +1361,12 @@ extern "C" int ti_gemm_prepare(void) {
       (const void*)gemv_wq_kernel<16, XM_NORM1>, (const void*)gemv_wq_kernel<16, XM_NORM>,
       (const void*)gemv_wq_kernel<4, XM_F16F>, (const void*)gemv_wq_kernel<8, XM_F16F>,
       (const void*)gemv_wq_kernel<16, XM_F16F>, (const void*)gemv_wq_kernel<4, XM_ATTN>,
-      (const void*)gemv_wq_kernel<8, XM_ATTN>, (const void*)gemv_wq_kernel<16, XM_ATTN>, TI_MB_FNS, TI_ROWS_FNS,
-      TI_TILE_FNS};
+      (const void*)gemv_wq_kernel<8, XM_ATTN>, (const void*)gemv_wq_kernel<16, XM_ATTN>, TI_MB_FNS, TI_ROWS_FNS};
   for (const void* f : fns)
     TI_HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024),
                  "hipFuncSetAttribute(gemv_wq_kernel)");
+  const int rc = wide_prepare();
+  if (rc != TI_OK) return rc;
   g_prepared.fetch_or(bit, std::memory_order_acq_rel);
   return TI_OK;
 }
@@ -2489,19 +1392,14 @@ static bool use_batched(int bits, int x_kind, int M, int N, int K) {
   return !fused_fits(M, N, K) || (mb_ok && M > fused_rows_pref(bits));
 }
 
-// 17..64 int4 rows of a WIDE output take the tile GEMM, whose time is nearly flat there (≈ 27–31 µs
-// at 64 rows for N = 22016 .. 32000, K = 4096), instead of the batched-rows kernel, which moves
-// every row's activations per workgroup: rows x N >= TI_GEMM_TILE_WIDE_MN (env, default 850000;
-// 0 = off) -- the measured crossover (tools/rows_ab.sh: 64 x 12288 rows kernel 19.0 vs tile 26.5 us,
-// 32 x 28672 rows 36.5 vs tile 28.4, 64 x 22016 35.5 vs 28.3, 32 x 22016 25.7 vs 27.2).
-// At 17..32 rows the tile kernel's 32-row waves (RB 2) move a quarter of the activation bytes the
-// batched-rows kernel does and win from N >= 16384 whatever the
-// rows (`profiles/r3c_tile_wide32.txt`: N = 22016 at 17-32 rows 25.1-25.5 -> 18.2-18.8 us, N = 32000
-// 36.1-36.4 -> 21.2-21.8; N = 12288 stays on the rows kernel, 13.8 vs 17.2).
+// 17..64 int4 rows of a WIDE output take the many-rows kernel, whose workgroups copy a row's activations once per
+// 64 columns or more, instead of the batched-rows kernel, which moves every row's activations per workgroup: from
+// rows x N = 850000 on, and at 17..32 rows from N = 16384 on (measured, us, batched-rows / many-rows: 64 x 12288
+// 19.0 / 18.4, 32 x 28672 36.5 / 19.6, 64 x 22016 35.5 / 27.3, 24 x 22016 25.2 / 19.2).
 static bool wide_tile(int bits, int M, int N) {
   constexpr long kWideMN = 850000, kWideN32 = 16384;
   if (bits != 4 || M <= 16 || M >= ti::tile_rows()) return false;
-  if (M <= 32 && ti::tile_rb2_on() && N >= kWideN32) return true;
+  if (M <= 32 && N >= kWideN32) return true;
   return (long)M * N >= kWideMN;
 }
 extern "C" int ti_gemm_packed_rows(int bits, int M) { return bits == 4 && M > 16 && M < ti::tile_rows() ? 1 : 0; }
@@ -2519,13 +1417,18 @@ extern "C" int ti_gemm_fold_partials(int bits, int M, int N, int K) {
 }
 
 extern "C" int ti_gemm_tile_plan(int bits, int M, int N, int K, int64_t ws_bytes, int* wmr, int* tpw, int* n_ks) {
-  const bool g32 = (bits & TI_BITS_G32) != 0;
   if (!wmr || !tpw || !n_ks) return ti_set_error(TI_ERR_ARG, "ti_gemm_tile_plan: null pointer");
   if ((bits & ~TI_BITS_G32) != 4 || M < ti::tile_rows() || M > TI_GEMM_MAX_ROWS || N < 16 || (N & 15) || K < 128 ||
       (K & 127))
     return ti_set_error(TI_ERR_UNSUPPORTED, "ti_gemm_tile_plan: M=%d N=%d K=%d bits %d is not a tile-kernel call", M, N,
                         K, bits);
-  ti::tile_plan(M, N, K, g32, query_cus(), ti::splitk_on() ? ws_bytes : 0, wmr, tpw, n_ks);
+  ti::WidePlan p;
+  if (!ti::wide_plan(bits, M, N, K, query_cus(), ws_bytes, &p))
+    return ti_set_error(TI_ERR_UNSUPPORTED, "ti_gemm_tile_plan: M=%d N=%d K=%d bits %d", M, N, K, bits);
+  // eight waves: one 64 x 384 workgroup, or two of four waves (64 x 128 or 64 x 64 each) on neighbouring row blocks
+  *wmr = p.tiles == 24 ? 1 : 2;
+  *tpw = p.tiles == 24 ? 3 : p.tiles / 4;
+  *n_ks = p.n_ks;
   return TI_OK;
 }
 
@@ -2580,16 +1483,17 @@ static int gemm_impl(const void* tiles, const uint16_t* scales, int bits, const 
   if ((bits != 4 && bits != 8 && bits != 16) || (g32 && bits == 16) || (aff && (!g32 || bits != 4)))
     return ti_set_error(TI_ERR_ARG, "ti_gemm_wq_a16: bits must be 4, 8 or 16 (+ TI_BITS_G32 for 4 / 8, + TI_BITS_AFF "
                         "for 4 | G32; got %d)", bits);
-  // group-32: int4 fp16 rows from tile_rows() on run on the tile kernel, everything else on the
-  // fused kernel (more than 16 rows: in 16-row pieces, below); affine blocks on the fused kernel only
-  const bool g32_tile = g32 && !aff && bits == 4 && x_kind == TI_X_F16 && M >= tile_rows() && !epi->out_packed;
-  // group-32 int4 fp16 rows 17..64: the batched-rows kernel (TI_GEMM_G32_ROWS=0: fused pieces, A/B knob)
-  const bool g32_rowsk = g32 && !aff && bits == 4 && x_kind == TI_X_F16 && M > 16 && M < tile_rows() &&
-                         !epi->out_packed && g32_rows_on();
+  // int4 fp16 rows, row-major: the many-rows kernel (gemm_wide.hip) from 65 rows on and for wide outputs from 17 (the
+  // batched-rows kernel below that: the packed and the row-major form of a call give the same bits), group-32 from 17,
+  // where its 16-byte row pieces are aligned; affine blocks, int8 and fp16 weights run the fused kernel here
+  // (ti_gemm_rows: any format)
+  const int64_t ws_bytes = epi->splitk_ws ? epi->splitk_bytes : 0;
+  WidePlan wp;
+  const bool wide = bits == 4 && !aff && x_kind == TI_X_F16 && M > 16 && (g32 || M >= tile_rows() || wide_tile(bits, M, N)) &&
+                    rows_aligned(x, ldx) && wide_plan(bits | (g32 ? TI_BITS_G32 : 0), M, N, K, query_cus(), ws_bytes, &wp);
   int g32_rows = 16;   // rows per fused launch (its LDS image holds the x rows)
   while (g32 && g32_rows > 1 && !fused_fits(g32_rows, N, K, true, aff)) --g32_rows;
-  if (g32 && (x_kind == TI_X_F16_PACKED ||
-              (!g32_tile && !g32_rowsk && !fused_fits(std::min(M, g32_rows), N, K, true, aff))))
+  if (g32 && (x_kind == TI_X_F16_PACKED || (!wide && !fused_fits(std::min(M, g32_rows), N, K, true, aff))))
     return ti_set_error(TI_ERR_UNSUPPORTED, "ti_gemm_wq_a16: group-32 weights: fused kernel rows (M=%d N=%d K=%d) "
                         "or int4 fp16 rows >= %d; no packed rows", M, N, K, tile_rows());
   if (bits != 16 && !scales) return ti_set_error(TI_ERR_ARG, "ti_gemm_wq_a16: scales required for bits %d", bits);
@@ -2624,32 +1528,19 @@ static int gemm_impl(const void* tiles, const uint16_t* scales, int bits, const 
     return ti_set_error(TI_ERR_UNSUPPORTED, "ti_gemm_wq_a16: K %d / ldx %d above 65535", K, ldx);
   if (x_kind == TI_X_F32_RMSNORM && !norm_w) return ti_set_error(TI_ERR_ARG, "ti_gemm_wq_a16: norm_w required");
   if (ldx < K) return ti_set_error(TI_ERR_ARG, "ti_gemm_wq_a16: ldx %d < K %d", ldx, K);
-  switch (epi->kind) {
-    case TI_EPI_STORE_F32: case TI_EPI_STORE_F16: case TI_EPI_RESID_F32:
-      if (epi->ldo < N) return ti_set_error(TI_ERR_ARG, "ti_gemm_wq_a16: ldo %d < N %d", epi->ldo, N);
-      break;
-    case TI_EPI_SILU_MUL_F16:
-      if (epi->ldo < N / 2) return ti_set_error(TI_ERR_ARG, "ti_gemm_wq_a16: ldo < N/2");
-      break;
-    case TI_EPI_QKV_ROPE_KV:
-      if (!epi->pos || !epi->rope_cs || !epi->k_cache || !epi->v_cache || epi->head_dim <= 0 || epi->head_dim > 128 ||
-          (epi->head_dim & 1) || epi->q_dim + 2 * epi->kv_dim != N || epi->q_dim % epi->head_dim ||
-          epi->kv_dim % epi->head_dim || epi->ldo < epi->q_dim)
-        return ti_set_error(TI_ERR_ARG, "ti_gemm_wq_a16: inconsistent QKV epilogue");
-      break;
-    case TI_EPI_LOGITS_ARGMAX:
-      if (!epi->argmax || epi->ldo < N) return ti_set_error(TI_ERR_ARG, "ti_gemm_wq_a16: argmax/ldo");
-      break;
-    default:
-      return ti_set_error(TI_ERR_ARG, "ti_gemm_wq_a16: unknown epilogue %d", epi->kind);
+  {
+    const int rc = check_epilogue(*epi, N, "ti_gemm_wq_a16");
+    if (rc != TI_OK) return rc;
   }
-  if (g32 && !g32_tile && !g32_rowsk && M > g32_rows) {   // pieces of g32_rows rows through the fused kernel
+  // pieces of rows: group-32 through the fused kernel; int4 rows past the batched-rows kernel that are not aligned
+  const int piece = wide ? 0 : g32 && M > g32_rows ? g32_rows : !g32 && bits == 4 && x_kind == TI_X_F16 && M >= tile_rows() ? tile_rows() - 1 : 0;
+  if (piece) {
     if (x_kind == TI_X_ATTN_SPLITS || x_kind == TI_X_F16_FOLDED || epi->out_packed)
-      return ti_set_error(TI_ERR_UNSUPPORTED, "ti_gemm_wq_a16: group-32 rows > 16 need plain x rows");
+      return ti_set_error(TI_ERR_UNSUPPORTED, "ti_gemm_wq_a16: rows in pieces need plain x rows");
     const size_t x_elem = x_kind == TI_X_F16 ? 2 : 4;
     const size_t out_elem = epi->kind == TI_EPI_STORE_F16 || epi->kind == TI_EPI_SILU_MUL_F16 ? 2 : 4;
-    for (int m0 = 0; m0 < M; m0 += g32_rows) {
-      const int mm = std::min(g32_rows, M - m0);
+    for (int m0 = 0; m0 < M; m0 += piece) {
+      const int mm = std::min(piece, M - m0);
       ti_epilogue ep = *epi;
       ep.out = static_cast<char*>(epi->out) + (size_t)m0 * epi->ldo * out_elem;
       if (ep.pos) ep.pos += m0;
@@ -2657,7 +1548,7 @@ static int gemm_impl(const void* tiles, const uint16_t* scales, int bits, const 
       if (ep.v_cache) ep.v_cache += (size_t)m0 * ep.kv_stream_stride;
       if (ep.argmax) ep.argmax += (size_t)m0 * TI_ARGMAX_SLOTS;
       if (m0 + mm < M) ep.step_ctr = nullptr;
-      const int rc = gemm_impl(tiles, scales, bits | TI_BITS_G32 | (aff ? TI_BITS_AFF : 0),
+      const int rc = gemm_impl(tiles, scales, bits | (g32 ? TI_BITS_G32 : 0) | (aff ? TI_BITS_AFF : 0),
                                static_cast<const char*>(x) + (size_t)m0 * ldx * x_elem,
                                x_kind, ldx, norm_w, eps, mm, N, K, &ep, stream);
       if (rc != TI_OK) return rc;
@@ -2665,7 +1556,7 @@ static int gemm_impl(const void* tiles, const uint16_t* scales, int bits, const 
     return TI_OK;
   }
   const bool packed_x = x_kind == TI_X_F16_PACKED;
-  const bool batched = g32 ? (g32_tile || g32_rowsk) : (packed_x || use_batched(bits, x_kind, M, N, K));
+  const bool batched = wide || (!g32 && (packed_x || use_batched(bits, x_kind, M, N, K)));
   if (epi->out_packed && (!batched || (epi->kind != TI_EPI_STORE_F16 && epi->kind != TI_EPI_SILU_MUL_F16) ||
                           (epi->ldo & 127)))
     return ti_set_error(TI_ERR_ARG, "ti_gemm_wq_a16: out_packed needs the batched-rows kernel, a fp16 store / SiLU "
@@ -2677,37 +1568,26 @@ static int gemm_impl(const void* tiles, const uint16_t* scales, int bits, const 
                         "ti_gemm_wq_a16: M=%d K=%d exceeds the fused kernel (ti_gemm_max_rows); the batched-rows "
                         "kernel needs bits 4 and fp16 rows (normalise with ti_rmsnorm_f16)", M, K);
   int grid = 0, lds = 0, ntl = 0, rMB = 0, rRG = 0, r_rb = 1;
-  const bool has_ws = epi->splitk_ws && epi->splitk_bytes > TI_SPLITK_TICKET_BYTES && splitk_on();
-  const bool tile = batched && x_kind == TI_X_F16 && (M >= tile_rows() || (!g32 && wide_tile(bits, M, N)));
-  const bool rows = !tile && batched && (g32_rowsk || packed_x || M > 32 || (M > 16 && rows_on()));
-  int n_cb = 0, n_rb = 0, n_ks = 1, tpw = 2, wmr = 2, xbuf = 2, trb = 4;
-  if (tile) {
-    tile_plan(M, N, K, g32, query_cus(), has_ws ? epi->splitk_bytes : 0, &wmr, &tpw, &n_ks, &trb);   // (tile_plan)
-    n_rb = (M + 16 * trb * wmr - 1) / (16 * trb * wmr);
-    n_cb = ((N >> 4) + (8 / wmr) * tpw - 1) / ((8 / wmr) * tpw);
-    grid = (n_cb + 7) / 8 * 8 * n_rb * n_ks;
-    xbuf = tile_xb(K, tpw, g32, wmr, trb);
-    lds = tile_lds_bytes(K, tpw, g32, wmr, xbuf, trb);
-  } else if (rows) {
-    rows_on();
-    rows_plan(M, N, K, query_cus(), &rMB, &rRG, &r_rb, &grid, &ntl, g32);   // grid: column groups
-    lds = rows_lds_bytes(rRG * rMB, ntl, K, g32);
+  const bool rows = !wide && batched && M > 16;
+  if (wide) {
+    } else if (rows) {
+    rows_plan(M, N, K, query_cus(), &rMB, &rRG, &r_rb, &grid, &ntl);   // grid: column groups
+    lds = rows_lds_bytes(rRG * rMB, ntl, K);
   } else if (batched) {
-    const int MB = M > 16 ? 2 : 1;
-    grid = mb_grid(MB, N, K, query_cus(), &ntl);
-    lds = mb_use_lds(MB) ? mb_lds_bytes(MB, ntl, K) : mbr_lds_bytes(MB, ntl, K);
+    grid = mb_grid(1, N, K, query_cus(), &ntl);
+    lds = mbr_lds_bytes(1, ntl, K);
   } else {
     grid = gemv_grid(M, N, K, query_cus(), g32, aff);
     lds = gemv_lds_bytes_tiles(M, K, ((N >> 4) + grid - 1) / grid, g32, aff);
   }
-  if ((fold_out && M > 1 && !rows) || (fold_in && !rows && !tile))
+  if ((fold_out && M > 1 && !rows) || (fold_in && !rows && !wide))
     return ti_set_error(TI_ERR_UNSUPPORTED, "ti_gemm_wq_a16: the batched fold runs on the batched-rows (fold_x) / "
-                        "rows or tile (folded input) kernels (M=%d N=%d K=%d)", M, N, K);
+                        "rows or many-rows (folded input) kernels (M=%d N=%d K=%d)", M, N, K);
   if (lds > 160 * 1024)
     return ti_set_error(TI_ERR_UNSUPPORTED, "ti_gemm_wq_a16: LDS image %d B too large (M=%d N=%d K=%d)", lds, M, N, K);
   if (!batched && grid > 0xfff)
     return ti_set_error(TI_ERR_UNSUPPORTED, "ti_gemm_wq_a16: %d workgroups (N=%d) above 4095", grid, N);
-  if (lds > 64 * 1024) {   // no-op once this device is prepared
+  if (wide || lds > 64 * 1024) {   // no-op once this device is prepared
     const int rc = ti_gemm_prepare();
     if (rc != TI_OK) return rc;
   }
@@ -2723,20 +1603,15 @@ static int gemm_impl(const void* tiles, const uint16_t* scales, int bits, const 
   a.N = N;
   a.K = K;
   a.epi = *epi;
+  a.vec = epilogue_vec(*epi);
   {   // workgroups of the launch below (stamp buffer sizing)
-    const long wgs = tile ? grid : rows ? (long)((grid + 7) / 8 * 8) * r_rb : grid;
-    a.stamp = ti_stamp_next(tile ? STAMP_TILE : rows ? STAMP_ROWS : batched ? STAMP_MB : STAMP_GEMV, wgs);
+    const long wgs = wide ? wide_workgroups(wp) : rows ? (long)((grid + 7) / 8 * 8) * r_rb : grid;
+    a.stamp = ti_stamp_next(wide ? STAMP_TILE : rows ? STAMP_ROWS : batched ? STAMP_MB : STAMP_GEMV, wgs);
   }
   hipStream_t s = (hipStream_t)stream;
-  if (tile) {
-    const void* f = tile_fn(tpw, g32, wmr, xbuf, trb);
-    void* args[] = {&a, &n_cb, &n_rb, &n_ks};
-    TI_HIP_CHECK(hipLaunchKernel(f, dim3(grid), dim3(kGemvThreads), args, lds, s), "hipLaunchKernel(gemm_tile_kernel)");
-    TI_LAUNCH_CHECK("gemm_tile_kernel");
-    return TI_OK;
-  }
-  if (rows) return launch_rows(a, rMB, rRG, ntl, grid, r_rb, lds, s, g32);
-  if (batched) return launch_mb(a, M > 16 ? 2 : 1, grid, ntl, lds, s);
+  if (wide) return wide_launch(bits | (g32 ? TI_BITS_G32 : 0), wp, a, s);
+  if (rows) return launch_rows(a, rMB, rRG, ntl, grid, r_rb, lds, s);
+  if (batched) return launch_mb(a, grid, ntl, lds, s);
   if (aff) return launch_gemv<4, true, true>(a, lds, s, grid);
   if (g32) return bits == 4 ? launch_gemv<4, true>(a, lds, s, grid) : launch_gemv<8, true>(a, lds, s, grid);
   if (bits == 4) return launch_gemv<4>(a, lds, s, grid);
@@ -2755,9 +1630,8 @@ extern "C" int ti_gemm_kernel_name(int bits, int x_kind, int M, int N, int K, ch
     return ti_set_error(TI_ERR_ARG, "ti_gemm_kernel_name: bits %d M %d N %d K %d", bits, M, N, K);
   const bool packed_x = x_kind == TI_X_F16_PACKED;
   const bool batched = packed_x || use_batched(bits, x_kind, M, N, K);
-  const bool tile = batched && x_kind == TI_X_F16 && (M >= tile_rows() || wide_tile(bits, M, N));
-  const bool rows = !tile && batched && (packed_x || M > 32 || (M > 16 && rows_on()));
-  const char* name = tile ? "gemm_tile_kernel" : rows ? "gemm_rows_kernel" : batched ? (mb_use_lds(M > 16 ? 2 : 1) ? "gemv_mb_kernel" : "gemv_mbr_kernel") : nullptr;
+  const bool wide = batched && x_kind == TI_X_F16 && (M >= tile_rows() || wide_tile(bits, M, N)), rows = !wide && batched && M > 16;
+  const char* name = wide ? "gemm_wide_kernel" : rows ? "gemm_rows_kernel" : batched ? "gemv_mbr_kernel" : nullptr;
   if (name) snprintf(buf, (size_t)len, "%s", name);
   else snprintf(buf, (size_t)len, "gemv_wq_kernel<%d,%d>", bits, gemv_xmode(x_kind, M, K));
   return TI_OK;
