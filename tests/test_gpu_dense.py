@@ -1,0 +1,81 @@
+"""Large tiles of the layer-stack products (ti_dense, dense_block_kernel) against float64: ragged rows and columns, short
+k, grouped tiles whose experts hold from 1 row to a whole tile.  Bound: K roundings of 2^-24 of the sum of magnitudes
+(fp32 accumulation), and half a unit in the last place of the stored type."""
+from __future__ import annotations
+
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def operands(M, N, K, dtype, batch=1, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    a = torch.randn(M, K, device="cuda", generator=g).to(dtype)
+    w = (torch.randn(batch, -(-N // 16) * 16, K, device="cuda", generator=g) * 0.05).to(dtype)
+    vec = 8 if dtype == torch.bfloat16 else 4
+    # fragment order: [column tile][k-tile][lane][vec], lane l: column l & 15, k from vec * (l >> 4)
+    f = w.view(batch, -1, 16, K // (4 * vec), 4, vec).permute(0, 1, 3, 4, 2, 5).contiguous()
+    return a, w[:, :N], f
+
+
+def call(ti, d):
+    torch.cuda.synchronize()
+    ti.check(ti.lib().ti_dense(C.byref(d), None))
+    ti.sync()
+
+
+def check(got, a, w, dtype, out16=False):
+    ref = a.double() @ w.double().T
+    tol = a.shape[1] * 2.0**-24 * (a.double().abs() @ w.double().abs().T) + (2.0**-8 if out16 else 2.0**-23) * ref.abs()
+    assert (got.double() - ref).abs().le(tol).all()
+
+
+@pytest.mark.parametrize("M,N,K,dtype", [
+    (1100, 8712, 2048, torch.bfloat16),   # 256 x 256: last row tile 76 rows, last columns 8
+    (1281, 8193, 2048, torch.bfloat16),   # .. 1 row, 1 column
+    (700, 8708, 2048, torch.bfloat16),    # 128 x 256
+    (1100, 2051, 8192, torch.bfloat16),   # 128 x 128
+    (1100, 2051, 8256, torch.bfloat16),
+])
+def test_blocks(ti, M, N, K, dtype):
+    a, w, f = operands(M, N, K, dtype)
+    ldo = N + 5
+    out = torch.full((M + 1, ldo), 7.0, device="cuda")
+    d = ti.DenseArgs(w=f.data_ptr(), a=a.data_ptr(), out=out.data_ptr(), lda=K, ldo=ldo, M=M, N=N, K=K, batch=1, epi=ti.DE_F32,
+                     dtype=ti.DT_BF16)
+    call(ti, d)
+    check(out[:M, :N], a, w[0], dtype)
+    assert (out[M] == 7).all() and (out[:, N:] == 7).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("tile_rows", [128, 256])
+@pytest.mark.parametrize("N,K", [(48, 64), (264, 128), (512, 192), (250, 448)])
+def test_grouped_tiles(ti, dtype, tile_rows, N, K):
+    counts = [1, 16, 17, 0, 31, 64, 65, 96, 127, 128, 129, 192, 193, 255, 256, 257]
+    E, M = len(counts), sum(counts)
+    a, w, f = operands(M, N, K, dtype, E, 3)
+    order = torch.randperm(M, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1)).int()
+    tiles, first = [], 0
+    for e, c in enumerate(counts):
+        tiles += [(e, first + i, min(tile_rows, c - i), 0) for i in range(0, c, tile_rows)]
+        first += c
+    tl = torch.zeros(len(tiles) + 9, 4, dtype=torch.int32, device="cuda")
+    tl[:len(tiles)] = torch.tensor(tiles, dtype=torch.int32)
+    n = torch.tensor([len(tiles)], dtype=torch.int32, device="cuda")
+    out = torch.full((M + 1, N), 7.0, device="cuda").to(dtype)
+    d = ti.DenseArgs(w=f.data_ptr(), w_batch=f[0].numel(), a=a.data_ptr(), out=out.data_ptr(), lda=K, ldo=N, M=M, N=N, K=K, batch=1,
+                     epi=ti.DE_T, dtype=ti.DT_BF16 if dtype == torch.bfloat16 else ti.DT_F32, tile_rows=tile_rows,
+                     max_tiles=len(tl), tiles=tl.data_ptr(), n_tiles=n.data_ptr(), rows_in=order.data_ptr(), rows_out=order.data_ptr(),
+                     row_div=1)
+    call(ti, d)
+    first = 0
+    for e, c in enumerate(counts):
+        r = order[first:first + c].long()
+        check(out[r], a[r], w[e], dtype, dtype == torch.bfloat16)
+        first += c
+    assert (out[M] == 7).all()

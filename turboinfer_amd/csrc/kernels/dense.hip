@@ -2,14 +2,16 @@
 // weights x row-major activations on MFMA, bf16 or fp32, with the consumer's first step fused into
 // the epilogue (SiLU * up, rotary pairs, head gates, logits + argmax, key / value fragments).
 //
-// Two kernels share the epilogue:
+// Three kernels share the epilogue:
 //   * dense_skinny_kernel (M <= 64): HBM-bound weight streaming.  One workgroup per 16 output columns,
 //     its waves split k; each weight fragment is one contiguous KiB read once and multiplied with up
 //     to 4 row tiles; the waves' partial sums meet in LDS.
-//   * dense_tile_kernel (more rows): 4 waves side by side over a BM x BN tile, activations staged through
-//     double-buffered LDS in fragment order, each wave's weight fragments straight from L2 into
-//     registers; both 2 or 4 k-stages (128 bytes each) ahead of their use.
-// Both take independent batches (per-head products) or grouped tiles (experts: a tile is up to
+//   * dense_tile_kernel (more rows, tiles up to 64 x 256): 4 waves side by side over a BM x BN tile, activations
+//     staged through double-buffered LDS in fragment order, each wave's weight fragments straight from
+//     L2 into registers; both 2 or 4 k-stages (128 bytes each) ahead of their use.
+//   * dense_block_kernel (tiles of 128 x 128 up to 256 x 256): both operands copied to an LDS ring by DMA,
+//     4 stages ahead, waves in a WM x WN grid.
+// All take independent batches (per-head products) or grouped tiles (experts: a tile is up to
 // tile_rows entries of one expert's list, rows gathered and scattered through the list).
 #include <algorithm>
 
@@ -260,32 +262,62 @@ __global__ __launch_bounds__(64 * W) void dense_skinny_kernel(const ti_dense_arg
   if (EPI == TI_DE_LOGITS && a.step_ctr && nt == 0 && blockIdx.z == 0 && tid == 0) *a.step_ctr += a.advance;
 }
 
+// Consecutive workgroups go to the 8 XCDs in turn.  An XCD gets a contiguous run of the work list, ordered so that
+// neighbours share weight columns (its L2 holds them once): row tiles fastest, for grouped products 4 tiles (mostly one
+// expert's) fastest, then the columns.  Grouped tiles of 128 rows and more: those groups of 4 dealt to the XCDs in turn,
+// since experts' rows differ and a run leaves XCDs waiting for the one with the largest (2048 rows of trained-like
+// routing, 64 experts, gate/up: 275 -> 253 us; 64-row tiles of few rows lose 5 % by it).
+struct TileAt {
+  int id, m, n, y;   // work item, row tile, column tile, batch / grouped tile
+};
+__host__ __device__ inline bool tiles_dealt(const ti_dense_args& a) { return a.tile_rows >= 128; }
+inline int tile_grid(const ti_dense_args& a, int m_tiles, int n_tiles) {
+  if (tiles_dealt(a)) return ((a.max_tiles + 3) / 4 * n_tiles + 7) / 8 * 32;
+  return ((a.tile_rows ? (a.max_tiles + 3) / 4 * 4 : m_tiles) * n_tiles + 7) / 8 * 8;
+}
+__device__ __forceinline__ bool tile_at(const ti_dense_args& a, int m_tiles, int n_tiles, TileAt& t) {
+  if (tiles_dealt(a)) {
+    const int q = (int)(blockIdx.x >> 5) * 8 + (int)(blockIdx.x & 7), b = q / n_tiles;
+    t = {(int)blockIdx.x, 0, q - b * n_tiles, b * 4 + (int)((blockIdx.x >> 3) & 3)};
+    return t.y < *a.n_tiles;
+  }
+  const int list = a.tile_rows ? (*a.n_tiles + 3) / 4 * 4 * n_tiles : m_tiles * n_tiles, per = (list + 7) >> 3;
+  t.id = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per || t.id >= list) return false;
+  if (a.tile_rows) {
+    const int b = t.id / (4 * n_tiles), r = t.id - b * 4 * n_tiles;
+    t.m = 0;
+    t.n = r >> 2;
+    t.y = b * 4 + (r & 3);
+  } else {
+    t.m = t.id % m_tiles;
+    t.n = t.id / m_tiles;
+    t.y = blockIdx.y;
+  }
+  return true;
+}
+
+// One 16 x 16 block of products: row tile mt.. (row m, out row mo of this lane), column tile nt.
+template <class T, int EPI>
+__device__ __forceinline__ void dense_out(const ti_dense_args& a, const DenseSpan& sp, int m, int mo, int mt, int nt, f32x4 v, int lane) {
+  if constexpr (EPI == TI_DE_VFRAG)
+    dense_store_v<T>(a, mt + 4 * (lane >> 4), nt * 16 + (lane & 15), v);
+  else if constexpr (EPI == TI_DE_LOGITS)
+    dense_argmax(a, m, sp.rows, nt * 16 + 4 * (lane >> 4), v, lane, nt);
+  else
+    dense_store<T, EPI>(a, sp.batch, m, mo, sp.rows, nt * 16 + 4 * (lane >> 4), v);
+}
+
 template <class T, int BM, int BN, int D, int EPI>
 __global__ __launch_bounds__(256, BM * BN > 16384 ? 1 : 2) void dense_tile_kernel(const ti_dense_args a, int m_tiles, int n_tiles) {
   typedef typename El<T>::V V;
   constexpr int KT = El<T>::KT, VEC = El<T>::VEC, FM = BM / 16, FN = BN / 64, NA = BM / 32;
   constexpr bool VF = EPI == TI_DE_VFRAG;
   __shared__ V as[2][FM * 2][64];
-  // Consecutive workgroups go to the 8 XCDs in turn; each XCD gets a contiguous run of the work list,
-  // ordered so that neighbours share weight columns (its L2 holds them once): row tiles fastest, for
-  // grouped products 4 tiles (mostly one expert's) fastest, then the columns.
-  const int list = a.tile_rows ? (*a.n_tiles + 3) / 4 * 4 * n_tiles : m_tiles * n_tiles, per = (list + 7) >> 3;
-  const int id = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
-  if ((int)(blockIdx.x >> 3) >= per || id >= list) return;
-  int mtile, ntile, y;
-  if (a.tile_rows) {
-    const int b = id / (4 * n_tiles), r = id - b * 4 * n_tiles;
-    mtile = 0;
-    ntile = r >> 2;
-    y = b * 4 + (r & 3);
-  } else {
-    mtile = id % m_tiles;
-    ntile = id / m_tiles;
-    y = blockIdx.y;
-  }
-  const int m_base = mtile * BM;
+  TileAt at;
   DenseSpan sp;
-  if (!dense_span(a, y, sp, sizeof(T))) return;
+  if (!tile_at(a, m_tiles, n_tiles, at) || !dense_span(a, at.y, sp, sizeof(T))) return;
+  const int m_base = at.m * BM;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int nk = a.K / KT, nst = nk >> 1, NT = (a.N + 15) >> 4;
   const V* ap[NA];
@@ -299,7 +331,7 @@ __global__ __launch_bounds__(256, BM * BN > 16384 ? 1 : 2) void dense_tile_kerne
   const V* wp[FN];
 #pragma unroll
   for (int j = 0; j < FN; ++j)
-    wp[j] = (const V*)sp.w + (size_t)min(ntile * (BN / 16) + wave * FN + j, NT - 1) * nk * 64 + lane;
+    wp[j] = (const V*)sp.w + (size_t)min(at.n * (BN / 16) + wave * FN + j, NT - 1) * nk * 64 + lane;
   f32x4 acc[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
@@ -370,17 +402,148 @@ __global__ __launch_bounds__(256, BM * BN > 16384 ? 1 : 2) void dense_tile_kerne
     const int mo = m < sp.rows ? row_out(a, sp.first + m) : 0;
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
-      const int nt = ntile * (BN / 16) + wave * FN + j;
-      if (nt >= NT) continue;
-      if constexpr (VF)
-        dense_store_v<T>(a, mt + 4 * (lane >> 4), nt * 16 + (lane & 15), acc[i][j]);
-      else if constexpr (EPI == TI_DE_LOGITS)
-        dense_argmax(a, m, sp.rows, nt * 16 + 4 * (lane >> 4), acc[i][j], lane, nt);
-      else
-        dense_store<T, EPI>(a, sp.batch, m, mo, sp.rows, nt * 16 + 4 * (lane >> 4), acc[i][j]);
+      const int nt = at.n * (BN / 16) + wave * FN + j;
+      if (nt < NT) dense_out<T, EPI>(a, sp, m, mo, mt, nt, acc[i][j], lane);
     }
   }
-  if (EPI == TI_DE_LOGITS && a.step_ctr && id == 0 && tid == 0) *a.step_ctr += a.advance;
+  if (EPI == TI_DE_LOGITS && a.step_ctr && at.id == 0 && tid == 0) *a.step_ctr += a.advance;
+}
+
+template <int N>
+__device__ __forceinline__ void wait_dma() {   // all but the wave's N newest vector memory operations done
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+template <int WM, int WN, int FM, int FN, int NS>
+struct BlockCfg {
+  static constexpr int kWaves = WM * WN, BM = 16 * FM * WM, BN = 16 * FN * WN;
+  static constexpr int kFrags = FM * WM + FN * WN, kDma = kFrags / kWaves, kLds = NS * kFrags * 1024;
+  static_assert(kFrags % kWaves == 0 && kLds <= 160 * 1024 && NS >= 4 && FM % 4 == 0 && FN <= FM);
+};
+
+// Bound: a 256 x 256 block's stage takes ~ 0.7 us on a CU alone and ~ 1 us with all CUs at it, of which the products are
+// ~ 0.5; the copies take the rest (32 KiB a stage: ~ 45 KB/us is what a CU takes in from the L2), so the largest block
+// that still gives every CU one wins: it reads least per product.  Wave tiles of 128 x 64 keep the LDS reads (12 KiB per
+// 32 products) below the products' time; fragments are read a stage ahead into the registers just used (208 VGPRs, two
+// waves a SIMD).  Measured, us, best dense_tile_kernel -> this one, bf16: 2048 x 8192, K 2048 95 -> 74; 1500 x 8704,
+// K 2048 88 -> 65; 1500 x 2048, K 8192 105 -> 89; 64 experts x 192 rows, 2816 x 2048 286 -> 226, 2048 x 1408 156 -> 124.
+template <class T, int WM, int WN, int FM, int FN, int NS, int EPI>
+__global__ __launch_bounds__(64 * WM * WN, 2) void dense_block_kernel(const ti_dense_args a, int m_tiles, int n_tiles) {
+  typedef typename El<T>::V V;
+  typedef BlockCfg<WM, WN, FM, FN, NS> C;
+  constexpr int KT = El<T>::KT, VEC = El<T>::VEC, NW = C::kWaves, NF = C::kFrags, ND = C::kDma;
+  constexpr bool VF = EPI == TI_DE_VFRAG;
+  extern __shared__ __attribute__((aligned(1024))) char ring[];
+  TileAt at;
+  DenseSpan sp;
+  if (!tile_at(a, m_tiles, n_tiles, at) || !dense_span(a, at.y, sp, sizeof(T))) return;
+  const int m_base = at.m * C::BM;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int nk = a.K / KT, NT = (a.N + 15) >> 4;
+  // this wave's fragments of a stage (one k-tile of the block): row tiles first, then weight tiles
+  const V* src[ND];
+  uint32_t dst[ND], step[ND];
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)ring;
+#pragma unroll
+  for (int i = 0; i < ND; ++i) {
+    const int f = i * NW + wave;
+    dst[i] = lds0 + (uint32_t)f * 1024;
+    if (f < FM * WM) {
+      const int p = sp.first + min(m_base + f * 16 + (lane & 15), sp.rows - 1);
+      src[i] = (const V*)((const T*)a.a + (size_t)sp.batch * a.a_batch + (size_t)row_in(a, p) * a.lda) + (lane >> 4);
+      step[i] = KT / VEC;
+    } else {
+      src[i] = (const V*)sp.w + (size_t)min(at.n * (FN * WN) + f - FM * WM, NT - 1) * nk * 64 + lane;
+      step[i] = 64;
+    }
+  }
+  uint32_t fill = 0;   // ring byte the next stage is copied to
+  auto dma1 = [&](int i) {
+    dma_1k_asm(src[i], dst[i] + fill);
+    src[i] += step[i];
+  };
+  auto filled = [&] { fill = fill == (NS - 1) * NF * 1024 ? 0 : fill + NF * 1024; };
+  f32x4 acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  V af[FM], w[2][FN];
+  const V* const first = (const V*)ring + lane;
+  const V* cur = first;   // the stage being multiplied
+  // wave (wm, wn): row tiles wm, wm + WM, ..; weight tiles wn * FN ..
+  auto read_a = [&](const V* st, int i) { af[i] = st[(i * WM + wm) * 64]; };
+  auto read_w = [&](const V* st, V (&d)[FN], int j) { d[j] = st[(FM * WM + wn * FN + j) * 64]; };
+  // One stage, the wave's first R row tiles.  Its weights and all but its last R / 4 row tiles were read a stage ago;
+  // each register takes the next stage's fragment as soon as its products are issued.  The last ones are read here, so
+  // that reads of a ring slot end with its stage and the slot is free once every wave has passed the next barrier.
+  auto stage = [&]<int R, int B>(int s) {
+    constexpr int EARLY = R - R / 4;
+    if (s + NS - 2 < nk) wait_dma<(NS - 3) * ND>();   // stage s + 1 is here (the last ones: everything)
+    else wait_dma<0>();
+    __builtin_amdgcn_s_barrier();
+    const bool more = s + NS - 1 < nk;
+    const V* nxt = cur == first + (NS - 1) * NF * 64 ? first : cur + NF * 64;
+#pragma unroll
+    for (int i = EARLY; i < R; ++i) read_a(cur, i);
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[i][j] = VF ? mma(af[i], w[B][j], acc[i][j]) : mma(w[B][j], af[i], acc[i][j]);
+      if (i < EARLY) read_a(nxt, i);
+#pragma unroll
+      for (int j = i * FN / R; j < (i + 1) * FN / R; ++j) read_w(nxt, w[B ^ 1], j);
+      __builtin_amdgcn_sched_barrier(0);
+      if (more) {   // the copies spread over the products: a bunch of them blocks the wave's issue
+#pragma unroll
+        for (int d = 0; d < ND; ++d)
+          if (min(1 + d, R - 1) == i) dma1(d);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (more) filled();
+    cur = nxt;
+  };
+#pragma unroll
+  for (int d = 0; d < NS - 1; ++d)
+    if (d < nk) {
+#pragma unroll
+      for (int i = 0; i < ND; ++i) dma1(i);
+      filled();
+    }
+  if (NS - 1 <= nk) wait_dma<(NS - 2) * ND>();
+  else wait_dma<0>();
+  __builtin_amdgcn_s_barrier();
+#pragma unroll
+  for (int j = 0; j < FN; ++j) read_w(cur, w[0], j);
+  auto product = [&]<int R>() {
+#pragma unroll
+    for (int i = 0; i < R - R / 4; ++i) read_a(cur, i);
+    for (int s = 0; s < nk; s += 2) {   // (K is padded to two k-tiles)
+      stage.template operator()<R, 0>(s);
+      stage.template operator()<R, 1>(s + 1);
+    }
+  };
+  // row tiles a wave needs: a ragged last tile or a small expert's leaves the rest out (the fragment epilogues
+  // write padding rows too)
+  const int live = EPI == TI_DE_KFRAG || EPI == TI_DE_VFRAG ? FM : ((min(sp.rows - m_base, C::BM) + 15) / 16 + WM - 1) / WM;
+  if (live > FM * 3 / 4) product.template operator()<FM>();
+  else if (live > FM / 2) product.template operator()<FM * 3 / 4>();
+  else product.template operator()<FM / 2>();
+#pragma unroll
+  for (int i = 0; i < FM; ++i) {
+    const int mt = m_base + (i * WM + wm) * 16;
+    if (i >= live) break;
+    const int m = mt + (lane & 15);
+    const int mo = m < sp.rows ? row_out(a, sp.first + m) : 0;
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const int nt = at.n * (FN * WN) + wn * FN + j;
+      if (nt < NT) dense_out<T, EPI>(a, sp, m, mo, mt, nt, acc[i][j], lane);
+    }
+  }
+  if (EPI == TI_DE_LOGITS && a.step_ctr && at.id == 0 && tid == 0) *a.step_ctr += a.advance;
 }
 
 template <class T, int MT, int EPI>
@@ -398,10 +561,21 @@ int launch_skinny(const ti_dense_args& a, hipStream_t s) {
 template <class T, int BM, int BN, int D, int EPI>
 int launch_tile(const ti_dense_args& a, hipStream_t s) {
   const int mt = (a.M + BM - 1) / BM, nt = (a.N + BN - 1) / BN;
-  const int list = a.tile_rows ? (a.max_tiles + 3) / 4 * 4 * nt : mt * nt;
-  hipLaunchKernelGGL((dense_tile_kernel<T, BM, BN, D, EPI>), dim3((list + 7) / 8 * 8, a.tile_rows ? 1 : a.batch), dim3(256), 0,
+  hipLaunchKernelGGL((dense_tile_kernel<T, BM, BN, D, EPI>), dim3(tile_grid(a, mt, nt), a.tile_rows ? 1 : a.batch), dim3(256), 0,
                      s, a, mt, nt);
   TI_LAUNCH_CHECK("dense_tile_kernel");
+  return TI_OK;
+}
+
+template <class T, int WM, int WN, int FM, int FN, int NS, int EPI>
+int launch_block(const ti_dense_args& a, hipStream_t s) {
+  typedef BlockCfg<WM, WN, FM, FN, NS> C;
+  const int mt = (a.M + C::BM - 1) / C::BM, nt = (a.N + C::BN - 1) / C::BN;
+  auto* fn = dense_block_kernel<T, WM, WN, FM, FN, NS, EPI>;
+  TI_HIP_CHECK(hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, C::kLds),
+               "hipFuncSetAttribute(dense_block_kernel)");
+  hipLaunchKernelGGL(fn, dim3(tile_grid(a, mt, nt), a.tile_rows ? 1 : a.batch), dim3(64 * C::kWaves), C::kLds, s, a, mt, nt);
+  TI_LAUNCH_CHECK("dense_block_kernel");
   return TI_OK;
 }
 
@@ -415,21 +589,34 @@ int skinny(const ti_dense_args& a, hipStream_t s) {
   return launch_skinny<T, 4, EPI>(a, s);
 }
 
-// More rows: the tile whose rounds over the 256 CUs cost least, by the time of one round of each tile
-// (us at K 2048, measured).
+// More rows: the tile whose rounds over the 256 CUs cost least: us of a launch and per round at K 2048, measured (bf16
+// M 100 .. 2048, N 1024 .. 8704, K 1024 .. 8192; fp32: the products decide, so the smallest tile that fills the chip).
 template <class T, int EPI>
 int tiled(const ti_dense_args& a, hipStream_t s) {
-  auto cost = [&](int bm, int bn, float us) {
-    const long wgs = (long)((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn) * a.batch;
-    return (float)((wgs + 255) / 256) * us;
-  };
-  const float c[4] = {cost(128, 256, 37.f), cost(64, 256, 27.f), cost(64, 128, 15.f), cost(32, 128, 11.5f)};
-  switch (std::min_element(c, c + 4) - c) {
-    case 0: return launch_tile<T, 128, 256, 2, EPI>(a, s);
-    case 1: return launch_tile<T, 64, 256, 2, EPI>(a, s);
-    case 2: return launch_tile<T, 64, 128, 4, EPI>(a, s);
+  constexpr bool F = sizeof(T) == 4;
+  const int bm[6] = {256, 128, 128, 64, 64, 32}, bn[6] = {256, 256, 128, 256, 128, 128};
+  const float fix[6] = {12.f, 5.f, 5.5f, 2.5f, 2.f, 2.f};
+  const float per[6] = {F ? 485.f : 56.f, F ? 250.f : 36.f, F ? 134.f : 24.f, F ? 130.f : 25.f, F ? 72.f : 15.f, F ? 37.f : 10.f};
+  float c[6];
+  for (int i = 0; i < 6; ++i) {
+    const long wgs = (long)((a.M + bm[i] - 1) / bm[i]) * ((a.N + bn[i] - 1) / bn[i]) * a.batch;
+    c[i] = fix[i] + (float)((wgs + 255) / 256) * per[i] * (float)a.K * (1.f / 2048);
+  }
+  switch (std::min_element(c, c + 6) - c) {
+    case 0: return launch_block<T, 2, 4, 8, 4, 5, EPI>(a, s);
+    case 1: return launch_block<T, 2, 4, 4, 4, 5, EPI>(a, s);
+    case 2: return launch_block<T, 2, 2, 4, 4, 5, EPI>(a, s);
+    case 3: return launch_tile<T, 64, 256, 2, EPI>(a, s);
+    case 4: return launch_tile<T, 64, 128, 4, EPI>(a, s);
     default: return launch_tile<T, 32, 128, 4, EPI>(a, s);
   }
+}
+// Grouped products: the tile of the list's rows.
+template <class T, int EPI>
+int grouped(const ti_dense_args& a, hipStream_t s) {
+  if (a.tile_rows == 256) return launch_block<T, 2, 4, 8, 4, 5, EPI>(a, s);
+  if (a.tile_rows == 128) return launch_block<T, 2, 4, 4, 4, 5, EPI>(a, s);
+  return launch_tile<T, 64, 256, 2, EPI>(a, s);
 }
 
 template <class T>
@@ -444,13 +631,10 @@ int dispatch_dense(const ti_dense_args& a, hipStream_t s) {
     case TI_DE_GATE: return few ? skinny<T, TI_DE_GATE>(a, s) : launch_tile<T, 64, 64, 4, TI_DE_GATE>(a, s);
     case TI_DE_SWIGLU:
       if (few) return skinny<T, TI_DE_SWIGLU>(a, s);
-      if (a.tile_rows == 128) return launch_tile<T, 128, 256, 2, TI_DE_SWIGLU>(a, s);
-      return launch_tile<T, 64, 256, 2, TI_DE_SWIGLU>(a, s);
+      return a.tile_rows ? grouped<T, TI_DE_SWIGLU>(a, s) : tiled<T, TI_DE_SWIGLU>(a, s);
     case TI_DE_T:
       if (few) return skinny<T, TI_DE_T>(a, s);
-      if (a.tile_rows == 128) return launch_tile<T, 128, 256, 2, TI_DE_T>(a, s);
-      if (a.tile_rows) return launch_tile<T, 64, 256, 2, TI_DE_T>(a, s);
-      return launch_tile<T, 64, 64, 4, TI_DE_T>(a, s);
+      return a.tile_rows ? grouped<T, TI_DE_T>(a, s) : launch_tile<T, 64, 64, 4, TI_DE_T>(a, s);
     // (every row of a 128-row tile is written by the fragment epilogues)
     case TI_DE_KFRAG: return launch_tile<T, 128, 128, 2, TI_DE_KFRAG>(a, s);
     default: return launch_tile<T, 128, 128, 2, TI_DE_VFRAG>(a, s);
@@ -533,7 +717,8 @@ extern "C" int ti_dense(const ti_dense_args* a, ti_stream_t stream) {
     return ti_set_error(TI_ERR_ARG, "ti_dense: K %d / lda %d not padded", a->K, a->lda);
   if ((!a->tile_rows && !a->rows_in && a->lda < a->K) || a->batch > 65535)
     return ti_set_error(TI_ERR_ARG, "ti_dense: lda %d < K %d or batch %d", a->lda, a->K, a->batch);
-  const bool rows_ok = a->tile_rows == 1 || a->tile_rows == 16 || a->tile_rows == 64 || a->tile_rows == 128;
+  const bool rows_ok = a->tile_rows == 1 || a->tile_rows == 16 || a->tile_rows == 64 || a->tile_rows == 128 ||
+                       a->tile_rows == 256;
   if (a->tile_rows && (a->epi == TI_DE_F32 || a->epi > TI_DE_SWIGLU || !rows_ok || a->max_tiles < 1 || a->max_tiles > 65535 ||
                        a->batch != 1 || (a->rows_in && a->row_div < 1) || !a->tiles ||
                        (a->tile_rows == 1 ? a->rows_in || a->rows_out : !a->n_tiles)))
