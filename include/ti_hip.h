@@ -303,6 +303,16 @@ int ti_attn_decode(const float* q, const uint16_t* k_cache, const uint16_t* v_ca
                    int64_t kv_stream_stride, int max_seq, const int32_t* pos, int M, int heads,
                    int kv_heads, int head_dim, int splits, float* workspace, uint16_t* out,
                    ti_stream_t s);
+/* ti_attn_decode for batches of GQA streams (heads/kv_heads 4 or 8, head_dim 64 or 128): the keys of all streams are
+ * dealt evenly to about `parts` (1 .. 256) workgroups per kv-head, whatever the streams' lengths.  Results agree with
+ * ti_attn_decode to rounding, and depend by rounding on parts and on the other streams' positions.  kv_stream_stride >= kv_heads * max_seq
+ * * head_dim.  Workspace: ti_attn_spread_workspace_bytes for the largest M and parts, zeroed once; its ticket region is
+ * ti_attn_decode's, so one workspace may serve both. */
+size_t ti_attn_spread_workspace_bytes(int M, int heads, int head_dim, int parts);
+int ti_attn_decode_spread(const float* q, const uint16_t* k_cache, const uint16_t* v_cache,
+                          int64_t kv_stream_stride, int max_seq, const int32_t* pos, int M, int heads,
+                          int kv_heads, int head_dim, int parts, float* workspace, uint16_t* out,
+                          ti_stream_t s);
 /* ti_attn_decode writing out in TI_X_F16_PACKED order (K = heads * head_dim, a multiple of 128):
  * the batched O projection's operand. */
 int ti_attn_decode_packed(const float* q, const uint16_t* k_cache, const uint16_t* v_cache,

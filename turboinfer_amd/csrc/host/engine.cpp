@@ -194,6 +194,21 @@ struct ti_engine {
   // 681 tok/s); GQA partials with 8 splits
   static constexpr int attn_target = 256;
   static constexpr int gqa_part_splits = 8;
+  // Workgroups per kv-head of a GQA batch's attention on ti_attn_decode_spread (half the CUs: more of them merge longer
+  // and share CUs, 820 MB of keys 136 us at 128, 144 at 384, 165 at 256); 0: the step runs ti_attn_decode.  4 q-heads a
+  // kv-head at head_dim 128: from 96 streams x kv-heads (measured, us, ti_attn_decode / spread, 8 kv-heads: 2 streams of
+  // 1000 keys 11.2 / 14.1, 8 of 700 13.7 / 15.7, 8 of 3000 27.9 / 25.4, 16 of 750 19.1 / 17.1, 32 of 45 7.4 / 7.4, 32 of 750
+  // 27.8 / 23.0, 32 of 3000 87 / 74); head_dim 64: from 32 (4 kv-heads x 8: 16 of 1200 15.1 / 12.6, 64 of 1200 37.8 / 17.8;
+  // below, the launch alone gains, 2 of 1300 11.2 / 10.9, but a step of 3 streams of 1000 does not, 979 / 997); 8 q-heads
+  // at head_dim 128: any batch (8 x 8: 2 of 60 15.3 / 7.9, 2 of 3000 26.7 / 17.7).
+  int spread_parts(int M) const {
+    const int G = c.kv_heads > 0 && c.heads % c.kv_heads == 0 ? c.heads / c.kv_heads : 0;
+    if (c.compat || c.attn_splits > 0 || M < 2 || (G != 4 && G != 8) || (c.head_dim != 64 && c.head_dim != 128) ||
+        (int64_t)c.max_seq * c.head_dim * 2 > 0x7fffffff || M * c.kv_heads < (c.head_dim == 64 ? 32 : G == 4 ? 96 : 2))
+      return 0;
+    return std::max(1, std::min(256, attn_target / 2 / c.kv_heads));
+  }
+
   int splits_for(int M) const {
     if (c.attn_splits > 0) return c.attn_splits;
     // one stream of a GQA model (>= 4 q-heads per kv-head) with a small cache per kv-head
@@ -446,6 +461,16 @@ int enqueue_head(ti_engine* e, int n, float* x) {
   return gemm_rows(e, e->lm, n, x, TI_X_F32_RMSNORM, c.hidden, e->out_norm, el, 4, false);
 }
 
+// Decode attention of M streams, q -> attn.
+int attn_rows(ti_engine* e, const DevLayer& L, int M) {
+  const ti_engine_config& c = e->c;
+  if (const int parts = e->spread_parts(M))
+    return ti_attn_decode_spread(e->q, L.kc, L.vc, e->kv_stride, c.max_seq, e->pos, M, c.heads, c.kv_heads, c.head_dim, parts,
+                                 e->ws, e->attn, e->s);
+  return ti_attn_decode(e->q, L.kc, L.vc, e->kv_stride, c.max_seq, e->pos, M, c.heads, c.kv_heads, c.head_dim,
+                        e->splits_for(M), e->ws, e->attn, e->s);
+}
+
 // One decode step for streams [0, M) on e->s.  Graph-capturable (no host sync / alloc).
 int enqueue_step(ti_engine* e, int M, int advance) {
   const ti_engine_config& c = e->c;
@@ -581,8 +606,7 @@ int enqueue_step(ti_engine* e, int M, int advance) {
       stamp_tag(TI_STAMP_TAG_QKV);
       TI_TRY(gemm(L.qkv, e->h, TI_X_F32_RMSNORM, H, 4, L.attn_norm, ep, 4, false));
       stamp_tag(TI_STAMP_TAG_ATTN);
-      TI_TRY(ti_attn_decode(e->q, L.kc, L.vc, e->kv_stride, c.max_seq, e->pos, M, c.heads, c.kv_heads, c.head_dim,
-                            e->splits_for(M), e->ws, e->attn, e->s));
+      TI_TRY(attn_rows(e, L, M));
       stamp_tag(TI_STAMP_TAG_O);
       TI_TRY(gemm(L.o, e->attn, TI_X_F16, qd, 2, nullptr, eo, 4, false));
     }
@@ -634,7 +658,10 @@ size_t ws_bytes(const ti_engine* e) {
   const ti_engine_config& c = e->c;
   const int R = prefill_attn_on() ? c.max_batch : e->rows_cap;
   size_t b = 0;
-  for (int M = 1; M <= R; ++M) b = std::max(b, ti_attn_workspace_bytes(M, c.heads, c.head_dim, e->splits_for(M)));
+  for (int M = 1; M <= R; ++M) {
+    b = std::max(b, ti_attn_workspace_bytes(M, c.heads, c.head_dim, e->splits_for(M)));
+    if (e->spread_parts(M) > 0) b = std::max(b, ti_attn_spread_workspace_bytes(M, c.heads, c.head_dim, e->spread_parts(M)));
+  }
   return b;
 }
 
@@ -1933,8 +1960,7 @@ int ti_engine_time_kernel(ti_engine* e, int which, int n, int kv_len, int reps, 
       return ti_attn_decode_partials(e->q, L.kc, L.vc, e->kv_stride, c.max_seq, e->pos, n, c.heads, c.kv_heads,
                                      c.head_dim, e->splits_for(n), e->part_o, e->part_ml, e->s);
     if (which == 5)
-      return ti_attn_decode(e->q, L.kc, L.vc, e->kv_stride, c.max_seq, e->pos, n, c.heads, c.kv_heads, c.head_dim,
-                            e->splits_for(n), e->ws, e->attn, e->s);
+      return attn_rows(e, L, n);
     return gemm_rows(e, *W, n, x, xk, ldx, nw, ep, which == 2 ? 2 : 4, false);
   };
   // The `reps` launches are captured once into a graph and the graph is replayed `rounds`
