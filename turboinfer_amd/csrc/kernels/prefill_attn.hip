@@ -47,6 +47,9 @@ struct PfRaw<64> {
   using V = uint2;      // 4 dims
 };
 
+__device__ __forceinline__ uint32_t pf_word(const u32x4& v, int i) { return v[i]; }
+__device__ __forceinline__ uint32_t pf_word(const uint2& v, int i) { return i == 0 ? v.x : v.y; }
+
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 
 // fp32 x -> (hi, lo) fp16 with hi + lo = x to ~2^-22 relative
@@ -298,7 +301,7 @@ __global__ __launch_bounds__(64, WPE) void attn_prefill_kernel(const float* __re
   }
 }
 
-// ---------------------------------------------------------------- shared K / V blocks (hd 128)
+// ---------------------------------------------------------------- shared K / V blocks
 // The kernel above gives every wave its own K / V stream from L2, and that stream bounds it
 // (profiles/r5_prefill_attn_diag.txt: 21.5 of 24 us at 512 rows; half-line K reads, ~80 block loads
 // per CU).  Here a workgroup takes 4 query blocks of one kv-head -- query wave q block j + q QG, so
@@ -308,6 +311,7 @@ __global__ __launch_bounds__(64, WPE) void attn_prefill_kernel(const float* __re
 // online softmax per column, two blocks per step, and O^T += V^T P^T as one 32-key 16x16x32 product.
 //   K block in LDS: [16 keys][16 chunks of 16 B], the logical chunk c of key row r at physical c ^ r
 //   (an A-fragment read, lane (r, g) chunk 4c + g, is conflict-free in every ds_read_b128 lane group);
+//   head_dim 64: 8 chunks a row, chunk c at c ^ (r >> 1) (a lane group's 16 rows hit each 16 bytes of 256 once);
 //   V block: [16 keys][16 chunks], unswizzled (lane (r, g) reads chunk r of rows 4g + j).
 // Per iteration of BI blocks (2 per half): wait for this wave's 4 DMAs of the iteration; barrier
 // (everyone's landed, and everyone is done with the previous iteration's blocks); DMA the iteration
@@ -328,12 +332,15 @@ __global__ __launch_bounds__(64, WPE) void attn_prefill_kernel(const float* __re
 // HALVES 2: 8 waves, two per SIMD -- waves w and w + 4 share query block w & 3 and take alternate
 // pairs of its key blocks (iteration = 4 blocks, half h computes blocks 2 h, 2 h + 1 of it), merging
 // their (max, sum, O) through LDS at the end: two chains per SIMD hide each other's latencies.
-template <int HALVES, int R>
-__global__ __launch_bounds__(256 * HALVES, 1) void attn_prefill_wg_kernel(const float* __restrict__ q, const uint16_t* __restrict__ kc,
+template <int HD, int HALVES, int R>
+__global__ __launch_bounds__(256 * HALVES, HD == 64 ? 4 : 1) void attn_prefill_wg_kernel(const float* __restrict__ q, const uint16_t* __restrict__ kc,
                                                                  const uint16_t* __restrict__ vc, int max_seq,
                                                                  const int32_t* __restrict__ pos, int M, int heads, int gsh,
                                                                  float scale, uint16_t* __restrict__ out) {
-  constexpr int HD = 128, DV = HD / 16, KW = HD / 32, NB = 2, BI = NB * HALVES;   // BI: blocks per iteration
+  constexpr int DV = HD / 16, KW = HD / 32, NB = 2, BI = NB * HALVES;   // BI: blocks per iteration
+  constexpr int ND = HD / 32, RPD = 16 / ND;   // DMAs of a K or V block, key rows each copies
+  using VRaw = typename PfRaw<HD>::V;
+  auto swz = [](int row) { return HD == 128 ? row : (row >> 1) & 7; };   // chunk c of key row `row` at c ^ swz(row)
   static_assert(R % BI == 0 && R >= 2 * BI, "ring: whole iterations, one in flight beside the one computed");
   // K and V rings in ONE array: the halves' merge at the end reuses it as scratch (4 query blocks x
   // 64 lanes x (4 DV + 2) floats), which is larger than the K ring alone
@@ -380,9 +387,9 @@ __global__ __launch_bounds__(256 * HALVES, 1) void attn_prefill_wg_kernel(const 
   const uint16_t* kbase = kc + (size_t)kvh * max_seq * HD;
   const uint16_t* vbase = vc + (size_t)kvh * max_seq * HD;
   const uint32_t sk_lds = (uint32_t)(uintptr_t)&sk[0][0], sv_lds = (uint32_t)(uintptr_t)&sv[0][0];
-  // An iteration's BI blocks are 8 BI DMA instructions of 1 KiB (a block: K rows 0-3, 4-7, 8-11, 12-15,
-  // then V's); wave w issues instructions 4 w .. 4 w + 3: all of K or all of V of block w / 2.
-  const int dblk = wave >> 1, dv = wave & 1, dch = lane & 15;
+  // An iteration's BI blocks are 2 ND BI DMA instructions of 1 KiB (a block: RPD rows of K each, then V's); wave w
+  // issues ND of them: all of K or all of V of block w / 2.
+  const int dblk = wave >> 1, dv = wave & 1, dch = lane & (HD / 8 - 1);
   auto issue = [&](int kb0) {   // the iteration starting at block kb0
 #if TI_PF_DIAG & 8   // diagnostic: no copies past the prologue (the math on stale blocks)
     if (kb0 >= R - BI) return;
@@ -390,10 +397,10 @@ __global__ __launch_bounds__(256 * HALVES, 1) void attn_prefill_wg_kernel(const 
     const int kb = kb0 + dblk, slot = kb % R;
     const uint32_t base = (dv ? sv_lds : sk_lds) + (uint32_t)(slot * 16 * HD * 2);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = 4 * i + (lane >> 4), key = min(kb * 16 + row, kl);
-      const uint16_t* src = dv ? vbase + (size_t)key * HD + dch * 8 : kbase + (size_t)key * HD + ((dch ^ row) * 8);
-      dma_1k_asm(src, __builtin_amdgcn_readfirstlane(base + (uint32_t)(i * 4 * HD * 2)));
+    for (int i = 0; i < ND; ++i) {
+      const int row = RPD * i + lane / (HD / 8), key = min(kb * 16 + row, kl);
+      const uint16_t* src = dv ? vbase + (size_t)key * HD + dch * 8 : kbase + (size_t)key * HD + ((dch ^ swz(row)) * 8);
+      dma_1k_asm(src, __builtin_amdgcn_readfirstlane(base + (uint32_t)(i * 1024)));
     }
   };
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // q and pos in: only the DMAs are counted below
@@ -405,8 +412,8 @@ __global__ __launch_bounds__(256 * HALVES, 1) void attn_prefill_wg_kernel(const 
   float m_run = -INFINITY, l_run = 0.0f;
   constexpr float kPfSlack = 8.0f;   // as above: O rescaled only when a column max moves by > 8
   for (int kbi = 0; kbi < nkb; kbi += BI) {
-    // this wave's 4 DMAs of iteration kbi are the oldest of the 4 (R / BI - 1) in flight
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * (R / BI - 2)) : "memory");
+    // this wave's ND DMAs of iteration kbi are the oldest of the ND (R / BI - 1) in flight
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(ND * (R / BI - 2)) : "memory");
     __syncthreads();
 #if !TI_PF_WG_LATE_DMA
     issue(kbi + R - BI);
@@ -418,7 +425,7 @@ __global__ __launch_bounds__(256 * HALVES, 1) void attn_prefill_wg_kernel(const 
     const bool act = kb < nkb_w;      // wave-uniform
 #endif
     f32x4 sacc[NB];
-    u32x4 vraw[NB][4];
+    VRaw vraw[NB][4];
     if (act) {
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
@@ -427,7 +434,7 @@ __global__ __launch_bounds__(256 * HALVES, 1) void attn_prefill_wg_kernel(const 
         f32x4 sh = (f32x4){0.0f, 0.0f, 0.0f, 0.0f}, sl = sh;
 #pragma unroll
         for (int c = 0; c < KW; ++c) {
-          const f16x8 kf = __builtin_bit_cast(f16x8, *(const u32x4*)(kr + (((4 * c + g) ^ r) * 8)));
+          const f16x8 kf = __builtin_bit_cast(f16x8, *(const u32x4*)(kr + (((4 * c + g) ^ swz(r)) * 8)));
           sh = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qh[c], sh, 0, 0, 0);
           sl = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, ql[c], sl, 0, 0, 0);
         }
@@ -436,14 +443,14 @@ __global__ __launch_bounds__(256 * HALVES, 1) void attn_prefill_wg_kernel(const 
         sacc[b] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int c = 0; c < KW; ++c) {
-          const f16x8 kf = __builtin_bit_cast(f16x8, *(const u32x4*)(kr + (((4 * c + g) ^ r) * 8)));
+          const f16x8 kf = __builtin_bit_cast(f16x8, *(const u32x4*)(kr + (((4 * c + g) ^ swz(r)) * 8)));
           sacc[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qh[c], sacc[b], 0, 0, 0);
           sacc[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, ql[c], sacc[b], 0, 0, 0);
         }
 #endif
         const uint16_t* vb = &sv[(kb + b) % R][0];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) vraw[b][j] = *(const u32x4*)(vb + (4 * g + j) * HD + r * DV);
+        for (int j = 0; j < 4; ++j) vraw[b][j] = *(const VRaw*)(vb + (4 * g + j) * HD + r * DV);
       }
     }
 #if TI_PF_WG_LATE_DMA   // the next DMAs issued under this step's S = K Q^T rather than before it
@@ -512,8 +519,8 @@ __global__ __launch_bounds__(256 * HALVES, 1) void attn_prefill_wg_kernel(const 
         uint32_t w[4];
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
-          w[2 * b] = __builtin_amdgcn_perm(vraw[b][1][t >> 1], vraw[b][0][t >> 1], sel);
-          w[2 * b + 1] = __builtin_amdgcn_perm(vraw[b][3][t >> 1], vraw[b][2][t >> 1], sel);
+          w[2 * b] = __builtin_amdgcn_perm(pf_word(vraw[b][1], t >> 1), pf_word(vraw[b][0], t >> 1), sel);
+          w[2 * b + 1] = __builtin_amdgcn_perm(pf_word(vraw[b][3], t >> 1), pf_word(vraw[b][2], t >> 1), sel);
         }
         const f16x8 bf = __builtin_bit_cast(f16x8, (u32x4){w[0], w[1], w[2], w[3]});
         acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf, ph, acc[t], 0, 0, 0);
@@ -561,7 +568,8 @@ __global__ __launch_bounds__(256 * HALVES, 1) void attn_prefill_wg_kernel(const 
         const uint16_t hi = __builtin_bit_cast(uint16_t, ti::mul_f16(acc[2 * t + 1][i], inv));
         o[t] = lo | ((uint32_t)hi << 16);
       }
-      *(ti::u32x4*)(dst + i * DV) = (ti::u32x4){o[0], o[1], o[2], o[3]};
+      if constexpr (HD == 128) *(ti::u32x4*)(dst + i * DV) = (ti::u32x4){o[0], o[1], o[2], o[3]};
+      else *(uint2*)(dst + i * DV) = make_uint2(o[0], o[1]);
     }
   }
 }
@@ -613,14 +621,14 @@ extern "C" int ti_attn_prefill(const float* q, const uint16_t* k_cache, const ui
   const bool wg = k > 0, wg2 = k == 2;
   const dim3 gw((grid.x + 3) / 4, kv_heads);
   // 4 query blocks of a kv-head per workgroup, K / V shared in LDS -- when that still gives every CU
-  // a workgroup (256 rows of 7B: 128 workgroups, the per-wave kernel's 512 waves are faster)
-  if (head_dim == 128 && wg && (forced > 1 || (long)gw.x * gw.y * 4 >= ns)) {
-    if (wg2)
-      hipLaunchKernelGGL((ti::attn_prefill_wg_kernel<2, TI_PF_WG_RING2>), gw, dim3(512), 0, s, q, k_cache, v_cache, max_seq,
-                         pos, M, heads, gsh, scale, out);
-    else
-      hipLaunchKernelGGL((ti::attn_prefill_wg_kernel<1, TI_PF_WG_RING>), gw, dim3(256), 0, s, q, k_cache, v_cache, max_seq,
-                         pos, M, heads, gsh, scale, out);
+  // a workgroup (256 rows of 7B: 128 workgroups, the per-wave kernel's 512 waves are faster).  head_dim 64, whose
+  // 8-wave workgroups go two to a CU: from 257 rows at any grid (us, per-wave / shared, 32 heads on 4: 128 rows 5.4 / 6.1,
+  // 256 7.9 / 7.7, 333 10.2 / 9.1, 333 behind 600 keys 20.4 / 16.4, 512 14.5 / 11.0, 1000 36.9 / 25.3; 8 on 8: 256 7.3 /
+  // 7.6, 333 9.4 / 8.8, 1000 20.8 / 16.7).
+  if (wg && (forced > 1 || (head_dim == 64 && wg2 ? M > 256 : (long)gw.x * gw.y * 4 >= ns))) {
+    auto* fn = head_dim == 128 ? (wg2 ? ti::attn_prefill_wg_kernel<128, 2, TI_PF_WG_RING2> : ti::attn_prefill_wg_kernel<128, 1, TI_PF_WG_RING>)
+                               : (wg2 ? ti::attn_prefill_wg_kernel<64, 2, TI_PF_WG_RING2> : ti::attn_prefill_wg_kernel<64, 1, TI_PF_WG_RING>);
+    hipLaunchKernelGGL(fn, gw, dim3(wg2 ? 512 : 256), 0, s, q, k_cache, v_cache, max_seq, pos, M, heads, gsh, scale, out);
   } else if (head_dim == 128) {
     if (deep)
       hipLaunchKernelGGL((ti::attn_prefill_kernel<128, TI_PF_RING_DEEP>), grid, dim3(64), 0, s, q, k_cache, v_cache,
