@@ -441,6 +441,10 @@ typedef struct ti_step_args {
   int32_t xn_ld;
 } ti_step_args;
 int ti_step_begin(const ti_step_args* a, ti_stream_t s);
+/* One-token inputs of n rows for ti_step_begin, read by one launch from page-locked host memory `in` (n tokens, n
+ * positions, and with `slot` n slots): in_tokens[i * in_stride], n_in[i] = 1, base_pos[i], slot[i], *step_ctr = 0. */
+int ti_step_inputs(const int32_t* in, int n, int in_stride, int32_t* in_tokens, int32_t* n_in, int32_t* base_pos,
+                   int32_t* slot, int32_t* step_ctr, ti_stream_t s);
 
 /* ------------------------------------------------------- on-device sampling
  * InferenceEngine::sample_next_token (inference_engine.cpp:1554-1673) per stream, the uniform

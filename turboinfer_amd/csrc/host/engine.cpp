@@ -226,7 +226,19 @@ struct ti_engine {
     return std::max(1, std::min(sp, std::min(cap, 64)));
   }
 
+  // Device rows to the caller's (pageable) memory through page-locked pieces: the copies of the next pieces run while
+  // the host moves this one out (logits_out).  One engine's (pin_io).
+  static constexpr size_t out_piece = (size_t)1 << 20;
+  static constexpr int out_pieces = 8;
+  char* out_pin = nullptr;
+  int32_t* in_pin = nullptr;   // step_rows: tokens, positions, slots
+  hipEvent_t out_ev[out_pieces] = {};
+
   ~ti_engine() {
+    for (hipEvent_t v : out_ev)
+      if (v) hipEventDestroy(v);
+    if (out_pin) hipHostFree(out_pin);
+    if (in_pin) hipHostFree(in_pin);
     for (auto& g : graphs) hipGraphExecDestroy(g.second);
     for (void* p : allocs) hipFree(p);
     stack.reset();
@@ -382,21 +394,30 @@ bool part_usable(ti_engine* e, int M) {
 
 // The fused launch's bounded waits: after the stream's work, a set error word means a workgroup's q part or
 // new key never came (wrong results for that step) -- reported, and the exchange zeroed so the generations
-// agree again.  One 4-byte read on the engine's stream (synchronous).
+// agree again.  qa_fault_read puts the 8-byte read on the engine's stream (err: page-locked, or waited for at once).
 bool qa_usable(ti_engine* e, int M);
-int qa_fault_check(ti_engine* e) {
+int qa_fault_read(ti_engine* e, uint32_t* err) {
+  err[0] = err[1] = 0u;
   if (!e->qa_xchg || !qa_usable(e, 1)) return TI_OK;   // (only engines whose 1-stream steps take the launch)
   const ti_engine_config& c = e->c;
   const size_t off = ti_qkv_attn_error_offset(c.heads, e->splits_for(1));
   if (off + 8 > ti_qkv_attn_xchg_bytes(c.heads, TI_ATTN_MAX_PART_SPLITS))
     return ti_set_error(TI_ERR_ARG, "engine: exchange error word outside the buffer");
-  uint32_t err[2] = {0u, 0u};
-  TI_TRY(ti_memcpy_d2h(err, static_cast<char*>(e->qa_xchg) + off, sizeof(err), e->s));
+  E_CHECK(hipMemcpyAsync(err, static_cast<char*>(e->qa_xchg) + off, 8, hipMemcpyDeviceToHost, e->s), "hipMemcpyAsync(D2H)");
+  return TI_OK;
+}
+int qa_fault_report(ti_engine* e, const uint32_t* err) {
   if (!err[0] && !err[1]) return TI_OK;
-  TI_TRY(ti_memset(e->qa_xchg, 0, ti_qkv_attn_xchg_bytes(c.heads, TI_ATTN_MAX_PART_SPLITS), e->s));
+  TI_TRY(ti_memset(e->qa_xchg, 0, ti_qkv_attn_xchg_bytes(e->c.heads, TI_ATTN_MAX_PART_SPLITS), e->s));
   TI_TRY(ti_stream_sync(e->s));
   return ti_set_error(TI_ERR_HIP, "engine: the fused QKV + attention launch's exchange timed out (a workgroup's q "
                       "part or the new key never arrived); results of the last call are wrong, exchange reset");
+}
+int qa_fault_check(ti_engine* e) {
+  uint32_t err[2];
+  TI_TRY(qa_fault_read(e, err));
+  TI_TRY(ti_stream_sync(e->s));
+  return qa_fault_report(e, err);
 }
 
 // QKV + attention in one launch (ti_qkv_attn_partials): one stream with the fold and split partials,
@@ -459,6 +480,45 @@ int enqueue_head(ti_engine* e, int n, float* x) {
   el.out = e->logits;
   el.argmax = e->argmax;
   return gemm_rows(e, e->lm, n, x, TI_X_F32_RMSNORM, c.hidden, e->out_norm, el, 4, false);
+}
+
+// Page-locked memory of an engine's steps (at its creation: 2 ms).
+int pin_io(ti_engine* e) {
+  const ti_engine_config& c = e->c;
+  E_CHECK(hipHostMalloc(reinterpret_cast<void**>(&e->in_pin), (size_t)(3 * c.max_batch + 2) * 4, hipHostMallocDefault), "hipHostMalloc");
+  if ((size_t)c.max_batch * c.vocab * 4 <= e->out_piece * 3 / 2) return TI_OK;
+  E_CHECK(hipHostMalloc(reinterpret_cast<void**>(&e->out_pin), e->out_piece * e->out_pieces, hipHostMallocDefault), "hipHostMalloc");
+  memset(e->out_pin, 0, e->out_piece * e->out_pieces);   // (its pages are mapped at their first touch: here, not in a step)
+  for (hipEvent_t& v : e->out_ev) E_CHECK(hipEventCreateWithFlags(&v, hipEventDisableTiming), "hipEventCreate");
+  return TI_OK;
+}
+
+// Logits to the caller, after the stream's work.  Above 1.5 MiB and to ordinary memory in pieces of 1 MiB (measured, us,
+// one pageable hipMemcpyAsync / this: 2 MB 110 / 103, 3 MB 165 / 137, 8.2 MB 465 / 307, 16.4 MB 960 / 625; pieces of
+// 256 KiB 1222, of 4 MiB 660).
+int logits_out(ti_engine* e, float* dst, const float* src, size_t bytes) {
+  hipPointerAttribute_t at{};
+  if (bytes <= e->out_piece * 3 / 2) return ti_memcpy_d2h(dst, src, bytes, e->s);
+  if (hipPointerGetAttributes(&at, dst) != hipSuccess) (void)hipGetLastError();   // (not known to the runtime)
+  else if (at.type != hipMemoryTypeUnregistered) return ti_memcpy_d2h(dst, src, bytes, e->s);
+  if (!e->out_pin) return ti_memcpy_d2h(dst, src, bytes, e->s);
+  const int n = (int)((bytes + e->out_piece - 1) / e->out_piece);
+  auto piece = [&](int i) { return std::min(e->out_piece, bytes - (size_t)i * e->out_piece); };
+  auto start = [&](int i) -> int {
+    const int k = i % e->out_pieces;
+    E_CHECK(hipMemcpyAsync(e->out_pin + (size_t)k * e->out_piece, reinterpret_cast<const char*>(src) + (size_t)i * e->out_piece, piece(i),
+                          hipMemcpyDeviceToHost, e->s), "hipMemcpyAsync(D2H)");
+    E_CHECK(hipEventRecord(e->out_ev[k], e->s), "hipEventRecord");
+    return TI_OK;
+  };
+  for (int i = 0; i < std::min(n, e->out_pieces); ++i) TI_TRY(start(i));
+  for (int i = 0; i < n; ++i) {
+    const int k = i % e->out_pieces;
+    E_CHECK(hipEventSynchronize(e->out_ev[k]), "hipEventSynchronize");
+    memcpy(reinterpret_cast<char*>(dst) + (size_t)i * e->out_piece, e->out_pin + (size_t)k * e->out_piece, piece(i));
+    if (i + e->out_pieces < n) TI_TRY(start(i + e->out_pieces));
+  }
+  return TI_OK;
 }
 
 // Decode attention of M streams, q -> attn.
@@ -913,7 +973,7 @@ int ti_engine_create(const ti_engine_config* cfg, ti_engine** out) {
       (rc = e->alloc_t(&e->logits, (size_t)B * V)) ||
       (rc = e->alloc_t(&e->argmax, (size_t)R * TI_ARGMAX_SLOTS)) || (rc = e->alloc_t(&e->pos, (size_t)R)) ||
       (rc = e->alloc_t(&e->base_pos, (size_t)B)) || (rc = e->alloc_t(&e->step_ctr, (size_t)1)) ||
-      (rc = e->alloc_t(&e->n_in, (size_t)B)) || (rc = ensure_io(e, 8, 8)))
+      (rc = e->alloc_t(&e->n_in, (size_t)B)) || (rc = ensure_io(e, 8, 8)) || (rc = pin_io(e)))
     return fail(rc);
   if (hipStreamSynchronize(e->s) != hipSuccess) return fail(ti_check_hip(hipErrorUnknown, "hipStreamSynchronize"));
   *out = e;
@@ -972,6 +1032,7 @@ int ti_engine_create_stack(const ti_stack_config* cfg, const ti_stack_layer* lay
   TI_TRY(e->alloc_t(&e->row_slot, (size_t)B));
   if (e->stack->recurrent) e->state_pos.assign((size_t)B, 0);
   TI_TRY(ensure_io(e.get(), 8, 8));
+  TI_TRY(pin_io(e.get()));
   const std::vector<int32_t> ones((size_t)R, 1);
   TI_TRY(ti_memcpy_h2d(e->pf_ones, ones.data(), ones.size() * 4, e->s));
   TI_TRY(ti_stream_sync(e->s));
@@ -1030,7 +1091,7 @@ int ti_engine_prefill(ti_engine* e, int slot, const int32_t* tokens, int n, int 
       for (; k < B && w + k < n_want && want[w + k] < t0 + rows; ++k)
         TI_TRY(ti_memcpy_d2d(e->h_last + (size_t)k * H, e->h + (size_t)(want[w + k] - t0) * H, (size_t)H * 4, e->s));
       TI_TRY(enqueue_head(e, k, e->h_last));
-      TI_TRY(ti_memcpy_d2h(logits + (size_t)w * c.vocab, e->logits, (size_t)k * c.vocab * 4, e->s));
+      TI_TRY(logits_out(e, logits + (size_t)w * c.vocab, e->logits, (size_t)k * c.vocab * 4));
       w += k;
     }
   }
@@ -1325,7 +1386,7 @@ int ti_engine_generate(ti_engine* e, int n, const int32_t* prompts, const int32_
       out_tokens[(size_t)m * max_new + t] = tok;
     }
   }
-  if (last_logits) TI_TRY(ti_memcpy_d2h(last_logits, e->logits, (size_t)n * c.vocab * 4, e->s));
+  if (last_logits) TI_TRY(logits_out(e, last_logits, e->logits, (size_t)n * c.vocab * 4));
   if (n == 1) TI_TRY(qa_fault_check(e));
   return TI_OK;
 }
@@ -1728,22 +1789,32 @@ static int step_rows(ti_engine* e, int n, const int32_t* slots, const int32_t* t
     TI_TRY(state_at(e, slots ? slots[m] : m, pos[m]));
   }
   TI_TRY(ensure_io(e, 1, 1));
-  std::vector<int32_t> in((size_t)n * e->in_cap, 0), one(n, 1);
-  for (int m = 0; m < n; ++m) in[(size_t)m * e->in_cap] = tokens[m];
-  TI_TRY(ti_memcpy_h2d(e->in_tokens, in.data(), in.size() * 4, e->s));
-  TI_TRY(ti_memcpy_h2d(e->n_in, one.data(), (size_t)n * 4, e->s));
-  TI_TRY(ti_memcpy_h2d(e->base_pos, pos, (size_t)n * 4, e->s));
-  if (slots) TI_TRY(ti_memcpy_h2d(e->row_slot, slots, (size_t)n * 4, e->s));
-  TI_TRY(ti_memset(e->step_ctr, 0, 4, e->s));
-  e->slots_on = slots != nullptr;
-  const int rc = run_steps(e, n, 1, 1);
-  e->slots_on = false;
-  TI_TRY(rc);
+  // The step's inputs by one launch that reads them from page-locked memory, in place of four or five synchronous
+  // copies (the token rows' with the stride of the longest prompt so far).  Free again: the last step was waited for.
+  for (int m = 0; m < n; ++m) {
+    e->in_pin[m] = tokens[m];
+    e->in_pin[n + m] = pos[m];
+    if (slots) e->in_pin[2 * n + m] = slots[m];
+  }
+  int rc = ti_step_inputs(e->in_pin, n, e->in_cap, e->in_tokens, e->n_in, e->base_pos, slots ? e->row_slot : nullptr, e->step_ctr, e->s);
+  if (rc == TI_OK) {
+    e->slots_on = slots != nullptr;
+    rc = run_steps(e, n, 1, 1);
+    e->slots_on = false;
+  }
+  uint32_t* err = reinterpret_cast<uint32_t*>(e->in_pin + 3 * c.max_batch);
+  if (rc == TI_OK && n == 1) rc = qa_fault_read(e, err);
+  if (rc != TI_OK) {
+    (void)hipStreamSynchronize(e->s);
+    return rc;
+  }
   for (int m = 0; m < n; ++m) state_set(e, slots ? slots[m] : m, pos[m] + 1);
-  TI_TRY(ti_stream_sync(e->s));
-  if (logits) TI_TRY(ti_memcpy_d2h(logits, e->logits, (size_t)n * c.vocab * 4, e->s));
-  if (n == 1) TI_TRY(qa_fault_check(e));
-  return TI_OK;
+  rc = logits ? logits_out(e, logits, e->logits, (size_t)n * c.vocab * 4) : ti_stream_sync(e->s);
+  if (rc != TI_OK) {
+    (void)hipStreamSynchronize(e->s);
+    return rc;
+  }
+  return n == 1 ? qa_fault_report(e, err) : TI_OK;
 }
 
 int ti_engine_step(ti_engine* e, int n, const int32_t* tokens, const int32_t* pos, float* logits) {

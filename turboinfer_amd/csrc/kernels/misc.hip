@@ -347,6 +347,19 @@ __global__ __launch_bounds__(512) void hbm_read_kernel(const hbm_u32x4* src, siz
   if (acc == 0x9e3779b9u) sink[blockIdx.x] = acc;   // keeps the loads; practically never stores
 }
 
+// Inputs of one step of n rows from page-locked host memory in[3 n]: tokens, positions, slots.  Bound by one read
+// over the bus (~ 2 us); the copies and the fill it replaces took ~ 8 us each, waited for one by one.
+__global__ void step_inputs_kernel(const int32_t* in, int n, int in_stride, int32_t* in_tokens, int32_t* n_in, int32_t* base_pos,
+                                   int32_t* slot, int32_t* step_ctr) {
+  for (int i = threadIdx.x; i < n; i += blockDim.x) {
+    in_tokens[(size_t)i * in_stride] = in[i];
+    n_in[i] = 1;
+    base_pos[i] = in[n + i];
+    if (slot) slot[i] = in[2 * n + i];
+  }
+  if (threadIdx.x == 0) *step_ctr = 0;
+}
+
 }  // namespace ti
 
 extern "C" int ti_step_begin(const ti_step_args* a, ti_stream_t stream) {
@@ -368,6 +381,17 @@ extern "C" int ti_step_begin(const ti_step_args* a, ti_stream_t stream) {
   return TI_OK;
 }
 
+
+extern "C" int ti_step_inputs(const int32_t* in, int n, int in_stride, int32_t* in_tokens, int32_t* n_in, int32_t* base_pos,
+                              int32_t* slot, int32_t* step_ctr, ti_stream_t stream) {
+  using namespace ti;
+  if (!in || !in_tokens || !n_in || !base_pos || !step_ctr || n < 1 || in_stride < 1)
+    return ti_set_error(TI_ERR_ARG, "ti_step_inputs: bad arguments");
+  hipLaunchKernelGGL(step_inputs_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, in, n, in_stride, in_tokens, n_in, base_pos, slot,
+                     step_ctr);
+  TI_LAUNCH_CHECK("step_inputs_kernel");
+  return TI_OK;
+}
 
 extern "C" int ti_wsynth_device(uint64_t seed, uint32_t tensor_id, int K, int N_src, int N_total, int bits,
                                 int row_map, int row_offset, void* tiles, uint16_t* scales, ti_stream_t stream) {
