@@ -79,3 +79,23 @@ def test_grouped_tiles(ti, dtype, tile_rows, N, K):
         check(out[r], a[r], w[e], dtype, dtype == torch.bfloat16)
         first += c
     assert (out[M] == 7).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M", [5, 200])
+def test_gelu(ti, dtype, M):
+    """GELU (erf form) over both tails and its zeros, from a product with the identity: bf16 half a unit in the last
+    place of the exact value plus 4e-6 of it (the erfc fit's tail), fp32 the cancellation of 1 + erf, 2^-23 |z|."""
+    N = 512
+    z = torch.cat([torch.linspace(-9, 9, M * N - 6, device="cuda"), torch.tensor([0.0, -0.0, 1e-30, -1e-30, 60.0, -60.0], device="cuda")])
+    a = z[torch.randperm(M * N, device="cuda", generator=torch.Generator(device="cuda").manual_seed(0))].view(M, N).to(dtype)
+    vec = 8 if dtype == torch.bfloat16 else 4
+    w = torch.eye(N, device="cuda", dtype=dtype).view(-1, 16, N // (4 * vec), 4, vec).permute(0, 2, 3, 1, 4).contiguous()
+    out = torch.empty(M, N, device="cuda", dtype=dtype)
+    d = ti.DenseArgs(w=w.data_ptr(), a=a.data_ptr(), out=out.data_ptr(), lda=N, ldo=N, M=M, N=N, K=N, batch=1, epi=ti.DE_ACT, t_cols=N,
+                     act=2, act_cols=N, dtype=ti.DT_BF16 if dtype == torch.bfloat16 else ti.DT_F32)
+    call(ti, d)
+    zd = a.double()
+    ref = 0.5 * zd * torch.special.erfc(-zd / 2**0.5)
+    tol = (2.0**-8 + 4e-6) * ref.abs() + 1e-38 if dtype == torch.bfloat16 else 2.0**-23 * zd.abs() + 2.0**-22 * ref.abs() + 1e-38
+    assert (out.double() - ref).abs().le(tol).all()
