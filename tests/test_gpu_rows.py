@@ -206,3 +206,9 @@ def test_rows_refusals(ti):
         assert L.ti_gemm_rows(*a, C.byref(ep), None) != 0, (i, v)
     ep.kind, ep.fold_x = ti.EPI_RESID_F32, b.ptr
     assert L.ti_gemm_rows(*ok, C.byref(ep), None) != 0
+
+
+@pytest.mark.parametrize("M,K,N", [(300, 256, 11280), (129, 384, 22016), (1000, 128, 12304)])
+def test_rows_fp16_wide_blocks(ti, oracle, ws, M, K, N):
+    """fp16 outputs wide enough for 128 x 192 blocks: ragged last rows and columns."""
+    test_rows_store(ti, oracle, ws, 16, M, K, N)

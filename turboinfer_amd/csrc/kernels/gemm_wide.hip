@@ -132,7 +132,7 @@ __device__ __forceinline__ float wide_fold_share(const GemvArgs& a, int m, int p
 // to share a dequantised tile), small row counts and fp16 by what a CU takes in from the L2 (~ 45 KB/us), so a block
 // keeps 64 rows as soon as the call has them.  DMA straight to LDS leaves the registers to the accumulators; the
 // next stage's unpacking is interleaved with this one's MFMAs.  Measured, us (fused kernel in 16-row pieces / tile and
-// batched-rows kernels -> this one): int8 1000 rows 2048 -> 11264 784 -> 79, fp16 333 rows 2048 -> 11264 600 -> 52,
+// batched-rows kernels -> this one): int8 1000 rows 2048 -> 11264 784 -> 79, fp16 333 rows 2048 -> 11264 600 -> 34,
 // int4 64 rows 4096 -> 12288 29 -> 18.4, 11008 -> 4096 24 -> 17.6, 512 rows 4096 -> 22016 110 -> 104.
 //
 // Block of 16 TM WM rows x 16 TN WN columns per workgroup; wave (wm, wn) owns 16 TM rows x TN weight tiles.  A
@@ -461,7 +461,7 @@ static WideShape wide_shape(float alone, float full) {
 }
 constexpr int kWideShapes = 5;
 template <int F>
-static const WideShape* wide_shapes() {   // 64 x 384 (fp16, blocks of 32: none) | 64 x 128 (fp16: 128 x 128) | 64 x 64 | 32 x 64 | 16 x 64
+static const WideShape* wide_shapes() {   // 64 x 384 (fp16: 128 x 192, blocks of 32: none) | 64 x 128 (fp16: 128 x 128) | 64 x 64 | 32 x 64 | 16 x 64
   if constexpr (F == 4) {
     static const WideShape s[kWideShapes] = {wide_shape<F, 1, 8, 4, 3, 2>(1.25f, 1.53f), wide_shape<F, 1, 4, 4, 2, 2>(1.00f, 0.51f),
                                              wide_shape<F, 1, 4, 4, 1, 3>(0.42f, 0.345f), wide_shape<F, 1, 4, 2, 1, 3>(0.30f, 0.22f),
@@ -473,7 +473,8 @@ static const WideShape* wide_shapes() {   // 64 x 384 (fp16, blocks of 32: none)
                                              wide_shape<F, 1, 4, 1, 1, 3>(0.32f, 0.32f)};
     return s;
   } else if constexpr (F == 16) {
-    static const WideShape s[kWideShapes] = {{nullptr}, wide_shape<F, 2, 4, 4, 2, 2>(1.30f, 1.30f),
+    // (128 x 192 beside 128 x 128, us: 333 rows 2048 -> 11264 49 -> 34, one round instead of two; 1000 rows 81 -> 68)
+    static const WideShape s[kWideShapes] = {wide_shape<F, 2, 4, 4, 3, 2>(1.62f, 1.62f), wide_shape<F, 2, 4, 4, 2, 2>(1.30f, 1.30f),
                                              wide_shape<F, 1, 4, 4, 1, 3>(0.57f, 0.56f), wide_shape<F, 1, 4, 2, 1, 3>(0.60f, 0.64f),
                                              wide_shape<F, 1, 4, 1, 1, 3>(0.55f, 0.60f)};
     return s;
