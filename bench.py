@@ -419,6 +419,11 @@ def main() -> int:
     qa_on = B == 1 and hasattr(e, "set_qkv_attn") and e.set_qkv_attn(None)
     lib = T.lib()
 
+    # the engine's rule for GQA batches (ti_attn_decode_spread)
+    spread = B >= 2 and not args.attn_splits and nh // nkv in (4, 8) and \
+        B * nkv >= (32 if hd == 64 else 96 if nh // nkv == 4 else 2)
+    attn_kernel = "attn_spread_kernel" if spread else "attn_split_kernel"
+
     def class_kernel(name):
         N_, K_ = shapes[name]
         if B >= (9 if bits == 4 else 6):
@@ -464,7 +469,7 @@ def main() -> int:
         iso_us, by = e.time_kernel(w, B, L, args.kernel_reps)
         c = in_step[tag_of[name]]
         us = c["period"] / c["n"]
-        kname = "attn_split_kernel" if name == "attention" else class_kernel(name)
+        kname = attn_kernel if name == "attention" else class_kernel(name)
         if name == "qkv" and qa_on:   # the fused launch: the q / k / v weights and the K / V it attends over
             by += att_iso[1]
             iso_us += att_iso[0]      # (isolated: the two unfused launches, for comparison)
@@ -518,7 +523,7 @@ def main() -> int:
             "roofline": dict({"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                               "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
                               "traffic_source": traffic_src}, **dom),
-            "attention_roofline": ({"bound": "hbm", "kernel": "attn_split_kernel", "achieved": per["attention"]["GBps"],
+            "attention_roofline": ({"bound": "hbm", "kernel": attn_kernel, "achieved": per["attention"]["GBps"],
                                     "peak": HBM_PEAK_GBS, "unit": "GB/s",
                                     "frac": round(per["attention"]["GBps"] / HBM_PEAK_GBS, 4), "traffic": att_traffic,
                                     "share_of_step_bytes": round(layers * att_bytes / sb, 4)} if not qa_on else
