@@ -212,3 +212,82 @@ def test_rows_refusals(ti):
 def test_rows_fp16_wide_blocks(ti, oracle, ws, M, K, N):
     """fp16 outputs wide enough for 128 x 192 blocks: ragged last rows and columns."""
     test_rows_store(ti, oracle, ws, 16, M, K, N)
+
+
+@pytest.mark.parametrize("bits", [4, 8, 16, 4 | G32])
+@pytest.mark.parametrize("M", [6, 17, 33, 64])
+def test_rows_fold_range(ti, oracle, ws, bits, M):
+    """Rows whose h * w fp16 does not hold: past 65504 in a few columns or in all, or all of it in the subnormal steps.
+    Their sums are negative, and the consumer normalises them first.  Bound: fp16 inputs, half a unit in
+    the last place of every x (2^-11, or 2^-25 below the normal range), beside the fp32 sums."""
+    L, K, H, N = ti.lib(), 256, 1024, 208
+    rng = np.random.RandomState(M + bits)
+    to, so, wo = weight(ti, oracle, bits, K, H, rng)
+    t2, s2, w2 = weight(ti, oracle, bits, H, N, rng)
+    act = rng.standard_normal((M, K)).astype(f16)
+    h0 = rng.standard_normal((M, H)).astype(f32)
+    nw = (1 + 0.1 * rng.standard_normal(H)).astype(f32)
+    h0[1, [5, 700]] = 1e5, -3e5
+    h0[M - 1] *= 1e6
+    h0[2] *= 3e-7
+    act[2] = 0
+    h0[4], act[4] = 0, 0
+    bad = np.isin(np.arange(M), [1, 2, 4, M - 1])
+    n_ss = L.ti_gemm_rows_fold_partials(bits, M, H, K, WS)
+    hd, fx, ss, yd, nwd = dev(ti, h0), ti.DeviceBuffer(M * H * 2), ti.DeviceBuffer(n_ss * 64 * 4), ti.DeviceBuffer(M * N * 4), dev(ti, nw)
+    out = []
+    for _ in range(2):   # (the second call over rows that the first rewrote)
+        ti.check(L.ti_memcpy_h2d(hd.ptr, h0.ctypes.data_as(C.c_void_p), h0.nbytes, None))
+        ep = ti.Epilogue()
+        ep.kind, ep.ldo, ep.out = ti.EPI_RESID_F32, H, hd.ptr
+        ep.fold_w, ep.fold_x, ep.fold_ss = nwd.ptr, fx.ptr, ss.ptr
+        rows(ti, bits, to, so, dev(ti, act), M, H, K, ep, ws=ws)
+        np.testing.assert_array_equal(np.signbit(ss.download(f32, (n_ss, 64))[:, :M]).any(axis=0), bad)
+        h1 = hd.download(f32, (M, H)).astype(np.float64)
+        ep = ti.Epilogue()
+        ep.kind, ep.ldo, ep.out, ep.ss_in, ep.n_ss = ti.EPI_STORE_F32, N, yd.ptr, ss.ptr, n_ss
+        ep.splitk_ws, ep.splitk_bytes = ws.ptr, ws.nbytes
+        ti.check(L.ti_gemm_rows_folded(t2.ptr, s2.ptr, bits, fx.ptr, H, hd.ptr, nwd.ptr, 1e-5, M, N, H, C.byref(ep), None))
+        ti.sync()
+        out.append(yd.download(f32, (M, N)))
+    x = h1 / np.sqrt((h1**2).mean(axis=1) + 1e-5)[:, None] * nw
+    err = np.abs(out[0] - x @ w2.astype(np.float64))
+    assert np.all(err <= (2.0**-11 + H * 2.0**-24) * (np.abs(x) @ np.abs(w2)) + 2.0**-25 * np.abs(w2).sum(axis=0) + 1e-9)
+    np.testing.assert_array_equal(*out)
+
+
+@pytest.mark.parametrize("bits", [4, 8, 16, 4 | G32, 8 | G32])
+def test_step_with_large_residuals(ti, bits):
+    """An embedding whose product with the norm weight passes fp16's range: a step of 9 streams (batched fold) against the
+    same streams in steps of 5 and 4 (normalised first).  Both round the same fp16 inputs: 1e-2 of the largest logit."""
+    V, H, layers, heads, kv, hd, inter = 512, 256, 2, 4, 2, 64, 512
+    e = ti.Engine(V, H, layers, heads, kv, hd, inter, bits=bits, max_seq=32, max_batch=9)
+    rng = np.random.RandomState(bits)
+    if bits & G32:
+        for i in range(layers + 1):
+            for slot, K, N in [(ti.W_Q, H, heads * hd), (ti.W_K, H, kv * hd), (ti.W_V, H, kv * hd), (ti.W_O, heads * hd, H), (ti.W_GATE, H, inter),
+                               (ti.W_UP, H, inter), (ti.W_DOWN, inter, H)] if i < layers else [(ti.W_LM_HEAD, H, V)]:
+                q, d, _ = g32_weight(rng, K, N, bits & 15)
+                e.set_tensor_q(slot, i % layers if i < layers else 0, q, d)
+    else:
+        e.synth(5, 0.1)
+    emb = (0.02 * rng.standard_normal((V, H))).astype(f32)
+    emb[::3, 7] = 6e4
+    emb[1::3] *= 5e-5
+    nw = np.ones(H, f32)
+    nw[7] = 2
+    e.set_tensor(ti.E_EMBED, 0, emb)
+    for i in range(layers):
+        e.set_tensor(ti.V_ATTN_NORM, i, nw)
+        e.set_tensor(ti.V_FFN_NORM, i, nw)
+    e.set_tensor(ti.V_OUT_NORM, 0, nw)
+    tok = rng.randint(0, V, (3, 9)).astype(np.int32)
+    tok[0] = np.arange(9)
+    got = [e.step(t, np.full(9, i, np.int32)) for i, t in enumerate(tok)]
+    # streams 0 .. 4, then 5 .. 8 in slots 0 .. 3
+    ref = [[e.step(t[a:b], np.full(b - a, i, np.int32)) for i, t in enumerate(tok)] for a, b in ((0, 5), (5, 9))]
+    e.close()
+    for i in range(len(tok)):
+        r = np.concatenate([ref[0][i], ref[1][i]])
+        assert np.isfinite(got[i]).all() and np.isfinite(r).all()
+        assert np.abs(got[i] - r).max() <= 1e-2 * np.abs(r).max(), (i, np.abs(got[i] - r).max(axis=1), np.abs(r).max())

@@ -343,7 +343,9 @@ int gemm_rows(ti_engine* e, const DevLinear& W, int M, const void* x, int x_kind
     ep.splitk_ws = e->splitk_ws;
     ep.splitk_bytes = (int64_t)e->splitk_bytes;
     const void* xm = static_cast<const char*>(x) + (size_t)m0 * ldx * x_elem;
-    if (wide) TI_TRY(ti_gemm_rows(W.tiles, W.scales, c.bits, xm, ldx, c.eps, mm, W.N, W.K, &ep, e->s));
+    if (wide && ep.ss_in && nw)   // folded rows of the residual (one piece)
+      TI_TRY(ti_gemm_rows_folded(W.tiles, W.scales, c.bits, e->xn, ldx, e->h, nw, c.eps, mm, W.N, W.K, &ep, e->s));
+    else if (wide) TI_TRY(ti_gemm_rows(W.tiles, W.scales, c.bits, xm, ldx, c.eps, mm, W.N, W.K, &ep, e->s));
     else TI_TRY(ti_gemm_wq_a16(W.tiles, W.scales, c.bits, xm, x_kind, ldx, nw, c.eps, mm, W.N, W.K, &ep, e->s));
   }
   return TI_OK;
@@ -570,7 +572,8 @@ int enqueue_step(ti_engine* e, int M, int advance) {
   // fold (M == 1): every rms_norm input is handed over as fx + ss partials by its producer
   const bool fold = fold_usable(e, M), part = part_usable(e, M), qa = qa_usable(e, M);
   // batched fold (many-rows kernel, up to 64 rows): O / down write xn = fp16(h * next norm weight) and per-row
-  // sums of h^2; QKV (after layer 0), gate/up and the lm_head normalise behind their GEMM (ti_hip.h)
+  // sums of h^2; QKV (after layer 0), gate/up and the lm_head normalise behind their GEMM, rows past fp16's range
+  // before it (ti_hip.h)
   const bool bfold = !fold && bfold_usable(e, M);
   int bn_ss = 0;   // partials per row the last batched producer wrote (0: none yet, rms_norm prep)
   auto next_norm = [&](int l) -> const float* { return l < c.layers ? e->layer[l].attn_norm : e->out_norm; };
@@ -602,12 +605,11 @@ int enqueue_step(ti_engine* e, int M, int advance) {
       ep.ss_in = e->ss;
       ep.n_ss = n_ss;
     } else if (bfold && bn_ss > 0) {
-      x = e->xn;
-      xk = TI_X_F16;
-      ldx = H;
-      nw = nullptr;
       ep.ss_in = e->ss_rows;
       ep.n_ss = bn_ss;
+      x = e->xn;
+      xk = TI_X_F16;   // (nw stays: gemm_rows)
+      ldx = H;
     }
   };
 

@@ -20,7 +20,7 @@ struct GemvArgs {
   const u32x4* tiles;
   const uint16_t* scales;
   const void* x;
-  const float* norm_w;
+  const float* norm_w;         // (gemm_wide_kernel: of a folded input whose rows are at hand as epi.fold_w, or NULL)
   float eps;
   int32_t x_kind, ldx, M, N, K;
   ti_epilogue epi;
@@ -196,7 +196,7 @@ __device__ __forceinline__ float fold_share(const GemvArgs& a, int m, int part, 
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = b0 + j * P < a.epi.n_ss ? ss[(size_t)(b0 + j * P) * TI_FOLD_SS_ROWS] : 0.0f;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) t += v[j];
+    for (int j = 0; j < 8; ++j) t += fabsf(v[j]);   // (negative: ti_gemm_rows_folded; x is taken as it is here)
   }
   return t;
 }

@@ -48,10 +48,12 @@ struct WideCfg {
   static constexpr int kScaleDma = W::kScale == 0 ? 0 : (TN * W::kScale + 255) / 256 * (W::kAff ? 2 : 1);   // dword DMAs per wave
   static constexpr int kS = kWaves * kScaleDma * 256;
   static constexpr int kStage = kA + kW + kS;
-  // after the stream: rms per row | each wave's staging block | sums of h^2 per column-wave and row | ticket
+  // after the stream: rms per row | each wave's staging block | (sum of h^2, largest |h w|) per column-wave and row | ticket
   static constexpr int kEpiStg = kRows * 4, kEpiRed = kEpiStg + kWaves * 16 * TM * kTileEpiStride * 4;
-  static constexpr int kEpiFlag = kEpiRed + WN * kRows * 4, kEpi = kEpiFlag + 16;
+  static constexpr int kEpiFlag = kEpiRed + 2 * WN * kRows * 4, kEpi = kEpiFlag + 16;
   static constexpr int kLds = NS * kStage > kEpi ? NS * kStage : kEpi;
+  static constexpr bool kFold = kRows <= TI_FOLD_SS_ROWS;   // (every wave of these has all rows)
+  static_assert(!kFold || WM == 1, "a wave sees every row's rms");
   static constexpr int kDmaA = kRows / 4 / kWaves, kDmaW = kTiles * (W::kTile / 1024) / kWaves;
   static constexpr int kDma = kDmaA + kDmaW + kScaleDma;
   static_assert(kRows / 4 % kWaves == 0 && kTiles * (W::kTile / 1024) % kWaves == 0, "equal DMA counts per wave");
@@ -112,9 +114,11 @@ __device__ __forceinline__ bool wide_merge(const GemvArgs& a, f32x4 (&acc)[TN][T
   return true;
 }
 
-// Batched fold, consumer side: this thread's share of row m's partial sums of h^2 (part, part + P, ...), summed in order.
+// Batched fold, consumer side: this thread's share of row m's partial sums of h^2 (part, part + P, ...), summed in order;
+// negative if one of them is.
 __device__ __forceinline__ float wide_fold_share(const GemvArgs& a, int m, int part, int P) {
   float t = 0.0f;
+  uint32_t any = 0;
   if (m >= a.M) return t;
   const float* ss = a.epi.ss_in + m;
   for (int b0 = part; b0 < a.epi.n_ss; b0 += 16 * P) {
@@ -122,9 +126,51 @@ __device__ __forceinline__ float wide_fold_share(const GemvArgs& a, int m, int p
 #pragma unroll
     for (int j = 0; j < 16; ++j) v[j] = b0 + j * P < a.epi.n_ss ? ss[(size_t)(b0 + j * P) * TI_FOLD_SS_ROWS] : 0.0f;
 #pragma unroll
-    for (int j = 0; j < 16; ++j) t += v[j];
+    for (int j = 0; j < 16; ++j) {
+      t += fabsf(v[j]);
+      any |= __builtin_bit_cast(uint32_t, v[j]);
+    }
   }
-  return t;
+  return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, t) | (any & 0x80000000u));
+}
+// The threads' shares to the rms of every row, negative as they are (behind a barrier; one follows).
+template <int ROWS, int NW>
+__device__ __forceinline__ void wide_fold_rms(const GemvArgs& a, float share, int tid, float* rmsv) {
+  rmsv[ROWS + tid] = share;
+  lds_barrier();
+  if (tid < ROWS) {
+    float t = 0.0f;
+    uint32_t any = 0;
+    for (int p = 0; p < 64 * NW / ROWS; ++p) {
+      const float v = rmsv[ROWS + p * ROWS + tid];
+      t += fabsf(v);
+      any |= __builtin_bit_cast(uint32_t, v);
+    }
+    rmsv[tid] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, sqrtf(t / (float)a.K + a.eps)) | (any & 0x80000000u));
+  }
+  lds_barrier();
+}
+// The rows whose rms is negative as ti_rmsnorm_f16 gives them.  Every workgroup rewrites them whole, with the same values,
+// before it reads them.
+template <int ROWS, int NW>
+__device__ __forceinline__ void wide_refold(const GemvArgs& a, int wave, int lane, const float* rmsv) {
+  typedef f16 f16x4 __attribute__((ext_vector_type(4)));
+#pragma unroll 1
+  for (int m = wave; m < ROWS; m += NW) {   // (rows past M have a positive one)
+    const float rms = -rmsv[m];
+    if (__builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, rms)) < 0) continue;
+#pragma unroll 1
+    for (int k0 = 0; k0 < a.K; k0 += 4 * kWave) {   // (K is a multiple of 128: the upper lanes repeat the last piece)
+      const int k = min(k0 + 4 * lane, a.K - 4);
+      const f32x4 v = *(const f32x4*)(a.epi.fold_w + (size_t)m * a.K + k), w = *(const f32x4*)(a.norm_w + k);
+      f16x4 y;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) y[i] = mul_f16(v[i] / rms, w[i]);
+      *(f16x4*)((f16*)a.x + (size_t)m * a.ldx + k) = y;
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  lds_barrier();
 }
 
 // Bound: int4 and int8 by the vector unit beside the matrix cores (a 16x16x32 MFMA and its share of dequant and scale
@@ -308,7 +354,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const GemvAr
 #pragma unroll
   for (int s = 0; s < NS; ++s) issue(min(kb + s, ke - 1), s);
   // batched fold (decode rows, ti_hip.h TI_FOLD_SS_ROWS): this thread's share of its row's sum of squares
-  const bool fold_in = a.epi.ss_in != nullptr;
+  const bool fold_in = C::kFold && a.epi.ss_in != nullptr;
   const float share = fold_in ? wide_fold_share(a, m0 + tid % C::kRows, tid / C::kRows, 64 * NW / C::kRows) : 0.0f;
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * C::kDma) : "memory");
   lds_barrier();
@@ -347,41 +393,76 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const GemvAr
     stage(kg + 1, sg[1], sg[0]);
   }
   if (kg < nk) stage(kg, sg[0], sg[1]);
-  if constexpr (Fm::kBits != 16)   // what the last unit left
+  auto last = [&]() __attribute__((always_inline)) {   // what the last unit left
+    if constexpr (Fm::kBits != 16)
 #pragma unroll
-    for (int b = 0; b < TM; ++b) {
-      acc[TN - 1][b] = fma_scale4(pend, part[Fm::kG32 ? 1 : TN - 1][b], acc[TN - 1][b]);
-      if constexpr (Fm::kAff) acc[TN - 1][b] = fma_scale4(pm, xs[1][b], acc[TN - 1][b]);
-    }
+      for (int b = 0; b < TM; ++b) {
+        acc[TN - 1][b] = fma_scale4(pend, part[Fm::kG32 ? 1 : TN - 1][b], acc[TN - 1][b]);
+        if constexpr (Fm::kAff) acc[TN - 1][b] = fma_scale4(pm, xs[1][b], acc[TN - 1][b]);
+      }
+  };
+  last();
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the clamped stages past the end
   lds_barrier();
 
   float* rmsv = (float*)smem;
+  float rms[TM][4];
+#pragma unroll
+  for (int b = 0; b < TM; ++b)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) rms[b][i] = 1.0f;
   if (fold_in) {
-    ((float*)smem)[C::kRows + tid] = share;
-    lds_barrier();
-    if (tid < C::kRows) {
-      float t = 0.0f;
-      for (int p = 0; p < 64 * NW / C::kRows; ++p) t += ((float*)smem)[C::kRows + p * C::kRows + tid];
-      rmsv[tid] = sqrtf(t / (float)a.K + a.eps);
+    wide_fold_rms<C::kRows, NW>(a, share, tid, rmsv);
+    uint32_t any = 0;
+#pragma unroll
+    for (int b = 0; b < TM; ++b)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        rms[b][i] = rmsv[wm * 16 * TM + b * 16 + 4 * kq + i];
+        any |= __builtin_bit_cast(uint32_t, rms[b][i]);
+      }
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64((int32_t)any < 0) != 0, 0)) {
+      if (a.norm_w) {   // rows that fp16 did not hold: again, behind their rewriting, a stage at a time
+        wide_refold<C::kRows, NW>(a, wave, lane, rmsv);
+#pragma unroll
+        for (int t = 0; t < TN; ++t)
+#pragma unroll
+          for (int b = 0; b < TM; ++b) acc[t][b] = zero;
+        pend = pm = 0.0f;
+        if constexpr (Fm::kBits != 16)
+#pragma unroll
+          for (int b = 0; b < TM; ++b) part[Fm::kG32 ? 1 : TN - 1][b] = xs[Fm::kAff ? 1 : 0][b] = zero;
+#pragma unroll 1
+        for (int kg = kb; kg < ke; ++kg) {
+          issue(kg, 0);
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+          lds_barrier();
+          read_stage(sg[0], 0);
+          if constexpr (Fm::kBits != 16) bfn = deq(sg[0], 0, 0);
+          [&]<int... S>(std::integer_sequence<int, S...>) __attribute__((always_inline)) {
+            ((read_step(st[0], 0, S), mul(st[0], sg[0], sg[0], std::integral_constant<int, S>())), ...);
+          }(std::make_integer_sequence<int, 4>());
+          lds_barrier();
+        }
+        last();
+      }
+#pragma unroll
+      for (int b = 0; b < TM; ++b)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) rms[b][i] = rms[b][i] < 0.0f && a.norm_w ? 1.0f : fabsf(rms[b][i]);
     }
-    lds_barrier();
   }
   if (n_ks > 1 && !wide_merge<TN, TM>(a, acc, cb * n_rb + rb, n_cb * n_rb, NW, wave, ks, n_ks, lane, (int*)(smem + C::kEpiFlag))) {
     stamp_end(a.stamp, t_entry);
     return;
   }
   const ti_epilogue& e = a.epi;
-  const bool fold_out = e.kind == TI_EPI_RESID_F32 && e.fold_x != nullptr;
+  const bool fold_out = C::kFold && e.kind == TI_EPI_RESID_F32 && e.fold_x != nullptr;
   float* stg = (float*)(smem + C::kEpiStg) + wave * (16 * TM * kTileEpiStride);
   const int mb = m0 + wm * 16 * TM;
-  float rms[TM][4], hsq[TM];
+  float hsq[TM], top[TM];
 #pragma unroll
-  for (int b = 0; b < TM; ++b) {
-    hsq[b] = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) rms[b][i] = fold_in ? rmsv[wm * 16 * TM + b * 16 + 4 * kq + i] : 1.0f;
-  }
+  for (int b = 0; b < TM; ++b) hsq[b] = top[b] = 0.0f;
 #pragma unroll 1
   for (int t = 0; t < TN; ++t) {   // (rolled: the tile's accumulators by static selects, so acc stays in registers)
     const int tn = t0 + wn * TN + t;
@@ -410,8 +491,11 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const GemvAr
           float4* o = (float4*)((float*)e.out + (size_t)m * e.ldo + ng);
           const float4 h0 = *o, h = make_float4(h0.x + v.x, h0.y + v.y, h0.z + v.z, h0.w + v.w);
           *o = h;
-          auto f = [](float x, float y) { return (uint32_t)__builtin_bit_cast(uint16_t, mul_f16(x, y)); };
-          *(uint2*)(e.fold_x + (size_t)m * e.ldo + ng) = make_uint2(f(h.x, w.x) | (f(h.y, w.y) << 16), f(h.z, w.z) | (f(h.w, w.w) << 16));
+          float p[4] = {h.x * w.x, h.y * w.y, h.z * w.z, h.w * w.w};
+          // (largest |p|; as outputs the products are rounded on their own, as in mul_f16)
+          asm("v_max3_f32 %0, %0, |%1|, |%2|\n\tv_max3_f32 %0, %0, |%3|, |%4|" : "+v"(top[it]), "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]));
+          auto f = [](float v) { return (uint32_t)f2h(v); };
+          *(uint2*)(e.fold_x + (size_t)m * e.ldo + ng) = make_uint2(f(p[0]) | (f(p[1]) << 16), f(p[2]) | (f(p[3]) << 16));
           q = (h.x * h.x + h.y * h.y) + (h.z * h.z + h.w * h.w);
         }
         q += lane_xor<1>(q);
@@ -428,16 +512,23 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const GemvAr
     }
   }
   if (fold_out) {   // this column block's sum of h^2 per row, column-waves in order
-    float* red = (float*)(smem + C::kEpiRed);
-    if ((lane & 3) == 0)
+    float2* red = (float2*)(smem + C::kEpiRed);
 #pragma unroll
-      for (int it = 0; it < TM; ++it) red[wn * C::kRows + wm * 16 * TM + 16 * it + (lane >> 2)] = hsq[it];
+    for (int it = 0; it < TM; ++it) {
+      const float t2 = fmaxf(top[it], lane_xor<1>(top[it])), t4 = fmaxf(t2, lane_xor<2>(t2));
+      if ((lane & 3) == 0) red[wn * C::kRows + wm * 16 * TM + 16 * it + (lane >> 2)] = make_float2(hsq[it], t4);
+    }
     lds_barrier();
     if (tid < C::kRows && m0 + tid < a.M) {
-      float t = 0.0f;
+      float t = 0.0f, mx = 0.0f;
 #pragma unroll
-      for (int w = 0; w < WN; ++w) t += red[w * C::kRows + tid];
-      e.fold_ss[(size_t)cb * TI_FOLD_SS_ROWS + m0 + tid] = t;
+      for (int w = 0; w < WN; ++w) {
+        const float2 v = red[w * C::kRows + tid];
+        t += v.x;
+        mx = fmaxf(mx, v.y);
+      }
+      // negative where fp16(h w) is infinite, or all so small that its steps of 2^-24 are not far below 2^-12 of the largest
+      e.fold_ss[(size_t)cb * TI_FOLD_SS_ROWS + m0 + tid] = mx > 65504.0f || mx < 0x1p-10f ? -t : t;
     }
   }
   if (e.kind == TI_EPI_LOGITS_ARGMAX && e.step_ctr && cb == 0 && rb == 0 && tid == 0) *e.step_ctr += e.advance;
@@ -498,10 +589,11 @@ static const WideShape* wide_shapes_of(int fmt) {
   }
 }
 
-// The shape and split whose busiest CU is done first.  Rows per block: 16, 32 and 64 (128) as the call's rows need;
+// The shape and split whose busiest CU is done first.  Rows per block: 16, 32 and 64 (128; a fold's block has all rows in
+// every wave) as the call's rows need;
 // splits only into slices of at least 4 stages, whose blocks fit the workspace, and of at most two workgroups a CU
 // (the seam, measured: ~ 0.5 us + 0.65 us per MB of partial blocks).
-bool wide_plan(int fmt, int M, int N, int K, int cus, int64_t ws_bytes, WidePlan* p) {
+bool wide_plan(int fmt, int M, int N, int K, int cus, int64_t ws_bytes, bool fold, WidePlan* p) {
   const WideShape* sh = wide_shapes_of(fmt);
   if (!sh || M < 1 || M > TI_GEMM_MAX_ROWS || N < 16 || (N & 15) || K < 128 || (K & 127)) return false;
   const int NT = N >> 4, KT = K >> 7;
@@ -511,7 +603,7 @@ bool wide_plan(int fmt, int M, int N, int K, int cus, int64_t ws_bytes, WidePlan
   p->shape = -1;
   for (int i = 0; i < kWideShapes; ++i) {
     const WideShape& s = sh[i];
-    if (!s.fn || (s.rows < 64 && M > s.rows) || (s.rows >= 64 && M <= 32)) continue;
+    if (!s.fn || (s.rows < 64 && M > s.rows) || (s.rows >= 64 && M <= 32) || (fold && s.rows > TI_FOLD_SS_ROWS)) continue;
     const int n_cb = (NT + s.tiles - 1) / s.tiles, n_rb = (M + s.rows - 1) / s.rows;
     const long per_xcd = (long)((n_cb + 7) / 8) * n_rb;   // (launched: whole XCD rows)
     for (int ks = 1; ks <= 8; ks += ks < 4 ? 1 : 2) {
@@ -559,12 +651,12 @@ int wide_launch(int fmt, const WidePlan& p, const GemvArgs& a, hipStream_t strea
 
 extern "C" int ti_gemm_rows_fold_partials(int bits, int M, int N, int K, int64_t ws_bytes) {
   ti::WidePlan p;
-  if (M > TI_FOLD_SS_ROWS || !ti::wide_plan(bits, M, N, K, ti::gemm_cus(), ws_bytes, &p)) return 0;
+  if (M > TI_FOLD_SS_ROWS || !ti::wide_plan(bits, M, N, K, ti::gemm_cus(), ws_bytes, true, &p)) return 0;
   return p.n_cb;
 }
 
-extern "C" int ti_gemm_rows(const void* tiles, const uint16_t* scales, int bits, const void* x, int ldx, float eps, int M, int N,
-                            int K, const ti_epilogue* epi, ti_stream_t stream) {
+static int rows_impl(const void* tiles, const uint16_t* scales, int bits, const void* x, int ldx, const float* h, const float* norm_w,
+                     float eps, int M, int N, int K, const ti_epilogue* epi, ti_stream_t stream) {
   using namespace ti;
   if (!tiles || !x || !epi || !epi->out) return ti_set_error(TI_ERR_ARG, "ti_gemm_rows: null pointer");
   if (bits != 16 && !scales) return ti_set_error(TI_ERR_ARG, "ti_gemm_rows: scales required for bits %d", bits);
@@ -588,14 +680,32 @@ extern "C" int ti_gemm_rows(const void* tiles, const uint16_t* scales, int bits,
   a.K = K;
   a.epi = *epi;
   a.vec = epilogue_vec(*epi);
-  if (epi->kind == TI_EPI_RESID_F32 && epi->fold_x &&
+  const bool fold_out = epi->kind == TI_EPI_RESID_F32 && epi->fold_x;
+  if (fold_out &&
       (M > TI_FOLD_SS_ROWS || !epi->fold_w || !epi->fold_ss || epi->fold_packed || !a.vec))
     return ti_set_error(TI_ERR_ARG, "ti_gemm_rows: fold_x needs M <= %d, fold_w, fold_ss and 16-byte aligned rows", TI_FOLD_SS_ROWS);
   WidePlan p;
-  if (!wide_plan(bits, M, N, K, gemm_cus(), epi->splitk_ws ? epi->splitk_bytes : 0, &p))
+  if (h) {
+    if (!epi->ss_in || fold_out || !norm_w || (((uintptr_t)h | (uintptr_t)norm_w) & 15))
+      return ti_set_error(TI_ERR_ARG, "ti_gemm_rows_folded: ss_in, no fold_x, and 16-byte aligned h and norm_w");
+    a.norm_w = norm_w;
+    a.epi.fold_w = h;
+  }
+  if (!wide_plan(bits, M, N, K, gemm_cus(), epi->splitk_ws ? epi->splitk_bytes : 0, epi->ss_in || fold_out, &p))
     return ti_set_error(TI_ERR_UNSUPPORTED, "ti_gemm_rows: bits %d, M=%d N=%d K=%d", bits, M, N, K);
   const int rp = ti_gemm_prepare();   // no-op once this device is prepared
   if (rp != TI_OK) return rp;
   a.stamp = ti_stamp_next(STAMP_TILE, wide_workgroups(p));
   return wide_launch(bits, p, a, (hipStream_t)stream);
+}
+
+extern "C" int ti_gemm_rows(const void* tiles, const uint16_t* scales, int bits, const void* x, int ldx, float eps, int M, int N,
+                            int K, const ti_epilogue* epi, ti_stream_t stream) {
+  return rows_impl(tiles, scales, bits, x, ldx, nullptr, nullptr, eps, M, N, K, epi, stream);
+}
+
+extern "C" int ti_gemm_rows_folded(const void* tiles, const uint16_t* scales, int bits, uint16_t* x, int ldx, const float* h,
+                                   const float* norm_w, float eps, int M, int N, int K, const ti_epilogue* epi, ti_stream_t stream) {
+  if (!h) return ti_set_error(TI_ERR_ARG, "ti_gemm_rows_folded: null pointer");
+  return rows_impl(tiles, scales, bits, x, ldx, h, norm_w, eps, M, N, K, epi, stream);
 }

@@ -9,8 +9,9 @@ struct WidePlan {
   int n_cb, n_rb, n_ks;  // column blocks x row blocks x k-slices
   int rows, tiles;       // of a block
 };
-// fmt: the bits of ti_gemm_wq_a16.  False: not a call of this kernel (shape or format).
-bool wide_plan(int fmt, int M, int N, int K, int cus, int64_t ws_bytes, WidePlan* p);
+// fmt: the bits of ti_gemm_wq_a16.  fold: a call with a folded input or output.  False: not a call of this kernel (shape
+// or format).
+bool wide_plan(int fmt, int M, int N, int K, int cus, int64_t ws_bytes, bool fold, WidePlan* p);
 long wide_workgroups(const WidePlan& p);
 int wide_launch(int fmt, const WidePlan& p, const GemvArgs& a, hipStream_t s);
 int gemm_cus();       // CUs of the current device (gemv.hip)

@@ -1423,7 +1423,7 @@ extern "C" int ti_gemm_tile_plan(int bits, int M, int N, int K, int64_t ws_bytes
     return ti_set_error(TI_ERR_UNSUPPORTED, "ti_gemm_tile_plan: M=%d N=%d K=%d bits %d is not a tile-kernel call", M, N,
                         K, bits);
   ti::WidePlan p;
-  if (!ti::wide_plan(bits, M, N, K, query_cus(), ws_bytes, &p))
+  if (!ti::wide_plan(bits, M, N, K, query_cus(), ws_bytes, false, &p))
     return ti_set_error(TI_ERR_UNSUPPORTED, "ti_gemm_tile_plan: M=%d N=%d K=%d bits %d", M, N, K, bits);
   // eight waves: one 64 x 384 workgroup, or two of four waves (64 x 128 or 64 x 64 each) on neighbouring row blocks
   *wmr = p.tiles == 24 ? 1 : 2;
@@ -1490,7 +1490,7 @@ static int gemm_impl(const void* tiles, const uint16_t* scales, int bits, const 
   const int64_t ws_bytes = epi->splitk_ws ? epi->splitk_bytes : 0;
   WidePlan wp;
   const bool wide = bits == 4 && !aff && x_kind == TI_X_F16 && M > 16 && (g32 || M >= tile_rows() || wide_tile(bits, M, N)) &&
-                    rows_aligned(x, ldx) && wide_plan(bits | (g32 ? TI_BITS_G32 : 0), M, N, K, query_cus(), ws_bytes, &wp);
+                    rows_aligned(x, ldx) && wide_plan(bits | (g32 ? TI_BITS_G32 : 0), M, N, K, query_cus(), ws_bytes, epi->ss_in, &wp);
   int g32_rows = 16;   // rows per fused launch (its LDS image holds the x rows)
   while (g32 && g32_rows > 1 && !fused_fits(g32_rows, N, K, true, aff)) --g32_rows;
   if (g32 && (x_kind == TI_X_F16_PACKED || (!wide && !fused_fits(std::min(M, g32_rows), N, K, true, aff))))
@@ -1609,6 +1609,7 @@ static int gemm_impl(const void* tiles, const uint16_t* scales, int bits, const 
     a.stamp = ti_stamp_next(wide ? STAMP_TILE : rows ? STAMP_ROWS : batched ? STAMP_MB : STAMP_GEMV, wgs);
   }
   hipStream_t s = (hipStream_t)stream;
+  if (wide) a.norm_w = nullptr;
   if (wide) return wide_launch(bits | (g32 ? TI_BITS_G32 : 0), wp, a, s);
   if (rows) return launch_rows(a, rMB, rRG, ntl, grid, r_rb, lds, s);
   if (batched) return launch_mb(a, grid, ntl, lds, s);
