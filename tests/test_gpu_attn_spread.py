@@ -84,6 +84,47 @@ def test_queries_past_fp16(ti):
     assert np.abs(got - ref).max() <= 2.0**-11 * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("hd,G", [(64, 4), (64, 8), (128, 4), (128, 8)])
+@pytest.mark.parametrize("qscale", [0.01, 0.3, 1.0, 4.0])
+def test_error_of_the_fp32_rows(ti, hd, G, qscale):
+    """The segments' fp32 rows, merged in float64, against float64: no further off than ti_attn_decode's (fp32 throughout).
+    Both add the same terms in another order, so their errors over 10^4 values agree to the scatter of such sums: a
+    quarter, and a third where the scores' own roundings decide (|score| ~ 4)."""
+    lens, kvh, parts, splits = [1000, 1400, 700, 900, 1200, 450], 2, 32, 4
+    rng = np.random.default_rng(hd + G)
+    M, heads, S, L_ = len(lens), kvh * G, max(lens), ti.lib()
+    q = (rng.standard_normal((M, heads, hd)) * qscale).astype(np.float32)
+    k, v = (rng.standard_normal((M, kvh, S, hd)).astype(np.float16) for _ in range(2))
+    ref = reference(q, k, v, lens, G)
+    bufs = [dev(ti, x) for x in (q, k, v, np.array(lens, np.int32) - 1)]
+    a = (bufs[0].ptr, bufs[1].ptr, bufs[2].ptr, kvh * S * hd, S, bufs[3].ptr, M, heads, kvh, hd)
+    out, err = ti.DeviceBuffer(M * heads * hd * 2), []
+
+    def merged(rows):   # rows [parts][heads][hd + 4]: o, maximum, sum
+        f = np.exp(rows[..., hd] - rows[..., hd].max(axis=0))
+        return (rows[..., :hd] * f[..., None]).sum(axis=0) / (rows[..., hd + 1] * f).sum(axis=0)[..., None]
+
+    for spread in (False, True):
+        n = L_.ti_attn_spread_workspace_bytes(M, heads, hd, parts) if spread else L_.ti_attn_workspace_bytes(M, heads, hd, splits)
+        ws = ti.DeviceBuffer(n)
+        ws.zero()
+        ti.check((L_.ti_attn_decode_spread if spread else L_.ti_attn_decode)(*a, parts if spread else splits, ws.ptr, out.ptr, None))
+        ti.sync()
+        raw = ws.download(np.float32, (n // 4,)).astype(np.float64)
+        if spread:
+            rows = raw[n // 4 - (parts + M) * heads * (hd + 4):].reshape(parts + M, heads, hd + 4)
+            units = [-(-x // 32) for x in lens]
+            segs = [-(-u // max(12, -(-sum(units) // parts))) for u in units]
+            first = np.cumsum([0] + segs)
+            assert min(segs) > 1
+            got = np.stack([merged(rows[first[m]:first[m + 1]]) for m in range(M)])
+        else:
+            rows = raw[n // 4 - M * heads * splits * (hd + 4):].reshape(M, heads, splits, hd + 4)
+            got = np.stack([merged(rows[m].transpose(1, 0, 2)) for m in range(M)])
+        err.append(np.linalg.norm(got - ref) / np.linalg.norm(ref))
+    assert err[1] <= (1.25 if qscale < 4 else 1.35) * err[0], err
+
+
 def test_refusals(ti):
     f = ti.lib().ti_attn_decode_spread
     ok = [1, 1, 1, 8 * 64 * 64, 64, 1, 2, 32, 8, 64, 4, 1, 1, None]
