@@ -99,3 +99,33 @@ def test_gelu(ti, dtype, M):
     ref = 0.5 * zd * torch.special.erfc(-zd / 2**0.5)
     tol = (2.0**-8 + 4e-6) * ref.abs() + 1e-38 if dtype == torch.bfloat16 else 2.0**-23 * zd.abs() + 2.0**-22 * ref.abs() + 1e-38
     assert (out.double() - ref).abs().le(tol).all()
+
+
+@pytest.mark.parametrize("lo,hi", [(0.0, 0.3), (-0.3, 0.0), (0.3, 1.5), (-1.0, -0.3), (-3.0, -1.0)])
+def test_gelu_roundings(ti, lo, hi):
+    """GELU's error before the bf16 store, by how many outputs are not the nearest bf16 of the exact value: an error of e
+    (relative, mean) crosses a boundary of the 2^-8 .. 2^-9 steps for about e / 2^-8.5 of the values.  No more than 0.5 z (1
+    + erff) gives in fp32 (its roundings: half a unit of 1 + erff, of erff and of the two products), by three standard
+    deviations of the count.  z has all its 24 bits: a product of three bf16 parts with three identities."""
+    M, N = 4096, 512
+    g = torch.Generator(device="cuda").manual_seed(5)
+    z = torch.rand(M, N, device="cuda", generator=g) * (hi - lo) + lo
+    top = z.bfloat16()
+    mid = (z - top.float()).bfloat16()
+    a = torch.cat([top, mid, (z - top.float() - mid.float()).bfloat16()], 1)
+    z = a.double().view(M, 3, N).sum(1)
+    w = torch.eye(N, device="cuda", dtype=torch.bfloat16).repeat(1, 3).view(-1, 16, 3 * N // 32, 4, 8).permute(0, 2, 3, 1, 4).contiguous()
+    out = torch.empty(M, N, device="cuda", dtype=torch.bfloat16)
+    call(ti, ti.DenseArgs(w=w.data_ptr(), a=a.data_ptr(), out=out.data_ptr(), lda=3 * N, ldo=N, M=M, N=N, K=3 * N, batch=1, epi=ti.DE_ACT,
+                          t_cols=N, act=2, act_cols=N, dtype=ti.DT_BF16))
+    ref = 0.5 * z * torch.special.erfc(-z / 2**0.5)
+    zf = z.float()
+    assert (zf.double() == z).all()
+    fp32 = 0.5 * zf * (1 + torch.erf(zf * 0.70710678118654752))
+
+    def wrong(x):   # 64-bit distance to the stored value against half a step
+        step = torch.exp2(torch.floor(torch.log2(ref.abs().clamp_min(1e-30))) - 7)
+        return int(((x.double() - ref).abs() > 0.5 * step * (1 + 1e-9)).sum())
+
+    n32 = wrong(fp32.bfloat16())
+    assert wrong(out) <= n32 + 3 * (n32 + 1) ** 0.5, (wrong(out), n32)

@@ -23,31 +23,38 @@ __device__ __forceinline__ unsigned long long logit_key(float v, int n) {
   return ((unsigned long long)float_order_key(v) << 32) | (unsigned long long)(0xFFFFFFFFu - (uint32_t)n);
 }
 
-// GELU for 16-bit outputs: z (1 - E / 2) or z E / 2 with E = erfc(|z| / sqrt 2) = t 2^(P(t) - x^2 log2 e), t = 1 / (1 + x / 2);
-// P fitted to log2(erfcx(x) / t) over x 0 .. 16 (Chebyshev basis, reweighted towards equal errors).  Relative error
-// below 6e-7 for z > 0 and 3e-6 for -5 < z < 0, where 0.5 z (1 + erff) cancels to 5e-2; absolute 3.8e-7 against 4.5e-7.
-// ~ 20 instructions; erff's two branches, ~ 60, took a third of a 256-row block's time (1500 x 8192, K 2048, us:
-// 88 -> 75).
-__device__ __forceinline__ float gelu_erfc(float z) {
-  const float x = fabsf(z) * 0.70710678118654752f, t = __builtin_amdgcn_rcpf(fmaf(0.5f, x, 1.0f));
-  float p = 2.386054695e-01f;
-  p = fmaf(p, t, -1.141786098e+00f);
-  p = fmaf(p, t, 2.040967464e+00f);
-  p = fmaf(p, t, -1.494438052e+00f);
-  p = fmaf(p, t, 2.840158641e-01f);
-  p = fmaf(p, t, -2.070800960e-01f);
-  p = fmaf(p, t, 1.195044965e-01f);
-  p = fmaf(p, t, 5.436215997e-01f);
-  p = fmaf(p, t, 1.442320585e+00f);
-  p = fmaf(p, t, -1.825731039e+00f);
-  const float e = t * __builtin_amdgcn_exp2f(fmaf(-x, x * 1.44269504088896341f, p));
-  return z * (z >= 0.0f ? fmaf(-0.5f, e, 1.0f) : 0.5f * e);
+// GELU for 16-bit outputs, h = z / 2: |z| < 1: h + h erf, erf(z / sqrt 2) = z Q(z^2); beyond: z - h E or h E with E =
+// erfc(|z| / sqrt 2) = t 2^(P(t) - x^2 log2 e), t = 1 / (1 + x / 2) (the form of erfcc in Numerical Recipes, Press,
+// Teukolsky, Vetterling, Flannery), P fitted to log2(erfcx(x) / t) over x 0.7 .. 16 and Q over its range (Chebyshev bases,
+// reweighted towards equal errors).  Against float64 no further off than 0.5 z (1 + erff) in any part of the range
+// (relative, rms): |z| < 0.3 2.8e-8 against 4.2e-8, 0.3 .. 6 2.9e-8 against 4.0e-8, -1.4 .. -1 1.0e-7 against 1.4e-7,
+// -5 .. -3 3.5e-7 against 6.6e-3 (its cancellation).  ~ 28 instructions; erff's two branches, ~ 60 (1500 x 8192, K 2048, us:
+// 88 -> 78).
+__device__ __forceinline__ float gelu_erf(float z) {
+  const float h = 0.5f * z, w = z * z;
+  float q = 1.84936216e-04f;
+  q = fmaf(q, w, -2.33070040e-03f);
+  q = fmaf(q, w, 1.99283324e-02f);
+  q = fmaf(q, w, -1.32977456e-01f);
+  q = fmaf(q, w, 7.97884405e-01f);
+  const float t = __builtin_amdgcn_rcpf(fmaf(fabsf(z), 0.35355339059327376f, 1.0f));
+  float p = -3.10784221e-01f;
+  p = fmaf(p, t, 1.23818982e+00f);
+  p = fmaf(p, t, -1.68483531e+00f);
+  p = fmaf(p, t, 7.01514661e-01f);
+  p = fmaf(p, t, -1.47596598e-01f);
+  p = fmaf(p, t, 5.91505647e-01f);
+  p = fmaf(p, t, 1.43761384e+00f);
+  p = fmaf(p, t, -1.82553995e+00f);
+  const float e = t * __builtin_amdgcn_exp2f(fmaf(w, -0.72134752044448170f, p));
+  const float far = z >= 0.0f ? fmaf(-fminf(h, 1e38f), e, z) : h * e;   // (inf - inf * 0)
+  return w < 1.0f ? fmaf(h, z * q, h) : far;
 }
 
 template <class T>
 __device__ __forceinline__ float activate(int act, float z) {
   if (act == TI_ACT_GELU_ERF) {
-    if constexpr (sizeof(T) == 2) return gelu_erfc(z);
+    if constexpr (sizeof(T) == 2) return gelu_erf(z);
     else return 0.5f * z * (1.0f + erff(z * 0.70710678118654752f));
   }
   // (1 + tanh x) / 2 is the logistic function of 2 x
