@@ -377,3 +377,29 @@ def test_generate_stop_at_the_prefill_token(ti):
         d1, _ = e.counters()
         assert got == [ref[0]] + [-1] * (k - 1) and d1 == d0, (got, d1 - d0)
     e.close()
+
+
+@pytest.mark.parametrize("bits", [4, 8, 16])
+def test_engine_without_layers(ti, bits):
+    """A model of no layers (ti_engine_create takes it): embedding, final norm and lm_head, in steps of one and of nine
+    streams and as a prompt.  fp16 weights and inputs: fp32 sums of H terms, and half a unit in the last place of x."""
+    V, H, n = 512, 256, 9
+    rng = np.random.RandomState(bits)
+    e = ti.Engine(V, H, 0, 4, 2, 64, 512, bits=bits, max_seq=32, max_batch=n)
+    e.synth(5, 0.1)
+    emb, w = (rng.standard_normal((V, H)) * 0.02).astype(np.float16).astype(f32), (rng.standard_normal((H, V)) * 0.05).astype(np.float16).astype(f32)
+    e.set_tensor(ti.E_EMBED, 0, emb)
+    e.set_tensor(ti.W_LM_HEAD, 0, w)
+    e.set_tensor(ti.V_OUT_NORM, 0, np.ones(H, f32))
+    tok = rng.randint(0, V, n).astype(np.int32)
+    nine = e.step(tok, np.zeros(n, np.int32))
+    one = np.concatenate([e.step(tok[i : i + 1], np.zeros(1, np.int32)) for i in range(n)])
+    prompt = e.prefill(0, tok)
+    e.close()
+    x = emb[tok].astype(np.float64)
+    x /= np.sqrt((x * x).mean(axis=1, keepdims=True) + 1e-5)
+    bound = 2.0**-10 * (np.abs(x) @ np.abs(w))   # (twice that for quantised weights, whose magnitudes exceed w's a little)
+    np.testing.assert_array_less(np.abs(nine - one), bound * (1 if bits == 16 else 2))
+    np.testing.assert_array_less(np.abs(prompt.reshape(-1) - one[n - 1]), (bound * (1 if bits == 16 else 2))[n - 1])
+    if bits == 16:
+        np.testing.assert_array_less(np.abs(nine - x @ w), bound)

@@ -937,8 +937,8 @@ int ti_engine_create(const ti_engine_config* cfg, ti_engine** out) {
     e->splits_max = e->splits_for(1);
     // the many-rows kernel's byte offsets into a weight are 32 bits; wider ones keep the fused kernel's 16-row pieces
     e->wide_ok = true;
-    for (const DevLinear* w : {&e->layer[0].qkv, &e->layer[0].o, &e->layer[0].gu, &e->layer[0].down, &e->lm})
-      e->wide_ok = e->wide_ok && ti_gemm_rows_fold_partials(c.bits, TI_FOLD_SS_ROWS, w->N, w->K, 0) > 0;
+    const int shapes[][2] = {{H, qd + 2 * kvd}, {qd, H}, {H, 2 * I}, {I, H}, {H, V}};   // (a model may have no layers)
+    for (const auto& w : shapes) e->wide_ok = e->wide_ok && ti_gemm_rows_fold_partials(c.bits, TI_FOLD_SS_ROWS, w[1], w[0], 0) > 0;
     e->pf_rows = !e->wide_ok && (c.bits & ~TI_BITS_G32) != 4 ? 16 : TI_GEMM_MAX_ROWS;
     if ((c.bits & ~TI_BITS_G32) != 4) e->pf_rows = std::min(e->pf_rows, std::max(16, c.max_seq));
     e->rows_cap = std::max(B, e->pf_rows);
