@@ -199,7 +199,9 @@ int ti_engine_serve(ti_engine* e, int n_req, const int32_t* prompts, const int32
  * instead of one token per decode step.  Greedy streams whose prompts have one length (at least
  * 2 tokens) run the last token as a prefill row too, and their first token comes from the final
  * rms_norm + lm_head on that row (env TI_PREFILL_LOGITS=0: a decode step instead).
- * Default: TI_GEMM_MAX_ROWS (int4) or 16; 0 = off. */
+ * Default, and the most that is taken: TI_GEMM_MAX_ROWS for int4 (also blocks of 32); other formats
+ * TI_GEMM_MAX_ROWS or max(16, max_seq), whichever is less (16 with weights of 4 GiB and more);
+ * layer-stack models as the engine's buffers hold.  0 = off. */
 int ti_engine_set_prefill(ti_engine* e, int rows);
 
 /* Fused hand-offs of single-stream steps: (1) the folded rms_norm (ti_hip.h TI_X_F16_FOLDED):

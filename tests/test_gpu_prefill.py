@@ -91,3 +91,28 @@ def test_prefill_tile_chunk_vs_oracle(ti, oracle, rows, n):
     assert_greedy(got[0].tolist(), ref, ref_logits)
     assert_logits_close(lg[0], ref_logits[-1])
     e.close()
+
+
+@pytest.mark.parametrize("bits,max_seq", [(8, 300), (16, 300), (4 | 32 | 64, 300), (4, 300), (8, 8)])
+def test_chunk_rows_and_back(ti, bits, max_seq):
+    """The default chunk can be set again after a smaller one, and no larger one than the buffers hold."""
+    n = min(100, max_seq)
+    e = ti.Engine(512, 256, 2, 4, 2, 64, 512, bits=bits, max_seq=max_seq, max_batch=64)
+    if not bits & 32:
+        e.synth(3, 0.1)
+    tok = np.random.RandomState(bits).randint(0, 512, n).astype(np.int32)
+    default = 1024 if bits == 4 else max(16, max_seq)
+    out, chunks = [], []
+    for rows in (None, 16, 7, default):
+        if rows is not None:
+            e.set_prefill(rows)
+        before = e.counters()[1]
+        out.append(e.prefill(0, tok))
+        chunks.append(e.counters()[1] - before)
+    with pytest.raises(ti.TiError):
+        e.set_prefill(default + 1)
+    e.close()
+    assert chunks == [1, -(-n // 16), -(-n // 7), 1]
+    np.testing.assert_array_equal(out[0], out[3])
+    if not bits & 32:
+        np.testing.assert_allclose(out[1], out[0], rtol=0, atol=1e-2 * np.abs(out[0]).max())

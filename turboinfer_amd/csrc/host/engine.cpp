@@ -132,6 +132,7 @@ struct ti_engine {
   // prefill (forward_pass over prompt tokens): up to pf_rows prompt tokens of one stream run
   // as rows of the batched path, sharing that stream's KV cache (stride 0)
   int pf_rows = 0;             // 0 = off (prompts consumed one token per decode step)
+  int pf_cap = 0;              // the most: what pf_ones and pf_base hold (the default)
   int rows_cap = 0;            // R = max(max_batch, pf_rows): rows the step buffers hold
   int32_t* pf_ones = nullptr;  // [pf_rows] 1
   int32_t* pf_zero = nullptr;  // [1] 0
@@ -941,6 +942,7 @@ int ti_engine_create(const ti_engine_config* cfg, ti_engine** out) {
     for (const auto& w : shapes) e->wide_ok = e->wide_ok && ti_gemm_rows_fold_partials(c.bits, TI_FOLD_SS_ROWS, w[1], w[0], 0) > 0;
     e->pf_rows = !e->wide_ok && (c.bits & ~TI_BITS_G32) != 4 ? 16 : TI_GEMM_MAX_ROWS;
     if ((c.bits & ~TI_BITS_G32) != 4) e->pf_rows = std::min(e->pf_rows, std::max(16, c.max_seq));
+    e->pf_cap = e->pf_rows;
     e->rows_cap = std::max(B, e->pf_rows);
     const int R = e->rows_cap;
     if ((rc = e->alloc_t(&e->q, (size_t)R * qd)) || (rc = e->alloc_t(&e->attn, (size_t)R * qd)) ||
@@ -1777,7 +1779,7 @@ int ti_engine_counters(ti_engine* e, uint64_t* decode_steps, uint64_t* prefill_c
 }
 
 int ti_engine_set_prefill(ti_engine* e, int rows) {
-  if (!e || e->c.compat || rows < 0 || rows > e->rows_cap || (rows > 0 && (!e->stack && rows > ((e->c.bits & ~TI_BITS_G32) == 4 ? TI_GEMM_MAX_ROWS : 16))))
+  if (!e || e->c.compat || rows < 0 || rows > (e->stack ? e->rows_cap : e->pf_cap))
     return ti_set_error(TI_ERR_ARG, "ti_engine_set_prefill: rows %d", rows);
   DeviceScope bind_(e);
   e->pf_rows = rows;
