@@ -485,3 +485,28 @@ def test_batched_fold_refuses_other_kernels(ti):
     ep = ti.Epilogue()
     ep.kind, ep.ldo, ep.out, ep.ss_in, ep.n_ss = ti.EPI_STORE_F32, N, buf.ptr, buf.ptr, 4
     assert L.ti_gemm_wq_a16(td.ptr, sd.ptr, 4, buf.ptr, ti.X_F16, K, None, 1e-5, 100, N, K, C.byref(ep), None) != 0
+
+
+@pytest.mark.parametrize("M", [65, 66, 80, 81, 100, 129, 300])
+def test_packed_outputs_of_unaligned_rows(ti, M):
+    """int4 rows past 64 whose pitch is no multiple of 8 run in pieces, packed outputs too: the aligned call's numbers, to the
+    fp32 sums' order (2^-11 of an output's magnitude and K roundings of 2^-24).  Blocks of 32 stay without packed outputs."""
+    L, K, N = ti.lib(), 256, 512
+    rng = np.random.RandomState(M)
+    t, s = ti.wpack_host((rng.standard_normal((K, N)) * 0.05).astype(f32), 4)
+    td, sd = dev(ti, t), dev(ti, s)
+    x = rng.standard_normal((M, K)).astype(np.float16)
+    Mp, outs = (M + 15) // 16 * 16, []
+    for ldx, packed in ((K, 0), (K + 4, 1)):
+        xp = np.zeros((M, ldx), np.float16)
+        xp[:, :K] = x
+        xd, yd = dev(ti, xp), ti.DeviceBuffer(Mp * N * 2)
+        ep = ti.Epilogue()
+        ep.kind, ep.ldo, ep.out, ep.out_packed = ti.EPI_STORE_F16, N, yd.ptr, packed
+        ti.check(L.ti_gemm_wq_a16(td.ptr, sd.ptr, 4, xd.ptr, ti.X_F16, ldx, None, 1e-5, M, N, K, C.byref(ep), None))
+        ti.sync()
+        y = yd.download(np.uint16, Mp * N)
+        outs.append((ti.unpack_rows(y, M, N) if packed else y[: M * N].reshape(M, N)).view(np.float16).astype(np.float64))
+    mag = np.abs(x.astype(np.float64)) @ np.full((K, N), 0.2)
+    assert np.all(np.abs(outs[0] - outs[1]) <= 2.0**-10 * np.abs(outs[0]) + K * 2.0**-24 * mag)
+    assert L.ti_gemm_wq_a16(td.ptr, sd.ptr, 4 | 32, xd.ptr, ti.X_F16, K + 8, None, 1e-5, M, N, K, C.byref(ep), None) == 3

@@ -1486,10 +1486,10 @@ static int gemm_impl(const void* tiles, const uint16_t* scales, int bits, const 
   // int4 fp16 rows, row-major: the many-rows kernel (gemm_wide.hip) from 65 rows on and for wide outputs from 17 (the
   // batched-rows kernel below that: the packed and the row-major form of a call give the same bits), group-32 from 17,
   // where its 16-byte row pieces are aligned; affine blocks, int8 and fp16 weights run the fused kernel here
-  // (ti_gemm_rows: any format)
+  // (ti_gemm_rows: any format).  Blocks of 32 write no packed output
   const int64_t ws_bytes = epi->splitk_ws ? epi->splitk_bytes : 0;
   WidePlan wp;
-  const bool wide = bits == 4 && !aff && x_kind == TI_X_F16 && M > 16 && (g32 || M >= tile_rows() || wide_tile(bits, M, N)) &&
+  const bool wide = bits == 4 && !aff && x_kind == TI_X_F16 && M > 16 && (g32 ? !epi->out_packed : M >= tile_rows() || wide_tile(bits, M, N)) &&
                     rows_aligned(x, ldx) && wide_plan(bits | (g32 ? TI_BITS_G32 : 0), M, N, K, query_cus(), ws_bytes, epi->ss_in, &wp);
   int g32_rows = 16;   // rows per fused launch (its LDS image holds the x rows)
   while (g32 && g32_rows > 1 && !fused_fits(g32_rows, N, K, true, aff)) --g32_rows;
@@ -1535,12 +1535,13 @@ static int gemm_impl(const void* tiles, const uint16_t* scales, int bits, const 
   // pieces of rows: group-32 through the fused kernel; int4 rows past the batched-rows kernel that are not aligned
   const int piece = wide ? 0 : g32 && M > g32_rows ? g32_rows : !g32 && bits == 4 && x_kind == TI_X_F16 && M >= tile_rows() ? tile_rows() - 1 : 0;
   if (piece) {
-    if (x_kind == TI_X_ATTN_SPLITS || x_kind == TI_X_F16_FOLDED || epi->out_packed)
+    if (x_kind == TI_X_ATTN_SPLITS || x_kind == TI_X_F16_FOLDED || (epi->out_packed && g32))
       return ti_set_error(TI_ERR_UNSUPPORTED, "ti_gemm_wq_a16: rows in pieces need plain x rows");
     const size_t x_elem = x_kind == TI_X_F16 ? 2 : 4;
     const size_t out_elem = epi->kind == TI_EPI_STORE_F16 || epi->kind == TI_EPI_SILU_MUL_F16 ? 2 : 4;
-    for (int m0 = 0; m0 < M; m0 += piece) {
-      const int mm = std::min(piece, M - m0);
+    for (int m0 = 0, mm; m0 < M; m0 += mm) {
+      mm = std::min(piece, M - m0);
+      if (epi->out_packed && M - m0 > piece && M - m0 <= piece + 16) mm = piece - 16;   // (packed outputs need more than 16 rows)
       ti_epilogue ep = *epi;
       ep.out = static_cast<char*>(epi->out) + (size_t)m0 * epi->ldo * out_elem;
       if (ep.pos) ep.pos += m0;
@@ -1570,7 +1571,8 @@ static int gemm_impl(const void* tiles, const uint16_t* scales, int bits, const 
   int grid = 0, lds = 0, ntl = 0, rMB = 0, rRG = 0, r_rb = 1;
   const bool rows = !wide && batched && M > 16;
   if (wide) {
-    } else if (rows) {
+    // (its plan has the grid)
+  } else if (rows) {
     rows_plan(M, N, K, query_cus(), &rMB, &rRG, &r_rb, &grid, &ntl);   // grid: column groups
     lds = rows_lds_bytes(rRG * rMB, ntl, K);
   } else if (batched) {
