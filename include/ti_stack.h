@@ -98,6 +98,8 @@ typedef struct ti_dense_args {
 } ti_dense_args;
 int ti_dense(const ti_dense_args* a, ti_stream_t s);
 size_t ti_dense_args_bytes(void);
+/* Rows and columns of the tiles that an ungrouped F32, SWIGLU, ROPE or ACT call runs on (0 x 0: the kernel of few rows). */
+int ti_dense_tile(const ti_dense_args* a, int* rows, int* cols);
 
 /* ------------------------------------------------------------------- norms and residual
  * One row per workgroup:

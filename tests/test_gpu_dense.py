@@ -1,6 +1,7 @@
-"""Large tiles of the layer-stack products (ti_dense, dense_block_kernel) against float64: ragged rows and columns, short
-k, grouped tiles whose experts hold from 1 row to a whole tile.  Bound: K roundings of 2^-24 of the sum of magnitudes
-(fp32 accumulation), and half a unit in the last place of the stored type."""
+"""Large tiles of the layer-stack products (ti_dense, dense_block_kernel) against float64: the tiles that the dispatch picks
+(ti_dense_tile), ragged rows and columns, short k, the epilogues that run on them, grouped tiles whose experts hold from 1
+row to a whole tile.  Bound: K roundings of 2^-24 of the sum of magnitudes (fp32 accumulation), and half a unit in the last
+place of the stored type."""
 from __future__ import annotations
 
 import ctypes as C
@@ -34,22 +35,84 @@ def check(got, a, w, dtype, out16=False):
     assert (got.double() - ref).abs().le(tol).all()
 
 
-@pytest.mark.parametrize("M,N,K,dtype", [
-    (1100, 8712, 2048, torch.bfloat16),   # 256 x 256: last row tile 76 rows, last columns 8
-    (1281, 8193, 2048, torch.bfloat16),   # .. 1 row, 1 column
-    (700, 8708, 2048, torch.bfloat16),    # 128 x 256
-    (1100, 2051, 8192, torch.bfloat16),   # 128 x 128
-    (1100, 2051, 8256, torch.bfloat16),
-])
-def test_blocks(ti, M, N, K, dtype):
+def tile(ti, d):
+    rows, cols = C.c_int(0), C.c_int(0)
+    ti.check(ti.lib().ti_dense_tile(C.byref(d), C.byref(rows), C.byref(cols)))
+    return rows.value, cols.value
+
+
+BLOCKS = [   # a tile's shape, and a call that runs on it: last rows and columns ragged
+    ((256, 256), 1100, 8712, 2048, torch.bfloat16),   # last row tile 76 rows, last columns 8
+    ((256, 256), 1281, 8193, 2048, torch.bfloat16),   # .. 1 row, 1 column
+    ((128, 256), 700, 8708, 2048, torch.bfloat16),
+    ((128, 128), 1100, 2051, 8192, torch.bfloat16),
+    ((128, 128), 1100, 2051, 8256, torch.bfloat16),
+    ((256, 256), 1601, 8705, 2048, torch.float32),
+    ((128, 256), 2000, 4008, 512, torch.float32),
+]
+
+
+@pytest.mark.parametrize("shape,M,N,K,dtype", BLOCKS)
+def test_blocks(ti, shape, M, N, K, dtype):
     a, w, f = operands(M, N, K, dtype)
     ldo = N + 5
     out = torch.full((M + 1, ldo), 7.0, device="cuda")
     d = ti.DenseArgs(w=f.data_ptr(), a=a.data_ptr(), out=out.data_ptr(), lda=K, ldo=ldo, M=M, N=N, K=K, batch=1, epi=ti.DE_F32,
-                     dtype=ti.DT_BF16)
+                     dtype=ti.DT_BF16 if dtype == torch.bfloat16 else ti.DT_F32)
+    assert tile(ti, d) == shape
     call(ti, d)
     check(out[:M, :N], a, w[0], dtype)
     assert (out[M] == 7).all() and (out[:, N:] == 7).all()
+
+
+def swiglu(y):   # even columns gate, odd ones up
+    g, u = y[:, 0::2], y[:, 1::2]
+    return g * torch.sigmoid(g) * u
+
+
+def check_swiglu(got, a, w, dtype):
+    """|d silu| <= 1.1, so an output moves by the roundings of its two products, each times the other's size; and half a
+    unit in the last place of the stored type."""
+    y, mag = a.double() @ w.double().T, a.shape[1] * 2.0**-24 * (a.double().abs() @ w.double().abs().T)
+    ref = swiglu(y)
+    tol = 1.1 * mag[:, 0::2] * y[:, 1::2].abs() + mag[:, 1::2] * y[:, 0::2].abs() + (2.0**-8 if dtype == torch.bfloat16 else 2.0**-20) * ref.abs()
+    assert (got.double() - ref).abs().le(tol + 1e-9).all()
+
+
+@pytest.mark.parametrize("shape,M,N,K,dtype", [(s, m, n + n % 2, k, t) for s, m, n, k, t in BLOCKS])
+def test_swiglu_blocks(ti, shape, M, N, K, dtype):
+    a, w, f = operands(M, N, K, dtype)
+    out = torch.full((M + 1, N // 2), 7.0, device="cuda").to(dtype)
+    d = ti.DenseArgs(w=f.data_ptr(), a=a.data_ptr(), out=out.data_ptr(), lda=K, ldo=N // 2, M=M, N=N, K=K, batch=1, epi=ti.DE_SWIGLU,
+                     dtype=ti.DT_BF16 if dtype == torch.bfloat16 else ti.DT_F32)
+    assert tile(ti, d) == shape
+    call(ti, d)
+    check_swiglu(out[:M], a, w[0], dtype)
+    assert (out[M] == 7).all()
+
+
+@pytest.mark.parametrize("shape,M,N,K,dtype", [(s, m, (n + 31) // 32 * 32, k, t) for s, m, n, k, t in BLOCKS])
+def test_rotary_blocks(ti, shape, M, N, K, dtype):
+    """Rotary pairs of the last 16 of a head's 32 columns; bound: the pair's roundings of both products."""
+    a, w, f = operands(M, N, K, dtype)
+    pos = torch.randperm(M, device="cuda", generator=torch.Generator(device="cuda").manual_seed(2)).int()
+    ang = torch.arange(M, device="cuda")[:, None].double() * 100.0 ** (-torch.arange(8, device="cuda").double() / 8)
+    cs = torch.stack([ang.cos(), ang.sin()], -1).float().contiguous()
+    out = torch.full((M + 1, N), 7.0, device="cuda").to(dtype)
+    d = ti.DenseArgs(w=f.data_ptr(), a=a.data_ptr(), out=out.data_ptr(), lda=K, ldo=N, M=M, N=N, K=K, batch=1, epi=ti.DE_ROPE, head_w=32,
+                     rot_off=16, rope_cs=cs.data_ptr(), pos=pos.data_ptr(), dtype=ti.DT_BF16 if dtype == torch.bfloat16 else ti.DT_F32)
+    assert tile(ti, d) == shape
+    call(ti, d)
+    y, mag = a.double() @ w[0].double().T, K * 2.0**-24 * (a.double().abs() @ w[0].double().abs().T)
+    y, mag = y.view(M, -1, 32), mag.view(M, -1, 32)
+    c, s = (cs[pos.long()].double()[:, None, :, i] for i in (0, 1))
+    e, o = y[..., 16::2], y[..., 17::2]
+    ref, tol = y.clone(), mag.clone()
+    ref[..., 16::2], ref[..., 17::2] = e * c - o * s, o * c + e * s
+    tol[..., 16:] = (mag[..., 16::2] + mag[..., 17::2]).repeat_interleave(2, -1) + 2.0**-22 * (e.abs() + o.abs()).repeat_interleave(2, -1)
+    err = (out[:M].double().view(M, -1, 32) - ref).abs()
+    assert err.le(tol + (2.0**-8 if dtype == torch.bfloat16 else 2.0**-23) * ref.abs()).all()
+    assert (out[M] == 7).all()
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
@@ -77,6 +140,35 @@ def test_grouped_tiles(ti, dtype, tile_rows, N, K):
     for e, c in enumerate(counts):
         r = order[first:first + c].long()
         check(out[r], a[r], w[e], dtype, dtype == torch.bfloat16)
+        first += c
+    assert (out[M] == 7).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("tile_rows", [128, 256])
+@pytest.mark.parametrize("N,K", [(48, 64), (264, 128), (512, 192), (250, 448)])
+def test_grouped_swiglu(ti, dtype, tile_rows, N, K):
+    counts = [1, 16, 17, 0, 31, 64, 65, 96, 127, 128, 129, 192, 193, 255, 256, 257]
+    E, M = len(counts), sum(counts)
+    a, w, f = operands(M, N, K, dtype, E, 3)
+    order = torch.randperm(M, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1)).int()
+    tiles, first = [], 0
+    for e, c in enumerate(counts):
+        tiles += [(e, first + i, min(tile_rows, c - i), 0) for i in range(0, c, tile_rows)]
+        first += c
+    tl = torch.zeros(len(tiles) + 9, 4, dtype=torch.int32, device="cuda")
+    tl[:len(tiles)] = torch.tensor(tiles, dtype=torch.int32)
+    n = torch.tensor([len(tiles)], dtype=torch.int32, device="cuda")
+    out = torch.full((M + 1, N // 2), 7.0, device="cuda").to(dtype)
+    d = ti.DenseArgs(w=f.data_ptr(), w_batch=f[0].numel(), a=a.data_ptr(), out=out.data_ptr(), lda=K, ldo=N // 2, M=M, N=N, K=K, batch=1,
+                     epi=ti.DE_SWIGLU, dtype=ti.DT_BF16 if dtype == torch.bfloat16 else ti.DT_F32, tile_rows=tile_rows,
+                     max_tiles=len(tl), tiles=tl.data_ptr(), n_tiles=n.data_ptr(), rows_in=order.data_ptr(), rows_out=order.data_ptr(),
+                     row_div=1)
+    call(ti, d)
+    first = 0
+    for e, c in enumerate(counts):
+        r = order[first:first + c].long()
+        check_swiglu(out[r], a[r], w[e], dtype)
         first += c
     assert (out[M] == 7).all()
 

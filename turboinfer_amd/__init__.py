@@ -148,7 +148,7 @@ EXPORTED = [
     "ti_engine_describe", "ti_engine_prefill", "ti_engine_create_config", "ti_engine_step_slots",
     "ti_gqa_prep", "ti_gqa_block_elems", "ti_gqa_decode", "ti_gqa_prefill", "ti_gqa_splits", "ti_recurrent_prepare", "ti_conv",
     "ti_ssd_step", "ti_ssd_scan", "ti_ssd_norm", "ti_lru_scan", "ti_lru_step", "ti_lru_step_max_block", "ti_stack_kpad", "ti_stack_weight_bytes", "ti_stack_pack",
-    "ti_stack_convert", "ti_stack_fill", "ti_dense", "ti_dense_args_bytes", "ti_rownorm", "ti_rownorm_routes", "ti_route", "ti_route_max_tiles",
+    "ti_stack_convert", "ti_stack_fill", "ti_dense", "ti_dense_tile", "ti_dense_args_bytes", "ti_rownorm", "ti_rownorm_routes", "ti_route", "ti_route_max_tiles",
     "ti_latent_prep", "ti_latent_prepare", "ti_latent_attn_decode", "ti_latent_attn_splits", "ti_latent_attn_prefill", "ti_latent_attn_out",
 ]
 
@@ -296,6 +296,7 @@ def lib() -> C.CDLL:
             L.ti_stack_convert.argtypes = [vp, u64, i32, vp, vp]
             L.ti_stack_fill.argtypes = [u64, C.c_uint32, u64, f32, i32, vp, vp]
             L.ti_dense.argtypes = [C.POINTER(DenseArgs), vp]
+            L.ti_dense_tile.argtypes = [C.POINTER(DenseArgs), C.POINTER(i32), C.POINTER(i32)]
             L.ti_dense_args_bytes.restype = sz
             L.ti_rownorm.argtypes = [C.POINTER(RownormArgs), vp]
             L.ti_route.argtypes = [C.POINTER(RouteArgs), vp]

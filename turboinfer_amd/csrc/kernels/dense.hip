@@ -623,18 +623,21 @@ int skinny(const ti_dense_args& a, hipStream_t s) {
 
 // More rows: the tile whose rounds over the 256 CUs cost least: us of a launch and per round at K 2048, measured (bf16
 // M 100 .. 2048, N 1024 .. 8704, K 1024 .. 8192; fp32: the products decide, so the smallest tile that fills the chip).
-template <class T, int EPI>
-int tiled(const ti_dense_args& a, hipStream_t s) {
-  constexpr bool F = sizeof(T) == 4;
-  const int bm[6] = {256, 128, 128, 64, 64, 32}, bn[6] = {256, 256, 128, 256, 128, 128};
+constexpr int kTileM[6] = {256, 128, 128, 64, 64, 32}, kTileN[6] = {256, 256, 128, 256, 128, 128};
+inline int tile_of(const ti_dense_args& a) {
+  const bool F = a.dtype == TI_DT_F32;
   const float fix[6] = {12.f, 5.f, 5.5f, 2.5f, 2.f, 2.f};
   const float per[6] = {F ? 485.f : 56.f, F ? 250.f : 36.f, F ? 134.f : 24.f, F ? 130.f : 25.f, F ? 72.f : 15.f, F ? 37.f : 10.f};
   float c[6];
   for (int i = 0; i < 6; ++i) {
-    const long wgs = (long)((a.M + bm[i] - 1) / bm[i]) * ((a.N + bn[i] - 1) / bn[i]) * a.batch;
+    const long wgs = (long)((a.M + kTileM[i] - 1) / kTileM[i]) * ((a.N + kTileN[i] - 1) / kTileN[i]) * a.batch;
     c[i] = fix[i] + (float)((wgs + 255) / 256) * per[i] * (float)a.K * (1.f / 2048);
   }
-  switch (std::min_element(c, c + 6) - c) {
+  return (int)(std::min_element(c, c + 6) - c);
+}
+template <class T, int EPI>
+int tiled(const ti_dense_args& a, hipStream_t s) {
+  switch (tile_of(a)) {
     case 0: return launch_block<T, 2, 4, 8, 4, 5, EPI>(a, s);
     case 1: return launch_block<T, 2, 4, 4, 4, 5, EPI>(a, s);
     case 2: return launch_block<T, 2, 2, 4, 4, 5, EPI>(a, s);
@@ -651,9 +654,10 @@ int grouped(const ti_dense_args& a, hipStream_t s) {
   return launch_tile<T, 64, 256, 2, EPI>(a, s);
 }
 
+inline bool few_rows(const ti_dense_args& a) { return a.tile_rows == 1 || a.tile_rows == 16 || (!a.tile_rows && a.M <= 64); }
 template <class T>
 int dispatch_dense(const ti_dense_args& a, hipStream_t s) {
-  const bool few = a.tile_rows == 1 || a.tile_rows == 16 || (!a.tile_rows && a.M <= 64);
+  const bool few = few_rows(a);
   switch (a.epi) {
     case TI_DE_F32: return few ? skinny<T, TI_DE_F32>(a, s) : tiled<T, TI_DE_F32>(a, s);
     case TI_DE_ROPE: return few ? skinny<T, TI_DE_ROPE>(a, s) : tiled<T, TI_DE_ROPE>(a, s);
@@ -738,6 +742,16 @@ extern "C" int ti_stack_convert(const float* src, uint64_t n, int dtype, void* d
 }
 
 extern "C" size_t ti_dense_args_bytes(void) { return sizeof(ti_dense_args); }
+
+extern "C" int ti_dense_tile(const ti_dense_args* a, int* rows, int* cols) {
+  using namespace ti;
+  if (!a || !rows || !cols || a->M < 1 || a->N < 1 || a->K < 1 || a->batch < 1 ||
+      (a->epi != TI_DE_F32 && a->epi != TI_DE_SWIGLU && a->epi != TI_DE_ROPE && a->epi != TI_DE_ACT) || a->tile_rows)
+    return ti_set_error(TI_ERR_ARG, "ti_dense_tile: bad arguments");
+  *rows = few_rows(*a) ? 0 : kTileM[tile_of(*a)];
+  *cols = few_rows(*a) ? 0 : kTileN[tile_of(*a)];
+  return TI_OK;
+}
 
 extern "C" int ti_dense(const ti_dense_args* a, ti_stream_t stream) {
   using namespace ti;
