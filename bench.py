@@ -414,12 +414,13 @@ def main() -> int:
     shapes = {"qkv": (nh * hd + 2 * nkv * hd, H), "o": (H, nh * hd), "gate_up": (2 * I, H), "down": (H, I),
               "lm_head": (V, H)}
     fold_on = B == 1 and e.set_fold(None)
-    # one stream of a GQA head_dim-64 model: QKV and the attention run as ONE launch (ti_qkv_attn_partials,
-    # DESIGN 4.19); its class "qkv" then carries the attention's bytes too and there is no attention class
+    # one stream of a GQA head_dim-64 model: QKV and the attention run as ONE launch (ti_qkv_attn_partials);
+    # its class "qkv" then carries the attention's bytes too and there is no attention class
     qa_on = B == 1 and hasattr(e, "set_qkv_attn") and e.set_qkv_attn(None)
     lib = T.lib()
 
-    # the engine's rule for GQA batches (ti_attn_decode_spread)
+    # the engine's rule for GQA batches (ti_attn_decode_spread), repeated here to name the class's kernel, as is
+    # rows_wide's line in class_kernel
     spread = B >= 2 and not args.attn_splits and nh // nkv in (4, 8) and \
         B * nkv >= (32 if hd == 64 else 96 if nh // nkv == 4 else 2)
     attn_kernel = "attn_spread_kernel" if spread else "attn_split_kernel"

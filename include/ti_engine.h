@@ -240,7 +240,7 @@ int ti_engine_sync(ti_engine* e);
 /* tokens decided by the last replay step, [n_streams] */
 int ti_engine_last_tokens(ti_engine* e, int n_streams, int32_t* tokens);
 
-/* In-step launch timing (bench.py's roofline, DESIGN 5; not a reference interface -- the reference
+/* In-step launch timing (bench.py's roofline; not a reference interface -- the reference
  * times wall clock only, benchmarks/benchmark_inference.cpp:309-384).  The replay step graph
  * (ti_engine_replay_prepare) is captured again with every decode kernel writing, per workgroup,
  * s_memrealtime stamps (100 MHz) of wave 0's entry and of each wave's end into an engine-owned

@@ -160,7 +160,8 @@ int ti_fill_kv_uniform(uint64_t seed, uint32_t tensor_id, int n, int kv_heads, i
 enum ti_x_kind { TI_X_F16 = 0, TI_X_F32 = 1, TI_X_F32_RMSNORM = 2, TI_X_F16_FOLDED = 3, TI_X_ATTN_SPLITS = 4,
                  TI_X_F16_PACKED = 5 };
 /* TI_X_F16_PACKED: fp16 rows in the batched-rows kernel's fragment order, so every load of its
- * MFMA operands is one contiguous KiB per wave (bits 4).  Element (m, k) of an M x K operand
+ * MFMA operands is one contiguous KiB per wave (bits 4); for callers of these functions (ti_engine's
+ * rows are row-major, for ti_gemm_rows).  Element (m, k) of an M x K operand
  * (K % 128 == 0) sits at TI_PACKED_INDEX(m, k, K / 128); the buffer holds ceil(M / 16) * 16
  * rows (16-row blocks of 16 * K elements, block b at b * 16 * K).  Producers: ti_rmsnorm_f16_packed,
  * ti_attn_decode_packed, and the batched epilogues TI_EPI_STORE_F16 / TI_EPI_SILU_MUL_F16 with
@@ -220,7 +221,7 @@ typedef struct ti_epilogue {
   /* TI_EPI_STORE_F16 / TI_EPI_SILU_MUL_F16 of the batched-rows kernels (M > 16 or packed x):
    * write the fp16 output in TI_X_F16_PACKED order (K = ldo, ldo % 128 == 0) */
   int32_t out_packed;
-  /* Split-K workspace of the tile GEMM (int4 fp16 rows from TI_GEMM_TILE_ROWS on): device memory
+  /* Split-K workspace of the many-rows GEMM (ti_gemm_rows, ti_gemm_wq_a16's int4 fp16 rows from 65 on): device memory
    * of splitk_bytes bytes whose first TI_SPLITK_TICKET_BYTES the owner zeroes once (every launch
    * leaves them zeroed); the fp32 partial blocks follow.  With it, narrow outputs split K over
    * workgroups to fill the chip (ti_gemm_tile_plan); NULL = no split.  One launch at a time per
@@ -243,21 +244,21 @@ int ti_gemm_lds_bytes(int M, int N, int K);
  * Two kernels: the fused one (rms_norm prologue, any bits) takes up to 16 rows while its LDS
  * image fits; for bits 4 with TI_X_F16 rows the batched-rows kernel takes up to
  * TI_GEMM_MAX_ROWS rows at any K (batched decode, generate_batch inference_engine.cpp:804-828)
- * and is used above 2 rows (a fixed crossover, DESIGN 4.5).  An int4 caller with more rows
+ * and is used above 2 rows (a fixed crossover).  An int4 caller with more rows
  * than this returns for TI_X_F32_RMSNORM should normalise them with ti_rmsnorm_f16 and pass
  * TI_X_F16 rows.  0 = shape unsupported. */
 #define TI_GEMM_MAX_ROWS 1024
 int ti_gemm_max_rows(int bits, int x_kind, int N, int K);
-/* 1 when M rows of an int4 GEMM go to the batched-rows kernel (17 .. 64 rows): its fp16
- * operands are best given as TI_X_F16_PACKED.  From 65 rows (TI_GEMM_TILE_ROWS, env, <= 65) on
- * the LDS-tiled kernel takes TI_X_F16 rows. */
+/* 1 when M rows of an int4 ti_gemm_wq_a16 call go to the batched-rows kernel (17 .. 64 rows): its
+ * fp16 operands are best given as TI_X_F16_PACKED.  From 65 rows on the many-rows kernel
+ * (ti_gemm_rows) takes TI_X_F16 rows. */
 int ti_gemm_packed_rows(int bits, int M);
-/* The same for one M x N x K call: 0 also where 17..64 int4 rows of a wide output take the tile
- * GEMM (rows x N >= TI_GEMM_TILE_WIDE_MN, env, default 850000), which needs TI_X_F16 rows. */
+/* The same for one M x N x K call: 0 also where 17..64 int4 rows of a wide output take the many-rows
+ * kernel (rows x N >= 850000, or N >= 16384 at 17..32 rows), which needs TI_X_F16 rows. */
 int ti_gemm_packed_rows_for(int bits, int M, int N, int K);
 /* The many-rows GEMM's plan for an int4 (bits 4 or 4 | TI_BITS_G32) M x N x K call with a split-K
  * workspace of ws_bytes (0 = none), for eight waves (one workgroup or two): row-waves, weight tiles
- * per wave and k-slices (1 = no split, TI_GEMM_SPLITK=0 never).  TI_ERR_UNSUPPORTED when the call would not take the tile kernel. */
+ * per wave and k-slices (1 = no split, TI_GEMM_SPLITK=0 never).  TI_ERR_UNSUPPORTED when the call would not take it. */
 int ti_gemm_tile_plan(int bits, int M, int N, int K, int64_t ws_bytes, int* wmr, int* tpw, int* n_ks);
 /* y[m][0:K] = fp16(rms_norm(x[m][0:K]) * w), tensor_engine.cpp:1452-1508 (the batched path's
  * activation prep; the same arithmetic as the fused TI_X_F32_RMSNORM prologue). */
@@ -397,10 +398,9 @@ int ti_gemm_kernel_name(int bits, int x_kind, int M, int N, int K, char* buf, in
  * the box it ran on. */
 int ti_hbm_calibrate(size_t bytes, int reps, double* read_gbps, double* copy_gbps, ti_stream_t s);
 
-/* (Round 5: the persistent decode launch ti_pds_decode, its ti_pds_args / ti_pds_layer structs,
- * ti_pds_supported and ti_pds_granule_words were removed -- the per-layer launches beat it at every
- * shape; the ti_engine_set_pds / _pds_error / _pds_timestamps stubs left in round 6,
- * INTEGRATION.md 3.) */
+/* (The persistent decode launch ti_pds_decode, its ti_pds_args / ti_pds_layer structs,
+ * ti_pds_supported, ti_pds_granule_words and the ti_engine_set_pds / _pds_error / _pds_timestamps
+ * entry points were removed: the per-layer launches beat it at every shape.) */
 
 /* ------------------------------------------------------- step begin (device loop)
  * One block per stream: picks the token of this step (prompt token while step < n_in[m],

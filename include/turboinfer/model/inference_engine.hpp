@@ -13,8 +13,7 @@
 // fp16 KV cache in HBM, the whole decode step captured in a hipGraph.  Greedy requests
 // (top_k == 1) run their token loop on the device; other sampling settings and logprobs
 // take the logits to the host each step unless the device sampler runs them.  Prompts are
-// prefilled in chunks of up to 1024 rows through the tile GEMM and the MFMA causal attention
-// (DESIGN 4.6).
+// prefilled in chunks of up to 1024 rows through the tile GEMM and the MFMA causal attention.
 //
 // Binary layout: every public class has the reference's layout (InferenceConfig 48 bytes, the
 // engine's private members mirrored: tensor_engine_, impl_, the vocabulary maps), so a program

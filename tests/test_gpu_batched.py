@@ -116,7 +116,7 @@ def test_tile_three_tiles_per_wave(ti, oracle, M, K, N):
 def test_tile_32_row_waves(ti, oracle, M, K, N):
     """Wide outputs at <= 32 rows take the tile kernel with 32-row waves (half the activation
     block per group); ragged rows and tiles."""
-    L = ti.lib()   # the wide-output tile path (TI_GEMM_TILE_WIDE_MN), not the batched-rows kernel
+    L = ti.lib()   # the many-rows kernel's wide outputs, not the batched-rows kernel
     assert L.ti_gemm_packed_rows(4, M) == 1 and L.ti_gemm_packed_rows_for(4, M, N, K) == 0
     rng = np.random.RandomState(M + K)
     w = (rng.standard_normal((K, N)) * 0.03).astype(f32)

@@ -61,7 +61,7 @@ const core::Tensor* layer_tensor(const ModelData& m, size_t l, const char* hf, c
   return find(m, {a + hf, b + meta, b + hf});
 }
 
-// A ModelData read from a llama GGUF (ModelLoader::load, DESIGN 4.13) carries llama.cpp's
+// A ModelData read from a llama GGUF (ModelLoader::load) carries llama.cpp's
 // tensor names and [out][in] linear weights; the engine takes the reference's names and [in][out]
 // (ti_engine.h slots).  llama.cpp's q / k rows are already ordered for adjacent-pair RoPE, the
 // rotation apply_rope implements (tensor_engine.cpp:1602-1612), so only names and the transpose
@@ -418,7 +418,7 @@ class InferenceEngineImpl {
         const std::vector<float> v = api::to_f32(*up0);
         for (float x : v)
           if (x < -8.0f || x > 7.0f) bits = 8;
-      } else if (gguf_src && q0) {   // Q4_0 / Q4_1 / Q8_0 checkpoint: keep its blocks (DESIGN 4.13)
+      } else if (gguf_src && q0) {   // Q4_0 / Q4_1 / Q8_0 checkpoint: keep its blocks
         const size_t kvd = k0 ? k0->shape().total_size() / H : H;
         if (all_g32(m, L, H, H, kvd, I, V, 4 | TI_BITS_G32)) bits = 4 | TI_BITS_G32;
         else if (all_g32(m, L, H, H, kvd, I, V, 4 | TI_BITS_G32 | TI_BITS_AFF)) bits = 4 | TI_BITS_G32 | TI_BITS_AFF;
@@ -810,7 +810,7 @@ std::unique_ptr<InferenceEngine> create_engine(const std::string& model_path, co
 }
 
 // Reference inference_engine.cpp:2075-2082: build an engine from the checkpoint, then
-// generate(prompt) and decode().  The checkpoint loads (GGUF, DESIGN 4.13); the string prompt
+// generate(prompt) and decode().  The checkpoint loads (GGUF); the string prompt
 // needs the tokenizer, which is out of scope, so this throws from generate(std::string) rather
 // than returning text it cannot produce.
 std::string quick_generate(const std::string& model_path, const std::string& prompt, size_t max_tokens,

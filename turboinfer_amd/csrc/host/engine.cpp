@@ -114,8 +114,8 @@ struct ti_engine {
   bool part_on = true;         // TI_ATTN_PART=0 turns it off
   uint16_t* part_o = nullptr;  // [heads][TI_ATTN_MAX_PART_SPLITS][head_dim]
   float* part_ml = nullptr;    // [heads][TI_ATTN_MAX_PART_SPLITS][2]
-  // one stream (head_dim 64 GQA or head_dim 128 MHA): QKV and the attention in one launch (ti_qkv_attn_partials,
-  // DESIGN 4.19), O merging its splits (TI_X_ATTN_SPLITS); TI_QKV_ATTN=0 turns it off
+  // one stream (head_dim 64 GQA or head_dim 128 MHA): QKV and the attention in one launch (ti_qkv_attn_partials),
+  // O merging its splits (TI_X_ATTN_SPLITS); TI_QKV_ATTN=0 turns it off
   bool qa_on = true;
   void* qa_xchg = nullptr;     // the q exchange of ti_qkv_attn_partials (zeroed once, generations kept)
   // on-device sampling (ti_engine_generate_sampled): the step graph ends with ti_sample_step
@@ -192,7 +192,7 @@ struct ti_engine {
     return TI_OK;
   }
   // attention workgroups aimed at: one 8-wave workgroup per CU (128 / 256 / 512 measured 717 / 751 /
-  // 681 tok/s, DESIGN 4.2); GQA partials with 8 splits (DESIGN 4.16)
+  // 681 tok/s); GQA partials with 8 splits
   static constexpr int attn_target = 256;
   static constexpr int gqa_part_splits = 8;
   // Workgroups per kv-head of a GQA batch's attention on ti_attn_decode_spread (half the CUs: more of them merge longer
@@ -214,7 +214,7 @@ struct ti_engine {
     if (c.attn_splits > 0) return c.attn_splits;
     // one stream of a GQA model (>= 4 q-heads per kv-head) with a small cache per kv-head
     // (<= 1 MiB of K + V: TinyLlama at 2048): few long splits whose partials the O projection
-    // merges (part_usable), instead of 64+ short splits merged by a last arriver (DESIGN 4.16)
+    // merges (part_usable), instead of 64+ short splits merged by a last arriver
     // (attention run head by head: ti_attn_decode_partials' GQA expansion, heads x splits workgroups)
     if (M == 1 && gqa_part_splits >= 2 && part_on && c.heads >= 4 * c.kv_heads &&
         (size_t)c.max_seq * c.head_dim * 4 <= ((size_t)1 << 20))
@@ -303,9 +303,6 @@ int validate(const ti_engine_config& c) {
   return TI_OK;
 }
 
-// Rows of the batched-rows kernel (int4, M > 16) take their fp16 operands in fragment order
-// (TI_X_F16_PACKED): the rms_norm prep, the attention output and the SiLU*up output are written
-// that way, so every operand load of the kernel is one contiguous KiB per wave.
 // Rows whose projections run on the many-rows kernel (ti_gemm_rows).  From the rows where a layer's four launches
 // take less there, the rms_norm folded into them, than the fused kernel's (int8 / fp16: its rms_norm prologue and, from
 // 8 rows on, several launches for a long K) or the 3..16-row int4 kernel's beside two rms_norm launches.  Measured at

@@ -27,7 +27,7 @@ struct AttnArgs {
   int32_t out_kt;     // > 0: out in TI_X_F16_PACKED order with K / 128 = out_kt (ti_attn_decode_packed)
   // GQA run head by head (kv_heads here = heads, G = 1): workgroup head h reads the cache of kv-head
   // h >> kv_shift.  The G q-heads of a kv-head then stream its K/V from the L2 / MALL in parallel
-  // instead of one workgroup serving all of them (one stream, partials mode: DESIGN 4.16).
+  // instead of one workgroup serving all of them (one stream, partials mode).
   int32_t kv_shift;
   unsigned long long* stamp;   // in-step launch stamps (common.hpp stamp_end), NULL in product launches
 };

@@ -212,7 +212,7 @@ __host__ __device__ __forceinline__ size_t tile_index(int nt, int kt, int KT) {
 constexpr int kStampWords = 24;
 __device__ __forceinline__ unsigned long long stamp_now() { return __builtin_amdgcn_s_memrealtime(); }
 // Diagnostic builds (TI_STAMP_PHASES=1, never the product) also keep up to 6 phase marks of wave 0 in
-// words 9..14 (kernel-specific; gemv_wq_kernel: DESIGN 4.18).
+// words 9..14 (kernel-specific).
 #ifndef TI_STAMP_PHASES
 #define TI_STAMP_PHASES 0
 #endif

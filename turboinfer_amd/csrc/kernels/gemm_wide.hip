@@ -177,9 +177,11 @@ __device__ __forceinline__ void wide_refold(const GemvArgs& a, int wave, int lan
 // FMAs take ~ 0.87 (16 + 4 V) cycles with V vector instructions per MFMA: V 3 at 64 rows a wave, more with fewer rows
 // to share a dequantised tile), small row counts and fp16 by what a CU takes in from the L2 (~ 45 KB/us), so a block
 // keeps 64 rows as soon as the call has them.  DMA straight to LDS leaves the registers to the accumulators; the
-// next stage's unpacking is interleaved with this one's MFMAs.  Measured, us (fused kernel in 16-row pieces / tile and
-// batched-rows kernels -> this one): int8 1000 rows 2048 -> 11264 784 -> 79, fp16 333 rows 2048 -> 11264 600 -> 34,
-// int4 64 rows 4096 -> 12288 29 -> 18.4, 11008 -> 4096 24 -> 17.6, 512 rows 4096 -> 22016 110 -> 104.
+// next stage's unpacking is interleaved with this one's MFMAs.  Measured inside a pass, us (fused kernel in 16-row
+// pieces / tile and batched-rows kernels -> this one): int8 1000 rows 2048 -> 11264 63 x 22.8 -> 79, fp16 333 rows the
+// same 21 x 25.7 -> 33; int4 64 rows 4096 -> 12288 24.0 -> 23.1, 4096 -> 22016 32.6 -> 29.0, the mean of 4096 -> 4096 and
+// 11008 -> 4096 18.1 -> 17.2; int4 512 rows 4096 -> 12288 65.0 -> 62.4, 4096 -> 22016 113.6 -> 114.9 (1 % slower, the
+// layer's four together 0.8 % faster).
 //
 // Block of 16 TM WM rows x 16 TN WN columns per workgroup; wave (wm, wn) owns 16 TM rows x TN weight tiles.  A
 // stage is one 128-k group of the block: the rows' activations (chunks XOR-swizzled by row, tile_swz), the packed
@@ -564,7 +566,7 @@ static const WideShape* wide_shapes() {   // 64 x 384 (fp16: 128 x 192, blocks o
                                              wide_shape<F, 1, 4, 1, 1, 3>(0.32f, 0.32f)};
     return s;
   } else if constexpr (F == 16) {
-    // (128 x 192 beside 128 x 128, us: 333 rows 2048 -> 11264 49 -> 34, one round instead of two; 1000 rows 81 -> 68)
+    // (128 x 128 -> 128 x 192, us: 333 rows 2048 -> 11264 49 -> 33, one round instead of two; 1000 rows 81 -> 68)
     static const WideShape s[kWideShapes] = {wide_shape<F, 2, 4, 4, 3, 2>(1.62f, 1.62f), wide_shape<F, 2, 4, 4, 2, 2>(1.30f, 1.30f),
                                              wide_shape<F, 1, 4, 4, 1, 3>(0.57f, 0.56f), wide_shape<F, 1, 4, 2, 1, 3>(0.60f, 0.64f),
                                              wide_shape<F, 1, 4, 1, 1, 3>(0.55f, 0.60f)};

@@ -64,8 +64,8 @@ __device__ unsigned long long g_rows_ts[4096 * 8 * 8];   // [wg][wave][phase] (g
 #define ROWS_TS(k) do { } while (0)
 #endif
 
-// Workgroups per launch: one 8-wave workgroup per CU (a second workgroup per CU measured slower,
-// DESIGN 4.1), never more than there are 16-row tiles.
+// Workgroups per launch: one 8-wave workgroup per CU (a second workgroup per CU measured slower),
+// never more than there are 16-row tiles.
 
 __host__ __device__ inline int gemv_lds_bytes_tiles(int M, int K, int tiles_per_wg, bool g32 = false, bool aff = false);
 
@@ -1260,7 +1260,7 @@ __host__ inline int rows_grid(int MB, int N, int K, int num_cus, int* ntl_out, i
 // Rows per workgroup (16 RG MB): the fewest activation + weight bytes per workgroup over the
 // launch's rounds -- a workgroup streams its rows' activations (R K 2 bytes, L2) and its tiles'
 // weights (ntl 8 K bytes); narrow outputs (O, down) take 16-row blocks, wide ones all the rows.
-// TI_GEMM_ROWS_SPLIT=0 keeps all rows in one workgroup (A/B knob, DESIGN 9).
+// TI_GEMM_ROWS_SPLIT=0 keeps all rows in one workgroup (A/B knob).
 __host__ inline void rows_plan(int M, int N, int K, int cus, int* MB, int* RG, int* n_rb, int* n_cg, int* ntl) {
   rows_shape(M, MB, RG);   // all rows in one workgroup
   *n_rb = 1;

@@ -1,6 +1,5 @@
-// qkv_attn.hip -- one decode stream (TinyLlama-1.1B GQA head_dim 64, configs[1]; Llama-2-7B MHA head_dim 128,
-// configs[2]): the QKV projection and the attention over the cache in ONE launch (ti_qkv_attn_partials,
-// DESIGN 4.19), i.e. TransformerLayer::forward_incremental's q / k / v projections, RoPE, KV append and
+// qkv_attn.hip -- one decode stream (TinyLlama-1.1B GQA head_dim 64; Llama-2-7B MHA head_dim 128): the
+// QKV projection and the attention over the cache in ONE launch (ti_qkv_attn_partials), i.e. TransformerLayer::forward_incremental's q / k / v projections, RoPE, KV append and
 // compute_attention (inference_engine.cpp:203-279, 291-368; tensor_engine.cpp:1254-1388).
 //
 // Workgroup (head h, split s) = blockIdx (s + S h); S = splits workgroups per head.
