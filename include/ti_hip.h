@@ -205,7 +205,8 @@ typedef struct ti_epilogue {
   /* TI_X_F16_FOLDED input: n_ss partial sums of squares of the row at ss_in.
    * Batched fold (17..64 int4 rows, TI_X_F16 / TI_X_F16_PACKED x holding fp16(h * nw), ss_in
    * non-NULL): row m is normalised behind the GEMM, y[m] = (W . x[m]) / sqrt(sum over
-   * b < n_ss of ss_in[b * TI_FOLD_SS_ROWS + m] / K + eps) -- the batched-rows / tile kernels */
+   * b < n_ss of ss_in[b * TI_FOLD_SS_ROWS + m] / K + eps) -- the batched-rows /
+   * many-rows kernels (blocks of 32: many-rows only, x and its rows 16-byte aligned) */
   int32_t n_ss;
   const float* ss_in;
   /* TI_EPI_RESID_F32, M == 1, fold_x non-NULL: besides h, write fold_x[n] = fp16(h[n] * fold_w[n])
