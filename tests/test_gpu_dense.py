@@ -221,3 +221,40 @@ def test_gelu_roundings(ti, lo, hi):
 
     n32 = wrong(fp32.bfloat16())
     assert wrong(out) <= n32 + 3 * (n32 + 1) ** 0.5, (wrong(out), n32)
+
+
+# Tiles of few rows, their two groups of waves over k, and row tiles of 3/4 of a block: odd numbers of stages, fewer stages
+# than the ring holds, ragged last rows and columns.
+SPREAD = [
+    ((32, 64), 65, 70, 64, torch.bfloat16),        # one stage
+    ((32, 64), 97, 1001, 192, torch.bfloat16),     # three; last row tile 1 row
+    ((64, 64), 333, 2051, 1088, torch.bfloat16),
+    ((64, 128), 700, 2061, 2112, torch.bfloat16),  # 48 rows a tile
+    ((64, 128), 250, 6201, 1088, torch.bfloat16),  # 64
+    ((128, 128), 650, 4101, 320, torch.bfloat16),  # 96
+    ((128, 128), 1300, 2501, 1088, torch.bfloat16),
+    ((128, 128), 300, 8201, 320, torch.bfloat16),  # without the groups
+    ((128, 256), 2000, 2101, 320, torch.bfloat16),  # 96
+    ((32, 64), 97, 1001, 96, torch.float32),
+    ((64, 64), 333, 2051, 1056, torch.float32),
+    ((128, 128), 650, 4101, 352, torch.float32),
+]
+
+
+@pytest.mark.parametrize("epi", ["f32", "swiglu"])
+@pytest.mark.parametrize("shape,M,N,K,dtype", SPREAD)
+def test_small_tiles(ti, shape, M, N, K, dtype, epi):
+    N += epi == "swiglu" and N % 2
+    a, w, f = operands(M, N, K, dtype)
+    ldo = N + 5 if epi == "f32" else N // 2
+    out = torch.full((M + 1, ldo), 7.0, device="cuda").to(torch.float32 if epi == "f32" else dtype)
+    d = ti.DenseArgs(w=f.data_ptr(), a=a.data_ptr(), out=out.data_ptr(), lda=K, ldo=ldo, M=M, N=N, K=K, batch=1,
+                     epi=ti.DE_F32 if epi == "f32" else ti.DE_SWIGLU, dtype=ti.DT_BF16 if dtype == torch.bfloat16 else ti.DT_F32)
+    assert tile(ti, d) == shape
+    call(ti, d)
+    if epi == "f32":
+        check(out[:M, :N], a, w[0], dtype)
+        assert (out[:, N:] == 7).all()
+    else:
+        check_swiglu(out[:M], a, w[0], dtype)
+    assert (out[M] == 7).all()

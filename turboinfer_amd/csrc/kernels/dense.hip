@@ -6,11 +6,11 @@
 //   * dense_skinny_kernel (M <= 64): HBM-bound weight streaming.  One workgroup per 16 output columns,
 //     its waves split k; each weight fragment is one contiguous KiB read once and multiplied with up
 //     to 4 row tiles; the waves' partial sums meet in LDS.
-//   * dense_tile_kernel (more rows, tiles up to 64 x 256): 4 waves side by side over a BM x BN tile, activations
-//     staged through double-buffered LDS in fragment order, each wave's weight fragments straight from
-//     L2 into registers; both 2 or 4 k-stages (128 bytes each) ahead of their use.
-//   * dense_block_kernel (tiles of 128 x 128 up to 256 x 256): both operands copied to an LDS ring by DMA,
-//     4 stages ahead, waves in a WM x WN grid.
+//   * dense_block_kernel (more rows: tiles of 32 x 64 up to 256 x 256): both operands copied to an LDS ring by DMA,
+//     4 to 12 stages ahead, waves in a WM x WN grid, for the smaller tiles one such grid per half of k.
+//   * dense_tile_kernel (its 64-row tiles for grouped products and the epilogues of short or narrow products): 4 waves
+//     side by side over a BM x BN tile, activations staged through double-buffered LDS in fragment order, each wave's
+//     weight fragments straight from L2 into registers; both 2 or 4 k-stages (128 bytes each) ahead of their use.
 // All take independent batches (per-head products) or grouped tiles (experts: a tile is up to
 // tile_rows entries of one expert's list, rows gathered and scattered through the list).
 #include <algorithm>
@@ -446,136 +446,180 @@ __device__ __forceinline__ void wait_dma() {   // all but the wave's N newest ve
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-template <int WM, int WN, int FM, int FN, int NS>
+template <int KG, int WM, int WN, int FM, int FN, int NS>
 struct BlockCfg {
-  static constexpr int kWaves = WM * WN, BM = 16 * FM * WM, BN = 16 * FN * WN;
-  static constexpr int kFrags = FM * WM + FN * WN, kDma = kFrags / kWaves, kLds = NS * kFrags * 1024;
-  static_assert(kFrags % kWaves == 0 && kLds <= 160 * 1024 && NS >= 4 && FM % 4 == 0 && FN <= FM);
+  static constexpr int kWaves = KG * WM * WN, BM = 16 * FM * WM, BN = 16 * FN * WN;
+  static constexpr int kLds = NS * KG * (FM * WM + FN * WN) * 1024;
+  static constexpr bool kBig = FM * FN > 16;
+  static_assert(kLds <= 160 * 1024 && NS >= 4 && KG <= 2 && (KG == 1 || kLds >= WM * WN * FM * FN * 1024));
 };
 
-// Bound: a 256 x 256 block's stage takes ~ 0.7 us on a CU alone and ~ 1 us with all CUs at it, of which the products are
-// ~ 0.5; the copies take the rest (32 KiB a stage: ~ 45 KB/us is what a CU takes in from the L2), so the largest block
-// that still gives every CU one wins: it reads least per product.  Wave tiles of 128 x 64 keep the LDS reads (12 KiB per
-// 32 products) below the products' time; fragments are read a stage ahead into the registers just used (208 VGPRs, two
-// waves a SIMD).  Measured, us, best dense_tile_kernel -> this one, bf16: 2048 x 8192, K 2048 95 -> 74; 1500 x 8704,
-// K 2048 88 -> 65; 1500 x 2048, K 8192 105 -> 89; 64 experts x 192 rows, 2816 x 2048 286 -> 226, 2048 x 1408 156 -> 124.
-template <class T, int WM, int WN, int FM, int FN, int NS, int EPI>
-__global__ __launch_bounds__(64 * WM * WN, 2) void dense_block_kernel(const ti_dense_args a, int m_tiles, int n_tiles) {
+// Bound: with every CU at it the products (~ 1340 TFLOP/s is what the chip's power leaves a bf16 product of random data);
+// a block alone on its CU, LDS traffic and the hand-over of a stage.  So waves take tiles of up to 128 x 64 (LDS reads
+// 12 KiB per 32 products), fragments are read a stage ahead into the registers just used, and blocks of at most 128 x 128
+// run two groups of waves (KG 2) that take alternate k-tiles and meet in LDS at the end: a barrier and its skew per two
+// k-tiles, fewer LDS reads per product than tiles of half the size.  Deeper rings than NS give nothing.  A row of a stage
+// is 64 bytes: four lanes fetch it (chunks XOR-swizzled by row against LDS bank conflicts), 2 - 10 % over a lane per row.
+// Measured, us, bf16, dense_tile_kernel and blocks without KG -> this: 2048 x 2048 at 100 rows 10.8 -> 8.6, 333 11.4 ->
+// 9.2, 1000 18.4 -> 15.0; 2048 x 8192 (N x K) at 333 46.5 -> 29, 1500 85.5 -> 64; 5120 x 2048 at 700 29.8 -> 22; fp32
+// 2048 x 2048 at 100 rows 45 -> 24.
+//
+// One tile: `step` rows at most (ungrouped calls: rows a row tile covers, tile_plan), BN columns.  A wave multiplies R row
+// tiles, R the fewest of FM, 3/4 and 1/2 of it that hold the tile's rows: a ragged last tile, a small expert's and calls that
+// spread over the CUs better by 3/4-high tiles leave the rest out, copies included.
+template <class T, int KG, int WM, int WN, int FM, int FN, int NS, int EPI>
+__global__ __launch_bounds__(64 * KG * WM * WN, 2) void dense_block_kernel(const ti_dense_args a, int m_tiles, int n_tiles, int step_rows) {
   typedef typename El<T>::V V;
-  typedef BlockCfg<WM, WN, FM, FN, NS> C;
-  constexpr int KT = El<T>::KT, VEC = El<T>::VEC, NW = C::kWaves, NF = C::kFrags, ND = C::kDma;
+  typedef BlockCfg<KG, WM, WN, FM, FN, NS> C;
+  constexpr int KT = El<T>::KT, VEC = El<T>::VEC, NW = C::kWaves;
   constexpr bool VF = EPI == TI_DE_VFRAG;
   extern __shared__ __attribute__((aligned(1024))) char ring[];
   TileAt at;
   DenseSpan sp;
   if (!tile_at(a, m_tiles, n_tiles, at) || !dense_span(a, at.y, sp, sizeof(T))) return;
-  const int m_base = at.m * C::BM;
+  const int m_base = at.m * step_rows, m_end = min(sp.rows, m_base + step_rows);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave / WN, wn = wave % WN;
-  const int nk = a.K / KT, NT = (a.N + 15) >> 4;
-  // this wave's fragments of a stage (one k-tile of the block): row tiles first, then weight tiles
-  const V* src[ND];
-  uint32_t dst[ND], step[ND];
+  const int kg = wave / (WM * WN), wm = wave / WN % WM, wn = wave % WN;
+  const int nk = a.K / KT, NT = (a.N + 15) >> 4, ns = nk / KG;   // (K is padded to two k-tiles)
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)ring;
+  const int live = EPI == TI_DE_KFRAG || EPI == TI_DE_VFRAG ? FM : ((m_end - m_base + 15) / 16 + WM - 1) / WM;
+
+  auto tile = [&]<int R>() __attribute__((always_inline)) {
+    constexpr int NA = KG * R * WM, NF = NA + KG * FN * WN, ND = (NF + NW - 1) / NW, REST = NF % NW;
+    static_assert(NS * ND < 64, "vmcnt");
+    const bool whole = REST == 0 || wave < REST;   // this wave copies ND fragments a stage, else one less
+    // this wave's fragments of a stage (KG k-tiles of the block): row tiles by k-tile, then weight tiles by k-tile
+    const V* src[ND];
+    uint32_t dst[ND], step[ND];
 #pragma unroll
-  for (int i = 0; i < ND; ++i) {
-    const int f = i * NW + wave;
-    dst[i] = lds0 + (uint32_t)f * 1024;
-    if (f < FM * WM) {
-      const int p = sp.first + min(m_base + f * 16 + (lane & 15), sp.rows - 1);
-      src[i] = (const V*)((const T*)a.a + (size_t)sp.batch * a.a_batch + (size_t)row_in(a, p) * a.lda) + (lane >> 4);
-      step[i] = KT / VEC;
-    } else {
-      src[i] = (const V*)sp.w + (size_t)min(at.n * (FN * WN) + f - FM * WM, NT - 1) * nk * 64 + lane;
-      step[i] = 64;
-    }
-  }
-  uint32_t fill = 0;   // ring byte the next stage is copied to
-  auto dma1 = [&](int i) {
-    dma_1k_asm(src[i], dst[i] + fill);
-    src[i] += step[i];
-  };
-  auto filled = [&] { fill = fill == (NS - 1) * NF * 1024 ? 0 : fill + NF * 1024; };
-  f32x4 acc[FM][FN];
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  V af[FM], w[2][FN];
-  const V* const first = (const V*)ring + lane;
-  const V* cur = first;   // the stage being multiplied
-  // wave (wm, wn): row tiles wm, wm + WM, ..; weight tiles wn * FN ..
-  auto read_a = [&](const V* st, int i) { af[i] = st[(i * WM + wm) * 64]; };
-  auto read_w = [&](const V* st, V (&d)[FN], int j) { d[j] = st[(FM * WM + wn * FN + j) * 64]; };
-  // One stage, the wave's first R row tiles.  Its weights and all but its last R / 4 row tiles were read a stage ago;
-  // each register takes the next stage's fragment as soon as its products are issued.  The last ones are read here, so
-  // that reads of a ring slot end with its stage and the slot is free once every wave has passed the next barrier.
-  auto stage = [&]<int R, int B>(int s) {
-    constexpr int EARLY = R - R / 4;
-    if (s + NS - 2 < nk) wait_dma<(NS - 3) * ND>();   // stage s + 1 is here (the last ones: everything)
-    else wait_dma<0>();
-    __builtin_amdgcn_s_barrier();
-    const bool more = s + NS - 1 < nk;
-    const V* nxt = cur == first + (NS - 1) * NF * 64 ? first : cur + NF * 64;
-#pragma unroll
-    for (int i = EARLY; i < R; ++i) read_a(cur, i);
-#pragma unroll
-    for (int i = 0; i < R; ++i) {
-#pragma unroll
-      for (int j = 0; j < FN; ++j) acc[i][j] = VF ? mma(af[i], w[B][j], acc[i][j]) : mma(w[B][j], af[i], acc[i][j]);
-      if (i < EARLY) read_a(nxt, i);
-#pragma unroll
-      for (int j = i * FN / R; j < (i + 1) * FN / R; ++j) read_w(nxt, w[B ^ 1], j);
-      __builtin_amdgcn_sched_barrier(0);
-      if (more) {   // the copies spread over the products: a bunch of them blocks the wave's issue
-#pragma unroll
-        for (int d = 0; d < ND; ++d)
-          if (min(1 + d, R - 1) == i) dma1(d);
+    for (int i = 0; i < ND; ++i) {
+      const int f = min(i * NW + wave, NF - 1);
+      dst[i] = lds0 + (uint32_t)f * 1024;
+      if (f < NA) {
+        const int g = f / (R * WM), rt = f % (R * WM);
+        const int p = sp.first + min(m_base + rt * 16 + (lane >> 2), sp.rows - 1);
+        src[i] = (const V*)((const T*)a.a + (size_t)sp.batch * a.a_batch + (size_t)row_in(a, p) * a.lda) + g * (KT / VEC) +
+                 ((lane & 3) ^ (lane >> 3 & 3));
+        step[i] = KG * KT / VEC;
+      } else {
+        const int g = (f - NA) / (FN * WN), ct = (f - NA) % (FN * WN);
+        src[i] = (const V*)sp.w + ((size_t)min(at.n * (FN * WN) + ct, NT - 1) * nk + g) * 64 + lane;
+        step[i] = KG * 64;
       }
-      __builtin_amdgcn_sched_barrier(0);
     }
-    if (more) filled();
-    cur = nxt;
-  };
+    uint32_t fill = 0;   // ring byte the next stage is copied to
+    auto dma1 = [&](int i) __attribute__((always_inline)) {
+      if (i == ND - 1 && !whole) return;
+      dma_1k_asm(src[i], dst[i] + fill);
+      src[i] += step[i];
+    };
+    auto filled = [&] { fill = fill == (NS - 1) * NF * 1024 ? 0 : fill + NF * 1024; };
+    auto wait = [&]<int STAGES>() __attribute__((always_inline)) {   // all but this wave's copies of the newest STAGES stages
+      if (whole) wait_dma<STAGES * ND>();
+      else wait_dma<STAGES * (ND - 1)>();
+    };
+    f32x4 acc[R][FN];
 #pragma unroll
-  for (int d = 0; d < NS - 1; ++d)
-    if (d < nk) {
+    for (int i = 0; i < R; ++i)
 #pragma unroll
-      for (int i = 0; i < ND; ++i) dma1(i);
-      filled();
-    }
-  if (NS - 1 <= nk) wait_dma<(NS - 2) * ND>();
-  else wait_dma<0>();
-  __builtin_amdgcn_s_barrier();
+      for (int j = 0; j < FN; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    V af[R], w[2][FN];
+    const V* const first = (const V*)ring;
+    const V* cur = first;   // the stage being multiplied
+    // wave (kg, wm, wn): k-tile kg of a stage, row tiles wm, wm + WM, .., weight tiles wn * FN ..
+    const int at_a = (kg * R * WM + wm) * 64 + (lane & 15) * 4 + (lane >> 4 ^ (lane >> 1 & 3));
+    const int at_w = (NA + kg * FN * WN + wn * FN) * 64 + lane;
+    auto read_a = [&](const V* st, int i) { af[i] = st[i * WM * 64 + at_a]; };
+    auto read_w = [&](const V* st, V (&d)[FN], int j) { d[j] = st[j * 64 + at_w]; };
+    // One stage.  Its weights and all but its last R / 4 row tiles were read a stage ago; each register takes the next
+    // stage's fragment as soon as its products are issued.  The last ones are read here, so that reads of a ring slot end
+    // with its stage and the slot is free once every wave has passed the next barrier.  MORE: another stage is copied
+    // (2: found out here).
+    auto stage = [&]<int B, int MORE>(int s) __attribute__((always_inline)) {
+      constexpr int EARLY = R - R / 4;
+      const bool more = MORE == 2 ? s + NS - 1 < ns : MORE;
+      if (MORE == 2 && s + NS - 2 >= ns) wait_dma<0>();   // stage s + 1 is here (the last ones: everything)
+      else wait.template operator()<NS - 3>();
+      __builtin_amdgcn_s_barrier();
+      const V* nxt = cur == first + (NS - 1) * NF * 64 ? first : cur + NF * 64;
 #pragma unroll
-  for (int j = 0; j < FN; ++j) read_w(cur, w[0], j);
-  auto product = [&]<int R>() {
+      for (int i = EARLY; i < R; ++i) read_a(cur, i);
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = VF ? mma(af[i], w[B][j], acc[i][j]) : mma(w[B][j], af[i], acc[i][j]);
+        if (i < EARLY) read_a(nxt, i);
+#pragma unroll
+        for (int j = i * FN / R; j < (i + 1) * FN / R; ++j) read_w(nxt, w[B ^ 1], j);
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) {   // the copies spread over the products: a bunch of them blocks the wave's issue
+#pragma unroll
+          for (int d = 0; d < ND; ++d)
+            if (min(1 + d, R - 1) == i) dma1(d);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (more) filled();
+      cur = nxt;
+    };
+#pragma unroll
+    for (int d = 0; d < NS - 1; ++d)
+      if (d < ns) {
+#pragma unroll
+        for (int i = 0; i < ND; ++i) dma1(i);
+        filled();
+      }
+    if (NS - 1 > ns) wait_dma<0>();
+    else wait.template operator()<NS - 2>();
+    __builtin_amdgcn_s_barrier();
+#pragma unroll
+    for (int j = 0; j < FN; ++j) read_w(cur, w[0], j);
 #pragma unroll
     for (int i = 0; i < R - R / 4; ++i) read_a(cur, i);
-    for (int s = 0; s < nk; s += 2) {   // (K is padded to two k-tiles)
-      stage.template operator()<R, 0>(s);
-      stage.template operator()<R, 1>(s + 1);
+    int s = 0;
+    if constexpr (!C::kBig)   // (a second copy of the largest tiles' loop spills)
+      for (; s + NS < ns; s += 2) {
+        stage.template operator()<0, 1>(s);
+        stage.template operator()<1, 1>(s + 1);
+      }
+    for (; s < ns; s += 2) {
+      stage.template operator()<0, 2>(s);
+      if (KG == 1 || s + 1 < ns) stage.template operator()<1, 2>(s + 1);
+    }
+    constexpr int H = KG == 1 ? R : (R + 1) / 2;
+    if constexpr (KG == 2) {   // the halves of k meet: a wave of the first finishes row tiles < H, its partner the others
+      __builtin_amdgcn_s_barrier();   // (every wave's reads of the ring are done)
+      f32x4* x = (f32x4*)ring + (size_t)(wm * WN + wn) * R * FN * 64 + lane;
+#pragma unroll
+      for (int i = 0; i < R; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+          if ((i >= H) == (kg == 0)) x[(i * FN + j) * 64] = acc[i][j];
+      lds_sync();
+#pragma unroll
+      for (int i = 0; i < R; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+          if ((i >= H) != (kg == 0)) acc[i][j] += x[(i * FN + j) * 64];
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int mt = m_base + (i * WM + wm) * 16;
+      if (i >= live) break;
+      if (KG == 2 && (i >= H) == (kg == 0)) continue;
+      const int m = mt + (lane & 15);
+      const int mo = m < m_end ? row_out(a, sp.first + m) : 0;
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+        const int nt = at.n * (FN * WN) + wn * FN + j;
+        if (nt < NT) dense_out<T, EPI>(a, sp, m, mo, mt, nt, acc[i][j], lane);
+      }
     }
   };
-  // row tiles a wave needs: a ragged last tile or a small expert's leaves the rest out (the fragment epilogues
-  // write padding rows too)
-  const int live = EPI == TI_DE_KFRAG || EPI == TI_DE_VFRAG ? FM : ((min(sp.rows - m_base, C::BM) + 15) / 16 + WM - 1) / WM;
-  if (live > FM * 3 / 4) product.template operator()<FM>();
-  else if (live > FM / 2) product.template operator()<FM * 3 / 4>();
-  else product.template operator()<FM / 2>();
-#pragma unroll
-  for (int i = 0; i < FM; ++i) {
-    const int mt = m_base + (i * WM + wm) * 16;
-    if (i >= live) break;
-    const int m = mt + (lane & 15);
-    const int mo = m < sp.rows ? row_out(a, sp.first + m) : 0;
-#pragma unroll
-    for (int j = 0; j < FN; ++j) {
-      const int nt = at.n * (FN * WN) + wn * FN + j;
-      if (nt < NT) dense_out<T, EPI>(a, sp, m, mo, mt, nt, acc[i][j], lane);
-    }
-  }
-  if (EPI == TI_DE_LOGITS && a.step_ctr && at.id == 0 && tid == 0) *a.step_ctr += a.advance;
+  constexpr int R2 = FM / 2, R1 = FM * 3 / 4;
+  if (live > R1) tile.template operator()<FM>();
+  else if (R1 != R2 && live > R2) tile.template operator()<R1>();
+  else tile.template operator()<R2>();
 }
 
 template <class T, int MT, int EPI>
@@ -599,14 +643,14 @@ int launch_tile(const ti_dense_args& a, hipStream_t s) {
   return TI_OK;
 }
 
-template <class T, int WM, int WN, int FM, int FN, int NS, int EPI>
-int launch_block(const ti_dense_args& a, hipStream_t s) {
-  typedef BlockCfg<WM, WN, FM, FN, NS> C;
-  const int mt = (a.M + C::BM - 1) / C::BM, nt = (a.N + C::BN - 1) / C::BN;
-  auto* fn = dense_block_kernel<T, WM, WN, FM, FN, NS, EPI>;
+template <class T, int KG, int WM, int WN, int FM, int FN, int NS, int EPI>
+int launch_block(const ti_dense_args& a, int step_rows, hipStream_t s) {
+  typedef BlockCfg<KG, WM, WN, FM, FN, NS> C;
+  const int mt = (a.M + step_rows - 1) / step_rows, nt = (a.N + C::BN - 1) / C::BN;
+  auto* fn = dense_block_kernel<T, KG, WM, WN, FM, FN, NS, EPI>;
   TI_HIP_CHECK(hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, C::kLds),
                "hipFuncSetAttribute(dense_block_kernel)");
-  hipLaunchKernelGGL(fn, dim3(tile_grid(a, mt, nt), a.tile_rows ? 1 : a.batch), dim3(64 * C::kWaves), C::kLds, s, a, mt, nt);
+  hipLaunchKernelGGL(fn, dim3(tile_grid(a, mt, nt), a.tile_rows ? 1 : a.batch), dim3(64 * C::kWaves), C::kLds, s, a, mt, nt, step_rows);
   TI_LAUNCH_CHECK("dense_block_kernel");
   return TI_OK;
 }
@@ -621,36 +665,54 @@ int skinny(const ti_dense_args& a, hipStream_t s) {
   return launch_skinny<T, 4, EPI>(a, s);
 }
 
-// More rows: the tile whose rounds over the 256 CUs cost least: us of a launch and per round at K 2048, measured (bf16
-// M 100 .. 2048, N 1024 .. 8704, K 1024 .. 8192; fp32: the products decide, so the smallest tile that fills the chip).
-constexpr int kTileM[6] = {256, 128, 128, 64, 64, 32}, kTileN[6] = {256, 256, 128, 256, 128, 128};
+// More rows: the tile whose rounds over the 256 CUs cost least: us of a launch, of a round and of 2048 k in it, fitted to
+// measurements (bf16: M 70 .. 2048, N 512 .. 14336, K 256 .. 8192, fp32 M 70 .. 700; the choice costs 0.4 % more than the best
+// tile of each point, in the mean).  rows: how many of the block's a tile takes.
+struct BlockTile {
+  int m, n, rows;
+  float fix[2], round[2], k2048[2];   // bf16, fp32
+};
+constexpr int kTiles = 11;
+constexpr BlockTile kTile[kTiles] = {
+    {256, 256, 256, {-2.41f, 4.2f}, {13.0f, 4.2f}, {40.8f, 349.3f}}, {256, 256, 192, {-1.68f, 4.8f}, {11.36f, 4.8f}, {34.07f, 275.6f}},
+    {128, 256, 128, {-0.74f, 7.4f}, {7.51f, 7.4f}, {26.02f, 232.9f}}, {128, 256, 96, {-0.75f, 6.8f}, {6.83f, 6.8f}, {22.84f, 195.5f}},
+    {128, 128, 128, {2.40f, 4.6f}, {2.35f, 3.8f}, {16.59f, 128.8f}}, {128, 128, 128, {-0.97f, -2.3f}, {6.58f, 11.9f}, {14.30f, 132.9f}},
+    {128, 128, 96, {0.49f, 0.4f}, {4.73f, 8.8f}, {13.01f, 99.2f}}, {64, 128, 64, {-0.16f, 1.4f}, {4.73f, 5.0f}, {9.26f, 69.0f}},
+    {64, 128, 48, {0.39f, -0.5f}, {4.03f, 5.7f}, {8.37f, 54.0f}}, {64, 64, 64, {0.73f, -0.2f}, {3.40f, 4.4f}, {6.13f, 36.7f}},
+    {32, 64, 32, {1.57f, 0.3f}, {2.27f, 3.9f}, {5.34f, 20.6f}}};
 inline int tile_of(const ti_dense_args& a) {
-  const bool F = a.dtype == TI_DT_F32;
-  const float fix[6] = {12.f, 5.f, 5.5f, 2.5f, 2.f, 2.f};
-  const float per[6] = {F ? 485.f : 56.f, F ? 250.f : 36.f, F ? 134.f : 24.f, F ? 130.f : 25.f, F ? 72.f : 15.f, F ? 37.f : 10.f};
-  float c[6];
-  for (int i = 0; i < 6; ++i) {
-    const long wgs = (long)((a.M + kTileM[i] - 1) / kTileM[i]) * ((a.N + kTileN[i] - 1) / kTileN[i]) * a.batch;
-    c[i] = fix[i] + (float)((wgs + 255) / 256) * per[i] * (float)a.K * (1.f / 2048);
+  const int f = a.dtype == TI_DT_F32;
+  int best = 0;
+  float least = 0.0f;
+  for (int i = 0; i < kTiles; ++i) {
+    const BlockTile& t = kTile[i];
+    const long wgs = (long)((a.M + t.rows - 1) / t.rows) * ((a.N + t.n - 1) / t.n) * a.batch;
+    const float us = t.fix[f] + (float)((wgs + 255) / 256) * (t.round[f] + t.k2048[f] * (float)a.K * (1.f / 2048));
+    if (i == 0 || us < least) {
+      least = us;
+      best = i;
+    }
   }
-  return (int)(std::min_element(c, c + 6) - c);
+  return best;
 }
 template <class T, int EPI>
 int tiled(const ti_dense_args& a, hipStream_t s) {
-  switch (tile_of(a)) {
-    case 0: return launch_block<T, 2, 4, 8, 4, 5, EPI>(a, s);
-    case 1: return launch_block<T, 2, 4, 4, 4, 5, EPI>(a, s);
-    case 2: return launch_block<T, 2, 2, 4, 4, 5, EPI>(a, s);
-    case 3: return launch_tile<T, 64, 256, 2, EPI>(a, s);
-    case 4: return launch_tile<T, 64, 128, 4, EPI>(a, s);
-    default: return launch_tile<T, 32, 128, 4, EPI>(a, s);
+  const int i = tile_of(a), rows = kTile[i].rows;
+  switch (i) {
+    case 0: case 1: return launch_block<T, 1, 2, 4, 8, 4, 5, EPI>(a, rows, s);
+    case 2: case 3: return launch_block<T, 1, 2, 4, 4, 4, 5, EPI>(a, rows, s);
+    case 4: return launch_block<T, 1, 2, 2, 4, 4, 5, EPI>(a, rows, s);
+    case 5: case 6: return launch_block<T, 2, 2, 2, 4, 4, 5, EPI>(a, rows, s);
+    case 7: case 8: return launch_block<T, 2, 1, 4, 4, 2, 6, EPI>(a, rows, s);
+    case 9: return launch_block<T, 2, 2, 2, 2, 2, 9, EPI>(a, rows, s);
+    default: return launch_block<T, 2, 1, 4, 2, 1, 13, EPI>(a, rows, s);
   }
 }
 // Grouped products: the tile of the list's rows.
 template <class T, int EPI>
 int grouped(const ti_dense_args& a, hipStream_t s) {
-  if (a.tile_rows == 256) return launch_block<T, 2, 4, 8, 4, 5, EPI>(a, s);
-  if (a.tile_rows == 128) return launch_block<T, 2, 4, 4, 4, 5, EPI>(a, s);
+  if (a.tile_rows == 256) return launch_block<T, 1, 2, 4, 8, 4, 5, EPI>(a, 256, s);
+  if (a.tile_rows == 128) return launch_block<T, 1, 2, 4, 4, 4, 5, EPI>(a, 128, s);
   return launch_tile<T, 64, 256, 2, EPI>(a, s);
 }
 
@@ -672,8 +734,8 @@ int dispatch_dense(const ti_dense_args& a, hipStream_t s) {
       if (few) return skinny<T, TI_DE_T>(a, s);
       return a.tile_rows ? grouped<T, TI_DE_T>(a, s) : launch_tile<T, 64, 64, 4, TI_DE_T>(a, s);
     // (every row of a 128-row tile is written by the fragment epilogues; 2048 x 2048, K 512: 15.0 -> 14.4 us by blocks)
-    case TI_DE_KFRAG: return launch_block<T, 2, 2, 4, 4, 5, TI_DE_KFRAG>(a, s);
-    default: return launch_block<T, 2, 2, 4, 4, 5, TI_DE_VFRAG>(a, s);
+    case TI_DE_KFRAG: return launch_block<T, 1, 2, 2, 4, 4, 5, TI_DE_KFRAG>(a, 128, s);
+    default: return launch_block<T, 1, 2, 2, 4, 4, 5, TI_DE_VFRAG>(a, 128, s);
   }
 }
 
@@ -748,8 +810,8 @@ extern "C" int ti_dense_tile(const ti_dense_args* a, int* rows, int* cols) {
   if (!a || !rows || !cols || a->M < 1 || a->N < 1 || a->K < 1 || a->batch < 1 ||
       (a->epi != TI_DE_F32 && a->epi != TI_DE_SWIGLU && a->epi != TI_DE_ROPE && a->epi != TI_DE_ACT) || a->tile_rows)
     return ti_set_error(TI_ERR_ARG, "ti_dense_tile: bad arguments");
-  *rows = few_rows(*a) ? 0 : kTileM[tile_of(*a)];
-  *cols = few_rows(*a) ? 0 : kTileN[tile_of(*a)];
+  *rows = few_rows(*a) ? 0 : kTile[tile_of(*a)].m;
+  *cols = few_rows(*a) ? 0 : kTile[tile_of(*a)].n;
   return TI_OK;
 }
 
