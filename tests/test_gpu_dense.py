@@ -258,3 +258,31 @@ def test_small_tiles(ti, shape, M, N, K, dtype, epi):
     else:
         check_swiglu(out[:M], a, w[0], dtype)
     assert (out[M] == 7).all()
+
+
+@pytest.mark.parametrize("M,E,top,tile_rows", [(1, 5, 3, 16), (17, 7, 2, 16), (300, 64, 6, 128), (700, 130, 5, 64), (640, 3, 2, 256), (64, 1, 1, 64)])
+def test_route_tiles(ti, M, E, top, tile_rows):
+    """Tiles of a given choice: every entry once, in its expert's tile; whole tiles first, then the rests, largest first."""
+    g = torch.Generator(device="cuda").manual_seed(M)
+    skew = torch.rand(M, E, device="cuda", generator=g) ** torch.linspace(1, 4, E, device="cuda")
+    idx = skew.topk(top, 1).indices.int().contiguous()
+    cap = ti.lib().ti_route_max_tiles(M, E, top, tile_rows)
+    wgt = torch.zeros(M, top, device="cuda")
+    lst = torch.full((M * top,), -1, dtype=torch.int32, device="cuda")
+    tiles = torch.full((cap, 4), -1, dtype=torch.int32, device="cuda")
+    n = torch.zeros(1, dtype=torch.int32, device="cuda")
+    r = ti.RouteArgs(logits=None, ld=E, M=M, E=E, top=top, idx=idx.data_ptr(), wgt=wgt.data_ptr(), list=lst.data_ptr(),
+                     tiles=tiles.data_ptr(), n_tiles=n.data_ptr(), tile_rows=tile_rows)
+    torch.cuda.synchronize()
+    ti.check(ti.lib().ti_route(C.byref(r), None))
+    ti.sync()
+    idx, lst, tiles, n = idx.flatten().cpu().numpy(), lst.cpu().numpy(), tiles.cpu().numpy(), int(n)
+    counts = np.bincount(idx, minlength=E)
+    assert n == (-(-counts // tile_rows)).sum() <= cap and sorted(lst) == list(range(M * top))
+    seen = []
+    for e, first, rows, _ in tiles[:n]:
+        assert (idx[lst[first:first + rows]] == e).all()
+        seen += range(first, first + rows)
+    assert sorted(seen) == list(range(M * top))
+    rows = tiles[:n, 2]
+    assert (np.diff(rows) <= 0).all() and (rows == tile_rows).sum() == (counts // tile_rows).sum()

@@ -296,21 +296,23 @@ __global__ __launch_bounds__(64 * W) void dense_skinny_kernel(const ti_dense_arg
 
 // Consecutive workgroups go to the 8 XCDs in turn.  An XCD gets a contiguous run of the work list, ordered so that
 // neighbours share weight columns (its L2 holds them once): row tiles fastest, for grouped products 4 tiles (mostly one
-// expert's) fastest, then the columns.  Grouped tiles of 128 rows and more: those groups of 4 dealt to the XCDs in turn,
-// since experts' rows differ and a run leaves XCDs waiting for the one with the largest (2048 rows of trained-like
-// routing, 64 experts, gate/up: 275 -> 253 us; 64-row tiles of few rows lose 5 % by it).
+// expert's) fastest, then the columns.  Grouped tiles of 128 rows and more are dealt to the XCDs, there and back, each with
+// all its columns (its rows are read into one L2): lists come with the large tiles first, so the XCDs' loads match and
+// the small tiles fill the last round (2048 rows of trained-like routing, 64 experts, 75 tiles, us: a run per XCD by expert 275 / -, 4
+// tiles by expert in turn 249 / 147 (gate/up 2816 x 2048 / down 2048 x 1408), this 231 / 129; 863 MB of weights, 5.4 TB/s at
+// best, are 160 of the 231).
 struct TileAt {
   int id, m, n, y;   // work item, row tile, column tile, batch / grouped tile
 };
 __host__ __device__ inline bool tiles_dealt(const ti_dense_args& a) { return a.tile_rows >= 128; }
 inline int tile_grid(const ti_dense_args& a, int m_tiles, int n_tiles) {
-  if (tiles_dealt(a)) return ((a.max_tiles + 3) / 4 * n_tiles + 7) / 8 * 32;
+  if (tiles_dealt(a)) return (a.max_tiles + 7) / 8 * 8 * n_tiles;
   return ((a.tile_rows ? (a.max_tiles + 3) / 4 * 4 : m_tiles) * n_tiles + 7) / 8 * 8;
 }
 __device__ __forceinline__ bool tile_at(const ti_dense_args& a, int m_tiles, int n_tiles, TileAt& t) {
   if (tiles_dealt(a)) {
-    const int q = (int)(blockIdx.x >> 5) * 8 + (int)(blockIdx.x & 7), b = q / n_tiles;
-    t = {(int)blockIdx.x, 0, q - b * n_tiles, b * 4 + (int)((blockIdx.x >> 3) & 3)};
+    const int x = (int)(blockIdx.x & 7), i = (int)(blockIdx.x >> 3) / n_tiles;
+    t = {(int)blockIdx.x, 0, (int)(blockIdx.x >> 3) - i * n_tiles, i * 8 + (i & 1 ? 7 - x : x)};
     return t.y < *a.n_tiles;
   }
   const int list = a.tile_rows ? (*a.n_tiles + 3) / 4 * 4 * n_tiles : m_tiles * n_tiles, per = (list + 7) >> 3;
@@ -616,10 +618,19 @@ __global__ __launch_bounds__(64 * KG * WM * WN, 2) void dense_block_kernel(const
       }
     }
   };
-  constexpr int R2 = FM / 2, R1 = FM * 3 / 4;
-  if (live > R1) tile.template operator()<FM>();
-  else if (R1 != R2 && live > R2) tile.template operator()<R1>();
-  else tile.template operator()<R2>();
+  if constexpr (FM == 8) {
+    if (live > 7) tile.template operator()<8>();
+    else if (live > 6) tile.template operator()<7>();
+    else if (live > 5) tile.template operator()<6>();
+    else if (live > 4) tile.template operator()<5>();
+    else if (live > 2) tile.template operator()<4>();
+    else tile.template operator()<2>();
+  } else {
+    constexpr int R2 = FM / 2, R1 = FM * 3 / 4;
+    if (live > R1) tile.template operator()<FM>();
+    else if (R1 != R2 && live > R2) tile.template operator()<R1>();
+    else tile.template operator()<R2>();
+  }
 }
 
 template <class T, int MT, int EPI>

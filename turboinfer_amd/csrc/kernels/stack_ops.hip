@@ -305,19 +305,21 @@ __device__ __forceinline__ void route_row(const ti_route_args& a, int m) {
   }
 }
 
-// One workgroup groups the M * top entries by expert: counts, a scan over the experts of entries and
-// tiles, then the lists.
+// One workgroup groups the M * top entries by expert: counts, scans over the experts of entries and whole tiles, then the
+// lists.  Tiles: the whole ones by expert, then each expert's rest, the largest first: workgroups start in this order, so
+// the small ones fill the CUs that the large ones leave (dense.hip, tile_at).
 __device__ __forceinline__ void route_group(const ti_route_args& a) {
-  __shared__ int cnt[kMaxE], at[kMaxE], tl[kMaxE];
+  __shared__ int cnt[kMaxE], at[kMaxE], tl[kMaxE], rest[kMaxE];
+  __shared__ int n_whole;
   const int tid = threadIdx.x, nt = blockDim.x, n = a.M * a.top;
   for (int e = tid; e < a.E; e += nt) cnt[e] = 0;
   __syncthreads();
   for (int p = tid; p < n; p += nt) atomicAdd(&cnt[a.idx[p]], 1);
   __syncthreads();
   if (tid < 64) {   // wave 0: exclusive scans over the experts, 64 at a time
-    int base = 0, tbase = 0;
+    int base = 0, tbase = 0, rests = 0;
     for (int e0 = 0; e0 < a.E; e0 += 64) {
-      const int e = e0 + tid, c = e < a.E ? cnt[e] : 0, t = (c + a.tile_rows - 1) / a.tile_rows;
+      const int e = e0 + tid, c = e < a.E ? cnt[e] : 0, t = c / a.tile_rows, r = c - t * a.tile_rows;
       int ic = c, it = t;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) {
@@ -330,21 +332,35 @@ __device__ __forceinline__ void route_group(const ti_route_args& a) {
       if (e < a.E) {
         at[e] = base + ic - c;
         tl[e] = tbase + it - t;
+        rest[e] = r;
       }
       base += __shfl(ic, 63, 64);
       tbase += __shfl(it, 63, 64);
+      rests += __popcll(__ballot(r != 0));
     }
-    if (tid == 0) *a.n_tiles = tbase;
+    if (tid == 0) {
+      n_whole = tbase;
+      *a.n_tiles = tbase + rests;
+    }
   }
   __syncthreads();
-  for (int e = tid; e < a.E; e += nt)
-    for (int i = 0, c = cnt[e]; i < c; i += a.tile_rows) {
-      int* t = a.tiles + 4 * (tl[e] + i / a.tile_rows);
+  for (int e = tid; e < a.E; e += nt) {
+    const int r = rest[e], whole = (cnt[e] - r) / a.tile_rows;
+    auto put = [&](int slot, int first, int rows) {
+      int* t = a.tiles + 4 * slot;
       t[0] = e;
-      t[1] = at[e] + i;
-      t[2] = min(a.tile_rows, c - i);
+      t[1] = first;
+      t[2] = rows;
       t[3] = 0;
+    };
+    for (int i = 0; i < whole; ++i) put(tl[e] + i, at[e] + i * a.tile_rows, a.tile_rows);
+    if (r) {
+      int rank = 0;
+#pragma unroll 8
+      for (int o = 0; o < a.E; ++o) rank += rest[o] > r || (rest[o] == r && o < e);
+      put(n_whole + rank, at[e] + whole * a.tile_rows, r);
     }
+  }
   __syncthreads();
   for (int p = tid; p < n; p += nt) a.list[atomicAdd(&at[a.idx[p]], 1)] = p;
 }
