@@ -427,8 +427,8 @@ def main() -> int:
 
     def class_kernel(name):
         N_, K_ = shapes[name]
-        if B >= (9 if bits == 4 else 6):
-            return "gemm_wide_kernel"
+        if B >= 3:   # (up to 48 rows whichever of the two is estimated the faster)
+            return "gemm_wide_kernel" if B > 48 else "gemm_few_kernel / gemm_wide_kernel"
         if name in ("qkv", "gate_up", "lm_head"):
             if fold_on:
                 xk = T.X_F16_FOLDED

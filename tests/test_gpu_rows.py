@@ -65,6 +65,26 @@ def test_rows_store(ti, oracle, ws, bits, M, K, N):
         assert_close_dot(yd.download(f32, (M, N)), ref, xa, w)
 
 
+# the few-rows kernel (gemm_few.hip): rows at the edges of its 16-, 32- and 48-row blocks, waves without a group of k (K below
+# 1024), with one, two, three, four and five, columns of several rounds and a ragged last block of columns
+@pytest.mark.parametrize("M,K,N", [(2, 128, 16), (3, 896, 48), (15, 1024, 4112), (16, 1152, 2048), (4, 2176, 8208), (17, 3072, 80),
+                                   (31, 3968, 4112), (32, 2048, 2064), (33, 4224, 112), (47, 896, 1040), (48, 5120, 272)])
+@pytest.mark.parametrize("bits", [4, 8, 16, 4 | G32, 8 | G32])
+def test_rows_few(ti, oracle, bits, M, K, N):
+    rng = np.random.RandomState(M * 11 + K + N + bits)
+    td, sd, w = weight(ti, oracle, bits, K, N, rng)
+    ldx = K + 8 * (M % 2)
+    x = rng.standard_normal((M, ldx)).astype(f16)
+    xd, yd = dev(ti, x), ti.DeviceBuffer((M + 1) * N * 4)
+    yd.zero()
+    ep = ti.Epilogue()
+    ep.kind, ep.ldo, ep.out = ti.EPI_STORE_F32, N, yd.ptr
+    rows(ti, bits, td, sd, xd, M, N, K, ep, ldx)
+    y, xa = yd.download(f32, (M + 1, N)), x[:, :K].astype(f32)
+    assert_close_dot(y[:M], xa.astype(np.float64) @ w.astype(np.float64), xa, w)
+    assert not y[M].any()
+
+
 def test_rows_affine_blocks(ti, oracle, ws):
     """Q4_1 blocks (4 | 32 | 64): the offset term through the block's sum of x."""
     from test_gpu_g32 import pack_q1

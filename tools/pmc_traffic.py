@@ -25,7 +25,7 @@ MODELS = {   # bench.py MODELS: vocab, hidden, layers, heads, kv_heads, head_dim
     "tinyllama-1.1b": (32000, 2048, 22, 32, 4, 64, 5632, 8),
     "llama3-8b": (128256, 4096, 32, 32, 8, 128, 14336, 4),
 }
-GEMM = ("gemv_wq_kernel", "gemm_rows_kernel", "gemm_wide_kernel", "gemv_mbr_kernel",
+GEMM = ("gemv_wq_kernel", "gemm_rows_kernel", "gemm_wide_kernel", "gemm_few_kernel", "gemv_mbr_kernel",
         "qkv_attn_kernel")   # (the fused QKV + attention of one stream, DESIGN 4.19: its step position is QKV's)
 
 

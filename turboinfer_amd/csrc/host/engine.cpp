@@ -303,14 +303,11 @@ int validate(const ti_engine_config& c) {
   return TI_OK;
 }
 
-// Rows whose projections run on the many-rows kernel (ti_gemm_rows).  From the rows where a layer's four launches
-// take less there, the rms_norm folded into them, than the fused kernel's (int8 / fp16: its rms_norm prologue and, from
-// 8 rows on, several launches for a long K) or the 3..16-row int4 kernel's beside two rms_norm launches.  Measured at
-// 4 / 8 / 16 rows, us per layer: int8 2048 x 5632 30.6 / 30.5 / 30.6 against 30.3 / 33 / 35, fp16 35 / 35 / 35 against
-// 37 / 40 / 45, int4 4096 x 11008 50 / 50 / 50 against 42 / 46 / 55.
-bool rows_wide(const ti_engine* e, int M) {
-  return e->wide_ok && M >= ((e->c.bits & ~TI_BITS_G32) == 4 ? 9 : 6);
-}
+// Rows whose projections run on ti_gemm_rows, the rms_norm folded into them: from 3 on.  Below, the fused kernel (its rms_norm
+// prologue) takes as long.  Measured, the mean over the products of four models, its time or that of the int4 kernel of 3 .. 16
+// rows beside its rms_norm over this: at 2 rows 1.01 (int4) / 0.99 (int8) / 0.97 (blocks of 32), at 4 1.07 / 1.17 / 1.17, at 8
+// 1.13 / 1.39 / 1.36.
+bool rows_wide(const ti_engine* e, int M) { return e->wide_ok && M >= 3; }
 
 // One projection for rows [0, M): the many-rows kernel, fp32 rows normalised into fp16 first (e->xn); or the fused
 // kernel in chunks of the rows its LDS image holds (int4 rows that do not fit: the batched kernel behind the same

@@ -7,15 +7,6 @@
 
 namespace ti {
 
-// Formats by their bits value (ti_hip.h): 4, 8, 16, 4 | 32, 8 | 32, 4 | 32 | 64.
-template <int F>
-struct WideFmt {
-  static constexpr int kBits = F & 31;
-  static constexpr bool kG32 = (F & TI_BITS_G32) != 0, kAff = (F & TI_BITS_AFF) != 0;
-  static constexpr int kTile = kBits * 256;                               // bytes of a 16 x 128 weight tile
-  static constexpr int kScale = kBits == 16 ? 0 : kG32 ? 128 : 32;        // bytes of its scales
-};
-
 typedef uint32_t u32x4s __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ u32x4s raw_rsrc(const void* p, uint32_t bytes) {
@@ -112,65 +103,6 @@ __device__ __forceinline__ bool wide_merge(const GemvArgs& a, f32x4 (&acc)[TN][T
     for (int b = 0; b < TM; ++b) acc[t][b] = sum[t][b];
   if (threadIdx.x == 0) __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // re-arm
   return true;
-}
-
-// Batched fold, consumer side: this thread's share of row m's partial sums of h^2 (part, part + P, ...), summed in order;
-// negative if one of them is.
-__device__ __forceinline__ float wide_fold_share(const GemvArgs& a, int m, int part, int P) {
-  float t = 0.0f;
-  uint32_t any = 0;
-  if (m >= a.M) return t;
-  const float* ss = a.epi.ss_in + m;
-  for (int b0 = part; b0 < a.epi.n_ss; b0 += 16 * P) {
-    float v[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) v[j] = b0 + j * P < a.epi.n_ss ? ss[(size_t)(b0 + j * P) * TI_FOLD_SS_ROWS] : 0.0f;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      t += fabsf(v[j]);
-      any |= __builtin_bit_cast(uint32_t, v[j]);
-    }
-  }
-  return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, t) | (any & 0x80000000u));
-}
-// The threads' shares to the rms of every row, negative as they are (behind a barrier; one follows).
-template <int ROWS, int NW>
-__device__ __forceinline__ void wide_fold_rms(const GemvArgs& a, float share, int tid, float* rmsv) {
-  rmsv[ROWS + tid] = share;
-  lds_barrier();
-  if (tid < ROWS) {
-    float t = 0.0f;
-    uint32_t any = 0;
-    for (int p = 0; p < 64 * NW / ROWS; ++p) {
-      const float v = rmsv[ROWS + p * ROWS + tid];
-      t += fabsf(v);
-      any |= __builtin_bit_cast(uint32_t, v);
-    }
-    rmsv[tid] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, sqrtf(t / (float)a.K + a.eps)) | (any & 0x80000000u));
-  }
-  lds_barrier();
-}
-// The rows whose rms is negative as ti_rmsnorm_f16 gives them.  Every workgroup rewrites them whole, with the same values,
-// before it reads them.
-template <int ROWS, int NW>
-__device__ __forceinline__ void wide_refold(const GemvArgs& a, int wave, int lane, const float* rmsv) {
-  typedef f16 f16x4 __attribute__((ext_vector_type(4)));
-#pragma unroll 1
-  for (int m = wave; m < ROWS; m += NW) {   // (rows past M have a positive one)
-    const float rms = -rmsv[m];
-    if (__builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, rms)) < 0) continue;
-#pragma unroll 1
-    for (int k0 = 0; k0 < a.K; k0 += 4 * kWave) {   // (K is a multiple of 128: the upper lanes repeat the last piece)
-      const int k = min(k0 + 4 * lane, a.K - 4);
-      const f32x4 v = *(const f32x4*)(a.epi.fold_w + (size_t)m * a.K + k), w = *(const f32x4*)(a.norm_w + k);
-      f16x4 y;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) y[i] = mul_f16(v[i] / rms, w[i]);
-      *(f16x4*)((f16*)a.x + (size_t)m * a.ldx + k) = y;
-    }
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  lds_barrier();
 }
 
 // Bound: int4 and int8 by the vector unit beside the matrix cores (a 16x16x32 MFMA and its share of dequant and scale
@@ -481,57 +413,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const GemvAr
       for (int i = 0; i < 4; ++i)
         stg[(b * 16 + 4 * kq + i) * kTileEpiStride + r] = fold_in ? av[b][i] / rms[b][i] : av[b][i];
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    if (fold_out) {   // residual add + the next call's folded input (fp16(h * w), sum of h^2 per row)
-      const int c4 = 4 * (lane & 3), ng = tn * 16 + c4;
-      const float4 w = *(const float4*)(e.fold_w + ng);
-#pragma unroll
-      for (int it = 0; it < TM; ++it) {
-        const int row = 16 * it + (lane >> 2), m = mb + row;
-        const float4 v = *(const float4*)(stg + row * kTileEpiStride + c4);
-        float q = 0.0f;
-        if (m < a.M) {
-          float4* o = (float4*)((float*)e.out + (size_t)m * e.ldo + ng);
-          const float4 h0 = *o, h = make_float4(h0.x + v.x, h0.y + v.y, h0.z + v.z, h0.w + v.w);
-          *o = h;
-          float p[4] = {h.x * w.x, h.y * w.y, h.z * w.z, h.w * w.w};
-          // (largest |p|; as outputs the products are rounded on their own, as in mul_f16)
-          asm("v_max3_f32 %0, %0, |%1|, |%2|\n\tv_max3_f32 %0, %0, |%3|, |%4|" : "+v"(top[it]), "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]));
-          auto f = [](float v) { return (uint32_t)f2h(v); };
-          *(uint2*)(e.fold_x + (size_t)m * e.ldo + ng) = make_uint2(f(p[0]) | (f(p[1]) << 16), f(p[2]) | (f(p[3]) << 16));
-          q = (h.x * h.x + h.y * h.y) + (h.z * h.z + h.w * h.w);
-        }
-        q += lane_xor<1>(q);
-        hsq[it] += q + lane_xor<2>(q);
-      }
-    } else if (a.vec) {
-      tile_epilogue_lds<TM>(a, tn, mb, stg, lane);
-    } else {
-#pragma unroll 1
-      for (int q = 0; q < TM * 4; ++q) {
-        const int row = q * 4 + kq, m = mb + row;
-        epilogue_mb(a, tn, min(m, a.M - 1), r, stg[row * kTileEpiStride + r], m < a.M);
-      }
-    }
+    wide_tile_out<TM>(a, tn, mb, stg, lane, r, kq, fold_out, hsq, top);
   }
   if (fold_out) {   // this column block's sum of h^2 per row, column-waves in order
     float2* red = (float2*)(smem + C::kEpiRed);
-#pragma unroll
-    for (int it = 0; it < TM; ++it) {
-      const float t2 = fmaxf(top[it], lane_xor<1>(top[it])), t4 = fmaxf(t2, lane_xor<2>(t2));
-      if ((lane & 3) == 0) red[wn * C::kRows + wm * 16 * TM + 16 * it + (lane >> 2)] = make_float2(hsq[it], t4);
-    }
+    wide_fold_part<TM>(red + wn * C::kRows + wm * 16 * TM, hsq, top, lane);
     lds_barrier();
-    if (tid < C::kRows && m0 + tid < a.M) {
-      float t = 0.0f, mx = 0.0f;
-#pragma unroll
-      for (int w = 0; w < WN; ++w) {
-        const float2 v = red[w * C::kRows + tid];
-        t += v.x;
-        mx = fmaxf(mx, v.y);
-      }
-      // negative where fp16(h w) is infinite, or all so small that its steps of 2^-24 are not far below 2^-12 of the largest
-      e.fold_ss[(size_t)cb * TI_FOLD_SS_ROWS + m0 + tid] = mx > 65504.0f || mx < 0x1p-10f ? -t : t;
-    }
+    wide_fold_store<C::kRows, WN>(a, red, cb, m0, tid);
   }
   if (e.kind == TI_EPI_LOGITS_ARGMAX && e.step_ctr && cb == 0 && rb == 0 && tid == 0) *e.step_ctr += e.advance;
   stamp_end(a.stamp, t_entry);
@@ -618,7 +506,7 @@ bool wide_plan(int fmt, int M, int N, int K, int cus, int64_t ws_bytes, bool fol
       const float us = 4.5f + (float)nk * (one > s.alone ? one : s.alone) + seam;
       if (p->shape < 0 || us < best) {
         best = us;
-        *p = {i, n_cb, n_rb, ks, s.rows, s.tiles};
+        *p = {i, n_cb, n_rb, ks, s.rows, s.tiles, us};
       }
     }
   }
@@ -651,10 +539,23 @@ int wide_launch(int fmt, const WidePlan& p, const GemvArgs& a, hipStream_t strea
 
 }  // namespace ti
 
+// Which kernel a call of ti_gemm_rows takes: the few-rows one where its estimate is the lower (the many-rows kernel's is 8 % low
+// for calls of up to 48 rows; the choice costs 0.6 % more than the better one of each of 1000 measured points, in the mean).
+struct RowsPlan {
+  bool few;
+  ti::FewPlan f;
+  ti::WidePlan w;
+};
+static bool rows_plan_of(int bits, int M, int N, int K, int64_t ws_bytes, bool fold, RowsPlan* p) {
+  const bool wide = ti::wide_plan(bits, M, N, K, ti::gemm_cus(), ws_bytes, fold, &p->w);
+  p->few = ti::few_plan(bits, M, N, K, ti::gemm_cus(), &p->f) && (!wide || p->f.us < 1.08f * p->w.us);
+  return p->few || wide;
+}
+
 extern "C" int ti_gemm_rows_fold_partials(int bits, int M, int N, int K, int64_t ws_bytes) {
-  ti::WidePlan p;
-  if (M > TI_FOLD_SS_ROWS || !ti::wide_plan(bits, M, N, K, ti::gemm_cus(), ws_bytes, true, &p)) return 0;
-  return p.n_cb;
+  RowsPlan p;
+  if (M > TI_FOLD_SS_ROWS || !rows_plan_of(bits, M, N, K, ws_bytes, true, &p)) return 0;
+  return p.few ? p.f.n_cb : p.w.n_cb;
 }
 
 static int rows_impl(const void* tiles, const uint16_t* scales, int bits, const void* x, int ldx, const float* h, const float* norm_w,
@@ -686,19 +587,19 @@ static int rows_impl(const void* tiles, const uint16_t* scales, int bits, const 
   if (fold_out &&
       (M > TI_FOLD_SS_ROWS || !epi->fold_w || !epi->fold_ss || epi->fold_packed || !a.vec))
     return ti_set_error(TI_ERR_ARG, "ti_gemm_rows: fold_x needs M <= %d, fold_w, fold_ss and 16-byte aligned rows", TI_FOLD_SS_ROWS);
-  WidePlan p;
+  RowsPlan p;
   if (h) {
     if (!epi->ss_in || fold_out || !norm_w || (((uintptr_t)h | (uintptr_t)norm_w) & 15))
       return ti_set_error(TI_ERR_ARG, "ti_gemm_rows_folded: ss_in, no fold_x, and 16-byte aligned h and norm_w");
     a.norm_w = norm_w;
     a.epi.fold_w = h;
   }
-  if (!wide_plan(bits, M, N, K, gemm_cus(), epi->splitk_ws ? epi->splitk_bytes : 0, epi->ss_in || fold_out, &p))
+  if (!rows_plan_of(bits, M, N, K, epi->splitk_ws ? epi->splitk_bytes : 0, epi->ss_in || fold_out, &p))
     return ti_set_error(TI_ERR_UNSUPPORTED, "ti_gemm_rows: bits %d, M=%d N=%d K=%d", bits, M, N, K);
   const int rp = ti_gemm_prepare();   // no-op once this device is prepared
   if (rp != TI_OK) return rp;
-  a.stamp = ti_stamp_next(STAMP_TILE, wide_workgroups(p));
-  return wide_launch(bits, p, a, (hipStream_t)stream);
+  a.stamp = ti_stamp_next(STAMP_TILE, p.few ? few_workgroups(p.f) : wide_workgroups(p.w));
+  return p.few ? few_launch(bits, p.f, a, (hipStream_t)stream) : wide_launch(bits, p.w, a, (hipStream_t)stream);
 }
 
 extern "C" int ti_gemm_rows(const void* tiles, const uint16_t* scales, int bits, const void* x, int ldx, float eps, int M, int N,

@@ -4,10 +4,141 @@
 
 namespace ti {
 
+// Formats by their bits value (ti_hip.h): 4, 8, 16, 4 | 32, 8 | 32, 4 | 32 | 64.
+template <int F>
+struct WideFmt {
+  static constexpr int kBits = F & 31;
+  static constexpr bool kG32 = (F & TI_BITS_G32) != 0, kAff = (F & TI_BITS_AFF) != 0;
+  static constexpr int kTile = kBits * 256;                               // bytes of a 16 x 128 weight tile
+  static constexpr int kScale = kBits == 16 ? 0 : kG32 ? 128 : 32;        // bytes of its scales
+};
+
+// Batched fold, consumer side: this thread's share of row m's partial sums of h^2 (part, part + P, ...), summed in order;
+// negative if one of them is.
+__device__ __forceinline__ float wide_fold_share(const GemvArgs& a, int m, int part, int P) {
+  float t = 0.0f;
+  uint32_t any = 0;
+  if (m >= a.M) return t;
+  const float* ss = a.epi.ss_in + m;
+  for (int b0 = part; b0 < a.epi.n_ss; b0 += 16 * P) {
+    float v[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) v[j] = b0 + j * P < a.epi.n_ss ? ss[(size_t)(b0 + j * P) * TI_FOLD_SS_ROWS] : 0.0f;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      t += fabsf(v[j]);
+      any |= __builtin_bit_cast(uint32_t, v[j]);
+    }
+  }
+  return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, t) | (any & 0x80000000u));
+}
+// The threads' shares to the rms of every row, negative as they are (behind a barrier; one follows).
+template <int ROWS, int NW>
+__device__ __forceinline__ void wide_fold_rms(const GemvArgs& a, float share, int tid, float* rmsv) {
+  rmsv[ROWS + tid] = share;
+  lds_barrier();
+  if (tid < ROWS) {
+    float t = 0.0f;
+    uint32_t any = 0;
+    for (int p = 0; p < 64 * NW / ROWS; ++p) {
+      const float v = rmsv[ROWS + p * ROWS + tid];
+      t += fabsf(v);
+      any |= __builtin_bit_cast(uint32_t, v);
+    }
+    rmsv[tid] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, sqrtf(t / (float)a.K + a.eps)) | (any & 0x80000000u));
+  }
+  lds_barrier();
+}
+// The rows whose rms is negative as ti_rmsnorm_f16 gives them.  Every workgroup rewrites them whole, with the same values,
+// before it reads them.
+template <int ROWS, int NW>
+__device__ __forceinline__ void wide_refold(const GemvArgs& a, int wave, int lane, const float* rmsv) {
+  typedef f16 f16x4 __attribute__((ext_vector_type(4)));
+#pragma unroll 1
+  for (int m = wave; m < ROWS; m += NW) {   // (rows past M have a positive one)
+    const float rms = -rmsv[m];
+    if (__builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, rms)) < 0) continue;
+#pragma unroll 1
+    for (int k0 = 0; k0 < a.K; k0 += 4 * kWave) {   // (K is a multiple of 128: the upper lanes repeat the last piece)
+      const int k = min(k0 + 4 * lane, a.K - 4);
+      const f32x4 v = *(const f32x4*)(a.epi.fold_w + (size_t)m * a.K + k), w = *(const f32x4*)(a.norm_w + k);
+      f16x4 y;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) y[i] = mul_f16(v[i] / rms, w[i]);
+      *(f16x4*)((f16*)a.x + (size_t)m * a.ldx + k) = y;
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  lds_barrier();
+}
+
+// One weight tile's outputs (16 columns from tn) for the 16 TM rows from mb, from the wave's staging block.  fold_out: the
+// residual add and the next call's folded input; hsq, top: the lane's sums of h^2 and largest |h w| (wide_fold_part).
+template <int TM>
+__device__ __forceinline__ void wide_tile_out(const GemvArgs& a, int tn, int mb, const float* stg, int lane, int r, int kq, bool fold_out,
+                                              float (&hsq)[TM], float (&top)[TM]) {
+  const ti_epilogue& e = a.epi;
+  if (fold_out) {   // residual add + the next call's folded input (fp16(h * w), sum of h^2 per row)
+    const int c4 = 4 * (lane & 3), ng = tn * 16 + c4;
+    const float4 w = *(const float4*)(e.fold_w + ng);
+#pragma unroll
+    for (int it = 0; it < TM; ++it) {
+      const int row = 16 * it + (lane >> 2), m = mb + row;
+      const float4 v = *(const float4*)(stg + row * kTileEpiStride + c4);
+      float q = 0.0f;
+      if (m < a.M) {
+        float4* o = (float4*)((float*)e.out + (size_t)m * e.ldo + ng);
+        const float4 h0 = *o, h = make_float4(h0.x + v.x, h0.y + v.y, h0.z + v.z, h0.w + v.w);
+        *o = h;
+        float p[4] = {h.x * w.x, h.y * w.y, h.z * w.z, h.w * w.w};
+        // (largest |p|; as outputs the products are rounded on their own, as in mul_f16)
+        asm("v_max3_f32 %0, %0, |%1|, |%2|\n\tv_max3_f32 %0, %0, |%3|, |%4|" : "+v"(top[it]), "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]));
+        auto f = [](float v) { return (uint32_t)f2h(v); };
+        *(uint2*)(e.fold_x + (size_t)m * e.ldo + ng) = make_uint2(f(p[0]) | (f(p[1]) << 16), f(p[2]) | (f(p[3]) << 16));
+        q = (h.x * h.x + h.y * h.y) + (h.z * h.z + h.w * h.w);
+      }
+      q += lane_xor<1>(q);
+      hsq[it] += q + lane_xor<2>(q);
+    }
+  } else if (a.vec) {
+    tile_epilogue_lds<TM>(a, tn, mb, stg, lane);
+  } else {
+#pragma unroll 1
+    for (int q = 0; q < TM * 4; ++q) {
+      const int row = q * 4 + kq, m = mb + row;
+      epilogue_mb(a, tn, min(m, a.M - 1), r, stg[row * kTileEpiStride + r], m < a.M);
+    }
+  }
+}
+// The wave's (sum of h^2, largest |h w|) of its 16 TM rows to part.
+template <int TM>
+__device__ __forceinline__ void wide_fold_part(float2* part, const float (&hsq)[TM], const float (&top)[TM], int lane) {
+#pragma unroll
+  for (int it = 0; it < TM; ++it) {
+    const float t2 = fmaxf(top[it], lane_xor<1>(top[it])), t4 = fmaxf(t2, lane_xor<2>(t2));
+    if ((lane & 3) == 0) part[16 * it + (lane >> 2)] = make_float2(hsq[it], t4);
+  }
+}
+// The W parts of a column block (behind a barrier), in order, to fold_ss.
+template <int ROWS, int W>
+__device__ __forceinline__ void wide_fold_store(const GemvArgs& a, const float2* part, int cb, int m0, int tid) {
+  if (tid >= ROWS || m0 + tid >= a.M) return;
+  float t = 0.0f, mx = 0.0f;
+#pragma unroll
+  for (int w = 0; w < W; ++w) {
+    const float2 v = part[w * ROWS + tid];
+    t += v.x;
+    mx = fmaxf(mx, v.y);
+  }
+  // negative where fp16(h w) is infinite, or all so small that its steps of 2^-24 are not far below 2^-12 of the largest
+  a.epi.fold_ss[(size_t)cb * TI_FOLD_SS_ROWS + m0 + tid] = mx > 65504.0f || mx < 0x1p-10f ? -t : t;
+}
+
 struct WidePlan {
   int shape;             // workgroup shape (gemm_wide.hip), -1: none
   int n_cb, n_rb, n_ks;  // column blocks x row blocks x k-slices
   int rows, tiles;       // of a block
+  float us;              // estimate
 };
 // fmt: the bits of ti_gemm_wq_a16.  fold: a call with a folded input or output.  False: not a call of this kernel (shape
 // or format).
@@ -16,5 +147,16 @@ long wide_workgroups(const WidePlan& p);
 int wide_launch(int fmt, const WidePlan& p, const GemvArgs& a, hipStream_t s);
 int gemm_cus();       // CUs of the current device (gemv.hip)
 int wide_prepare();   // dynamic-LDS limits on the current device
+
+
+// gemm_few.hip: up to 48 rows, a workgroup's waves split K
+struct FewPlan {
+  int shape, n_cb;   // workgroup shape, column blocks
+  float us;          // estimate
+};
+bool few_plan(int fmt, int M, int N, int K, int cus, FewPlan* p);
+long few_workgroups(const FewPlan& p);
+int few_launch(int fmt, const FewPlan& p, const GemvArgs& a, hipStream_t s);
+int few_prepare();
 
 }  // namespace ti

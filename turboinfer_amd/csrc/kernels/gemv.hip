@@ -1365,7 +1365,8 @@ extern "C" int ti_gemm_prepare(void) {
   for (const void* f : fns)
     TI_HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024),
                  "hipFuncSetAttribute(gemv_wq_kernel)");
-  const int rc = wide_prepare();
+  int rc = wide_prepare();
+  if (rc == TI_OK) rc = few_prepare();
   if (rc != TI_OK) return rc;
   g_prepared.fetch_or(bit, std::memory_order_acq_rel);
   return TI_OK;
