@@ -376,14 +376,19 @@ int ti_qkv_attn_supported(int bits, int K, int heads, int kv_heads, int head_dim
  * them on fp16 MFMA with the fp32 operands split into fp16 hi + lo parts (fp32-accurate products;
  * ti_attn_decode reads the prefix once per row).  head_dim 64 or 128;
  * heads % kv_heads == 0.  Replaces ti_attn_decode(kv_stream_stride = 0) for row-major chunks.
- * Chunks whose grid fills the chip (head_dim 64: of more than 256 rows) run the shared-K/V kernel: a workgroup per
- * (kv-head, 4 query blocks) copies each K / V block once into LDS for all its waves. */
+ * From 129 keys on the shared-K/V kernel runs: a workgroup per kv-head and 4 query blocks (2, their keys in more parts,
+ * where those workgroups fit the CUs) copies each K / V block once into LDS for all its waves.
+ * ti_attn_prefill_keys: the same with the number of keys that the last row attends to (0: not known; a hint for the
+ * choice of kernel only, ti_attn_prefill takes M for it). */
 int ti_attn_prefill(const float* q, const uint16_t* k_cache, const uint16_t* v_cache, int max_seq,
                     const int32_t* pos, int M, int heads, int kv_heads, int head_dim, uint16_t* out,
                     ti_stream_t s);
+int ti_attn_prefill_keys(const float* q, const uint16_t* k_cache, const uint16_t* v_cache, int max_seq,
+                         const int32_t* pos, int M, int keys, int heads, int kv_heads, int head_dim, uint16_t* out,
+                         ti_stream_t s);
 /* Kernel choice of later ti_attn_prefill calls in this process (parity tests and A/Bs; not a
  * reference interface): 0 automatic (the default, TI_PF_WG applies), 1 the per-wave kernel,
- * 2 the shared-K/V kernel with 4-wave workgroups, 3 with 8-wave workgroups (key-split halves).
+ * 2 the shared-K/V kernel with 4-wave workgroups, 3 with 8-wave workgroups (keys in parts).
  * Modes 2 and 3 apply at any grid size.
  * Returns the previous mode, or -1 for a mode outside 0..3 (nothing changed). */
 int ti_attn_prefill_set_kernel(int mode);

@@ -120,3 +120,24 @@ def test_prefill_attention_rejects_bad_sizes(ti):
     assert L.ti_attn_prefill(1, 1, 1, 16, 1, 0, 4, 4, 128, 1, None) != 0
     assert L.ti_attn_prefill(1, 1, 1, 16, 1, 4, 6, 4, 128, 1, None) != 0
     assert L.ti_attn_prefill(1, 1, 1, 16, 1, 4, 4, 4, 96, 1, None) != 0
+
+
+@pytest.mark.parametrize("M,nh,nkv,hd,start,keys", [
+    (3, 8, 2, 64, 126, 129),        # the first size of the shared kernel: one row of workgroups, waves without a chain
+    (3, 8, 2, 64, 125, 128),        # the last of the per-wave kernel
+    (8, 4, 4, 128, 1000, 1008),     # two query blocks a workgroup, the second past the rows; four parts of 16 blocks
+    (33, 32, 8, 128, 200, 233),     # an odd number of query blocks
+    (333, 32, 8, 128, 0, 333),      # four query blocks a workgroup, two parts
+    (333, 32, 4, 64, 70, 0),        # keys unknown: the rows decide
+    (40, 8, 2, 64, 300, 0),
+])
+def test_prefill_attention_keys(ti, M, nh, nkv, hd, start, keys):
+    """ti_attn_prefill_keys: the hint changes the kernel, not the rows; against the decode kernel (its tolerance above)."""
+    pos = (start + np.arange(M)).astype(np.int32)
+    q, kc, vc, _, dec = _case(ti, M, nh, nkv, hd, pos, start + M, seed=M + hd)
+    qd_, kd, vd, pd, out = dev(ti, q), dev(ti, kc), dev(ti, vc), dev(ti, pos), ti.DeviceBuffer(M * nh * hd * 2)
+    ti.check(ti.lib().ti_attn_prefill_keys(qd_.ptr, kd.ptr, vd.ptr, start + M, pd.ptr, M, keys, nh, nkv, hd, out.ptr, None))
+    ti.sync()
+    got = out.download(f16, (M, nh * hd)).astype(f32)
+    assert np.all(np.isfinite(got))
+    np.testing.assert_allclose(got, dec, rtol=4e-3, atol=4e-3)

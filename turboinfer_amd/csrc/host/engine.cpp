@@ -801,7 +801,7 @@ int enqueue_prefill(ti_engine* e, int m, int t0, int rows, int base, float* laye
     ep.kv_stream_stride = 0;
     TI_TRY(gemm_rows(e, L.qkv, rows, e->h, TI_X_F32_RMSNORM, H, L.attn_norm, ep, 4, false));
     if (prefill_attn_on())   // one pass over the prefix per 16 rows (MFMA)
-      TI_TRY(ti_attn_prefill(e->q, kc, vc, c.max_seq, e->pos, rows, c.heads, c.kv_heads, c.head_dim, e->attn, e->s));
+      TI_TRY(ti_attn_prefill_keys(e->q, kc, vc, c.max_seq, e->pos, rows, base + t0 + rows, c.heads, c.kv_heads, c.head_dim, e->attn, e->s));
     else
       TI_TRY(ti_attn_decode(e->q, kc, vc, 0, c.max_seq, e->pos, rows, c.heads, c.kv_heads, c.head_dim, e->splits_for(rows),
                             e->ws, e->attn, e->s));

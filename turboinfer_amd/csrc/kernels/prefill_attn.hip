@@ -26,6 +26,7 @@
 #include <math.h>
 #include <stdlib.h>
 
+#include <algorithm>
 #include <atomic>
 
 #include "common.hpp"
@@ -57,6 +58,17 @@ __device__ __forceinline__ void pf_split(float x, _Float16& hi, _Float16& lo) {
   asm("" : "+v"(x));   // one value for both roundings (ti::mul_f16's note)
   hi = (_Float16)x;
   lo = (_Float16)(x - (float)hi);
+}
+
+// the same for a pair, to elements i and i + 1: packed conversions (round to nearest), the remainders by one mixed fma each
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void pf_split2(float x, float y, f16x8& hi, f16x8& lo, int i) {
+  const f16x2 h = __builtin_convertvector((f32x2){x, y}, f16x2);
+  const f16x2 l = __builtin_convertvector((f32x2){__builtin_fmaf((float)h[0], -1.0f, x), __builtin_fmaf((float)h[1], -1.0f, y)}, f16x2);
+  hi[i] = h[0];
+  hi[i + 1] = h[1];
+  lo[i] = l[0];
+  lo[i + 1] = l[1];
 }
 
 #ifndef TI_PF_DIAG
@@ -304,16 +316,16 @@ __global__ __launch_bounds__(64, WPE) void attn_prefill_kernel(const float* __re
 // ---------------------------------------------------------------- shared K / V blocks
 // The kernel above gives every wave its own K / V stream from L2, and that stream bounds it
 // (profiles/r5_prefill_attn_diag.txt: 21.5 of 24 us at 512 rows; half-line K reads, ~80 block loads
-// per CU).  Here a workgroup takes 4 query blocks of one kv-head -- query wave q block j + q QG, so
+// per CU).  Here a workgroup takes QB query blocks of one kv-head -- query wave q block j + q QG, so
 // every workgroup holds long and short chains -- and copies each K / V block of their union once
 // into an LDS ring (LDS-DMA, full 128-byte lines), which all its waves read.
 // The per-wave math is the kernel above's: S^T = K Q^T on fp16 MFMA with the fp32 operand in hi + lo,
-// online softmax per column, two blocks per step, and O^T += V^T P^T as one 32-key 16x16x32 product.
+// online softmax per column (here in powers of 2), two blocks per step, and O^T += V^T P^T as one 32-key 16x16x32 product.
 //   K block in LDS: [16 keys][16 chunks of 16 B], the logical chunk c of key row r at physical c ^ r
 //   (an A-fragment read, lane (r, g) chunk 4c + g, is conflict-free in every ds_read_b128 lane group);
 //   head_dim 64: 8 chunks a row, chunk c at c ^ (r >> 1) (a lane group's 16 rows hit each 16 bytes of 256 once);
 //   V block: [16 keys][16 chunks], unswizzled (lane (r, g) reads chunk r of rows 4g + j).
-// Per iteration of BI blocks (2 per half): wait for this wave's 4 DMAs of the iteration; barrier
+// Per iteration of BI blocks (2 per part): wait for this wave's DMAs of the iteration; barrier
 // (everyone's landed, and everyone is done with the previous iteration's blocks); DMA the iteration
 // R / BI - 1 ahead into the slots just freed; compute.  Waves past their own chain keep copying until
 // the workgroup's longest is done; the last DMAs drain before the ring's LDS is reused or released.
@@ -329,11 +341,14 @@ __global__ __launch_bounds__(64, WPE) void attn_prefill_kernel(const float* __re
 #ifndef TI_PF_WG_RING2
 #define TI_PF_WG_RING2 8   // the same, 8-wave workgroups (4 blocks per iteration; 8 beat 12 and 16, profiles/r5_prefill_wg_ring_ab.txt)
 #endif
-// HALVES 2: 8 waves, two per SIMD -- waves w and w + 4 share query block w & 3 and take alternate
-// pairs of its key blocks (iteration = 4 blocks, half h computes blocks 2 h, 2 h + 1 of it), merging
-// their (max, sum, O) through LDS at the end: two chains per SIMD hide each other's latencies.
-template <int HD, int HALVES, int R>
-__global__ __launch_bounds__(256 * HALVES, HD == 64 ? 4 : 1) void attn_prefill_wg_kernel(const float* __restrict__ q, const uint16_t* __restrict__ kc,
+// HALVES: parts of a query block's keys, a wave each (iteration = 2 HALVES blocks, part h computes blocks 2 h, 2 h + 1 of it),
+// merging their (max, sum, O) through LDS at the end: two chains per SIMD hide each other's latencies.  The step is a chain
+// of dependent latencies beside ~ 110 vector instructions, so what counts is that the SIMDs have equal work: waves w and w +
+// 4 (one SIMD) take a long and a short chain (1000 rows of 32 heads on 4, head_dim 64: 26.5 -> 23.6 us with two parts of the
+// same chain before), packed conversions and one fma a score in the softmax (-> 22.2).  Few workgroups: 2 query
+// blocks in 4 parts (918 rows of 8 heads on 2, head_dim 128: 19.4 -> 15.3; 476 rows behind 1024 keys 29 -> 20).
+template <int HD, int QB, int HALVES, int R>
+__global__ __launch_bounds__(64 * QB * HALVES, HD == 64 ? 4 : 1) void attn_prefill_wg_kernel(const float* __restrict__ q, const uint16_t* __restrict__ kc,
                                                                  const uint16_t* __restrict__ vc, int max_seq,
                                                                  const int32_t* __restrict__ pos, int M, int heads, int gsh,
                                                                  float scale, uint16_t* __restrict__ out) {
@@ -345,12 +360,14 @@ __global__ __launch_bounds__(256 * HALVES, HD == 64 ? 4 : 1) void attn_prefill_w
   // K and V rings in ONE array: the halves' merge at the end reuses it as scratch (4 query blocks x
   // 64 lanes x (4 DV + 2) floats), which is larger than the K ring alone
   __shared__ __attribute__((aligned(16))) uint16_t skv[2][R][16 * HD];
-  static_assert(HALVES == 1 || 4 * 64 * (4 * DV + 2) * sizeof(float) <= sizeof(skv), "halves' merge scratch");
+  static_assert((HALVES - 1) * QB * 64 * (4 * DV + 2) * sizeof(float) <= sizeof(skv), "the parts' merge scratch");
   auto& sk = skv[0];
   auto& sv = skv[1];
-  __shared__ int s_kmax[4];
+  __shared__ int s_kmax[QB];
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), qw = wave & 3, half = wave >> 2;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // (a SIMD holds waves w and w + 4: one of a long and one of a short chain)
+  const int part = wave / QB, qw = wave < 4 ? wave % QB : QB - 1 - wave % QB;
   const int G = 1 << gsh, qpw = 16 >> gsh;
   const int kvh = blockIdx.y, QG = gridDim.x, nq = (M + qpw - 1) / qpw;
   const int qb = (QG - 1 - blockIdx.x) + qw * QG;   // longest chains first
@@ -363,7 +380,7 @@ __global__ __launch_bounds__(256 * HALVES, HD == 64 ? 4 : 1) void attn_prefill_w
     kmax = max(kmax, __shfl_xor(kmax, o, 64));
     kmin = min(kmin, __shfl_xor(kmin, o, 64));
   }
-  if (lane == 0 && half == 0) s_kmax[qw] = live ? kmax : 0;
+  if (lane == 0 && part == 0) s_kmax[qw] = live ? kmax : 0;
   f16x8 qh[KW], ql[KW];
   {
     const float* qr = q + ((size_t)qi * heads + h) * HD + 8 * g;
@@ -381,26 +398,32 @@ __global__ __launch_bounds__(256 * HALVES, HD == 64 ? 4 : 1) void attn_prefill_w
     }
   }
   __syncthreads();
-  const int kmax_wg = max(max(s_kmax[0], s_kmax[1]), max(s_kmax[2], s_kmax[3]));
+  int kmax_wg = s_kmax[0];
+#pragma unroll
+  for (int i = 1; i < QB; ++i) kmax_wg = max(kmax_wg, s_kmax[i]);
   const int kl = min(kmax_wg, max_seq - 1);   // rows past it may be unwritten: read row kl instead
   const int nkb = kmax_wg / 16 + 1, nkb_w = live ? kmax / 16 + 1 : 0;
   const uint16_t* kbase = kc + (size_t)kvh * max_seq * HD;
   const uint16_t* vbase = vc + (size_t)kvh * max_seq * HD;
   const uint32_t sk_lds = (uint32_t)(uintptr_t)&sk[0][0], sv_lds = (uint32_t)(uintptr_t)&sv[0][0];
-  // An iteration's BI blocks are 2 ND BI DMA instructions of 1 KiB (a block: RPD rows of K each, then V's); wave w
-  // issues ND of them: all of K or all of V of block w / 2.
-  const int dblk = wave >> 1, dv = wave & 1, dch = lane & (HD / 8 - 1);
+  // An iteration's BI blocks are 2 BI copies (K or V of a block) of ND DMA instructions of 1 KiB (RPD rows each); wave w
+  // makes copies w U ...
+  constexpr int U = 4 / QB;
+  const int dch = lane & (HD / 8 - 1);
   auto issue = [&](int kb0) {   // the iteration starting at block kb0
 #if TI_PF_DIAG & 8   // diagnostic: no copies past the prologue (the math on stale blocks)
     if (kb0 >= R - BI) return;
 #endif
-    const int kb = kb0 + dblk, slot = kb % R;
-    const uint32_t base = (dv ? sv_lds : sk_lds) + (uint32_t)(slot * 16 * HD * 2);
 #pragma unroll
-    for (int i = 0; i < ND; ++i) {
-      const int row = RPD * i + lane / (HD / 8), key = min(kb * 16 + row, kl);
-      const uint16_t* src = dv ? vbase + (size_t)key * HD + dch * 8 : kbase + (size_t)key * HD + ((dch ^ swz(row)) * 8);
-      dma_1k_asm(src, __builtin_amdgcn_readfirstlane(base + (uint32_t)(i * 1024)));
+    for (int u = 0; u < U; ++u) {
+      const int cp = wave * U + u, dv = cp & 1, kb = kb0 + (cp >> 1), slot = kb % R;
+      const uint32_t base = (dv ? sv_lds : sk_lds) + (uint32_t)(slot * 16 * HD * 2);
+#pragma unroll
+      for (int i = 0; i < ND; ++i) {
+        const int row = RPD * i + lane / (HD / 8), key = min(kb * 16 + row, kl);
+        const uint16_t* src = dv ? vbase + (size_t)key * HD + dch * 8 : kbase + (size_t)key * HD + ((dch ^ swz(row)) * 8);
+        dma_1k_asm(src, __builtin_amdgcn_readfirstlane(base + (uint32_t)(i * 1024)));
+      }
     }
   };
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // q and pos in: only the DMAs are counted below
@@ -410,15 +433,15 @@ __global__ __launch_bounds__(256 * HALVES, HD == 64 ? 4 : 1) void attn_prefill_w
 #pragma unroll
   for (int t = 0; t < DV; ++t) acc[t] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
   float m_run = -INFINITY, l_run = 0.0f;
-  constexpr float kPfSlack = 8.0f;   // as above: O rescaled only when a column max moves by > 8
+  constexpr float kLog2e = 1.44269504088896341f, kPfSlack = 8.0f * kLog2e;   // as above: O rescaled only when a column max moves by > 8
   for (int kbi = 0; kbi < nkb; kbi += BI) {
-    // this wave's ND DMAs of iteration kbi are the oldest of the ND (R / BI - 1) in flight
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(ND * (R / BI - 2)) : "memory");
+    // this wave's U ND DMAs of iteration kbi are the oldest of the U ND (R / BI - 1) in flight
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(U * ND * (R / BI - 2)) : "memory");
     __syncthreads();
 #if !TI_PF_WG_LATE_DMA
     issue(kbi + R - BI);
 #endif
-    const int kb = kbi + NB * half;   // this half's pair
+    const int kb = kbi + NB * part;   // this part's pair
 #if TI_PF_DIAG & 4   // diagnostic: the ring and its barriers alone, no math
     const bool act = false;
 #else
@@ -480,9 +503,9 @@ __global__ __launch_bounds__(256 * HALVES, HD == 64 ? 4 : 1) void attn_prefill_w
       bm = fmaxf(bm, __shfl_xor(bm, 16, 64));
       bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
 #endif
-      const float mn = fmaxf(m_run, bm);
+      const float mn = fmaxf(m_run, bm * kLog2e);   // (m_run, l_run, acc: relative to 2^m_run)
       if (__builtin_amdgcn_ballot_w64(mn > m_run + kPfSlack) != 0) {
-        const float alpha = m_run == mn ? 1.0f : __expf(m_run - mn);
+        const float alpha = m_run == mn ? 1.0f : __builtin_amdgcn_exp2f(m_run - mn);
         l_run *= alpha;
         m_run = mn;
 #pragma unroll
@@ -490,13 +513,14 @@ __global__ __launch_bounds__(256 * HALVES, HD == 64 ? 4 : 1) void attn_prefill_w
 #pragma unroll
           for (int i = 0; i < 4; ++i) acc[t][i] *= alpha;
       }
+      // (a part may meet a column whose keys so far are all masked: m_run -inf, p 0)
+      const float off = HALVES > 1 && m_run == -INFINITY ? 0.0f : m_run;
       float ps = 0.0f;
 #pragma unroll
       for (int b = 0; b < NB; ++b)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          // (half 1 may meet a column whose keys so far are all masked: m_run -inf, p 0)
-          pv[b][i] = HALVES == 2 && m_run == -INFINITY ? 0.0f : __expf(pv[b][i] - m_run);
+          pv[b][i] = __builtin_amdgcn_exp2f(fmaf(pv[b][i], kLog2e, -off));
           ps += pv[b][i];
         }
       l_run += ps;
@@ -507,12 +531,7 @@ __global__ __launch_bounds__(256 * HALVES, HD == 64 ? 4 : 1) void attn_prefill_w
 #pragma unroll
       for (int b = 0; b < NB; ++b)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          _Float16 hi, lo;
-          pf_split(pv[b][e], hi, lo);
-          ph[4 * b + e] = hi;
-          pl[4 * b + e] = lo;
-        }
+        for (int e = 0; e < 4; e += 2) pf_split2(pv[b][e], pv[b][e + 1], ph, pl, 4 * b + e);
 #pragma unroll
       for (int t = 0; t < DV; ++t) {
         const uint32_t sel = (t & 1) ? 0x07060302u : 0x05040100u;
@@ -531,25 +550,31 @@ __global__ __launch_bounds__(256 * HALVES, HD == 64 ? 4 : 1) void attn_prefill_w
   // the ring's last copies (clamped rows past the end) land before the ring is reused / released
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  if constexpr (HALVES == 2) {   // half 1 hands (m, l, O) to half 0 through the ring's LDS
-    float* xs = (float*)&skv[0][0][0] + (size_t)qw * 64 * (4 * DV + 2);   // (within skv: static_assert above)
-    if (half == 1) {
+  if constexpr (HALVES > 1) {   // the other parts hand (m, l, O) to part 0 through the ring's LDS
+    auto at = [&](int p_) { return (float*)&skv[0][0][0] + (size_t)((p_ - 1) * QB + qw) * 64 * (4 * DV + 2); };   // (within skv: static_assert above)
+    if (part > 0) {
+      float* xs = at(part);
 #pragma unroll
       for (int t = 0; t < DV; ++t) *(f32x4*)(xs + (4 * t) * 64 + 4 * lane) = acc[t];
       xs[4 * DV * 64 + lane] = m_run;
       xs[4 * DV * 64 + 64 + lane] = l_run;
     }
     __syncthreads();
-    if (half == 1) return;
-    const float m1 = xs[4 * DV * 64 + lane], l1 = xs[4 * DV * 64 + 64 + lane];
-    const float mx = fmaxf(m_run, m1);
-    const float f0 = m_run == -INFINITY ? 0.0f : __expf(m_run - mx), f1 = m1 == -INFINITY ? 0.0f : __expf(m1 - mx);
-    l_run = l_run * f0 + l1 * f1;
+    if (part > 0) return;
 #pragma unroll
-    for (int t = 0; t < DV; ++t) {
-      const f32x4 o1 = *(const f32x4*)(xs + (4 * t) * 64 + 4 * lane);
+    for (int o = 1; o < HALVES; ++o) {
+      const float* xs = at(o);
+      const float m1 = xs[4 * DV * 64 + lane], l1 = xs[4 * DV * 64 + 64 + lane];
+      const float mx = fmaxf(m_run, m1);
+      const float f0 = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - mx), f1 = m1 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m1 - mx);
+      m_run = mx;
+      l_run = l_run * f0 + l1 * f1;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[t][i] = acc[t][i] * f0 + o1[i] * f1;
+      for (int t = 0; t < DV; ++t) {
+        const f32x4 o1 = *(const f32x4*)(xs + (4 * t) * 64 + 4 * lane);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[t][i] = acc[t][i] * f0 + o1[i] * f1;
+      }
     }
   }
   if (!live) return;
@@ -586,6 +611,12 @@ extern "C" int ti_attn_prefill_set_kernel(int mode) {
 extern "C" int ti_attn_prefill(const float* q, const uint16_t* k_cache, const uint16_t* v_cache, int max_seq,
                                const int32_t* pos, int M, int heads, int kv_heads, int head_dim, uint16_t* out,
                                ti_stream_t stream) {
+  return ti_attn_prefill_keys(q, k_cache, v_cache, max_seq, pos, M, 0, heads, kv_heads, head_dim, out, stream);
+}
+
+extern "C" int ti_attn_prefill_keys(const float* q, const uint16_t* k_cache, const uint16_t* v_cache, int max_seq,
+                                    const int32_t* pos, int M, int keys, int heads, int kv_heads, int head_dim, uint16_t* out,
+                                    ti_stream_t stream) {
   if (!q || !k_cache || !v_cache || !pos || !out) return ti_set_error(TI_ERR_ARG, "ti_attn_prefill: null pointer");
   if (M < 1 || heads < 1 || kv_heads < 1 || heads % kv_heads || max_seq < 1 || M > 65535 * 16 || heads > 65535)
     return ti_set_error(TI_ERR_ARG, "ti_attn_prefill: bad sizes M=%d heads=%d kv_heads=%d max_seq=%d", M, heads,
@@ -619,15 +650,19 @@ extern "C" int ti_attn_prefill(const float* q, const uint16_t* k_cache, const ui
   const int forced = g_pf_kernel.load(std::memory_order_relaxed);   // ti_attn_prefill_set_kernel
   const int k = forced == 0 ? wgk : forced - 1;
   const bool wg = k > 0, wg2 = k == 2;
-  const dim3 gw((grid.x + 3) / 4, kv_heads);
-  // 4 query blocks of a kv-head per workgroup, K / V shared in LDS -- when that still gives every CU
-  // a workgroup (256 rows of 7B: 128 workgroups, the per-wave kernel's 512 waves are faster).  head_dim 64, whose
-  // 8-wave workgroups go two to a CU: from 257 rows at any grid (us, per-wave / shared, 32 heads on 4: 128 rows 5.4 / 6.1,
-  // 256 7.9 / 7.7, 333 10.2 / 9.1, 333 behind 600 keys 20.4 / 16.4, 512 14.5 / 11.0, 1000 36.9 / 25.3; 8 on 8: 256 7.3 /
-  // 7.6, 333 9.4 / 8.8, 1000 20.8 / 16.7).
-  if (wg && (forced > 1 || (head_dim == 64 && wg2 ? M > 256 : (long)gw.x * gw.y * 4 >= ns))) {
-    auto* fn = head_dim == 128 ? (wg2 ? ti::attn_prefill_wg_kernel<128, 2, TI_PF_WG_RING2> : ti::attn_prefill_wg_kernel<128, 1, TI_PF_WG_RING>)
-                               : (wg2 ? ti::attn_prefill_wg_kernel<64, 2, TI_PF_WG_RING2> : ti::attn_prefill_wg_kernel<64, 1, TI_PF_WG_RING>);
+  // K / V shared in LDS from 129 keys on (a call that does not say how many: its rows); 2 query blocks of a kv-head per
+  // workgroup while those fit the CUs at once, else 4.  Measured, us, per-wave / 4 blocks / 2 blocks: head_dim 128, 32 heads on 32,
+  // 64 rows 4.9 / 6.7 / 6.7, 100 7.1 / 7.4 / 7.2, 150 9.6 / 8.2 / 8.3, 200 11.2 / 9.4 / 8.9, 330 15.2 / 11.4 / 17; 32 on 8, 440 rows 18.8
+  // / 12.9 / 18.6; 8 rows behind 300 keys 10.3 / 9.0 / 8.8, behind 1000 28.7 / 17.1 / 14.8; head_dim 64, 32 on 4, 100 rows 4.9 / 5.4 /
+  // 5.1, 256 7.5 / 6.8 / 5.9, 330 9.8 / 8.0 / 9.1, 64 rows behind 300 keys 9.0 / 8.1 / 6.5.
+  const int cus = ns > 0 ? ns / 4 : 256;
+  const bool two = wg2 && (long)((grid.x + 1) / 2) * kv_heads <= cus;
+  const dim3 gw(two ? (grid.x + 1) / 2 : (grid.x + 3) / 4, kv_heads);
+  if (wg && (forced > 1 || std::max(keys, M) > 128)) {
+    auto* fn = head_dim == 128 ? (!wg2 ? ti::attn_prefill_wg_kernel<128, 4, 1, TI_PF_WG_RING>
+                                  : two ? ti::attn_prefill_wg_kernel<128, 2, 4, 2 * TI_PF_WG_RING2> : ti::attn_prefill_wg_kernel<128, 4, 2, TI_PF_WG_RING2>)
+                               : (!wg2 ? ti::attn_prefill_wg_kernel<64, 4, 1, TI_PF_WG_RING>
+                                  : two ? ti::attn_prefill_wg_kernel<64, 2, 4, 2 * TI_PF_WG_RING2> : ti::attn_prefill_wg_kernel<64, 4, 2, TI_PF_WG_RING2>);
     hipLaunchKernelGGL(fn, gw, dim3(wg2 ? 512 : 256), 0, s, q, k_cache, v_cache, max_seq, pos, M, heads, gsh, scale, out);
   } else if (head_dim == 128) {
     if (deep)
