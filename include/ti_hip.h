@@ -457,6 +457,14 @@ int ti_step_begin(const ti_step_args* a, ti_stream_t s);
  * positions, and with `slot` n slots): in_tokens[i * in_stride], n_in[i] = 1, base_pos[i], slot[i], *step_ctr = 0. */
 int ti_step_inputs(const int32_t* in, int n, int in_stride, int32_t* in_tokens, int32_t* n_in, int32_t* base_pos,
                    int32_t* slot, int32_t* step_ctr, ti_stream_t s);
+/* Inputs of a prompt chunk of `rows` rows: base_pos[i] = pos0 + i, and with `in` (page-locked host memory) tokens[i] = in[i]. */
+int ti_prompt_inputs(const int32_t* in, int rows, int pos0, int32_t* tokens, int32_t* base_pos, ti_stream_t s);
+/* n floats of device memory to coherent page-locked host memory (both 16-byte aligned) in chunks of TI_OUT_CHUNK bytes:
+ * flags[i] (such memory too) becomes gen once chunk i is there; with `words` two 32-bit words of device memory go to
+ * words_out before flags[0].  The stream's earlier work is done when a flag is set. */
+#define TI_OUT_CHUNK 16384
+int ti_rows_out(const float* src, float* dst, int64_t n, uint32_t* flags, uint32_t gen, const uint32_t* words,
+                uint32_t* words_out, ti_stream_t s);
 
 /* ------------------------------------------------------- on-device sampling
  * InferenceEngine::sample_next_token (inference_engine.cpp:1554-1673) per stream, the uniform

@@ -17,6 +17,7 @@
 #include <atomic>
 #include <cmath>
 #include <queue>
+#include <sched.h>
 #include <cstdlib>
 #include <cstring>
 #include <map>
@@ -227,18 +228,19 @@ struct ti_engine {
     return std::max(1, std::min(sp, std::min(cap, 64)));
   }
 
-  // Device rows to the caller's (pageable) memory through page-locked pieces: the copies of the next pieces run while
-  // the host moves this one out (logits_out).  One engine's (pin_io).
-  static constexpr size_t out_piece = (size_t)1 << 20;
+  // Device rows to the caller's (pageable) memory through a ring of page-locked pieces: the next chunks come while the
+  // host moves one out (logits_out).  One engine's (pin_io).
+  static constexpr size_t out_piece = (size_t)1 << 20, out_chunk = TI_OUT_CHUNK;
   static constexpr int out_pieces = 8;
   char* out_pin = nullptr;
-  int32_t* in_pin = nullptr;   // step_rows: tokens, positions, slots
-  hipEvent_t out_ev[out_pieces] = {};
+  size_t out_bytes = 0;          // of the ring: a whole number of chunks, of pieces from out_pieces pieces on
+  uint32_t* out_flag = nullptr;  // a word per chunk of the ring, then two error words (qa_fault_word)
+  uint32_t out_gen = 0;
+  int32_t* in_pin = nullptr;     // step_rows: tokens, positions, slots; ti_engine_prefill: tokens
 
   ~ti_engine() {
-    for (hipEvent_t v : out_ev)
-      if (v) hipEventDestroy(v);
     if (out_pin) hipHostFree(out_pin);
+    if (out_flag) hipHostFree(out_flag);
     if (in_pin) hipHostFree(in_pin);
     for (auto& g : graphs) hipGraphExecDestroy(g.second);
     for (void* p : allocs) hipFree(p);
@@ -391,16 +393,15 @@ bool part_usable(ti_engine* e, int M) {
 
 // The fused launch's bounded waits: after the stream's work, a set error word means a workgroup's q part or
 // new key never came (wrong results for that step) -- reported, and the exchange zeroed so the generations
-// agree again.  qa_fault_read puts the 8-byte read on the engine's stream (err: page-locked, or waited for at once).
+// agree again.  qa_fault_word: the two words on the device, or null for engines whose 1-stream steps do not take the launch.
 bool qa_usable(ti_engine* e, int M);
-int qa_fault_read(ti_engine* e, uint32_t* err) {
+const uint32_t* qa_fault_word(ti_engine* e) {
+  if (!e->qa_xchg || !qa_usable(e, 1)) return nullptr;
+  return reinterpret_cast<const uint32_t*>(static_cast<char*>(e->qa_xchg) + ti_qkv_attn_error_offset(e->c.heads, e->splits_for(1)));
+}
+int qa_fault_read(ti_engine* e, uint32_t* err) {   // on the engine's stream
   err[0] = err[1] = 0u;
-  if (!e->qa_xchg || !qa_usable(e, 1)) return TI_OK;   // (only engines whose 1-stream steps take the launch)
-  const ti_engine_config& c = e->c;
-  const size_t off = ti_qkv_attn_error_offset(c.heads, e->splits_for(1));
-  if (off + 8 > ti_qkv_attn_xchg_bytes(c.heads, TI_ATTN_MAX_PART_SPLITS))
-    return ti_set_error(TI_ERR_ARG, "engine: exchange error word outside the buffer");
-  E_CHECK(hipMemcpyAsync(err, static_cast<char*>(e->qa_xchg) + off, 8, hipMemcpyDeviceToHost, e->s), "hipMemcpyAsync(D2H)");
+  if (const uint32_t* w = qa_fault_word(e)) E_CHECK(hipMemcpyAsync(err, w, 8, hipMemcpyDeviceToHost, e->s), "hipMemcpyAsync(D2H)");
   return TI_OK;
 }
 int qa_fault_report(ti_engine* e, const uint32_t* err) {
@@ -479,41 +480,93 @@ int enqueue_head(ti_engine* e, int n, float* x) {
   return gemm_rows(e, e->lm, n, x, TI_X_F32_RMSNORM, c.hidden, e->out_norm, el, 4, false);
 }
 
-// Page-locked memory of an engine's steps (at its creation: 2 ms).
+// Page-locked memory of an engine's passes (at its creation: 2 ms).  The ring and its flags are coherent: the host reads
+// them while the kernel that writes them runs.
 int pin_io(ti_engine* e) {
   const ti_engine_config& c = e->c;
-  E_CHECK(hipHostMalloc(reinterpret_cast<void**>(&e->in_pin), (size_t)(3 * c.max_batch + 2) * 4, hipHostMallocDefault), "hipHostMalloc");
-  if ((size_t)c.max_batch * c.vocab * 4 <= e->out_piece * 3 / 2) return TI_OK;
-  E_CHECK(hipHostMalloc(reinterpret_cast<void**>(&e->out_pin), e->out_piece * e->out_pieces, hipHostMallocDefault), "hipHostMalloc");
-  memset(e->out_pin, 0, e->out_piece * e->out_pieces);   // (its pages are mapped at their first touch: here, not in a step)
-  for (hipEvent_t& v : e->out_ev) E_CHECK(hipEventCreateWithFlags(&v, hipEventDisableTiming), "hipEventCreate");
+  const size_t in = std::max((size_t)3 * c.max_batch, (size_t)c.max_seq) * 4, all = (size_t)c.max_batch * c.vocab * 4;
+  const unsigned kind = hipHostMallocMapped | hipHostMallocCoherent;
+  e->out_bytes = std::min((all + e->out_chunk - 1) / e->out_chunk * e->out_chunk, e->out_piece * e->out_pieces);
+  const size_t words = e->out_bytes / e->out_chunk + 2;
+  E_CHECK(hipHostMalloc(reinterpret_cast<void**>(&e->in_pin), in, hipHostMallocDefault), "hipHostMalloc");
+  E_CHECK(hipHostMalloc(reinterpret_cast<void**>(&e->out_pin), e->out_bytes, kind), "hipHostMalloc");
+  E_CHECK(hipHostMalloc(reinterpret_cast<void**>(&e->out_flag), words * 4, kind), "hipHostMalloc");
+  memset(e->out_pin, 0, e->out_bytes);   // (its pages are mapped at their first touch: here, not in a step)
+  memset(e->out_flag, 0, words * 4);
   return TI_OK;
 }
 
-// Logits to the caller, after the stream's work.  Above 1.5 MiB and to ordinary memory in pieces of 1 MiB (measured, us,
-// one pageable hipMemcpyAsync / this: 2 MB 110 / 103, 3 MB 165 / 137, 8.2 MB 465 / 307, 16.4 MB 960 / 625; pieces of
-// 256 KiB 1222, of 4 MiB 660).
-int logits_out(ti_engine* e, float* dst, const float* src, size_t bytes) {
+// Waits until *flag is gen: polled, for a wake-up by the runtime costs 20 - 30 us.  Ends with the stream in any case.
+int out_wait(ti_engine* e, const uint32_t* flag, uint32_t gen) {
+  for (unsigned i = 1;; ++i) {
+    if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == gen) return TI_OK;
+    if (i % 64) {
+      __builtin_ia32_pause();
+    } else if (i % 4096) {
+      sched_yield();
+    } else {
+      const hipError_t q = hipStreamQuery(e->s);
+      if (q == hipErrorNotReady) continue;
+      E_CHECK(q, "hipStreamQuery");
+      if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == gen) return TI_OK;
+      return ti_set_error(TI_ERR_HIP, "engine: the stream ended without its output");
+    }
+  }
+}
+
+// One chunk on to the caller's memory; `far`: past the caches, for outputs that a core's would not hold anyway (a step of
+// 8 streams, 1 MB of logits, 567 -> 555 us; 128 KB are faster through them).
+void out_move(char* dst, const char* src, size_t n, bool far) {
+  typedef long long v2 __attribute__((vector_size(16)));
+  if (!far || (reinterpret_cast<uintptr_t>(dst) & 15) || n % 64) {
+    memcpy(dst, src, n);
+    return;
+  }
+  for (size_t i = 0; i < n; i += 64) {
+    v2 v[4];
+    for (int j = 0; j < 4; ++j) v[j] = reinterpret_cast<const v2*>(src + i)[j];
+    for (int j = 0; j < 4; ++j) __builtin_nontemporal_store(v[j], reinterpret_cast<v2*>(dst + i) + j);
+  }
+  __builtin_ia32_sfence();
+}
+
+// Logits to the caller, after the stream's work; err (nullable): the two error words `words` of device memory.  To
+// ordinary memory through the ring; its slots are launched again by the piece as the host has moved them out.  us beyond
+// the replayed step's, against the runtime's copies (pageable up to 1.5 MiB, pieces above): 128 KB 60 -> 33, 1 MB 88 -> 68.
+int logits_out(ti_engine* e, float* dst, const float* src, size_t bytes, const uint32_t* words = nullptr, uint32_t* err = nullptr) {
+  uint32_t* const pin_err = e->out_flag + e->out_bytes / e->out_chunk;
+  pin_err[0] = pin_err[1] = 0u;
   hipPointerAttribute_t at{};
-  if (bytes <= e->out_piece * 3 / 2) return ti_memcpy_d2h(dst, src, bytes, e->s);
+  bool plain = true;
   if (hipPointerGetAttributes(&at, dst) != hipSuccess) (void)hipGetLastError();   // (not known to the runtime)
-  else if (at.type != hipMemoryTypeUnregistered) return ti_memcpy_d2h(dst, src, bytes, e->s);
-  if (!e->out_pin) return ti_memcpy_d2h(dst, src, bytes, e->s);
-  const int n = (int)((bytes + e->out_piece - 1) / e->out_piece);
-  auto piece = [&](int i) { return std::min(e->out_piece, bytes - (size_t)i * e->out_piece); };
-  auto start = [&](int i) -> int {
-    const int k = i % e->out_pieces;
-    E_CHECK(hipMemcpyAsync(e->out_pin + (size_t)k * e->out_piece, reinterpret_cast<const char*>(src) + (size_t)i * e->out_piece, piece(i),
-                          hipMemcpyDeviceToHost, e->s), "hipMemcpyAsync(D2H)");
-    E_CHECK(hipEventRecord(e->out_ev[k], e->s), "hipEventRecord");
-    return TI_OK;
-  };
-  for (int i = 0; i < std::min(n, e->out_pieces); ++i) TI_TRY(start(i));
-  for (int i = 0; i < n; ++i) {
-    const int k = i % e->out_pieces;
-    E_CHECK(hipEventSynchronize(e->out_ev[k]), "hipEventSynchronize");
-    memcpy(reinterpret_cast<char*>(dst) + (size_t)i * e->out_piece, e->out_pin + (size_t)k * e->out_piece, piece(i));
-    if (i + e->out_pieces < n) TI_TRY(start(i + e->out_pieces));
+  else plain = at.type == hipMemoryTypeUnregistered;
+  if (!plain) {
+    if (words) E_CHECK(hipMemcpyAsync(pin_err, words, 8, hipMemcpyDeviceToHost, e->s), "hipMemcpyAsync(D2H)");
+    TI_TRY(ti_memcpy_d2h(dst, src, bytes, e->s));
+  } else {
+    uint32_t gen[ti_engine::out_pieces];   // of each slot's launch
+    auto start = [&](size_t at, size_t n, bool first) -> int {   // bytes [at, at + n): n fits the ring from at's place on
+      const size_t r = at % e->out_bytes;
+      if (++e->out_gen == 0) ++e->out_gen;
+      for (size_t k = r / e->out_piece; k * e->out_piece < r + n; ++k) gen[k] = e->out_gen;
+      return ti_rows_out(src + at / 4, reinterpret_cast<float*>(e->out_pin + r), (int64_t)(n / 4), e->out_flag + r / e->out_chunk,
+                         e->out_gen, first ? words : nullptr, pin_err, e->s);
+    };
+    TI_TRY(start(0, std::min(bytes, e->out_bytes), true));
+    // the caller's pages are mapped while the GPU works (fresh ones cost 120 us a MB at their first touch); their contents stay
+    volatile char* page = reinterpret_cast<volatile char*>(dst);
+    for (size_t i = 0; i < bytes; i += 4096) page[i] = page[i];
+    for (size_t i = 0; i < bytes; i += e->out_chunk) {
+      const size_t r = i % e->out_bytes, n = std::min(e->out_chunk, bytes - i);
+      TI_TRY(out_wait(e, e->out_flag + r / e->out_chunk, gen[r / e->out_piece]));
+      out_move(reinterpret_cast<char*>(dst) + i, e->out_pin + r, n, bytes >= e->out_piece / 2);
+      const size_t done = i + e->out_chunk, next = done - e->out_piece + e->out_bytes;   // a slot is free: its next piece
+      if (done % e->out_piece == 0 && next < bytes) TI_TRY(start(next, std::min(e->out_piece, bytes - next), false));
+    }
+  }
+  if (err) {
+    err[0] = pin_err[0];
+    err[1] = pin_err[1];
   }
   return TI_OK;
 }
@@ -739,14 +792,14 @@ static bool prefill_attn_on() {
   return on != 0;
 }
 
-int enqueue_prefill(ti_engine* e, int m, int t0, int rows, int base, float* layers_out = nullptr, int layers_stride = 0) {
+// in: page-locked, tokens t0 .. of the prompt (null: they are in in_tokens); free again when the stream's work is done.
+int enqueue_prefill(ti_engine* e, int m, int t0, int rows, int base, const int32_t* in = nullptr, float* layers_out = nullptr,
+                    int layers_stride = 0) {
   const ti_engine_config& c = e->c;
   TI_TRY(state_at(e, m, base + t0));
   state_set(e, m, base + t0 + rows);
   ++e->n_prefill_chunks;
-  std::vector<int32_t> bp(rows);
-  for (int j = 0; j < rows; ++j) bp[j] = base + t0 + j;
-  TI_TRY(ti_memcpy_h2d(e->pf_base, bp.data(), (size_t)rows * 4, e->s));
+  TI_TRY(ti_prompt_inputs(in, rows, base + t0, e->in_tokens + (size_t)m * e->in_cap + t0, e->pf_base, e->s));
   ti_step_args sa{};
   step_embedding(e, sa);
   sa.h = e->h;
@@ -1065,6 +1118,33 @@ int ti_engine_describe(ti_engine* e, ti_engine_config* out) {
   return TI_OK;
 }
 
+// The prompt in in_pin: chunks of pf rows, then the wanted rows of each.
+static int prefill_rows(ti_engine* e, int slot, int n, int pos0, int pf, const int32_t* want, int n_want, float* logits, float* layers_out) {
+  const ti_engine_config& c = e->c;
+  const int H = c.hidden, B = c.max_batch;
+  bool done = false;   // the stream's work, waited for
+  for (int t0 = 0, w = 0; t0 < n; t0 += pf) {
+    const int rows = std::min(pf, n - t0);
+    TI_TRY(enqueue_prefill(e, slot, t0, rows, pos0, e->in_pin + t0, layers_out ? layers_out + (size_t)t0 * H : nullptr, n));
+    done = false;
+    while (w < n_want && want[w] < t0 + rows) {   // the wanted rows, as many at once as the logits buffer holds
+      int k = 1;
+      while (k < B && w + k < n_want && want[w + k] < t0 + rows) ++k;
+      float* x = e->h + (size_t)(want[w] - t0) * H;
+      if (want[w + k - 1] - want[w] != k - 1 || H % 8) {   // consecutive rows of whole 32 bytes: in place
+        for (int i = 0; i < k; ++i)
+          TI_TRY(ti_memcpy_d2d(e->h_last + (size_t)i * H, e->h + (size_t)(want[w + i] - t0) * H, (size_t)H * 4, e->s));
+        x = e->h_last;
+      }
+      TI_TRY(enqueue_head(e, k, x));
+      TI_TRY(logits_out(e, logits + (size_t)w * c.vocab, e->logits, (size_t)k * c.vocab * 4));
+      done = true;
+      w += k;
+    }
+  }
+  return done ? TI_OK : ti_stream_sync(e->s);
+}
+
 int ti_engine_prefill(ti_engine* e, int slot, const int32_t* tokens, int n, int pos0, const int32_t* want, int n_want,
                       float* logits, float* layers_out) {
   if (!e || !tokens || n < 1 || n_want < 0 || (n_want && (!want || !logits)) || slot < 0 || slot >= e->c.max_batch || pos0 < 0 ||
@@ -1075,25 +1155,13 @@ int ti_engine_prefill(ti_engine* e, int slot, const int32_t* tokens, int n, int 
     if (want[i] < 0 || want[i] >= n || (i && want[i] <= want[i - 1]))
       return ti_set_error(TI_ERR_ARG, "ti_engine_prefill: place %d of %d tokens", want[i], n);
   DeviceScope bind_(e);
-  const ti_engine_config& c = e->c;
   if (e->stack) TI_TRY(e->stack->ready());
-  const int pf = e->pf_rows > 0 ? e->pf_rows : std::min(e->rows_cap, 16), H = c.hidden, B = c.max_batch;
+  const int pf = e->pf_rows > 0 ? e->pf_rows : std::min(e->rows_cap, 16);
   TI_TRY(ensure_io(e, n, 1));
-  TI_TRY(ti_memcpy_h2d(e->in_tokens + (size_t)slot * e->in_cap, tokens, (size_t)n * 4, e->s));
-  int w = 0;
-  for (int t0 = 0; t0 < n; t0 += pf) {
-    const int rows = std::min(pf, n - t0);
-    TI_TRY(enqueue_prefill(e, slot, t0, rows, pos0, layers_out ? layers_out + (size_t)t0 * H : nullptr, n));
-    while (w < n_want && want[w] < t0 + rows) {   // the wanted rows, as many at once as the logits buffer holds
-      int k = 0;
-      for (; k < B && w + k < n_want && want[w + k] < t0 + rows; ++k)
-        TI_TRY(ti_memcpy_d2d(e->h_last + (size_t)k * H, e->h + (size_t)(want[w + k] - t0) * H, (size_t)H * 4, e->s));
-      TI_TRY(enqueue_head(e, k, e->h_last));
-      TI_TRY(logits_out(e, logits + (size_t)w * c.vocab, e->logits, (size_t)k * c.vocab * 4));
-      w += k;
-    }
-  }
-  return ti_stream_sync(e->s);
+  std::memcpy(e->in_pin, tokens, (size_t)n * 4);   // (free: every call that reads it ends with the stream's work done)
+  const int rc = prefill_rows(e, slot, n, pos0, pf, want, n_want, logits, layers_out);
+  if (rc != TI_OK) (void)hipStreamSynchronize(e->s);
+  return rc;
 }
 
 int ti_engine_destroy(ti_engine* e) {
@@ -1800,14 +1868,18 @@ static int step_rows(ti_engine* e, int n, const int32_t* slots, const int32_t* t
     rc = run_steps(e, n, 1, 1);
     e->slots_on = false;
   }
-  uint32_t* err = reinterpret_cast<uint32_t*>(e->in_pin + 3 * c.max_batch);
-  if (rc == TI_OK && n == 1) rc = qa_fault_read(e, err);
   if (rc != TI_OK) {
     (void)hipStreamSynchronize(e->s);
     return rc;
   }
   for (int m = 0; m < n; ++m) state_set(e, slots ? slots[m] : m, pos[m] + 1);
-  rc = logits ? logits_out(e, logits, e->logits, (size_t)n * c.vocab * 4) : ti_stream_sync(e->s);
+  uint32_t err[2] = {};
+  if (logits) {
+    rc = logits_out(e, logits, e->logits, (size_t)n * c.vocab * 4, n == 1 ? qa_fault_word(e) : nullptr, err);
+  } else {
+    if (n == 1) rc = qa_fault_read(e, err);
+    if (rc == TI_OK) rc = ti_stream_sync(e->s);
+  }
   if (rc != TI_OK) {
     (void)hipStreamSynchronize(e->s);
     return rc;
