@@ -166,3 +166,21 @@ def test_attention_partials_merged_by_o_projection(ti, oracle, heads, kv_heads, 
     bound = 2.5e-3 * (np.abs(xa) @ wf) + 1e-6
     err = np.abs(got - ref)
     assert np.all(err <= bound), f"max err {err.max()} (bound {bound.min()})"
+
+
+@pytest.mark.parametrize("bits", [4, 8, 16])
+@pytest.mark.parametrize("n", [2, 3, 16, 17, 48, 49, 64, 65])
+def test_prompt_fold(ti, bits, n):
+    """Prompts of up to 64 rows fold their norms: the logits of separate norms (fp16 rounds h * w before or behind the
+    division by the rms: a relative 2^-11 of each input either way, as between two kernels of the same product)."""
+    e = ti.Engine(512, 256, 3, 4, 2, 64, 512, bits=bits, max_seq=192, max_batch=2)
+    e.synth(11, 0.3)
+    t = (np.arange(n + 30) * 37 % 512).astype(np.int32)
+    got = []
+    for on in (1, 0):
+        ti.check(ti.lib().ti_engine_set_fold(e.h, on, None))
+        got.append(np.concatenate([e.prefill(0, t[:n], want=[0, n - 1]), e.prefill(0, t[n:], pos0=n)]))   # (a second one behind it)
+    assert np.linalg.norm(got[0] - got[1]) <= 4e-3 * np.linalg.norm(got[1])
+    if n > 64:
+        assert np.array_equal(got[0][:2], got[1][:2])
+    e.close()

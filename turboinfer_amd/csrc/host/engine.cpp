@@ -835,6 +835,29 @@ int enqueue_prefill(ti_engine* e, int m, int t0, int rows, int base, const int32
     return e->stack->forward(r, false, nullptr, nullptr, nullptr, 0);
   }
   const int H = c.hidden, qd = e->qd(), kvd = e->kvd(), I = c.inter;
+  // Few rows: the norms folded into O's and down's epilogues as in a batched step, two launches of 4 us less a layer (us,
+  // separate norms -> this, TinyLlama int8 prompts of 7 tokens 881 -> 777, 20 1009 -> 929, 64 1290 -> 1253).  Longer ones are bound by their products.
+  const bool bfold = bfold_usable(e, rows);
+  int n_ss = 0;
+  auto produce = [&](const DevLinear& W, const uint16_t* x, int ldx, const float* next) -> int {   // h += x W, folded for the norm `next`
+    ti_epilogue ep{};
+    ep.kind = TI_EPI_RESID_F32;
+    ep.ldo = H;
+    ep.out = e->h;
+    if (bfold && next) {
+      ep.fold_w = next;
+      ep.fold_x = e->xn;
+      ep.fold_ss = e->ss_rows;
+      n_ss = ti_gemm_rows_fold_partials(c.bits, rows, W.N, W.K, (int64_t)e->splitk_bytes);
+    }
+    return gemm_rows(e, W, rows, x, TI_X_F16, ldx, nullptr, ep, 4, false);
+  };
+  auto consume = [&](const DevLinear& W, const float* nw, ti_epilogue ep, size_t out_elem) -> int {   // the norm nw of h, W
+    if (n_ss == 0) return gemm_rows(e, W, rows, e->h, TI_X_F32_RMSNORM, H, nw, ep, out_elem, false);
+    ep.ss_in = e->ss_rows;
+    ep.n_ss = n_ss;
+    return gemm_rows(e, W, rows, e->xn, TI_X_F16, H, nw, ep, out_elem, false);
+  };
   for (int l = 0; l < c.layers; ++l) {
     DevLayer& L = e->layer[l];
     uint16_t* kc = L.kc + (size_t)m * e->kv_stride;
@@ -852,27 +875,19 @@ int enqueue_prefill(ti_engine* e, int m, int t0, int rows, int base, const int32
     ep.k_cache = kc;
     ep.v_cache = vc;
     ep.kv_stream_stride = 0;
-    TI_TRY(gemm_rows(e, L.qkv, rows, e->h, TI_X_F32_RMSNORM, H, L.attn_norm, ep, 4, false));
+    TI_TRY(consume(L.qkv, L.attn_norm, ep, 4));
     if (prefill_attn_on())   // one pass over the prefix per 16 rows (MFMA)
       TI_TRY(ti_attn_prefill_keys(e->q, kc, vc, c.max_seq, e->pos, rows, base + t0 + rows, c.heads, c.kv_heads, c.head_dim, e->attn, e->s));
     else
       TI_TRY(ti_attn_decode(e->q, kc, vc, 0, c.max_seq, e->pos, rows, c.heads, c.kv_heads, c.head_dim, e->splits_for(rows),
                             e->ws, e->attn, e->s));
-    ti_epilogue eo{};
-    eo.kind = TI_EPI_RESID_F32;
-    eo.ldo = H;
-    eo.out = e->h;
-    TI_TRY(gemm_rows(e, L.o, rows, e->attn, TI_X_F16, qd, nullptr, eo, 4, false));
+    TI_TRY(produce(L.o, e->attn, qd, L.ffn_norm));
     ti_epilogue eg{};
     eg.kind = TI_EPI_SILU_MUL_F16;
     eg.ldo = I;
     eg.out = e->act;
-    TI_TRY(gemm_rows(e, L.gu, rows, e->h, TI_X_F32_RMSNORM, H, L.ffn_norm, eg, 2, false));
-    ti_epilogue ed{};
-    ed.kind = TI_EPI_RESID_F32;
-    ed.ldo = H;
-    ed.out = e->h;
-    TI_TRY(gemm_rows(e, L.down, rows, e->act, TI_X_F16, I, nullptr, ed, 4, false));
+    TI_TRY(consume(L.gu, L.ffn_norm, eg, 2));
+    TI_TRY(produce(L.down, e->act, I, l + 1 < c.layers ? e->layer[l + 1].attn_norm : nullptr));
   }
   return TI_OK;
 }
