@@ -286,3 +286,23 @@ def test_route_tiles(ti, M, E, top, tile_rows):
     assert sorted(seen) == list(range(M * top))
     rows = tiles[:n, 2]
     assert (np.diff(rows) <= 0).all() and (rows == tile_rows).sum() == (counts // tile_rows).sum()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M", [1, 7, 8, 9, 15, 16])
+@pytest.mark.parametrize("N,K", [(16, 64), (1, 128), (23, 192), (64, 2048), (2041, 1088), (2048, 8192), (2049, 512)])
+def test_few_rows_halves(ti, dtype, M, N, K):
+    """Two k-tiles a product (dense_half_kernel, N <= 2048): one pair of them, fewer pairs than waves, ragged columns in
+    either half of a column tile, rows of one and of two products; added columns and untouched surroundings."""
+    a, w, f = operands(M, N, K, dtype)
+    add = torch.randn(N, device="cuda", generator=torch.Generator(device="cuda").manual_seed(5))
+    out = torch.full((M + 1, N + 3), 7.0, device="cuda")
+    d = ti.DenseArgs(w=f.data_ptr(), a=a.data_ptr(), out=out.data_ptr(), lda=K, ldo=N + 3, M=M, N=N, K=K, batch=1, epi=ti.DE_F32,
+                     dtype=ti.DT_BF16 if dtype == torch.bfloat16 else ti.DT_F32)
+    call(ti, d)
+    check(out[:M, :N], a, w[0], dtype)
+    plain = out[:M, :N].clone()
+    d.add = add.data_ptr()
+    call(ti, d)
+    assert torch.equal(out[:M, :N], plain + add)
+    assert (out[:, N:] == 7).all() and (out[M] == 7).all()
