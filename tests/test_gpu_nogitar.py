@@ -185,6 +185,17 @@ def test_convolution_taps(ti, taps, kind):
         e.close()
 
 
+@pytest.mark.parametrize("vdim,state", [(3, 5), (16, 64), (20, 120), (33, 130), (16, 256)])
+def test_step_inputs_of_two_rounds(ti, vdim, state):
+    """Known taps: 512 inputs of the convolution at once, a round more for the largest state; padded states."""
+    cfg = config(40, 32, [(mamba2(2, vdim, state, 1, 1, 4), None)])
+    w, t = random_weights(cfg, state), tokens(cfg, 12, 3)
+    ref = S.forward(t, f64(w), cfg)
+    e = build(ti, cfg, w, max_seq=16, max_batch=2)
+    close(np.concatenate([e.step([t[i], t[i]], [i, i]) for i in range(12)])[1::2], ref, "decoded")
+    e.close()
+
+
 # ------------------------------------------------------------------ whole models
 @pytest.mark.parametrize("name", ["mixed", "odd", "wide"])
 @pytest.mark.parametrize("n", [1, 2, 3, 15, 16, 17, 63, 64, 65, 128, 129])

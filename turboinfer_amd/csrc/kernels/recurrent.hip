@@ -117,15 +117,19 @@ __global__ __launch_bounds__(256) void conv_vec_kernel(const ti_conv_args a, int
 }
 
 // ------------------------------------------------------------------ SSD, one token per row
-// Grid (slices of ps value dimensions, heads, rows).  LPR lanes share a state row (4 elements each).
-template <class T, int LPR>
+// Grid (slices of ps value dimensions, heads, rows).  LPR lanes share a state row (4 elements each).  TP > 0: a.taps, known:
+// a thread's convolution inputs of two channels are in flight together, ahead of the state's (one tap after another each
+// waited for the last), and states of up to 256 take no loop over their pieces (92 -> 70 VGPRs).  Bound: the state's bytes
+// twice, and for few rows the launch with this chain of loads.  A step of Nogitar 2k (3 of them, 64 heads of 64 x 128): 8
+// streams 477 -> 469 us, 32 672 -> 653.  (8 waves a SIMD by spilling 12 bytes: no faster.)
+template <class T, int LPR, int TP>
 __global__ __launch_bounds__(256) void ssd_step_kernel(const ti_ssd_args a, int ps) {
   constexpr int RW = 64 / LPR, PF = 4;
   extern __shared__ float sh[];
   const int h = blockIdx.y, m = blockIdx.z, p0 = blockIdx.x * ps, N = a.state_n, np = (N + 3) & ~3, n4 = np >> 2;
   const int np_ = min(ps, a.vdim - p0), tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l = lane % LPR;
   const int hpg = a.heads / a.groups, grp = h / hpg, inner = a.heads * a.vdim, channels = inner + 2 * a.groups * N;
-  const int pos = a.pos[m], slot = a.slot ? a.slot[m] : m;
+  const int pos = __builtin_amdgcn_readfirstlane(a.pos[m]), slot = __builtin_amdgcn_readfirstlane(a.slot ? a.slot[m] : m);
   float *xs = sh, *bs = sh + ((ps + 3) & ~3), *cs = bs + np;
   f32x4* st = (f32x4*)(a.state + (((size_t)slot * a.heads + h) * a.vdim + p0) * np);
   const int q0 = min(l, n4 - 1), pr = wave * RW + lane / LPR;
@@ -136,41 +140,71 @@ __global__ __launch_bounds__(256) void ssd_step_kernel(const ti_ssd_args a, int 
 #pragma unroll
     for (int u = 0; u < PF; ++u) s[u] = pos > 0 ? st[(size_t)min(base + u * 4 * RW, np_ - 1) * n4 + q] : zero;
   };
-  load(pr, q0);
+  if constexpr (TP == 0) load(pr, q0);
   const T* raw = (const T*)a.a + (size_t)m * a.lda + inner;
   T* ring = (T*)a.ring + (size_t)slot * a.taps * channels;
-  for (int i = tid; i < np_ + 2 * np; i += 256) {
-    int c, own;
-    float* dst;
-    if (i < np_) {
-      c = h * a.vdim + p0 + i;
-      own = 1;
-      dst = xs + i;
-    } else {
-      const int j = i - np_, isc = j >= np, n = j - isc * np;
-      c = n < N ? inner + (isc * a.groups + grp) * N + n : -1;
-      own = blockIdx.x == 0 && h == grp * hpg;
-      dst = (isc ? cs : bs) + n;
+  const int places = np_ + 2 * np;
+  // input i: its LDS place is xs + i, with B and C behind the values' padding
+  const int gap = (int)(bs - xs) - np_;
+  const bool own_bc = blockIdx.x == 0 && h == grp * hpg;
+  auto channel = [&](int i) __attribute__((always_inline)) -> int {   // -1: padding
+    const int j = i - np_, isc = j >= np, n = j - isc * np;
+    return i < np_ ? h * a.vdim + p0 + i : n < N ? inner + (isc * a.groups + grp) * N + n : -1;
+  };
+  if constexpr (TP > 0) {
+    for (int i0 = tid; i0 == tid || i0 < places; i0 += 512) {
+      float w[2][TP], bias[2];
+      T x[2][TP];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const uint32_t k = (uint32_t)max(channel(min(i0 + 256 * u, places - 1)), 0);
+        // (uniform bases and 32-bit byte offsets: fewer registers, so more workgroups a CU)
+        auto at = [k]<class E>(const E* p) __attribute__((always_inline)) { return *(const E*)((const char*)p + k * (uint32_t)sizeof(E)); };
+        bias[u] = at(a.conv_b);
+        x[u][TP - 1] = at(raw);
+#pragma unroll
+        for (int t = 0; t < TP; ++t) w[u][t] = at(a.conv_w + (size_t)t * channels);
+#pragma unroll
+        for (int back = 1; back < TP; ++back) x[u][TP - 1 - back] = at((const T*)ring + (size_t)(max(pos - back, 0) % TP) * channels);
+      }
+      if (i0 == tid) load(pr, q0);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int i = i0 + 256 * u, c = channel(min(i, places - 1));
+        float v = bias[u];
+#pragma unroll
+        for (int back = TP - 1; back > 0; --back) v = pos >= back ? fmaf(w[u][TP - 1 - back], (float)x[u][TP - 1 - back], v) : v;
+        v = fmaf(w[u][TP - 1], (float)x[u][TP - 1], v);
+        v = c >= 0 ? (float)(T)(v * fast_sigmoid(v)) : 0.0f;
+        if (i < places) {
+          if (c >= 0 && (i < np_ || own_bc)) ring[(size_t)(pos % TP) * channels + c] = x[u][TP - 1];   // (a place that no sum takes)
+          xs[i < np_ ? i : i + gap] = v;
+        }
+      }
     }
-    float v = 0.0f;
-    if (c >= 0) {
-      v = a.conv_b[c];
-      const T cur = raw[c];
-      for (int back = a.taps - 1; back > 0; --back)
-        if (pos >= back)
-          v = fmaf(a.conv_w[(size_t)(a.taps - 1 - back) * channels + c], (float)ring[(size_t)((pos - back) % a.taps) * channels + c], v);
-      v = fmaf(a.conv_w[(size_t)(a.taps - 1) * channels + c], (float)cur, v);
-      // (the place written is read by no one: it held position pos - taps)
-      if (own) ring[(size_t)(pos % a.taps) * channels + c] = cur;
-      v = (float)(T)(v * fast_sigmoid(v));
+  } else {
+    for (int i = tid; i < places; i += 256) {
+      const int c = channel(i);
+      float v = 0.0f;
+      if (c >= 0) {
+        v = a.conv_b[c];
+        const T cur = raw[c];
+        for (int back = a.taps - 1; back > 0; --back)
+          if (pos >= back)
+            v = fmaf(a.conv_w[(size_t)(a.taps - 1 - back) * channels + c], (float)ring[(size_t)((pos - back) % a.taps) * channels + c], v);
+        v = fmaf(a.conv_w[(size_t)(a.taps - 1) * channels + c], (float)cur, v);
+        // (the place written is read by no one: it held position pos - taps)
+        if (i < np_ || own_bc) ring[(size_t)(pos % a.taps) * channels + c] = cur;
+        v = (float)(T)(v * fast_sigmoid(v));
+      }
+      xs[i < np_ ? i : i + gap] = v;
     }
-    *dst = v;
   }
   const float dt = softplusf(a.dt[(size_t)m * a.heads + h] + a.dt_bias[h]), decay = expf(-expf(a.a_log[h]) * dt), D = a.d[h];
   lds_sync();
   for (int base = pr; base - pr < np_; base += PF * 4 * RW) {
     float acc[PF] = {};
-    for (int q = l; q - l < n4; q += LPR) {   // (one pass unless the state is longer than 256)
+    for (int q = l; LPR < 64 ? q == l : q - l < n4; q += LPR) {   // (one pass unless the state is longer than 256)
       if (base != pr || q != l) load(base, min(q, n4 - 1));
       const bool on = q < n4;
       const f32x4 bq = *(const f32x4*)(bs + 4 * min(q, n4 - 1)) * dt, cq = *(const f32x4*)(cs + 4 * min(q, n4 - 1));
@@ -697,11 +731,15 @@ int launch_ssd_step(const ti_ssd_args& a, hipStream_t s) {
   const int ps = (long)a.M * a.heads >= 1024 ? std::min(a.vdim, 128) : 16;
   const dim3 grid((a.vdim + ps - 1) / ps, a.heads, a.M), blk(256);
   const size_t lds = (size_t)((ps + 3) / 4 * 4 + 2 * np) * 4;
-  if (n4 <= 4) hipLaunchKernelGGL((ssd_step_kernel<T, 4>), grid, blk, lds, s, a, ps);
-  else if (n4 <= 8) hipLaunchKernelGGL((ssd_step_kernel<T, 8>), grid, blk, lds, s, a, ps);
-  else if (n4 <= 16) hipLaunchKernelGGL((ssd_step_kernel<T, 16>), grid, blk, lds, s, a, ps);
-  else if (n4 <= 32) hipLaunchKernelGGL((ssd_step_kernel<T, 32>), grid, blk, lds, s, a, ps);
-  else hipLaunchKernelGGL((ssd_step_kernel<T, 64>), grid, blk, lds, s, a, ps);
+  auto run = [&]<int LPR>() {
+    if (a.taps == 4) hipLaunchKernelGGL((ssd_step_kernel<T, LPR, 4>), grid, blk, lds, s, a, ps);
+    else hipLaunchKernelGGL((ssd_step_kernel<T, LPR, 0>), grid, blk, lds, s, a, ps);
+  };
+  if (n4 <= 4) run.template operator()<4>();
+  else if (n4 <= 8) run.template operator()<8>();
+  else if (n4 <= 16) run.template operator()<16>();
+  else if (n4 <= 32) run.template operator()<32>();
+  else run.template operator()<64>();
   TI_LAUNCH_CHECK("ssd_step_kernel");
   return TI_OK;
 }
