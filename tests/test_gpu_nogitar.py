@@ -185,6 +185,18 @@ def test_convolution_taps(ti, taps, kind):
         e.close()
 
 
+@pytest.mark.parametrize("kv_heads", [1, 2, 3, 4, 8, 16])
+@pytest.mark.parametrize("n", [17, 130])
+def test_prompt_heads_on_xcds(ti, kv_heads, n):
+    """Heads that divide the 8 XCDs (each with every share-th tile group) and others (a run of the list): fewer groups than
+    XCDs of a head, one more than a multiple of them."""
+    cfg = config(40, 32, [(attn(2 * kv_heads if kv_heads < 16 else 16, kv_heads, 16, 24), None)])
+    w, t = random_weights(cfg, kv_heads), tokens(cfg, n, 6)
+    e = build(ti, cfg, w, max_seq=136, max_batch=1)
+    close(e.prefill(0, t, 0, range(n)), S.forward(t, f64(w), cfg), f"{kv_heads} heads")
+    e.close()
+
+
 @pytest.mark.parametrize("vdim,state", [(3, 5), (16, 64), (20, 120), (33, 130), (16, 256)])
 def test_step_inputs_of_two_rounds(ti, vdim, state):
     """Known taps: 512 inputs of the convolution at once, a round more for the largest state; padded states."""
