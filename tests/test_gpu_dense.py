@@ -306,3 +306,18 @@ def test_few_rows_halves(ti, dtype, M, N, K):
     call(ti, d)
     assert torch.equal(out[:M, :N], plain + add)
     assert (out[:, N:] == 7).all() and (out[M] == 7).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,N", [(2, 40), (7, 2048), (16, 1001), (16, 2064), (50, 300), (130, 300)])
+def test_shared_rows(ti, dtype, M, N):
+    """row_div without row lists: output row m is the product of row m / row_div of a, on the kernels of every row count."""
+    K, div = 320, 3
+    a, w, f = operands(M, N, K, dtype)
+    a = a[: (M - 1) // div + 1].contiguous()
+    out = torch.full((M + 1, N), 7.0, device="cuda")
+    d = ti.DenseArgs(w=f.data_ptr(), a=a.data_ptr(), out=out.data_ptr(), lda=K, ldo=N, M=M, N=N, K=K, batch=1, epi=ti.DE_F32, row_div=div,
+                     dtype=ti.DT_BF16 if dtype == torch.bfloat16 else ti.DT_F32)
+    call(ti, d)
+    check(out[:M], a[torch.arange(M, device="cuda") // div], w[0], dtype)
+    assert (out[M] == 7).all()

@@ -311,7 +311,7 @@ __global__ __launch_bounds__(64 * W) void dense_half_kernel(const ti_dense_args 
   const V* ap[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
-    ap[mt] = (const V*)((const T*)a.a + (size_t)min(mt * 8 + (lane & 7), a.M - 1) * a.lda + second * KT) + (lane >> 4);
+    ap[mt] = (const V*)((const T*)a.a + (size_t)row_in(a, min(mt * 8 + (lane & 7), a.M - 1)) * a.lda + second * KT) + (lane >> 4);
   f32x4 acc[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) acc[mt] = (f32x4){0.f, 0.f, 0.f, 0.f};
