@@ -107,6 +107,15 @@ def test_argument_errors_are_reported_without_launch(L):
     assert rc in (1, 3)
 
 
+def test_exchange_error_words_lie_in_the_buffer(L):
+    """The fused launch's two error words behind every number of splits, in the buffer that an engine keeps for the most."""
+    for f in (L.ti_qkv_attn_xchg_bytes, L.ti_qkv_attn_error_offset):
+        f.restype, f.argtypes = C.c_size_t, [C.c_int32, C.c_int32]
+    for heads in (1, 8, 32, 64):
+        for splits in range(1, 9):   # (TI_ATTN_MAX_PART_SPLITS)
+            assert L.ti_qkv_attn_error_offset(heads, splits) + 8 <= L.ti_qkv_attn_xchg_bytes(heads, 8)
+
+
 def test_engine_config_validation(L):
     cfg = T.EngineConfig(1000, 256, 2, 4, 4, 64, 512, 1e4, 1e-5, 4, 64, 1, 0, 0, 0)
     h = C.c_void_p()

@@ -395,13 +395,20 @@ bool part_usable(ti_engine* e, int M) {
 // new key never came (wrong results for that step) -- reported, and the exchange zeroed so the generations
 // agree again.  qa_fault_word: the two words on the device, or null for engines whose 1-stream steps do not take the launch.
 bool qa_usable(ti_engine* e, int M);
-const uint32_t* qa_fault_word(ti_engine* e) {
-  if (!e->qa_xchg || !qa_usable(e, 1)) return nullptr;
-  return reinterpret_cast<const uint32_t*>(static_cast<char*>(e->qa_xchg) + ti_qkv_attn_error_offset(e->c.heads, e->splits_for(1)));
+int qa_fault_word(ti_engine* e, const uint32_t** word) {
+  *word = nullptr;
+  if (!e->qa_xchg || !qa_usable(e, 1)) return TI_OK;
+  const size_t off = ti_qkv_attn_error_offset(e->c.heads, e->splits_for(1));
+  if (off + 8 > ti_qkv_attn_xchg_bytes(e->c.heads, TI_ATTN_MAX_PART_SPLITS))
+    return ti_set_error(TI_ERR_ARG, "engine: exchange error word outside the buffer");
+  *word = reinterpret_cast<const uint32_t*>(static_cast<char*>(e->qa_xchg) + off);
+  return TI_OK;
 }
 int qa_fault_read(ti_engine* e, uint32_t* err) {   // on the engine's stream
+  const uint32_t* w;
   err[0] = err[1] = 0u;
-  if (const uint32_t* w = qa_fault_word(e)) E_CHECK(hipMemcpyAsync(err, w, 8, hipMemcpyDeviceToHost, e->s), "hipMemcpyAsync(D2H)");
+  TI_TRY(qa_fault_word(e, &w));
+  if (w) E_CHECK(hipMemcpyAsync(err, w, 8, hipMemcpyDeviceToHost, e->s), "hipMemcpyAsync(D2H)");
   return TI_OK;
 }
 int qa_fault_report(ti_engine* e, const uint32_t* err) {
@@ -1890,7 +1897,9 @@ static int step_rows(ti_engine* e, int n, const int32_t* slots, const int32_t* t
   for (int m = 0; m < n; ++m) state_set(e, slots ? slots[m] : m, pos[m] + 1);
   uint32_t err[2] = {};
   if (logits) {
-    rc = logits_out(e, logits, e->logits, (size_t)n * c.vocab * 4, n == 1 ? qa_fault_word(e) : nullptr, err);
+    const uint32_t* word = nullptr;
+    if (n == 1) rc = qa_fault_word(e, &word);
+    if (rc == TI_OK) rc = logits_out(e, logits, e->logits, (size_t)n * c.vocab * 4, word, err);
   } else {
     if (n == 1) rc = qa_fault_read(e, err);
     if (rc == TI_OK) rc = ti_stream_sync(e->s);
