@@ -280,12 +280,13 @@ int ti_gemm_fold_partials(int bits, int M, int N, int K);
  * outputs; splits K with epi->splitk_ws.  ss_in / n_ss: x holds fp16(h * nw), outputs divided by the row's rms
  * (M <= TI_FOLD_SS_ROWS).  TI_EPI_RESID_F32 with fold_x: also the next call's folded input, rows of ldo, and
  * fold_ss[b * TI_FOLD_SS_ROWS + m], b < ti_gemm_rows_fold_partials(same call and workspace), negated where fp16 does not
- * hold the row's columns of the block: |h * fold_w| past 65504, or all of it below 2^-10. */
+ * hold the row's columns of the block: the mantissa's lowest bit clear where |h * fold_w| passes 65504, else set where its
+ * mean square is below 2^-22. */
 int ti_gemm_rows(const void* tiles, const uint16_t* scales, int bits, const void* x, int ldx, float eps, int M, int N, int K,
                  const ti_epilogue* epi, ti_stream_t s);
 /* ti_gemm_rows of a folded input (ss_in; no fold_x) and the rows h [M][K] and norm weight [K] (16-byte aligned) that x was
- * folded from: rows with a negative sum in ss_in are normalised before they are rounded, as ti_rmsnorm_f16 does it -- the
- * call rewrites them in x.  (ti_gemm_rows takes x as it is, and the sums by their magnitude.) */
+ * folded from: rows with a block past 65504, or more than half of whose n_ss blocks are small, are normalised before they are
+ * rounded, as ti_rmsnorm_f16 does it -- the call rewrites them in x.  (ti_gemm_rows takes x as it is, and the sums by their magnitude.) */
 int ti_gemm_rows_folded(const void* tiles, const uint16_t* scales, int bits, uint16_t* x, int ldx, const float* h, const float* norm_w,
                         float eps, int M, int N, int K, const ti_epilogue* epi, ti_stream_t s);
 int ti_gemm_rows_fold_partials(int bits, int M, int N, int K, int64_t ws_bytes);

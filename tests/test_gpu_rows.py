@@ -276,6 +276,47 @@ def test_rows_fold_range(ti, oracle, ws, bits, M):
     np.testing.assert_array_equal(*out)
 
 
+@pytest.mark.parametrize("bits", [4, 8, 16, 4 | G32])
+@pytest.mark.parametrize("M", [7, 24, 40, 64])
+def test_rows_fold_small_columns(ti, oracle, ws, bits, M):
+    """Small columns of a row are taken as they are unless most of the row is small, however wide the blocks that carry the marks
+    are.  Bound: fp16 inputs, half a unit in the last place of every h w (2^-11, or 2^-25 below the normal range, over the rms)
+    beside the fp32 sums; rows normalised first as in test_rows_fold_range."""
+    L, K, H, N = ti.lib(), 256, 1024, 208
+    rng = np.random.RandomState(M + bits)
+    to, so, wo = weight(ti, oracle, bits, K, H, rng)
+    t2, s2, w2 = weight(ti, oracle, bits, H, N, rng)
+    act = np.zeros((M, K), f16)
+    h = rng.standard_normal((M, H)).astype(f32)
+    nw = (1 + 0.1 * rng.standard_normal(H)).astype(f32)
+    h[1, 32:48] *= 1e-6    # a weight tile's columns
+    h[2, 128:192] *= 1e-6
+    h[3, :448] *= 1e-6     # nearly half
+    h[4] *= 1e-3           # (all of it just above 2^-11, with the columns of h w below 2^-10 in the majority)
+    h[5, 64:] *= 1e-6
+    h[M - 1] *= 2e-4
+    first = np.isin(np.arange(M), [5, M - 1])
+    n_ss = L.ti_gemm_rows_fold_partials(bits, M, H, K, WS)
+    hd, fx, ss, yd, nwd = dev(ti, h), ti.DeviceBuffer(M * H * 2), ti.DeviceBuffer(n_ss * 64 * 4), ti.DeviceBuffer(M * N * 4), dev(ti, nw)
+    ep = ti.Epilogue()
+    ep.kind, ep.ldo, ep.out = ti.EPI_RESID_F32, H, hd.ptr
+    ep.fold_w, ep.fold_x, ep.fold_ss = nwd.ptr, fx.ptr, ss.ptr
+    rows(ti, bits, to, so, dev(ti, act), M, H, K, ep, ws=ws)
+    np.testing.assert_allclose(np.abs(ss.download(f32, (n_ss, 64))[:, :M]).sum(axis=0), (h.astype(np.float64) ** 2).sum(axis=1), rtol=1e-5)
+    ep = ti.Epilogue()
+    ep.kind, ep.ldo, ep.out, ep.ss_in, ep.n_ss = ti.EPI_STORE_F32, N, yd.ptr, ss.ptr, n_ss
+    ep.splitk_ws, ep.splitk_bytes = ws.ptr, ws.nbytes
+    ti.check(L.ti_gemm_rows_folded(t2.ptr, s2.ptr, bits, fx.ptr, H, hd.ptr, nwd.ptr, 1e-5, M, N, H, C.byref(ep), None))
+    ti.sync()
+    plain = (h * nw).astype(f16).view(np.uint16)
+    np.testing.assert_array_equal((fx.download(np.uint16, (M, H)) != plain).any(axis=1), first)
+    rms = np.sqrt((h.astype(np.float64) ** 2).mean(axis=1) + 1e-5)[:, None]
+    x = h.astype(np.float64) / rms * nw
+    step = 2.0**-25 / np.where(first[:, None], 1.0, rms)
+    tol = (2.0**-11 + H * 2.0**-24) * (np.abs(x) @ np.abs(w2)) + step * np.abs(w2).sum(axis=0) + 1e-9
+    assert np.all(np.abs(yd.download(f32, (M, N)) - x @ w2.astype(np.float64)) <= tol)
+
+
 @pytest.mark.parametrize("bits", [4, 8, 16, 4 | G32, 8 | G32])
 def test_step_with_large_residuals(ti, bits):
     """An embedding whose product with the norm weight passes fp16's range: a step of 9 streams (batched fold) against the

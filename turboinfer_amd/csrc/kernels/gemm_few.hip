@@ -9,8 +9,8 @@ constexpr int kFewWaves = 8;
 template <int F, int TM, int TN>
 struct FewCfg {
   static constexpr int kRows = 16 * TM;
-  // rms per row and its shares | every wave's rows of a group | partial sums of every wave | each tile's staging block
-  static constexpr int kX = (kRows + kFewWaves * kWave) * 4, kRed = kX + kFewWaves * kRows * 256;
+  // rms per row, its shares and their marks | every wave's rows of a group | partial sums of every wave | each tile's staging block
+  static constexpr int kX = (kRows + 2 * kFewWaves * kWave) * 4, kRed = kX + kFewWaves * kRows * 256;
   static constexpr int kStg = kRed + kFewWaves * TN * TM * 1024, kSs = kStg + TN * kRows * kTileEpiStride * 4;
   static constexpr int kLds = kSs + TN * kRows * 8;
   static_assert(TN <= kFewWaves && kLds <= 160 * 1024);
@@ -182,10 +182,11 @@ __global__ __launch_bounds__(64 * kFewWaves, 2) void gemm_few_kernel(const GemvA
   };
   const bool fold_in = a.epi.ss_in != nullptr;
   float* rmsv = (float*)smem;
-  const float share = fold_in ? wide_fold_share(a, tid % C::kRows, tid / C::kRows, 64 * NW / C::kRows) : 0.0f;
+  uint32_t* const marks = (uint32_t*)rmsv + C::kRows + 64 * NW;
+  const float share = fold_in ? wide_fold_share(a, tid % C::kRows, tid / C::kRows, 64 * NW / C::kRows, marks + tid) : 0.0f;
   product();
   if (fold_in) {
-    wide_fold_rms<C::kRows, NW>(a, share, tid, rmsv);
+    wide_fold_rms<C::kRows, NW>(a, share, tid, rmsv, marks);
     const float mine = rmsv[lane % C::kRows];
     if (__builtin_expect(a.norm_w && __builtin_amdgcn_ballot_w64(__builtin_bit_cast(int32_t, mine) < 0) != 0, 0)) {
       // rows that fp16 did not hold: again, behind their rewriting
@@ -201,9 +202,9 @@ __global__ __launch_bounds__(64 * kFewWaves, 2) void gemm_few_kernel(const GemvA
   const bool fold_out = e.kind == TI_EPI_RESID_F32 && e.fold_x != nullptr;
   if (wave < TN) {
     const int t = wave, tn = t0 + t;
-    float hsq[TM], top[TM];
+    float hsq[TM], psq[TM];
 #pragma unroll
-    for (int b = 0; b < TM; ++b) hsq[b] = top[b] = 0.0f;
+    for (int b = 0; b < TM; ++b) hsq[b] = psq[b] = 0.0f;
     if (tn < NT) {
       f32x4 av[TM];
       const f32x4* red = (const f32x4*)(smem + C::kRed) + t * TM * 64 + lane;
@@ -222,13 +223,13 @@ __global__ __launch_bounds__(64 * kFewWaves, 2) void gemm_few_kernel(const GemvA
           stg[row * kTileEpiStride + r] = fold_in ? av[b][i] / fabsf(rmsv[row]) : av[b][i];
         }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      wide_tile_out<TM>(a, tn, 0, stg, lane, r, kq, fold_out, hsq, top);
+      wide_tile_out<TM>(a, tn, 0, stg, lane, r, kq, fold_out, hsq, psq);
     }
-    if (fold_out) wide_fold_part<TM>((float2*)(smem + C::kSs) + t * C::kRows, hsq, top, lane);
+    if (fold_out) wide_fold_part<TM>((float2*)(smem + C::kSs) + t * C::kRows, hsq, psq, lane);
   }
   if (fold_out) {
     lds_barrier();
-    wide_fold_store<C::kRows, TN>(a, (const float2*)(smem + C::kSs), cb, 0, tid);
+    wide_fold_store<C::kRows, TN, TN>(a, (const float2*)(smem + C::kSs), cb, 0, tid);
   }
   if (e.kind == TI_EPI_LOGITS_ARGMAX && e.step_ctr && cb == 0 && tid == 0) *e.step_ctr += e.advance;
   stamp_end(a.stamp, t_entry);

@@ -39,12 +39,13 @@ struct WideCfg {
   static constexpr int kScaleDma = W::kScale == 0 ? 0 : (TN * W::kScale + 255) / 256 * (W::kAff ? 2 : 1);   // dword DMAs per wave
   static constexpr int kS = kWaves * kScaleDma * 256;
   static constexpr int kStage = kA + kW + kS;
-  // after the stream: rms per row | each wave's staging block | (sum of h^2, largest |h w|) per column-wave and row | ticket
+  // after the stream: rms per row | each wave's staging block | (sum of h^2, of (h w)^2) per column-wave and row | ticket
   static constexpr int kEpiStg = kRows * 4, kEpiRed = kEpiStg + kWaves * 16 * TM * kTileEpiStride * 4;
   static constexpr int kEpiFlag = kEpiRed + 2 * WN * kRows * 4, kEpi = kEpiFlag + 16;
-  static constexpr int kLds = NS * kStage > kEpi ? NS * kStage : kEpi;
+  static constexpr int kMarks = NS * kStage > kEpi ? NS * kStage : kEpi;   // each thread's word of wide_fold_share
   static constexpr bool kFold = kRows <= TI_FOLD_SS_ROWS;   // (every wave of these has all rows)
   static_assert(!kFold || WM == 1, "a wave sees every row's rms");
+  static constexpr int kLds = kMarks + (kFold ? 64 * kWaves * 4 : 0);
   static constexpr int kDmaA = kRows / 4 / kWaves, kDmaW = kTiles * (W::kTile / 1024) / kWaves;
   static constexpr int kDma = kDmaA + kDmaW + kScaleDma;
   static_assert(kRows / 4 % kWaves == 0 && kTiles * (W::kTile / 1024) % kWaves == 0, "equal DMA counts per wave");
@@ -289,7 +290,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const GemvAr
   for (int s = 0; s < NS; ++s) issue(min(kb + s, ke - 1), s);
   // batched fold (decode rows, ti_hip.h TI_FOLD_SS_ROWS): this thread's share of its row's sum of squares
   const bool fold_in = C::kFold && a.epi.ss_in != nullptr;
-  const float share = fold_in ? wide_fold_share(a, m0 + tid % C::kRows, tid / C::kRows, 64 * NW / C::kRows) : 0.0f;
+  uint32_t* const marks = (uint32_t*)(smem + C::kMarks);
+  const float share = fold_in ? wide_fold_share(a, m0 + tid % C::kRows, tid / C::kRows, 64 * NW / C::kRows, marks + tid) : 0.0f;
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * C::kDma) : "memory");
   lds_barrier();
   Step st[2];
@@ -346,7 +348,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const GemvAr
 #pragma unroll
     for (int i = 0; i < 4; ++i) rms[b][i] = 1.0f;
   if (fold_in) {
-    wide_fold_rms<C::kRows, NW>(a, share, tid, rmsv);
+    wide_fold_rms<C::kRows, NW>(a, share, tid, rmsv, marks);
     uint32_t any = 0;
 #pragma unroll
     for (int b = 0; b < TM; ++b)
@@ -394,9 +396,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const GemvAr
   const bool fold_out = C::kFold && e.kind == TI_EPI_RESID_F32 && e.fold_x != nullptr;
   float* stg = (float*)(smem + C::kEpiStg) + wave * (16 * TM * kTileEpiStride);
   const int mb = m0 + wm * 16 * TM;
-  float hsq[TM], top[TM];
+  float hsq[TM], psq[TM];
 #pragma unroll
-  for (int b = 0; b < TM; ++b) hsq[b] = top[b] = 0.0f;
+  for (int b = 0; b < TM; ++b) hsq[b] = psq[b] = 0.0f;
 #pragma unroll 1
   for (int t = 0; t < TN; ++t) {   // (rolled: the tile's accumulators by static selects, so acc stays in registers)
     const int tn = t0 + wn * TN + t;
@@ -413,13 +415,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const GemvAr
       for (int i = 0; i < 4; ++i)
         stg[(b * 16 + 4 * kq + i) * kTileEpiStride + r] = fold_in ? av[b][i] / rms[b][i] : av[b][i];
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    wide_tile_out<TM>(a, tn, mb, stg, lane, r, kq, fold_out, hsq, top);
+    wide_tile_out<TM>(a, tn, mb, stg, lane, r, kq, fold_out, hsq, psq);
   }
   if (fold_out) {   // this column block's sum of h^2 per row, column-waves in order
     float2* red = (float2*)(smem + C::kEpiRed);
-    wide_fold_part<TM>(red + wn * C::kRows + wm * 16 * TM, hsq, top, lane);
+    wide_fold_part<TM>(red + wn * C::kRows + wm * 16 * TM, hsq, psq, lane);
     lds_barrier();
-    wide_fold_store<C::kRows, WN>(a, red, cb, m0, tid);
+    wide_fold_store<C::kRows, WN, C::kTiles>(a, red, cb, m0, tid);
   }
   if (e.kind == TI_EPI_LOGITS_ARGMAX && e.step_ctr && cb == 0 && rb == 0 && tid == 0) *e.step_ctr += e.advance;
   stamp_end(a.stamp, t_entry);

@@ -13,9 +13,18 @@ struct WideFmt {
   static constexpr int kScale = kBits == 16 ? 0 : kG32 ? 128 : 32;        // bytes of its scales
 };
 
-// Batched fold, consumer side: this thread's share of row m's partial sums of h^2 (part, part + P, ...), summed in order;
-// negative if one of them is.
-__device__ __forceinline__ float wide_fold_share(const GemvArgs& a, int m, int part, int P) {
+// Batched fold: a column block's sum of h^2 of a row is negative where fp16 does not hold its h w, the lowest bit of the
+// mantissa 0 where one of them passes 65504, 1 where they are small (wide_fold_store; an infinite sum counts as the former).
+// A row is normalised before it is rounded if one block of it is past 65504 or more than half of them are small: small ones
+// beside others are within the row's rounding, and what is done does not hang on the blocks' width.
+__device__ __forceinline__ float fold_mark(float t, bool over, bool small) {
+  const uint32_t b = __builtin_bit_cast(uint32_t, t);
+  if (over) return __builtin_bit_cast(float, (b & ~1u) | 0x80000000u);
+  return small ? __builtin_bit_cast(float, b | (t < INFINITY ? 0x80000001u : 0x80000000u)) : t;
+}
+// Consumer side: this thread's share of row m's partial sums (part, part + P, ...), summed in order; negative if one of them is,
+// and then *marks (LDS) counts the small ones, the top bit for one past 65504.
+__device__ __forceinline__ float wide_fold_share(const GemvArgs& a, int m, int part, int P, uint32_t* marks) {
   float t = 0.0f;
   uint32_t any = 0;
   if (m >= a.M) return t;
@@ -30,22 +39,44 @@ __device__ __forceinline__ float wide_fold_share(const GemvArgs& a, int m, int p
       any |= __builtin_bit_cast(uint32_t, v[j]);
     }
   }
-  return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, t) | (any & 0x80000000u));
+  any &= 0x80000000u;
+  if (__builtin_expect(any != 0, 0)) {
+    uint32_t n = 0, over = 0;
+#pragma unroll 8
+    for (int b = part; b < a.epi.n_ss; b += P) {
+      const uint32_t v = __builtin_bit_cast(uint32_t, ss[(size_t)b * TI_FOLD_SS_ROWS]);
+      n += v & (v >> 31);
+      over |= v & ~(v << 31);
+    }
+    *marks = n | (over & 0x80000000u);
+  }
+  return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, t) | any);
 }
-// The threads' shares to the rms of every row, negative as they are (behind a barrier; one follows).
+// The threads' shares to the rms of every row, negative where the row is to be normalised first (behind a barrier; one follows).
 template <int ROWS, int NW>
-__device__ __forceinline__ void wide_fold_rms(const GemvArgs& a, float share, int tid, float* rmsv) {
+__device__ __forceinline__ void wide_fold_rms(const GemvArgs& a, float share, int tid, float* rmsv, const uint32_t* marks) {
+  constexpr int P = 64 * NW / ROWS;
   rmsv[ROWS + tid] = share;
   lds_barrier();
   if (tid < ROWS) {
     float t = 0.0f;
     uint32_t any = 0;
-    for (int p = 0; p < 64 * NW / ROWS; ++p) {
+    for (int p = 0; p < P; ++p) {
       const float v = rmsv[ROWS + p * ROWS + tid];
       t += fabsf(v);
       any |= __builtin_bit_cast(uint32_t, v);
     }
-    rmsv[tid] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, sqrtf(t / (float)a.K + a.eps)) | (any & 0x80000000u));
+    float rms = sqrtf(t / (float)a.K + a.eps);
+    if (__builtin_expect((int32_t)any < 0, 0)) {
+      uint32_t n = 0, over = 0;
+      for (int p = 0; p < P; ++p) {
+        const uint32_t v = __builtin_bit_cast(int32_t, rmsv[ROWS + p * ROWS + tid]) < 0 ? marks[p * ROWS + tid] : 0u;
+        n += v & 0xffffu;
+        over |= v;
+      }
+      if ((int32_t)over < 0 || 2 * (int)n > a.epi.n_ss) rms = -rms;
+    }
+    rmsv[tid] = rms;
   }
   lds_barrier();
 }
@@ -73,10 +104,11 @@ __device__ __forceinline__ void wide_refold(const GemvArgs& a, int wave, int lan
 }
 
 // One weight tile's outputs (16 columns from tn) for the 16 TM rows from mb, from the wave's staging block.  fold_out: the
-// residual add and the next call's folded input; hsq, top: the lane's sums of h^2 and largest |h w| (wide_fold_part).
+// residual add and the next call's folded input; hsq, psq: the lane's sums of h^2 and of (h w)^2, the latter infinite where an
+// |h w| passes 65504 (wide_fold_part).
 template <int TM>
 __device__ __forceinline__ void wide_tile_out(const GemvArgs& a, int tn, int mb, const float* stg, int lane, int r, int kq, bool fold_out,
-                                              float (&hsq)[TM], float (&top)[TM]) {
+                                              float (&hsq)[TM], float (&psq)[TM]) {
   const ti_epilogue& e = a.epi;
   if (fold_out) {   // residual add + the next call's folded input (fp16(h * w), sum of h^2 per row)
     const int c4 = 4 * (lane & 3), ng = tn * 16 + c4;
@@ -92,10 +124,12 @@ __device__ __forceinline__ void wide_tile_out(const GemvArgs& a, int tn, int mb,
         *o = h;
         float p[4] = {h.x * w.x, h.y * w.y, h.z * w.z, h.w * w.w};
         // (largest |p|; as outputs the products are rounded on their own, as in mul_f16)
-        asm("v_max3_f32 %0, %0, |%1|, |%2|\n\tv_max3_f32 %0, %0, |%3|, |%4|" : "+v"(top[it]), "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]));
+        float top = 0.0f;
+        asm("v_max3_f32 %0, %0, |%1|, |%2|\n\tv_max3_f32 %0, %0, |%3|, |%4|" : "+v"(top), "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]));
         auto f = [](float v) { return (uint32_t)f2h(v); };
         *(uint2*)(e.fold_x + (size_t)m * e.ldo + ng) = make_uint2(f(p[0]) | (f(p[1]) << 16), f(p[2]) | (f(p[3]) << 16));
         q = (h.x * h.x + h.y * h.y) + (h.z * h.z + h.w * h.w);
+        psq[it] = top > 65504.0f ? INFINITY : psq[it] + ((p[0] * p[0] + p[1] * p[1]) + (p[2] * p[2] + p[3] * p[3]));
       }
       q += lane_xor<1>(q);
       hsq[it] += q + lane_xor<2>(q);
@@ -110,28 +144,30 @@ __device__ __forceinline__ void wide_tile_out(const GemvArgs& a, int tn, int mb,
     }
   }
 }
-// The wave's (sum of h^2, largest |h w|) of its 16 TM rows to part.
+// The wave's sums of its 16 TM rows to part.
 template <int TM>
-__device__ __forceinline__ void wide_fold_part(float2* part, const float (&hsq)[TM], const float (&top)[TM], int lane) {
+__device__ __forceinline__ void wide_fold_part(float2* part, const float (&hsq)[TM], const float (&psq)[TM], int lane) {
 #pragma unroll
   for (int it = 0; it < TM; ++it) {
-    const float t2 = fmaxf(top[it], lane_xor<1>(top[it])), t4 = fmaxf(t2, lane_xor<2>(t2));
-    if ((lane & 3) == 0) part[16 * it + (lane >> 2)] = make_float2(hsq[it], t4);
+    const float p2 = psq[it] + lane_xor<1>(psq[it]), p4 = p2 + lane_xor<2>(p2);
+    if ((lane & 3) == 0) part[16 * it + (lane >> 2)] = make_float2(hsq[it], p4);
   }
 }
-// The W parts of a column block (behind a barrier), in order, to fold_ss.
-template <int ROWS, int W>
+// The W parts of a block of TILES weight tiles (behind a barrier), in order, to fold_ss.  Small: their mean square below 2^-22.
+// A row that is taken as it is has a mean square of 2^-23 at least, so fp16's steps of 2^-24 (an error of 2^-25 / sqrt 3 rms) are
+// 5e-5 of it, beside 2e-4 by which fp16 rounds larger values.
+template <int ROWS, int W, int TILES>
 __device__ __forceinline__ void wide_fold_store(const GemvArgs& a, const float2* part, int cb, int m0, int tid) {
   if (tid >= ROWS || m0 + tid >= a.M) return;
-  float t = 0.0f, mx = 0.0f;
+  float t = 0.0f, p = 0.0f;
 #pragma unroll
   for (int w = 0; w < W; ++w) {
     const float2 v = part[w * ROWS + tid];
     t += v.x;
-    mx = fmaxf(mx, v.y);
+    p += v.y;
   }
-  // negative where fp16(h w) is infinite, or all so small that its steps of 2^-24 are not far below 2^-12 of the largest
-  a.epi.fold_ss[(size_t)cb * TI_FOLD_SS_ROWS + m0 + tid] = mx > 65504.0f || mx < 0x1p-10f ? -t : t;
+  const int cols = min(16 * TILES, a.N - cb * 16 * TILES);
+  a.epi.fold_ss[(size_t)cb * TI_FOLD_SS_ROWS + m0 + tid] = fold_mark(t, p == INFINITY, p < (float)cols * 0x1p-22f);
 }
 
 struct WidePlan {
