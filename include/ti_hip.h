@@ -290,6 +290,12 @@ int ti_gemm_rows(const void* tiles, const uint16_t* scales, int bits, const void
 int ti_gemm_rows_folded(const void* tiles, const uint16_t* scales, int bits, uint16_t* x, int ldx, const float* h, const float* norm_w,
                         float eps, int M, int N, int K, const ti_epilogue* epi, ti_stream_t s);
 int ti_gemm_rows_fold_partials(int bits, int M, int N, int K, int64_t ws_bytes);
+/* The same calls on a kernel of the caller's choice (parity tests and comparisons; h NULL: ti_gemm_rows, else
+ * ti_gemm_rows_folded).  TI_ERR_UNSUPPORTED (0 partials) where it does not take the call: the few-rows kernel has up to 48 rows. */
+enum ti_rows_kernel { TI_ROWS_AUTO = 0, TI_ROWS_FEW, TI_ROWS_MANY };
+int ti_gemm_rows_on(int kernel, const void* tiles, const uint16_t* scales, int bits, uint16_t* x, int ldx, const float* h,
+                    const float* norm_w, float eps, int M, int N, int K, const ti_epilogue* epi, ti_stream_t s);
+int ti_gemm_rows_fold_partials_on(int kernel, int bits, int M, int N, int K, int64_t ws_bytes);
 /* One-time kernel attribute setup; call before capturing ti_gemm_wq_a16 into a graph. */
 int ti_gemm_prepare(void);
 

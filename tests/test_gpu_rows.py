@@ -1,5 +1,6 @@
-"""The many-rows GEMM (ti_gemm_rows, gemm_wide.hip): row-major fp16 rows against packed weights of every format,
-against the weights' exact values in float64 (test_gpu_kernels.py's bound: fp32 summation order)."""
+"""ti_gemm_rows: row-major fp16 rows against packed weights of every format, against the weights' exact values in float64
+(test_gpu_kernels.py's bound: fp32 summation order).  Calls of up to 48 rows run on both of its kernels, the few-rows one
+(gemm_few.hip) and the many-rows one (gemm_wide.hip), whichever the call itself would take."""
 from __future__ import annotations
 
 import ctypes as C
@@ -33,10 +34,13 @@ def weight(ti, oracle, bits, K, N, rng):
     return dev(ti, t), dev(ti, s), w.astype(f16).astype(f32) if bits == 16 else deq(oracle, w, bits)
 
 
-def rows(ti, bits, td, sd, xd, M, N, K, ep, ldx=None, ws=None):
-    if ws is not None:
-        ep.splitk_ws, ep.splitk_bytes = ws.ptr, ws.nbytes
-    rc = ti.lib().ti_gemm_rows(td.ptr, sd.ptr, bits, xd.ptr, ldx or K, 1e-5, M, N, K, C.byref(ep), None)
+def kernels(ti, M):
+    return (ti.ROWS_FEW, ti.ROWS_MANY) if M <= 48 else (ti.ROWS_AUTO,)
+
+
+def rows(ti, bits, td, sd, xd, M, N, K, ep, ldx=None, ws=None, kernel=0, h=None, norm_w=None):
+    ep.splitk_ws, ep.splitk_bytes = (ws.ptr, ws.nbytes) if ws is not None else (None, 0)
+    rc = ti.lib().ti_gemm_rows_on(kernel, td.ptr, sd.ptr, bits, xd.ptr, ldx or K, h, norm_w, 1e-5, M, N, K, C.byref(ep), None)
     ti.check(rc)
     ti.sync()
     if ws is not None:
@@ -57,12 +61,13 @@ def test_rows_store(ti, oracle, ws, bits, M, K, N):
     xd, yd = dev(ti, x), ti.DeviceBuffer(M * N * 4)
     xa = x[:, :K].astype(f32)
     ref = xa.astype(np.float64) @ w.astype(np.float64)
-    for k in (None, ws):
-        yd.zero()
-        ep = ti.Epilogue()
-        ep.kind, ep.ldo, ep.out = ti.EPI_STORE_F32, N, yd.ptr
-        rows(ti, bits, td, sd, xd, M, N, K, ep, ldx, k)
-        assert_close_dot(yd.download(f32, (M, N)), ref, xa, w)
+    for kernel in kernels(ti, M):
+        for k in (None, ws):
+            yd.zero()
+            ep = ti.Epilogue()
+            ep.kind, ep.ldo, ep.out = ti.EPI_STORE_F32, N, yd.ptr
+            rows(ti, bits, td, sd, xd, M, N, K, ep, ldx, k, kernel)
+            assert_close_dot(yd.download(f32, (M, N)), ref, xa, w)
 
 
 # the few-rows kernel (gemm_few.hip): rows at the edges of its 16-, 32- and 48-row blocks, waves without a group of k (K below
@@ -79,28 +84,32 @@ def test_rows_few(ti, oracle, bits, M, K, N):
     yd.zero()
     ep = ti.Epilogue()
     ep.kind, ep.ldo, ep.out = ti.EPI_STORE_F32, N, yd.ptr
-    rows(ti, bits, td, sd, xd, M, N, K, ep, ldx)
+    rows(ti, bits, td, sd, xd, M, N, K, ep, ldx, kernel=ti.ROWS_FEW)
     y, xa = yd.download(f32, (M + 1, N)), x[:, :K].astype(f32)
     assert_close_dot(y[:M], xa.astype(np.float64) @ w.astype(np.float64), xa, w)
     assert not y[M].any()
 
 
-def test_rows_affine_blocks(ti, oracle, ws):
+# (24 .. 47 rows by the few-rows kernel: waves with none to five groups of k, its 16- and 32-column blocks with a ragged last one)
+@pytest.mark.parametrize("M,K,N", [(24, 384, 96), (100, 1152, 1040), (700, 2048, 512), (3, 2176, 4112), (16, 5120, 4112), (31, 2176, 4112),
+                                   (47, 5120, 272)])
+def test_rows_affine_blocks(ti, oracle, ws, M, K, N):
     """Q4_1 blocks (4 | 32 | 64): the offset term through the block's sum of x."""
     from test_gpu_g32 import pack_q1
-    for M, K, N in [(24, 384, 96), (100, 1152, 1040), (700, 2048, 512)]:
-        rng = np.random.RandomState(M)
-        q = rng.randint(0, 16, (K, N)).astype(np.uint8)
-        d = (rng.uniform(0.5, 1.5, (K // 32, N)) * 0.01).astype(f16)
-        m = (rng.standard_normal((K // 32, N)) * 0.05).astype(f16)
-        td, sd = pack_q1(ti, q, d, m)
-        w = np.repeat(d.astype(np.float64), 32, 0) * q + np.repeat(m.astype(np.float64), 32, 0)
-        parts = np.repeat(np.abs(d.astype(np.float64)), 32, 0) * 16 + np.repeat(np.abs(m.astype(np.float64)), 32, 0)
-        x = rng.standard_normal((M, K)).astype(f16)
-        yd = ti.DeviceBuffer(M * N * 4)
+    rng = np.random.RandomState(M)
+    q = rng.randint(0, 16, (K, N)).astype(np.uint8)
+    d = (rng.uniform(0.5, 1.5, (K // 32, N)) * 0.01).astype(f16)
+    m = (rng.standard_normal((K // 32, N)) * 0.05).astype(f16)
+    td, sd = pack_q1(ti, q, d, m)
+    w = np.repeat(d.astype(np.float64), 32, 0) * q + np.repeat(m.astype(np.float64), 32, 0)
+    parts = np.repeat(np.abs(d.astype(np.float64)), 32, 0) * 16 + np.repeat(np.abs(m.astype(np.float64)), 32, 0)
+    x = rng.standard_normal((M, K)).astype(f16)
+    xd, yd = dev(ti, x), ti.DeviceBuffer(M * N * 4)
+    for kernel in kernels(ti, M):
+        yd.zero()
         ep = ti.Epilogue()
         ep.kind, ep.ldo, ep.out = ti.EPI_STORE_F32, N, yd.ptr
-        rows(ti, 4 | G32 | 64, td, sd, dev(ti, x), M, N, K, ep, ws=ws)
+        rows(ti, 4 | G32 | 64, td, sd, xd, M, N, K, ep, ws=ws, kernel=kernel)
         # fp32 sums of d (q - 8) x and (8 d + m) x: the bound is on the parts' magnitudes
         assert np.all(np.abs(yd.download(f32, (M, N)) - x.astype(np.float64) @ w) <= 2e-5 * (np.abs(x.astype(np.float64)) @ parts) + 1e-6)
 
@@ -115,12 +124,12 @@ def test_rows_epilogues(ti, oracle, ws, bits, M):
     x = rng.standard_normal((M, K)).astype(f16)
     xd, xa = dev(ti, x), x.astype(np.float64)
     ref = xa @ w.astype(np.float64)
-    for ldo in (N, N + 3):
+    for kernel, ldo in [(k, l) for k in kernels(ti, M) for l in (N, N + 3)]:
         r = rng.standard_normal((M, ldo)).astype(f32)
         rd = dev(ti, r)
         ep = ti.Epilogue()
         ep.kind, ep.ldo, ep.out = ti.EPI_RESID_F32, ldo, rd.ptr
-        rows(ti, bits, td, sd, xd, M, N, K, ep, ws=ws)
+        rows(ti, bits, td, sd, xd, M, N, K, ep, ws=ws, kernel=kernel)
         got = rd.download(f32, (M, ldo))
         assert_close_dot(got[:, :N] - r[:, :N], ref, x.astype(f32), w, rel=5e-5)
         np.testing.assert_array_equal(got[:, N:], r[:, N:])
@@ -129,20 +138,21 @@ def test_rows_epilogues(ti, oracle, ws, bits, M):
         hd = ti.DeviceBuffer(M * ldo * 2)
         ep = ti.Epilogue()
         ep.kind, ep.ldo, ep.out = ti.EPI_SILU_MUL_F16, ldo, hd.ptr
-        rows(ti, bits, td, sd, xd, M, N, K, ep, ws=ws)
+        rows(ti, bits, td, sd, xd, M, N, K, ep, ws=ws, kernel=kernel)
         np.testing.assert_allclose(hd.download(f16, (M, ldo))[:, : N // 2].astype(np.float64), sil, rtol=3e-3, atol=2e-3)
         ep.kind = ti.EPI_STORE_F16
-        rows(ti, bits, td, sd, xd, M, N, K, ep, ws=ws)
+        rows(ti, bits, td, sd, xd, M, N, K, ep, ws=ws, kernel=kernel)
         np.testing.assert_allclose(hd.download(f16, (M, ldo))[:, :N].astype(np.float64), ref, rtol=2e-3, atol=1e-4)
-    ld, am = ti.DeviceBuffer(M * N * 4), ti.DeviceBuffer(M * ti.ARGMAX_SLOTS * 8)
-    am.zero()
-    ep = ti.Epilogue()
-    ep.kind, ep.ldo, ep.out, ep.argmax = ti.EPI_LOGITS_ARGMAX, N, ld.ptr, am.ptr
-    rows(ti, bits, td, sd, xd, M, N, K, ep, ws=ws)
-    lg = ld.download(f32, (M, N))
-    keys = am.download(np.uint64, (M, ti.ARGMAX_SLOTS)).max(axis=1)
-    np.testing.assert_array_equal((0xFFFFFFFF - (keys & 0xFFFFFFFF)).astype(np.int64), np.argmax(lg, axis=1))
-    np.testing.assert_allclose(lg, ref, rtol=1e-4, atol=1e-4)
+    for kernel in kernels(ti, M):
+        ld, am = ti.DeviceBuffer(M * N * 4), ti.DeviceBuffer(M * ti.ARGMAX_SLOTS * 8)
+        am.zero()
+        ep = ti.Epilogue()
+        ep.kind, ep.ldo, ep.out, ep.argmax = ti.EPI_LOGITS_ARGMAX, N, ld.ptr, am.ptr
+        rows(ti, bits, td, sd, xd, M, N, K, ep, ws=ws, kernel=kernel)
+        lg = ld.download(f32, (M, N))
+        keys = am.download(np.uint64, (M, ti.ARGMAX_SLOTS)).max(axis=1)
+        np.testing.assert_array_equal((0xFFFFFFFF - (keys & 0xFFFFFFFF)).astype(np.int64), np.argmax(lg, axis=1))
+        np.testing.assert_allclose(lg, ref, rtol=1e-4, atol=1e-4)
 
 
 @pytest.mark.parametrize("hd,M", [(64, 21), (128, 70)])
@@ -158,15 +168,15 @@ def test_rows_qkv(ti, oracle, ws, hd, M):
     pd = dev(ti, pos)
     cs = dev(ti, ti.rope_table(np.arange(S), hd, 10000.0))
     outs = []
-    for wide in (True, False):
+    for kernel in kernels(ti, M) + (None,):
         q, k, v = ti.DeviceBuffer(M * qd * 4), ti.DeviceBuffer(kvh * S * hd * 2), ti.DeviceBuffer(kvh * S * hd * 2)
         for b in (k, v):
             b.zero()
         ep = ti.Epilogue()
         ep.kind, ep.ldo, ep.out, ep.q_dim, ep.kv_dim, ep.head_dim, ep.max_seq = ti.EPI_QKV_ROPE_KV, qd, q.ptr, qd, kd, hd, S
         ep.pos, ep.rope_cs, ep.k_cache, ep.v_cache, ep.kv_stream_stride = pd.ptr, cs.ptr, k.ptr, v.ptr, 0
-        if wide:
-            rows(ti, 8, td, sd, xd, M, N, K, ep, ws=ws)
+        if kernel is not None:
+            rows(ti, 8, td, sd, xd, M, N, K, ep, ws=ws, kernel=kernel)
         else:
             for m in range(0, M, 16):
                 ep.out, ep.pos = q.ptr + m * qd * 4, pd.ptr + 4 * m
@@ -174,8 +184,9 @@ def test_rows_qkv(ti, oracle, ws, hd, M):
                                                  C.byref(ep), None))
             ti.sync()
         outs.append([q.download(f32, (M, qd)), k.download(f16, (kvh, S, hd)).astype(f32), v.download(f16, (kvh, S, hd)).astype(f32)])
-    for a, b in zip(*outs):
-        np.testing.assert_allclose(a, b, rtol=2e-3, atol=2e-3)
+    for out in outs[:-1]:
+        for a, b in zip(out, outs[-1]):
+            np.testing.assert_allclose(a, b, rtol=2e-3, atol=2e-3)
 
 
 @pytest.mark.parametrize("bits", [4, 8, 16, 4 | G32])
@@ -189,29 +200,30 @@ def test_rows_fold(ti, oracle, ws, bits, M):
     act = rng.standard_normal((M, K)).astype(f16)
     h0 = rng.standard_normal((M, H)).astype(f32)
     nw = (1 + 0.1 * rng.standard_normal(H)).astype(f32)
-    n_ss = L.ti_gemm_rows_fold_partials(bits, M, H, K, WS)
-    assert 1 <= n_ss <= 4096
-    bits_out = []
-    for _ in range(2):
-        hd, fx, ss, yd = dev(ti, h0), ti.DeviceBuffer(M * H * 2), ti.DeviceBuffer(n_ss * 64 * 4), ti.DeviceBuffer(M * N * 4)
-        nwd = dev(ti, nw)
-        ep = ti.Epilogue()
-        ep.kind, ep.ldo, ep.out = ti.EPI_RESID_F32, H, hd.ptr
-        ep.fold_w, ep.fold_x, ep.fold_ss = nwd.ptr, fx.ptr, ss.ptr
-        rows(ti, bits, to, so, dev(ti, act), M, H, K, ep, ws=ws)
-        h1 = hd.download(f32, (M, H))
-        assert_close_dot(h1 - h0, act.astype(np.float64) @ wo.astype(np.float64), act.astype(f32), wo, rel=5e-5)
-        np.testing.assert_array_equal(fx.download(np.uint16, (M, H)), (h1 * nw).astype(f16).view(np.uint16))
-        np.testing.assert_allclose(ss.download(f32, (n_ss, 64))[:, :M].sum(axis=0), (h1.astype(np.float64) ** 2).sum(axis=1), rtol=1e-5)
-        ep = ti.Epilogue()
-        ep.kind, ep.ldo, ep.out, ep.ss_in, ep.n_ss = ti.EPI_STORE_F32, N, yd.ptr, ss.ptr, n_ss
-        rows(ti, bits, t2, s2, fx, M, N, H, ep, ws=ws)
-        y = yd.download(f32, (M, N))
-        bits_out.append(y.view(np.uint32))
-    rms = np.sqrt((h1.astype(np.float64) ** 2).mean(axis=1) + 1e-5)
-    xf = (h1 * nw).astype(f16).astype(np.float64) / rms[:, None]
-    assert_close_dot(y, xf @ w2.astype(np.float64), xf.astype(f32), w2, rel=5e-5)
-    np.testing.assert_array_equal(*bits_out)   # fixed-order sums
+    ad, nwd = dev(ti, act), dev(ti, nw)
+    for kernel, k in [(a, b) for a in kernels(ti, M) for b in (ws, None)]:   # (the many-rows kernel splits K with a workspace)
+        n_ss = L.ti_gemm_rows_fold_partials_on(kernel, bits, M, H, K, WS if k else 0)
+        assert 1 <= n_ss <= 4096
+        bits_out = []
+        for _ in range(2):
+            hd, fx, ss, yd = dev(ti, h0), ti.DeviceBuffer(M * H * 2), ti.DeviceBuffer(n_ss * 64 * 4), ti.DeviceBuffer(M * N * 4)
+            ep = ti.Epilogue()
+            ep.kind, ep.ldo, ep.out = ti.EPI_RESID_F32, H, hd.ptr
+            ep.fold_w, ep.fold_x, ep.fold_ss = nwd.ptr, fx.ptr, ss.ptr
+            rows(ti, bits, to, so, ad, M, H, K, ep, ws=k, kernel=kernel)
+            h1 = hd.download(f32, (M, H))
+            assert_close_dot(h1 - h0, act.astype(np.float64) @ wo.astype(np.float64), act.astype(f32), wo, rel=5e-5)
+            np.testing.assert_array_equal(fx.download(np.uint16, (M, H)), (h1 * nw).astype(f16).view(np.uint16))
+            np.testing.assert_allclose(ss.download(f32, (n_ss, 64))[:, :M].sum(axis=0), (h1.astype(np.float64) ** 2).sum(axis=1), rtol=1e-5)
+            ep = ti.Epilogue()
+            ep.kind, ep.ldo, ep.out, ep.ss_in, ep.n_ss = ti.EPI_STORE_F32, N, yd.ptr, ss.ptr, n_ss
+            rows(ti, bits, t2, s2, fx, M, N, H, ep, ws=k, kernel=kernel)
+            y = yd.download(f32, (M, N))
+            bits_out.append(y.view(np.uint32))
+        rms = np.sqrt((h1.astype(np.float64) ** 2).mean(axis=1) + 1e-5)
+        xf = (h1 * nw).astype(f16).astype(np.float64) / rms[:, None]
+        assert_close_dot(y, xf @ w2.astype(np.float64), xf.astype(f32), w2, rel=5e-5)
+        np.testing.assert_array_equal(*bits_out)   # fixed-order sums
 
 
 def test_rows_refusals(ti):
@@ -224,6 +236,10 @@ def test_rows_refusals(ti):
         a = list(ok)
         a[i] = v
         assert L.ti_gemm_rows(*a, C.byref(ep), None) != 0, (i, v)
+    on = (b.ptr, b.ptr, 8, b.ptr, 256, None, None, 1e-5)
+    for kernel, M in [(3, 4), (-1, 4), (ti.ROWS_FEW, 49)]:
+        assert L.ti_gemm_rows_on(kernel, *on, M, 64, 256, C.byref(ep), None) != 0
+        assert L.ti_gemm_rows_fold_partials_on(kernel, 8, M, 64, 256, 0) == 0
     ep.kind, ep.fold_x = ti.EPI_RESID_F32, b.ptr
     assert L.ti_gemm_rows(*ok, C.byref(ep), None) != 0
 
@@ -253,27 +269,27 @@ def test_rows_fold_range(ti, oracle, ws, bits, M):
     act[2] = 0
     h0[4], act[4] = 0, 0
     bad = np.isin(np.arange(M), [1, 2, 4, M - 1])
-    n_ss = L.ti_gemm_rows_fold_partials(bits, M, H, K, WS)
-    hd, fx, ss, yd, nwd = dev(ti, h0), ti.DeviceBuffer(M * H * 2), ti.DeviceBuffer(n_ss * 64 * 4), ti.DeviceBuffer(M * N * 4), dev(ti, nw)
-    out = []
-    for _ in range(2):   # (the second call over rows that the first rewrote)
-        ti.check(L.ti_memcpy_h2d(hd.ptr, h0.ctypes.data_as(C.c_void_p), h0.nbytes, None))
-        ep = ti.Epilogue()
-        ep.kind, ep.ldo, ep.out = ti.EPI_RESID_F32, H, hd.ptr
-        ep.fold_w, ep.fold_x, ep.fold_ss = nwd.ptr, fx.ptr, ss.ptr
-        rows(ti, bits, to, so, dev(ti, act), M, H, K, ep, ws=ws)
-        np.testing.assert_array_equal(np.signbit(ss.download(f32, (n_ss, 64))[:, :M]).any(axis=0), bad)
-        h1 = hd.download(f32, (M, H)).astype(np.float64)
-        ep = ti.Epilogue()
-        ep.kind, ep.ldo, ep.out, ep.ss_in, ep.n_ss = ti.EPI_STORE_F32, N, yd.ptr, ss.ptr, n_ss
-        ep.splitk_ws, ep.splitk_bytes = ws.ptr, ws.nbytes
-        ti.check(L.ti_gemm_rows_folded(t2.ptr, s2.ptr, bits, fx.ptr, H, hd.ptr, nwd.ptr, 1e-5, M, N, H, C.byref(ep), None))
-        ti.sync()
-        out.append(yd.download(f32, (M, N)))
-    x = h1 / np.sqrt((h1**2).mean(axis=1) + 1e-5)[:, None] * nw
-    err = np.abs(out[0] - x @ w2.astype(np.float64))
-    assert np.all(err <= (2.0**-11 + H * 2.0**-24) * (np.abs(x) @ np.abs(w2)) + 2.0**-25 * np.abs(w2).sum(axis=0) + 1e-9)
-    np.testing.assert_array_equal(*out)
+    ad, nwd = dev(ti, act), dev(ti, nw)
+    for kernel, k in [(a, b) for a in kernels(ti, M) for b in (ws, None)]:
+        n_ss = L.ti_gemm_rows_fold_partials_on(kernel, bits, M, H, K, WS if k else 0)
+        hd, fx, ss, yd = dev(ti, h0), ti.DeviceBuffer(M * H * 2), ti.DeviceBuffer(n_ss * 64 * 4), ti.DeviceBuffer(M * N * 4)
+        out = []
+        for _ in range(2):   # (the second call over rows that the first rewrote)
+            ti.check(L.ti_memcpy_h2d(hd.ptr, h0.ctypes.data_as(C.c_void_p), h0.nbytes, None))
+            ep = ti.Epilogue()
+            ep.kind, ep.ldo, ep.out = ti.EPI_RESID_F32, H, hd.ptr
+            ep.fold_w, ep.fold_x, ep.fold_ss = nwd.ptr, fx.ptr, ss.ptr
+            rows(ti, bits, to, so, ad, M, H, K, ep, ws=k, kernel=kernel)
+            np.testing.assert_array_equal(np.signbit(ss.download(f32, (n_ss, 64))[:, :M]).any(axis=0), bad)
+            h1 = hd.download(f32, (M, H)).astype(np.float64)
+            ep = ti.Epilogue()
+            ep.kind, ep.ldo, ep.out, ep.ss_in, ep.n_ss = ti.EPI_STORE_F32, N, yd.ptr, ss.ptr, n_ss
+            rows(ti, bits, t2, s2, fx, M, N, H, ep, ws=k, kernel=kernel, h=hd.ptr, norm_w=nwd.ptr)
+            out.append(yd.download(f32, (M, N)))
+        x = h1 / np.sqrt((h1**2).mean(axis=1) + 1e-5)[:, None] * nw
+        err = np.abs(out[0] - x @ w2.astype(np.float64))
+        assert np.all(err <= (2.0**-11 + H * 2.0**-24) * (np.abs(x) @ np.abs(w2)) + 2.0**-25 * np.abs(w2).sum(axis=0) + 1e-9)
+        np.testing.assert_array_equal(*out)
 
 
 @pytest.mark.parametrize("bits", [4, 8, 16, 4 | G32])
@@ -296,33 +312,34 @@ def test_rows_fold_small_columns(ti, oracle, ws, bits, M):
     h[5, 64:] *= 1e-6
     h[M - 1] *= 2e-4
     first = np.isin(np.arange(M), [5, M - 1])
-    n_ss = L.ti_gemm_rows_fold_partials(bits, M, H, K, WS)
-    hd, fx, ss, yd, nwd = dev(ti, h), ti.DeviceBuffer(M * H * 2), ti.DeviceBuffer(n_ss * 64 * 4), ti.DeviceBuffer(M * N * 4), dev(ti, nw)
-    ep = ti.Epilogue()
-    ep.kind, ep.ldo, ep.out = ti.EPI_RESID_F32, H, hd.ptr
-    ep.fold_w, ep.fold_x, ep.fold_ss = nwd.ptr, fx.ptr, ss.ptr
-    rows(ti, bits, to, so, dev(ti, act), M, H, K, ep, ws=ws)
-    np.testing.assert_allclose(np.abs(ss.download(f32, (n_ss, 64))[:, :M]).sum(axis=0), (h.astype(np.float64) ** 2).sum(axis=1), rtol=1e-5)
-    ep = ti.Epilogue()
-    ep.kind, ep.ldo, ep.out, ep.ss_in, ep.n_ss = ti.EPI_STORE_F32, N, yd.ptr, ss.ptr, n_ss
-    ep.splitk_ws, ep.splitk_bytes = ws.ptr, ws.nbytes
-    ti.check(L.ti_gemm_rows_folded(t2.ptr, s2.ptr, bits, fx.ptr, H, hd.ptr, nwd.ptr, 1e-5, M, N, H, C.byref(ep), None))
-    ti.sync()
     plain = (h * nw).astype(f16).view(np.uint16)
-    np.testing.assert_array_equal((fx.download(np.uint16, (M, H)) != plain).any(axis=1), first)
     rms = np.sqrt((h.astype(np.float64) ** 2).mean(axis=1) + 1e-5)[:, None]
     x = h.astype(np.float64) / rms * nw
     step = 2.0**-25 / np.where(first[:, None], 1.0, rms)
     tol = (2.0**-11 + H * 2.0**-24) * (np.abs(x) @ np.abs(w2)) + step * np.abs(w2).sum(axis=0) + 1e-9
-    assert np.all(np.abs(yd.download(f32, (M, N)) - x @ w2.astype(np.float64)) <= tol)
+    ad, nwd = dev(ti, act), dev(ti, nw)
+    for kernel in kernels(ti, M):
+        n_ss = L.ti_gemm_rows_fold_partials_on(kernel, bits, M, H, K, WS)
+        hd, fx, ss, yd = dev(ti, h), ti.DeviceBuffer(M * H * 2), ti.DeviceBuffer(n_ss * 64 * 4), ti.DeviceBuffer(M * N * 4)
+        ep = ti.Epilogue()
+        ep.kind, ep.ldo, ep.out = ti.EPI_RESID_F32, H, hd.ptr
+        ep.fold_w, ep.fold_x, ep.fold_ss = nwd.ptr, fx.ptr, ss.ptr
+        rows(ti, bits, to, so, ad, M, H, K, ep, ws=ws, kernel=kernel)
+        np.testing.assert_allclose(np.abs(ss.download(f32, (n_ss, 64))[:, :M]).sum(axis=0), (h.astype(np.float64) ** 2).sum(axis=1), rtol=1e-5)
+        ep = ti.Epilogue()
+        ep.kind, ep.ldo, ep.out, ep.ss_in, ep.n_ss = ti.EPI_STORE_F32, N, yd.ptr, ss.ptr, n_ss
+        rows(ti, bits, t2, s2, fx, M, N, H, ep, ws=ws, kernel=kernel, h=hd.ptr, norm_w=nwd.ptr)
+        np.testing.assert_array_equal((fx.download(np.uint16, (M, H)) != plain).any(axis=1), first)
+        assert np.all(np.abs(yd.download(f32, (M, N)) - x @ w2.astype(np.float64)) <= tol)
 
 
 @pytest.mark.parametrize("bits", [4, 8, 16, 4 | G32, 8 | G32])
 def test_step_with_large_residuals(ti, bits):
-    """An embedding whose product with the norm weight passes fp16's range: a step of 9 streams (batched fold) against the
-    same streams in steps of 5 and 4 (normalised first).  Both round the same fp16 inputs: 1e-2 of the largest logit."""
+    """An embedding whose product with the norm weight passes fp16's range, or lies in its subnormal steps: steps of 9 streams and
+    prompts with the norms folded against the same with the fold off (ti_rmsnorm_f16 in front of every product).  Both round
+    the same fp16 inputs: 1e-2 of the largest logit."""
     V, H, layers, heads, kv, hd, inter = 512, 256, 2, 4, 2, 64, 512
-    e = ti.Engine(V, H, layers, heads, kv, hd, inter, bits=bits, max_seq=32, max_batch=9)
+    e = ti.Engine(V, H, layers, heads, kv, hd, inter, bits=bits, max_seq=96, max_batch=9)
     rng = np.random.RandomState(bits)
     if bits & G32:
         for i in range(layers + 1):
@@ -335,20 +352,20 @@ def test_step_with_large_residuals(ti, bits):
     emb = (0.02 * rng.standard_normal((V, H))).astype(f32)
     emb[::3, 7] = 6e4
     emb[1::3] *= 5e-5
-    nw = np.ones(H, f32)
-    nw[7] = 2
     e.set_tensor(ti.E_EMBED, 0, emb)
-    for i in range(layers):
-        e.set_tensor(ti.V_ATTN_NORM, i, nw)
-        e.set_tensor(ti.V_FFN_NORM, i, nw)
-    e.set_tensor(ti.V_OUT_NORM, 0, nw)
+    for slot, i in [(ti.V_ATTN_NORM, 0), (ti.V_ATTN_NORM, 1), (ti.V_FFN_NORM, 0), (ti.V_FFN_NORM, 1), (ti.V_OUT_NORM, 0)]:
+        nw = rng.uniform(0.7, 1.3, H).astype(f32)   # (each its own)
+        nw[7] = 2
+        e.set_tensor(slot, i, nw)
     tok = rng.randint(0, V, (3, 9)).astype(np.int32)
     tok[0] = np.arange(9)
-    got = [e.step(t, np.full(9, i, np.int32)) for i, t in enumerate(tok)]
-    # streams 0 .. 4, then 5 .. 8 in slots 0 .. 3
-    ref = [[e.step(t[a:b], np.full(b - a, i, np.int32)) for i, t in enumerate(tok)] for a, b in ((0, 5), (5, 9))]
+    prompts = [rng.randint(0, V, n).astype(np.int32) for n in (3, 17, 48, 64)]
+    out = []
+    for on in (True, False):
+        e.set_fold(on)
+        out.append([e.step(t, np.full(9, i, np.int32)) for i, t in enumerate(tok)] +
+                   [e.prefill(1, p, want=[0, p.size // 2, p.size - 1]) for p in prompts])
     e.close()
-    for i in range(len(tok)):
-        r = np.concatenate([ref[0][i], ref[1][i]])
-        assert np.isfinite(got[i]).all() and np.isfinite(r).all()
-        assert np.abs(got[i] - r).max() <= 1e-2 * np.abs(r).max(), (i, np.abs(got[i] - r).max(axis=1), np.abs(r).max())
+    for got, ref in zip(*out):
+        assert np.isfinite(got).all() and np.isfinite(ref).all()
+        assert np.abs(got - ref).max() <= 1e-2 * np.abs(ref).max(), (np.abs(got - ref).max(axis=1), np.abs(ref).max())

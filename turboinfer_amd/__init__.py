@@ -33,6 +33,7 @@ BITS_G32 = 32                       # TI_BITS_G32 (include/ti_hip.h): group-32 w
 BITS_AFF = 64                       # TI_BITS_AFF: affine group-32 int4 (GGUF Q4_1), with BITS_G32 | 4
 SCALE_GROUP, SCALE_TENSOR, SCALE_UNIT = 0, 1, 2
 ROWS_CONCAT, ROWS_INTERLEAVE8 = 0, 1
+ROWS_AUTO, ROWS_FEW, ROWS_MANY = 0, 1, 2   # ti_rows_kernel
 (W_Q, W_K, W_V, W_O, W_GATE, W_UP, W_DOWN, W_LM_HEAD, V_ATTN_NORM, V_FFN_NORM, V_OUT_NORM, E_EMBED) = range(12)
 
 
@@ -141,7 +142,7 @@ EXPORTED = [
     "ti_wpack_q_host", "ti_engine_set_tensor_q", "ti_sample_workspace_bytes", "ti_sample_device_ws",
     "ti_wpack_q1_host", "ti_engine_set_tensor_q1", "ti_epilogue_bytes",
     "ti_sample_step_ws", "ti_hbm_calibrate", "ti_gemm_kernel_name",
-    "ti_gemm_fold_partials", "ti_gemm_rows", "ti_gemm_rows_folded", "ti_gemm_rows_fold_partials", "ti_engine_set_stop", "ti_engine_counters",
+    "ti_gemm_fold_partials", "ti_gemm_rows", "ti_gemm_rows_folded", "ti_gemm_rows_fold_partials", "ti_gemm_rows_on", "ti_gemm_rows_fold_partials_on", "ti_engine_set_stop", "ti_engine_counters",
     "ti_qkv_attn_partials", "ti_qkv_attn_part_o_elems", "ti_qkv_attn_part_ml_elems", "ti_engine_set_qkv_attn",
     "ti_qkv_attn_xchg_bytes", "ti_qkv_attn_supported", "ti_qkv_attn_error_offset",
     "ti_engine_create_stack", "ti_engine_weight_count", "ti_engine_weight_info", "ti_engine_set_weight", "ti_engine_load",
@@ -193,6 +194,9 @@ def lib() -> C.CDLL:
             L.ti_gemm_rows.argtypes = [vp, vp, i32, vp, i32, f32, i32, i32, i32, C.POINTER(Epilogue), vp]
             L.ti_gemm_rows_folded.argtypes = [vp, vp, i32, vp, i32, vp, vp, f32, i32, i32, i32, C.POINTER(Epilogue), vp]
             L.ti_gemm_rows_fold_partials.argtypes = [i32, i32, i32, i32, i64]
+        if hasattr(L, "ti_gemm_rows_on"):
+            L.ti_gemm_rows_on.argtypes = [i32, vp, vp, i32, vp, i32, vp, vp, f32, i32, i32, i32, C.POINTER(Epilogue), vp]
+            L.ti_gemm_rows_fold_partials_on.argtypes = [i32, i32, i32, i32, i32, i64]
         L.ti_gemm_lds_bytes.argtypes = [i32, i32, i32]
         L.ti_gemm_max_rows.argtypes = [i32, i32, i32, i32]
         L.ti_gemm_packed_rows.argtypes = [i32, i32]

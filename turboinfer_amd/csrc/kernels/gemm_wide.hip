@@ -548,22 +548,26 @@ struct RowsPlan {
   ti::FewPlan f;
   ti::WidePlan w;
 };
-static bool rows_plan_of(int bits, int M, int N, int K, int64_t ws_bytes, bool fold, RowsPlan* p) {
-  const bool wide = ti::wide_plan(bits, M, N, K, ti::gemm_cus(), ws_bytes, fold, &p->w);
-  p->few = ti::few_plan(bits, M, N, K, ti::gemm_cus(), &p->f) && (!wide || p->f.us < 1.08f * p->w.us);
+static bool rows_plan_of(int kernel, int bits, int M, int N, int K, int64_t ws_bytes, bool fold, RowsPlan* p) {
+  const bool wide = kernel != TI_ROWS_FEW && ti::wide_plan(bits, M, N, K, ti::gemm_cus(), ws_bytes, fold, &p->w);
+  p->few = kernel != TI_ROWS_MANY && ti::few_plan(bits, M, N, K, ti::gemm_cus(), &p->f) && (!wide || p->f.us < 1.08f * p->w.us);
   return p->few || wide;
 }
 
-extern "C" int ti_gemm_rows_fold_partials(int bits, int M, int N, int K, int64_t ws_bytes) {
+extern "C" int ti_gemm_rows_fold_partials_on(int kernel, int bits, int M, int N, int K, int64_t ws_bytes) {
   RowsPlan p;
-  if (M > TI_FOLD_SS_ROWS || !rows_plan_of(bits, M, N, K, ws_bytes, true, &p)) return 0;
+  if (M > TI_FOLD_SS_ROWS || kernel < TI_ROWS_AUTO || kernel > TI_ROWS_MANY || !rows_plan_of(kernel, bits, M, N, K, ws_bytes, true, &p)) return 0;
   return p.few ? p.f.n_cb : p.w.n_cb;
 }
+extern "C" int ti_gemm_rows_fold_partials(int bits, int M, int N, int K, int64_t ws_bytes) {
+  return ti_gemm_rows_fold_partials_on(TI_ROWS_AUTO, bits, M, N, K, ws_bytes);
+}
 
-static int rows_impl(const void* tiles, const uint16_t* scales, int bits, const void* x, int ldx, const float* h, const float* norm_w,
+static int rows_impl(int kernel, const void* tiles, const uint16_t* scales, int bits, const void* x, int ldx, const float* h, const float* norm_w,
                      float eps, int M, int N, int K, const ti_epilogue* epi, ti_stream_t stream) {
   using namespace ti;
   if (!tiles || !x || !epi || !epi->out) return ti_set_error(TI_ERR_ARG, "ti_gemm_rows: null pointer");
+  if (kernel < TI_ROWS_AUTO || kernel > TI_ROWS_MANY) return ti_set_error(TI_ERR_ARG, "ti_gemm_rows: kernel %d", kernel);
   if (bits != 16 && !scales) return ti_set_error(TI_ERR_ARG, "ti_gemm_rows: scales required for bits %d", bits);
   if (M < 1 || M > TI_GEMM_MAX_ROWS || K <= 0 || (K & 127) || N <= 0 || (N & 15) || ldx < K || K > 0xffff || ldx > 0xffff)
     return ti_set_error(TI_ERR_ARG, "ti_gemm_rows: M=%d N=%d K=%d ldx=%d", M, N, K, ldx);
@@ -596,7 +600,7 @@ static int rows_impl(const void* tiles, const uint16_t* scales, int bits, const 
     a.norm_w = norm_w;
     a.epi.fold_w = h;
   }
-  if (!rows_plan_of(bits, M, N, K, epi->splitk_ws ? epi->splitk_bytes : 0, epi->ss_in || fold_out, &p))
+  if (!rows_plan_of(kernel, bits, M, N, K, epi->splitk_ws ? epi->splitk_bytes : 0, epi->ss_in || fold_out, &p))
     return ti_set_error(TI_ERR_UNSUPPORTED, "ti_gemm_rows: bits %d, M=%d N=%d K=%d", bits, M, N, K);
   const int rp = ti_gemm_prepare();   // no-op once this device is prepared
   if (rp != TI_OK) return rp;
@@ -606,11 +610,16 @@ static int rows_impl(const void* tiles, const uint16_t* scales, int bits, const 
 
 extern "C" int ti_gemm_rows(const void* tiles, const uint16_t* scales, int bits, const void* x, int ldx, float eps, int M, int N,
                             int K, const ti_epilogue* epi, ti_stream_t stream) {
-  return rows_impl(tiles, scales, bits, x, ldx, nullptr, nullptr, eps, M, N, K, epi, stream);
+  return rows_impl(TI_ROWS_AUTO, tiles, scales, bits, x, ldx, nullptr, nullptr, eps, M, N, K, epi, stream);
 }
 
 extern "C" int ti_gemm_rows_folded(const void* tiles, const uint16_t* scales, int bits, uint16_t* x, int ldx, const float* h,
                                    const float* norm_w, float eps, int M, int N, int K, const ti_epilogue* epi, ti_stream_t stream) {
   if (!h) return ti_set_error(TI_ERR_ARG, "ti_gemm_rows_folded: null pointer");
-  return rows_impl(tiles, scales, bits, x, ldx, h, norm_w, eps, M, N, K, epi, stream);
+  return rows_impl(TI_ROWS_AUTO, tiles, scales, bits, x, ldx, h, norm_w, eps, M, N, K, epi, stream);
+}
+
+extern "C" int ti_gemm_rows_on(int kernel, const void* tiles, const uint16_t* scales, int bits, uint16_t* x, int ldx, const float* h,
+                               const float* norm_w, float eps, int M, int N, int K, const ti_epilogue* epi, ti_stream_t stream) {
+  return rows_impl(kernel, tiles, scales, bits, x, ldx, h, norm_w, eps, M, N, K, epi, stream);
 }
