@@ -204,11 +204,12 @@ int ti_engine_serve(ti_engine* e, int n_req, const int32_t* prompts, const int32
  * layer-stack models as the engine's buffers hold.  0 = off. */
 int ti_engine_set_prefill(ti_engine* e, int rows);
 
-/* Fused hand-offs of single-stream steps: (1) the folded rms_norm (ti_hip.h TI_X_F16_FOLDED):
+/* Fused hand-offs between a pass's launches: (1) the folded rms_norm (single-stream steps: ti_hip.h TI_X_F16_FOLDED; steps of 3
+ * to 64 streams and prompts of as many tokens: ti_gemm_rows_folded):
  * the epilogue that updates the residual also writes fp16(h * next norm weight) and
  * per-workgroup sums of h^2, and the next projection divides its outputs by the rms instead of
  * normalising its input first; (2) the attention's split partials (ti_attn_decode_partials)
- * merged by the O projection (TI_X_ATTN_SPLITS) when the step uses 2..8 splits.  Default on
+ * merged by the O projection (TI_X_ATTN_SPLITS) when a single-stream step uses 2..8 splits.  Default on
  * (env TI_FOLD=0 / TI_ATTN_PART=0 turn them off one by one).
  * on = 0/1 sets both, -1 leaves them; *active (nullable) receives whether 1-stream steps fold. */
 int ti_engine_set_fold(ti_engine* e, int on, int* active);

@@ -206,7 +206,8 @@ typedef struct ti_epilogue {
    * Batched fold (17..64 int4 rows, TI_X_F16 / TI_X_F16_PACKED x holding fp16(h * nw), ss_in
    * non-NULL): row m is normalised behind the GEMM, y[m] = (W . x[m]) / sqrt(sum over
    * b < n_ss of ss_in[b * TI_FOLD_SS_ROWS + m] / K + eps) -- the batched-rows /
-   * many-rows kernels (blocks of 32: many-rows only, x and its rows 16-byte aligned) */
+   * many-rows kernels (blocks of 32: many-rows only, x and its rows 16-byte aligned); ti_gemm_rows: 1..64 rows of every
+   * format */
   int32_t n_ss;
   const float* ss_in;
   /* TI_EPI_RESID_F32, M == 1, fold_x non-NULL: besides h, write fold_x[n] = fp16(h[n] * fold_w[n])
@@ -252,7 +253,7 @@ int ti_gemm_lds_bytes(int M, int N, int K);
 int ti_gemm_max_rows(int bits, int x_kind, int N, int K);
 /* 1 when M rows of an int4 ti_gemm_wq_a16 call go to the batched-rows kernel (17 .. 64 rows): its
  * fp16 operands are best given as TI_X_F16_PACKED.  From 65 rows on the many-rows kernel
- * (ti_gemm_rows) takes TI_X_F16 rows. */
+ * of ti_gemm_rows takes TI_X_F16 rows. */
 int ti_gemm_packed_rows(int bits, int M);
 /* The same for one M x N x K call: 0 also where 17..64 int4 rows of a wide output take the many-rows
  * kernel (rows x N >= 850000, or N >= 16384 at 17..32 rows), which needs TI_X_F16 rows. */

@@ -1,5 +1,5 @@
-"""A step's inputs and logits across the bus: logits in page-locked pieces (ordinary memory, above 1.5 MiB) against one
-copy to page-locked memory, bit for bit, for sizes around a piece and past the ring of pieces; inputs after a longer
+"""A step's inputs and logits across the bus: logits to ordinary memory through the ring of page-locked pieces against one
+copy to page-locked memory, bit for bit, for sizes around a piece and past the ring; inputs after a longer
 prompt (the token rows' stride grows with it) against a fresh engine."""
 from __future__ import annotations
 

@@ -308,10 +308,12 @@ int validate(const ti_engine_config& c) {
 // Rows whose projections run on ti_gemm_rows, the rms_norm folded into them: from 3 on.  Below, the fused kernel (its rms_norm
 // prologue) takes as long.  Measured, the mean over the products of four models, its time or that of the int4 kernel of 3 .. 16
 // rows beside its rms_norm over this: at 2 rows 1.01 (int4) / 0.99 (int8) / 0.97 (blocks of 32), at 4 1.07 / 1.17 / 1.17, at 8
-// 1.13 / 1.39 / 1.36.
+// 1.13 / 1.39 / 1.36.  Rows that must be normalised first (ti_gemm_rows_folded) cost their consumer a second product: Llama-2-7B
+// int4, every row of every layer like that, a step of 3 streams 1650 -> 2710 us, of 24 2340 -> 4950, a prompt of 64 2760 -> 7940
+// (the norms apart: 1760, 2390, 2840).
 bool rows_wide(const ti_engine* e, int M) { return e->wide_ok && M >= 3; }
 
-// One projection for rows [0, M): the many-rows kernel, fp32 rows normalised into fp16 first (e->xn); or the fused
+// One projection for rows [0, M): ti_gemm_rows, fp32 rows normalised into fp16 first (e->xn); or the fused
 // kernel in chunks of the rows its LDS image holds (int4 rows that do not fit: the batched kernel behind the same
 // rms_norm).  Graph-capturable.
 int gemm_rows(ti_engine* e, const DevLinear& W, int M, const void* x, int x_kind, int ldx, const float* nw,
@@ -372,7 +374,7 @@ bool fold_usable(ti_engine* e, int M) {
   return g_o > 0 && g_o <= 256 && g_d > 0 && g_d <= 256 && ti_gemm_max_rows(c.bits, TI_X_F16, H, qd) >= 1;
 }
 
-// The batched fold: up to 64 rows on the many-rows kernel, the O / down producers' column blocks within the partial
+// The batched fold: up to 64 rows on ti_gemm_rows, the O / down producers' column blocks within the partial
 // buffer.
 bool bfold_usable(ti_engine* e, int M) {
   const ti_engine_config& c = e->c;
@@ -626,7 +628,7 @@ int enqueue_step(ti_engine* e, int M, int advance) {
   const int H = c.hidden, qd = e->qd(), kvd = e->kvd(), I = c.inter, V = c.vocab;
   // fold (M == 1): every rms_norm input is handed over as fx + ss partials by its producer
   const bool fold = fold_usable(e, M), part = part_usable(e, M), qa = qa_usable(e, M);
-  // batched fold (many-rows kernel, up to 64 rows): O / down write xn = fp16(h * next norm weight) and per-row
+  // batched fold (ti_gemm_rows, up to 64 rows): O / down write xn = fp16(h * next norm weight) and per-row
   // sums of h^2; QKV (after layer 0), gate/up and the lm_head normalise behind their GEMM, rows past fp16's range
   // before it (ti_hip.h)
   const bool bfold = !fold && bfold_usable(e, M);
@@ -1005,7 +1007,7 @@ int ti_engine_create(const ti_engine_config* cfg, ti_engine** out) {
     if ((rc = ti_memcpy_h2d(e->rope_cs, cs.data(), cs.size() * 4, e->s))) return fail(rc);
     if (const char* env = getenv("TI_ATTN_PART")) e->part_on = atoi(env) != 0;
     e->splits_max = e->splits_for(1);
-    // the many-rows kernel's byte offsets into a weight are 32 bits; wider ones keep the fused kernel's 16-row pieces
+    // the byte offsets of ti_gemm_rows' kernels into a weight are 32 bits; wider ones keep the fused kernel's 16-row pieces
     e->wide_ok = true;
     const int shapes[][2] = {{H, qd + 2 * kvd}, {qd, H}, {H, 2 * I}, {I, H}, {H, V}};   // (a model may have no layers)
     for (const auto& w : shapes) e->wide_ok = e->wide_ok && ti_gemm_rows_fold_partials(c.bits, TI_FOLD_SS_ROWS, w[1], w[0], 0) > 0;

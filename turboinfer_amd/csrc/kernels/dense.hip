@@ -299,7 +299,11 @@ __global__ __launch_bounds__(64 * W) void dense_skinny_kernel(const ti_dense_arg
 // these take 8.  A product's 16 x 16 tile holds two k-tiles: its weight rows 0 .. 7 and rows of a 0 .. 7 are the first's, 8 ..
 // 15 the second's, and the diagonal blocks are summed at the end (the other two mean nothing); rows 8 .. 15 of a are a
 // second product.  2048 columns, K 8192 (33.5 MB), 8 rows: 13.6 -> 10.4 us; a step of Nogitar 2k (15 of them) of 8 streams 477 ->
-// 450 us, of 16 550 -> 529, fp32 of one 710 -> 609.
+// 450 us, of 16 550 -> 529, fp32 of one 710 -> 609.  Up to 2048 columns these workgroups fit the CUs at once; beyond, a
+// second round starts.  us at 1 / 8 / 16 rows, skinny -> this, N x K: bf16 256 x 2048 4.1 / 4.7 / 5.2 -> 3.4 / 3.8 / 4.6, 2048 x
+// 1024 3.6 / 3.9 / 4.1 -> 3.2 / 3.4 / 3.9, 2048 x 8192 11.2 / 13.1 / 16.5 -> 8.7 / 9.8 / 13.6, 2176 x 8192 11.2 / 13.2 / 16.2 -> 11.0 /
+// 14.7 / 20.6, 4096 x 2048 5.4 / 5.7 / 6.3 -> 5.2 / 5.6 / 7.0; fp32 2048 x 8192 29.2 / 29.7 / 31.1 -> 18.0 / 18.0 / 22.8, 2176 x 8192 29.6 /
+// 29.9 / 31.4 -> 20.5 / 27.5 / 39.0.
 template <class T, int MT, int W, int EPI>
 __global__ __launch_bounds__(64 * W) void dense_half_kernel(const ti_dense_args a) {
   typedef typename El<T>::V V;

@@ -17,7 +17,7 @@ struct FewCfg {
 };
 
 // Bound: the launch (~ 3 us from the first workgroup's entry to the last one's end without any work), one memory latency and
-// what a CU takes in (~ 100 KB/us): the rows, once per workgroup, and its weights.  So a workgroup owns 16 TN whole columns and
+// what a CU takes in (~ 100 KB/us; reads of 2 MB that the L2 holds reach 110 on every CU at once, 140 on one): the rows, once per workgroup, and its weights.  So a workgroup owns 16 TN whole columns and
 // its 8 waves split K and meet in LDS (a split over workgroups meets in memory: ~ 3 us); a wave has two groups of 128 k in
 // flight in registers, rows as whole 256-byte pieces that it turns into fragments in its own part of the LDS (fragment-shaped
 // loads, 16 bytes of 16 rows, take four times as long: 2048 columns, K 5632, 24 rows 13.6 -> 9.8 us).  Against the many-rows

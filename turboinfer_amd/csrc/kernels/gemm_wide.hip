@@ -108,7 +108,8 @@ __device__ __forceinline__ bool wide_merge(const GemvArgs& a, f32x4 (&acc)[TN][T
 
 // Bound: int4 and int8 by the vector unit beside the matrix cores (a 16x16x32 MFMA and its share of dequant and scale
 // FMAs take ~ 0.87 (16 + 4 V) cycles with V vector instructions per MFMA: V 3 at 64 rows a wave, more with fewer rows
-// to share a dequantised tile), small row counts and fp16 by what a CU takes in from the L2 (~ 45 KB/us), so a block
+// to share a dequantised tile), small row counts and fp16 by the copies into a CU (~ 45 KB/us with the
+// hand-overs of the stages; plain reads reach 110), so a block
 // keeps 64 rows as soon as the call has them.  DMA straight to LDS leaves the registers to the accumulators; the
 // next stage's unpacking is interleaved with this one's MFMAs.  Measured inside a pass, us (fused kernel in 16-row
 // pieces / tile and batched-rows kernels -> this one): int8 1000 rows 2048 -> 11264 63 x 22.8 -> 79, fp16 333 rows the

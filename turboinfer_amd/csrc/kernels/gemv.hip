@@ -800,7 +800,8 @@ __global__ __launch_bounds__(kGemvThreads, 1) void gemv_wq_kernel(const u32x4* p
 
 // ================================================================= batched rows
 // gemv_mbr_kernel<MB, NTL>: int4 weights x 3..16 fp16 rows (a batch of a few streams, and long-K projections whose
-// rows no longer fit gemv_wq_kernel's LDS image).  Weights are read once per launch, straight into registers, in
+// rows no longer fit gemv_wq_kernel's LDS image): direct calls of ti_gemm_wq_a16, and engines with a weight of 4 GiB or more
+// (others run ti_gemm_rows from 3 rows on).  Weights are read once per launch, straight into registers, in
 // chunks of 1024 k (8 k-tiles, one per wave), one chunk ahead.
 __host__ __device__ inline int mbr_slab_bytes(int MB, int ntl) { return align16(ntl * MB * kGemvWaves * kWave * 16); }
 __host__ __device__ inline int mbr_lds_bytes(int MB, int ntl, int K) {
