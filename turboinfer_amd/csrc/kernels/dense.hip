@@ -315,7 +315,7 @@ __global__ __launch_bounds__(64 * W) void dense_half_kernel(const ti_dense_args 
   const V* ap[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
-    ap[mt] = (const V*)((const T*)a.a + (size_t)row_in(a, min(mt * 8 + (lane & 7), a.M - 1)) * a.lda + second * KT) + (lane >> 4);
+    ap[mt] = (const V*)((const T*)a.a + (size_t)min(mt * 8 + (lane & 7), a.M - 1) * a.lda + second * KT) + (lane >> 4);
   f32x4 acc[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) acc[mt] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -745,7 +745,8 @@ int skinny(const ti_dense_args& a, hipStream_t s) {
   const long g = (long)((a.N + 15) / 16) * a.batch;
   const int mt = (a.M + 15) / 16;
   if constexpr (EPI == TI_DE_F32)
-    if (!a.tile_rows && mt == 1 && a.batch == 1 && a.N <= 2048) return launch_half<T, EPI>(a, s);
+    // (row_div: its check in the kernel costs steps of small models 1 - 3 %)
+    if (!a.tile_rows && mt == 1 && a.batch == 1 && a.N <= 2048 && a.row_div <= 1) return launch_half<T, EPI>(a, s);
   if (a.tile_rows || mt == 1 || g < 256) return launch_skinny<T, 1, EPI>(a, s);
   if (mt == 2 || g < 512) return launch_skinny<T, 2, EPI>(a, s);
   return launch_skinny<T, 4, EPI>(a, s);

@@ -731,7 +731,7 @@ int launch_ssd_step(const ti_ssd_args& a, hipStream_t s) {
   const int ps = (long)a.M * a.heads >= 1024 ? std::min(a.vdim, 128) : 16;
   const dim3 grid((a.vdim + ps - 1) / ps, a.heads, a.M), blk(256);
   const size_t lds = (size_t)((ps + 3) / 4 * 4 + 2 * np) * 4;
-  auto run = [&]<int LPR>() {
+  auto run = [&]<int LPR>() {   // (4 taps: what the models have; others one input after another)
     if (a.taps == 4) hipLaunchKernelGGL((ssd_step_kernel<T, LPR, 4>), grid, blk, lds, s, a, ps);
     else hipLaunchKernelGGL((ssd_step_kernel<T, LPR, 0>), grid, blk, lds, s, a, ps);
   };
