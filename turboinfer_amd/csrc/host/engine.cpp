@@ -308,9 +308,9 @@ int validate(const ti_engine_config& c) {
 // Rows whose projections run on ti_gemm_rows, the rms_norm folded into them: from 3 on.  Below, the fused kernel (its rms_norm
 // prologue) takes as long.  Measured, the mean over the products of four models, its time or that of the int4 kernel of 3 .. 16
 // rows beside its rms_norm over this: at 2 rows 1.01 (int4) / 0.99 (int8) / 0.97 (blocks of 32), at 4 1.07 / 1.17 / 1.17, at 8
-// 1.13 / 1.39 / 1.36.  Rows that must be normalised first (ti_gemm_rows_folded) cost their consumer a second product: Llama-2-7B
-// int4, every row of every layer like that, a step of 3 streams 1650 -> 2710 us, of 24 2340 -> 4950, a prompt of 64 2760 -> 7940
-// (the norms apart: 1760, 2390, 2840).
+// 1.13 / 1.39 / 1.36.  Rows that must be normalised first (ti_gemm_rows_folded) cost their consumer the rewriting, by every
+// workgroup, and a second product: Llama-2-7B int4, every row of every layer like that, a step of 3 streams 1650 -> 2710 us, of
+// 24 2340 -> 4950, a prompt of 64 2760 -> 7940 (the norms apart: 1760, 2390, 2840).
 bool rows_wide(const ti_engine* e, int M) { return e->wide_ok && M >= 3; }
 
 // One projection for rows [0, M): ti_gemm_rows, fp32 rows normalised into fp16 first (e->xn); or the fused

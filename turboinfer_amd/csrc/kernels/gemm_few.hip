@@ -17,10 +17,11 @@ struct FewCfg {
 };
 
 // Bound: the launch (~ 3 us from the first workgroup's entry to the last one's end without any work), one memory latency and
-// what a CU takes in (~ 100 KB/us; reads of 2 MB that the L2 holds reach 110 on every CU at once, 140 on one): the rows, once per workgroup, and its weights.  So a workgroup owns 16 TN whole columns and
-// its 8 waves split K and meet in LDS (a split over workgroups meets in memory: ~ 3 us); a wave has two groups of 128 k in
-// flight in registers, rows as whole 256-byte pieces that it turns into fragments in its own part of the LDS (fragment-shaped
-// loads, 16 bytes of 16 rows, take four times as long: 2048 columns, K 5632, 24 rows 13.6 -> 9.8 us).  Against the many-rows
+// what a CU takes in (~ 100 KB/us; reads of 2 MB that the L2 holds reach 110 on every CU at once, 140 on one): the rows, once
+// per workgroup, and its weights.  So a workgroup owns 16 TN whole columns and its 8 waves split K and meet in LDS (a split over
+// workgroups meets in memory: ~ 3 us); a wave has two groups of 128 k in flight in registers, rows as whole 256-byte pieces that
+// it turns into fragments in its own part of the LDS (fragment-shaped loads, 16 bytes of 16 rows, take four times as long: 2048
+// columns, K 5632, 24 rows 13.6 -> 9.8 us).  Against the many-rows
 // kernel (gemm_wide.hip), us, many-rows -> this: int8 2048 -> 2560 at 8 rows 7.3 -> 5.7, 24 rows 8.3 -> 6.9; 2048 -> 2048 6.6 ->
 // 5.0; 5632 -> 2048 8.6 -> 7.5; int4 4096 -> 12288 at 16 rows 12.2 -> 10.4, 11008 -> 4096 12.2 -> 10.9; blocks of 32 bytes'
 // 1024 -> 5632 at 24 rows 8.3 -> 6.3.  Wide outputs that take several rounds of workgroups stay with the many-rows
