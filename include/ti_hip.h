@@ -282,7 +282,7 @@ int ti_gemm_fold_partials(int bits, int M, int N, int K);
  * (M <= TI_FOLD_SS_ROWS).  TI_EPI_RESID_F32 with fold_x: also the next call's folded input, rows of ldo, and
  * fold_ss[b * TI_FOLD_SS_ROWS + m], b < ti_gemm_rows_fold_partials(same call and workspace), negated where fp16 does not
  * hold the row's columns of the block: the mantissa's lowest bit clear where |h * fold_w| passes 65504, else set where its
- * mean square is below 2^-22. */
+ * mean square is below 2^-23. */
 int ti_gemm_rows(const void* tiles, const uint16_t* scales, int bits, const void* x, int ldx, float eps, int M, int N, int K,
                  const ti_epilogue* epi, ti_stream_t s);
 /* ti_gemm_rows of a folded input (ss_in; no fold_x) and the rows h [M][K] and norm weight [K] (16-byte aligned) that x was
