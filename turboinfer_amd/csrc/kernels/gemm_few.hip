@@ -9,8 +9,8 @@ constexpr int kFewWaves = 8;
 template <int F, int TM, int TN>
 struct FewCfg {
   static constexpr int kRows = 16 * TM;
-  // rms per row, its shares and their marks | every wave's rows of a group | partial sums of every wave | each tile's staging block
-  static constexpr int kX = (kRows + 2 * kFewWaves * kWave) * 4, kRed = kX + kFewWaves * kRows * 256;
+  // rms per row and its shares | every wave's rows of a group | partial sums of every wave | each tile's staging block
+  static constexpr int kX = (kRows + kFewWaves * kWave) * 4, kRed = kX + kFewWaves * kRows * 256;
   static constexpr int kStg = kRed + kFewWaves * TN * TM * 1024, kSs = kStg + TN * kRows * kTileEpiStride * 4;
   static constexpr int kLds = kSs + TN * kRows * 8;
   static_assert(TN <= kFewWaves && kLds <= 160 * 1024);
@@ -183,19 +183,22 @@ __global__ __launch_bounds__(64 * kFewWaves, 2) void gemm_few_kernel(const GemvA
   };
   const bool fold_in = a.epi.ss_in != nullptr;
   float* rmsv = (float*)smem;
-  uint32_t* const marks = (uint32_t*)rmsv + C::kRows + 64 * NW;
-  const float share = fold_in ? wide_fold_share(a, tid % C::kRows, tid / C::kRows, 64 * NW / C::kRows, marks + tid) : 0.0f;
+  const float share = fold_in ? wide_fold_share(a, tid % C::kRows, tid / C::kRows, 64 * NW / C::kRows) : 0.0f;
   product();
   if (fold_in) {
-    wide_fold_rms<C::kRows, NW>(a, share, tid, rmsv, marks);
-    const float mine = rmsv[lane % C::kRows];
-    if (__builtin_expect(a.norm_w && __builtin_amdgcn_ballot_w64(__builtin_bit_cast(int32_t, mine) < 0) != 0, 0)) {
-      // rows that fp16 did not hold: again, behind their rewriting
-      wide_refold<C::kRows, NW>(a, wave, lane, rmsv);
-      lds_barrier();
-      product();
-      lds_barrier();
-      if (tid < C::kRows && rmsv[tid] < 0.0f) rmsv[tid] = 1.0f;
+    wide_fold_rms<C::kRows, NW>(a, share, tid, rmsv);
+    auto marked = [&]() __attribute__((always_inline)) {   // (a row's rms is negative)
+      return __builtin_amdgcn_ballot_w64(__builtin_bit_cast(int32_t, rmsv[lane % C::kRows]) < 0) != 0;
+    };
+    if (__builtin_expect(a.norm_w && marked(), 0)) {
+      wide_fold_settle<C::kRows, NW>(a, tid, rmsv);
+      if (marked()) {   // rows that fp16 did not hold: again, behind their rewriting
+        wide_refold<C::kRows, NW>(a, wave, lane, rmsv);
+        lds_barrier();
+        product();
+        lds_barrier();
+        if (tid < C::kRows && rmsv[tid] < 0.0f) rmsv[tid] = 1.0f;
+      }
     }
   }
   lds_barrier();

@@ -42,10 +42,9 @@ struct WideCfg {
   // after the stream: rms per row | each wave's staging block | (sum of h^2, of (h w)^2) per column-wave and row | ticket
   static constexpr int kEpiStg = kRows * 4, kEpiRed = kEpiStg + kWaves * 16 * TM * kTileEpiStride * 4;
   static constexpr int kEpiFlag = kEpiRed + 2 * WN * kRows * 4, kEpi = kEpiFlag + 16;
-  static constexpr int kMarks = NS * kStage > kEpi ? NS * kStage : kEpi;   // each thread's word of wide_fold_share
+  static constexpr int kLds = NS * kStage > kEpi ? NS * kStage : kEpi;
   static constexpr bool kFold = kRows <= TI_FOLD_SS_ROWS;   // (every wave of these has all rows)
   static_assert(!kFold || WM == 1, "a wave sees every row's rms");
-  static constexpr int kLds = kMarks + (kFold ? 64 * kWaves * 4 : 0);
   static constexpr int kDmaA = kRows / 4 / kWaves, kDmaW = kTiles * (W::kTile / 1024) / kWaves;
   static constexpr int kDma = kDmaA + kDmaW + kScaleDma;
   static_assert(kRows / 4 % kWaves == 0 && kTiles * (W::kTile / 1024) % kWaves == 0, "equal DMA counts per wave");
@@ -291,8 +290,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const GemvAr
   for (int s = 0; s < NS; ++s) issue(min(kb + s, ke - 1), s);
   // batched fold (decode rows, ti_hip.h TI_FOLD_SS_ROWS): this thread's share of its row's sum of squares
   const bool fold_in = C::kFold && a.epi.ss_in != nullptr;
-  uint32_t* const marks = (uint32_t*)(smem + C::kMarks);
-  const float share = fold_in ? wide_fold_share(a, m0 + tid % C::kRows, tid / C::kRows, 64 * NW / C::kRows, marks + tid) : 0.0f;
+  const float share = fold_in ? wide_fold_share(a, m0 + tid % C::kRows, tid / C::kRows, 64 * NW / C::kRows) : 0.0f;
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * C::kDma) : "memory");
   lds_barrier();
   Step st[2];
@@ -349,17 +347,21 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const GemvAr
 #pragma unroll
     for (int i = 0; i < 4; ++i) rms[b][i] = 1.0f;
   if (fold_in) {
-    wide_fold_rms<C::kRows, NW>(a, share, tid, rmsv, marks);
-    uint32_t any = 0;
+    wide_fold_rms<C::kRows, NW>(a, share, tid, rmsv);
+    auto marked = [&]() __attribute__((always_inline)) {   // (reads the rows' rms; one of them is negative)
+      uint32_t any = 0;
 #pragma unroll
-    for (int b = 0; b < TM; ++b)
+      for (int b = 0; b < TM; ++b)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        rms[b][i] = rmsv[wm * 16 * TM + b * 16 + 4 * kq + i];
-        any |= __builtin_bit_cast(uint32_t, rms[b][i]);
-      }
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64((int32_t)any < 0) != 0, 0)) {
-      if (a.norm_w) {   // rows that fp16 did not hold: again, behind their rewriting, a stage at a time
+        for (int i = 0; i < 4; ++i) {
+          rms[b][i] = rmsv[wm * 16 * TM + b * 16 + 4 * kq + i];
+          any |= __builtin_bit_cast(uint32_t, rms[b][i]);
+        }
+      return __builtin_amdgcn_ballot_w64((int32_t)any < 0) != 0;
+    };
+    if (__builtin_expect(marked(), 0)) {
+      if (a.norm_w) wide_fold_settle<C::kRows, NW>(a, tid, rmsv);
+      if (a.norm_w && marked()) {   // rows that fp16 did not hold: again, behind their rewriting, a stage at a time
         wide_refold<C::kRows, NW>(a, wave, lane, rmsv);
 #pragma unroll
         for (int t = 0; t < TN; ++t)

@@ -22,68 +22,70 @@ __device__ __forceinline__ float fold_mark(float t, bool over, bool small) {
   if (over) return __builtin_bit_cast(float, (b & ~1u) | 0x80000000u);
   return small ? __builtin_bit_cast(float, b | (t < INFINITY ? 0x80000001u : 0x80000000u)) : t;
 }
-// Consumer side: this thread's share of row m's partial sums (part, part + P, ...), summed in order; negative if one of them is,
-// and then *marks (LDS) counts the small ones, the top bit for one past 65504.
-__device__ __forceinline__ float wide_fold_share(const GemvArgs& a, int m, int part, int P, uint32_t* marks) {
+// Consumer side: this thread's share of row m's partial sums (part, part + P, ...), summed in order; negative if one of them is.
+__device__ __forceinline__ float wide_fold_share(const GemvArgs& a, int m, int part, int P) {
   float t = 0.0f;
   uint32_t any = 0;
   if (m >= a.M) return t;
   const float* ss = a.epi.ss_in + m;
-  auto load = [&](float (&v)[16], int b0) __attribute__((always_inline)) {
+  for (int b0 = part; b0 < a.epi.n_ss; b0 += 16 * P) {
+    float v[16];
 #pragma unroll
     for (int j = 0; j < 16; ++j) v[j] = b0 + j * P < a.epi.n_ss ? ss[(size_t)(b0 + j * P) * TI_FOLD_SS_ROWS] : 0.0f;
-  };
-  float v[16];
-  for (int b0 = part; b0 < a.epi.n_ss; b0 += 16 * P) {
-    load(v, b0);
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
       t += fabsf(v[j]);
       any |= __builtin_bit_cast(uint32_t, v[j]);
     }
   }
-  any &= 0x80000000u;
-  if (__builtin_expect(any != 0, 0)) {
-    uint32_t n = 0, over = 0;
-    for (int b0 = part; b0 < a.epi.n_ss; b0 += 16 * P) {   // (again: counted on the way, they would cost every call)
-      load(v, b0);
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const uint32_t b = __builtin_bit_cast(uint32_t, v[j]);
-        n += b & (b >> 31);
-        over |= b & ~(b << 31);
-      }
-    }
-    *marks = n | (over & 0x80000000u);
-  }
-  return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, t) | any);
+  return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, t) | (any & 0x80000000u));
 }
-// The threads' shares to the rms of every row, negative where the row is to be normalised first (behind a barrier; one follows).
+// The threads' shares to the rms of every row, negative as they are (behind a barrier; one follows).
 template <int ROWS, int NW>
-__device__ __forceinline__ void wide_fold_rms(const GemvArgs& a, float share, int tid, float* rmsv, const uint32_t* marks) {
-  constexpr int P = 64 * NW / ROWS;
+__device__ __forceinline__ void wide_fold_rms(const GemvArgs& a, float share, int tid, float* rmsv) {
   rmsv[ROWS + tid] = share;
   lds_barrier();
   if (tid < ROWS) {
     float t = 0.0f;
     uint32_t any = 0;
-    for (int p = 0; p < P; ++p) {
+    for (int p = 0; p < 64 * NW / ROWS; ++p) {
       const float v = rmsv[ROWS + p * ROWS + tid];
       t += fabsf(v);
       any |= __builtin_bit_cast(uint32_t, v);
     }
-    float rms = sqrtf(t / (float)a.K + a.eps);
-    if (__builtin_expect((int32_t)any < 0, 0)) {
-      uint32_t n = 0, over = 0;
-#pragma unroll 8
-      for (int p = 0; p < P; ++p) {
-        const uint32_t v = marks[p * ROWS + tid], mine = (uint32_t)(__builtin_bit_cast(int32_t, rmsv[ROWS + p * ROWS + tid]) >> 31);   // (unwritten: 0)
-        n += v & mine & 0xffffu;
-        over |= v & mine;
-      }
-      if ((int32_t)over < 0 || 2 * (int)n > a.epi.n_ss) rms = -rms;
+    rmsv[tid] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, sqrtf(t / (float)a.K + a.eps)) | (any & 0x80000000u));
+  }
+  lds_barrier();
+}
+// Where a row's rms is negative: the marks counted, the rms of rows that are taken as they are made positive (behind a barrier; one
+// follows).  Apart, so that calls without a mark do not pay for it (0.1 us each).
+template <int ROWS, int NW>
+__device__ __forceinline__ void wide_fold_settle(const GemvArgs& a, int tid, float* rmsv) {
+  constexpr int P = 64 * NW / ROWS;
+  uint32_t* marks = (uint32_t*)rmsv + ROWS;   // small blocks; the top bit: one is past 65504
+  const int m = tid % ROWS, part = tid / ROWS;
+  uint32_t n = 0, over = 0;
+  for (int b0 = m < a.M && part < P ? part : a.epi.n_ss; b0 < a.epi.n_ss; b0 += 16 * P) {
+    uint32_t v[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+      v[j] = b0 + j * P < a.epi.n_ss ? __builtin_bit_cast(uint32_t, a.epi.ss_in[(size_t)(b0 + j * P) * TI_FOLD_SS_ROWS + m]) : 0u;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      n += v[j] & (v[j] >> 31);
+      over |= v[j] & ~(v[j] << 31);
     }
-    rmsv[tid] = rms;
+  }
+  marks[tid] = n | (over & 0x80000000u);
+  lds_barrier();
+  if (tid < ROWS && rmsv[tid] < 0.0f) {
+    n = over = 0;
+#pragma unroll 8
+    for (int p = 0; p < P; ++p) {
+      n += marks[p * ROWS + tid] & 0xffffu;
+      over |= marks[p * ROWS + tid];
+    }
+    if ((int32_t)over >= 0 && 2 * (int)n <= a.epi.n_ss) rmsv[tid] = -rmsv[tid];
   }
   lds_barrier();
 }
