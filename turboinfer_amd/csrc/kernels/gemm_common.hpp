@@ -212,12 +212,53 @@ __device__ __forceinline__ void fold_rms_finish(const GemvArgs& a, const float* 
 
 constexpr int kTileEpiStride = 20;   // floats per row of a wave's 64 x 16 staging block (padded: no bank conflicts)
 
-// Epilogue of weight tile tn (16 outputs) for rows mb .. mb + 63 of one wave, from its LDS block
+// What the epilogue of weight tile tn reads beside the products, for rows mb .. mb + 16 RB - 1 of one wave (a.vec): the residual,
+// or the positions and their (cos, sin) pairs -- two dependent loads.  Fetched ahead of the tile's products or of the tile before
+// it: read row by row where they are used, each row waits for its own (a 7B
+// int4 prompt of 512 whose products all end here: 8684 -> 8579 us).
+template <int RB>
+struct TilePre {
+  float4 v[RB];
+  int32_t pos[RB];
+};
+struct TileQkv {   // a tile lies in one of q / k / v and in one head (head_dim % 16 == 0)
+  bool q, k;
+  int head, d;   // of its first column
+};
+__device__ __forceinline__ TileQkv tile_qkv(const ti_epilogue& e, int tn) {
+  const int n = tn * 16;
+  const bool q = n < e.q_dim, k = !q && n < e.q_dim + e.kv_dim;
+  const int c = q ? n : k ? n - e.q_dim : n - e.q_dim - e.kv_dim, head = c / e.head_dim;
+  return {q, k, head, c - head * e.head_dim};
+}
+template <int RB>
+__device__ __forceinline__ void tile_pos(const GemvArgs& a, int mb, int lane, TilePre<RB>& p) {   // (any time before the others)
+  if (a.epi.kind == TI_EPI_QKV_ROPE_KV)
+#pragma unroll
+    for (int it = 0; it < RB; ++it) p.pos[it] = a.epi.pos[min(mb + (lane >> 2) + 16 * it, a.M - 1)];
+}
+template <int RB>
+__device__ __forceinline__ void tile_pre(const GemvArgs& a, int tn, int mb, int lane, TilePre<RB>& p) {
+  const ti_epilogue& e = a.epi;
+  const int c4 = 4 * (lane & 3), m0 = mb + (lane >> 2);
+  if (!a.vec) return;
+  if (e.kind == TI_EPI_RESID_F32) {
+#pragma unroll
+    for (int it = 0; it < RB; ++it) p.v[it] = *(const float4*)((const float*)e.out + (size_t)min(m0 + 16 * it, a.M - 1) * e.ldo + tn * 16 + c4);
+  } else if (e.kind == TI_EPI_QKV_ROPE_KV) {
+    const TileQkv t = tile_qkv(e, tn);
+    if (t.q || t.k)
+#pragma unroll
+      for (int it = 0; it < RB; ++it) p.v[it] = *(const float4*)(e.rope_cs + (size_t)p.pos[it] * e.head_dim + t.d + c4);
+  }
+}
+
+// Epilogue of weight tile tn (16 outputs) for rows mb .. mb + 16 RB - 1 of one wave, from its LDS block
 // stg[row][col] (row stride kTileEpiStride).  Same arithmetic as epilogue_mb, element for element.
 //   STORE_F32 / RESID_F32 / QKV_ROPE_KV: lane l owns columns 4 (l & 3) .. + 3 of rows 16 it + l / 4
 //   SILU_MUL_F16: lane l owns outputs 4 (l & 1) .. + 3 (gate columns, up = column + 8) of rows 32 it + l / 2
-template <int RB = 4>   // the wave's rows: 16 RB
-__device__ __forceinline__ void tile_epilogue_lds(const GemvArgs& a, int tn, int mb, const float* stg, int lane) {
+template <int RB>
+__device__ __forceinline__ void tile_epilogue_lds(const GemvArgs& a, int tn, int mb, const float* stg, int lane, const TilePre<RB>& p) {
   const ti_epilogue& e = a.epi;
   if (e.kind == TI_EPI_SILU_MUL_F16) {
     const int h = 4 * (lane & 1);
@@ -234,41 +275,44 @@ __device__ __forceinline__ void tile_epilogue_lds(const GemvArgs& a, int tn, int
     }
     return;
   }
-  const int c4 = 4 * (lane & 3), ng = tn * 16 + c4;
-  // QKV: the tile lies in one of q / k / v and one head (head_dim % 16 == 0)
-  const int hd = e.head_dim;
-  const bool in_q = ng < e.q_dim, in_k = !in_q && ng < e.q_dim + e.kv_dim;
-  const int c = in_q ? ng : in_k ? ng - e.q_dim : ng - e.q_dim - e.kv_dim;
-  const int kvh = e.kind == TI_EPI_QKV_ROPE_KV ? c / hd : 0, d = c - kvh * hd;
+  const int c4 = 4 * (lane & 3), ng = tn * 16 + c4, m0 = mb + (lane >> 2);
+  float4 v[RB];
 #pragma unroll
-  for (int it = 0; it < RB; ++it) {
-    const int row = 16 * it + (lane >> 2), m = mb + row;
-    const float4 v = *(const float4*)(stg + row * kTileEpiStride + c4);
-    if (m >= a.M) continue;
-    if (e.kind == TI_EPI_STORE_F32) {
-      *(float4*)((float*)e.out + (size_t)m * e.ldo + ng) = v;
-    } else if (e.kind == TI_EPI_RESID_F32) {
-      float4* o = (float4*)((float*)e.out + (size_t)m * e.ldo + ng);
-      const float4 h = *o;
-      *o = make_float4(h.x + v.x, h.y + v.y, h.z + v.z, h.w + v.w);
-    } else {   // TI_EPI_QKV_ROPE_KV
-      const int p = e.pos[m];
-      if (in_q || in_k) {
-        // (cos, sin) of pairs d / 2 and d / 2 + 1: even output fmaf(-odd, sin, even * cos), odd
-        // output fmaf(odd, cos, even * sin) (epilogue_mb with partner = the other of the pair)
-        const float4 cs = *(const float4*)(e.rope_cs + (size_t)p * hd + d);
-        const float r0 = fmaf(-v.y, cs.y, v.x * cs.x), r1 = fmaf(v.y, cs.x, v.x * cs.y);
-        const float r2 = fmaf(-v.w, cs.w, v.z * cs.z), r3 = fmaf(v.w, cs.z, v.z * cs.w);
-        if (in_q) {
-          *(float4*)((float*)e.out + (size_t)m * e.ldo + ng) = make_float4(r0, r1, r2, r3);
-        } else {
-          *(uint2*)(e.k_cache + (size_t)m * e.kv_stream_stride + ((size_t)kvh * e.max_seq + p) * hd + d) =
-              make_uint2(f2h(r0) | ((uint32_t)f2h(r1) << 16), f2h(r2) | ((uint32_t)f2h(r3) << 16));
-        }
-      } else {
-        *(uint2*)(e.v_cache + (size_t)m * e.kv_stream_stride + ((size_t)kvh * e.max_seq + p) * hd + d) =
-            make_uint2(f2h(v.x) | ((uint32_t)f2h(v.y) << 16), f2h(v.z) | ((uint32_t)f2h(v.w) << 16));
+  for (int it = 0; it < RB; ++it) v[it] = *(const float4*)(stg + (16 * it + (lane >> 2)) * kTileEpiStride + c4);
+  if (e.kind == TI_EPI_STORE_F32) {
+#pragma unroll
+    for (int it = 0; it < RB; ++it)
+      if (m0 + 16 * it < a.M) *(float4*)((float*)e.out + (size_t)(m0 + 16 * it) * e.ldo + ng) = v[it];
+  } else if (e.kind == TI_EPI_RESID_F32) {
+#pragma unroll
+    for (int it = 0; it < RB; ++it) {
+      const float4 h = p.v[it];
+      if (m0 + 16 * it < a.M)
+        *(float4*)((float*)e.out + (size_t)(m0 + 16 * it) * e.ldo + ng) = make_float4(h.x + v[it].x, h.y + v[it].y, h.z + v[it].z, h.w + v[it].w);
+    }
+  } else {   // TI_EPI_QKV_ROPE_KV
+    const TileQkv t = tile_qkv(e, tn);
+    const int hd = e.head_dim, d = t.d + c4;
+    if (t.q || t.k)
+      // (cos, sin) of pairs d / 2 and d / 2 + 1: even output fmaf(-odd, sin, even * cos), odd
+      // output fmaf(odd, cos, even * sin) (epilogue_mb with partner = the other of the pair)
+#pragma unroll
+      for (int it = 0; it < RB; ++it) {
+        const float4 cs = p.v[it], x = v[it];
+        v[it] = make_float4(fmaf(-x.y, cs.y, x.x * cs.x), fmaf(x.y, cs.x, x.x * cs.y), fmaf(-x.w, cs.w, x.z * cs.z), fmaf(x.w, cs.z, x.z * cs.w));
       }
+    uint16_t *kc = e.k_cache, *vc = e.v_cache;
+    asm("" : "+s"(kc), "+s"(vc));   // (values: a choice between the argument's fields would copy it to scratch)
+    uint16_t* cache = t.k ? kc : vc;
+#pragma unroll
+    for (int it = 0; it < RB; ++it) {
+      const int m = m0 + 16 * it;
+      if (m >= a.M) continue;
+      if (t.q)
+        *(float4*)((float*)e.out + (size_t)m * e.ldo + ng) = v[it];
+      else
+        *(uint2*)(cache + (size_t)m * e.kv_stream_stride + ((size_t)t.head * e.max_seq + p.pos[it]) * hd + d) =
+            make_uint2(f2h(v[it].x) | ((uint32_t)f2h(v[it].y) << 16), f2h(v[it].z) | ((uint32_t)f2h(v[it].w) << 16));
     }
   }
 }

@@ -184,7 +184,10 @@ __global__ __launch_bounds__(64 * kFewWaves, 2) void gemm_few_kernel(const GemvA
   const bool fold_in = a.epi.ss_in != nullptr;
   float* rmsv = (float*)smem;
   const float share = fold_in ? wide_fold_share(a, tid % C::kRows, tid / C::kRows, 64 * NW / C::kRows) : 0.0f;
+  TilePre<TM> pre;   // (of the tile that this wave finishes)
+  tile_pos<TM>(a, 0, lane, pre);
   product();
+  if (wave < TN) tile_pre<TM>(a, min(t0 + wave, NT - 1), 0, lane, pre);
   if (fold_in) {
     wide_fold_rms<C::kRows, NW>(a, share, tid, rmsv);
     auto marked = [&]() __attribute__((always_inline)) {   // (a row's rms is negative)
@@ -227,7 +230,7 @@ __global__ __launch_bounds__(64 * kFewWaves, 2) void gemm_few_kernel(const GemvA
           stg[row * kTileEpiStride + r] = fold_in ? av[b][i] / fabsf(rmsv[row]) : av[b][i];
         }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      wide_tile_out<TM>(a, tn, 0, stg, lane, r, kq, fold_out, hsq, psq);
+      wide_tile_out<TM>(a, tn, 0, stg, lane, r, kq, fold_out, pre, hsq, psq);
     }
     if (fold_out) wide_fold_part<TM>((float2*)(smem + C::kSs) + t * C::kRows, hsq, psq, lane);
   }

@@ -291,6 +291,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const GemvAr
   // batched fold (decode rows, ti_hip.h TI_FOLD_SS_ROWS): this thread's share of its row's sum of squares
   const bool fold_in = C::kFold && a.epi.ss_in != nullptr;
   const float share = fold_in ? wide_fold_share(a, m0 + tid % C::kRows, tid / C::kRows, 64 * NW / C::kRows) : 0.0f;
+  TilePre<TM> pre;
+  if constexpr (TN == 1) tile_pos<TM>(a, m0 + wm * 16 * TM, lane, pre);
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * C::kDma) : "memory");
   lds_barrier();
   Step st[2];
@@ -337,6 +339,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const GemvAr
       }
   };
   last();
+  if constexpr (TN == 1) tile_pre<TM>(a, min(t0 + wn * TN, NT - 1), m0 + wm * 16 * TM, lane, pre);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the clamped stages past the end
   lds_barrier();
 
@@ -402,6 +405,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const GemvAr
   float hsq[TM], psq[TM];
 #pragma unroll
   for (int b = 0; b < TM; ++b) hsq[b] = psq[b] = 0.0f;
+  if constexpr (TN > 1) tile_pos<TM>(a, mb, lane, pre);
 #pragma unroll 1
   for (int t = 0; t < TN; ++t) {   // (rolled: the tile's accumulators by static selects, so acc stays in registers)
     const int tn = t0 + wn * TN + t;
@@ -412,13 +416,14 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const GemvAr
 #pragma unroll
         for (int b = 0; b < TM; ++b) av[b] = acc[tt][b];
     if (tn >= NT) continue;
+    if constexpr (TN > 1) tile_pre<TM>(a, tn, mb, lane, pre);
 #pragma unroll
     for (int b = 0; b < TM; ++b)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         stg[(b * 16 + 4 * kq + i) * kTileEpiStride + r] = fold_in ? av[b][i] / rms[b][i] : av[b][i];
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    wide_tile_out<TM>(a, tn, mb, stg, lane, r, kq, fold_out, hsq, psq);
+    wide_tile_out<TM>(a, tn, mb, stg, lane, r, kq, fold_out, pre, hsq, psq);
   }
   if (fold_out) {   // this column block's sum of h^2 per row, column-waves in order
     float2* red = (float2*)(smem + C::kEpiRed);

@@ -124,12 +124,12 @@ __device__ __forceinline__ void wide_refold(const GemvArgs& a, int wave, int lan
   lds_barrier();
 }
 
-// One weight tile's outputs (16 columns from tn) for the 16 TM rows from mb, from the wave's staging block.  fold_out: the
-// residual add and the next call's folded input; hsq, psq: the lane's sums of h^2 and of (h w)^2, the latter infinite where an
+// One weight tile's outputs (16 columns from tn) for the 16 TM rows from mb, from the wave's staging block and what tile_pre
+// fetched.  fold_out: the residual add and the next call's folded input; hsq, psq: the lane's sums of h^2 and of (h w)^2, the latter infinite where an
 // |h w| passes 65504 (wide_fold_part).
 template <int TM>
 __device__ __forceinline__ void wide_tile_out(const GemvArgs& a, int tn, int mb, const float* stg, int lane, int r, int kq, bool fold_out,
-                                              float (&hsq)[TM], float (&psq)[TM]) {
+                                              const TilePre<TM>& pre, float (&hsq)[TM], float (&psq)[TM]) {
   const ti_epilogue& e = a.epi;
   if (fold_out) {   // residual add + the next call's folded input (fp16(h * w), sum of h^2 per row)
     const int c4 = 4 * (lane & 3), ng = tn * 16 + c4;
@@ -141,7 +141,7 @@ __device__ __forceinline__ void wide_tile_out(const GemvArgs& a, int tn, int mb,
       float q = 0.0f;
       if (m < a.M) {
         float4* o = (float4*)((float*)e.out + (size_t)m * e.ldo + ng);
-        const float4 h0 = *o, h = make_float4(h0.x + v.x, h0.y + v.y, h0.z + v.z, h0.w + v.w);
+        const float4 h0 = pre.v[it], h = make_float4(h0.x + v.x, h0.y + v.y, h0.z + v.z, h0.w + v.w);
         *o = h;
         float p[4] = {h.x * w.x, h.y * w.y, h.z * w.z, h.w * w.w};
         // (largest |p|; as outputs the products are rounded on their own, as in mul_f16)
@@ -156,7 +156,7 @@ __device__ __forceinline__ void wide_tile_out(const GemvArgs& a, int tn, int mb,
       hsq[it] += q + lane_xor<2>(q);
     }
   } else if (a.vec) {
-    tile_epilogue_lds<TM>(a, tn, mb, stg, lane);
+    tile_epilogue_lds<TM>(a, tn, mb, stg, lane, pre);
   } else {
 #pragma unroll 1
     for (int q = 0; q < TM * 4; ++q) {
