@@ -34,12 +34,16 @@ $(BUILD)/k_ops_exact.o: turboinfer_amd/csrc/kernels/ops_exact.hip $(HDRS)
 	$(HIPCC) $(DEVFLAGS) -ffp-contract=off -c $< -o $@
 
 # gemv: preload its leading kernel arguments into SGPRs (gfx950 kernarg preload).
-# gemv, gemm_wide, gemm_few, attention and qkv_attn compile without fp contraction (the rounding sequence the parity tests pin).
+# gemv, gemm_wide, gemm_block, gemm_few, attention and qkv_attn compile without fp contraction (the rounding sequence the parity tests pin).
 $(BUILD)/k_gemv.o: turboinfer_amd/csrc/kernels/gemv.hip $(HDRS)
 	@mkdir -p $(BUILD)
 	$(HIPCC) $(DEVFLAGS) -ffp-contract=off -mllvm -amdgpu-kernarg-preload-count=16 -c $< -o $@
 
 $(BUILD)/k_gemm_wide.o: turboinfer_amd/csrc/kernels/gemm_wide.hip $(HDRS)
+	@mkdir -p $(BUILD)
+	$(HIPCC) $(DEVFLAGS) -ffp-contract=off -c $< -o $@
+
+$(BUILD)/k_gemm_block.o: turboinfer_amd/csrc/kernels/gemm_block.hip $(HDRS)
 	@mkdir -p $(BUILD)
 	$(HIPCC) $(DEVFLAGS) -ffp-contract=off -c $< -o $@
 

@@ -369,3 +369,69 @@ def test_step_with_large_residuals(ti, bits):
     for got, ref in zip(*out):
         assert np.isfinite(got).all() and np.isfinite(ref).all()
         assert np.abs(got - ref).max() <= 1e-2 * np.abs(ref).max(), (np.abs(got - ref).max(axis=1), np.abs(ref).max())
+
+
+# the block kernel (gemm_block.hip): the fewest rows, the last block of rows by one row, one group of k (waves without one of their
+# own), 2, 3, 5, 7, 11, 17 and 24 of them (its ring of 2 or 3 slots and the last stages), a last block of columns of 1 .. 15 tiles, each
+# block shape; the outputs it writes, rows of a pitch of their own, with fp16 rows of one where 16-byte pieces are not aligned
+@pytest.mark.parametrize("M,K,N", [(65, 128, 16), (97, 384, 1040), (129, 256, 4112), (500, 2176, 2064), (97, 896, 16400), (257, 640, 12304),
+                                   (512, 640, 12304), (577, 640, 16400), (1024, 1408, 2576), (97, 3072, 8208), (161, 3072, 11280)])
+@pytest.mark.parametrize("bits", [4, 8, 16])
+def test_rows_block(ti, oracle, bits, M, K, N):
+    rng = np.random.RandomState(M * 3 + K + N + bits)
+    td, sd, w = weight(ti, oracle, bits, K, N, rng)
+    ldx, ldo = K + 8 * (M % 3), N + 4
+    x = rng.standard_normal((M, ldx)).astype(f16)
+    xd, xa = dev(ti, x), x[:, :K].astype(f32)
+    ref = xa.astype(np.float64) @ w.astype(np.float64)
+
+    def run(kind, out):
+        ep = ti.Epilogue()
+        ep.kind, ep.ldo, ep.out = kind, ldo, out.ptr
+        rows(ti, bits, td, sd, xd, M, N, K, ep, ldx, kernel=ti.ROWS_BLOCK)
+
+    r = rng.standard_normal((M + 1, ldo)).astype(f32)
+    yd, rd, hd = ti.DeviceBuffer(r.nbytes), dev(ti, r), ti.DeviceBuffer(r.nbytes // 2)
+    yd.zero()
+    hd.zero()
+    run(ti.EPI_STORE_F32, yd)
+    run(ti.EPI_RESID_F32, rd)
+    run(ti.EPI_SILU_MUL_F16, hd)
+    y, h = yd.download(f32, r.shape), hd.download(f16, r.shape)
+    assert_close_dot(y[:M, :N], ref, xa, w)
+    assert not y[M].any() and not y[:, N:].any()
+    np.testing.assert_array_equal(rd.download(f32, r.shape), r + y)   # one addition to the same sums
+    g = y[:M, :N].astype(np.float64).reshape(M, N // 16, 2, 8)
+    sil = (g[:, :, 1] * (g[:, :, 0] / (1 + np.exp(-g[:, :, 0])))).reshape(M, N // 2)
+    # (fp32 arithmetic of ~ 1e-6 and fp16's rounding, 2^-11)
+    np.testing.assert_allclose(h[:M, : N // 2].astype(np.float64), sil, rtol=2.0 ** -11 + 1e-5, atol=2.0 ** -25)
+    assert not h[M].any() and not h[:, N // 2:].any()
+
+
+@pytest.mark.parametrize("bits", [4, 8, 16])
+@pytest.mark.parametrize("hd,M", [(16, 65), (48, 200), (128, 130)])
+def test_rows_block_qkv(ti, oracle, bits, hd, M):
+    """Queries, keys and values of a prompt chunk: the many-rows kernel's on the same rows, to the order of the sums; streams of
+    their own where the rows belong to several."""
+    heads, kvh, K, S = 6, 2, 640, 256
+    qd, kd = heads * hd, kvh * hd
+    N, rng = qd + 2 * kd, np.random.RandomState(hd + bits)
+    td, sd, _ = weight(ti, oracle, bits, K, N, rng)
+    xd, pd = dev(ti, rng.standard_normal((M, K)).astype(f16)), dev(ti, rng.permutation(S)[:M].astype(np.int32))
+    cs = dev(ti, ti.rope_table(np.arange(S), hd, 10000.0))
+    stride = kvh * S * hd if M < 100 else 0
+    outs = []
+    for kernel in (ti.ROWS_MANY, ti.ROWS_BLOCK):
+        n = kvh * S * hd * (M if stride else 1)
+        q, k, v = ti.DeviceBuffer(M * qd * 4), ti.DeviceBuffer(n * 2), ti.DeviceBuffer(n * 2)
+        for b in (k, v):
+            b.zero()
+        ep = ti.Epilogue()
+        ep.kind, ep.ldo, ep.out, ep.q_dim, ep.kv_dim, ep.head_dim, ep.max_seq = ti.EPI_QKV_ROPE_KV, qd, q.ptr, qd, kd, hd, S
+        ep.pos, ep.rope_cs, ep.k_cache, ep.v_cache, ep.kv_stream_stride = pd.ptr, cs.ptr, k.ptr, v.ptr, stride
+        rows(ti, bits, td, sd, xd, M, N, K, ep, kernel=kernel)
+        outs.append([q.download(f32, (M, qd)), k.download(f16, (n,)).astype(f32), v.download(f16, (n,)).astype(f32)])
+    # (sums of 640 products of ~ 0.03: their fp32 rounding in either order is below 1e-5; fp16 rows may round apart by a step)
+    np.testing.assert_allclose(outs[0][0], outs[1][0], rtol=1e-5, atol=1e-5)
+    for a, b in zip(outs[0][1:], outs[1][1:]):
+        np.testing.assert_allclose(a, b, rtol=2.0 ** -10, atol=1e-5)

@@ -110,11 +110,9 @@ __device__ __forceinline__ bool wide_merge(const GemvArgs& a, f32x4 (&acc)[TN][T
 // to share a dequantised tile), small row counts and fp16 by the copies into a CU (~ 45 KB/us with the
 // hand-overs of the stages; plain reads reach 110), so a block
 // keeps 64 rows as soon as the call has them.  DMA straight to LDS leaves the registers to the accumulators; the
-// next stage's unpacking is interleaved with this one's MFMAs.  Measured inside a pass, us (fused kernel in 16-row
-// pieces / tile and batched-rows kernels -> this one): int8 1000 rows 2048 -> 11264 63 x 22.8 -> 79, fp16 333 rows the
-// same 21 x 25.7 -> 33; int4 64 rows 4096 -> 12288 24.0 -> 23.1, 4096 -> 22016 32.6 -> 29.0, the mean of 4096 -> 4096 and
-// 11008 -> 4096 18.1 -> 17.2; int4 512 rows 4096 -> 12288 65.0 -> 62.4, 4096 -> 22016 113.6 -> 114.9 (1 % slower, the
-// layer's four together 0.8 % faster).
+// next stage's unpacking is interleaved with this one's MFMAs.  Measured inside a pass, us (tile and batched-rows
+// kernels -> this one): int4 64 rows 4096 -> 12288 24.0 -> 23.1, 4096 -> 22016 32.6 -> 29.0, the mean of 4096 -> 4096 and
+// 11008 -> 4096 18.1 -> 17.2.  (Prompt chunks: gemm_block.hip.)
 //
 // Block of 16 TM WM rows x 16 TN WN columns per workgroup; wave (wm, wn) owns 16 TM rows x TN weight tiles.  A
 // stage is one 128-k group of the block: the rows' activations (chunks XOR-swizzled by row, tile_swz), the packed
@@ -551,21 +549,33 @@ int wide_launch(int fmt, const WidePlan& p, const GemvArgs& a, hipStream_t strea
 
 // Which kernel a call of ti_gemm_rows takes: the few-rows one where its estimate is the lower (the many-rows kernel's is 8 % low
 // for calls of up to 48 rows; the choice costs 0.6 % more than the better one of each of 1000 measured points, in the mean).
+// block: the call has more rows than a fold's and an output gemm_block_kernel writes.  It takes the call where its estimate is
+// below the many-rows kernel's (0.95 of it for fp16: from there up the many-rows kernel was the faster as often as not); that one
+// keeps what it splits over K, few rows by narrow outputs (us, many-rows / block, int4 11008 -> 4096: 65 rows 23.0 / 37.5, 128
+// rows 25.2 / 38.5, 512 rows 64 / 56), and short K, where the blocks' ends weigh.
 struct RowsPlan {
-  bool few;
+  int kernel;   // TI_ROWS_FEW, _MANY or _BLOCK
   ti::FewPlan f;
   ti::WidePlan w;
+  ti::BlockPlan b;
+  int n_cb() const { return kernel == TI_ROWS_FEW ? f.n_cb : kernel == TI_ROWS_MANY ? w.n_cb : b.n_cb; }
 };
-static bool rows_plan_of(int kernel, int bits, int M, int N, int K, int64_t ws_bytes, bool fold, RowsPlan* p) {
-  const bool wide = kernel != TI_ROWS_FEW && ti::wide_plan(bits, M, N, K, ti::gemm_cus(), ws_bytes, fold, &p->w);
-  p->few = kernel != TI_ROWS_MANY && ti::few_plan(bits, M, N, K, ti::gemm_cus(), &p->f) && (!wide || p->f.us < 1.08f * p->w.us);
-  return p->few || wide;
+static bool rows_plan_of(int kernel, int bits, int M, int N, int K, int64_t ws_bytes, bool fold, bool block, RowsPlan* p) {
+  const int cus = ti::gemm_cus();
+  auto asked = [&](int k) { return kernel == TI_ROWS_AUTO || kernel == k; };
+  const bool wide = asked(TI_ROWS_MANY) && ti::wide_plan(bits, M, N, K, cus, ws_bytes, fold, &p->w);
+  p->kernel = wide ? TI_ROWS_MANY : TI_ROWS_AUTO;
+  if (asked(TI_ROWS_FEW) && ti::few_plan(bits, M, N, K, cus, &p->f) && (!wide || p->f.us < 1.08f * p->w.us)) p->kernel = TI_ROWS_FEW;
+  if (asked(TI_ROWS_BLOCK) && block && ti::block_plan(bits, M, N, K, cus, &p->b) && (!wide || p->b.us < (bits == 16 ? 0.95f : 1.0f) * p->w.us))
+    p->kernel = TI_ROWS_BLOCK;
+  return p->kernel != TI_ROWS_AUTO;
 }
 
 extern "C" int ti_gemm_rows_fold_partials_on(int kernel, int bits, int M, int N, int K, int64_t ws_bytes) {
   RowsPlan p;
-  if (M > TI_FOLD_SS_ROWS || kernel < TI_ROWS_AUTO || kernel > TI_ROWS_MANY || !rows_plan_of(kernel, bits, M, N, K, ws_bytes, true, &p)) return 0;
-  return p.few ? p.f.n_cb : p.w.n_cb;
+  if (M > TI_FOLD_SS_ROWS || kernel < TI_ROWS_AUTO || kernel > TI_ROWS_BLOCK || !rows_plan_of(kernel, bits, M, N, K, ws_bytes, true, false, &p))
+    return 0;
+  return p.n_cb();
 }
 extern "C" int ti_gemm_rows_fold_partials(int bits, int M, int N, int K, int64_t ws_bytes) {
   return ti_gemm_rows_fold_partials_on(TI_ROWS_AUTO, bits, M, N, K, ws_bytes);
@@ -575,7 +585,7 @@ static int rows_impl(int kernel, const void* tiles, const uint16_t* scales, int 
                      float eps, int M, int N, int K, const ti_epilogue* epi, ti_stream_t stream) {
   using namespace ti;
   if (!tiles || !x || !epi || !epi->out) return ti_set_error(TI_ERR_ARG, "ti_gemm_rows: null pointer");
-  if (kernel < TI_ROWS_AUTO || kernel > TI_ROWS_MANY) return ti_set_error(TI_ERR_ARG, "ti_gemm_rows: kernel %d", kernel);
+  if (kernel < TI_ROWS_AUTO || kernel > TI_ROWS_BLOCK) return ti_set_error(TI_ERR_ARG, "ti_gemm_rows: kernel %d", kernel);
   if (bits != 16 && !scales) return ti_set_error(TI_ERR_ARG, "ti_gemm_rows: scales required for bits %d", bits);
   if (M < 1 || M > TI_GEMM_MAX_ROWS || K <= 0 || (K & 127) || N <= 0 || (N & 15) || ldx < K || K > 0xffff || ldx > 0xffff)
     return ti_set_error(TI_ERR_ARG, "ti_gemm_rows: M=%d N=%d K=%d ldx=%d", M, N, K, ldx);
@@ -608,12 +618,17 @@ static int rows_impl(int kernel, const void* tiles, const uint16_t* scales, int 
     a.norm_w = norm_w;
     a.epi.fold_w = h;
   }
-  if (!rows_plan_of(kernel, bits, M, N, K, epi->splitk_ws ? epi->splitk_bytes : 0, epi->ss_in || fold_out, &p))
+  const bool fold = epi->ss_in || fold_out, block = !fold && a.vec;   // (a.vec: fp32, residual, SiLU and query-key-value outputs)
+  if (!rows_plan_of(kernel, bits, M, N, K, epi->splitk_ws ? epi->splitk_bytes : 0, fold, block, &p))
     return ti_set_error(TI_ERR_UNSUPPORTED, "ti_gemm_rows: bits %d, M=%d N=%d K=%d", bits, M, N, K);
   const int rp = ti_gemm_prepare();   // no-op once this device is prepared
   if (rp != TI_OK) return rp;
-  a.stamp = ti_stamp_next(STAMP_TILE, p.few ? few_workgroups(p.f) : wide_workgroups(p.w));
-  return p.few ? few_launch(bits, p.f, a, (hipStream_t)stream) : wide_launch(bits, p.w, a, (hipStream_t)stream);
+  const hipStream_t s = (hipStream_t)stream;
+  switch (p.kernel) {
+    case TI_ROWS_FEW: a.stamp = ti_stamp_next(STAMP_TILE, few_workgroups(p.f)); return few_launch(bits, p.f, a, s);
+    case TI_ROWS_MANY: a.stamp = ti_stamp_next(STAMP_TILE, wide_workgroups(p.w)); return wide_launch(bits, p.w, a, s);
+    default: a.stamp = ti_stamp_next(STAMP_TILE, block_workgroups(p.b)); return block_launch(bits, p.b, a, s);
+  }
 }
 
 extern "C" int ti_gemm_rows(const void* tiles, const uint16_t* scales, int bits, const void* x, int ldx, float eps, int M, int N,

@@ -216,4 +216,14 @@ long few_workgroups(const FewPlan& p);
 int few_launch(int fmt, const FewPlan& p, const GemvArgs& a, hipStream_t s);
 int few_prepare();
 
+// gemm_block.hip: prompt chunks (more than TI_FOLD_SS_ROWS rows; outputs of whole 16-byte pieces, a.vec)
+struct BlockPlan {
+  int shape, n_cb, n_rb;   // workgroup shape, column blocks x row blocks
+  float us;                // estimate
+};
+bool block_plan(int fmt, int M, int N, int K, int cus, BlockPlan* p);
+long block_workgroups(const BlockPlan& p);
+int block_launch(int fmt, const BlockPlan& p, const GemvArgs& a, hipStream_t s);
+int block_prepare();
+
 }  // namespace ti

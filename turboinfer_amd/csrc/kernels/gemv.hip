@@ -1368,6 +1368,7 @@ extern "C" int ti_gemm_prepare(void) {
                  "hipFuncSetAttribute(gemv_wq_kernel)");
   int rc = wide_prepare();
   if (rc == TI_OK) rc = few_prepare();
+  if (rc == TI_OK) rc = block_prepare();
   if (rc != TI_OK) return rc;
   g_prepared.fetch_or(bit, std::memory_order_acq_rel);
   return TI_OK;
