@@ -435,3 +435,30 @@ def test_rows_block_qkv(ti, oracle, bits, hd, M):
     np.testing.assert_allclose(outs[0][0], outs[1][0], rtol=1e-5, atol=1e-5)
     for a, b in zip(outs[0][1:], outs[1][1:]):
         np.testing.assert_allclose(a, b, rtol=2.0 ** -10, atol=1e-5)
+
+
+# the few-rows kernel's blocks of 3, 4 and 6 tiles, and of 2 at 48 rows (other formats of a size: of 3), a last block short by 1 .. 5
+@pytest.mark.parametrize("M,K,N", [(16, 384, 11296), (13, 2176, 12336), (5, 896, 22064), (31, 1152, 11296), (32, 384, 16432), (47, 2176, 5648)])
+@pytest.mark.parametrize("bits", [4, 8, 4 | G32, 8 | G32])
+def test_rows_few_wide_blocks(ti, oracle, bits, M, K, N):
+    """A folded input into the residual with a folded output."""
+    rng = np.random.RandomState(M + K + N + bits)
+    td, sd, w = weight(ti, oracle, bits, K, N, rng)
+    h, r = rng.standard_normal((M, K)).astype(f32), rng.standard_normal((M + 1, N)).astype(f32)
+    nw, ow = (1 + 0.1 * rng.standard_normal(K)).astype(f32), (1 + 0.1 * rng.standard_normal(N)).astype(f32)
+    x, sq = (h * nw).astype(f16), np.zeros((1, 64), f32)
+    sq[0, :M] = (h.astype(np.float64) ** 2).sum(axis=1)
+    xd, sqd, rd, owd, fx = dev(ti, x), dev(ti, sq), dev(ti, r), dev(ti, ow), ti.DeviceBuffer(M * N * 2)
+    n_ss = ti.lib().ti_gemm_rows_fold_partials_on(ti.ROWS_FEW, bits, M, N, K, 0)
+    assert n_ss < N // 16   # (blocks of more than a tile)
+    ss = ti.DeviceBuffer(n_ss * 64 * 4)
+    ep = ti.Epilogue()
+    ep.kind, ep.ldo, ep.out, ep.ss_in, ep.n_ss = ti.EPI_RESID_F32, N, rd.ptr, sqd.ptr, 1
+    ep.fold_w, ep.fold_x, ep.fold_ss = owd.ptr, fx.ptr, ss.ptr
+    rows(ti, bits, td, sd, xd, M, N, K, ep, kernel=ti.ROWS_FEW)
+    got = rd.download(f32, (M + 1, N))
+    xf = x.astype(np.float64) / np.sqrt(sq[0, :M, None].astype(np.float64) / K + 1e-5)
+    assert_close_dot(got[:M] - r[:M], xf @ w.astype(np.float64), xf.astype(f32), w, rel=5e-5)
+    np.testing.assert_array_equal(got[M], r[M])
+    np.testing.assert_array_equal(fx.download(np.uint16, (M, N)), (got[:M] * ow).astype(f16).view(np.uint16))
+    np.testing.assert_allclose(ss.download(f32, (n_ss, 64))[:, :M].sum(axis=0), (got[:M].astype(np.float64) ** 2).sum(axis=1), rtol=1e-5)

@@ -24,8 +24,8 @@ struct FewCfg {
 // columns, K 5632, 24 rows 13.6 -> 9.8 us).  Against the many-rows
 // kernel (gemm_wide.hip), us, many-rows -> this: int8 2048 -> 2560 at 8 rows 7.3 -> 5.7, 24 rows 8.3 -> 6.9; 2048 -> 2048 6.6 ->
 // 5.0; 5632 -> 2048 8.6 -> 7.5; int4 4096 -> 12288 at 16 rows 12.2 -> 10.4, 11008 -> 4096 12.2 -> 10.9; blocks of 32 bytes'
-// 1024 -> 5632 at 24 rows 8.3 -> 6.3.  Wide outputs that take several rounds of workgroups stay with the many-rows
-// kernel (its workgroups share a row's copy among 64 columns): int4 4096 -> 28672 at 16 rows 17.3, here 19.2.
+// 1024 -> 5632 at 24 rows 8.3 -> 6.3.  Wide outputs that take several rounds of workgroups stay with the
+// many-rows kernel (its workgroups share a row's copy among 64 columns).
 template <int F, int TM, int TN>
 __global__ __launch_bounds__(64 * kFewWaves, 2) void gemm_few_kernel(const GemvArgs a) {
   typedef FewCfg<F, TM, TN> C;
@@ -243,8 +243,12 @@ __global__ __launch_bounds__(64 * kFewWaves, 2) void gemm_few_kernel(const GemvA
 }
 
 // ------------------------------------------------------------------ host: shapes, plan, launch
-// us of a launch, of a round over the 256 CUs and of a group per wave in it: fitted to ~ 1000 measured points (M 2 .. 48, N 512 ..
-// 32000, K 256 .. 14336, every format; where a shape is within 1/3 of the best).
+// us of a launch, of a round over the 256 CUs and of a group per wave in it: fitted to measured points (int4, int8 and blocks of 32:
+// 8 numbers of rows from 5 to 48 by 15 .. 18 (columns, K) from 1024 x 1024 to 32000 x 4096; where a shape is within 1/3 of the best).
+// Blocks of 3 tiles and more, and 2 at 48 rows, keep 5632 .. 22016 columns in one round, where the many-rows kernel took them or a
+// second round began.  us, before -> this: int4 2048 -> 11264 at 24 rows 8.8 -> 7.1, 4096 -> 12288 at 16 rows 9.1 -> 8.3, 32 rows 14.0 ->
+// 10.7, 4096 -> 6144 at 48 rows 13.9 -> 12.3; int8 2048 -> 11264 at 24 rows 9.7 -> 8.7; blocks of 32 bytes' 1024 -> 5632 at 40 rows
+// 9.7 -> 6.0.  (fp16: 16 x 48 spills and gains 0 .. 10 %.)
 struct FewShape {
   const void* fn;
   int rows, tiles, lds;
@@ -255,37 +259,43 @@ static FewShape few_shape(float fix, float round, float group) {
   typedef FewCfg<F, TM, TN> C;
   return {(const void*)gemm_few_kernel<F, TM, TN>, C::kRows, TN, C::kLds, fix, round, group};
 }
-constexpr int kFewShapes = 6;
+constexpr int kFewShapes = 11;
 template <int F>
-static const FewShape* few_shapes() {   // rows x columns: 16 x 16 | 16 x 32 | 32 x 16 | 32 x 32 (fp16: its weights spill) | 48 x 16 | 16 x 64 (int4)
+static const FewShape* few_shapes() {   // rows x columns: 16 x 16, 32, 48, 64, 96 | 32 x 16, 32 (fp16: its weights spill), 48, 64 | 48 x 16, 32
   if constexpr (F == 4) {
-    static const FewShape s[kFewShapes] = {few_shape<F, 1, 1>(2.64f, 1.19f, 0.529f), few_shape<F, 1, 2>(0.75f, 3.20f, 0.731f),
-                                           few_shape<F, 2, 1>(0.74f, 3.62f, 0.989f), few_shape<F, 2, 2>(0.62f, 3.80f, 1.165f),
-                                           few_shape<F, 3, 1>(1.07f, 3.81f, 1.378f), few_shape<F, 1, 4>(-1.74f, 5.73f, 1.260f)};
+    static const FewShape s[kFewShapes] = {few_shape<F, 1, 1>(2.155f, 0.744f, 0.627f), few_shape<F, 1, 2>(2.503f, 0.708f, 0.733f),
+                                           few_shape<F, 1, 3>(1.689f, 1.425f, 1.122f), few_shape<F, 1, 4>(0.775f, 2.378f, 1.356f),
+                                           few_shape<F, 1, 6>(1.618f, 1.482f, 2.109f), few_shape<F, 2, 1>(1.705f, 1.705f, 1.004f),
+                                           few_shape<F, 2, 2>(1.211f, 2.443f, 1.144f), few_shape<F, 2, 3>(0.75f, 3.18f, 1.384f),
+                                           few_shape<F, 2, 4>(-0.074f, 3.974f, 1.665f), few_shape<F, 3, 1>(1.944f, 1.944f, 1.335f),
+                                           few_shape<F, 3, 2>(0.957f, 2.992f, 1.707f)};
     return s;
   } else if constexpr (F == 8) {
-    static const FewShape s[kFewShapes] = {few_shape<F, 1, 1>(2.57f, 1.18f, 0.688f), few_shape<F, 1, 2>(1.55f, 2.27f, 0.990f),
-                                           few_shape<F, 2, 1>(0.45f, 3.76f, 1.173f), few_shape<F, 2, 2>(0.07f, 4.32f, 1.493f),
-                                           few_shape<F, 3, 1>(0.70f, 3.97f, 1.599f), {}};
+    static const FewShape s[kFewShapes] = {few_shape<F, 1, 1>(2.393f, 0.354f, 0.861f), few_shape<F, 1, 2>(2.024f, 0.93f, 1.172f),
+                                           few_shape<F, 1, 3>(1.131f, 1.238f, 2.023f), few_shape<F, 2, 1>(1.721f, 1.721f, 1.175f),
+                                           few_shape<F, 2, 2>(0.553f, 3.222f, 1.425f), few_shape<F, 2, 3>(0.737f, 2.437f, 2.25f),
+                                           few_shape<F, 3, 1>(1.877f, 1.877f, 1.6f), few_shape<F, 3, 2>(0.485f, 3.656f, 1.912f)};
     return s;
   } else if constexpr (F == 16) {
     static const FewShape s[kFewShapes] = {few_shape<F, 1, 1>(2.40f, 1.08f, 1.110f), few_shape<F, 1, 2>(-1.83f, 5.58f, 1.634f),
-                                           few_shape<F, 2, 1>(0.84f, 3.03f, 1.531f), {}, few_shape<F, 3, 1>(0.60f, 3.68f, 1.936f), {}};
+                                           few_shape<F, 2, 1>(0.84f, 3.03f, 1.531f), few_shape<F, 3, 1>(0.60f, 3.68f, 1.936f)};
     return s;
   } else if constexpr (F == (4 | TI_BITS_G32)) {
-    static const FewShape s[kFewShapes] = {few_shape<F, 1, 1>(1.50f, 2.56f, 0.516f), few_shape<F, 1, 2>(2.51f, 1.65f, 0.720f),
-                                           few_shape<F, 2, 1>(1.24f, 3.15f, 1.022f), few_shape<F, 2, 2>(-0.13f, 4.65f, 1.227f),
-                                           few_shape<F, 3, 1>(0.95f, 3.73f, 1.564f), {}};
+    static const FewShape s[kFewShapes] = {few_shape<F, 1, 1>(2.769f, 0.207f, 0.687f), few_shape<F, 1, 2>(2.626f, 0.44f, 0.902f),
+                                           few_shape<F, 1, 3>(1.89f, 0.783f, 1.613f), few_shape<F, 2, 1>(1.675f, 1.675f, 1.054f),
+                                           few_shape<F, 2, 2>(1.103f, 2.339f, 1.357f), few_shape<F, 2, 3>(1.512f, 1.689f, 2.06f),
+                                           few_shape<F, 3, 1>(0.879f, 2.81f, 1.464f), few_shape<F, 3, 2>(0.428f, 3.366f, 1.85f)};
     return s;
   } else if constexpr (F == (8 | TI_BITS_G32)) {
-    static const FewShape s[kFewShapes] = {few_shape<F, 1, 1>(2.70f, 1.07f, 0.768f), few_shape<F, 1, 2>(-0.57f, 4.47f, 1.073f),
-                                           few_shape<F, 2, 1>(0.96f, 3.34f, 1.136f), few_shape<F, 2, 2>(-0.81f, 4.98f, 1.652f),
-                                           few_shape<F, 3, 1>(0.83f, 3.92f, 1.579f), {}};
+    static const FewShape s[kFewShapes] = {few_shape<F, 1, 1>(2.451f, 0.298f, 0.915f), few_shape<F, 1, 2>(1.465f, 1.245f, 1.437f),
+                                           few_shape<F, 1, 3>(1.376f, 0.674f, 2.549f), few_shape<F, 2, 1>(-2.158f, 5.345f, 1.246f),
+                                           few_shape<F, 2, 2>(0.277f, 2.838f, 1.76f), few_shape<F, 2, 3>(0.914f, 1.589f, 2.866f),
+                                           few_shape<F, 3, 1>(0.763f, 2.694f, 1.695f), few_shape<F, 3, 2>(-0.171f, 3.767f, 2.15f)};
     return s;
   } else {
     static const FewShape s[kFewShapes] = {few_shape<F, 1, 1>(2.92f, 0.96f, 0.721f), few_shape<F, 1, 2>(-0.34f, 4.37f, 1.038f),
                                            few_shape<F, 2, 1>(1.21f, 3.09f, 1.199f), few_shape<F, 2, 2>(-0.32f, 4.74f, 1.656f),
-                                           few_shape<F, 3, 1>(0.86f, 3.91f, 1.661f), {}};
+                                           few_shape<F, 3, 1>(0.86f, 3.91f, 1.661f)};
     return s;
   }
 }

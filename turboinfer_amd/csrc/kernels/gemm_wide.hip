@@ -547,8 +547,9 @@ int wide_launch(int fmt, const WidePlan& p, const GemvArgs& a, hipStream_t strea
 
 }  // namespace ti
 
-// Which kernel a call of ti_gemm_rows takes: the few-rows one where its estimate is the lower (the many-rows kernel's is 8 % low
-// for calls of up to 48 rows; the choice costs 0.6 % more than the better one of each of 1000 measured points, in the mean).
+// Which kernel a call of ti_gemm_rows takes: the few-rows one where its estimate is the lower (the many-rows kernel's is 4 % (int4,
+// also in blocks of 32) or 8 % low for calls of up to 48 rows; the choice costs 0.1 .. 0.8 % more than the better one of each of 700
+// measured points, by format, in the mean).
 // block: the call has more rows than a fold's and an output gemm_block_kernel writes.  It takes the call where its estimate is
 // below the many-rows kernel's (0.95 of it for fp16: from there up the many-rows kernel was the faster as often as not); that one
 // keeps what it splits over K, few rows by narrow outputs (us, many-rows / block, int4 11008 -> 4096: 65 rows 23.0 / 37.5, 128
@@ -565,7 +566,8 @@ static bool rows_plan_of(int kernel, int bits, int M, int N, int K, int64_t ws_b
   auto asked = [&](int k) { return kernel == TI_ROWS_AUTO || kernel == k; };
   const bool wide = asked(TI_ROWS_MANY) && ti::wide_plan(bits, M, N, K, cus, ws_bytes, fold, &p->w);
   p->kernel = wide ? TI_ROWS_MANY : TI_ROWS_AUTO;
-  if (asked(TI_ROWS_FEW) && ti::few_plan(bits, M, N, K, cus, &p->f) && (!wide || p->f.us < 1.08f * p->w.us)) p->kernel = TI_ROWS_FEW;
+  if (asked(TI_ROWS_FEW) && ti::few_plan(bits, M, N, K, cus, &p->f) && (!wide || p->f.us < ((bits & ~TI_BITS_G32) == 4 ? 1.04f : 1.08f) * p->w.us))
+    p->kernel = TI_ROWS_FEW;
   if (asked(TI_ROWS_BLOCK) && block && ti::block_plan(bits, M, N, K, cus, &p->b) && (!wide || p->b.us < (bits == 16 ? 0.95f : 1.0f) * p->w.us))
     p->kernel = TI_ROWS_BLOCK;
   return p->kernel != TI_ROWS_AUTO;
