@@ -372,10 +372,11 @@ def test_step_with_large_residuals(ti, bits):
 
 
 # the block kernel (gemm_block.hip): the fewest rows, the last block of rows by one row, one group of k (waves without one of their
-# own), 2, 3, 5, 7, 11, 17 and 24 of them (its ring of 2 or 3 slots and the last stages), a last block of columns of 1 .. 15 tiles, each
-# block shape; the outputs it writes, rows of a pitch of their own, with fp16 rows of one where 16-byte pieces are not aligned
+# own), 2, 3, 5, 7, 9, 11, 17, 23 and 24 of them (its ring of 2 or 3 slots and the last stages, of up to 4 groups), a last block of
+# columns of 1 .. 15 tiles, each block shape; the outputs it writes, rows of a pitch of their own, with fp16 rows of one where 16-byte pieces are not aligned
 @pytest.mark.parametrize("M,K,N", [(65, 128, 16), (97, 384, 1040), (129, 256, 4112), (500, 2176, 2064), (97, 896, 16400), (257, 640, 12304),
-                                   (512, 640, 12304), (577, 640, 16400), (1024, 1408, 2576), (97, 3072, 8208), (161, 3072, 11280)])
+                                   (512, 640, 12304), (577, 640, 16400), (1024, 1408, 2576), (97, 3072, 8208), (161, 3072, 11280),
+                                   (65, 1152, 400), (66, 384, 3088), (70, 2944, 3088), (97, 2944, 4112)])
 @pytest.mark.parametrize("bits", [4, 8, 16])
 def test_rows_block(ti, oracle, bits, M, K, N):
     rng = np.random.RandomState(M * 3 + K + N + bits)

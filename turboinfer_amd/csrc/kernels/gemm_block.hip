@@ -407,8 +407,11 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_block_kernel(const GemvA
 
 // ------------------------------------------------------------------ host: shapes, plan, launch
 // Estimated us: fix + stages * max(alone, full * rounds) + round * rounds, a round being one workgroup on each CU (fitted, per
-// shape and format, to 13 numbers of rows from 65 to 1024 by 14 (columns, K) from 1024 x 2048 to 22016 x 4096 and 4096 x 11008
-// with the epilogues a model has there, weights from HBM).
+// shape and format, to 10 .. 13 numbers of rows from 65 to 1024 by 14 (columns, K) from 1024 x 2048 to 22016 x 4096 and 4096 x 11008
+// with the epilogues a model has there, weights from HBM).  Blocks of 32 rows and of 4 groups of waves are for grids that would leave
+// CUs idle or a wave a SIMD (us, without -> with, int4: 2048 -> 2048 at 128 rows 9.9 -> 7.3, 5632 -> 2048 at 333 22.4 -> 17.5, 4096 -> 12288 at
+// 150 30.8 -> 23.7; int8: 11008 -> 4096 at 150 38.8 -> 31.9, 5632 -> 2048 at 333 22.6 -> 19.4; fp16: 2048 -> 2560 at 128 11.3 -> 9.8; the
+// mean up to 640 rows 9 %, 6 % and 4 %).
 struct BlockShape {
   const void* fn;
   int rows, cols, groups, threads, lds;
@@ -423,37 +426,47 @@ struct BlockShapes {
   const BlockShape* s;
   int n;
 };
-static BlockShapes block_shapes_of(int fmt) {
+static BlockShapes block_shapes_of(int fmt) {   // rows x columns (by groups of waves)
   if (fmt == 4) {
     static const BlockShape s[] = {
         block_shape<4, 8, 1, 4, 1, 2>(0.0f, 0.368f, 1.432f, 7.200f),     // 128 x 256
         block_shape<4, 4, 1, 2, 2, 4>(1.294f, 0.946f, 0.803f, 3.204f),   // 64 x 256
         block_shape<4, 6, 1, 3, 1, 3>(0.855f, 1.039f, 1.029f, 4.991f),   // 96 x 192
-        block_shape<4, 4, 2, 2, 1, 3>(1.227f, 0.604f, 1.016f, 3.220f),   // 64 x 128 by 2 groups
+        block_shape<4, 4, 2, 2, 1, 3>(1.227f, 0.604f, 1.016f, 3.220f),   // 64 x 128 (2)
         block_shape<4, 4, 1, 2, 1, 3>(1.882f, 0.683f, 0.469f, 1.334f),   // 64 x 128
-        block_shape<4, 2, 2, 2, 1, 2>(2.332f, 0.807f, 0.636f, 1.092f)};  // 64 x 64 by 2 groups
-    return {s, 6};
+        block_shape<4, 4, 2, 1, 1, 3>(3.245f, 0.602f, 0.557f, 0.939f),   // 32 x 128 (2)
+        block_shape<4, 2, 4, 1, 1, 2>(2.771f, 0.801f, 0.688f, 1.218f),   // 32 x 64 (4)
+        block_shape<4, 2, 2, 1, 1, 3>(3.256f, 0.475f, 0.354f, 0.521f),   // 32 x 64 (2)
+        block_shape<4, 1, 4, 1, 1, 2>(2.905f, 0.654f, 0.503f, 0.789f)};  // 32 x 32 (4)
+    return {s, (int)(sizeof(s) / sizeof(s[0]))};
   }
   if (fmt == 8) {
     static const BlockShape s[] = {
         block_shape<8, 8, 1, 4, 1, 2>(0.0f, 1.171f, 1.539f, 7.474f),     // 128 x 256
-        block_shape<8, 4, 2, 4, 1, 2>(2.693f, 1.358f, 2.026f, 3.539f),   // 128 x 128 by 2 groups
+        block_shape<8, 4, 2, 4, 1, 2>(2.693f, 1.358f, 2.026f, 3.539f),   // 128 x 128 (2)
         block_shape<8, 4, 1, 4, 1, 2>(2.800f, 1.168f, 0.972f, 1.691f),   // 128 x 128
         block_shape<8, 6, 1, 3, 1, 3>(1.304f, 1.119f, 1.106f, 4.927f),   // 96 x 192
-        block_shape<8, 4, 2, 2, 1, 3>(0.571f, 0.379f, 1.097f, 4.039f),   // 64 x 128 by 2 groups
+        block_shape<8, 4, 2, 2, 1, 3>(0.571f, 0.379f, 1.097f, 4.039f),   // 64 x 128 (2)
         block_shape<8, 4, 1, 2, 1, 3>(3.613f, 0.597f, 0.550f, 0.396f),   // 64 x 128
-        block_shape<8, 2, 2, 2, 1, 2>(2.422f, 0.834f, 0.711f, 1.151f)};  // 64 x 64 by 2 groups
-    return {s, 7};
+        block_shape<8, 2, 4, 2, 1, 2>(1.490f, 1.272f, 1.335f, 3.557f),   // 64 x 64 (4)
+        block_shape<8, 2, 2, 2, 1, 2>(2.422f, 0.834f, 0.711f, 1.151f),   // 64 x 64 (2)
+        block_shape<8, 4, 2, 1, 1, 3>(2.706f, 0.771f, 0.758f, 1.251f),   // 32 x 128 (2)
+        block_shape<8, 2, 4, 1, 1, 2>(2.734f, 0.920f, 0.877f, 1.168f),   // 32 x 64 (4)
+        block_shape<8, 2, 2, 1, 1, 3>(2.489f, 0.539f, 0.445f, 0.716f),   // 32 x 64 (2)
+        block_shape<8, 1, 4, 1, 1, 2>(3.013f, 0.705f, 0.635f, 0.583f)};  // 32 x 32 (4)
+    return {s, (int)(sizeof(s) / sizeof(s[0]))};
   }
   if (fmt == 16) {
     static const BlockShape s[] = {
         block_shape<16, 8, 1, 4, 1, 2>(1.278f, 1.734f, 1.703f, 2.529f),   // 128 x 256
-        block_shape<16, 4, 2, 4, 1, 2>(1.963f, 1.301f, 2.077f, 2.948f),   // 128 x 128 by 2 groups
+        block_shape<16, 4, 2, 4, 1, 2>(1.963f, 1.301f, 2.077f, 2.948f),   // 128 x 128 (2)
         block_shape<16, 4, 1, 4, 1, 2>(3.563f, 1.155f, 1.016f, 0.0f),     // 128 x 128
         block_shape<16, 6, 1, 3, 1, 3>(3.988f, 1.243f, 1.228f, 0.279f),   // 96 x 192
         block_shape<16, 4, 1, 2, 1, 3>(2.426f, 0.835f, 0.702f, 0.0f),     // 64 x 128
-        block_shape<16, 2, 2, 2, 1, 2>(2.637f, 0.996f, 0.903f, 0.078f)};  // 64 x 64 by 2 groups
-    return {s, 6};
+        block_shape<16, 2, 2, 2, 1, 2>(2.637f, 0.996f, 0.903f, 0.078f),   // 64 x 64 (2)
+        block_shape<16, 2, 2, 1, 1, 3>(2.225f, 0.807f, 0.709f, 0.0f),     // 32 x 64 (2)
+        block_shape<16, 1, 4, 1, 1, 2>(3.066f, 0.913f, 0.886f, 0.186f)};  // 32 x 32 (4)
+    return {s, (int)(sizeof(s) / sizeof(s[0]))};
   }
   return {nullptr, 0};
 }

@@ -552,8 +552,8 @@ int wide_launch(int fmt, const WidePlan& p, const GemvArgs& a, hipStream_t strea
 // measured points, by format, in the mean).
 // block: the call has more rows than a fold's and an output gemm_block_kernel writes.  It takes the call where its estimate is
 // below the many-rows kernel's (0.95 of it for fp16: from there up the many-rows kernel was the faster as often as not); that one
-// keeps what it splits over K, few rows by narrow outputs (us, many-rows / block, int4 11008 -> 4096: 65 rows 23.0 / 37.5, 128
-// rows 25.2 / 38.5, 512 rows 64 / 56), and short K, where the blocks' ends weigh.
+// keeps few rows by long K, split over workgroups, where the two are even (us, many-rows / block: int4 14336 -> 4096 at 96 rows
+// 27.4 / 27.3, fp16 11008 -> 4096 at 128 rows 36.7 / 37.9), and short K, where the blocks' ends weigh.
 struct RowsPlan {
   int kernel;   // TI_ROWS_FEW, _MANY or _BLOCK
   ti::FewPlan f;
