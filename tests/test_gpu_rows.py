@@ -463,3 +463,52 @@ def test_rows_few_wide_blocks(ti, oracle, bits, M, K, N):
     np.testing.assert_array_equal(got[M], r[M])
     np.testing.assert_array_equal(fx.download(np.uint16, (M, N)), (got[:M] * ow).astype(f16).view(np.uint16))
     np.testing.assert_allclose(ss.download(f32, (n_ss, 64))[:, :M].sum(axis=0), (got[:M].astype(np.float64) ** 2).sum(axis=1), rtol=1e-5)
+
+
+# (block kernel: two row blocks of 32, the last one by a row, one of 64; 1, 2 and 4 groups of waves)
+@pytest.mark.parametrize("M,K,H,N", [(33, 384, 1152, 80), (40, 256, 1024, 4112), (33, 1152, 2048, 400), (50, 640, 22016, 2064),
+                                     (64, 2944, 4096, 12304), (64, 512, 12288, 208), (48, 384, 2944, 28688)])
+@pytest.mark.parametrize("bits", [4, 8, 16])
+def test_rows_block_fold(ti, oracle, ws, bits, M, K, H, N):
+    """Folds of up to 64 rows on the block kernel, into it and into the many-rows one, with rows that must be normalised first in its
+    first and last block.  Bounds: test_rows_fold_range's."""
+    L, rng = ti.lib(), np.random.RandomState(M + bits)
+    to, so, wo = weight(ti, oracle, bits, K, H, rng)
+    t2, s2, w2 = weight(ti, oracle, bits, H, N, rng)
+    act = rng.standard_normal((M, K)).astype(f16)
+    h0 = rng.standard_normal((M, H)).astype(f32)
+    nw = (1 + 0.1 * rng.standard_normal(H)).astype(f32)
+    nwd = dev(ti, nw)
+    for marked in (False, True):
+        if marked:
+            h0[1, [5, 600]] = 1e5, -3e5
+            h0[M - 1] *= 1e6
+            h0[2] *= 3e-7
+            act[2] = 0
+        bad = np.isin(np.arange(M), [1, 2, M - 1]) & marked
+        ad = dev(ti, act)
+        n_ss = L.ti_gemm_rows_fold_partials_on(ti.ROWS_BLOCK, bits, M, H, K, WS)
+        hd, fx, ss, yd = dev(ti, h0), ti.DeviceBuffer(M * H * 2), ti.DeviceBuffer(n_ss * 64 * 4), ti.DeviceBuffer(M * N * 4)
+        ep = ti.Epilogue()
+        ep.kind, ep.ldo, ep.out = ti.EPI_RESID_F32, H, hd.ptr
+        ep.fold_w, ep.fold_x, ep.fold_ss = nwd.ptr, fx.ptr, ss.ptr
+        rows(ti, bits, to, so, ad, M, H, K, ep, ws=ws, kernel=ti.ROWS_BLOCK)
+        h1 = hd.download(f32, (M, H))
+        assert_close_dot(h1[~bad] - h0[~bad], act[~bad].astype(np.float64) @ wo.astype(np.float64), act[~bad].astype(f32), wo, rel=5e-5)
+        sums, plain = ss.download(f32, (n_ss, 64))[:, :M], fx.download(np.uint16, (M, H))
+        np.testing.assert_allclose(np.abs(sums).sum(axis=0), (h1.astype(np.float64) ** 2).sum(axis=1), rtol=1e-5)
+        np.testing.assert_array_equal(np.signbit(sums).any(axis=0), bad)
+        with np.errstate(over="ignore"):
+            np.testing.assert_array_equal(plain, (h1 * nw).astype(f16).view(np.uint16))
+        x = h1 / np.sqrt((h1.astype(np.float64) ** 2).mean(axis=1) + 1e-5)[:, None] * nw
+        ref, tol = x @ w2, (2.0**-11 + H * 2.0**-24) * (np.abs(x) @ np.abs(w2)) + 2.0**-25 * np.abs(w2).sum(axis=0) + 1e-9
+        for second in (ti.ROWS_MANY, ti.ROWS_BLOCK):
+            out = []
+            for _ in range(2):   # (the second call over rows that the first rewrote)
+                ep = ti.Epilogue()
+                ep.kind, ep.ldo, ep.out, ep.ss_in, ep.n_ss = ti.EPI_STORE_F32, N, yd.ptr, ss.ptr, n_ss
+                rows(ti, bits, t2, s2, fx, M, N, H, ep, ws=ws, kernel=second, h=hd.ptr, norm_w=nwd.ptr)
+                out.append(yd.download(f32, (M, N)))
+            assert np.all(np.abs(out[0] - ref) <= tol), (marked, second)
+            np.testing.assert_array_equal(*out)
+        np.testing.assert_array_equal((fx.download(np.uint16, (M, H)) != plain).any(axis=1), bad)

@@ -1,5 +1,4 @@
-// gemm_block.hip -- packed weights x fp16 rows for prompt chunks (more rows than a batched fold's): int4 and int8 per group of
-// 128, and fp16.
+// gemm_block.hip -- packed weights x fp16 rows for prompt chunks and large batches: int4 and int8 per group of 128, and fp16.
 #include "gemm_wide.hpp"
 
 namespace ti {
@@ -38,15 +37,19 @@ struct BlockGemm {
   static constexpr int kFin = KG < RT ? KG : RT, kRf = RT / kFin;         // groups that finish row tiles, and how many each
   static constexpr int kPart = (KG - 1) * WN * CT * RT * 4096;            // the other groups' sums (behind the rows, once read)
   static constexpr int kEpi = kPart + kFin * WN * kTurn * 4, kLds = NS * kA > kEpi ? NS * kA : kEpi;
-  static_assert(kRows / 4 % WN == 0 && (kDma % 4 == 0 || kDma <= 2) && RT % kFin == 0 && kLds <= 160 * 1024);
+  // folds: the column-waves' sums of the next one, the threads' shares (kP a row) of this one's and the waves' marks
+  static constexpr int kRed = kEpi, kSums = NS * kA > kRed + WN * kRows * 8 ? NS * kA : kRed + WN * kRows * 8, kMarks = kSums + kWaves * 256;
+  static constexpr int kFoldLds = kMarks + kWaves * 4, kP = 64 * kWaves / kRows;
+  static_assert(kRows / 4 % WN == 0 && (kDma % 4 == 0 || kDma <= 2) && RT % kFin == 0 && kFoldLds <= 160 * 1024);
   static constexpr int vm(int n) { return n > 63 ? 63 : n; }
 };
 
 // The epilogue (a.vec; same arithmetic as epilogue_mb): acc[t][b] are columns 0 .. 15 of weight tile n + 2 t in row m + 32 b.  A
 // lane's 16 columns are 64 bytes (SiLU's 8 outputs 16) of one row, and what a row tile reads beside its products is in
 // flight together.
-template <int CT, int RT>
-__device__ __forceinline__ void block_out(const GemvArgs& a, f32x16 (&acc)[CT][RT], int n, int m, int NT) {
+// FOLD: a folded output also takes the next call's input, fp16(h w), and the lanes' sums of h^2 and (h w)^2 (wide_tile_out's) to hsq, psq.
+template <bool FOLD, int CT, int RT>
+__device__ __forceinline__ void block_out(const GemvArgs& a, f32x16 (&acc)[CT][RT], int n, int m, int NT, float (&hsq)[RT], float (&psq)[RT]) {
   typedef uint32_t u32x4a8 __attribute__((ext_vector_type(4), aligned(8)));
   const ti_epilogue& e = a.epi;
   auto pair = [](float lo, float hi) { return f2h(lo) | ((uint32_t)f2h(hi) << 16); };
@@ -77,7 +80,10 @@ __device__ __forceinline__ void block_out(const GemvArgs& a, f32x16 (&acc)[CT][R
   } else if (e.kind == TI_EPI_RESID_F32) {
 #pragma unroll
     for (int t = 0; t < CT; ++t) {
-      f32x4 h[RT][4];
+      f32x4 h[RT][4], w[4];
+      if (FOLD && e.fold_x)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) w[q] = *(const f32x4*)(e.fold_w + min(n + 2 * t, NT - 1) * 16 + 4 * q);
 #pragma unroll
       for (int b = 0; b < RT; ++b) {
         const f32x4* o = (const f32x4*)((const float*)e.out + (size_t)min(m + 32 * b, a.M - 1) * e.ldo + min(n + 2 * t, NT - 1) * 16);
@@ -90,6 +96,31 @@ __device__ __forceinline__ void block_out(const GemvArgs& a, f32x16 (&acc)[CT][R
         for (int i = 0; i < 16; ++i) acc[t][b][i] = h[b][i >> 2][i & 3] + acc[t][b][i];
         if (m + 32 * b < a.M && n + 2 * t < NT) store(acc[t][b], (float*)e.out + (size_t)(m + 32 * b) * e.ldo + (n + 2 * t) * 16);
       }
+      if (FOLD && e.fold_x)
+#pragma unroll
+        for (int b = 0; b < RT; ++b) {
+          const f32x16& v = acc[t][b];
+          float p[16], top = 0.0f, hs = 0.0f, ps = 0.0f;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) p[i] = v[i] * w[i >> 2][i & 3];
+#pragma unroll
+          for (int i = 0; i < 16; i += 4) {   // (as outputs the products are rounded on their own, as in mul_f16)
+            asm("v_max3_f32 %0, %0, |%1|, |%2|\n\tv_max3_f32 %0, %0, |%3|, |%4|" : "+v"(top), "+v"(p[i]), "+v"(p[i + 1]), "+v"(p[i + 2]), "+v"(p[i + 3]));
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              hs = fmaf(v[i + j], v[i + j], hs);
+              ps = fmaf(p[i + j], p[i + j], ps);
+            }
+          }
+          if (m + 32 * b < a.M && n + 2 * t < NT) {
+            uint16_t* o = e.fold_x + (size_t)(m + 32 * b) * e.ldo + (n + 2 * t) * 16;
+#pragma unroll
+            for (int i = 0; i < 16; i += 8)
+              *(u32x4a8*)(o + i) = (u32x4a8){pair(p[i], p[i + 1]), pair(p[i + 2], p[i + 3]), pair(p[i + 4], p[i + 5]), pair(p[i + 6], p[i + 7])};
+            hsq[b] += hs;
+            psq[b] += top > 65504.0f ? INFINITY : ps;
+          }
+        }
     }
   } else {   // TI_EPI_QKV_ROPE_KV: a tile lies in one of q / k / v and in one head (head_dim % 16 == 0)
     const int hd = e.head_dim;
@@ -134,6 +165,30 @@ __device__ __forceinline__ void block_out(const GemvArgs& a, f32x16 (&acc)[CT][R
   }
 }
 
+// A fold's sums (wide_fold_share), 8 of a thread's in flight: the first ones beside the first rows.
+__device__ __forceinline__ void block_share_load(const GemvArgs& a, int m, int b, int P, float (&v)[8]) {   // partials b, b + P, ..
+  constexpr uint32_t pitch = TI_FOLD_SS_ROWS * 4u;
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)a.epi.ss_in, 0, (uint32_t)a.epi.n_ss * pitch, 0x00020000);
+  const uint32_t o = m < a.M ? (uint32_t)b * pitch + (uint32_t)m * 4u : 0x80000000u;   // (past the end: 0)
+#pragma unroll
+  for (int j = 0; j < 8; ++j) v[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, o + (uint32_t)(j * P) * pitch, 0, 0));
+}
+__device__ __forceinline__ float block_share(const GemvArgs& a, int m, int part, int P, float (&v)[8]) {
+  float t = 0.0f;
+  uint32_t any = 0;
+  for (int b = part;;) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      t += fabsf(v[j]);
+      any |= __builtin_bit_cast(uint32_t, v[j]);
+    }
+    b += 8 * P;
+    if (b - part >= a.epi.n_ss) break;   // (uniform)
+    block_share_load(a, m, b, P, v);
+  }
+  return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, t) | (any & 0x80000000u));
+}
+
 // Bound: the vector unit beside the matrix cores, and the clock, which falls to 1.4 .. 2.0 GHz at this rate.  A 32x32x16 MFMA
 // holds the vector issue for ~ 8 cycles of its 32 and does twice a 16x16x32's work (7.5 of 16): as many scale FMAs per product
 // leave time for the unpacking.  The weights pass LDS by (each is read by one wave only): half the DMA, whose bursts with the
@@ -144,6 +199,10 @@ __device__ __forceinline__ void block_out(const GemvArgs& a, f32x16 (&acc)[CT][R
 // 2560 25.7 -> 22.5; fp16 333 rows 33.5 -> 25.4, 30.7 -> 23.5, 12.1 -> 11.2.  Whole prompts: 7B int4 of 512 rows 9159 -> 8184,
 // TinyLlama int8 of 1000 4346 -> 3807, fp16 of 333 2358 -> 2152.
 // Slices of K by workgroups, as gemm_wide_kernel has them, were no gain here beyond what it keeps.
+// FOLD: a batched fold's input or output.  The sums come in beside the first rows and are kept in LDS; rows that must be normalised
+// first are found before the products, not behind them (a loop around the products cost 27 registers), in calls of their own, as the
+// code costs the others 0 .. 2 us.  Steps of 64 streams of the 7B model, int4: 13 241 -> 12 943 us; prompts of 44 rows of TinyLlama
+// int8 1132 -> 1091, of 43 of Llama-3-8B int4 2719 -> 2608.
 //
 // Block of 32 RT rows x 32 CT WN columns per workgroup; wave (g, wn) owns all rows of 32 CT columns and the 128-k groups g, g +
 // KG, .. of the workgroup's (KG > 1: the groups meet in LDS at the end).  A stage is KG groups: their rows come to LDS by DMA, NS
@@ -151,7 +210,7 @@ __device__ __forceinline__ void block_out(const GemvArgs& a, f32x16 (&acc)[CT][R
 // straight to registers two groups ahead (fp16: one).  v_mfma_f32_32x32x16: lane l holds 8 k of row (column) l & 31; its k octet
 // s of the packed layout's quarter 2 j + (l >> 5) makes step u = 4 j + s, so a 32-column operand is two 16-column tiles' words as
 // they are packed.
-template <int F, int WN, int KG, int RT, int CT, int NS>
+template <int F, int WN, int KG, int RT, int CT, int NS, bool FOLD>
 __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_block_kernel(const GemvArgs a, int n_cb, int n_rb) {
   typedef BlockGemm<F, WN, KG, RT, CT, NS> C;
   typedef WideFmt<F> Fm;
@@ -174,7 +233,7 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_block_kernel(const GemvA
 #pragma unroll
   for (int q = 0; q < C::kDma; ++q) {   // (wave (g, wn) copies a share of group g's rows)
     const int row = 4 * (wn * C::kDma + q) + (lane >> 4), c = (lane & 15) ^ tile_swz(row);
-    // (rows_dma adds 1024 (q & 3): not more than the row's own offset, as a row is 256 bytes or more and M > 28)
+    // (rows_dma adds 1024 (q & 3): not more than the row's own offset, as a row is 256 bytes or more and M > 12)
     vx[q] = (uint32_t)min(m0 + row, a.M - 1) * (uint32_t)a.ldx * 2u + (uint32_t)c * 16u - (uint32_t)(q & 3) * 1024u;
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)smem + (uint32_t)(g * WN + wn) * (C::kDma * 1024u);
@@ -286,13 +345,39 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_block_kernel(const GemvA
     }
   };
 
-#pragma unroll
-  for (int q = 0; q < NS; ++q) issue(q, q);
+  const bool fold_in = FOLD && a.epi.ss_in != nullptr;
+  float* sums = (float*)(smem + C::kSums);
+  int* marks = (int*)(smem + C::kMarks);
   Set set[C::kSets];
+#pragma unroll 1
+  for (bool again = false;;) {   // (once, unless a fold's rows must be normalised first)
+    float fs[8];
+    const bool look = fold_in && !again;
+    if (look) block_share_load(a, m0 + tid % C::kRows, tid / C::kRows, C::kP, fs);
 #pragma unroll
-  for (int q = 0; q < C::kSets - 1; ++q) load_set(set[q], q);
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(C::vm((NS - 1) * C::kDma + (C::kSets - 1) * C::kLoads)) : "memory");
-  lds_barrier();
+    for (int q = 0; q < NS; ++q) issue(q, q);
+#pragma unroll
+    for (int q = 0; q < C::kSets - 1; ++q) load_set(set[q], q);
+    if (look) {
+      const float share = block_share(a, m0 + tid % C::kRows, tid / C::kRows, C::kP, fs);
+      sums[tid] = share;
+      if (a.norm_w) marks[wave] = __builtin_amdgcn_ballot_w64(__builtin_bit_cast(int32_t, share) < 0) != 0;
+    }
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(C::vm((NS - 1) * C::kDma + (C::kSets - 1) * C::kLoads)) : "memory");
+    lds_barrier();
+    if (!look || !a.norm_w) break;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(lane < C::kWaves && marks[lane < C::kWaves ? lane : 0]) == 0, 1)) break;
+    // a row has a mark: the marks counted, the rows that fp16 does not hold rewritten (every workgroup that reads them writes the same)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();
+    const float share = sums[tid];
+    float* rmsv = (float*)smem;
+    wide_fold_rms<C::kRows, C::kWaves>(a, share, tid, rmsv);
+    wide_fold_settle<C::kRows, C::kWaves>(a, m0, tid, rmsv);
+    sums[tid] = rmsv[tid % C::kRows] < 0.0f ? -fabsf(share) : fabsf(share);
+    wide_refold<C::kRows, C::kWaves>(a, m0, wave, lane, rmsv);
+    again = true;
+  }
   read_x(x[0], 0, 0);
 #pragma unroll
   for (int t = 0; t < CT; ++t) wq[t] = weights(set[0], t, 0);
@@ -377,16 +462,21 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_block_kernel(const GemvA
             for (int i = 0; i < 4; ++i) acc[t][b][4 * q + i] = v[i];
           }
   }
+  const bool fold_out = FOLD && a.epi.kind == TI_EPI_RESID_F32 && a.epi.fold_x != nullptr;
+  float2* red = (float2*)(smem + C::kRed);
   if (g < C::kFin)
 #pragma unroll
     for (int f = 0; f < C::kFin; ++f)
       if (f == g) {   // scaled sums: from a column's rows per lane to 16 columns of a row, by the wave's own block of LDS
         float* turn = (float*)(smem + C::kPart) + (g * WN + wn) * kTurn;
         f32x16 v[CT][C::kRf];
+        float hsq[C::kRf], psq[C::kRf];
 #pragma unroll
-        for (int t = 0; t < CT; ++t)
+        for (int b = 0; b < C::kRf; ++b) {
+          const int row = (f * C::kRf + b) * 32 + r;   // of the block
+          hsq[b] = psq[b] = 0.0f;
 #pragma unroll
-          for (int b = 0; b < C::kRf; ++b) {
+          for (int t = 0; t < CT; ++t) {
             const f32x16& c = acc[t][f * C::kRf + b];
             if constexpr (B == 16) {
               v[t][b] = c;
@@ -400,8 +490,33 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_block_kernel(const GemvA
             for (int i = 0; i < 16; ++i) v[t][b][i] = turn[(16 * h + i) * kTurnRow + h * 32 + r];
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (read before the next block is written)
           }
-        block_out<CT, C::kRf>(a, v, t0 + h, m0 + f * 32 * C::kRf + r, NT);
+          if (fold_in) {   // (times 1 / rms: a division is ~ 10 instructions, and a lane has up to 64 sums)
+            float t2 = 0.0f;
+            uint32_t any = 0;
+#pragma unroll
+            for (int p = 0; p < C::kP; ++p) {
+              t2 += fabsf(sums[p * C::kRows + row]);
+              any |= __builtin_bit_cast(uint32_t, sums[p * C::kRows + row]);
+            }
+            const float s = (int32_t)any < 0 && a.norm_w ? 1.0f : 1.0f / sqrtf(t2 / (float)a.K + a.eps);   // (negative: normalised)
+#pragma unroll
+            for (int t = 0; t < CT; ++t)
+#pragma unroll
+              for (int i = 0; i < 16; ++i) v[t][b][i] *= s;
+          }
+        }
+        block_out<FOLD, CT, C::kRf>(a, v, t0 + h, m0 + f * 32 * C::kRf + r, NT, hsq, psq);
+        if (fold_out)
+#pragma unroll
+          for (int b = 0; b < C::kRf; ++b) {
+            const float2 p = make_float2(hsq[b] + lane_xor<32>(hsq[b]), psq[b] + lane_xor<32>(psq[b]));
+            if (h == 0) red[wn * C::kRows + (f * C::kRf + b) * 32 + r] = p;
+          }
       }
+  if (fold_out) {
+    lds_barrier();
+    wide_fold_store<C::kRows, WN, C::kCols / 16>(a, red, cb, m0, tid);
+  }
   stamp_end(a.stamp, t_entry);
 }
 
@@ -413,14 +528,16 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_block_kernel(const GemvA
 // 150 30.8 -> 23.7; int8: 11008 -> 4096 at 150 38.8 -> 31.9, 5632 -> 2048 at 333 22.6 -> 19.4; fp16: 2048 -> 2560 at 128 11.3 -> 9.8; the
 // mean up to 640 rows 9 %, 6 % and 4 %).
 struct BlockShape {
-  const void* fn;
-  int rows, cols, groups, threads, lds;
+  const void* fn[2];   // [fold]
+  int rows, cols, groups, threads, lds[2];   // (lds: [fold])
   float fix, alone, full, round;
 };
 template <int F, int WN, int KG, int RT, int CT, int NS>
 static BlockShape block_shape(float fix, float alone, float full, float round) {
   typedef BlockGemm<F, WN, KG, RT, CT, NS> C;
-  return {(const void*)gemm_block_kernel<F, WN, KG, RT, CT, NS>, C::kRows, C::kCols, KG, 64 * C::kWaves, C::kLds, fix, alone, full, round};
+  const void* fold = nullptr;
+  if constexpr (RT <= 2) fold = (const void*)gemm_block_kernel<F, WN, KG, RT, CT, NS, true>;   // (a fold's calls have up to 64 rows)
+  return {{(const void*)gemm_block_kernel<F, WN, KG, RT, CT, NS, false>, fold}, C::kRows, C::kCols, KG, 64 * C::kWaves, {C::kLds, C::kFoldLds}, fix, alone, full, round};
 }
 struct BlockShapes {
   const BlockShape* s;
@@ -471,21 +588,24 @@ static BlockShapes block_shapes_of(int fmt) {   // rows x columns (by groups of 
   return {nullptr, 0};
 }
 
-// The shape whose busiest CU is done first.
-bool block_plan(int fmt, int M, int N, int K, int cus, BlockPlan* p) {
+// The shape whose busiest CU is done first.  A fold's sums and marks cost its calls ~ 1.5 us.  Up to 32 rows the few-rows and many-rows
+// kernels have shapes of fewer rows (us, theirs / 32 rows here: int4 4096 -> 12288 at 24 rows 10.5 / 12.1, 11008 -> 4096 13.6 / 17.1; only
+// 4096 -> 22016 and wider are faster here, 18.4 / 16.0, and not with a fold).
+bool block_plan(int fmt, int M, int N, int K, int cus, bool fold, BlockPlan* p) {
   const BlockShapes sh = block_shapes_of(fmt);
-  if (M <= TI_FOLD_SS_ROWS || M > TI_GEMM_MAX_ROWS || N < 16 || (N & 15) || K < 128 || (K & 127)) return false;
+  if (M <= 32 || M > (fold ? TI_FOLD_SS_ROWS : TI_GEMM_MAX_ROWS) || N < 16 || (N & 15) || K < 128 || (K & 127)) return false;
   const int NT = N >> 4, KT = K >> 7;
   // (the kernel's byte offsets into the weights and their scales are 32 bits)
   if ((uint64_t)NT * KT * (fmt * 256u) >= 0xfff00000ull) return false;
   p->shape = -1;
   for (int i = 0; i < sh.n; ++i) {
     const BlockShape& s = sh.s[i];
+    if (fold && !s.fn[1]) continue;
     const int n_cb = (N + s.cols - 1) / s.cols, n_rb = (M + s.rows - 1) / s.rows;
     const long n = ((long)((n_cb + 7) / 8) * n_rb + cus / 8 - 1) / (cus / 8);   // (launched: whole XCD rows)
     const float one = (float)n * s.full;
-    const float us = s.fix + (float)((KT + s.groups - 1) / s.groups) * (one > s.alone ? one : s.alone) + (float)n * s.round;
-    if (p->shape < 0 || us < p->us) *p = {i, n_cb, n_rb, us};
+    const float us = (fold ? 1.5f : 0.0f) + s.fix + (float)((KT + s.groups - 1) / s.groups) * (one > s.alone ? one : s.alone) + (float)n * s.round;
+    if (p->shape < 0 || us < p->us) *p = {i, n_cb, n_rb, fold, us};
   }
   return p->shape >= 0;
 }
@@ -494,9 +614,10 @@ int block_prepare() {
   for (int f : {4, 8, 16}) {
     const BlockShapes sh = block_shapes_of(f);
     for (int i = 0; i < sh.n; ++i)
-      if (sh.s[i].lds > 64 * 1024)
-        TI_HIP_CHECK(hipFuncSetAttribute(sh.s[i].fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024),
-                     "hipFuncSetAttribute(gemm_block_kernel)");
+      for (int f2 = 0; f2 < 2; ++f2)
+        if (sh.s[i].fn[f2] && sh.s[i].lds[f2] > 64 * 1024)
+          TI_HIP_CHECK(hipFuncSetAttribute(sh.s[i].fn[f2], hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024),
+                       "hipFuncSetAttribute(gemm_block_kernel)");
   }
   return TI_OK;
 }
@@ -508,7 +629,7 @@ int block_launch(int fmt, const BlockPlan& p, const GemvArgs& a, hipStream_t str
   GemvArgs arg = a;
   int n_cb = p.n_cb, n_rb = p.n_rb;
   void* args[] = {&arg, &n_cb, &n_rb};
-  TI_HIP_CHECK(hipLaunchKernel(s.fn, dim3((unsigned)block_workgroups(p)), dim3(s.threads), args, s.lds, stream),
+  TI_HIP_CHECK(hipLaunchKernel(s.fn[p.fold], dim3((unsigned)block_workgroups(p)), dim3(s.threads), args, s.lds[p.fold], stream),
                "hipLaunchKernel(gemm_block_kernel)");
   TI_LAUNCH_CHECK("gemm_block_kernel");
   return TI_OK;

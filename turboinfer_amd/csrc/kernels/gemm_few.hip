@@ -194,9 +194,9 @@ __global__ __launch_bounds__(64 * kFewWaves, 2) void gemm_few_kernel(const GemvA
       return __builtin_amdgcn_ballot_w64(__builtin_bit_cast(int32_t, rmsv[lane % C::kRows]) < 0) != 0;
     };
     if (__builtin_expect(a.norm_w && marked(), 0)) {
-      wide_fold_settle<C::kRows, NW>(a, tid, rmsv);
+      wide_fold_settle<C::kRows, NW>(a, 0, tid, rmsv);
       if (marked()) {   // rows that fp16 did not hold: again, behind their rewriting
-        wide_refold<C::kRows, NW>(a, wave, lane, rmsv);
+        wide_refold<C::kRows, NW>(a, 0, wave, lane, rmsv);
         lds_barrier();
         product();
         lds_barrier();

@@ -361,9 +361,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const GemvAr
       return __builtin_amdgcn_ballot_w64((int32_t)any < 0) != 0;
     };
     if (__builtin_expect(marked(), 0)) {
-      if (a.norm_w) wide_fold_settle<C::kRows, NW>(a, tid, rmsv);
+      if (a.norm_w) wide_fold_settle<C::kRows, NW>(a, m0, tid, rmsv);
       if (a.norm_w && marked()) {   // rows that fp16 did not hold: again, behind their rewriting, a stage at a time
-        wide_refold<C::kRows, NW>(a, wave, lane, rmsv);
+        wide_refold<C::kRows, NW>(a, m0, wave, lane, rmsv);
 #pragma unroll
         for (int t = 0; t < TN; ++t)
 #pragma unroll
@@ -550,10 +550,12 @@ int wide_launch(int fmt, const WidePlan& p, const GemvArgs& a, hipStream_t strea
 // Which kernel a call of ti_gemm_rows takes: the few-rows one where its estimate is the lower (the many-rows kernel's is 4 % (int4,
 // also in blocks of 32) or 8 % low for calls of up to 48 rows; the choice costs 0.1 .. 0.8 % more than the better one of each of 700
 // measured points, by format, in the mean).
-// block: the call has more rows than a fold's and an output gemm_block_kernel writes.  It takes the call where its estimate is
-// below the many-rows kernel's (0.95 of it for fp16: from there up the many-rows kernel was the faster as often as not); that one
-// keeps few rows by long K, split over workgroups, where the two are even (us, many-rows / block: int4 14336 -> 4096 at 96 rows
-// 27.4 / 27.3, fp16 11008 -> 4096 at 128 rows 36.7 / 37.9), and short K, where the blocks' ends weigh.
+// block: an output gemm_block_kernel writes (and 33 rows, of a fold to 64).  It takes the call where its estimate is below theirs
+// (0.95 of them for fp16: from there up the many-rows kernel was the faster as often as not; us, before / block at 64 rows: int4
+// 4096 -> 4096 11.9 / 9.4, 4096 -> 22016 26 / 21, 2048 -> 2560 9.8 / 6.4, int8 2048 -> 2048 9.4 / 6.0; at 48 rows int4 4096 ->
+// 12288 19.0 / 14.9, int8 4096 -> 22016 31.4 / 27.2).  The many-rows kernel keeps few rows by long K, split
+// over workgroups (int4 11008 -> 4096 at 64 rows 17.9 / 18.7; 14336 -> 4096 at 96 rows 27.4 / 27.3, fp16 11008 -> 4096 at 128 rows
+// 36.7 / 37.9), and short K, where the blocks' ends weigh.
 struct RowsPlan {
   int kernel;   // TI_ROWS_FEW, _MANY or _BLOCK
   ti::FewPlan f;
@@ -564,18 +566,26 @@ struct RowsPlan {
 static bool rows_plan_of(int kernel, int bits, int M, int N, int K, int64_t ws_bytes, bool fold, bool block, RowsPlan* p) {
   const int cus = ti::gemm_cus();
   auto asked = [&](int k) { return kernel == TI_ROWS_AUTO || kernel == k; };
-  const bool wide = asked(TI_ROWS_MANY) && ti::wide_plan(bits, M, N, K, cus, ws_bytes, fold, &p->w);
-  p->kernel = wide ? TI_ROWS_MANY : TI_ROWS_AUTO;
-  if (asked(TI_ROWS_FEW) && ti::few_plan(bits, M, N, K, cus, &p->f) && (!wide || p->f.us < ((bits & ~TI_BITS_G32) == 4 ? 1.04f : 1.08f) * p->w.us))
+  p->kernel = TI_ROWS_AUTO;
+  float us = 0.0f;   // of the kernel chosen, by the many-rows kernel's measure
+  if (asked(TI_ROWS_MANY) && ti::wide_plan(bits, M, N, K, cus, ws_bytes, fold, &p->w)) {
+    p->kernel = TI_ROWS_MANY;
+    us = p->w.us;
+  }
+  const float few = (bits & ~TI_BITS_G32) == 4 ? 1.04f : 1.08f;
+  if (asked(TI_ROWS_FEW) && ti::few_plan(bits, M, N, K, cus, &p->f) && (p->kernel == TI_ROWS_AUTO || p->f.us < few * us)) {
     p->kernel = TI_ROWS_FEW;
-  if (asked(TI_ROWS_BLOCK) && block && ti::block_plan(bits, M, N, K, cus, &p->b) && (!wide || p->b.us < (bits == 16 ? 0.95f : 1.0f) * p->w.us))
+    us = p->f.us / few;
+  }
+  if (asked(TI_ROWS_BLOCK) && block && ti::block_plan(bits, M, N, K, cus, fold, &p->b) &&
+      (p->kernel == TI_ROWS_AUTO || p->b.us < (bits == 16 ? 0.95f : 1.0f) * us))
     p->kernel = TI_ROWS_BLOCK;
   return p->kernel != TI_ROWS_AUTO;
 }
 
 extern "C" int ti_gemm_rows_fold_partials_on(int kernel, int bits, int M, int N, int K, int64_t ws_bytes) {
   RowsPlan p;
-  if (M > TI_FOLD_SS_ROWS || kernel < TI_ROWS_AUTO || kernel > TI_ROWS_BLOCK || !rows_plan_of(kernel, bits, M, N, K, ws_bytes, true, false, &p))
+  if (M > TI_FOLD_SS_ROWS || kernel < TI_ROWS_AUTO || kernel > TI_ROWS_BLOCK || !rows_plan_of(kernel, bits, M, N, K, ws_bytes, true, true, &p))
     return 0;
   return p.n_cb();
 }
@@ -620,7 +630,7 @@ static int rows_impl(int kernel, const void* tiles, const uint16_t* scales, int 
     a.norm_w = norm_w;
     a.epi.fold_w = h;
   }
-  const bool fold = epi->ss_in || fold_out, block = !fold && a.vec;   // (a.vec: fp32, residual, SiLU and query-key-value outputs)
+  const bool fold = epi->ss_in || fold_out, block = a.vec;   // (a.vec: fp32, residual, SiLU and query-key-value outputs)
   if (!rows_plan_of(kernel, bits, M, N, K, epi->splitk_ws ? epi->splitk_bytes : 0, fold, block, &p))
     return ti_set_error(TI_ERR_UNSUPPORTED, "ti_gemm_rows: bits %d, M=%d N=%d K=%d", bits, M, N, K);
   const int rp = ti_gemm_prepare();   // no-op once this device is prepared

@@ -60,10 +60,10 @@ __device__ __forceinline__ void wide_fold_rms(const GemvArgs& a, float share, in
 // Where a row's rms is negative: the marks counted, the rms of rows that are taken as they are made positive (behind a barrier; one
 // follows).  Apart, so that calls without a mark do not pay for it (0.1 us each).
 template <int ROWS, int NW>
-__device__ __forceinline__ void wide_fold_settle(const GemvArgs& a, int tid, float* rmsv) {
+__device__ __forceinline__ void wide_fold_settle(const GemvArgs& a, int m0, int tid, float* rmsv) {
   constexpr int P = 64 * NW / ROWS;
   uint32_t* marks = (uint32_t*)rmsv + ROWS;   // small blocks; the top bit: one is past 65504
-  const int m = tid % ROWS, part = tid / ROWS;
+  const int m = m0 + tid % ROWS, part = tid / ROWS;
   uint32_t n = 0, over = 0;
   for (int b0 = m < a.M && part < P ? part : a.epi.n_ss; b0 < a.epi.n_ss; b0 += 16 * P) {
     uint32_t v[16];
@@ -89,12 +89,12 @@ __device__ __forceinline__ void wide_fold_settle(const GemvArgs& a, int tid, flo
   }
   lds_barrier();
 }
-// The rows whose rms is negative as ti_rmsnorm_f16 gives them.  Every workgroup rewrites them whole, with the same values,
+// The rows (from m0) whose rms is negative as ti_rmsnorm_f16 gives them.  Every workgroup rewrites them whole, with the same values,
 // before it reads them: a chain of loads per piece, so a row's pieces fly 4 at a time (Llama-2-7B int4 with every row like this, us,
 // one at a time -> this: steps of 3 rows 2807 -> 2710, of 24 5713 -> 4950, prompts of 20 5049 -> 4420, of 64 10400 -> 7941;
 // none of them 1650, 2340, 2070 and 2760).
 template <int ROWS, int NW>
-__device__ __forceinline__ void wide_refold(const GemvArgs& a, int wave, int lane, const float* rmsv) {
+__device__ __forceinline__ void wide_refold(const GemvArgs& a, int m0, int wave, int lane, const float* rmsv) {
   typedef f16 f16x4 __attribute__((ext_vector_type(4)));
   constexpr int U = 4;
 #pragma unroll 1
@@ -107,7 +107,7 @@ __device__ __forceinline__ void wide_refold(const GemvArgs& a, int wave, int lan
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int k = min(k0 + 4 * (kWave * u + lane), a.K - 4);
-        v[u] = *(const f32x4*)(a.epi.fold_w + (size_t)m * a.K + k);
+        v[u] = *(const f32x4*)(a.epi.fold_w + (size_t)(m0 + m) * a.K + k);
         w[u] = *(const f32x4*)(a.norm_w + k);
       }
 #pragma unroll
@@ -115,7 +115,7 @@ __device__ __forceinline__ void wide_refold(const GemvArgs& a, int wave, int lan
         f16x4 y;
 #pragma unroll
         for (int i = 0; i < 4; ++i) y[i] = mul_f16(v[u][i] / rms, w[u][i]);
-        *(f16x4*)((f16*)a.x + (size_t)m * a.ldx + min(k0 + 4 * (kWave * u + lane), a.K - 4)) = y;
+        *(f16x4*)((f16*)a.x + (size_t)(m0 + m) * a.ldx + min(k0 + 4 * (kWave * u + lane), a.K - 4)) = y;
         __builtin_amdgcn_sched_barrier(0);   // (one piece's divisions at a time: registers)
       }
     }
@@ -216,12 +216,13 @@ long few_workgroups(const FewPlan& p);
 int few_launch(int fmt, const FewPlan& p, const GemvArgs& a, hipStream_t s);
 int few_prepare();
 
-// gemm_block.hip: prompt chunks (more than TI_FOLD_SS_ROWS rows; outputs of whole 16-byte pieces, a.vec)
+// gemm_block.hip: 33 rows and more (outputs of whole 16-byte pieces, a.vec).  fold: a call with a folded input or output.
 struct BlockPlan {
   int shape, n_cb, n_rb;   // workgroup shape, column blocks x row blocks
+  bool fold;
   float us;                // estimate
 };
-bool block_plan(int fmt, int M, int N, int K, int cus, BlockPlan* p);
+bool block_plan(int fmt, int M, int N, int K, int cus, bool fold, BlockPlan* p);
 long block_workgroups(const BlockPlan& p);
 int block_launch(int fmt, const BlockPlan& p, const GemvArgs& a, hipStream_t s);
 int block_prepare();
