@@ -512,3 +512,36 @@ def test_rows_block_fold(ti, oracle, ws, bits, M, K, H, N):
             assert np.all(np.abs(out[0] - ref) <= tol), (marked, second)
             np.testing.assert_array_equal(*out)
         np.testing.assert_array_equal((fx.download(np.uint16, (M, H)) != plain).any(axis=1), bad)
+
+
+@pytest.mark.parametrize("bits", [4, 8, 16, 8 | G32])
+@pytest.mark.parametrize("M,N", [(3, 48), (17, 4112), (48, 1040), (50, 400), (130, 2064)])
+def test_rows_logits_keys(ti, oracle, bits, M, N):
+    """Logits in 16-byte pieces and, at a pitch that is none, one by one: the plain product's values, and each row's key at the first
+    of its largest columns where several are equal (columns of the same weights)."""
+    K, rng = 512, np.random.RandomState(M + N + bits)
+    w = np.tile(rng.standard_normal((K, 16)).astype(f32) * 0.03, (1, N // 16))
+    if bits & G32:
+        q, d, _ = g32_weight(rng, K, 16, bits & 15)
+        td, sd = pack_g32(ti, np.tile(q, (1, N // 16)), np.tile(d, (1, N // 16)), bits & 15)
+    else:
+        td, sd = (dev(ti, a) for a in ti.wpack_host(w, bits))
+    x = rng.standard_normal((M, K)).astype(f16)
+    xd, yd = dev(ti, x), ti.DeviceBuffer(M * N * 4)
+    for kernel in kernels(ti, M):
+        ep = ti.Epilogue()
+        ep.kind, ep.ldo, ep.out = ti.EPI_STORE_F32, N, yd.ptr
+        rows(ti, bits, td, sd, xd, M, N, K, ep, kernel=ti.ROWS_MANY if M > 48 else kernel)
+        ref = yd.download(f32, (M, N))
+        for ldo in (N, N + 4, N + 1):
+            ld, am = ti.DeviceBuffer(M * ldo * 4), ti.DeviceBuffer(M * ti.ARGMAX_SLOTS * 8)
+            ld.zero()
+            am.zero()
+            ep = ti.Epilogue()
+            ep.kind, ep.ldo, ep.out, ep.argmax = ti.EPI_LOGITS_ARGMAX, ldo, ld.ptr, am.ptr
+            rows(ti, bits, td, sd, xd, M, N, K, ep, kernel=kernel)
+            lg = ld.download(f32, (M, ldo))
+            np.testing.assert_array_equal(lg[:, :N], ref)
+            assert not lg[:, N:].any()
+            keys = am.download(np.uint64, (M, ti.ARGMAX_SLOTS)).max(axis=1)
+            np.testing.assert_array_equal((0xFFFFFFFF - (keys & 0xFFFFFFFF)).astype(np.int64), np.argmax(lg[:, :N], axis=1))

@@ -36,7 +36,7 @@ __host__ inline bool rows_aligned(const void* x, int ldx) { return ((uintptr_t)x
 __host__ inline int epilogue_vec(const ti_epilogue& e) {
   auto al = [](const void* p, unsigned n) { return ((uintptr_t)p & (n - 1)) == 0; };
   switch (e.kind) {
-    case TI_EPI_STORE_F32: return al(e.out, 16) && (e.ldo & 3) == 0;
+    case TI_EPI_STORE_F32: case TI_EPI_LOGITS_ARGMAX: return al(e.out, 16) && (e.ldo & 3) == 0;
     case TI_EPI_RESID_F32: return al(e.out, 16) && (e.ldo & 3) == 0 && (!e.fold_x || (al(e.fold_x, 8) && al(e.fold_w, 16)));
     case TI_EPI_SILU_MUL_F16: return !e.out_packed && al(e.out, 8) && (e.ldo & 3) == 0;
     case TI_EPI_QKV_ROPE_KV:
@@ -255,7 +255,7 @@ __device__ __forceinline__ void tile_pre(const GemvArgs& a, int tn, int mb, int 
 
 // Epilogue of weight tile tn (16 outputs) for rows mb .. mb + 16 RB - 1 of one wave, from its LDS block
 // stg[row][col] (row stride kTileEpiStride).  Same arithmetic as epilogue_mb, element for element.
-//   STORE_F32 / RESID_F32 / QKV_ROPE_KV: lane l owns columns 4 (l & 3) .. + 3 of rows 16 it + l / 4
+//   STORE_F32 / RESID_F32 / QKV_ROPE_KV / LOGITS_ARGMAX: lane l owns columns 4 (l & 3) .. + 3 of rows 16 it + l / 4
 //   SILU_MUL_F16: lane l owns outputs 4 (l & 1) .. + 3 (gate columns, up = column + 8) of rows 32 it + l / 2
 template <int RB>
 __device__ __forceinline__ void tile_epilogue_lds(const GemvArgs& a, int tn, int mb, const float* stg, int lane, const TilePre<RB>& p) {
@@ -289,6 +289,29 @@ __device__ __forceinline__ void tile_epilogue_lds(const GemvArgs& a, int tn, int
       const float4 h = p.v[it];
       if (m0 + 16 * it < a.M)
         *(float4*)((float*)e.out + (size_t)(m0 + 16 * it) * e.ldo + ng) = make_float4(h.x + v[it].x, h.y + v[it].y, h.z + v[it].z, h.w + v[it].w);
+    }
+  } else if (e.kind == TI_EPI_LOGITS_ARGMAX) {
+    // A row's 16 columns are 4 lanes: keys by register moves, all rows' at once (epilogue_mb's 16 lanes exchange 64-bit keys through
+    // LDS four times a row, one row after another: us, 32000 columns, int4 K 4096 at 64 rows 43.1 -> 34.6, int8 K 2048 at 24 26.2 -> 23.4).
+#pragma unroll
+    for (int it = 0; it < RB; ++it) {
+      const int m = m0 + 16 * it;
+      const float x[4] = {v[it].x, v[it].y, v[it].z, v[it].w};
+      unsigned long long key = 0ull;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const unsigned long long k = ((unsigned long long)float_order_key(x[i]) << 32) | (unsigned long long)(0xFFFFFFFFu - (uint32_t)(ng + i));
+        key = k > key ? k : key;
+      }
+      auto meet = [&](uint32_t hi, uint32_t lo) {
+        const unsigned long long k = ((unsigned long long)hi << 32) | lo;
+        key = k > key ? k : key;
+      };
+      meet(lane_xor_u32<1>((uint32_t)(key >> 32)), lane_xor_u32<1>((uint32_t)key));
+      meet(lane_xor_u32<2>((uint32_t)(key >> 32)), lane_xor_u32<2>((uint32_t)key));
+      if (m >= a.M) continue;
+      *(float4*)((float*)e.out + (size_t)m * e.ldo + ng) = v[it];
+      if ((lane & 3) == 0) atomicMax(e.argmax + (size_t)m * TI_ARGMAX_SLOTS + (blockIdx.x & (TI_ARGMAX_SLOTS - 1)), key);
     }
   } else {   // TI_EPI_QKV_ROPE_KV
     const TileQkv t = tile_qkv(e, tn);

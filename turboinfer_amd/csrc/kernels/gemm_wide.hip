@@ -630,7 +630,7 @@ static int rows_impl(int kernel, const void* tiles, const uint16_t* scales, int 
     a.norm_w = norm_w;
     a.epi.fold_w = h;
   }
-  const bool fold = epi->ss_in || fold_out, block = a.vec;   // (a.vec: fp32, residual, SiLU and query-key-value outputs)
+  const bool fold = epi->ss_in || fold_out, block = a.vec && epi->kind != TI_EPI_LOGITS_ARGMAX;
   if (!rows_plan_of(kernel, bits, M, N, K, epi->splitk_ws ? epi->splitk_bytes : 0, fold, block, &p))
     return ti_set_error(TI_ERR_UNSUPPORTED, "ti_gemm_rows: bits %d, M=%d N=%d K=%d", bits, M, N, K);
   const int rp = ti_gemm_prepare();   // no-op once this device is prepared
