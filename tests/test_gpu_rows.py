@@ -465,14 +465,17 @@ def test_rows_few_wide_blocks(ti, oracle, bits, M, K, N):
     np.testing.assert_allclose(ss.download(f32, (n_ss, 64))[:, :M].sum(axis=0), (got[:M].astype(np.float64) ** 2).sum(axis=1), rtol=1e-5)
 
 
-# (block kernel: two row blocks of 32, the last one by a row, one of 64; 1, 2 and 4 groups of waves)
+# (block kernel: one and two row blocks of 32, the last one by a row, one of 64; 1, 2 and 4 groups of waves)
 @pytest.mark.parametrize("M,K,H,N", [(33, 384, 1152, 80), (40, 256, 1024, 4112), (33, 1152, 2048, 400), (50, 640, 22016, 2064),
-                                     (64, 2944, 4096, 12304), (64, 512, 12288, 208), (48, 384, 2944, 28688)])
+                                     (64, 2944, 4096, 12304), (64, 512, 12288, 208), (48, 384, 2944, 28688), (17, 1152, 2048, 4112), (32, 384, 1024, 28688)])
 @pytest.mark.parametrize("bits", [4, 8, 16])
 def test_rows_block_fold(ti, oracle, ws, bits, M, K, H, N):
     """Folds of up to 64 rows on the block kernel, into it and into the many-rows one, with rows that must be normalised first in its
     first and last block.  Bounds: test_rows_fold_range's."""
     L, rng = ti.lib(), np.random.RandomState(M + bits)
+    if bits == 16 and M <= 32:
+        assert L.ti_gemm_rows_fold_partials_on(ti.ROWS_BLOCK, bits, M, H, K, WS) == 0
+        return
     to, so, wo = weight(ti, oracle, bits, K, H, rng)
     t2, s2, w2 = weight(ti, oracle, bits, H, N, rng)
     act = rng.standard_normal((M, K)).astype(f16)

@@ -588,12 +588,12 @@ static BlockShapes block_shapes_of(int fmt) {   // rows x columns (by groups of 
   return {nullptr, 0};
 }
 
-// The shape whose busiest CU is done first.  A fold's sums and marks cost its calls ~ 1.5 us.  Up to 32 rows the few-rows and many-rows
-// kernels have shapes of fewer rows (us, theirs / 32 rows here: int4 4096 -> 12288 at 24 rows 10.5 / 12.1, 11008 -> 4096 13.6 / 17.1; only
-// 4096 -> 22016 and wider are faster here, 18.4 / 16.0, and not with a fold).
+// The shape whose busiest CU is done first.  A fold's sums and marks cost its calls ~ 1.5 us.  Up to 32 rows only
+// wide outputs are faster here (us, few-rows or many-rows kernel / 32 rows here: int4 4096 -> 28672 at 32 rows, folded, 22.3 / 20.1, 4096 -> 22016
+// 19.0 / 16.3; 4096 -> 12288 11.0 / 12.3, 11008 -> 4096 13.8 / 17.9), fp16 ones are not (prompts of 22 of the 7B model 3472 / 3749).
 bool block_plan(int fmt, int M, int N, int K, int cus, bool fold, BlockPlan* p) {
   const BlockShapes sh = block_shapes_of(fmt);
-  if (M <= 32 || M > (fold ? TI_FOLD_SS_ROWS : TI_GEMM_MAX_ROWS) || N < 16 || (N & 15) || K < 128 || (K & 127)) return false;
+  if (M <= (fmt == 16 ? 32 : 16) || M > (fold ? TI_FOLD_SS_ROWS : TI_GEMM_MAX_ROWS) || N < 16 || (N & 15) || K < 128 || (K & 127)) return false;
   const int NT = N >> 4, KT = K >> 7;
   // (the kernel's byte offsets into the weights and their scales are 32 bits)
   if ((uint64_t)NT * KT * (fmt * 256u) >= 0xfff00000ull) return false;

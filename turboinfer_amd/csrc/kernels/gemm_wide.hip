@@ -550,7 +550,7 @@ int wide_launch(int fmt, const WidePlan& p, const GemvArgs& a, hipStream_t strea
 // Which kernel a call of ti_gemm_rows takes: the few-rows one where its estimate is the lower (the many-rows kernel's is 4 % (int4,
 // also in blocks of 32) or 8 % low for calls of up to 48 rows; the choice costs 0.1 .. 0.8 % more than the better one of each of 700
 // measured points, by format, in the mean).
-// block: an output gemm_block_kernel writes (and 33 rows, of a fold to 64).  It takes the call where its estimate is below theirs
+// block: an output gemm_block_kernel writes (and 17 rows, fp16 33, of a fold to 64).  It takes the call where its estimate is below theirs
 // (0.95 of them for fp16: from there up the many-rows kernel was the faster as often as not; us, before / block at 64 rows: int4
 // 4096 -> 4096 11.9 / 9.4, 4096 -> 22016 26 / 21, 2048 -> 2560 9.8 / 6.4, int8 2048 -> 2048 9.4 / 6.0; at 48 rows int4 4096 ->
 // 12288 19.0 / 14.9, int8 4096 -> 22016 31.4 / 27.2).  The many-rows kernel keeps few rows by long K, split

@@ -216,7 +216,7 @@ long few_workgroups(const FewPlan& p);
 int few_launch(int fmt, const FewPlan& p, const GemvArgs& a, hipStream_t s);
 int few_prepare();
 
-// gemm_block.hip: 33 rows and more (outputs of whole 16-byte pieces, a.vec).  fold: a call with a folded input or output.
+// gemm_block.hip: 17 rows and more (fp16: 33) (outputs of whole 16-byte pieces, a.vec).  fold: a call with a folded input or output.
 struct BlockPlan {
   int shape, n_cb, n_rb;   // workgroup shape, column blocks x row blocks
   bool fold;
