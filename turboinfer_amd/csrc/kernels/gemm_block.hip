@@ -490,7 +490,7 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_block_kernel(const GemvA
             for (int i = 0; i < 16; ++i) v[t][b][i] = turn[(16 * h + i) * kTurnRow + h * 32 + r];
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (read before the next block is written)
           }
-          if (fold_in) {   // (times 1 / rms: a division is ~ 10 instructions, and a lane has up to 64 sums)
+          if (fold_in) {
             float t2 = 0.0f;
             uint32_t any = 0;
 #pragma unroll
@@ -498,11 +498,19 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_block_kernel(const GemvA
               t2 += fabsf(sums[p * C::kRows + row]);
               any |= __builtin_bit_cast(uint32_t, sums[p * C::kRows + row]);
             }
-            const float s = (int32_t)any < 0 && a.norm_w ? 1.0f : 1.0f / sqrtf(t2 / (float)a.K + a.eps);   // (negative: normalised)
+            const float rms = (int32_t)any < 0 && a.norm_w ? 1.0f : sqrtf(t2 / (float)a.K + a.eps);   // (negative: normalised)
+            // divided, as by the other kernels: v / rms ~ q = v (1 / rms), one correction by its remainder, which is exact, and infinities,
+            // zeros and NaN as a division gives them.  A plain division's ~ 10 instructions for each of up to 32 sums cost a call 2 .. 5 %
+            // (us, 64 rows, int4 4096 -> 22016 22.3 -> 22.9), these four 0.3 .. 1 %; the product with 1 / rms alone rounds twice (a call's
+            // error, 40 rows 4096 -> 4096: 8.4e-8 of the result, these 7.9e-8).
+            const float inv = 1.0f / rms;
 #pragma unroll
             for (int t = 0; t < CT; ++t)
 #pragma unroll
-              for (int i = 0; i < 16; ++i) v[t][b][i] *= s;
+              for (int i = 0; i < 16; ++i) {
+                const float y = v[t][b][i], q = y * inv;
+                v[t][b][i] = __builtin_amdgcn_div_fixupf(fmaf(fmaf(-q, rms, y), inv, q), rms, y);
+              }
           }
         }
         block_out<FOLD, CT, C::kRf>(a, v, t0 + h, m0 + f * 32 * C::kRf + r, NT, hsq, psq);
