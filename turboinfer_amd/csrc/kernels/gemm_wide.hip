@@ -289,8 +289,12 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const GemvAr
   // batched fold (decode rows, ti_hip.h TI_FOLD_SS_ROWS): this thread's share of its row's sum of squares
   const bool fold_in = C::kFold && a.epi.ss_in != nullptr;
   const float share = fold_in ? wide_fold_share(a, m0 + tid % C::kRows, tid / C::kRows, 64 * NW / C::kRows) : 0.0f;
+  // What the epilogue reads is asked for behind the main loop, a tile at a time: blocks of 64 x 64 (one tile a wave) start on it
+  // with their products.  Of 16 and 32 rows they lose by that (us, 16 x 64, int4: 512 -> 256 4.4 -> 4.0, 1024 -> 1024 split over K 5.9 ->
+  // 5.5; 7 .. 17 registers more, a wave a SIMD less).
+  constexpr bool kEarly = TN == 1 && TM == 4;
   TilePre<TM> pre;
-  if constexpr (TN == 1) tile_pos<TM>(a, m0 + wm * 16 * TM, lane, pre);
+  if constexpr (kEarly) tile_pos<TM>(a, m0 + wm * 16 * TM, lane, pre);
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * C::kDma) : "memory");
   lds_barrier();
   Step st[2];
@@ -337,7 +341,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const GemvAr
       }
   };
   last();
-  if constexpr (TN == 1) tile_pre<TM>(a, min(t0 + wn * TN, NT - 1), m0 + wm * 16 * TM, lane, pre);
+  if constexpr (kEarly) tile_pre<TM>(a, min(t0 + wn * TN, NT - 1), m0 + wm * 16 * TM, lane, pre);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the clamped stages past the end
   lds_barrier();
 
@@ -403,7 +407,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const GemvAr
   float hsq[TM], psq[TM];
 #pragma unroll
   for (int b = 0; b < TM; ++b) hsq[b] = psq[b] = 0.0f;
-  if constexpr (TN > 1) tile_pos<TM>(a, mb, lane, pre);
+  if constexpr (!kEarly) tile_pos<TM>(a, mb, lane, pre);
 #pragma unroll 1
   for (int t = 0; t < TN; ++t) {   // (rolled: the tile's accumulators by static selects, so acc stays in registers)
     const int tn = t0 + wn * TN + t;
@@ -414,14 +418,22 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const GemvAr
 #pragma unroll
         for (int b = 0; b < TM; ++b) av[b] = acc[tt][b];
     if (tn >= NT) continue;
-    if constexpr (TN > 1) tile_pre<TM>(a, tn, mb, lane, pre);
+    // (values of this tile: the rows' addresses of every epilogue, taken out of the loop, are 40 .. 55 registers, and int4's 64 x 128
+    // blocks run 3 a CU: 4096 -> 22016 at 1024 rows 215 -> 194 us)
+    int ln = lane;
+    if constexpr (TN > 1) {
+      asm volatile("" : "+v"(ln));
+#pragma unroll
+      for (int b = 0; b < TM; ++b) asm volatile("" : "+v"(pre.pos[b]));
+    }
+    if constexpr (!kEarly) tile_pre<TM>(a, tn, mb, ln, pre);
 #pragma unroll
     for (int b = 0; b < TM; ++b)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         stg[(b * 16 + 4 * kq + i) * kTileEpiStride + r] = fold_in ? av[b][i] / rms[b][i] : av[b][i];
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    wide_tile_out<TM>(a, tn, mb, stg, lane, r, kq, fold_out, pre, hsq, psq);
+    wide_tile_out<TM>(a, tn, mb, stg, ln, r, kq, fold_out, pre, hsq, psq);
   }
   if (fold_out) {   // this column block's sum of h^2 per row, column-waves in order
     float2* red = (float2*)(smem + C::kEpiRed);
