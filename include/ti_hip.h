@@ -293,8 +293,9 @@ int ti_gemm_rows_folded(const void* tiles, const uint16_t* scales, int bits, uin
 int ti_gemm_rows_fold_partials(int bits, int M, int N, int K, int64_t ws_bytes);
 /* The same calls on a kernel of the caller's choice (parity tests and comparisons; h NULL: ti_gemm_rows, else
  * ti_gemm_rows_folded).  TI_ERR_UNSUPPORTED (0 partials) where it does not take the call: the few-rows kernel has up to 48 rows, the block
- * one 17 and more (fp16: 33), bits 4, 8 and 16 and aligned outputs other than fp16 rows and logits. */
-enum ti_rows_kernel { TI_ROWS_AUTO = 0, TI_ROWS_FEW, TI_ROWS_MANY, TI_ROWS_BLOCK };
+ * one 17 and more (fp16: 33), bits 4, 8 and 16 and aligned outputs other than fp16 rows and logits.  A kernel + (i + 1) * TI_ROWS_SHAPE: its
+ * i-th block shape only. */
+enum ti_rows_kernel { TI_ROWS_AUTO = 0, TI_ROWS_FEW, TI_ROWS_MANY, TI_ROWS_BLOCK, TI_ROWS_SHAPE = 16 };
 int ti_gemm_rows_on(int kernel, const void* tiles, const uint16_t* scales, int bits, uint16_t* x, int ldx, const float* h,
                     const float* norm_w, float eps, int M, int N, int K, const ti_epilogue* epi, ti_stream_t s);
 int ti_gemm_rows_fold_partials_on(int kernel, int bits, int M, int N, int K, int64_t ws_bytes);

@@ -1,6 +1,7 @@
 """ti_gemm_rows: row-major fp16 rows against packed weights of every format, against the weights' exact values in float64
-(test_gpu_kernels.py's bound: fp32 summation order).  Calls of up to 48 rows run on both of its kernels, the few-rows one
-(gemm_few.hip) and the many-rows one (gemm_wide.hip), whichever the call itself would take."""
+(test_gpu_kernels.py's bound: fp32 summation order).  Calls run on each of its kernels that has their rows, the few-rows one
+(gemm_few.hip, up to 48), the many-rows one (gemm_wide.hip) and the block one (gemm_block.hip), whichever the call itself would take;
+test_rows_each_shape takes them through every block shape by name."""
 from __future__ import annotations
 
 import ctypes as C
@@ -34,8 +35,11 @@ def weight(ti, oracle, bits, K, N, rng):
     return dev(ti, t), dev(ti, s), w.astype(f16).astype(f32) if bits == 16 else deq(oracle, w, bits)
 
 
-def kernels(ti, M):
-    return (ti.ROWS_FEW, ti.ROWS_MANY) if M <= 48 else (ti.ROWS_AUTO,)
+def kernels(ti, M, bits, block=True):
+    """The kernels of a call of M rows; block: an output that the block kernel writes."""
+    if M <= 48:
+        return ti.ROWS_FEW, ti.ROWS_MANY
+    return (ti.ROWS_AUTO, ti.ROWS_MANY) + ((ti.ROWS_BLOCK,) if block and not bits & G32 else ())
 
 
 def rows(ti, bits, td, sd, xd, M, N, K, ep, ldx=None, ws=None, kernel=0, h=None, norm_w=None):
@@ -61,7 +65,7 @@ def test_rows_store(ti, oracle, ws, bits, M, K, N):
     xd, yd = dev(ti, x), ti.DeviceBuffer(M * N * 4)
     xa = x[:, :K].astype(f32)
     ref = xa.astype(np.float64) @ w.astype(np.float64)
-    for kernel in kernels(ti, M):
+    for kernel in kernels(ti, M, bits):
         for k in (None, ws):
             yd.zero()
             ep = ti.Epilogue()
@@ -105,7 +109,7 @@ def test_rows_affine_blocks(ti, oracle, ws, M, K, N):
     parts = np.repeat(np.abs(d.astype(np.float64)), 32, 0) * 16 + np.repeat(np.abs(m.astype(np.float64)), 32, 0)
     x = rng.standard_normal((M, K)).astype(f16)
     xd, yd = dev(ti, x), ti.DeviceBuffer(M * N * 4)
-    for kernel in kernels(ti, M):
+    for kernel in kernels(ti, M, 4 | G32 | 64):
         yd.zero()
         ep = ti.Epilogue()
         ep.kind, ep.ldo, ep.out = ti.EPI_STORE_F32, N, yd.ptr
@@ -124,7 +128,7 @@ def test_rows_epilogues(ti, oracle, ws, bits, M):
     x = rng.standard_normal((M, K)).astype(f16)
     xd, xa = dev(ti, x), x.astype(np.float64)
     ref = xa @ w.astype(np.float64)
-    for kernel, ldo in [(k, l) for k in kernels(ti, M) for l in (N, N + 3)]:
+    for kernel, ldo in [(k, l) for k in kernels(ti, M, bits, False) for l in (N, N + 3)]:   # (the block kernel: test_rows_block)
         r = rng.standard_normal((M, ldo)).astype(f32)
         rd = dev(ti, r)
         ep = ti.Epilogue()
@@ -143,7 +147,7 @@ def test_rows_epilogues(ti, oracle, ws, bits, M):
         ep.kind = ti.EPI_STORE_F16
         rows(ti, bits, td, sd, xd, M, N, K, ep, ws=ws, kernel=kernel)
         np.testing.assert_allclose(hd.download(f16, (M, ldo))[:, :N].astype(np.float64), ref, rtol=2e-3, atol=1e-4)
-    for kernel in kernels(ti, M):
+    for kernel in kernels(ti, M, bits, False):
         ld, am = ti.DeviceBuffer(M * N * 4), ti.DeviceBuffer(M * ti.ARGMAX_SLOTS * 8)
         am.zero()
         ep = ti.Epilogue()
@@ -168,7 +172,7 @@ def test_rows_qkv(ti, oracle, ws, hd, M):
     pd = dev(ti, pos)
     cs = dev(ti, ti.rope_table(np.arange(S), hd, 10000.0))
     outs = []
-    for kernel in kernels(ti, M) + (None,):
+    for kernel in kernels(ti, M, 8) + (None,):
         q, k, v = ti.DeviceBuffer(M * qd * 4), ti.DeviceBuffer(kvh * S * hd * 2), ti.DeviceBuffer(kvh * S * hd * 2)
         for b in (k, v):
             b.zero()
@@ -201,7 +205,7 @@ def test_rows_fold(ti, oracle, ws, bits, M):
     h0 = rng.standard_normal((M, H)).astype(f32)
     nw = (1 + 0.1 * rng.standard_normal(H)).astype(f32)
     ad, nwd = dev(ti, act), dev(ti, nw)
-    for kernel, k in [(a, b) for a in kernels(ti, M) for b in (ws, None)]:   # (the many-rows kernel splits K with a workspace)
+    for kernel, k in [(a, b) for a in kernels(ti, M, bits) for b in (ws, None)]:   # (the many-rows kernel splits K with a workspace)
         n_ss = L.ti_gemm_rows_fold_partials_on(kernel, bits, M, H, K, WS if k else 0)
         assert 1 <= n_ss <= 4096
         bits_out = []
@@ -237,9 +241,17 @@ def test_rows_refusals(ti):
         a[i] = v
         assert L.ti_gemm_rows(*a, C.byref(ep), None) != 0, (i, v)
     on = (b.ptr, b.ptr, 8, b.ptr, 256, None, None, 1e-5)
-    for kernel, M in [(3, 4), (-1, 4), (ti.ROWS_FEW, 49)]:
-        assert L.ti_gemm_rows_on(kernel, *on, M, 64, 256, C.byref(ep), None) != 0
-        assert L.ti_gemm_rows_fold_partials_on(kernel, 8, M, 64, 256, 0) == 0
+    S = ti.ROWS_SHAPE
+    for kernel, M in [(ti.ROWS_BLOCK + 1, 40), (-1, 4), (ti.ROWS_FEW, 49), (ti.ROWS_BLOCK, 16), (S, 40), (ti.ROWS_FEW + 12 * S, 4), (ti.ROWS_MANY + 6 * S, 4),
+                      (ti.ROWS_BLOCK + 13 * S, 40), (ti.ROWS_FEW + S, 17), (ti.ROWS_MANY + 5 * S, 17)]:
+        assert L.ti_gemm_rows_on(kernel, *on, M, 64, 256, C.byref(ep), None) != 0, (kernel, M)
+        assert L.ti_gemm_rows_fold_partials_on(kernel, 8, M, 64, 256, 0) == 0, (kernel, M)
+    # what the block kernel does not take: few rows, blocks of 32, fp16 rows, logits, a pitch of no whole 16-byte pieces
+    for bits, M, kind, ldo in [(4, 16, ti.EPI_STORE_F32, 64), (16, 32, ti.EPI_STORE_F32, 64), (8 | G32, 40, ti.EPI_STORE_F32, 64), (8, 40, ti.EPI_STORE_F16, 64),
+                               (8, 40, ti.EPI_LOGITS_ARGMAX, 64), (8, 40, ti.EPI_STORE_F32, 65)]:
+        e2 = ti.Epilogue()
+        e2.kind, e2.ldo, e2.out, e2.argmax = kind, ldo, b.ptr, b.ptr
+        assert L.ti_gemm_rows_on(ti.ROWS_BLOCK, b.ptr, b.ptr, bits, *on[3:], M, 64, 256, C.byref(e2), None) != 0, (bits, M, kind, ldo)
     ep.kind, ep.fold_x = ti.EPI_RESID_F32, b.ptr
     assert L.ti_gemm_rows(*ok, C.byref(ep), None) != 0
 
@@ -270,7 +282,7 @@ def test_rows_fold_range(ti, oracle, ws, bits, M):
     h0[4], act[4] = 0, 0
     bad = np.isin(np.arange(M), [1, 2, 4, M - 1])
     ad, nwd = dev(ti, act), dev(ti, nw)
-    for kernel, k in [(a, b) for a in kernels(ti, M) for b in (ws, None)]:
+    for kernel, k in [(a, b) for a in kernels(ti, M, bits) for b in (ws, None)]:
         n_ss = L.ti_gemm_rows_fold_partials_on(kernel, bits, M, H, K, WS if k else 0)
         hd, fx, ss, yd = dev(ti, h0), ti.DeviceBuffer(M * H * 2), ti.DeviceBuffer(n_ss * 64 * 4), ti.DeviceBuffer(M * N * 4)
         out = []
@@ -318,7 +330,7 @@ def test_rows_fold_small_columns(ti, oracle, ws, bits, M):
     step = 2.0**-25 / np.where(first[:, None], 1.0, rms)
     tol = (2.0**-11 + H * 2.0**-24) * (np.abs(x) @ np.abs(w2)) + step * np.abs(w2).sum(axis=0) + 1e-9
     ad, nwd = dev(ti, act), dev(ti, nw)
-    for kernel in kernels(ti, M):
+    for kernel in kernels(ti, M, bits):
         n_ss = L.ti_gemm_rows_fold_partials_on(kernel, bits, M, H, K, WS)
         hd, fx, ss, yd = dev(ti, h), ti.DeviceBuffer(M * H * 2), ti.DeviceBuffer(n_ss * 64 * 4), ti.DeviceBuffer(M * N * 4)
         ep = ti.Epilogue()
@@ -373,7 +385,7 @@ def test_step_with_large_residuals(ti, bits):
 
 # the block kernel (gemm_block.hip): the fewest rows, the last block of rows by one row, one group of k (waves without one of their
 # own), 2, 3, 5, 7, 9, 11, 17, 23 and 24 of them (its ring of 2 or 3 slots and the last stages, of up to 4 groups), a last block of
-# columns of 1 .. 15 tiles, each block shape; the outputs it writes, rows of a pitch of their own, with fp16 rows of one where 16-byte pieces are not aligned
+# columns of 1 .. 15 tiles, most block shapes as the call itself would take them; the outputs it writes, rows of a pitch of their own, with fp16 rows of one where 16-byte pieces are not aligned
 @pytest.mark.parametrize("M,K,N", [(65, 128, 16), (97, 384, 1040), (129, 256, 4112), (500, 2176, 2064), (97, 896, 16400), (257, 640, 12304),
                                    (512, 640, 12304), (577, 640, 16400), (1024, 1408, 2576), (97, 3072, 8208), (161, 3072, 11280),
                                    (65, 1152, 400), (66, 384, 3088), (70, 2944, 3088), (97, 2944, 4112)])
@@ -438,7 +450,7 @@ def test_rows_block_qkv(ti, oracle, bits, hd, M):
         np.testing.assert_allclose(a, b, rtol=2.0 ** -10, atol=1e-5)
 
 
-# the few-rows kernel's blocks of 3, 4 and 6 tiles, and of 2 at 48 rows (other formats of a size: of 3), a last block short by 1 .. 5
+# the few-rows kernel's blocks of 3 and 6 tiles, and of 2 at 48 rows (other formats of a size: of 3), a last block short by 1 .. 5
 @pytest.mark.parametrize("M,K,N", [(16, 384, 11296), (13, 2176, 12336), (5, 896, 22064), (31, 1152, 11296), (32, 384, 16432), (47, 2176, 5648)])
 @pytest.mark.parametrize("bits", [4, 8, 4 | G32, 8 | G32])
 def test_rows_few_wide_blocks(ti, oracle, bits, M, K, N):
@@ -557,7 +569,7 @@ def test_rows_logits_keys(ti, oracle, bits, M, N):
         td, sd = (dev(ti, a) for a in ti.wpack_host(w, bits))
     x = rng.standard_normal((M, K)).astype(f16)
     xd, yd = dev(ti, x), ti.DeviceBuffer(M * N * 4)
-    for kernel in kernels(ti, M):
+    for kernel in kernels(ti, M, bits, False):
         ep = ti.Epilogue()
         ep.kind, ep.ldo, ep.out = ti.EPI_STORE_F32, N, yd.ptr
         rows(ti, bits, td, sd, xd, M, N, K, ep, kernel=ti.ROWS_MANY if M > 48 else kernel)
@@ -574,3 +586,151 @@ def test_rows_logits_keys(ti, oracle, bits, M, N):
             assert not lg[:, N:].any()
             keys = am.download(np.uint64, (M, ti.ARGMAX_SLOTS)).max(axis=1)
             np.testing.assert_array_equal((0xFFFFFFFF - (keys & 0xFFFFFFFF)).astype(np.int64), np.argmax(lg[:, :N], axis=1))
+
+
+# (kernel, format): how many block shapes it has
+SHAPES = {("FEW", 4): 11, ("FEW", 8): 8, ("FEW", 16): 4, ("FEW", 36): 8, ("FEW", 40): 8, ("MANY", 4): 5, ("MANY", 8): 5, ("MANY", 16): 5, ("MANY", 36): 5,
+          ("MANY", 40): 5, ("BLOCK", 4): 9, ("BLOCK", 8): 12, ("BLOCK", 16): 8}
+FEW_ROWS = {4: [16] * 5 + [32] * 4 + [48] * 2, 16: [16, 16, 32, 48]}
+EACH = [(k, b, i) for (k, b), n in SHAPES.items() for i in range(n) if not (k == "MANY" and b & G32 and i == 0)]   # (no such block of 32)
+
+
+def each_rows(kernel, bits, i):
+    """Rows of a shape's calls: a ragged block, and several where it has them."""
+    if kernel == "FEW":
+        r = FEW_ROWS.get(bits, [16] * 3 + [32] * 3 + [48] * 2)[i]
+        return (r - 3, r)
+    return ((50, 161) if i < 3 else (29,) if i == 3 else (13,)) if kernel == "MANY" else (50, 161)
+
+
+def qkv_ref(ti, y, pos, cs, heads, kvh, hd):
+    """RoPE of the products y, as (q, k, v) rows in float64."""
+    qd, kd, (M, _) = heads * hd, kvh * hd, y.shape
+    c = cs.reshape(-1, hd // 2, 2)[pos].astype(np.float64)
+    p = y[:, : qd + kd].astype(np.float64).reshape(M, heads + kvh, hd // 2, 2)
+    co, si = c[:, None, :, 0], c[:, None, :, 1]
+    r = np.stack([p[..., 0] * co - p[..., 1] * si, p[..., 1] * co + p[..., 0] * si], -1).reshape(M, qd + kd)
+    return r[:, :qd], r[:, qd:], y[:, qd + kd :].astype(np.float64)
+
+
+@pytest.mark.parametrize("kernel,bits,i", EACH)
+def test_rows_each_shape(ti, oracle, ws, kernel, bits, i):
+    """Every block shape of each kernel by name, each output it writes: ragged rows and columns, k-groups that its waves or slices
+    do not share evenly; the many-rows kernel with and without its split.  The other outputs follow from the plain one's values (same
+    sums), which are within fp32 summation order of the weights' exact ones."""
+    K, heads, kvh, hd, S = 1152, 39, 17, 16, 256
+    qd, kd = heads * hd, kvh * hd
+    N = qd + 2 * kd   # (73 tiles: no shape's blocks end with them)
+    rng = np.random.RandomState(7 * bits + i)
+    td, sd, w = weight(ti, oracle, bits, K, N, rng)
+    cs = ti.rope_table(np.arange(S), hd, 10000.0)
+    csd, on = dev(ti, cs), getattr(ti, "ROWS_" + kernel) + (i + 1) * ti.ROWS_SHAPE
+    for M in each_rows(kernel, bits, i):
+        x, pos, r = rng.standard_normal((M, K)).astype(f16), rng.permutation(S)[:M].astype(np.int32), rng.standard_normal((M + 1, N)).astype(f32)
+        xd, pd = dev(ti, x), dev(ti, pos)
+        ref = x.astype(np.float64) @ w.astype(np.float64)
+        for k in (None, ws) if kernel == "MANY" else (None,):
+            yd, rd, hd_ = ti.DeviceBuffer(r.nbytes), dev(ti, r), ti.DeviceBuffer(r.nbytes // 2)
+            q, kc, vc = ti.DeviceBuffer(M * qd * 4), ti.DeviceBuffer(S * kd * 2), ti.DeviceBuffer(S * kd * 2)
+            for b in (yd, hd_, kc, vc):
+                b.zero()
+            for kind, out, ldo in ((ti.EPI_STORE_F32, yd, N), (ti.EPI_RESID_F32, rd, N), (ti.EPI_SILU_MUL_F16, hd_, N), (ti.EPI_QKV_ROPE_KV, q, qd)):
+                ep = ti.Epilogue()
+                ep.kind, ep.ldo, ep.out = kind, ldo, out.ptr
+                if kind == ti.EPI_QKV_ROPE_KV:
+                    ep.q_dim, ep.kv_dim, ep.head_dim, ep.max_seq = qd, kd, hd, S
+                    ep.pos, ep.rope_cs, ep.k_cache, ep.v_cache, ep.kv_stream_stride = pd.ptr, csd.ptr, kc.ptr, vc.ptr, 0
+                rows(ti, bits, td, sd, xd, M, N, K, ep, ws=k, kernel=on)
+            y = yd.download(f32, r.shape)
+            assert_close_dot(y[:M], ref, x.astype(f32), w, rel=5e-5)
+            assert not y[M].any()
+            np.testing.assert_array_equal(rd.download(f32, r.shape), r + y)
+            h = hd_.download(f16, r.shape)
+            g = y[:M].astype(np.float64).reshape(M, N // 16, 2, 8)
+            sil = (g[:, :, 1] * (g[:, :, 0] / (1 + np.exp(-g[:, :, 0])))).reshape(M, N // 2)
+            np.testing.assert_allclose(h[:M, : N // 2].astype(np.float64), sil, rtol=2.0 ** -11 + 1e-5, atol=2.0 ** -25)
+            assert not h[M].any() and not h[:, N // 2 :].any()
+            # (two products and a sum of fp32, of values of ~ 1; fp16 caches)
+            rq, rk, rv = qkv_ref(ti, y[:M], pos, cs, heads, kvh, hd)
+            np.testing.assert_allclose(q.download(f32, (M, qd)), rq, rtol=1e-6, atol=1e-6)
+            for buf, rr in ((kc, rk), (vc, rv)):
+                got = buf.download(f16, (kvh, S, hd)).astype(np.float64)
+                np.testing.assert_allclose(got[:, pos].transpose(1, 0, 2).reshape(M, kd), rr, rtol=2.0 ** -11 + 1e-5, atol=2e-6)
+                assert not np.delete(got, pos, axis=1).any()
+
+
+@pytest.mark.parametrize("kernel,bits,i", EACH)
+def test_rows_each_shape_fold(ti, oracle, ws, kernel, bits, i):
+    """The folds of every block shape that has them: queries, keys and values, SiLU and plain outputs of a folded input with and without
+    rows that are normalised first, in the first and the last block, and the folded output.  Bounds: test_rows_fold_range's, and
+    test_rows_block_fold's."""
+    K, heads, kvh, hd, S = 640, 39, 17, 16, 64
+    qd, kd = heads * hd, kvh * hd
+    N, M = qd + 2 * kd, each_rows(kernel, bits, i)[0]
+    on, L = getattr(ti, "ROWS_" + kernel) + (i + 1) * ti.ROWS_SHAPE, ti.lib()
+    n_out = L.ti_gemm_rows_fold_partials_on(on, bits, M, N, K, 0)
+    wide = {"MANY": lambda: bits == 16 and i < 2, "BLOCK": lambda: no_fold_shape(bits, i), "FEW": lambda: False}[kernel]()
+    assert (n_out == 0) == wide
+    if wide:
+        return
+    rng = np.random.RandomState(11 * bits + i)
+    td, sd, w = weight(ti, oracle, bits, K, N, rng)
+    w = w.astype(np.float64)
+    cs = ti.rope_table(np.arange(S), hd, 10000.0)
+    csd, pos = dev(ti, cs), rng.permutation(S)[:M].astype(np.int32)
+    pd, nw = dev(ti, pos), (1 + 0.1 * rng.standard_normal(K)).astype(f32)
+    nwd = dev(ti, nw)
+    h = rng.standard_normal((M, K)).astype(f32)
+    for marked in (False, True):
+        sq = np.zeros((1, 64), f32)
+        if marked:   # (past 65504: the sum negative, its lowest bit 0)
+            h[1, [5, 600]] = 1e5, -3e5
+            h[M - 1] *= 1e6
+        sq[0, :M] = (h.astype(np.float64) ** 2).sum(axis=1)
+        if marked:
+            b = sq.view(np.uint32)
+            b[0, [1, M - 1]] = (b[0, [1, M - 1]] & ~np.uint32(1)) | np.uint32(0x80000000)
+        with np.errstate(over="ignore"):
+            xd = dev(ti, (h * nw).astype(f16))
+        hd_, sqd = dev(ti, h), dev(ti, sq)
+        yd, od, q = ti.DeviceBuffer(M * N * 4), ti.DeviceBuffer(M * N * 2), ti.DeviceBuffer(M * qd * 4)
+        kc, vc = ti.DeviceBuffer(M * S * kd * 2), ti.DeviceBuffer(M * S * kd * 2)
+        kc.zero()
+        vc.zero()
+        for kind, out, ldo in ((ti.EPI_QKV_ROPE_KV, q, qd), (ti.EPI_SILU_MUL_F16, od, N), (ti.EPI_STORE_F32, yd, N)):
+            ep = ti.Epilogue()
+            ep.kind, ep.ldo, ep.out, ep.ss_in, ep.n_ss = kind, ldo, out.ptr, sqd.ptr, 1
+            if kind == ti.EPI_QKV_ROPE_KV:   # (decode rows: a cache of its own for each)
+                ep.q_dim, ep.kv_dim, ep.head_dim, ep.max_seq = qd, kd, hd, S
+                ep.pos, ep.rope_cs, ep.k_cache, ep.v_cache, ep.kv_stream_stride = pd.ptr, csd.ptr, kc.ptr, vc.ptr, S * kd
+            rows(ti, bits, td, sd, xd, M, N, K, ep, kernel=on, h=hd_.ptr, norm_w=nwd.ptr)
+        x = h / np.sqrt((h.astype(np.float64) ** 2).mean(axis=1) + 1e-5)[:, None] * nw
+        y = yd.download(f32, (M, N))
+        tol = (2.0**-11 + K * 2.0**-24) * (np.abs(x) @ np.abs(w)) + 2.0**-25 * np.abs(w).sum(axis=0) + 1e-9
+        assert np.all(np.abs(y - x @ w) <= tol), marked
+        g = y.astype(np.float64).reshape(M, N // 16, 2, 8)   # (the other outputs from the same sums)
+        sil = (g[:, :, 1] * (g[:, :, 0] / (1 + np.exp(-g[:, :, 0])))).reshape(M, N // 2)
+        np.testing.assert_allclose(od.download(f16, (M, N))[:, : N // 2].astype(np.float64), sil, rtol=2.0 ** -11 + 1e-5, atol=2.0 ** -25)
+        rq, rk, rv = qkv_ref(ti, y, pos, cs, heads, kvh, hd)
+        np.testing.assert_allclose(q.download(f32, (M, qd)), rq, rtol=1e-6, atol=1e-6)
+        for buf, rr in ((kc, rk), (vc, rv)):
+            got = buf.download(f16, (M, kvh, S, hd)).astype(np.float64)
+            np.testing.assert_allclose(got[np.arange(M), :, pos].reshape(M, kd), rr, rtol=2.0 ** -11 + 1e-5, atol=2e-6)
+            got[np.arange(M), :, pos] = 0
+            assert not got.any()
+    act, r, ow = rng.standard_normal((M, K)).astype(f16), rng.standard_normal((M + 1, N)).astype(f32), (1 + 0.1 * rng.standard_normal(N)).astype(f32)
+    ad, rd, owd, fx, ss = dev(ti, act), dev(ti, r), dev(ti, ow), ti.DeviceBuffer(M * N * 2), ti.DeviceBuffer(n_out * 64 * 4)
+    ep = ti.Epilogue()
+    ep.kind, ep.ldo, ep.out = ti.EPI_RESID_F32, N, rd.ptr
+    ep.fold_w, ep.fold_x, ep.fold_ss = owd.ptr, fx.ptr, ss.ptr
+    rows(ti, bits, td, sd, ad, M, N, K, ep, kernel=on)
+    got = rd.download(f32, (M + 1, N))
+    assert_close_dot(got[:M] - r[:M], act.astype(np.float64) @ w, act.astype(f32), w, rel=5e-5)
+    np.testing.assert_array_equal(got[M], r[M])
+    np.testing.assert_array_equal(fx.download(np.uint16, (M, N)), (got[:M] * ow).astype(f16).view(np.uint16))
+    np.testing.assert_allclose(ss.download(f32, (n_out, 64))[:, :M].sum(axis=0), (got[:M].astype(np.float64) ** 2).sum(axis=1), rtol=1e-5)
+
+
+def no_fold_shape(bits, i):
+    """The block kernel's shapes of more than 64 rows have no folds."""
+    return i in {4: (0, 2), 8: (0, 1, 2, 3), 16: (0, 1, 2, 3)}[bits]

@@ -33,7 +33,7 @@ BITS_G32 = 32                       # TI_BITS_G32 (include/ti_hip.h): group-32 w
 BITS_AFF = 64                       # TI_BITS_AFF: affine group-32 int4 (GGUF Q4_1), with BITS_G32 | 4
 SCALE_GROUP, SCALE_TENSOR, SCALE_UNIT = 0, 1, 2
 ROWS_CONCAT, ROWS_INTERLEAVE8 = 0, 1
-ROWS_AUTO, ROWS_FEW, ROWS_MANY, ROWS_BLOCK = 0, 1, 2, 3   # ti_rows_kernel
+ROWS_AUTO, ROWS_FEW, ROWS_MANY, ROWS_BLOCK, ROWS_SHAPE = 0, 1, 2, 3, 16   # ti_rows_kernel
 (W_Q, W_K, W_V, W_O, W_GATE, W_UP, W_DOWN, W_LM_HEAD, V_ATTN_NORM, V_FFN_NORM, V_OUT_NORM, E_EMBED) = range(12)
 
 

@@ -599,7 +599,7 @@ static BlockShapes block_shapes_of(int fmt) {   // rows x columns (by groups of 
 // The shape whose busiest CU is done first.  A fold's sums and marks cost its calls ~ 1.5 us.  Up to 32 rows only
 // wide outputs are faster here (us, few-rows or many-rows kernel / 32 rows here: int4 4096 -> 28672 at 32 rows, folded, 22.3 / 20.1, 4096 -> 22016
 // 19.0 / 16.3; 4096 -> 12288 11.0 / 12.3, 11008 -> 4096 13.8 / 17.9), fp16 ones are not (prompts of 22 of the 7B model 3472 / 3749).
-bool block_plan(int fmt, int M, int N, int K, int cus, bool fold, BlockPlan* p) {
+bool block_plan(int fmt, int M, int N, int K, int cus, bool fold, BlockPlan* p, int only) {
   const BlockShapes sh = block_shapes_of(fmt);
   if (M <= (fmt == 16 ? 32 : 16) || M > (fold ? TI_FOLD_SS_ROWS : TI_GEMM_MAX_ROWS) || N < 16 || (N & 15) || K < 128 || (K & 127)) return false;
   const int NT = N >> 4, KT = K >> 7;
@@ -608,7 +608,7 @@ bool block_plan(int fmt, int M, int N, int K, int cus, bool fold, BlockPlan* p) 
   p->shape = -1;
   for (int i = 0; i < sh.n; ++i) {
     const BlockShape& s = sh.s[i];
-    if (fold && !s.fn[1]) continue;
+    if ((only >= 0 && i != only) || (fold && !s.fn[1])) continue;
     const int n_cb = (N + s.cols - 1) / s.cols, n_rb = (M + s.rows - 1) / s.rows;
     const long n = ((long)((n_cb + 7) / 8) * n_rb + cus / 8 - 1) / (cus / 8);   // (launched: whole XCD rows)
     const float one = (float)n * s.full;

@@ -312,7 +312,7 @@ static const FewShape* few_shapes_of(int fmt) {
 }
 
 // The shape whose rounds cost least, one row block (more rows than 48 read the weights twice: the many-rows kernel).
-bool few_plan(int fmt, int M, int N, int K, int cus, FewPlan* p) {
+bool few_plan(int fmt, int M, int N, int K, int cus, FewPlan* p, int only) {
   const FewShape* sh = few_shapes_of(fmt);
   if (!sh || M < 1 || M > 48 || N < 16 || (N & 15) || K < 128 || (K & 127)) return false;
   // (the kernel's byte offsets into rows and scales are 32 bits)
@@ -320,12 +320,12 @@ bool few_plan(int fmt, int M, int N, int K, int cus, FewPlan* p) {
   p->shape = -1;
   for (int i = 0; i < kFewShapes; ++i) {
     const FewShape& s = sh[i];
-    if (!s.fn || M > s.rows) continue;
+    if (!s.fn || (only >= 0 && i != only) || M > s.rows) continue;
     const int n_cb = ((N >> 4) + s.tiles - 1) / s.tiles;
     const float us = s.fix + (float)((n_cb + cus - 1) / cus) * (s.round + s.group * (float)(((K >> 7) + kFewWaves - 1) / kFewWaves));
     if (p->shape < 0 || us < p->us) *p = {i, n_cb, us};
   }
-  return true;
+  return p->shape >= 0;
 }
 
 int few_prepare() {

@@ -503,7 +503,7 @@ static const WideShape* wide_shapes_of(int fmt) {
 // every wave) as the call's rows need;
 // splits only into slices of at least 4 stages, whose blocks fit the workspace, and of at most two workgroups a CU
 // (the seam, measured: ~ 0.5 us + 0.65 us per MB of partial blocks).
-bool wide_plan(int fmt, int M, int N, int K, int cus, int64_t ws_bytes, bool fold, WidePlan* p) {
+bool wide_plan(int fmt, int M, int N, int K, int cus, int64_t ws_bytes, bool fold, WidePlan* p, int only) {
   const WideShape* sh = wide_shapes_of(fmt);
   if (!sh || M < 1 || M > TI_GEMM_MAX_ROWS || N < 16 || (N & 15) || K < 128 || (K & 127)) return false;
   const int NT = N >> 4, KT = K >> 7;
@@ -513,7 +513,7 @@ bool wide_plan(int fmt, int M, int N, int K, int cus, int64_t ws_bytes, bool fol
   p->shape = -1;
   for (int i = 0; i < kWideShapes; ++i) {
     const WideShape& s = sh[i];
-    if (!s.fn || (s.rows < 64 && M > s.rows) || (s.rows >= 64 && M <= 32) || (fold && s.rows > TI_FOLD_SS_ROWS)) continue;
+    if (!s.fn || (only >= 0 && i != only) || (s.rows < 64 && M > s.rows) || (s.rows >= 64 && M <= 32) || (fold && s.rows > TI_FOLD_SS_ROWS)) continue;
     const int n_cb = (NT + s.tiles - 1) / s.tiles, n_rb = (M + s.rows - 1) / s.rows;
     const long per_xcd = (long)((n_cb + 7) / 8) * n_rb;   // (launched: whole XCD rows)
     for (int ks = 1; ks <= 8; ks += ks < 4 ? 1 : 2) {
@@ -576,28 +576,33 @@ struct RowsPlan {
   int n_cb() const { return kernel == TI_ROWS_FEW ? f.n_cb : kernel == TI_ROWS_MANY ? w.n_cb : b.n_cb; }
 };
 static bool rows_plan_of(int kernel, int bits, int M, int N, int K, int64_t ws_bytes, bool fold, bool block, RowsPlan* p) {
-  const int cus = ti::gemm_cus();
+  const int cus = ti::gemm_cus(), only = kernel / TI_ROWS_SHAPE - 1;
+  kernel %= TI_ROWS_SHAPE;
   auto asked = [&](int k) { return kernel == TI_ROWS_AUTO || kernel == k; };
   p->kernel = TI_ROWS_AUTO;
   float us = 0.0f;   // of the kernel chosen, by the many-rows kernel's measure
-  if (asked(TI_ROWS_MANY) && ti::wide_plan(bits, M, N, K, cus, ws_bytes, fold, &p->w)) {
+  if (asked(TI_ROWS_MANY) && ti::wide_plan(bits, M, N, K, cus, ws_bytes, fold, &p->w, only)) {
     p->kernel = TI_ROWS_MANY;
     us = p->w.us;
   }
   const float few = (bits & ~TI_BITS_G32) == 4 ? 1.04f : 1.08f;
-  if (asked(TI_ROWS_FEW) && ti::few_plan(bits, M, N, K, cus, &p->f) && (p->kernel == TI_ROWS_AUTO || p->f.us < few * us)) {
+  if (asked(TI_ROWS_FEW) && ti::few_plan(bits, M, N, K, cus, &p->f, only) && (p->kernel == TI_ROWS_AUTO || p->f.us < few * us)) {
     p->kernel = TI_ROWS_FEW;
     us = p->f.us / few;
   }
-  if (asked(TI_ROWS_BLOCK) && block && ti::block_plan(bits, M, N, K, cus, fold, &p->b) &&
+  if (asked(TI_ROWS_BLOCK) && block && ti::block_plan(bits, M, N, K, cus, fold, &p->b, only) &&
       (p->kernel == TI_ROWS_AUTO || p->b.us < (bits == 16 ? 0.95f : 1.0f) * us))
     p->kernel = TI_ROWS_BLOCK;
   return p->kernel != TI_ROWS_AUTO;
 }
 
+static bool rows_kernel_ok(int kernel) {   // (a shape is one kernel's)
+  return kernel >= 0 && kernel % TI_ROWS_SHAPE <= TI_ROWS_BLOCK && (kernel < TI_ROWS_SHAPE || kernel % TI_ROWS_SHAPE != TI_ROWS_AUTO);
+}
+
 extern "C" int ti_gemm_rows_fold_partials_on(int kernel, int bits, int M, int N, int K, int64_t ws_bytes) {
   RowsPlan p;
-  if (M > TI_FOLD_SS_ROWS || kernel < TI_ROWS_AUTO || kernel > TI_ROWS_BLOCK || !rows_plan_of(kernel, bits, M, N, K, ws_bytes, true, true, &p))
+  if (M > TI_FOLD_SS_ROWS || !rows_kernel_ok(kernel) || !rows_plan_of(kernel, bits, M, N, K, ws_bytes, true, true, &p))
     return 0;
   return p.n_cb();
 }
@@ -609,7 +614,7 @@ static int rows_impl(int kernel, const void* tiles, const uint16_t* scales, int 
                      float eps, int M, int N, int K, const ti_epilogue* epi, ti_stream_t stream) {
   using namespace ti;
   if (!tiles || !x || !epi || !epi->out) return ti_set_error(TI_ERR_ARG, "ti_gemm_rows: null pointer");
-  if (kernel < TI_ROWS_AUTO || kernel > TI_ROWS_BLOCK) return ti_set_error(TI_ERR_ARG, "ti_gemm_rows: kernel %d", kernel);
+  if (!rows_kernel_ok(kernel)) return ti_set_error(TI_ERR_ARG, "ti_gemm_rows: kernel %d", kernel);
   if (bits != 16 && !scales) return ti_set_error(TI_ERR_ARG, "ti_gemm_rows: scales required for bits %d", bits);
   if (M < 1 || M > TI_GEMM_MAX_ROWS || K <= 0 || (K & 127) || N <= 0 || (N & 15) || ldx < K || K > 0xffff || ldx > 0xffff)
     return ti_set_error(TI_ERR_ARG, "ti_gemm_rows: M=%d N=%d K=%d ldx=%d", M, N, K, ldx);

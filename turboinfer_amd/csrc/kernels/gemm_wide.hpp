@@ -197,9 +197,9 @@ struct WidePlan {
   int rows, tiles;       // of a block
   float us;              // estimate
 };
-// fmt: the bits of ti_gemm_wq_a16.  fold: a call with a folded input or output.  False: not a call of this kernel (shape
-// or format).
-bool wide_plan(int fmt, int M, int N, int K, int cus, int64_t ws_bytes, bool fold, WidePlan* p);
+// fmt: the bits of ti_gemm_wq_a16.  fold: a call with a folded input or output.  only: the one shape to consider (-1: all).  False: not a
+// call of this kernel (shape or format).
+bool wide_plan(int fmt, int M, int N, int K, int cus, int64_t ws_bytes, bool fold, WidePlan* p, int only = -1);
 long wide_workgroups(const WidePlan& p);
 int wide_launch(int fmt, const WidePlan& p, const GemvArgs& a, hipStream_t s);
 int gemm_cus();       // CUs of the current device (gemv.hip)
@@ -211,7 +211,7 @@ struct FewPlan {
   int shape, n_cb;   // workgroup shape, column blocks
   float us;          // estimate
 };
-bool few_plan(int fmt, int M, int N, int K, int cus, FewPlan* p);
+bool few_plan(int fmt, int M, int N, int K, int cus, FewPlan* p, int only = -1);
 long few_workgroups(const FewPlan& p);
 int few_launch(int fmt, const FewPlan& p, const GemvArgs& a, hipStream_t s);
 int few_prepare();
@@ -222,7 +222,7 @@ struct BlockPlan {
   bool fold;
   float us;                // estimate
 };
-bool block_plan(int fmt, int M, int N, int K, int cus, bool fold, BlockPlan* p);
+bool block_plan(int fmt, int M, int N, int K, int cus, bool fold, BlockPlan* p, int only = -1);
 long block_workgroups(const BlockPlan& p);
 int block_launch(int fmt, const BlockPlan& p, const GemvArgs& a, hipStream_t s);
 int block_prepare();
