@@ -298,6 +298,8 @@ int ti_gemm_rows_fold_partials(int bits, int M, int N, int K, int64_t ws_bytes);
 enum ti_rows_kernel { TI_ROWS_AUTO = 0, TI_ROWS_FEW, TI_ROWS_MANY, TI_ROWS_BLOCK, TI_ROWS_SHAPE = 16 };
 int ti_gemm_rows_on(int kernel, const void* tiles, const uint16_t* scales, int bits, uint16_t* x, int ldx, const float* h,
                     const float* norm_w, float eps, int M, int N, int K, const ti_epilogue* epi, ti_stream_t s);
+/* The kernel of ti_gemm_rows for a call of these sizes with aligned rows and that epilogue (fold: a folded input or output); 0: none. */
+int ti_gemm_rows_kernel(int bits, int M, int N, int K, int64_t ws_bytes, int epilogue_kind, int fold);
 int ti_gemm_rows_fold_partials_on(int kernel, int bits, int M, int N, int K, int64_t ws_bytes);
 /* One-time kernel attribute setup; call before capturing ti_gemm_wq_a16 into a graph. */
 int ti_gemm_prepare(void);

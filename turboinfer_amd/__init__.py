@@ -142,7 +142,7 @@ EXPORTED = [
     "ti_wpack_q_host", "ti_engine_set_tensor_q", "ti_sample_workspace_bytes", "ti_sample_device_ws",
     "ti_wpack_q1_host", "ti_engine_set_tensor_q1", "ti_epilogue_bytes",
     "ti_sample_step_ws", "ti_hbm_calibrate", "ti_gemm_kernel_name",
-    "ti_gemm_fold_partials", "ti_gemm_rows", "ti_gemm_rows_folded", "ti_gemm_rows_fold_partials", "ti_gemm_rows_on", "ti_gemm_rows_fold_partials_on", "ti_engine_set_stop", "ti_engine_counters",
+    "ti_gemm_fold_partials", "ti_gemm_rows", "ti_gemm_rows_folded", "ti_gemm_rows_fold_partials", "ti_gemm_rows_on", "ti_gemm_rows_kernel", "ti_gemm_rows_fold_partials_on", "ti_engine_set_stop", "ti_engine_counters",
     "ti_qkv_attn_partials", "ti_qkv_attn_part_o_elems", "ti_qkv_attn_part_ml_elems", "ti_engine_set_qkv_attn",
     "ti_qkv_attn_xchg_bytes", "ti_qkv_attn_supported", "ti_qkv_attn_error_offset",
     "ti_engine_create_stack", "ti_engine_weight_count", "ti_engine_weight_info", "ti_engine_set_weight", "ti_engine_load",
@@ -197,6 +197,7 @@ def lib() -> C.CDLL:
         if hasattr(L, "ti_gemm_rows_on"):
             L.ti_gemm_rows_on.argtypes = [i32, vp, vp, i32, vp, i32, vp, vp, f32, i32, i32, i32, C.POINTER(Epilogue), vp]
             L.ti_gemm_rows_fold_partials_on.argtypes = [i32, i32, i32, i32, i32, i64]
+            L.ti_gemm_rows_kernel.argtypes = [i32, i32, i32, i32, i64, i32, i32]
         L.ti_gemm_lds_bytes.argtypes = [i32, i32, i32]
         L.ti_gemm_max_rows.argtypes = [i32, i32, i32, i32]
         L.ti_gemm_packed_rows.argtypes = [i32, i32]

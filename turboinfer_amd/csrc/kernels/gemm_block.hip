@@ -596,9 +596,7 @@ static BlockShapes block_shapes_of(int fmt) {   // rows x columns (by groups of 
   return {nullptr, 0};
 }
 
-// The shape whose busiest CU is done first.  A fold's sums and marks cost its calls ~ 1.5 us.  Up to 32 rows only
-// wide outputs are faster here (us, few-rows or many-rows kernel / 32 rows here: int4 4096 -> 28672 at 32 rows, folded, 22.3 / 20.1, 4096 -> 22016
-// 19.0 / 16.3; 4096 -> 12288 11.0 / 12.3, 11008 -> 4096 13.8 / 17.9), fp16 ones are not (prompts of 22 of the 7B model 3472 / 3749).
+// The shape whose busiest CU is done first.  A fold's sums and marks cost its calls ~ 1.5 us.
 bool block_plan(int fmt, int M, int N, int K, int cus, bool fold, BlockPlan* p, int only) {
   const BlockShapes sh = block_shapes_of(fmt);
   if (M <= (fmt == 16 ? 32 : 16) || M > (fold ? TI_FOLD_SS_ROWS : TI_GEMM_MAX_ROWS) || N < 16 || (N & 15) || K < 128 || (K & 127)) return false;

@@ -522,11 +522,11 @@ bool wide_plan(int fmt, int M, int N, int K, int cus, int64_t ws_bytes, bool fol
         break;
       const int nk = (KT + ks - 1) / ks;
       const long n = (per_xcd * ks + cus / 8 - 1) / (cus / 8);
-      const float one = (float)n * s.full, seam = ks > 1 ? 0.5f + 0.65e-6f * (float)ks * (float)n_cb * (float)n_rb * (float)s.slab : 0.0f;
-      const float us = 4.5f + (float)nk * (one > s.alone ? one : s.alone) + seam;
+      const float one = (float)n * s.full, mb = 1e-6f * (float)ks * (float)n_cb * (float)n_rb * (float)s.slab;
+      const float alone = 4.5f + (float)nk * (one > s.alone ? one : s.alone), us = ks > 1 ? alone + 0.5f + 0.65f * mb : alone;
       if (p->shape < 0 || us < best) {
         best = us;
-        *p = {i, n_cb, n_rb, ks, s.rows, s.tiles, us};
+        *p = {i, n_cb, n_rb, ks, s.rows, s.tiles, us, ks > 1 ? alone + 0.8f + 0.3f * (float)ks + 0.35f * mb : us};
       }
     }
   }
@@ -559,15 +559,21 @@ int wide_launch(int fmt, const WidePlan& p, const GemvArgs& a, hipStream_t strea
 
 }  // namespace ti
 
-// Which kernel a call of ti_gemm_rows takes: the few-rows one where its estimate is the lower (the many-rows kernel's is 4 % (int4,
-// also in blocks of 32) or 8 % low for calls of up to 48 rows; the choice costs 0.1 .. 0.8 % more than the better one of each of 700
-// measured points, by format, in the mean).
-// block: an output gemm_block_kernel writes (and 17 rows, fp16 33, of a fold to 64).  It takes the call where its estimate is below theirs
-// (0.95 of them for fp16: from there up the many-rows kernel was the faster as often as not; us, before / block at 64 rows: int4
-// 4096 -> 4096 11.9 / 9.4, 4096 -> 22016 26 / 21, 2048 -> 2560 9.8 / 6.4, int8 2048 -> 2048 9.4 / 6.0; at 48 rows int4 4096 ->
-// 12288 19.0 / 14.9, int8 4096 -> 22016 31.4 / 27.2).  The many-rows kernel keeps few rows by long K, split
-// over workgroups (int4 11008 -> 4096 at 64 rows 17.9 / 18.7; 14336 -> 4096 at 96 rows 27.4 / 27.3, fp16 11008 -> 4096 at 128 rows
-// 36.7 / 37.9), and short K, where the blocks' ends weigh.
+// Which kernel a call of ti_gemm_rows takes, by their estimates (the many-rows kernel's is 4 % (int4, also in blocks of 32), 12 % (int8 in
+// blocks of 32) or 8 % low for calls of up to 48 rows).
+//   Few rows: more than one round of workgroups over the CUs only up to 16 rows, int4 only for logits (us, few / many rows: int4 4096 ->
+//   28672 at 16 rows 18.8 / 17.5, 32000 logits 21.8 / 23.5; blocks of 32 bytes' 4096 -> 22016 at 31 rows 24.3 / 22.1).
+//   Block: an output that it writes (not logits), 33 rows and more (us, before / block at 64 rows: int4 4096 -> 4096 11.9 / 9.4, 4096 -> 22016
+//   26 / 21, 2048 -> 2560 9.8 / 6.4, int8 2048 -> 2048 9.4 / 6.0; at 48 rows int4 4096 -> 12288 19.0 / 14.9, int8 4096 -> 22016 31.4 / 27.2);
+//   17 to 32 of int4 (32 rows, folded, 4096 -> 28672 22.3 / 20.1, 4096 -> 22016 19.0 / 16.3), as the other formats' weights fill the time
+//   (int8 4096 -> 28672 at 17 rows 28.5 / 31.0, 4096 -> 22016 25.9 / 27.0; prompts of 22 of the 7B model in fp16 3472 / 3749).
+//   Against it a split costs 0.8 us, 0.3 a slice and 0.35 a MB of partial blocks (fitted to 700
+//   calls; the split itself is chosen by 0.5 and 0.65 a MB, and with it the order of its sums): the many-rows kernel keeps long K of few rows
+//   or narrow outputs (int4 11008 -> 4096 at 64 rows 17.9 / 18.7; 14336 -> 4096 at 96 26.3 / 27.3, fp16 5632 -> 2048 at 700 34.5 / 37.8),
+//   and short K, where the blocks' ends weigh.  fp16 folds: by 0.95 of the others' (as often slower
+//   as faster from there up: 4096 -> 12288 at 60 rows 27.8 / 28.8, 2048 -> 11264 15.7 / 14.6).
+// 6000 calls (3 .. 1024 rows, 21 (columns, K) of five formats, outputs and folds of a model): the choice costs 0.3 .. 0.9 % more than the best
+// of the three in the mean, by format.
 struct RowsPlan {
   int kernel;   // TI_ROWS_FEW, _MANY or _BLOCK
   ti::FewPlan f;
@@ -575,23 +581,28 @@ struct RowsPlan {
   ti::BlockPlan b;
   int n_cb() const { return kernel == TI_ROWS_FEW ? f.n_cb : kernel == TI_ROWS_MANY ? w.n_cb : b.n_cb; }
 };
-static bool rows_plan_of(int kernel, int bits, int M, int N, int K, int64_t ws_bytes, bool fold, bool block, RowsPlan* p) {
+// kind: of the epilogue; vec: its rows are whole 16-byte pieces (epilogue_vec)
+static bool rows_plan_of(int kernel, int bits, int M, int N, int K, int64_t ws_bytes, bool fold, int kind, bool vec, RowsPlan* p) {
   const int cus = ti::gemm_cus(), only = kernel / TI_ROWS_SHAPE - 1;
   kernel %= TI_ROWS_SHAPE;
   auto asked = [&](int k) { return kernel == TI_ROWS_AUTO || kernel == k; };
   p->kernel = TI_ROWS_AUTO;
-  float us = 0.0f;   // of the kernel chosen, by the many-rows kernel's measure
+  float us = 0.0f, whole = 0.0f;   // of the kernel chosen, by the many-rows kernel's measure
   if (asked(TI_ROWS_MANY) && ti::wide_plan(bits, M, N, K, cus, ws_bytes, fold, &p->w, only)) {
     p->kernel = TI_ROWS_MANY;
     us = p->w.us;
+    whole = p->w.whole;
   }
-  const float few = (bits & ~TI_BITS_G32) == 4 ? 1.04f : 1.08f;
-  if (asked(TI_ROWS_FEW) && ti::few_plan(bits, M, N, K, cus, &p->f, only) && (p->kernel == TI_ROWS_AUTO || p->f.us < few * us)) {
+  const float low = (bits & ~TI_BITS_G32) == 4 ? 1.04f : bits == (8 | TI_BITS_G32) ? 1.12f : 1.08f;
+  if (asked(TI_ROWS_FEW) && ti::few_plan(bits, M, N, K, cus, &p->f, only) &&
+      (p->kernel == TI_ROWS_AUTO ||
+       (p->f.us < low * us && (p->f.n_cb <= cus || (M <= 16 && (bits != 4 || kind == TI_EPI_LOGITS_ARGMAX)))))) {
     p->kernel = TI_ROWS_FEW;
-    us = p->f.us / few;
+    whole = p->f.us / low;
   }
-  if (asked(TI_ROWS_BLOCK) && block && ti::block_plan(bits, M, N, K, cus, fold, &p->b, only) &&
-      (p->kernel == TI_ROWS_AUTO || p->b.us < (bits == 16 ? 0.95f : 1.0f) * us))
+  if (asked(TI_ROWS_BLOCK) && vec && kind != TI_EPI_LOGITS_ARGMAX && (kernel != TI_ROWS_AUTO || bits == 4 || M > 32) &&
+      ti::block_plan(bits, M, N, K, cus, fold, &p->b, only) &&
+      (p->kernel == TI_ROWS_AUTO || p->b.us < (bits == 16 && fold ? 0.95f : 1.0f) * whole))
     p->kernel = TI_ROWS_BLOCK;
   return p->kernel != TI_ROWS_AUTO;
 }
@@ -602,12 +613,18 @@ static bool rows_kernel_ok(int kernel) {   // (a shape is one kernel's)
 
 extern "C" int ti_gemm_rows_fold_partials_on(int kernel, int bits, int M, int N, int K, int64_t ws_bytes) {
   RowsPlan p;
-  if (M > TI_FOLD_SS_ROWS || !rows_kernel_ok(kernel) || !rows_plan_of(kernel, bits, M, N, K, ws_bytes, true, true, &p))
+  if (M > TI_FOLD_SS_ROWS || !rows_kernel_ok(kernel) || !rows_plan_of(kernel, bits, M, N, K, ws_bytes, true, TI_EPI_RESID_F32, true, &p))
     return 0;
   return p.n_cb();
 }
 extern "C" int ti_gemm_rows_fold_partials(int bits, int M, int N, int K, int64_t ws_bytes) {
   return ti_gemm_rows_fold_partials_on(TI_ROWS_AUTO, bits, M, N, K, ws_bytes);
+}
+
+extern "C" int ti_gemm_rows_kernel(int bits, int M, int N, int K, int64_t ws_bytes, int kind, int fold) {
+  RowsPlan p;
+  if (M < 1 || M > (fold ? TI_FOLD_SS_ROWS : TI_GEMM_MAX_ROWS)) return 0;
+  return rows_plan_of(TI_ROWS_AUTO, bits, M, N, K, ws_bytes, fold != 0, kind, kind != TI_EPI_STORE_F16, &p) ? p.kernel : 0;
 }
 
 static int rows_impl(int kernel, const void* tiles, const uint16_t* scales, int bits, const void* x, int ldx, const float* h, const float* norm_w,
@@ -647,8 +664,7 @@ static int rows_impl(int kernel, const void* tiles, const uint16_t* scales, int 
     a.norm_w = norm_w;
     a.epi.fold_w = h;
   }
-  const bool fold = epi->ss_in || fold_out, block = a.vec && epi->kind != TI_EPI_LOGITS_ARGMAX;
-  if (!rows_plan_of(kernel, bits, M, N, K, epi->splitk_ws ? epi->splitk_bytes : 0, fold, block, &p))
+  if (!rows_plan_of(kernel, bits, M, N, K, epi->splitk_ws ? epi->splitk_bytes : 0, epi->ss_in || fold_out, epi->kind, a.vec != 0, &p))
     return ti_set_error(TI_ERR_UNSUPPORTED, "ti_gemm_rows: bits %d, M=%d N=%d K=%d", bits, M, N, K);
   const int rp = ti_gemm_prepare();   // no-op once this device is prepared
   if (rp != TI_OK) return rp;

@@ -195,7 +195,7 @@ struct WidePlan {
   int shape;             // workgroup shape (gemm_wide.hip), -1: none
   int n_cb, n_rb, n_ks;  // column blocks x row blocks x k-slices
   int rows, tiles;       // of a block
-  float us;              // estimate
+  float us, whole;       // estimate; the same with a split's seam as it is beside other launches (for the choice between kernels)
 };
 // fmt: the bits of ti_gemm_wq_a16.  fold: a call with a folded input or output.  only: the one shape to consider (-1: all).  False: not a
 // call of this kernel (shape or format).
