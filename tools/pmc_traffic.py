@@ -11,7 +11,7 @@ so bytes = FETCH_SIZE * 1024 * 2.  Infinity-Cache hits are counted as fetches.  
 over every dispatch of the kernel family in the pass (the replayed decode steps plus the
 bench's per-shape timing launches, same mixture of shapes).
 
-Families: the decode GEMM (every launch of gemv_wq_kernel / gemm_rows_kernel / gemm_wide_kernel:
+Families: the decode GEMM (every launch of gemv_wq_kernel, gemm_rows_kernel or a kernel of ti_gemm_rows:
 one projection each) and the attention (attn_split_kernel, attn_spread_kernel).
 The GEMM family's key is the one bench.py's roofline names: "gemv_wq_kernel<BITS>" for one stream
 (the fused kernel runs every projection), "gemm_family" for batched steps (rows / tile kernels)."""
@@ -25,7 +25,7 @@ MODELS = {   # bench.py MODELS: vocab, hidden, layers, heads, kv_heads, head_dim
     "tinyllama-1.1b": (32000, 2048, 22, 32, 4, 64, 5632, 8),
     "llama3-8b": (128256, 4096, 32, 32, 8, 128, 14336, 4),
 }
-GEMM = ("gemv_wq_kernel", "gemm_rows_kernel", "gemm_wide_kernel", "gemm_few_kernel", "gemv_mbr_kernel",
+GEMM = ("gemv_wq_kernel", "gemm_rows_kernel", "gemm_wide_kernel", "gemm_few_kernel", "gemm_block_kernel", "gemv_mbr_kernel",
         "qkv_attn_kernel")   # (the fused QKV + attention of one stream, DESIGN 4.19: its step position is QKV's)
 
 
