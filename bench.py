@@ -427,8 +427,10 @@ def main() -> int:
 
     def class_kernel(name):
         N_, K_ = shapes[name]
-        if B >= 3:   # (up to 48 rows whichever of the two is estimated the faster)
-            return "gemm_wide_kernel" if B > 48 else "gemm_few_kernel / gemm_wide_kernel"
+        if B >= 3:   # (the engine folds the norms of up to 64 rows into every product but the lm_head's)
+            kind = {"qkv": T.EPI_QKV_ROPE_KV, "gate_up": T.EPI_SILU_MUL_F16, "lm_head": T.EPI_LOGITS_ARGMAX}.get(name, T.EPI_RESID_F32)
+            return T.rows_kernel_name(bits, B, N_, K_, kind, name != "lm_head" and B <= 64 and os.environ.get("TI_FOLD", "1") != "0",
+                                      max(0, int(os.environ.get("TI_SPLITK_MB", "64"))) << 20)
         if name in ("qkv", "gate_up", "lm_head"):
             if fold_on:
                 xk = T.X_F16_FOLDED

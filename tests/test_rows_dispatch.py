@@ -32,3 +32,12 @@ def test_rows_kernel_refuses():
     L = T.lib()
     for a in [(5, 4, 64, 128, 0, 0, 0), (4, 0, 64, 128, 0, 0, 0), (4, 1025, 64, 128, 0, 0, 0), (4, 65, 64, 128, 0, 0, 1), (4, 4, 60, 128, 0, 0, 0), (4, 4, 64, 100, 0, 0, 0)]:
         assert L.ti_gemm_rows_kernel(*a) == 0, a
+
+
+def test_rows_kernel_name():
+    """The labels of a step of 64 int4 streams: three products on the block kernel, the split one and the logits on the many-rows one."""
+    got = [T.rows_kernel_name(4, 64, n, k, kind, fold) for n, k, kind, fold in
+           [(12288, 4096, T.EPI_QKV_ROPE_KV, True), (4096, 4096, T.EPI_RESID_F32, True), (22016, 4096, T.EPI_SILU_MUL_F16, True),
+            (4096, 11008, T.EPI_RESID_F32, True), (32000, 4096, T.EPI_LOGITS_ARGMAX, False)]]
+    assert got == ["gemm_block_kernel"] * 3 + ["gemm_wide_kernel"] * 2
+    assert T.rows_kernel_name(4, 64, 60, 128, T.EPI_STORE_F32) == ""

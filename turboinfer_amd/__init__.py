@@ -388,6 +388,12 @@ def gemm_kernel_name(bits: int, x_kind: int, M: int, N: int, K: int) -> str:
     return buf.value.decode()
 
 
+def rows_kernel_name(bits: int, M: int, N: int, K: int, kind: int, fold: bool = False, ws_bytes: int = 64 << 20) -> str:
+    """The kernel of ti_gemm_rows for a call of these sizes (ti_gemm_rows_kernel; bench / profile labels)."""
+    k = lib().ti_gemm_rows_kernel(bits, M, N, K, ws_bytes, kind, int(fold))
+    return {ROWS_FEW: "gemm_few_kernel", ROWS_MANY: "gemm_wide_kernel", ROWS_BLOCK: "gemm_block_kernel"}.get(k, "")
+
+
 def sync() -> None:
     check(lib().ti_device_sync())
 
