@@ -217,8 +217,8 @@ def test_engine_7b_64_streams(ti, oracle):
 
 
 def test_engine_7b_40_streams(ti, oracle):
-    """40 streams of the 7B shape: every projection on the many-rows kernel, its row blocks
-    partly full; a stream in each third of the rows against the oracle (the 64-stream test's streams, same caches and first tokens)."""
+    """40 streams of the 7B shape: queries, keys and values and gate/up on the block kernel, O on the few-rows one and down on the
+    many-rows one (K split), their row blocks partly full; a stream in each third of the rows against the oracle (the 64-stream test's streams, same caches and first tokens)."""
     _full_shape_streams(ti, oracle, CFG_7B, 2025, 40, [1, 17, 35], 4)
 
 

@@ -189,11 +189,12 @@ __device__ __forceinline__ float block_share(const GemvArgs& a, int m, int part,
   return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, t) | (any & 0x80000000u));
 }
 
-// Bound: the vector unit beside the matrix cores, and the clock, which falls to 1.4 .. 2.0 GHz at this rate.  A 32x32x16 MFMA
+// Bound: the vector unit beside the matrix cores (7 .. 9 vector instructions an MFMA; the matrix cores are busy 44 .. 58 % of a
+// launch of a 7B int4 prompt of 512) and the clock, ~ 2.0 GHz while prompts run.  A 32x32x16 MFMA
 // holds the vector issue for ~ 8 cycles of its 32 and does twice a 16x16x32's work (7.5 of 16): as many scale FMAs per product
 // leave time for the unpacking.  The weights pass LDS by (each is read by one wave only): half the DMA, whose bursts with the
-// barriers' skew were half of a stage in gemm_wide_kernel (int4, cycles per 64 x 256 columns and 128 k: 64 x 384 blocks 2130,
-// 48 % MFMA -> 64 x 256 blocks here 1440 at 71 %).  Copies of the rows are issued four to an M0 setting, the weights' loads
+// barriers' skew were half of a stage in gemm_wide_kernel (int4, cycles of the main loop per 64 x 256 columns and 128 k: 64 x 384
+// blocks 2130, 48 % MFMA -> 64 x 256 blocks here 1440 at 71 %).  Copies of the rows are issued four to an M0 setting, the weights' loads
 // spread over the steps of a stage.  us, gemm_wide_kernel -> here: int4 512 rows 4096 -> 22016 114 -> 100, 11008 -> 4096 64 ->
 // 56, 4096 -> 4096 30 -> 23.5, 4096 -> 12288 63 -> 60; int8 1000 rows 2048 -> 11264 75 -> 60.5, 5632 -> 2048 43.5 -> 35, 2048 ->
 // 2560 25.7 -> 22.5; fp16 333 rows 33.5 -> 25.4, 30.7 -> 23.5, 12.1 -> 11.2.  Whole prompts: 7B int4 of 512 rows 9159 -> 8184,
@@ -531,7 +532,8 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_block_kernel(const GemvA
 // ------------------------------------------------------------------ host: shapes, plan, launch
 // Estimated us: fix + stages * max(alone, full * rounds) + round * rounds, a round being one workgroup on each CU (fitted, per
 // shape and format, to 10 .. 13 numbers of rows from 65 to 1024 by 14 (columns, K) from 1024 x 2048 to 22016 x 4096 and 4096 x 11008
-// with the epilogues a model has there, weights from HBM).  Blocks of 32 rows and of 4 groups of waves are for grids that would leave
+// with the epilogues a model has there, weights from HBM).  Fewer rows are taken by the same numbers: of 17 to 64 rows a launch takes 0.9 ..
+// 1.1 (int4), 1.0 .. 1.4 (int8) and 1.0 .. 1.5 (fp16) of its estimate, by shape, the more the more its weights fill the time.  Blocks of 32 rows and of 4 groups of waves are for grids that would leave
 // CUs idle or a wave a SIMD (us, without -> with, int4: 2048 -> 2048 at 128 rows 9.9 -> 7.3, 5632 -> 2048 at 333 22.4 -> 17.5, 4096 -> 12288 at
 // 150 30.8 -> 23.7; int8: 11008 -> 4096 at 150 38.8 -> 31.9, 5632 -> 2048 at 333 22.6 -> 19.4; fp16: 2048 -> 2560 at 128 11.3 -> 9.8; the
 // mean up to 640 rows 9 %, 6 % and 4 %).
@@ -544,7 +546,8 @@ template <int F, int WN, int KG, int RT, int CT, int NS>
 static BlockShape block_shape(float fix, float alone, float full, float round) {
   typedef BlockGemm<F, WN, KG, RT, CT, NS> C;
   const void* fold = nullptr;
-  if constexpr (RT <= 2) fold = (const void*)gemm_block_kernel<F, WN, KG, RT, CT, NS, true>;   // (a fold's calls have up to 64 rows)
+  // (a fold's calls have up to 64 rows; int4's 64 x 256 is the fastest of none of them, and spills)
+  if constexpr (RT <= 2 && CT == 1) fold = (const void*)gemm_block_kernel<F, WN, KG, RT, CT, NS, true>;
   return {{(const void*)gemm_block_kernel<F, WN, KG, RT, CT, NS, false>, fold}, C::kRows, C::kCols, KG, 64 * C::kWaves, {C::kLds, C::kFoldLds}, fix, alone, full, round};
 }
 struct BlockShapes {

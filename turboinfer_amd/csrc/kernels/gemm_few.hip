@@ -248,7 +248,8 @@ __global__ __launch_bounds__(64 * kFewWaves, 2) void gemm_few_kernel(const GemvA
 // Blocks of 3 tiles and more, and 2 at 48 rows, keep 5632 .. 22016 columns in one round, where the many-rows kernel took them or a
 // second round began.  us, before -> this: int4 2048 -> 11264 at 24 rows 8.8 -> 7.1, 4096 -> 12288 at 16 rows 9.1 -> 8.3, 32 rows 14.0 ->
 // 10.7, 4096 -> 6144 at 48 rows 13.9 -> 12.3; int8 2048 -> 11264 at 24 rows 9.7 -> 8.7; blocks of 32 bytes' 1024 -> 5632 at 40 rows
-// 9.7 -> 6.0.  (fp16: 16 x 48 spills and gains 0 .. 10 %.)
+// 9.7 -> 6.0.  (fp16: 16 x 48 spills and gains 0 .. 10 %; int4's 48 x 32 keeps three addresses in scratch, once, ahead of its
+// main loop, and gains 22 .. 32 % at 36 .. 48 rows.)
 struct FewShape {
   const void* fn;
   int rows, tiles, lds;
