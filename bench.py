@@ -1,6 +1,6 @@
 #!/usr/bin/env python3
 """bench.py -- decode tokens/s per GPU, Llama-2-7B-shape INT4 (group 128) at 2048-token KV,
-and the achieved fraction of the HBM-read roofline (BASELINE.json `metric`, configs[2]).
+and the achieved fraction of the HBM-read roofline.
 
     python bench.py [--gpus N] [--steps K] [--warmup W] [--batch B] [--kv L] [--model llama2-7b]
 
@@ -9,7 +9,7 @@ model with B decode streams (requests) and their fp16 KV caches in its own HBM: 
 shards by request, there is no collective on the data path (torch.distributed/gloo only
 carries the barrier and the max-over-ranks of the timing).  A step = one decode token for
 each of the rank's B streams, replayed at position L-1 so every step reads exactly L cache
-slots (SURVEY 8(d) replay mode), greedy feedback on the device.  Synthetic random weights of
+slots, greedy feedback on the device.  Synthetic random weights of
 the named architecture (no checkpoints are reachable); `data` says so.
 
 rank 0 prints ONE JSON line with the contract fields plus `roofline` (dominant kernel:
@@ -56,7 +56,7 @@ HBM_PEAK_GBS = 8000.0   # MI355X HBM3E spec peak (MI355X_MICROARCH.md, chip-leve
 
 
 def step_bytes(m, B, L):
-    """Algorithmic HBM bytes of one decode step (SURVEY 8(d)): weights once + B streams' KV."""
+    """Algorithmic HBM bytes of one decode step: weights once + B streams' KV."""
     import turboinfer_amd as T
     V, H, layers, nh, nkv, hd, I, bits, _ = m
     lib = T.lib()
@@ -373,7 +373,7 @@ def main() -> int:
     import turboinfer_amd as T
 
     T.init(g.local_rank)
-    # same-run calibration of this box's HBM: every rate below can be read
+    # same-run calibration of this card's HBM: every rate below can be read
     # against it (1 GiB read by 2 workgroups per CU; device-to-device copy, read + write bytes)
     hbm_read, hbm_copy = T.hbm_calibrate(1 << 30, 5)
     m = MODELS[args.model]
@@ -442,7 +442,7 @@ def main() -> int:
             xk = T.X_ATTN_SPLITS if name == "o" and B == 1 else T.X_F16
         return T.gemm_kernel_name(bits, xk, B, N_, K_)
 
-    # In-step timing (VERDICT r5 item 3): the replay step graph captured with per-workgroup
+    # In-step timing: the replay step graph captured with per-workgroup
     # s_memrealtime stamps (ti_engine_stamp_steps).  A launch's duration is its period in the step:
     # its first workgroup's entry -> the next launch's first entry (its boundary included; the
     # periods of a step add up to the step), averaged over the class's launches and `stamp_steps`

@@ -118,7 +118,7 @@ int ti_wpack_q_host(const int8_t* q, const uint16_t* d, int K, int N_src, int N_
 int ti_wpack_q1_host(const uint8_t* q, const uint16_t* d, const uint16_t* m, int K, int N_src, int N_total, int row_map,
                      int row_offset, void* tiles, uint16_t* scales);
 
-/* The synthetic model of SURVEY 8(d) generated straight into device tiles:
+/* The synthetic model (seeded uniform weights) generated straight into device tiles:
  * element (k, c) of tensor `tensor_id` = u(seed, tensor_id, k*N_src + c) * amp,
  * amp = sqrtf(3)/sqrtf(K) (u: or_synth_unit), quantized per group like ti_wpack_host. */
 int ti_wsynth_device(uint64_t seed, uint32_t tensor_id, int K, int N_src, int N_total, int bits,

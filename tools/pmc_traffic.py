@@ -1,12 +1,12 @@
-"""HBM traffic per launch from a rocprofv3 FETCH_SIZE pass (GPU-box output -> profiles/).
+"""HBM traffic per launch from a rocprofv3 FETCH_SIZE pass.
 
-    rocprofv3 --pmc FETCH_SIZE --output-format csv -d gpurun_out/pmc -o run -- \
+    rocprofv3 --pmc FETCH_SIZE --output-format csv -d out/pmc -o run -- \
         python3 bench.py --steps 4 --warmup 2 --kernel-reps 4 --no-cpu-baseline [--model M --batch B]
-    python tools/pmc_traffic.py gpurun_out/pmc/run_counter_collection.csv profiles/r5_pmc_traffic.json \
+    python tools/pmc_traffic.py out/pmc/run_counter_collection.csv profiles/pmc_traffic.json \
         [--model llama2-7b --batch 1 --kv 2048]
 
 FETCH_SIZE is reported in KiB and, on gfx950, counts a wide coalesced streaming read at
-exactly half its bytes (MI355X_MICROARCH.md, HBM section: 128-B requests tallied as 64 B),
+exactly half its bytes (128-B requests tallied as 64 B),
 so bytes = FETCH_SIZE * 1024 * 2.  Infinity-Cache hits are counted as fetches.  The mean is
 over every dispatch of the kernel family in the pass (the replayed decode steps plus the
 bench's per-shape timing launches, same mixture of shapes).
@@ -14,7 +14,7 @@ bench's per-shape timing launches, same mixture of shapes).
 Families: the decode GEMM (every launch of gemv_wq_kernel, gemm_rows_kernel or a kernel of ti_gemm_rows:
 one projection each) and the attention (attn_split_kernel, attn_spread_kernel).
 The GEMM family's key is the one bench.py's roofline names: "gemv_wq_kernel<BITS>" for one stream
-(the fused kernel runs every projection), "gemm_family" for batched steps (rows / tile kernels)."""
+(the fused kernel runs every projection), "gemm_family" for batched steps."""
 import argparse
 import csv
 import json
@@ -26,7 +26,7 @@ MODELS = {   # bench.py MODELS: vocab, hidden, layers, heads, kv_heads, head_dim
     "llama3-8b": (128256, 4096, 32, 32, 8, 128, 14336, 4),
 }
 GEMM = ("gemv_wq_kernel", "gemm_rows_kernel", "gemm_wide_kernel", "gemm_few_kernel", "gemm_block_kernel", "gemv_mbr_kernel",
-        "qkv_attn_kernel")   # (the fused QKV + attention of one stream, DESIGN 4.19: its step position is QKV's)
+        "qkv_attn_kernel")   # (the fused QKV + attention of one stream: its step position is QKV's)
 
 
 def lin_bytes(bits, K, N):
