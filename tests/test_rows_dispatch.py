@@ -12,6 +12,7 @@ CALLS = [
     (4, 16, 32000, 4096, T.EPI_LOGITS_ARGMAX, 0, T.ROWS_FEW),                           # few 21.8, many 23.5
     *[(8, m, 28672, 4096, T.EPI_SILU_MUL_F16, 1, T.ROWS_MANY) for m in (17, 24, 32)],   # block 31, many 28.5 .. 29.9
     *[(8, m, 22016, 4096, T.EPI_SILU_MUL_F16, 1, T.ROWS_MANY) for m in (17, 22)],       # block 27.0 .. 27.4, many 25.9 .. 26.8
+    (8, 32, 22016, 4096, T.EPI_SILU_MUL_F16, 1, T.ROWS_BLOCK),                          # block 27.0, many 27.9
     *[(36, m, 22016, 4096, T.EPI_SILU_MUL_F16, 1, T.ROWS_MANY) for m in (17, 24, 32)],  # few 23.7 .. 24.3, many 22
     *[(40, m, 4096, 11008, T.EPI_RESID_F32, 1, T.ROWS_FEW) for m in (3, 8)],            # few 12.7, many 15.5
     (16, 700, 2048, 5632, T.EPI_RESID_F32, 0, T.ROWS_MANY),                             # block 37.8, many 34.5

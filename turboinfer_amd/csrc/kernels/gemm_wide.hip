@@ -565,8 +565,9 @@ int wide_launch(int fmt, const WidePlan& p, const GemvArgs& a, hipStream_t strea
 //   28672 at 16 rows 18.8 / 17.5, 32000 logits 21.8 / 23.5; blocks of 32 bytes' 4096 -> 22016 at 31 rows 24.3 / 22.1).
 //   Block: an output that it writes (not logits), 33 rows and more (us, before / block at 64 rows: int4 4096 -> 4096 11.9 / 9.4, 4096 -> 22016
 //   26 / 21, 2048 -> 2560 9.8 / 6.4, int8 2048 -> 2048 9.4 / 6.0; at 48 rows int4 4096 -> 12288 19.0 / 14.9, int8 4096 -> 22016 31.4 / 27.2);
-//   17 to 32 of int4 (32 rows, folded, 4096 -> 28672 22.3 / 20.1, 4096 -> 22016 19.0 / 16.3), as the other formats' weights fill the time
-//   (int8 4096 -> 28672 at 17 rows 28.5 / 31.0, 4096 -> 22016 25.9 / 27.0; prompts of 22 of the 7B model in fp16 3472 / 3749).
+//   17 to 32 of int4 (32 rows, folded, 4096 -> 28672 22.3 / 20.1, 4096 -> 22016 19.0 / 16.3), and 25 to 32 of int8 up to 24576 columns (4096 ->
+//   22016 at 32 rows 27.9 / 27.0, at 17 25.8 / 26.8), as wider weights fill the time (int8 4096 -> 28672 at 17 rows 28.3 / 31.0, at 32 29.9 /
+//   30.7; prompts of 22 of the 7B model in fp16 3472 / 3749).
 //   Against it a split costs 0.8 us, 0.3 a slice and 0.35 a MB of partial blocks (fitted to 700
 //   calls; the split itself is chosen by 0.5 and 0.65 a MB, and with it the order of its sums): the many-rows kernel keeps long K of few rows
 //   or narrow outputs (int4 11008 -> 4096 at 64 rows 17.9 / 18.7; 14336 -> 4096 at 96 26.3 / 27.3, fp16 5632 -> 2048 at 700 34.5 / 37.8),
@@ -600,7 +601,7 @@ static bool rows_plan_of(int kernel, int bits, int M, int N, int K, int64_t ws_b
     p->kernel = TI_ROWS_FEW;
     whole = p->f.us / low;
   }
-  if (asked(TI_ROWS_BLOCK) && vec && kind != TI_EPI_LOGITS_ARGMAX && (kernel != TI_ROWS_AUTO || bits == 4 || M > 32) &&
+  if (asked(TI_ROWS_BLOCK) && vec && kind != TI_EPI_LOGITS_ARGMAX && (kernel != TI_ROWS_AUTO || M > 32 || bits == 4 || (bits == 8 && M > 24 && N <= 24576)) &&
       ti::block_plan(bits, M, N, K, cus, fold, &p->b, only) &&
       (p->kernel == TI_ROWS_AUTO || p->b.us < (bits == 16 && fold ? 0.95f : 1.0f) * whole))
     p->kernel = TI_ROWS_BLOCK;
