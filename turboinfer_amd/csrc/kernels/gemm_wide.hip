@@ -289,9 +289,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const GemvAr
   // batched fold (decode rows, ti_hip.h TI_FOLD_SS_ROWS): this thread's share of its row's sum of squares
   const bool fold_in = C::kFold && a.epi.ss_in != nullptr;
   const float share = fold_in ? wide_fold_share(a, m0 + tid % C::kRows, tid / C::kRows, 64 * NW / C::kRows) : 0.0f;
-  // What the epilogue reads is asked for behind the main loop, a tile at a time: blocks of 64 x 64 (one tile a wave) start on it
-  // with their products.  Of 16 and 32 rows they lose by that (us, 16 x 64, int4: 512 -> 256 4.4 -> 4.0, 1024 -> 1024 split over K 5.9 ->
-  // 5.5; 7 .. 17 registers more, a wave a SIMD less).
+  // What the epilogue reads: blocks of 64 x 64 (one tile a wave) ask for it beside their products, the others behind the main loop, a
+  // tile at a time (us, 16 x 64 blocks of int4, early -> late: 512 -> 256 4.4 -> 4.0, 1024 -> 1024 split over K 5.9 -> 5.5; early, 16 and 32 rows
+  // take 10 .. 17 registers more, a wave a SIMD).
   constexpr bool kEarly = TN == 1 && TM == 4;
   TilePre<TM> pre;
   if constexpr (kEarly) tile_pos<TM>(a, m0 + wm * 16 * TM, lane, pre);
@@ -418,7 +418,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const GemvAr
 #pragma unroll
         for (int b = 0; b < TM; ++b) av[b] = acc[tt][b];
     if (tn >= NT) continue;
-    // (values of this tile: the rows' addresses of every epilogue, taken out of the loop, are 40 .. 55 registers, and int4's 64 x 128
+    // (values of this tile: the rows' addresses of every epilogue, taken out of the loop, are up to 56 registers, and int4's 64 x 128
     // blocks run 3 a CU: 4096 -> 22016 at 1024 rows 215 -> 194 us)
     int ln = lane;
     if constexpr (TN > 1) {
