@@ -533,7 +533,8 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_block_kernel(const GemvA
 // Estimated us: fix + stages * max(alone, full * rounds) + round * rounds, a round being one workgroup on each CU (fitted, per
 // shape and format, to 10 .. 13 numbers of rows from 65 to 1024 by 14 (columns, K) from 1024 x 2048 to 22016 x 4096 and 4096 x 11008
 // with the epilogues a model has there, weights from HBM).  Fewer rows are taken by the same numbers: of 17 to 64 rows a launch takes 0.9 ..
-// 1.1 (int4), 1.0 .. 1.4 (int8) and 1.0 .. 1.5 (fp16) of its estimate, by shape, the more the more its weights fill the time.  Blocks of 32 rows and of 4 groups of waves are for grids that would leave
+// 1.1 (int4), 1.0 .. 1.4 (int8) and 1.0 .. 1.5 (fp16) of its estimate, by shape, the more the more its weights fill the time.
+// Blocks of 32 rows and of 4 groups of waves are for grids that would leave
 // CUs idle or a wave a SIMD (us, without -> with, int4: 2048 -> 2048 at 128 rows 9.9 -> 7.3, 5632 -> 2048 at 333 22.4 -> 17.5, 4096 -> 12288 at
 // 150 30.8 -> 23.7; int8: 11008 -> 4096 at 150 38.8 -> 31.9, 5632 -> 2048 at 333 22.6 -> 19.4; fp16: 2048 -> 2560 at 128 11.3 -> 9.8; the
 // mean up to 640 rows 9 %, 6 % and 4 %).
