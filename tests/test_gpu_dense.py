@@ -173,6 +173,37 @@ def test_grouped_swiglu(ti, dtype, tile_rows, N, K):
     assert (out[M] == 7).all()
 
 
+@pytest.mark.parametrize("epi", ["T", "SWIGLU"])
+@pytest.mark.parametrize("tiles_n,N,K", [(122, 1072, 192), (77, 1024, 256), (9, 520, 320), (3, 2048, 1408)])
+def test_expert_rounds(ti, epi, tiles_n, N, K):
+    """256-row tiles on workgroups that stay: from one block for some of them to four each, of every height, the last columns
+    ragged (1072, 520) or whole, the shortest k that they take; a second call finds nothing of the first."""
+    r = np.random.default_rng(tiles_n)
+    rows = np.sort(np.r_[256, 1, r.integers(1, 257, tiles_n - 2)])[::-1]
+    experts = 5
+    a, w, f = operands(int(rows.sum()) // 2 + 1, N, K, torch.bfloat16, experts, 3)
+    n_in = int(rows.sum())
+    order = torch.randperm(n_in, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1)).int()
+    first = np.r_[0, np.cumsum(rows)[:-1]]
+    tl = torch.zeros(tiles_n + 9, 4, dtype=torch.int32, device="cuda")
+    tl[:tiles_n] = torch.tensor([(i % experts, int(s), int(c), 0) for i, (s, c) in enumerate(zip(first, rows))], dtype=torch.int32)
+    n = torch.tensor([tiles_n], dtype=torch.int32, device="cuda")
+    cols = N // 2 if epi == "SWIGLU" else N
+    for _ in range(2):
+        out = torch.full((n_in + 1, cols), 7.0, device="cuda").bfloat16()
+        d = ti.DenseArgs(w=f.data_ptr(), w_batch=f[0].numel(), a=a.data_ptr(), out=out.data_ptr(), lda=K, ldo=cols, M=len(a), N=N, K=K, batch=1,
+                         epi=ti.DE_SWIGLU if epi == "SWIGLU" else ti.DE_T, dtype=ti.DT_BF16, tile_rows=256, max_tiles=len(tl), tiles=tl.data_ptr(),
+                         n_tiles=n.data_ptr(), rows_in=order.data_ptr(), rows_out=order.data_ptr(), row_div=2)
+        call(ti, d)
+        for i in range(tiles_n):
+            at = order[int(first[i]) : int(first[i] + rows[i])].long()
+            if epi == "SWIGLU":
+                check_swiglu(out[at], a[at // 2], w[i % experts], torch.bfloat16)
+            else:
+                check(out[at], a[at // 2], w[i % experts], torch.bfloat16, True)
+        assert (out[n_in] == 7).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M", [5, 200])
 def test_gelu(ti, dtype, M):

@@ -711,13 +711,15 @@ int StackModel::experts(const StackLayer& L, int M) {
     g.tiles = idx_;
     if (!routed) TI_TRY(ti_route(&ra, s_));
   } else {
-    // rows a tile: by the mean rows of an expert.  Measured, bf16 (64 experts, gate/up 2816 x 2048, us at 37 / 75 / 131 /
-    // 192 rows): 64-row tiles 137 / 211 / 246 / 297, 128 137 / 158 / 240 / 258, 256 148 / 165 / 190 / 226; 32 experts,
-    // 1536 x 1024, at 256 rows: 128 55, 256 83 -- too few blocks: 256 only from two a CU on.  fp32: the products decide,
-    // and the smaller tile has less padding (a 2048-wide model's 650 rows: 64 12.0 ms, 128 12.9).
+    // rows a tile: by the mean rows of an expert.  Measured, bf16, gate/up + down, us of 64 / 128 / 256-row tiles (256:
+    // dense_expert_kernel): 64 experts, 2816 x 2048, at 6 mean rows 189 / 189 / 192, 14 191 / 184 / 190, 28 228 / 200 / 202, 37 231 /
+    // 207 / 206, 48 243 / 212 / 209, 72 284 / 260 / 228, 96 307 / 285 / 238; 32 experts, 1536 x 1024 (too few blocks of 256 columns for the CUs),
+    // at 32 36.4 / 34.6 / 35.7, 64 49 / 45 / 43, 128 56 / 57 / 60, 162 67 / 65 / 63, 192 70 / 73 / 65, 256 89 / 92 / 71.  fp32: the products
+    // decide, and the smaller tile has less padding (a 2048-wide model's 650 rows: 64 12.0 ms, 128 12.9).
     const long mean = (long)M * k.top / k.experts, blocks = (long)k.experts * (std::min(W, 2 * k.ff) / 256);
     const bool f32 = c.dtype == TI_DT_F32;
-    ra.tile_rows = M <= 64 ? 16 : !f32 && mean >= 96 && blocks >= 512 ? 256 : mean >= (f32 ? 96 : 48) ? 128 : 64;
+    const bool wide = blocks >= 512;
+    ra.tile_rows = M <= 64 ? 16 : !f32 && mean >= (wide ? 36 : 160) ? 256 : mean >= (f32 ? 96 : wide ? 6 : 48) ? 128 : 64;
     TI_TRY(ti_route(&ra, s_));
     g.tile_rows = ra.tile_rows;
     g.max_tiles = ti_route_max_tiles(M, k.experts, k.top, ra.tile_rows);

@@ -137,6 +137,18 @@ __device__ __forceinline__ void dma_1k_asm(const void* src_lane, uint32_t lds) {
                : "memory");
 }
 
+// The same from a wave-uniform address and a byte offset a lane.
+__device__ __forceinline__ void dma_1k_asm(const void* src, uint32_t off_lane, uint32_t lds) {
+  const uint64_t u = (uint64_t)src;
+  const void* at = (const void*)((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(u >> 32)) << 32 |
+                                 (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)u));
+  uint32_t keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep)
+               : "v"(off_lane), "s"(at), "s"(__builtin_amdgcn_readfirstlane(lds))
+               : "memory");
+}
+
 // max / sum with the lane 16 or 32 apart (l ^ 16, l ^ 32) through gfx950's v_permlane16/32_swap,
 // VALU only (a __shfl_xor across rows is an LDS round trip): after a swap of x with itself, lane l
 // holds x[l] in one result and x[l ^ 16] (x[l ^ 32]) in the other, in some order -- max and + of
