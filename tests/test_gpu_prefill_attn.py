@@ -141,3 +141,18 @@ def test_prefill_attention_keys(ti, M, nh, nkv, hd, start, keys):
     got = out.download(f16, (M, nh * hd)).astype(f32)
     assert np.all(np.isfinite(got))
     np.testing.assert_allclose(got, dec, rtol=4e-3, atol=4e-3)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("nkv", [1, 2, 3, 4, 5, 8, 9, 17])
+@pytest.mark.parametrize("M,start", [(150, 0), (397, 31)])
+def test_prefill_attention_kv_heads(ti, nkv, hd, M, start):
+    """Every count of kv-heads finds its workgroups on the XCDs (1, 2 and 4 share them, others go round), with two and with four
+    query blocks a workgroup."""
+    for shared in (0, 3):
+        assert ti.lib().ti_attn_prefill_set_kernel(shared) == 0
+        try:
+            _, _, _, got, dec = _case(ti, M, 2 * nkv, nkv, hd, (start + np.arange(M)).astype(np.int32), start + M + 3, seed=nkv)
+        finally:
+            assert ti.lib().ti_attn_prefill_set_kernel(0) == shared
+        np.testing.assert_allclose(got, dec, rtol=4e-3, atol=4e-3)

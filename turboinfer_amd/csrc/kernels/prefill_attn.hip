@@ -52,6 +52,7 @@ __device__ __forceinline__ uint32_t pf_word(const u32x4& v, int i) { return v[i]
 __device__ __forceinline__ uint32_t pf_word(const uint2& v, int i) { return i == 0 ? v.x : v.y; }
 
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 // fp32 x -> (hi, lo) fp16 with hi + lo = x to ~2^-22 relative
 __device__ __forceinline__ void pf_split(float x, _Float16& hi, _Float16& lo) {
@@ -64,7 +65,10 @@ __device__ __forceinline__ void pf_split(float x, _Float16& hi, _Float16& lo) {
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void pf_split2(float x, float y, f16x8& hi, f16x8& lo, int i) {
   const f16x2 h = __builtin_convertvector((f32x2){x, y}, f16x2);
-  const f16x2 l = __builtin_convertvector((f32x2){__builtin_fmaf((float)h[0], -1.0f, x), __builtin_fmaf((float)h[1], -1.0f, y)}, f16x2);
+  float lx, ly;   // x - h (exact), one instruction each
+  asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(lx) : "v"(h), "v"(x));
+  asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(ly) : "v"(h), "v"(y));
+  const f16x2 l = __builtin_convertvector((f32x2){lx, ly}, f16x2);
   hi[i] = h[0];
   hi[i + 1] = h[1];
   lo[i] = l[0];
@@ -320,12 +324,13 @@ __global__ __launch_bounds__(64, WPE) void attn_prefill_kernel(const float* __re
 // every workgroup holds long and short chains -- and copies each K / V block of their union once
 // into an LDS ring (LDS-DMA, full 128-byte lines), which all its waves read.
 // The per-wave math is the kernel above's: S^T = K Q^T on fp16 MFMA with the fp32 operand in hi + lo,
-// online softmax per column (here in powers of 2), two blocks per step, and O^T += V^T P^T as one 32-key 16x16x32 product.
+// online softmax per column (here in powers of 2), NB blocks per step, and O^T += V^T P^T as 32-key 16x16x32 products.
 //   K block in LDS: [16 keys][16 chunks of 16 B], the logical chunk c of key row r at physical c ^ r
 //   (an A-fragment read, lane (r, g) chunk 4c + g, is conflict-free in every ds_read_b128 lane group);
 //   head_dim 64: 8 chunks a row, chunk c at c ^ (r >> 1) (a lane group's 16 rows hit each 16 bytes of 256 once);
-//   V block: [16 keys][16 chunks], unswizzled (lane (r, g) reads chunk r of rows 4g + j).
-// Per iteration of BI blocks (2 per part): wait for this wave's DMAs of the iteration; barrier
+//   V block: [16 keys][HD / 16 times 32 bytes], bytes t of key row r at t ^ (r & 7) (head_dim 64: ^ (r >> 1 & 3)): ds_read_b64_tr_b16
+//   gives lane (r, g) keys 4g .. of dim 16 t + r from 32 bytes of four rows, each 32 bytes of the banks hit twice.
+// Per iteration of BI blocks (NB per part): wait for this wave's DMAs of the iteration; barrier
 // (everyone's landed, and everyone is done with the previous iteration's blocks); DMA the iteration
 // R / BI - 1 ahead into the slots just freed; compute.  Waves past their own chain keep copying until
 // the workgroup's longest is done; the last DMAs drain before the ring's LDS is reused or released.
@@ -347,15 +352,21 @@ __global__ __launch_bounds__(64, WPE) void attn_prefill_kernel(const float* __re
 // 4 (one SIMD) take a long and a short chain (1000 rows of 32 heads on 4, head_dim 64: 26.5 -> 23.6 us with two parts of the
 // same chain before), packed conversions and one fma a score in the softmax (-> 22.2).  Few workgroups: 2 query
 // blocks in 4 parts (918 rows of 8 heads on 2, head_dim 128: 19.4 -> 15.3; 476 rows behind 1024 keys 29 -> 20).
-template <int HD, int QB, int HALVES, int R>
+// The vector unit is issuing half of the time (head_dim 64, 1000 rows of 32 heads on 4), the rest are those latencies.  So: a step's
+// keys all in flight, its blocks' products in turn; four blocks a step (two where there are 4 parts: 64 rows 6.3 against
+// 6.1 us); values transposed by their LDS reads instead of a v_perm per fragment word; a kv-head's workgroups on one XCD,
+// whose L2 its keys reach once (512 rows of 32 heads, head_dim 128: the copies alone 13.0 -> 7.4 us).  Together, us: head_dim
+// 64, 32 heads on 4, 1000 rows 20.8 -> 16.7, 333 behind 600 keys 14.0 -> 11.9, 256 5.4 -> 5.4; head_dim 128, 32 on 32, 512 rows 15.0 -> 12.2,
+// 1024 38.2 -> 34.3, 256 8.8 -> 7.9; 32 on 8, 400 behind 500 19.9 -> 18.3.
+template <int HD, int QB, int HALVES, int R, int NB>
 __global__ __launch_bounds__(64 * QB * HALVES, HD == 64 ? 4 : 1) void attn_prefill_wg_kernel(const float* __restrict__ q, const uint16_t* __restrict__ kc,
                                                                  const uint16_t* __restrict__ vc, int max_seq,
                                                                  const int32_t* __restrict__ pos, int M, int heads, int gsh,
-                                                                 float scale, uint16_t* __restrict__ out) {
-  constexpr int DV = HD / 16, KW = HD / 32, NB = 2, BI = NB * HALVES;   // BI: blocks per iteration
+                                                                 float scale, uint16_t* __restrict__ out, int QG, int spread) {
+  constexpr int DV = HD / 16, KW = HD / 32, BI = NB * HALVES;   // BI: blocks per iteration
   constexpr int ND = HD / 32, RPD = 16 / ND;   // DMAs of a K or V block, key rows each copies
-  using VRaw = typename PfRaw<HD>::V;
   auto swz = [](int row) { return HD == 128 ? row : (row >> 1) & 7; };   // chunk c of key row `row` at c ^ swz(row)
+  auto vsw = [](int row) { return HD == 128 ? row & 7 : (row >> 1) & 3; };   // of its values, 32 bytes t at t ^ vsw(row)
   static_assert(R % BI == 0 && R >= 2 * BI, "ring: whole iterations, one in flight beside the one computed");
   // K and V rings in ONE array: the halves' merge at the end reuses it as scratch (4 query blocks x
   // 64 lanes x (4 DV + 2) floats), which is larger than the K ring alone
@@ -369,8 +380,11 @@ __global__ __launch_bounds__(64 * QB * HALVES, HD == 64 ? 4 : 1) void attn_prefi
   // (a SIMD holds waves w and w + 4: one of a long and one of a short chain)
   const int part = wave / QB, qw = wave < 4 ? wave % QB : QB - 1 - wave % QB;
   const int G = 1 << gsh, qpw = 16 >> gsh;
-  const int kvh = blockIdx.y, QG = gridDim.x, nq = (M + qpw - 1) / qpw;
-  const int qb = (QG - 1 - blockIdx.x) + qw * QG;   // longest chains first
+  // (consecutive workgroups go to the 8 XCDs in turn: those of a kv-head to one, or to 2^spread)
+  const int x = blockIdx.x, at = ((int)blockIdx.y << spread) + (x & ((1 << spread) - 1)), kvh = (x >> spread) + 8 * (int)blockIdx.z;
+  const int nq = (M + qpw - 1) / qpw;
+  if (at >= QG || kvh * G >= heads) return;
+  const int qb = (QG - 1 - at) + qw * QG;   // longest chains first
   const bool live = qb < nq;                        // (a wave past the chunk only copies)
   const int q0 = qb * qpw, qi = min(q0 + (r >> gsh), M - 1), h = kvh * G + (r & (G - 1));
   const int p = pos[qi];
@@ -408,7 +422,7 @@ __global__ __launch_bounds__(64 * QB * HALVES, HD == 64 ? 4 : 1) void attn_prefi
   const uint32_t sk_lds = (uint32_t)(uintptr_t)&sk[0][0], sv_lds = (uint32_t)(uintptr_t)&sv[0][0];
   // An iteration's BI blocks are 2 BI copies (K or V of a block) of ND DMA instructions of 1 KiB (RPD rows each); wave w
   // makes copies w U ...
-  constexpr int U = 4 / QB;
+  constexpr int U = 2 * BI / (QB * HALVES);
   const int dch = lane & (HD / 8 - 1);
   auto issue = [&](int kb0) {   // the iteration starting at block kb0
 #if TI_PF_DIAG & 8   // diagnostic: no copies past the prologue (the math on stale blocks)
@@ -421,8 +435,8 @@ __global__ __launch_bounds__(64 * QB * HALVES, HD == 64 ? 4 : 1) void attn_prefi
 #pragma unroll
       for (int i = 0; i < ND; ++i) {
         const int row = RPD * i + lane / (HD / 8), key = min(kb * 16 + row, kl);
-        const uint16_t* src = dv ? vbase + (size_t)key * HD + dch * 8 : kbase + (size_t)key * HD + ((dch ^ swz(row)) * 8);
-        dma_1k_asm(src, __builtin_amdgcn_readfirstlane(base + (uint32_t)(i * 1024)));
+        const uint32_t off = (uint32_t)key * (HD * 2) + (uint32_t)(dch ^ (dv ? vsw(row) * 2 : swz(row))) * 16;
+        dma_1k_asm(dv ? vbase : kbase, off, base + (uint32_t)(i * 1024));
       }
     }
   };
@@ -433,6 +447,7 @@ __global__ __launch_bounds__(64 * QB * HALVES, HD == 64 ? 4 : 1) void attn_prefi
 #pragma unroll
   for (int t = 0; t < DV; ++t) acc[t] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
   float m_run = -INFINITY, l_run = 0.0f;
+  const int v_at = (4 * g + (r >> 2)) * HD + vsw(4 * g + (r >> 2)) * 16 + (r & 3) * 4;   // (a transposed read: four lanes a key's 16 dims)
   constexpr float kLog2e = 1.44269504088896341f, kPfSlack = 8.0f * kLog2e;   // as above: O rescaled only when a column max moves by > 8
   for (int kbi = 0; kbi < nkb; kbi += BI) {
     // this wave's U ND DMAs of iteration kbi are the oldest of the U ND (R / BI - 1) in flight
@@ -448,33 +463,29 @@ __global__ __launch_bounds__(64 * QB * HALVES, HD == 64 ? 4 : 1) void attn_prefi
     const bool act = kb < nkb_w;      // wave-uniform
 #endif
     f32x4 sacc[NB];
-    VRaw vraw[NB][4];
+    f16x4 vf[NB][DV];   // values of keys 4 g .. of a block, dim 16 t + r
     if (act) {
+      // all of the step's keys in flight together, then the blocks' products in turn (NB independent chains), then the values
+      f16x8 kf[NB][KW];
 #pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        const uint16_t* kr = &sk[(kb + b) % R][r * HD];
-#if TI_PF_QK_SPLIT   // the hi and lo products in two chains (four independent per step), summed after
-        f32x4 sh = (f32x4){0.0f, 0.0f, 0.0f, 0.0f}, sl = sh;
+      for (int c = 0; c < KW; ++c)
 #pragma unroll
-        for (int c = 0; c < KW; ++c) {
-          const f16x8 kf = __builtin_bit_cast(f16x8, *(const u32x4*)(kr + (((4 * c + g) ^ swz(r)) * 8)));
-          sh = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qh[c], sh, 0, 0, 0);
-          sl = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, ql[c], sl, 0, 0, 0);
-        }
-        sacc[b] = sh + sl;
-#else
-        sacc[b] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+        for (int b = 0; b < NB; ++b) kf[b][c] = __builtin_bit_cast(f16x8, *(const u32x4*)(&sk[kb % R + b][r * HD] + (((4 * c + g) ^ swz(r)) * 8)));
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int c = 0; c < KW; ++c) {
-          const f16x8 kf = __builtin_bit_cast(f16x8, *(const u32x4*)(kr + (((4 * c + g) ^ swz(r)) * 8)));
-          sacc[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qh[c], sacc[b], 0, 0, 0);
-          sacc[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, ql[c], sacc[b], 0, 0, 0);
-        }
-#endif
-        const uint16_t* vb = &sv[(kb + b) % R][0];
+      for (int c = 0; c < KW; ++c) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) vraw[b][j] = *(const VRaw*)(vb + (4 * g + j) * HD + r * DV);
+        for (int b = 0; b < NB; ++b) sacc[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[b][c], qh[c], c ? sacc[b] : (f32x4){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) sacc[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[b][c], ql[c], sacc[b], 0, 0, 0);
       }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < DV; ++t)
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+          vf[b][t] = __builtin_bit_cast(f16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(
+              &sv[kb % R + b][0] + (v_at ^ (16 * t)))));
     }
 #if TI_PF_WG_LATE_DMA   // the next DMAs issued under this step's S = K Q^T rather than before it
     issue(kbi + R - BI);
@@ -527,23 +538,19 @@ __global__ __launch_bounds__(64 * QB * HALVES, HD == 64 ? 4 : 1) void attn_prefi
       // O^T += V^T P^T over both blocks in one 32-key product (16x16x32, the full-rate form): k index
       // 8 g + e is key 4 g + e of the first block for e < 4 and of the second for e >= 4, in the
       // A fragment (V, lane (dim r DV + t, k)) and the B fragment (P, lane (column r, k)) alike
-      f16x8 ph, pl;
 #pragma unroll
-      for (int b = 0; b < NB; ++b)
+      for (int u = 0; u < NB; u += 2) {
+        f16x8 ph, pl;
 #pragma unroll
-        for (int e = 0; e < 4; e += 2) pf_split2(pv[b][e], pv[b][e + 1], ph, pl, 4 * b + e);
+        for (int b = 0; b < 2; ++b)
 #pragma unroll
-      for (int t = 0; t < DV; ++t) {
-        const uint32_t sel = (t & 1) ? 0x07060302u : 0x05040100u;
-        uint32_t w[4];
+          for (int e = 0; e < 4; e += 2) pf_split2(pv[u + b][e], pv[u + b][e + 1], ph, pl, 4 * b + e);
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-          w[2 * b] = __builtin_amdgcn_perm(pf_word(vraw[b][1], t >> 1), pf_word(vraw[b][0], t >> 1), sel);
-          w[2 * b + 1] = __builtin_amdgcn_perm(pf_word(vraw[b][3], t >> 1), pf_word(vraw[b][2], t >> 1), sel);
+        for (int t = 0; t < DV; ++t) {
+          const f16x8 bf = __builtin_shufflevector(vf[u][t], vf[u + 1][t], 0, 1, 2, 3, 4, 5, 6, 7);
+          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf, ph, acc[t], 0, 0, 0);
+          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf, pl, acc[t], 0, 0, 0);
         }
-        const f16x8 bf = __builtin_bit_cast(f16x8, (u32x4){w[0], w[1], w[2], w[3]});
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf, ph, acc[t], 0, 0, 0);
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf, pl, acc[t], 0, 0, 0);
       }
     }
   }
@@ -583,18 +590,17 @@ __global__ __launch_bounds__(64 * QB * HALVES, HD == 64 ? 4 : 1) void attn_prefi
   const float inv = 1.0f / lt;
   const int row = q0 + (r >> gsh), hh = kvh * G + (r & (G - 1));
   if (row < M) {
-    uint16_t* dst = out + ((size_t)row * heads + hh) * HD + 4 * g * DV;
+    uint16_t* dst = out + ((size_t)row * heads + hh) * HD + 4 * g;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      uint32_t o[DV / 2];
+    for (int t = 0; t < DV; ++t) {
+      uint32_t o[2];
 #pragma unroll
-      for (int t = 0; t < DV / 2; ++t) {
-        const uint16_t lo = __builtin_bit_cast(uint16_t, ti::mul_f16(acc[2 * t][i], inv));
-        const uint16_t hi = __builtin_bit_cast(uint16_t, ti::mul_f16(acc[2 * t + 1][i], inv));
-        o[t] = lo | ((uint32_t)hi << 16);
+      for (int i = 0; i < 2; ++i) {
+        const uint16_t lo = __builtin_bit_cast(uint16_t, ti::mul_f16(acc[t][2 * i], inv));
+        const uint16_t hi = __builtin_bit_cast(uint16_t, ti::mul_f16(acc[t][2 * i + 1], inv));
+        o[i] = lo | ((uint32_t)hi << 16);
       }
-      if constexpr (HD == 128) *(ti::u32x4*)(dst + i * DV) = (ti::u32x4){o[0], o[1], o[2], o[3]};
-      else *(uint2*)(dst + i * DV) = make_uint2(o[0], o[1]);
+      *(uint2*)(dst + 16 * t) = make_uint2(o[0], o[1]);
     }
   }
 }
@@ -657,13 +663,16 @@ extern "C" int ti_attn_prefill_keys(const float* q, const uint16_t* k_cache, con
   // 5.1, 256 7.5 / 6.8 / 5.9, 330 9.8 / 8.0 / 9.1, 64 rows behind 300 keys 9.0 / 8.1 / 6.5.
   const int cus = ns > 0 ? ns / 4 : 256;
   const bool two = wg2 && (long)((grid.x + 1) / 2) * kv_heads <= cus;
-  const dim3 gw(two ? (grid.x + 1) / 2 : (grid.x + 3) / 4, kv_heads);
+  const int qg = two ? (grid.x + 1) / 2 : (grid.x + 3) / 4;   // workgroups of a kv-head
   if (wg && (forced > 1 || std::max(keys, M) > 128)) {
-    auto* fn = head_dim == 128 ? (!wg2 ? ti::attn_prefill_wg_kernel<128, 4, 1, TI_PF_WG_RING>
-                                  : two ? ti::attn_prefill_wg_kernel<128, 2, 4, 2 * TI_PF_WG_RING2> : ti::attn_prefill_wg_kernel<128, 4, 2, TI_PF_WG_RING2>)
-                               : (!wg2 ? ti::attn_prefill_wg_kernel<64, 4, 1, TI_PF_WG_RING>
-                                  : two ? ti::attn_prefill_wg_kernel<64, 2, 4, 2 * TI_PF_WG_RING2> : ti::attn_prefill_wg_kernel<64, 4, 2, TI_PF_WG_RING2>);
-    hipLaunchKernelGGL(fn, gw, dim3(wg2 ? 512 : 256), 0, s, q, k_cache, v_cache, max_seq, pos, M, heads, gsh, scale, out);
+    auto* fn = head_dim == 128 ? (!wg2 ? ti::attn_prefill_wg_kernel<128, 4, 1, TI_PF_WG_RING, 2>
+                                  : two ? ti::attn_prefill_wg_kernel<128, 2, 4, 2 * TI_PF_WG_RING2, 2> : ti::attn_prefill_wg_kernel<128, 4, 2, 2 * TI_PF_WG_RING2, 4>)
+                               : (!wg2 ? ti::attn_prefill_wg_kernel<64, 4, 1, TI_PF_WG_RING, 2>
+                                  : two ? ti::attn_prefill_wg_kernel<64, 2, 4, 2 * TI_PF_WG_RING2, 2> : ti::attn_prefill_wg_kernel<64, 4, 2, 2 * TI_PF_WG_RING2, 4>);
+    // an XCD's workgroups: those of kv-heads x, x + 8, .., or a share of one of up to 4
+    const int spread = kv_heads > 4 ? 0 : kv_heads > 2 ? 1 : 4 - kv_heads;   // (log2; three: 8 / 4)
+    hipLaunchKernelGGL(fn, dim3(8, (qg + (1 << spread) - 1) >> spread, (kv_heads + 7) / 8), dim3(wg2 ? 512 : 256), 0, s, q, k_cache, v_cache,
+                       max_seq, pos, M, heads, gsh, scale, out, qg, spread);
   } else if (head_dim == 128) {
     if (deep)
       hipLaunchKernelGGL((ti::attn_prefill_kernel<128, TI_PF_RING_DEEP>), grid, dim3(64), 0, s, q, k_cache, v_cache,
