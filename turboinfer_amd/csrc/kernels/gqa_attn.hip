@@ -6,12 +6,13 @@
 //   * gqa_decode_kernel: the query heads that share a key/value head are the MFMA columns; a workgroup
 //     takes 64-position blocks, its waves split the positions for the scores and the value dimensions for
 //     the sums; keys are split over workgroups, merged by gqa_merge_kernel.
-//   * gqa_prefill_kernel: prompt chunks; a workgroup owns MQ tiles of 16 rows of one key/value head's query
+//   * gqa_block_kernel: prompt chunks of 16-bit heads of 64 or 128 dims, blocks of keys and values in LDS for eight waves;
+//   * gqa_prefill_kernel: other prompt chunks; a workgroup owns MQ tiles of 16 rows of one key/value head's query
 //     heads (heads of the same rows first), its waves split the key blocks.
 // Scores, softmax and sums are fp32; the denominator holds exp(sink) of the head once.
 #include <algorithm>
 
-#include "elem.hpp"
+#include "block_attn.hpp"
 
 namespace ti {
 
@@ -480,6 +481,72 @@ __global__ __launch_bounds__(256, NV * MQ > 16 ? 1 : 2) void gqa_prefill_kernel(
   }
 }
 
+// The same on keys and values that a workgroup's waves share (block_attn.hpp): 16-bit heads of 32 DKT dims, keys and values.  Row blocks
+// are MQ tiles as above.  us, the kernel above -> 16 / 32 rows a wave: 16 heads on 4 of 128 dims, 2048 rows 65 -> 61 / 48.7, 1500 47.0 ->
+// 44.9 / 38.4, 1000 27.9 -> 21.2 / 28.6, 500 13.4 -> 12.7, 200 10.4 -> 9.4, 40 10.5 -> 8.9; 8 on 2, 2048 rows 43.7 -> 33.2 / 43.3, 1000 20.5 -> 18.9, 500
+// 13.2 -> 13.4, 300 14.3 -> 12.2, 200 10.1 -> 10.8, 40 9.3 -> 8.8.
+template <int MQ, int DKT>
+__global__ __launch_bounds__(512, 2) void gqa_block_kernel(const ti_gqa_attn_args a, int QG, int spread) {
+  constexpr int NV = 2 * DKT, NF = 4 * DKT + 2 * NV;
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 15, g = lane >> 4;
+  // (consecutive workgroups go to the 8 XCDs in turn: those of a key/value head to one, or to 2^spread)
+  const int x = blockIdx.x, j = ((int)blockIdx.y << spread) + (x & ((1 << spread) - 1)), kvh = (x >> spread) + 8 * (int)blockIdx.z;
+  if (j >= QG || kvh >= a.kv_heads) return;
+  const int rep = a.heads / a.kv_heads, tiles = (a.M + 15) / 16 * rep, t0 = block_of(block_group(wave), j, QG) * MQ;
+  const bool live = t0 < tiles;
+  auto row = [&](int t) { return min(t, tiles - 1) / rep * 16; };   // a tile's first row
+  int top = 0;   // the workgroup's last tile
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    if (block_of(q, j, QG) * MQ < tiles) top = max(top, min(block_of(q, j, QG) * MQ + MQ, tiles) - 1);
+  int first[MQ], head[MQ];
+#pragma unroll
+  for (int q = 0; q < MQ; ++q) {
+    first[q] = row(t0 + q);
+    head[q] = kvh * rep + min(t0 + q, tiles - 1) % rep;
+  }
+  const char* cache = (const char*)a.cache + (size_t)kvh * (a.seq_p >> 6) * NF * 1024;
+  block_attention<MQ, DKT, NV>(
+      lds, a.scale * kBlockLog2e, live, a.pos0 + first[0], live ? a.pos0 + min(first[MQ - 1] + 16, a.M) - 1 : -1,
+      (a.pos0 + min(row(top) + 16, a.M) - 1) >> 6,
+      [&](int kt, int q) { return *(const bf16x8*)((const bf16*)a.q + ((size_t)min(first[q] + col, a.M - 1) * a.heads + head[q]) * (32 * DKT) + kt * 32 + g * 8); },
+      [](int t, int kt) { return t * DKT + kt; }, [&](int e, int blk, uint32_t&) -> const void* { return cache + ((size_t)blk * NF + e) * 1024; },
+      [&](int q) { return a.pos0 + first[q] + col; },
+      [&](int q, bool& counts) {
+        counts = a.sink != nullptr;
+        return a.sink ? a.sink[head[q]] * kBlockLog2e : -1e30f;
+      },
+      [&](int q, const f32x4 (&o)[NV], float l) {
+        const int m = first[q] + col;
+        if (m >= a.M || t0 + q >= tiles) return;
+        const float inv = 1.0f / l;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+          const int c = head[q] * a.vdim + v * 16 + 4 * g;
+          f32x4 y = o[v] * inv;
+          if (a.gate) {
+            const f32x4 gt = *(const f32x4*)(a.gate + (size_t)m * a.ldg + c);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) y[r] *= fast_sigmoid(gt[r]);
+          }
+          *(bf16x4*)((bf16*)a.out + (size_t)m * a.ldo + c) = quad<bf16>(y);
+        }
+      });
+}
+
+template <int MQ, int DKT>
+int launch_gqa_block(const ti_gqa_attn_args& a, hipStream_t s) {
+  constexpr int kLds = block_lds<DKT, 2 * DKT>();
+  const int tiles = (a.M + 15) / 16 * (a.heads / a.kv_heads), QG = ((tiles + MQ - 1) / MQ + 3) / 4;
+  const int spread = a.kv_heads > 4 ? 0 : a.kv_heads > 2 ? 1 : 4 - a.kv_heads;   // (log2; three: 8 / 4)
+  auto* fn = gqa_block_kernel<MQ, DKT>;
+  TI_HIP_CHECK(hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, kLds), "hipFuncSetAttribute(gqa_block_kernel)");
+  hipLaunchKernelGGL(fn, dim3(8, (QG + (1 << spread) - 1) >> spread, (a.kv_heads + 7) / 8), dim3(512), kLds, s, a, QG, spread);
+  TI_LAUNCH_CHECK("gqa_block_kernel");
+  return TI_OK;
+}
+
 template <class T>
 int launch_gqa_decode(const ti_gqa_attn_args& a, hipStream_t s) {
   const int nkt = gqa_dim_p<T>(a.dim) / El<T>::KT, nvw = (gqa_vdim_p(a.vdim) / 16 + 3) / 4, rep = a.heads / a.kv_heads;
@@ -498,6 +565,16 @@ int launch_gqa_decode(const ti_gqa_attn_args& a, hipStream_t s) {
 
 template <class T>
 int launch_gqa_prefill(const ti_gqa_attn_args& a, hipStream_t s) {
+  if constexpr (sizeof(T) == 2) {
+    const bool sized = a.dim == a.vdim && (a.dim == 64 || a.dim == 128) && a.ldo % 4 == 0 && (!a.gate || a.ldg % 4 == 0) &&
+                       (((uintptr_t)a.gate & 15) | ((uintptr_t)a.out & 7)) == 0 && a.scale > 0.0f;
+    // 16 rows a wave while such workgroups are on the CUs together (dims of 128: one a CU, of 64: two), else 32
+    if (sized) {
+      const bool wide = ((long)(a.M + 15) / 16 * (a.heads / a.kv_heads) + 3) / 4 * a.kv_heads > (a.dim == 128 ? 256 : 512);
+      if (a.dim == 128) return wide ? launch_gqa_block<2, 4>(a, s) : launch_gqa_block<1, 4>(a, s);
+      return wide ? launch_gqa_block<2, 2>(a, s) : launch_gqa_block<1, 2>(a, s);
+    }
+  }
   const int nkt = gqa_dim_p<T>(a.dim) / El<T>::KT, nv = gqa_vdim_p(a.vdim) / 16, rep = a.heads / a.kv_heads;
   const long tiles = (long)((a.M + 15) / 16) * rep;
   // two tiles per workgroup where they still give every CU two workgroups

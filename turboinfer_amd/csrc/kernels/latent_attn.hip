@@ -14,7 +14,7 @@
 // Scores, softmax and sums are fp32; the softmax denominator holds exp(sink) of the head once.
 #include <algorithm>
 
-#include "elem.hpp"
+#include "block_attn.hpp"
 
 namespace ti {
 
@@ -505,178 +505,52 @@ __global__ __launch_bounds__(256, NV > 8 ? 2 : 3) void latent_prefill_kernel(con
   }
 }
 
-// The same on keys and values that a workgroup's waves share: 16-bit heads of 32 DKT dims (keys without their rotated part, and
-// values) and 32 RKT rotated ones.  In the kernel above every wave streams its own 64-key blocks from L2, 40 KiB (dims 128 + 64) per
-// 2560 cycles of products of 32 rows: all that a CU can load.  Here eight waves hold four blocks of 16 MQ rows in two parts of
-// the keys; 128 keys at a time are copied to LDS once for all of them, the next 128 while these are multiplied.  What bounds it now:
-// LDS (MQ 2: 64 bytes a cycle of operand reads) beside the products and the softmax's chain.  us, per-wave streams -> 16 / 32 rows
-// a wave: 16 heads of 128 + 64, 2048 rows 73.5 -> 72 / 53.3, 1400 48.8 -> 47.0 / 38.0, 1024 37.0 -> 23.3 / 29.7, 500 19.1 -> 14.2, 150 10.7 -> 9.3, 32
-// 10.2 -> 7.0, 64 behind 1000 34.6 -> 27.1; 8 heads of 64 + 32, 2048 rows 35.0 -> 25.3 / 33.5, 300 10.8 -> 7.6.
+// The same on keys and values that a workgroup's waves share (block_attn.hpp): 16-bit heads of 32 DKT dims (keys without their
+// rotated part, and values) and 32 RKT rotated ones.  us, per-wave streams -> 16 / 32 rows a wave: 16 heads of 128 + 64, 2048 rows 73.5
+// -> 72 / 53.3, 1400 48.8 -> 47.0 / 38.0, 1024 37.0 -> 23.3 / 29.7, 500 19.1 -> 14.2, 150 10.7 -> 9.3, 32 10.2 -> 7.0, 64 behind 1000 34.6 ->
+// 27.1; 8 heads of 64 + 32, 2048 rows 35.0 -> 25.3 / 33.5, 300 10.8 -> 7.6.
 template <int MQ, int DKT, int RKT>
 __global__ __launch_bounds__(512, 2) void latent_block_kernel(const ti_latent_prefill_args a, int QG) {
-  typedef bf16x8 V;
-  constexpr int NV = 2 * DKT, NKT = DKT + RKT, NF = 4 * NKT + 2 * NV, NC = (2 * NF) / 8;   // 1-KiB fragments of 64 keys; copies of a wave
-  constexpr float kLog2e = 1.44269504088896341f, kSlack = 8.0f * kLog2e;
-  extern __shared__ __attribute__((aligned(1024))) char lds[];   // 2 iterations of 2 blocks of 64 keys
+  constexpr int NV = 2 * DKT, NKT = DKT + RKT;
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 15, g = lane >> 4;
-  const int h = (int)(blockIdx.x + 8 * blockIdx.z), j = blockIdx.y;
+  const int h = (int)(blockIdx.x + 8 * blockIdx.z), j = blockIdx.y;   // (an XCD's workgroups: heads x, x + 8, ..)
   if (h >= a.heads) return;
-  // row blocks j, 2 QG - 1 - j, 2 QG + j, 4 QG - 1 - j: as many keys in every workgroup, and in every SIMD, whose waves w and w + 4
-  // are a part of one block and of its mirror
-  const int part = wave >> 2, qw = part ? 3 - (wave & 3) : wave, rb = (qw + 1) / 2 * 2 * QG + (qw & 1 ? -1 - j : j);
-  const int row0 = rb * 16 * MQ, blocks = (a.M + 16 * MQ - 1) / (16 * MQ);
-  const bool live = rb < blocks;
-  int top = 0;   // the workgroup's last row block
+  const int row0 = block_of(block_group(wave), j, QG) * 16 * MQ, cw = a.lat_p + a.rot_p, nkb = a.key_blocks >> 1;
+  const bool live = row0 < a.M;
+  int top = 0;   // the workgroup's last row
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int b = (q + 1) / 2 * 2 * QG + (q & 1 ? -1 - j : j);
-    if (b < blocks) top = max(top, b);
-  }
-  const int last_wg = a.pos0 + min((top + 1) * 16 * MQ, a.M) - 1, last = live ? a.pos0 + min(row0 + 16 * MQ, a.M) - 1 : -1;
-  const int end = last_wg >> 6, iters = (end >> 1) + 1, cw = a.lat_p + a.rot_p, nkb = a.key_blocks >> 1;
-  V qf[NKT][MQ];
-#pragma unroll
-  for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-    for (int q = 0; q < MQ; ++q) {
-      const int m = min(row0 + q * 16 + col, a.M - 1);
-      qf[kt][q] = *(const V*)((const bf16*)a.q + ((size_t)m * a.heads + h) * (32 * NKT) + kt * 32 + g * 8);
-    }
+  for (int q = 0; q < 4; ++q)
+    if (block_of(q, j, QG) * 16 * MQ < a.M) top = max(top, min((block_of(q, j, QG) + 1) * 16 * MQ, a.M) - 1);
   const char* kb = (const char*)a.kfrag + (size_t)h * a.key_blocks * DKT * 1024;
   const char* vb = (const char*)a.vfrag + (size_t)h * NV * nkb * 1024;
   const char* rp = (const char*)a.cache + (size_t)a.lat_p * 2;
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
-  auto issue = [&](int it) {   // an iteration's two blocks (past the last key: the last block again)
+  block_attention<MQ, NKT, NV>(
+      lds, a.scale * kBlockLog2e, live, a.pos0 + row0, live ? a.pos0 + min(row0 + 16 * MQ, a.M) - 1 : -1, (a.pos0 + top) >> 6,
+      [&](int kt, int q) {
+        const int m = min(row0 + q * 16 + col, a.M - 1);
+        return *(const bf16x8*)((const bf16*)a.q + ((size_t)m * a.heads + h) * (32 * NKT) + kt * 32 + g * 8);
+      },
+      [](int t, int kt) { return kt < DKT ? t * DKT + kt : 4 * DKT + t * RKT + kt - DKT; },
+      [&](int e, int blk, uint32_t& off) -> const void* {
+        if (e < 4 * DKT) return kb + ((size_t)blk * 4 * DKT + e) * 1024;
+        if (e >= 4 * NKT) return vb + ((size_t)((e - 4 * NKT) >> 1) * nkb + blk * 2 + (e & 1)) * 1024;
+        off = (uint32_t)col * (uint32_t)cw * 2 + (uint32_t)g * 16;   // (the rotated part: from the cache's rows)
+        return rp + (size_t)(blk * 64 + (e - 4 * DKT) / RKT * 16) * cw * 2 + (e - 4 * DKT) % RKT * 64;
+      },
+      [&](int q) { return a.pos0 + row0 + q * 16 + col; },
+      [&](int, bool& counts) {
+        counts = true;
+        return a.sink[h] * kBlockLog2e;
+      },
+      [&](int q, const f32x4 (&o)[NV], float l) {
+        const int m = row0 + q * 16 + col;
+        if (m >= a.M) return;
+        const float sc = a.gate[(size_t)m * a.heads + h] / l;
+        bf16* out = (bf16*)a.out + (size_t)m * a.ldo + (size_t)h * a.vdim + 4 * g;
 #pragma unroll
-    for (int i = 0; i < NC; ++i) {
-      const int f = i * 8 + wave, b = f >= NF, e = b ? f - NF : f, k0 = min(2 * it + b, end);   // (64-key block)
-      const uint32_t to = lds0 + (uint32_t)((it & 1) * 2 * NF + f) * 1024;
-      const void* src;
-      uint32_t off = (uint32_t)lane * 16;
-      if (e < 4 * DKT) src = kb + ((size_t)k0 * 4 * DKT + e) * 1024;
-      else if (e < 4 * NKT) {
-        const int t = (e - 4 * DKT) / RKT, kt = (e - 4 * DKT) % RKT;
-        src = rp + (size_t)(k0 * 64 + t * 16) * cw * 2 + kt * 64;
-        off = (uint32_t)col * (uint32_t)cw * 2 + (uint32_t)g * 16;
-      } else src = vb + ((size_t)((e - 4 * NKT) >> 1) * nkb + k0 * 2 + (e & 1)) * 1024;
-      dma_1k_asm(src, off, to);
-    }
-  };
-  f32x4 o[MQ][NV];
-  float mr[MQ], lr[MQ];   // relative to 2^mr
-#pragma unroll
-  for (int q = 0; q < MQ; ++q) {
-    mr[q] = a.sink[h] * kLog2e;   // the sink: weight exp(sink - max), no value; counted by one part
-    lr[q] = part == 0 && g == 0 ? 1.0f : 0.0f;
-#pragma unroll
-    for (int v = 0; v < NV; ++v) o[q][v] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  }
-  const float scale = a.scale * kLog2e;
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (only copies are counted below)
-  issue(0);
-  for (int it = 0; it < iters; ++it) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    lds_sync();   // everyone's copies are here, and everyone has done with the other half
-    if (it + 1 < iters) issue(it + 1);
-    const int k0 = (2 * it + part) * 64;
-    if (k0 > last) continue;
-    const V* st = (const V*)lds + ((it & 1) * 2 + part) * NF * 64 + lane;
-    f32x4 s[MQ][4];
-#pragma unroll
-    for (int q = 0; q < MQ; ++q)
-#pragma unroll
-      for (int t = 0; t < 4; ++t) s[q][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int kt = 0; kt < NKT; ++kt) {
-      V k[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) k[t] = st[(kt < DKT ? t * DKT + kt : 4 * DKT + t * RKT + kt - DKT) * 64];
-#pragma unroll
-      for (int q = 0; q < MQ; ++q)
-#pragma unroll
-        for (int t = 0; t < 4; ++t) s[q][t] = mma(k[t], qf[kt][q], s[q][t]);
-    }
-    const bool ragged = k0 + 63 > a.pos0 + row0;   // (uniform: a row of these does not see all of the block)
-#pragma unroll
-    for (int q = 0; q < MQ; ++q) {
-      float mx = -INFINITY;
-      const int p = a.pos0 + row0 + q * 16 + col - k0 - 4 * g;
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          if (ragged) s[q][t][r] = t * 16 + r <= p ? s[q][t][r] : -INFINITY;
-          mx = fmaxf(mx, s[q][t][r]);
-        }
-      mx = fmaxf(xor32_max(xor16_max(mx)) * scale, mr[q]);
-      if (__builtin_amdgcn_ballot_w64(mx > mr[q] + kSlack) != 0) {   // sums are moved to a new maximum only when it is far
-        const float alpha = __builtin_amdgcn_exp2f(mr[q] - mx);
-        mr[q] = mx;
-        lr[q] *= alpha;
-#pragma unroll
-        for (int v = 0; v < NV; ++v) o[q][v] *= alpha;
-      }
-      float l = 0.0f;
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          s[q][t][r] = __builtin_amdgcn_exp2f(fmaf(s[q][t][r], scale, -mr[q]));
-          l += s[q][t][r];
-        }
-      lr[q] += l;
-    }
-    bf16x8 pf[MQ][2];
-#pragma unroll
-    for (int q = 0; q < MQ; ++q)
-#pragma unroll
-      for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          pf[q][b][r] = (bf16)s[q][2 * b][r];
-          pf[q][b][4 + r] = (bf16)s[q][2 * b + 1][r];
-        }
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-      V vv[2];
-#pragma unroll
-      for (int b = 0; b < 2; ++b) vv[b] = st[(4 * NKT + v * 2 + b) * 64];
-#pragma unroll
-      for (int q = 0; q < MQ; ++q)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) o[q][v] = mma(vv[b], pf[q][b], o[q][v]);
-    }
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  lds_sync();   // part 1 hands its sums to part 0 where the keys were
-  float* x = (float*)lds + (size_t)qw * MQ * (4 * NV + 2) * 64;
-  if (part) {
-#pragma unroll
-    for (int q = 0; q < MQ; ++q) {
-      float* d = x + q * (4 * NV + 2) * 64;
-#pragma unroll
-      for (int v = 0; v < NV; ++v) *(f32x4*)(d + v * 256 + lane * 4) = o[q][v];
-      d[NV * 256 + lane] = mr[q];
-      d[NV * 256 + 64 + lane] = lr[q];
-    }
-  }
-  lds_sync();
-  if (part || !live) return;
-#pragma unroll
-  for (int q = 0; q < MQ; ++q) {
-    const float* d = x + q * (4 * NV + 2) * 64;
-    const float m1 = d[NV * 256 + lane], l1 = d[NV * 256 + 64 + lane], mx = fmaxf(mr[q], m1);
-    const float f0 = __builtin_amdgcn_exp2f(mr[q] - mx), f1 = __builtin_amdgcn_exp2f(m1 - mx);
-    float l = lr[q] * f0 + l1 * f1;
-    l += lane_xor<16>(l);
-    l += lane_xor<32>(l);
-    const int m = row0 + q * 16 + col;
-    if (m >= a.M) continue;
-    const float sc = a.gate[(size_t)m * a.heads + h] / l;
-    bf16* out = (bf16*)a.out + (size_t)m * a.ldo + (size_t)h * a.vdim + 4 * g;
-#pragma unroll
-    for (int v = 0; v < NV; ++v) *(bf16x4*)(out + v * 16) = quad<bf16>((o[q][v] * f0 + *(const f32x4*)(d + v * 256 + lane * 4) * f1) * sc);
-  }
+        for (int v = 0; v < NV; ++v) *(bf16x4*)(out + v * 16) = quad<bf16>(o[v] * sc);
+      });
 }
 
 template <class T>
@@ -698,7 +572,7 @@ int launch_decode(const ti_latent_attn_args& a, hipStream_t s) {
 
 template <int MQ, int DKT, int RKT>
 int launch_block(const ti_latent_prefill_args& a, hipStream_t s) {
-  constexpr int kLds = 4 * (4 * (DKT + RKT) + 4 * DKT) * 1024;
+  constexpr int kLds = block_lds<DKT + RKT, 2 * DKT>();
   const int QG = ((a.M + 16 * MQ - 1) / (16 * MQ) + 3) / 4;
   auto* fn = latent_block_kernel<MQ, DKT, RKT>;
   TI_HIP_CHECK(hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, kLds),
@@ -712,7 +586,7 @@ template <class T>
 int launch_prefill(const ti_latent_prefill_args& a, hipStream_t s) {
   if constexpr (sizeof(T) == 2) {
     const bool sized = a.vdim == a.vdim_p && a.vdim == a.dim_p && (a.dim_p == 64 || a.dim_p == 128) && (a.rot_p == 32 || a.rot_p == 64) &&
-                       a.ldo % 4 == 0 && a.scale > 0.0f;
+                       a.ldo % 4 == 0 && ((uintptr_t)a.out & 7) == 0 && a.scale > 0.0f;
     // 16 rows a wave while such workgroups are on the CUs together (dims of 128: one a CU, of 64: two), else 32
     if (sized) {
       const bool wide = (long)((a.M + 63) / 64) * a.heads > (a.dim_p == 128 ? 256 : 512);
