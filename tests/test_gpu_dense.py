@@ -204,6 +204,33 @@ def test_expert_rounds(ti, epi, tiles_n, N, K):
         assert (out[n_in] == 7).all()
 
 
+@pytest.mark.parametrize("M,N,K,act_cols,t_cols,ldo", [
+    (1100, 8712, 2048, 4356, 8648, 8656),   # 256 x 256 blocks; an activation and fp32 columns that end inside 64 columns
+    (1100, 8712, 2048, 4352, 8704, 8704),   # .. at 64 columns, the last 8 fp32
+    (1100, 8712, 2048, 8712, 8712, 8717),   # .. rows that 16 bytes do not fit
+    (700, 2304, 2048, 1024, 2304, 2304),    # 128 x 128 in two groups of waves
+    (333, 2300, 512, 0, 2236, 2240),
+])
+@pytest.mark.parametrize("act", ["TANH", "ERF"])
+def test_act_blocks(ti, M, N, K, act_cols, t_cols, ldo, act):
+    """Bias, activation of the first columns, fp32 columns past the 16-bit ones.  Bound: |gelu'| <= 1.13 times the product's, and the
+    roundings of the stored types and of the activation (4e-6 of the value, as test_gelu has it; tanh form 1e-5)."""
+    a, w, f = operands(M, N, K, torch.bfloat16, 1, 7)
+    bias = torch.randn(N, device="cuda", generator=torch.Generator(device="cuda").manual_seed(3))
+    out = torch.full((M + 1, ldo), 7.0, device="cuda").bfloat16()
+    out2 = torch.full((M + 1, N - t_cols + 4), 7.0, device="cuda")
+    call(ti, ti.DenseArgs(w=f.data_ptr(), a=a.data_ptr(), out=out.data_ptr(), lda=K, ldo=ldo, M=M, N=N, K=K, batch=1, epi=ti.DE_ACT,
+                          dtype=ti.DT_BF16, add=bias.data_ptr(), act=ti.ACT_GELU_TANH if act == "TANH" else ti.ACT_GELU_ERF, act_cols=act_cols,
+                          t_cols=t_cols, out2=out2.data_ptr(), ld2=N - t_cols + 4))
+    y = a.double() @ w[0].double().T + bias.double()
+    tol = 1.13 * (K + 1) * 2.0**-24 * (a.double().abs() @ w[0].double().abs().T + bias.double().abs())
+    ref = torch.cat([torch.nn.functional.gelu(y[:, :act_cols], approximate="tanh" if act == "TANH" else "none"), y[:, act_cols:]], 1)
+    err = (torch.cat([out[:M, :t_cols].double(), out2[:M, : N - t_cols].double()], 1) - ref).abs()
+    assert err[:, :t_cols].le(tol[:, :t_cols] + (2.0**-8 + 1e-5) * ref[:, :t_cols].abs() + 1e-7).all()
+    assert err[:, t_cols:].le(tol[:, t_cols:] + 2.0**-23 * ref[:, t_cols:].abs()).all()
+    assert (out[M] == 7).all() and (out[:, t_cols:] == 7).all() and (out2[M] == 7).all() and (out2[:, N - t_cols :] == 7).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M", [5, 200])
 def test_gelu(ti, dtype, M):

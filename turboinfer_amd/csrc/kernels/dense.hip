@@ -432,19 +432,28 @@ __global__ __launch_bounds__(64 * KG * WM * WN, 2) void dense_block_kernel(const
         for (int j = 0; j < FN; ++j)
           if ((i >= H) != (kg == 0)) acc[i][j] += x[(i * FN + j) * 64];
     }
+    const int c0 = at.n * (FN * WN) + wn * FN;
+    auto rows = [&](auto&& put) __attribute__((always_inline)) {   // put(i, m, mo, mt): row tiles that this wave finishes
 #pragma unroll
-    for (int i = 0; i < R; ++i) {
-      const int mt = m_base + (i * WM + wm) * 16;
-      if (i >= live) break;
-      if (KG == 2 && (i >= H) == (kg == 0)) continue;
-      const int m = mt + (lane & 15);
-      const int mo = m < m_end ? row_out(a, sp.first + m) : 0;
-#pragma unroll
-      for (int j = 0; j < FN; ++j) {
-        const int nt = at.n * (FN * WN) + wn * FN + j;
-        if (nt < NT) dense_out<T, EPI>(a, sp, m, mo, mt, nt, acc[i][j], lane);
+      for (int i = 0; i < R; ++i) {
+        const int mt = m_base + (i * WM + wm) * 16;
+        if (i >= live) break;
+        if (KG == 2 && (i >= H) == (kg == 0)) continue;
+        const int m = mt + (lane & 15);
+        put(i, m, m < m_end ? row_out(a, sp.first + m) : 0, mt);
       }
-    }
+    };
+    if constexpr (FN == 4)
+      if (wave64<T, EPI>(a, c0)) {
+        Wave64<EPI> w64(a, c0, lane);
+        rows([&](int i, int m, int mo, int) __attribute__((always_inline)) { w64.out(a, m < m_end, m, mo, c0, acc[i], lane); });
+        return;
+      }
+    rows([&](int i, int m, int mo, int mt) __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+        if (c0 + j < NT) dense_out<T, EPI>(a, sp, m, mo, mt, c0 + j, acc[i][j], lane);
+    });
   };
   if constexpr (FM == 8) {
     if (live > 7) tile.template operator()<8>();

@@ -3,54 +3,6 @@
 
 namespace ti {
 
-// 4 x 4 dwords turned over between four registers and the four 16-lane groups: d[k] of group g becomes d[g] of group k.
-__device__ __forceinline__ void turn_groups(uint32_t (&d)[4]) {
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const auto t = __builtin_amdgcn_permlane32_swap(d[i], d[i + 2], false, false);
-    d[i] = t[0];
-    d[i + 2] = t[1];
-  }
-#pragma unroll
-  for (int i = 0; i < 4; i += 2) {
-    const auto t = __builtin_amdgcn_permlane16_swap(d[i], d[i + 1], false, false);
-    d[i] = t[0];
-    d[i + 1] = t[1];
-  }
-}
-
-// A row tile of four column tiles nt.. whose 64 columns all exist, outputs 16-byte aligned: a lane gets 16 (SiLU * up: 8)
-// consecutive columns of its row.
-template <int EPI>
-__device__ __forceinline__ void expert_out(const ti_dense_args& a, bool live, int mo, int nt, const f32x4 (&v)[4], int lane) {
-  const int g = lane >> 4;
-  if constexpr (EPI == TI_DE_SWIGLU) {
-    uint32_t d[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const bf16x2 q = {(bf16)(v[j][0] * sigmoidf(v[j][0]) * v[j][1]), (bf16)(v[j][2] * sigmoidf(v[j][2]) * v[j][3])};
-      d[j] = __builtin_bit_cast(uint32_t, q);
-    }
-    turn_groups(d);
-    if (live) *(u32x4*)((bf16*)a.out + (size_t)mo * a.ldo + nt * 8 + g * 8) = (u32x4){d[0], d[1], d[2], d[3]};
-  } else {
-    uint32_t d[2][4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const u32x2 q = __builtin_bit_cast(u32x2, quad<bf16>(v[j]));
-      d[0][j] = q[0];
-      d[1][j] = q[1];
-    }
-    turn_groups(d[0]);
-    turn_groups(d[1]);
-    if (live) {
-      u32x4* o = (u32x4*)((bf16*)a.out + (size_t)mo * a.ldo + nt * 16 + g * 16);
-      o[0] = (u32x4){d[0][0], d[1][0], d[0][1], d[1][1]};
-      o[1] = (u32x4){d[0][2], d[1][2], d[0][3], d[1][3]};
-    }
-  }
-}
-
 // Bound: experts of few rows, the weights (64 experts, gate/up 2816 x 2048: 738 MB in 127 us, 5.8 TB/s); of many, LDS beside the
 // matrix cores (a k-tile of 256 x 256: 96 KiB of operand reads and 32 of copies in the 1024 cycles of its products; alone, products
 // and reads take 0.49 us, products and copies 0.50, all three 0.66).  So, against dense_block_kernel's 256-row form:
@@ -221,7 +173,8 @@ __global__ __launch_bounds__(512, 2) void dense_expert_kernel(const ti_dense_arg
       if (mt >= done.rows) break;
       const int mo = m < done.rows ? row_out(a, done.first + m) : 0;
       if (whole) {
-        expert_out<EPI>(a, m < done.rows, mo, c0, acc[i], lane);
+        if constexpr (EPI == TI_DE_SWIGLU) store_swiglu64(a, m < done.rows, mo, c0, acc[i], lane);
+        else store64(a, m < done.rows, mo, c0, acc[i], lane);
         continue;
       }
       const DenseSpan sp = {done.rows, done.first, 0, nullptr};
