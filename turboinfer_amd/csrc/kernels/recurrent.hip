@@ -257,6 +257,37 @@ __device__ __forceinline__ double wave_prefix(double v) {
 
 constexpr int kSsdTok = 64;
 
+// Eight fp32 values as the sum of three bf16 ones, exactly: the top 8 bits of their significands, the next 8, the last 8 (infinities and
+// NaN in the first).
+struct Split3 {
+  bf16x8 part[3];
+  __device__ __forceinline__ Split3(f32x4 a, f32x4 b) {
+    uint32_t d[3][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float v[2] = {i < 2 ? a[2 * i] : b[2 * i - 4], i < 2 ? a[2 * i + 1] : b[2 * i - 3]};
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        d[k][i] = __builtin_amdgcn_perm(__float_as_uint(v[1]), __float_as_uint(v[0]), 0x07060302u);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const float top = __uint_as_float(__float_as_uint(v[j]) & 0xffff0000u);
+          v[j] = k == 0 && top == v[j] ? 0.0f : v[j] - top;
+        }
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) part[k] = __builtin_bit_cast(bf16x8, (u32x4){d[k][0], d[k][1], d[k][2], d[k][3]});
+  }
+};
+__device__ __forceinline__ f32x4 mma3(bf16x8 a, const Split3& b, f32x4 c) { return mma(a, b.part[0], mma(a, b.part[1], mma(a, b.part[2], c))); }
+// 4 rows x 16 columns of 16-bit LDS a group of 16 lanes, lane j at row j >> 2, columns 4 (j & 3) ..: column j of the rows.
+__device__ __forceinline__ bf16x4 read_turned(const bf16* p) {
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(uintptr_t)p));
+}
+__device__ __forceinline__ bf16x8 pair_of(bf16x4 a, bf16x4 b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7); }
+
 // Grid (slices of 16 value dimensions, heads).  Blocks of 64 tokens one after another; per block, with
 // L(t, s) = exp(cum_t - cum_s):
 //   y_t = sum_{s <= t} (C_t . B_s) L(t, s) dt_s x_s + exp(cum_t) S^T C_t + D x_t
@@ -264,9 +295,17 @@ constexpr int kSsdTok = 64;
 // Waves 0..3 carry the state, 16 * NTW of its rows each, tile i holding every NTW-th from the i-th (a lane's
 // rows are 4 * NTW consecutive ones, its operands of all tiles come in one read): its share of every token's output, then
 // its update.  Waves 4..7 own 16 tokens each: their scores within the block and the output.  Accumulators
-// are the operand fragments of the next product (scores, state).  Waves 4..7 also load the next block and
+// are the operand fragments of the next product (scores, state).  Waves 0..3 also load the next block and
 // stage it at the end of this one (DB: into the other buffer); wave 4, which has the fewest scores, prepares
 // its step sizes and decays.
+// S3 (16-bit operands, states of more than 64): the fp32 factors of a token's output -- the carried state, the decayed scores -- are
+// taken apart into three bf16 (Split3), the other factor is bf16 already: three 16x16x32 products instead of eight fp32
+// 16x16x4 ones, which hold the matrix cores 5 times as long.  Tiles then hold 16 consecutive state rows, and the state's update, on fp32 products
+// still (split, its error grew: 6.3e-8 -> 7.5e-8 of the state at 1500 tokens), reads B turned in LDS.
+// Bound: one workgroup a CU and its chain of blocks, 2.7 us each; waves 4..7 alone take 2.05 of it, waves 0..3 as long.  us, 64 heads of 64
+// dimensions, state 128 (fp32 products, waves 4..7 staging -> products in parts -> waves 0..3 staging): 1500 tokens 78 -> 67 -> 64.5, 2048
+// 102.6 -> 83.8 in all, 333 25.9 -> 21.4; outputs' error against float64 7.69e-8 -> 7.59e-8.  No gain: wave 0 preparing the step sizes, all waves
+// staging.
 template <class T, int NTW, bool DB>
 __global__ __launch_bounds__(512, 1) void ssd_scan_kernel(const ti_ssd_args a) {
   typedef typename El<T>::V V;
@@ -274,6 +313,7 @@ __global__ __launch_bounds__(512, 1) void ssd_scan_kernel(const ti_ssd_args a) {
   extern __shared__ char lds[];
   const int N = a.state_n, nk = (N + KT - 1) / KT * KT, np = (N + 3) & ~3;
   constexpr int LN = 64 * NTW, ld = LN + 16 / (int)sizeof(T);   // (places past nk stay 0)
+  constexpr bool S3 = sizeof(T) == 2 && NTW % 2 == 0;
   T* bc = (T*)lds;                       // [DB ? 2 : 1][B, C][64][ld]
   float* xts = (float*)(bc + (DB ? 4 : 2) * kSsdTok * ld);   // [2][16][XLD] values, transposed
   f32x4* reds = (f32x4*)(xts + 2 * 16 * XLD);                // [DB ? 2 : 1][4][4][64] the state's output shares
@@ -291,12 +331,16 @@ __global__ __launch_bounds__(512, 1) void ssd_scan_kernel(const ti_ssd_args a) {
   float* state = a.state + (((size_t)a.slot0 * a.heads + h) * a.vdim + p0) * np;
   const bool prow = p0 + col < a.vdim;
   const int n0 = 16 * NTW * (wave & 3);   // this wave's state rows
-  f32x4 S[NTW];   // S[i][r]: state row n0 + NTW (4 g + r) + i, value dimension col
+  f32x4 S[NTW];   // S[i][r]: state row n0 + NTW (4 g + r) + i (S3: n0 + 16 i + 4 g + r), value dimension col
 #pragma unroll
   for (int q = 0; q < NTW; ++q) {
-    const int n = n0 + 4 * NTW * g + 4 * q;
+    const int n = n0 + (S3 ? 16 * q + 4 * g : 4 * NTW * g + 4 * q);
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
     if (sw && a.pos[0] > 0 && prow && n < np) v = *(const f32x4*)(state + (size_t)col * np + n);
+    if constexpr (S3) {
+      S[q] = v;
+      continue;
+    }
 #pragma unroll
     for (int e = 0; e < 4; ++e) S[(4 * q + e) % NTW][(4 * q + e) / NTW] = v[e];
   }
@@ -356,7 +400,7 @@ __global__ __launch_bounds__(512, 1) void ssd_scan_kernel(const ti_ssd_args a) {
     k[4 * kSsdTok + lane] = __builtin_amdgcn_exp2f(hi);
   };
   auto raw_dt = [&](int m0) { return a.dt[(size_t)min(m0 + lane, a.M - 1) * a.heads + h]; };
-  if (!sw) {
+  if (sw) {
     load(reg, 0);
     stage(reg, 0, 0);
   }
@@ -370,7 +414,7 @@ __global__ __launch_bounds__(512, 1) void ssd_scan_kernel(const ti_ssd_args a) {
     f32x4* red = reds + (DB ? buf : 0) * 16 * 64;
     const bool more = m0 + kSsdTok < a.M;
     float rdt = 0.0f;
-    if (more && !sw) load(reg, m0 + kSsdTok);
+    if (more && sw) load(reg, m0 + kSsdTok);
     if (more && wave == 4) rdt = raw_dt(m0 + kSsdTok);
     const int tok = w4 * 16 + col;
     f32x4 y = {0.f, 0.f, 0.f, 0.f};
@@ -380,15 +424,32 @@ __global__ __launch_bounds__(512, 1) void ssd_scan_kernel(const ti_ssd_args a) {
       f32x4 yi[4];
 #pragma unroll
       for (int t = 0; t < 4; ++t) yi[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
-      typedef T TN __attribute__((ext_vector_type(4 * NTW), aligned(4 * NTW * sizeof(T) < 16 ? 4 * NTW * sizeof(T) : 16)));
-      TN c[4];
+      if constexpr (S3) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t) c[t] = *(const TN*)(Cs + (t * 16 + col) * ld + n0 + 4 * NTW * g);
+        for (int q = 0; q < NTW; q += 2) {
+          const Split3 st(S[q], S[q + 1]);
+          bf16x8 c[4];
 #pragma unroll
-      for (int k = 0; k < 4 * NTW; ++k)
+          for (int t = 0; t < 4; ++t) {
+            const T* ct = Cs + (t * 16 + col) * ld + n0 + 16 * q + 4 * g;
+            c[t] = pair_of(*(const bf16x4*)ct, *(const bf16x4*)(ct + 16));
+          }
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
-          yi[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(S[k % NTW][k / NTW], (float)c[t][k], yi[t], 0, 0, 0);
+          for (int k = 2; k >= 0; --k)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) yi[t] = mma(st.part[k], c[t], yi[t]);
+        }
+      } else {
+        typedef T TN __attribute__((ext_vector_type(4 * NTW), aligned(4 * NTW * sizeof(T) < 16 ? 4 * NTW * sizeof(T) : 16)));
+        TN c[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) c[t] = *(const TN*)(Cs + (t * 16 + col) * ld + n0 + 4 * NTW * g);
+#pragma unroll
+        for (int k = 0; k < 4 * NTW; ++k)
+#pragma unroll
+          for (int t = 0; t < 4; ++t)
+            yi[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(S[k % NTW][k / NTW], (float)c[t][k], yi[t], 0, 0, 0);
+      }
 #pragma unroll
       for (int t = 0; t < 4; ++t) red[(w4 * 4 + t) * 64 + lane] = yi[t];
       // the state over the block
@@ -400,20 +461,41 @@ __global__ __launch_bounds__(512, 1) void ssd_scan_kernel(const ti_ssd_args a) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) wx[t][r] = w[r] * x[r];
       }
+      if constexpr (S3) {
+        bf16x4 b[4][NTW];
 #pragma unroll
-      for (int i = 0; i < NTW; ++i)
+        for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) S[i][r] *= last;
+          for (int i = 0; i < NTW; ++i) b[t][i] = read_turned(Bs + (t * 16 + 4 * g + (col >> 2)) * ld + n0 + 16 * i + 4 * (col & 3));
+        f32x4 add[NTW];
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        typedef T TB __attribute__((ext_vector_type(NTW)));
-        TB b[4];
+        for (int i = 0; i < NTW; ++i) add[i] = (f32x4){0.f, 0.f, 0.f, 0.f};   // (summed by itself: 75 -> 64.5 us)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) b[r] = *(const TB*)(Bs + (t * 16 + 4 * g + r) * ld + n0 + NTW * col);
+        for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
+          for (int r = 0; r < 4; ++r)
 #pragma unroll
-          for (int i = 0; i < NTW; ++i) S[i] = __builtin_amdgcn_mfma_f32_16x16x4f32((float)b[r][i], wx[t][r], S[i], 0, 0, 0);
+            for (int i = 0; i < NTW; ++i) add[i] = __builtin_amdgcn_mfma_f32_16x16x4f32((float)b[t][i][r], wx[t][r], add[i], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < NTW; ++i)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) S[i][r] = fmaf(S[i][r], last, add[i][r]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < NTW; ++i)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) S[i][r] *= last;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          typedef T TB __attribute__((ext_vector_type(NTW)));
+          TB b[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) b[r] = *(const TB*)(Bs + (t * 16 + 4 * g + r) * ld + n0 + NTW * col);
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int i = 0; i < NTW; ++i) S[i] = __builtin_amdgcn_mfma_f32_16x16x4f32((float)b[r][i], wx[t][r], S[i], 0, 0, 0);
+        }
       }
     } else {
       // scores of this wave's tokens with the block's earlier ones, decayed, times their inputs
@@ -451,6 +533,17 @@ __global__ __launch_bounds__(512, 1) void ssd_scan_kernel(const ti_ssd_args a) {
             sc[i][r] = s0 + r <= tok ? sc[i][r] * (e * d[r]) : 0.0f;
           }
         }
+        if constexpr (S3) {
+#pragma unroll
+          for (int i = 0; i < NS; i += 2) {
+            const f32x4 x0 = *(const f32x4*)(xt + col * XLD + i * 16 + 4 * g), x1 = *(const f32x4*)(xt + col * XLD + i * 16 + 16 + 4 * g);
+            const bf16x8 x = pair_of(quad<bf16>(x0), quad<bf16>(x1));
+            const Split3 s3(sc[i], sc[i + 1]);
+            if (i & 2) y2 = mma3(x, s3, y2);
+            else y = mma3(x, s3, y);
+          }
+          return;
+        }
 #pragma unroll
         for (int i = 0; i < NS; ++i) {
           const f32x4 x = *(const f32x4*)(xt + col * XLD + i * 16 + 4 * g);
@@ -465,7 +558,7 @@ __global__ __launch_bounds__(512, 1) void ssd_scan_kernel(const ti_ssd_args a) {
       for (int r = 0; r < 4; ++r) y[r] = fmaf(D, xt[(4 * g + r) * XLD + tok], y[r]);
       if (wave == 4 && more) steps(buf ^ 1, m0 + kSsdTok, rdt);
     }
-    if (DB && more && !sw) stage(reg, buf ^ 1, m0 + kSsdTok);
+    if (DB && more && sw) stage(reg, buf ^ 1, m0 + kSsdTok);
     lds_sync();
     if (!sw && m0 + tok < a.M) {   // out: this wave's tokens, dimensions 4 g + r
       f32x4 z = red[w4 * 64 + lane];
@@ -484,17 +577,18 @@ __global__ __launch_bounds__(512, 1) void ssd_scan_kernel(const ti_ssd_args a) {
       }
     }
     if (!DB && more) {
-      if (!sw) stage(reg, buf ^ 1, m0 + kSsdTok);
+      if (sw) stage(reg, buf ^ 1, m0 + kSsdTok);
       lds_sync();
     }
   }
   if (!sw) return;
 #pragma unroll
   for (int q = 0; q < NTW; ++q) {
-    const int n = n0 + 4 * NTW * g + 4 * q;
-    f32x4 v;
+    const int n = n0 + (S3 ? 16 * q + 4 * g : 4 * NTW * g + 4 * q);
+    f32x4 v = S[q];
+    if constexpr (!S3)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = S[(4 * q + e) % NTW][(4 * q + e) / NTW];
+      for (int e = 0; e < 4; ++e) v[e] = S[(4 * q + e) % NTW][(4 * q + e) / NTW];
     if (prow && n < np) *(f32x4*)(state + (size_t)col * np + n) = v;
   }
 }
