@@ -380,3 +380,37 @@ def test_shared_rows(ti, dtype, M, N):
     call(ti, d)
     check(out[:M], a[torch.arange(M, device="cuda") // div], w[0], dtype)
     assert (out[M] == 7).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,per,blocks", [(65, 16, 2), (130, 24, 3), (100, 33, 2), (200, 100, 2), (129, 256, 3)])
+def test_lru_gates(ti, dtype, M, per, blocks):
+    """Gates of a linear recurrence: whole and ragged 16-byte outputs, odd blocks whose last channel stands alone, rows past a tile.
+    Bound: the products' roundings through the logistic functions (slope 1/4), 2^-20 of each function's own, times what the
+    coefficients make of them."""
+    K = ti.lib().ti_stack_kpad(ti.DT_BF16 if dtype == torch.bfloat16 else ti.DT_F32, per)
+    N = 2 * per
+    g = torch.Generator("cuda").manual_seed(M)
+    u, w, f = operands(M, N, blocks * K, dtype, 1, M)
+    _, w, f = operands(M, N, K, dtype, blocks, M + 1)
+    bias = torch.randn(blocks, N, device="cuda", generator=g)
+    rate = torch.rand(blocks * per, device="cuda", generator=g) * 8 + 0.01
+    out = torch.full((M + 1, blocks * per, 2), 7.0, device="cuda")
+    d = ti.DenseArgs(w=f.data_ptr(), w_batch=f[0].numel(), a=u.data_ptr(), a_batch=K, out=out.data_ptr(), lda=blocks * K, ldo=2 * blocks * per, M=M, N=N,
+                     K=K, batch=blocks, epi=ti.DE_LRU, add=bias.data_ptr(), lru_rate=rate.data_ptr(),
+                     dtype=ti.DT_BF16 if dtype == torch.bfloat16 else ti.DT_F32)
+    call(ti, d)
+    for b in range(blocks):
+        a = u[:, b * K : (b + 1) * K].double()
+        z, e = a @ w[b].double().T + bias[b].double(), K * 2.0**-24 * (a.abs() @ w[b].double().abs().T + bias[b].double().abs())
+        r, i, er, ei = z[:, 0::2], z[:, 1::2], e[:, 0::2], e[:, 1::2]
+        k = rate[b * per : (b + 1) * per].double()
+        la = -torch.sigmoid(r) * k
+        da = k * (er / 4 + 2.0**-20)
+        s2 = -torch.expm1(2 * la)
+        x = a[:, :per]
+        ref_b, s = s2.sqrt() * torch.sigmoid(i) * x, s2.sqrt()
+        got = out[:M, b * per : (b + 1) * per].double()
+        assert (got[..., 0] - la.exp()).abs().le(la.exp() * da + 2.0**-21).all()
+        assert (got[..., 1] - ref_b).abs().le(x.abs() * (s * (ei / 4 + 2.0**-19) + torch.exp(2 * la) * da / s.clamp(min=1e-30)) + 1e-12).all()
+    assert (out[M] == 7).all()
