@@ -414,3 +414,32 @@ def test_lru_gates(ti, dtype, M, per, blocks):
         assert (got[..., 0] - la.exp()).abs().le(la.exp() * da + 2.0**-21).all()
         assert (got[..., 1] - ref_b).abs().le(x.abs() * (s * (ei / 4 + 2.0**-19) + torch.exp(2 * la) * da / s.clamp(min=1e-30)) + 1e-12).all()
     assert (out[M] == 7).all()
+
+
+@pytest.mark.parametrize("dtype,M,N,K,few", [
+    (torch.bfloat16, 65, 16, 512, True), (torch.bfloat16, 65, 16, 448, False), (torch.bfloat16, 2048, 64, 1024, True),
+    (torch.bfloat16, 2049, 64, 512, False), (torch.bfloat16, 500, 250, 1088, True), (torch.bfloat16, 130, 914, 640, False),
+    (torch.float32, 65, 7, 256, True), (torch.float32, 65, 7, 224, False), (torch.float32, 250, 1018, 544, True), (torch.float32, 257, 1018, 544, False)])
+def test_few_tiles(ti, dtype, M, N, K, few):
+    """Products of more than 64 rows and few tiles of outputs, to either side of the line."""
+    a, w, f = operands(M, N, K, dtype)
+    out = torch.full((M + 1, N + 3), 7.0, device="cuda")
+    d = ti.DenseArgs(w=f.data_ptr(), a=a.data_ptr(), out=out.data_ptr(), lda=K, ldo=N + 3, M=M, N=N, K=K, batch=1, epi=ti.DE_F32,
+                     dtype=ti.DT_BF16 if dtype == torch.bfloat16 else ti.DT_F32)
+    assert (tile(ti, d) == (0, 0)) == few
+    call(ti, d)
+    check(out[:M, :N], a, w[0], dtype)
+    assert (out[M] == 7).all() and (out[:, N:] == 7).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,N,K", [(65, 64, 2048), (500, 250, 576), (100, 1024, 512)])
+def test_few_tiles_swiglu(ti, dtype, M, N, K):
+    a, w, f = operands(M, N, K, dtype)
+    out = torch.full((M + 1, N // 2), 7.0, device="cuda").to(dtype)
+    d = ti.DenseArgs(w=f.data_ptr(), a=a.data_ptr(), out=out.data_ptr(), lda=K, ldo=N // 2, M=M, N=N, K=K, batch=1, epi=ti.DE_SWIGLU,
+                     dtype=ti.DT_BF16 if dtype == torch.bfloat16 else ti.DT_F32)
+    assert tile(ti, d) == (0, 0)
+    call(ti, d)
+    check_swiglu(out[:M], a, w[0], dtype)
+    assert (out[M] == 7).all()

@@ -4,7 +4,7 @@
 //
 // Four kernels share the epilogue (dense_expert.hip has a fifth, for experts of many rows):
 //   * dense_half_kernel (M <= 16, N <= 2048, plain outputs): weight streaming by 8 columns a workgroup.
-//   * dense_skinny_kernel (M <= 64): HBM-bound weight streaming.  One workgroup per 16 output columns,
+//   * dense_skinny_kernel (M <= 64, or few tiles of outputs): HBM-bound weight streaming.  One workgroup per 16 output columns,
 //     its waves split k; each weight fragment is one contiguous KiB read once and multiplied with up
 //     to 4 row tiles; the waves' partial sums meet in LDS.
 //   * dense_block_kernel (more rows: tiles of 32 x 64 up to 256 x 256): both operands copied to an LDS ring by DMA,
@@ -601,8 +601,18 @@ inline int tile_of(const ti_dense_args& a) {
   }
   return best;
 }
+// Few 16 x 16 tiles of outputs (short prompts' narrower products, routers): a workgroup each (dense_skinny_kernel), its waves over k, where
+// blocks would leave most CUs idle.  The line is where a second round of workgroups begins, with fp32's a third.  Measured, us, blocks -> this,
+// bf16: 66 x 1024 (K 2048) 8.5 -> 5.7, 100 x 512 (1024) 6.2 -> 3.9, 1000 x 64 (2048) 8.5 -> 4.8, 2048 x 64 8.5 -> 7.3; at 512 tiles 250 x 512 (4096) 13.1 ->
+// 11.2, at 576 and 640 8.4 -> 7.8 and 13.2 -> 15.9; fp32: 100 x 1024 (2048) 22.8 -> 12.0, 2048 x 64 23.0 -> 13.3, at 1024 tiles 23.0 -> 20.6, at
+// 1216 13.2 -> 13.7.  Short k leaves the waves nothing to share (300 x 64, bf16: K 256 3.86 / 3.87, K 512 x 384 4.76 -> 3.88).
+inline bool few_tiles(const ti_dense_args& a) {
+  const int f = a.dtype == TI_DT_F32;
+  return a.K >= (f ? 256 : 512) && (long)((a.M + 15) / 16) * ((a.N + 15) / 16) * a.batch <= (f ? 1024 : 512);
+}
 template <class T, int EPI>
 int tiled(const ti_dense_args& a, hipStream_t s) {
+  if (few_tiles(a)) return launch_skinny<T, 1, EPI>(a, s);
   const int i = tile_of(a), rows = kTile[i].rows;
   switch (i) {
     case 0: case 1: return launch_block<T, 1, 2, 4, 8, 4, 5, EPI>(a, rows, s);
@@ -718,8 +728,9 @@ extern "C" int ti_dense_tile(const ti_dense_args* a, int* rows, int* cols) {
   if (!a || !rows || !cols || a->M < 1 || a->N < 1 || a->K < 1 || a->batch < 1 ||
       (a->epi != TI_DE_F32 && a->epi != TI_DE_SWIGLU && a->epi != TI_DE_ROPE && a->epi != TI_DE_ACT) || a->tile_rows)
     return ti_set_error(TI_ERR_ARG, "ti_dense_tile: bad arguments");
-  *rows = few_rows(*a) ? 0 : kTile[tile_of(*a)].m;
-  *cols = few_rows(*a) ? 0 : kTile[tile_of(*a)].n;
+  const bool none = few_rows(*a) || few_tiles(*a);
+  *rows = none ? 0 : kTile[tile_of(*a)].m;
+  *cols = none ? 0 : kTile[tile_of(*a)].n;
   return TI_OK;
 }
 
