@@ -443,3 +443,30 @@ def test_few_tiles_swiglu(ti, dtype, M, N, K):
     call(ti, d)
     check_swiglu(out[:M], a, w[0], dtype)
     assert (out[M] == 7).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("epi", ["key", "value"])
+@pytest.mark.parametrize("M,heads,hw,K", [(1, 2, 64, 64), (65, 8, 64, 256), (129, 3, 32, 320), (500, 16, 128, 512), (641, 13, 128, 128), (1025, 8, 128, 64),
+                                          (2049, 9, 128, 64)])
+def test_fragments(ti, dtype, epi, M, heads, hw, K):
+    """Key and value fragments on either size of block: whole blocks of 128 keys are written, the last key again past the end."""
+    N, kt, vec = heads * hw, 32 if dtype == torch.bfloat16 else 16, 8 if dtype == torch.bfloat16 else 4
+    a, w, f = operands(M, N, K, dtype)
+    rows = -(-M // 128) * 128
+    blocks = rows // 16 + 8
+    out = torch.full((blocks * 16 * N,), 7.0, device="cuda").to(dtype)
+    d = ti.DenseArgs(w=f.data_ptr(), a=a.data_ptr(), out=out.data_ptr(), lda=K, ldo=N, M=M, N=N, K=K, batch=1, head_w=hw, key_blocks=blocks,
+                     epi=ti.DE_KFRAG if epi == "key" else ti.DE_VFRAG, dtype=ti.DT_BF16 if dtype == torch.bfloat16 else ti.DT_F32)
+    call(ti, d)
+    m, n = torch.arange(rows, device="cuda")[:, None], torch.arange(N, device="cuda")[None, :]
+    h, c = n // hw, n % hw
+    if epi == "key":
+        at = (((h * blocks + (m >> 4)) * (hw // kt) + c // kt) * 64 + c % kt // vec * 16 + (m & 15)) * vec + c % vec
+    else:
+        at = (((h * (hw >> 4) + (c >> 4)) * (blocks * 16 // kt) + m // kt) * 64 + ((m & 15) >> 2) * 16 + (c & 15)) * vec + (m % kt >> 4) * 4 + (m & 3)
+    got = out[at]
+    check(got[:M], a, w[0], dtype, dtype == torch.bfloat16)
+    assert (got[M:] == got[M - 1]).all()
+    out[at] = 7.0
+    assert (out == 7).all()

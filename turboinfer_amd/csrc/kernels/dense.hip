@@ -537,7 +537,8 @@ int launch_tile(const ti_dense_args& a, hipStream_t s) {
 template <class T, int KG, int WM, int WN, int FM, int FN, int NS, int EPI>
 int launch_block(const ti_dense_args& a, int step_rows, hipStream_t s) {
   typedef BlockCfg<KG, WM, WN, FM, FN, NS> C;
-  const int mt = (a.M + step_rows - 1) / step_rows, nt = (a.N + C::BN - 1) / C::BN;
+  const int rows = EPI == TI_DE_KFRAG || EPI == TI_DE_VFRAG ? (a.M + 127) / 128 * 128 : a.M;   // (fragments: whole blocks of 128 keys)
+  const int mt = (rows + step_rows - 1) / step_rows, nt = (a.N + C::BN - 1) / C::BN;
   auto* fn = dense_block_kernel<T, KG, WM, WN, FM, FN, NS, EPI>;
   TI_HIP_CHECK(hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, C::kLds),
                "hipFuncSetAttribute(dense_block_kernel)");
@@ -634,6 +635,15 @@ int grouped(const ti_dense_args& a, hipStream_t s) {
   return launch_tile<T, 64, 256, 2, EPI>(a, s);
 }
 
+// Key and value fragments: blocks of 64 x 64 with two groups of waves while they are one round of workgroups (fp32: two), else of
+// 128 x 128.  us, 128 x 128 -> 64 x 64, bf16: 130 rows of 512 columns (K 256) 7.5 -> 4.3, 300 of 2048 (K 512) 9.2 -> 5.6, 500 9.2 -> 6.0, 700
+// 9.5 -> 9.8, 2048 10.4 -> 18.6; fp32 20.7 -> 8.0, 36 -> 13, 36 -> 13.3, 700 36 -> 23.4.
+template <class T, int EPI>
+int fragments(const ti_dense_args& a, hipStream_t s) {
+  if ((long)((a.M + 127) / 128) * ((a.N + 127) / 128) <= (sizeof(T) == 4 ? 128 : 64)) return launch_block<T, 2, 2, 2, 2, 2, 9, EPI>(a, 64, s);
+  return launch_block<T, 1, 2, 2, 4, 4, 5, EPI>(a, 128, s);
+}
+
 inline bool few_rows(const ti_dense_args& a) { return a.tile_rows == 1 || a.tile_rows == 16 || (!a.tile_rows && a.M <= 64); }
 template <class T>
 int dispatch_dense(const ti_dense_args& a, hipStream_t s) {
@@ -652,8 +662,8 @@ int dispatch_dense(const ti_dense_args& a, hipStream_t s) {
       if (few) return skinny<T, TI_DE_T>(a, s);
       return a.tile_rows ? grouped<T, TI_DE_T>(a, s) : launch_tile<T, 64, 64, 4, TI_DE_T>(a, s);
     // (every row of a 128-row tile is written by the fragment epilogues; 2048 x 2048, K 512: 15.0 -> 14.4 us by blocks)
-    case TI_DE_KFRAG: return launch_block<T, 1, 2, 2, 4, 4, 5, TI_DE_KFRAG>(a, 128, s);
-    default: return launch_block<T, 1, 2, 2, 4, 4, 5, TI_DE_VFRAG>(a, 128, s);
+    case TI_DE_KFRAG: return fragments<T, TI_DE_KFRAG>(a, s);
+    default: return fragments<T, TI_DE_VFRAG>(a, s);
   }
 }
 
