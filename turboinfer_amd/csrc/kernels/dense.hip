@@ -332,7 +332,9 @@ struct BlockCfg {
 // 12 KiB per 32 products), fragments are read a stage ahead into the registers just used, and blocks of at most 128 x 128
 // run two groups of waves (KG 2) that take alternate k-tiles and meet in LDS at the end: a barrier and its skew per two
 // k-tiles, fewer LDS reads per product than tiles of half the size.  Deeper rings than NS give nothing.  A row of a stage
-// is 64 bytes: four lanes fetch it (chunks XOR-swizzled by row against LDS bank conflicts), 2 - 10 % over a lane per row.
+// is 64 bytes: four lanes fetch it (chunks XOR-swizzled by row against LDS bank conflicts), 2 - 10 % over a lane per row; with two
+// k-tiles a stage 128 bytes, eight lanes (us a launch inside a prompt: 1500 rows, K 2048 .. 8192, 2048 columns 45.6 -> 39.8, 2048 rows
+// 31.1 -> 29.1; alone with weights in the caches K 2048 3 - 6 % faster, K 4096 and 8192 up to 4 % slower).
 // Measured, us, bf16, dense_tile_kernel and blocks without KG -> this: 2048 x 2048 at 100 rows 10.8 -> 8.6, 333 11.4 ->
 // 9.2, 1000 18.4 -> 15.0; 2048 x 8192 (N x K) at 333 46.5 -> 29, 1500 85.5 -> 64; 5120 x 2048 at 700 29.8 -> 22; fp32
 // 2048 x 2048 at 100 rows 45 -> 24.
@@ -361,18 +363,18 @@ __global__ __launch_bounds__(64 * KG * WM * WN, 2) void dense_block_kernel(const
     constexpr int NA = KG * R * WM, NF = NA + KG * FN * WN, ND = (NF + NW - 1) / NW, REST = NF % NW;
     static_assert(NS * ND < 64, "vmcnt");
     const bool whole = REST == 0 || wave < REST;   // this wave copies ND fragments a stage, else one less
-    // this wave's fragments of a stage (KG k-tiles of the block): row tiles by k-tile, then weight tiles by k-tile
+    // this wave's KiB of a stage (KG k-tiles of the block): rows, then weight tiles by k-tile
     const V* src[ND];
     uint32_t dst[ND], step[ND];
 #pragma unroll
     for (int i = 0; i < ND; ++i) {
       const int f = min(i * NW + wave, NF - 1);
       dst[i] = lds0 + (uint32_t)f * 1024;
-      if (f < NA) {
-        const int g = f / (R * WM), rt = f % (R * WM);
-        const int p = sp.first + min(m_base + rt * 16 + (lane >> 2), sp.rows - 1);
-        src[i] = (const V*)((const T*)a.a + (size_t)sp.batch * a.a_batch + (size_t)row_in(a, p) * a.lda) + g * (KT / VEC) +
-                 ((lane & 3) ^ (lane >> 3 & 3));
+      if (f < NA) {   // 16 rows x 64 bytes, or with two k-tiles a stage 8 x 128
+        const int m = KG == 2 ? f * 8 + (lane >> 3) : f * 16 + (lane >> 2);
+        const int p = sp.first + min(m_base + m, sp.rows - 1);
+        src[i] = (const V*)((const T*)a.a + (size_t)sp.batch * a.a_batch + (size_t)row_in(a, p) * a.lda) +
+                 (KG == 2 ? (lane & 7) ^ (m >> 1 & 7) : (lane & 3) ^ (lane >> 3 & 3));
         step[i] = KG * KT / VEC;
       } else {
         const int g = (f - NA) / (FN * WN), ct = (f - NA) % (FN * WN);
@@ -400,9 +402,10 @@ __global__ __launch_bounds__(64 * KG * WM * WN, 2) void dense_block_kernel(const
     const V* const first = (const V*)ring;
     const V* cur = first;   // the stage being multiplied
     // wave (kg, wm, wn): k-tile kg of a stage, row tiles wm, wm + WM, .., weight tiles wn * FN ..
-    const int at_a = (kg * R * WM + wm) * 64 + (lane & 15) * 4 + (lane >> 4 ^ (lane >> 1 & 3));
+    const int at_a = KG == 2 ? wm * 128 + (lane & 15) * 8 + ((kg * 4 + (lane >> 4)) ^ (lane >> 1 & 7))
+                             : wm * 64 + (lane & 15) * 4 + (lane >> 4 ^ (lane >> 1 & 3));
     const int at_w = (NA + kg * FN * WN + wn * FN) * 64 + lane;
-    auto read_a = [&](const V* st, int i) { af[i] = st[i * WM * 64 + at_a]; };
+    auto read_a = [&](const V* st, int i) { af[i] = st[i * KG * WM * 64 + at_a]; };
     auto read_w = [&](const V* st, V (&d)[FN], int j) { d[j] = st[j * 64 + at_w]; };
     // One stage.  Its weights and all but its last R / 4 row tiles were read a stage ago; each register takes the next
     // stage's fragment as soon as its products are issued.  The last ones are read here, so that reads of a ring slot end
