@@ -101,3 +101,64 @@ def test_gqa_prompt(ti, dim, M, pos0, heads, kv, extras):
         ref, mag = w @ vv * gt, w @ vv.abs() * gt
         err = (out[:M, h * dim : (h + 1) * dim].double() - ref).abs()
         assert err.le(2.0**-8 * mag + 2.0**-8 * ref.abs() + 1e-6).all(), (h, err.max().item())
+
+
+def latent_prompt(ti, q, k, v, kr, sink, scale, pos0):
+    """Outputs [row][head][dim] of keys k, values v [head][key][dim] and rotated parts kr [key][rot], without a gate."""
+    (M, heads, width), (_, seq, dim) = q.shape, k.shape
+    kf = k.view(heads, seq // 16, 16, dim // 32, 4, 8).permute(0, 1, 3, 4, 2, 5).contiguous()
+    vf = v.view(heads, seq // 32, 2, 4, 4, dim // 16, 16).permute(0, 5, 1, 3, 6, 2, 4).contiguous()
+    cache, gate, out = torch.cat([kr, kr], 1).contiguous(), torch.ones(M, heads, device="cuda"), torch.empty(M, heads, dim, device="cuda").bfloat16()
+    a = Args(q=q.data_ptr(), kfrag=kf.data_ptr(), vfrag=vf.data_ptr(), cache=cache.data_ptr(), sink=sink.data_ptr(), gate=gate.data_ptr(),
+             out=out.data_ptr(), scale=scale, M=M, pos0=pos0, heads=heads, dim_p=dim, rot_p=width - dim, lat_p=width - dim, vdim=dim, vdim_p=dim,
+             key_blocks=seq // 16, ldo=heads * dim, dtype=ti.DT_BF16)
+    torch.cuda.synchronize()
+    ti.check(ti.lib().ti_latent_attn_prefill(C.byref(a), None))
+    ti.sync()
+    return out
+
+
+def gqa_prompt(ti, q, k, v, sink, scale, pos0):
+    """Outputs [row][head][dim] of keys and values [kv-head][key][dim]."""
+    (M, heads, dim), (kv, seq, _) = q.shape, k.shape
+    kf = k.view(kv, seq // 64, 4, 16, dim // 32, 4, 8).permute(0, 1, 2, 4, 5, 3, 6).reshape(kv, seq // 64, -1)
+    vf = v.view(kv, seq // 64, 2, 2, 4, 4, dim // 16, 16).permute(0, 1, 6, 2, 4, 7, 3, 5).reshape(kv, seq // 64, -1)
+    cache, out = torch.cat([kf, vf], -1).contiguous(), torch.empty(M, heads, dim, device="cuda").bfloat16()
+    a = GqaArgs(q=q.data_ptr(), cache=cache.data_ptr(), sink=None if sink is None else sink.data_ptr(), out=out.data_ptr(), scale=scale, M=M,
+                pos0=pos0, heads=heads, kv_heads=kv, dim=dim, vdim=dim, seq_p=seq, ldo=heads * dim, dtype=ti.DT_BF16)
+    torch.cuda.synchronize()
+    ti.check(ti.lib().ti_gqa_prefill(C.byref(a), None))
+    ti.sync()
+    return out
+
+
+def prompt(ti, kind, dim, M, pos0, heads, sharp, sink):
+    """A call's outputs and, in float64, its weights [head][row][key] and values [head][key][dim]."""
+    g = torch.Generator(device="cuda").manual_seed(M + dim)
+    keys, rot = pos0 + M, 32 if kind == "latent" else 0
+    kv = heads if kind == "latent" else heads // 2
+    seq = -(-keys // 128) * 128
+
+    def rand(*shape):
+        return torch.randn(*shape, device="cuda", generator=g).bfloat16()
+
+    q, k, v, kr = rand(M, heads, dim + rot), rand(kv, seq, dim), rand(kv, seq, dim), rand(seq, rot)
+    scale = sharp * (dim + rot) ** -0.5
+    out = latent_prompt(ti, q, k, v, kr, sink, scale, pos0) if kind == "latent" else gqa_prompt(ti, q, k, v, sink, scale, pos0)
+    kk = torch.cat([k[:, :keys].double(), kr[:keys].double().expand(kv, keys, rot)], 2).repeat_interleave(heads // kv, 0)
+    sc = (q.double().transpose(0, 1) @ kk.transpose(1, 2).contiguous()) * scale
+    sc = sc.masked_fill(torch.arange(keys, device="cuda") > pos0 + torch.arange(M, device="cuda")[:, None], -float("inf"))
+    w = torch.softmax(torch.cat([sc, sink.double().view(heads, 1, 1).expand(heads, M, 1)], 2), 2)[:, :, :-1].contiguous()
+    return out, w, v[:, :keys].double().repeat_interleave(heads // kv, 0)
+
+
+@pytest.mark.parametrize("kind", ["latent", "gqa"])
+@pytest.mark.parametrize("dim,M,pos0,heads", [(128, 100, 3, 4), (128, 700, 0, 16), (128, 1401, 70, 24), (64, 300, 64, 8), (64, 1401, 5, 24)])
+def test_largest_weight_is_not_rounded(ti, kind, dim, M, pos0, heads):
+    """Sharp rows, one weight near 1: a block's largest weight is a power of 2 before the row's sum divides it, so bf16 rounds only the
+    others (2^-8 of each) and the output."""
+    out, w, v = prompt(ti, kind, dim, M, pos0, heads, 6.0, torch.full((heads,), -60.0, device="cuda"))
+    top, at = w.max(2)
+    ref, mag = w @ v, w @ v.abs() - top[:, :, None] * torch.gather(v.abs(), 1, at[:, :, None].expand(-1, -1, dim))
+    err = (out.transpose(0, 1).double() - ref).abs()
+    assert err.le(2.0**-8 * mag + 2.0**-8 * ref.abs() + 1e-5).all()
