@@ -162,3 +162,15 @@ def test_largest_weight_is_not_rounded(ti, kind, dim, M, pos0, heads):
     ref, mag = w @ v, w @ v.abs() - top[:, :, None] * torch.gather(v.abs(), 1, at[:, :, None].expand(-1, -1, dim))
     err = (out.transpose(0, 1).double() - ref).abs()
     assert err.le(2.0**-8 * mag + 2.0**-8 * ref.abs() + 1e-5).all()
+
+
+@pytest.mark.parametrize("kind", ["latent", "gqa"])
+@pytest.mark.parametrize("dim,M,pos0,heads", [(128, 100, 3, 4), (128, 1401, 16, 24), (64, 300, 41, 8), (64, 1401, 5, 40), (96, 200, 9, 6)])
+def test_sinks_of_minus_infinity(ti, kind, dim, M, pos0, heads):
+    """Heads without a sink beside ones with it; blocks whose keys a row does not see come before its first (positions that start inside
+    64).  Bound as above."""
+    sink = torch.randn(heads, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    sink[::2] = -float("inf")
+    out, w, v = prompt(ti, kind, dim, M, pos0, heads, 2.0, sink)
+    ref = w @ v
+    assert (out.transpose(0, 1).double() - ref).abs().le(2.0**-8 * (w @ v.abs()) + 2.0**-8 * ref.abs() + 1e-6).all()

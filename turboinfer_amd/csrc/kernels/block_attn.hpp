@@ -107,18 +107,19 @@ __device__ __forceinline__ void block_attention(char* lds, float scale2, bool li
       top[q] = fmaxf(top[q], mx);
       mx += fmaxf(ceilf(top[q] - mx), 0.0f);
       if (MQ > 1 || __builtin_amdgcn_ballot_w64(mx != mr[q]) != 0) {   // (hardly ever not; one tile a wave: the branch keeps its loads ahead, 42 -> 37 us)
-        const float alpha = __builtin_amdgcn_exp2f(mr[q] - mx);
+        const float alpha = mr[q] == mx ? 1.0f : __builtin_amdgcn_exp2f(mr[q] - mx);
         mr[q] = mx;
         lr[q] *= alpha;
 #pragma unroll
         for (int v = 0; v < NV; ++v) o[q][v] *= alpha;
       }
+      const float off = mr[q] == -INFINITY ? 0.0f : mr[q];   // (a sink of -inf and no key yet: weights 0)
       float l = 0.0f;
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          s[q][t][r] = __builtin_amdgcn_exp2f(fmaf(s[q][t][r], scale2, -mr[q]));
+          s[q][t][r] = __builtin_amdgcn_exp2f(fmaf(s[q][t][r], scale2, -off));
           l += s[q][t][r];
         }
       lr[q] += l;

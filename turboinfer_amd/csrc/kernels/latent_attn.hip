@@ -436,14 +436,14 @@ __global__ __launch_bounds__(256, NV > 8 ? 2 : 3) void latent_prefill_kernel(con
           mx = fmaxf(mx, s[q][t][r]);
         }
       mx = xor32_max(xor16_max(mx));
-      const float alpha = expf(mr[q] - mx);
+      const float off = mx == -INFINITY ? 0.0f : mx, alpha = expf(mr[q] - off);   // (a sink of -inf and no key yet: weights 0)
       mr[q] = mx;
       float l = 0.0f;
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          s[q][t][r] = expf(s[q][t][r] - mx);
+          s[q][t][r] = expf(s[q][t][r] - off);
           l += s[q][t][r];
         }
       lr[q] = lr[q] * alpha + l;
