@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import numpy as np
 import pytest
+import torch
 
 from test_gpu_kernels import dev
 
@@ -156,3 +157,21 @@ def test_prefill_attention_kv_heads(ti, nkv, hd, M, start):
         finally:
             assert ti.lib().ti_attn_prefill_set_kernel(0) == shared
         np.testing.assert_allclose(got, dec, rtol=4e-3, atol=4e-3)
+
+
+def test_prefill_attention_many_rows(ti):
+    """Four rows a workgroup of 16 query heads a kv-head: 65550 workgroups an XCD, more than the launch's y takes.  All rows are the same, at
+    one position: so are their outputs, and those of a call of 200 rows."""
+    M, nh, nkv, hd, keys = 262200, 128, 8, 64, 150
+    g = torch.Generator(device="cuda").manual_seed(5)
+    k, v = (torch.randn(nkv, keys, hd, device="cuda", generator=g).half() for _ in range(2))
+    q = torch.randn(1, nh * hd, device="cuda", generator=g).expand(M, -1).contiguous()
+    pos = torch.full((M,), keys - 1, device="cuda", dtype=torch.int32)
+    out = torch.zeros(M, nh * hd, device="cuda", dtype=torch.float16)
+    few = torch.zeros(200, nh * hd, device="cuda", dtype=torch.float16)
+    torch.cuda.synchronize()
+    for o, m in ((few, 200), (out, M)):
+        ti.check(ti.lib().ti_attn_prefill(q.data_ptr(), k.data_ptr(), v.data_ptr(), keys, pos.data_ptr(), m, nh, nkv, hd, o.data_ptr(), None))
+        ti.sync()
+    assert few.isfinite().all() and few[0].abs().max() > 0 and (few == few[0]).all()
+    assert (out - few[0]).abs().le(2.0**-10 * few[0].abs() + 2.0**-24).all()   # (another split of the keys: a unit in the last place)

@@ -4,7 +4,10 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "ti_hip.h"
+#include "xcd.hpp"
 
 namespace ti {
 
@@ -147,6 +150,17 @@ __device__ __forceinline__ void dma_1k_asm(const void* src, uint32_t off_lane, u
                : "=&s"(keep)
                : "v"(off_lane), "s"(at), "s"(__builtin_amdgcn_readfirstlane(lds))
                : "memory");
+}
+
+// The launch of a deal (x fastest: the XCDs in turn), and this workgroup's share of it.
+inline dim3 xcd_grid(const XcdDeal& d) { return dim3(8, std::min(d.per, kXcdRows), (d.per + kXcdRows - 1) / kXcdRows); }
+// one, two: any arguments from other 64-byte lines of the kernel's, which come in with the deal (behind the branch on what it says they
+// were a wait each: 0.1 - 0.2 us of a launch).
+template <class A, class B>
+__device__ __forceinline__ XcdWork xcd_work(const XcdDeal& d, A one, B two) {
+  int x = (int)blockIdx.x;
+  asm("" : "+s"(x) : "s"(one), "s"(two));   // (not volatile: loads behind it stay scalar)
+  return xcd_work(d, x, (int)(blockIdx.y + kXcdRows * blockIdx.z));
 }
 
 // max / sum with the lane 16 or 32 apart (l ^ 16, l ^ 32) through gfx950's v_permlane16/32_swap,

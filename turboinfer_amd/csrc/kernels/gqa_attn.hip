@@ -486,13 +486,13 @@ __global__ __launch_bounds__(256, NV * MQ > 16 ? 1 : 2) void gqa_prefill_kernel(
 // 44.9 / 38.4, 1000 27.9 -> 21.2 / 28.6, 500 13.4 -> 12.7, 200 10.4 -> 9.4, 40 10.5 -> 8.9; 8 on 2, 2048 rows 43.7 -> 33.2 / 43.3, 1000 20.5 -> 18.9, 500
 // 13.2 -> 13.4, 300 14.3 -> 12.2, 200 10.1 -> 10.8, 40 9.3 -> 8.8.
 template <int MQ, int DKT>
-__global__ __launch_bounds__(512, 2) void gqa_block_kernel(const ti_gqa_attn_args a, int QG, int spread) {
+__global__ __launch_bounds__(512, 2) void gqa_block_kernel(const ti_gqa_attn_args a, XcdDeal deal) {
   constexpr int NV = 2 * DKT, NF = 4 * DKT + 2 * NV;
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 15, g = lane >> 4;
-  // (consecutive workgroups go to the 8 XCDs in turn: those of a key/value head to one, or to 2^spread)
-  const int x = blockIdx.x, j = ((int)blockIdx.y << spread) + (x & ((1 << spread) - 1)), kvh = (x >> spread) + 8 * (int)blockIdx.z;
-  if (j >= QG || kvh >= a.kv_heads) return;
+  const XcdWork work = xcd_work(deal, a.q, a.heads);   // (a key/value head's workgroups on one XCD)
+  const int kvh = work.head, j = work.j, QG = deal.n;
+  if (kvh < 0) return;
   const int rep = a.heads / a.kv_heads, tiles = (a.M + 15) / 16 * rep, t0 = block_of(block_group(wave), j, QG) * MQ;
   const bool live = t0 < tiles;
   auto row = [&](int t) { return min(t, tiles - 1) / rep * 16; };   // a tile's first row
@@ -538,11 +538,11 @@ __global__ __launch_bounds__(512, 2) void gqa_block_kernel(const ti_gqa_attn_arg
 template <int MQ, int DKT>
 int launch_gqa_block(const ti_gqa_attn_args& a, hipStream_t s) {
   constexpr int kLds = block_lds<DKT, 2 * DKT>();
-  const int tiles = (a.M + 15) / 16 * (a.heads / a.kv_heads), QG = ((tiles + MQ - 1) / MQ + 3) / 4;
-  const int spread = a.kv_heads > 4 ? 0 : a.kv_heads > 2 ? 1 : 4 - a.kv_heads;   // (log2; three: 8 / 4)
+  const int tiles = (a.M + 15) / 16 * (a.heads / a.kv_heads);
+  const XcdDeal deal = xcd_deal(a.kv_heads, ((tiles + MQ - 1) / MQ + 3) / 4);
   auto* fn = gqa_block_kernel<MQ, DKT>;
   TI_HIP_CHECK(hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, kLds), "hipFuncSetAttribute(gqa_block_kernel)");
-  hipLaunchKernelGGL(fn, dim3(8, (QG + (1 << spread) - 1) >> spread, (a.kv_heads + 7) / 8), dim3(512), kLds, s, a, QG, spread);
+  hipLaunchKernelGGL(fn, xcd_grid(deal), dim3(512), kLds, s, a, deal);
   TI_LAUNCH_CHECK("gqa_block_kernel");
   return TI_OK;
 }

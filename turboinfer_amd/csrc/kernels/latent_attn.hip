@@ -510,12 +510,13 @@ __global__ __launch_bounds__(256, NV > 8 ? 2 : 3) void latent_prefill_kernel(con
 // -> 72 / 53.3, 1400 48.8 -> 47.0 / 38.0, 1024 37.0 -> 23.3 / 29.7, 500 19.1 -> 14.2, 150 10.7 -> 9.3, 32 10.2 -> 7.0, 64 behind 1000 34.6 ->
 // 27.1; 8 heads of 64 + 32, 2048 rows 35.0 -> 25.3 / 33.5, 300 10.8 -> 7.6.
 template <int MQ, int DKT, int RKT>
-__global__ __launch_bounds__(512, 2) void latent_block_kernel(const ti_latent_prefill_args a, int QG) {
+__global__ __launch_bounds__(512, 2) void latent_block_kernel(const ti_latent_prefill_args a, XcdDeal deal) {
   constexpr int NV = 2 * DKT, NKT = DKT + RKT;
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 15, g = lane >> 4;
-  const int h = (int)(blockIdx.x + 8 * blockIdx.z), j = blockIdx.y;   // (an XCD's workgroups: heads x, x + 8, ..)
-  if (h >= a.heads) return;
+  const XcdWork work = xcd_work(deal, a.q, a.heads);   // (a head's workgroups on one XCD)
+  const int h = work.head, j = work.j, QG = deal.n;
+  if (h < 0) return;
   const int row0 = block_of(block_group(wave), j, QG) * 16 * MQ, cw = a.lat_p + a.rot_p, nkb = a.key_blocks >> 1;
   const bool live = row0 < a.M;
   int top = 0;   // the workgroup's last row
@@ -573,11 +574,11 @@ int launch_decode(const ti_latent_attn_args& a, hipStream_t s) {
 template <int MQ, int DKT, int RKT>
 int launch_block(const ti_latent_prefill_args& a, hipStream_t s) {
   constexpr int kLds = block_lds<DKT + RKT, 2 * DKT>();
-  const int QG = ((a.M + 16 * MQ - 1) / (16 * MQ) + 3) / 4;
+  const XcdDeal deal = xcd_deal(a.heads, ((a.M + 16 * MQ - 1) / (16 * MQ) + 3) / 4);
   auto* fn = latent_block_kernel<MQ, DKT, RKT>;
   TI_HIP_CHECK(hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, kLds),
                "hipFuncSetAttribute(latent_block_kernel)");
-  hipLaunchKernelGGL(fn, dim3(8, QG, (a.heads + 7) / 8), dim3(512), kLds, s, a, QG);
+  hipLaunchKernelGGL(fn, xcd_grid(deal), dim3(512), kLds, s, a, deal);
   TI_LAUNCH_CHECK("latent_block_kernel");
   return TI_OK;
 }

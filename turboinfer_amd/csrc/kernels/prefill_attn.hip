@@ -362,7 +362,7 @@ template <int HD, int QB, int HALVES, int R, int NB>
 __global__ __launch_bounds__(64 * QB * HALVES, HD == 64 ? 4 : 1) void attn_prefill_wg_kernel(const float* __restrict__ q, const uint16_t* __restrict__ kc,
                                                                  const uint16_t* __restrict__ vc, int max_seq,
                                                                  const int32_t* __restrict__ pos, int M, int heads, int gsh,
-                                                                 float scale, uint16_t* __restrict__ out, int QG, int spread) {
+                                                                 float scale, uint16_t* __restrict__ out, ti::XcdDeal deal) {
   constexpr int DV = HD / 16, KW = HD / 32, BI = NB * HALVES;   // BI: blocks per iteration
   constexpr int ND = HD / 32, RPD = 16 / ND;   // DMAs of a K or V block, key rows each copies
   auto swz = [](int row) { return HD == 128 ? row : (row >> 1) & 7; };   // chunk c of key row `row` at c ^ swz(row)
@@ -380,10 +380,10 @@ __global__ __launch_bounds__(64 * QB * HALVES, HD == 64 ? 4 : 1) void attn_prefi
   // (a SIMD holds waves w and w + 4: one of a long and one of a short chain)
   const int part = wave / QB, qw = wave < 4 ? wave % QB : QB - 1 - wave % QB;
   const int G = 1 << gsh, qpw = 16 >> gsh;
-  // (consecutive workgroups go to the 8 XCDs in turn: those of a kv-head to one, or to 2^spread)
-  const int x = blockIdx.x, at = ((int)blockIdx.y << spread) + (x & ((1 << spread) - 1)), kvh = (x >> spread) + 8 * (int)blockIdx.z;
   const int nq = (M + qpw - 1) / qpw;
-  if (at >= QG || kvh * G >= heads) return;
+  const XcdWork work = xcd_work(deal, q, out);   // (a kv-head's workgroups on one XCD)
+  const int kvh = work.head, at = work.j, QG = deal.n;
+  if (kvh < 0) return;
   const int qb = (QG - 1 - at) + qw * QG;   // longest chains first
   const bool live = qb < nq;                        // (a wave past the chunk only copies)
   const int q0 = qb * qpw, qi = min(q0 + (r >> gsh), M - 1), h = kvh * G + (r & (G - 1));
@@ -669,10 +669,8 @@ extern "C" int ti_attn_prefill_keys(const float* q, const uint16_t* k_cache, con
                                   : two ? ti::attn_prefill_wg_kernel<128, 2, 4, 2 * TI_PF_WG_RING2, 2> : ti::attn_prefill_wg_kernel<128, 4, 2, 2 * TI_PF_WG_RING2, 4>)
                                : (!wg2 ? ti::attn_prefill_wg_kernel<64, 4, 1, TI_PF_WG_RING, 2>
                                   : two ? ti::attn_prefill_wg_kernel<64, 2, 4, 2 * TI_PF_WG_RING2, 2> : ti::attn_prefill_wg_kernel<64, 4, 2, 2 * TI_PF_WG_RING2, 4>);
-    // an XCD's workgroups: those of kv-heads x, x + 8, .., or a share of one of up to 4
-    const int spread = kv_heads > 4 ? 0 : kv_heads > 2 ? 1 : 4 - kv_heads;   // (log2; three: 8 / 4)
-    hipLaunchKernelGGL(fn, dim3(8, (qg + (1 << spread) - 1) >> spread, (kv_heads + 7) / 8), dim3(wg2 ? 512 : 256), 0, s, q, k_cache, v_cache,
-                       max_seq, pos, M, heads, gsh, scale, out, qg, spread);
+    const ti::XcdDeal deal = ti::xcd_deal(kv_heads, qg);
+    hipLaunchKernelGGL(fn, ti::xcd_grid(deal), dim3(wg2 ? 512 : 256), 0, s, q, k_cache, v_cache, max_seq, pos, M, heads, gsh, scale, out, deal);
   } else if (head_dim == 128) {
     if (deep)
       hipLaunchKernelGGL((ti::attn_prefill_kernel<128, TI_PF_RING_DEEP>), grid, dim3(64), 0, s, q, k_cache, v_cache,
