@@ -132,11 +132,11 @@ def gqa_prompt(ti, q, k, v, sink, scale, pos0):
     return out
 
 
-def prompt(ti, kind, dim, M, pos0, heads, sharp, sink):
+def prompt(ti, kind, dim, M, pos0, heads, sharp, sink, rot=32, group=2):
     """A call's outputs and, in float64, its weights [head][row][key] and values [head][key][dim]."""
     g = torch.Generator(device="cuda").manual_seed(M + dim)
-    keys, rot = pos0 + M, 32 if kind == "latent" else 0
-    kv = heads if kind == "latent" else heads // 2
+    keys, rot = pos0 + M, rot if kind == "latent" else 0
+    kv = heads if kind == "latent" else heads // group
     seq = -(-keys // 128) * 128
 
     def rand(*shape):
@@ -172,5 +172,16 @@ def test_sinks_of_minus_infinity(ti, kind, dim, M, pos0, heads):
     sink = torch.randn(heads, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
     sink[::2] = -float("inf")
     out, w, v = prompt(ti, kind, dim, M, pos0, heads, 2.0, sink)
+    ref = w @ v
+    assert (out.transpose(0, 1).double() - ref).abs().le(2.0**-8 * (w @ v.abs()) + 2.0**-8 * ref.abs() + 1e-6).all()
+
+
+@pytest.mark.parametrize("kind,dim,rot,M,pos0,heads,group", [   # one of every kernel, by attn_plan.hpp
+    ("gqa", 128, 0, 500, 0, 8, 4), ("gqa", 128, 0, 1000, 0, 16, 4), ("gqa", 128, 0, 2041, 0, 16, 4), ("gqa", 128, 0, 100, 20, 8, 4),
+    ("gqa", 64, 0, 500, 0, 8, 4), ("gqa", 64, 0, 1999, 0, 16, 4), ("gqa", 64, 0, 1601, 0, 32, 4), ("gqa", 64, 0, 100, 20, 8, 4)])
+def test_prompt_kernels(ti, kind, dim, rot, M, pos0, heads, group):
+    """Bound as above."""
+    sink = torch.randn(heads, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    out, w, v = prompt(ti, kind, dim, M, pos0, heads, 2.0, sink, rot, group)
     ref = w @ v
     assert (out.transpose(0, 1).double() - ref).abs().le(2.0**-8 * (w @ v.abs()) + 2.0**-8 * ref.abs() + 1e-6).all()

@@ -6,12 +6,13 @@
 //   * gqa_decode_kernel: the query heads that share a key/value head are the MFMA columns; a workgroup
 //     takes 64-position blocks, its waves split the positions for the scores and the value dimensions for
 //     the sums; keys are split over workgroups, merged by gqa_merge_kernel.
-//   * gqa_block_kernel: prompt chunks of 16-bit heads of 64 or 128 dims, blocks of keys and values in LDS for eight waves;
+//   * gqa_block_kernel: larger prompt chunks of 16-bit heads of 64 or 128 dims (attn_plan.hpp), blocks of keys and values in LDS for eight waves;
 //   * gqa_prefill_kernel: other prompt chunks; a workgroup owns MQ tiles of 16 rows of one key/value head's query
 //     heads (heads of the same rows first), its waves split the key blocks.
 // Scores, softmax and sums are fp32; the denominator holds exp(sink) of the head once.
 #include <algorithm>
 
+#include "attn_plan.hpp"
 #include "block_attn.hpp"
 
 namespace ti {
@@ -482,9 +483,7 @@ __global__ __launch_bounds__(256, NV * MQ > 16 ? 1 : 2) void gqa_prefill_kernel(
 }
 
 // The same on keys and values that a workgroup's waves share (block_attn.hpp): 16-bit heads of 32 DKT dims, keys and values.  Row blocks
-// are MQ tiles as above.  us, the kernel above -> 16 / 32 rows a wave: 16 heads on 4 of 128 dims, 2048 rows 65 -> 61 / 48.7, 1500 47.0 ->
-// 44.9 / 38.4, 1000 27.9 -> 21.2 / 28.6, 500 13.4 -> 12.7, 200 10.4 -> 9.4, 40 10.5 -> 8.9; 8 on 2, 2048 rows 43.7 -> 33.2 / 43.3, 1000 20.5 -> 18.9, 500
-// 13.2 -> 13.4, 300 14.3 -> 12.2, 200 10.1 -> 10.8, 40 9.3 -> 8.8.
+// are MQ tiles as above.  (attn_plan.hpp: where, and what it measured.)
 template <int MQ, int DKT>
 __global__ __launch_bounds__(512, 2) void gqa_block_kernel(const ti_gqa_attn_args a, XcdDeal deal) {
   constexpr int NV = 2 * DKT, NF = 4 * DKT + 2 * NV;
@@ -568,12 +567,9 @@ int launch_gqa_prefill(const ti_gqa_attn_args& a, hipStream_t s) {
   if constexpr (sizeof(T) == 2) {
     const bool sized = a.dim == a.vdim && (a.dim == 64 || a.dim == 128) && a.ldo % 4 == 0 && (!a.gate || a.ldg % 4 == 0) &&
                        (((uintptr_t)a.gate & 15) | ((uintptr_t)a.out & 7)) == 0 && a.scale > 0.0f;
-    // 16 rows a wave while such workgroups are on the CUs together (dims of 128: one a CU, of 64: two), else 32
-    if (sized) {
-      const bool wide = ((long)(a.M + 15) / 16 * (a.heads / a.kv_heads) + 3) / 4 * a.kv_heads > (a.dim == 128 ? 256 : 512);
-      if (a.dim == 128) return wide ? launch_gqa_block<2, 4>(a, s) : launch_gqa_block<1, 4>(a, s);
-      return wide ? launch_gqa_block<2, 2>(a, s) : launch_gqa_block<1, 2>(a, s);
-    }
+    const int rows = sized ? gqa_rows_a_wave(a.dim, a.M, a.pos0, a.heads, a.kv_heads) : 0;
+    if (rows && a.dim == 128) return rows == 32 ? launch_gqa_block<2, 4>(a, s) : launch_gqa_block<1, 4>(a, s);
+    if (rows) return rows == 32 ? launch_gqa_block<2, 2>(a, s) : launch_gqa_block<1, 2>(a, s);
   }
   const int nkt = gqa_dim_p<T>(a.dim) / El<T>::KT, nv = gqa_vdim_p(a.vdim) / 16, rep = a.heads / a.kv_heads;
   const long tiles = (long)((a.M + 15) / 16) * rep;
