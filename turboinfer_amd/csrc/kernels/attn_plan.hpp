@@ -18,4 +18,21 @@ constexpr int gqa_rows_a_wave(int dim, long M, long pos0, int heads, int kv_head
   return (tiles + 3) / 4 * kv_heads > (dim == 64 ? 768 : 256) ? 32 : 16;
 }
 
+// Latent heads of dim + rot dims, each with its own keys.  Waves on their own while they are at most one workgroup a CU (128 + 64: one and a half)
+// from 321 keys on (128 + 64: 129), unless the heads that an XCD's run touches overflow its L2 (4 MiB; every block is then read once a wave and
+// again); and where blocks of 32 rows a wave would fill a last round of workgroups, one a CU, by less than a half.  us, own / 16 / 32 rows: 128 + 64,
+// 4 heads, 700 rows 14.0 / 16.8; 8, 700 15.4 / 17.1; 8, 500 behind 1000 25.4 / 30.9; 4, 1000 behind 3000 (5 MB) 100 / 71; 16, 1024 28.3 / 22.2 /
+// 30.5, 2048 65 / 68 / 53; 24, 1300 48 / 51 / 57, 2048 98 / 103 / 96; 12, 3000 103 / 142 / 127; 64 + 32, 16, 300 7.6 / 7.0, 2048 42 / 33; 24, 2048 61
+// / 50 / 62 (two workgroups a CU: 16 rows at any size).
+constexpr int latent_rows_a_wave(int dim, int rot, long M, long pos0, int heads) {
+  const bool one = dim != 64 || rot != 32;   // workgroups a CU, by their LDS
+  const long keys = pos0 + M, wide = (M + 127) / 128 * heads, rounds = (wide + 255) / 256;
+  const int touched = heads == 1 ? 1 : heads / 8 + (heads % 8 ? 2 : 0);   // heads in an eighth of the (head, rows) list
+  const bool l2 = touched * keys * (2 * dim + rot) * 2 <= 4l << 20;
+  const bool large = dim == 128 && rot == 64;
+  if (keys > (large ? 128 : 320) &&
+      (((M + 15) / 16 * heads <= (large && keys > 320 ? 384 : 256) && l2) || (one && wide > 256 && 3 * 256 * rounds >= 4 * wide))) return 0;
+  return one && (M + 63) / 64 * heads > 256 ? 32 : 16;
+}
+
 }  // namespace ti

@@ -10,10 +10,12 @@
 //     workgroups (splits) and over the waves of each.
 //   * latent_prefill_kernel: prompt chunks, keys and values expanded per head into MFMA fragments
 //     (dense.hip TI_DE_KFRAG / TI_DE_VFRAG); a workgroup owns 16 or 32 query rows of one head, its waves
-//     split the keys.  latent_block_kernel: 16-bit heads of 64 or 128 dims, blocks of keys in LDS for four times as many rows.
+//     split the keys.  latent_block_kernel: larger chunks of 16-bit heads of 64 or 128 dims (attn_plan.hpp), blocks of keys in LDS for four
+//     times as many rows.
 // Scores, softmax and sums are fp32; the softmax denominator holds exp(sink) of the head once.
 #include <algorithm>
 
+#include "attn_plan.hpp"
 #include "block_attn.hpp"
 
 namespace ti {
@@ -506,9 +508,7 @@ __global__ __launch_bounds__(256, NV > 8 ? 2 : 3) void latent_prefill_kernel(con
 }
 
 // The same on keys and values that a workgroup's waves share (block_attn.hpp): 16-bit heads of 32 DKT dims (keys without their
-// rotated part, and values) and 32 RKT rotated ones.  us, per-wave streams -> 16 / 32 rows a wave: 16 heads of 128 + 64, 2048 rows 73.5
-// -> 72 / 53.3, 1400 48.8 -> 47.0 / 38.0, 1024 37.0 -> 23.3 / 29.7, 500 19.1 -> 14.2, 150 10.7 -> 9.3, 32 10.2 -> 7.0, 64 behind 1000 34.6 ->
-// 27.1; 8 heads of 64 + 32, 2048 rows 35.0 -> 25.3 / 33.5, 300 10.8 -> 7.6.
+// rotated part, and values) and 32 RKT rotated ones.  (attn_plan.hpp: where, and what it measured.)
 template <int MQ, int DKT, int RKT>
 __global__ __launch_bounds__(512, 2) void latent_block_kernel(const ti_latent_prefill_args a, XcdDeal deal) {
   constexpr int NV = 2 * DKT, NKT = DKT + RKT;
@@ -588,14 +588,12 @@ int launch_prefill(const ti_latent_prefill_args& a, hipStream_t s) {
   if constexpr (sizeof(T) == 2) {
     const bool sized = a.vdim == a.vdim_p && a.vdim == a.dim_p && (a.dim_p == 64 || a.dim_p == 128) && (a.rot_p == 32 || a.rot_p == 64) &&
                        a.ldo % 4 == 0 && ((uintptr_t)a.out & 7) == 0 && a.scale > 0.0f;
-    // 16 rows a wave while such workgroups are on the CUs together (dims of 128: one a CU, of 64: two), else 32
-    if (sized) {
-      const bool wide = (long)((a.M + 63) / 64) * a.heads > (a.dim_p == 128 ? 256 : 512);
-#define TI_LB(D, R) return wide ? launch_block<2, D, R>(a, s) : launch_block<1, D, R>(a, s)
+    if (const int rows = sized ? latent_rows_a_wave(a.dim_p, a.rot_p, a.M, a.pos0, a.heads) : 0) {
+#define TI_LB(D, R) return rows == 32 ? launch_block<2, D, R>(a, s) : launch_block<1, D, R>(a, s)
       if (a.dim_p == 128 && a.rot_p == 64) TI_LB(4, 2);
       if (a.dim_p == 128) TI_LB(4, 1);
       if (a.rot_p == 64) TI_LB(2, 2);
-      TI_LB(2, 1);
+      return launch_block<1, 2, 1>(a, s);
 #undef TI_LB
     }
   }
