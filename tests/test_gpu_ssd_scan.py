@@ -64,3 +64,53 @@ def test_ssd_scan(ti, dtype, M, heads, vdim, n, groups, carry):
         assert (y[t].view(heads, vdim).double() - ref).abs().le(unit * size).all(), t
     assert (state[0, :, :, :n].double() - s).abs().le(unit * mag).all()
     assert (y[M] == 7).all() and (state[1] == 3).all() and (state[0, :, :, n:] == 0).all()
+
+
+@pytest.mark.parametrize("n", [100, 128, 256])
+@pytest.mark.parametrize("what", ["c", "x"])
+def test_ssd_scan_infinities(ti, what, n):
+    """One infinite C (of token 5), or input of a token (70, dimension 3 of every head), beside positive ones: outputs that it takes part in are infinite
+    as a sum of whole products has them, the others what they are without it (but for the rows before an infinite input in its block of 64), up to
+    the order of fp32 sums of positive values."""
+    g = torch.Generator("cuda").manual_seed(n)
+    M, heads, vdim = 150, 16, 16
+    nk, np_, inner = -(-n // 32) * 32, -(-n // 4) * 4, heads * vdim
+
+    def rand(*s):
+        return torch.randn(*s, device="cuda", generator=g).abs() + 0.1
+
+    a = torch.zeros(M, inner + 2 * nk, device="cuda").bfloat16()
+    a[:, :inner], a[:, inner : inner + n], a[:, inner + nk : inner + nk + n] = rand(M, inner), rand(M, n), rand(M, n)
+    dt, bias, a_log, d = rand(M, heads), rand(heads), torch.full((heads,), -3.0, device="cuda"), rand(heads)
+    carry = torch.zeros(heads, vdim, np_, device="cuda")
+    carry[:, :, :n] = rand(heads, vdim, n).bfloat16().float()   # (parts of 0)
+    pos = torch.arange(M, device="cuda", dtype=torch.int32) + 9
+    fn = ti.lib().ti_ssd_scan
+    fn.argtypes = [C.c_void_p, C.c_void_p]
+
+    def run():
+        state, y = carry.clone(), torch.full((M, inner), 7.0, device="cuda")
+        args = SsdArgs(a=a.data_ptr(), dt=dt.data_ptr(), dt_bias=bias.data_ptr(), a_log=a_log.data_ptr(), d=d.data_ptr(), state=state.data_ptr(),
+                       y=y.data_ptr(), pos=pos.data_ptr(), M=M, heads=heads, vdim=vdim, state_n=n, groups=1, taps=4, lda=a.shape[1], ldy=inner, o0=inner,
+                       slot0=0, dtype=ti.DT_BF16)
+        torch.cuda.synchronize()
+        ti.check(fn(C.addressof(args), None))
+        ti.sync()
+        return y.view(M, heads, vdim)
+
+    plain = run()
+    assert plain.isfinite().all()
+    if what == "c":
+        a[5, inner + nk + 7] = float("inf")
+        y = run()
+        assert (y[5] == float("inf")).all()
+        same = torch.arange(M, device="cuda") != 5
+        assert ((y - plain)[same].abs() <= 2.0**-19 * plain[same]).all()
+    else:
+        a[70, 3:inner:vdim] = float("inf")
+        y = run()
+        # (a state's rows past n are 0 times the input in the blocks behind)
+        assert (y[70 : M if n % 64 == 0 else 128, :, 3] == float("inf")).all()
+        assert ((y - plain)[:64].abs() <= 2.0**-19 * plain[:64]).all()
+        other = torch.arange(vdim, device="cuda") != 3
+        assert ((y - plain)[:, :, other].abs() <= 2.0**-19 * plain[:, :, other]).all()

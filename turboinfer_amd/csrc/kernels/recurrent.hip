@@ -286,6 +286,13 @@ __device__ __forceinline__ bf16x4 read_turned(const bf16* p) {
   typedef short s16x4 __attribute__((ext_vector_type(4)));
   return __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(uintptr_t)p));
 }
+// s plus the squares of v.
+__device__ __forceinline__ float squares(bf16x8 v, float s) {
+  s = __builtin_amdgcn_fdot2_f32_bf16(__builtin_shufflevector(v, v, 0, 1), __builtin_shufflevector(v, v, 0, 1), s, false);
+  s = __builtin_amdgcn_fdot2_f32_bf16(__builtin_shufflevector(v, v, 2, 3), __builtin_shufflevector(v, v, 2, 3), s, false);
+  s = __builtin_amdgcn_fdot2_f32_bf16(__builtin_shufflevector(v, v, 4, 5), __builtin_shufflevector(v, v, 4, 5), s, false);
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_shufflevector(v, v, 6, 7), __builtin_shufflevector(v, v, 6, 7), s, false);
+}
 __device__ __forceinline__ bf16x8 pair_of(bf16x4 a, bf16x4 b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7); }
 
 // Grid (slices of 16 value dimensions, heads).  Blocks of 64 tokens one after another; per block, with
@@ -301,10 +308,12 @@ __device__ __forceinline__ bf16x8 pair_of(bf16x4 a, bf16x4 b) { return __builtin
 // S3 (16-bit operands, states of more than 64): the fp32 factors of a token's output -- the carried state, the decayed scores -- are
 // taken apart into three bf16 (Split3), the other factor is bf16 already: three 16x16x32 products instead of eight fp32
 // 16x16x4 ones, which hold the matrix cores 5 times as long.  Tiles then hold 16 consecutive state rows, and the state's update, on fp32 products
-// still (split, its error grew: 6.3e-8 -> 7.5e-8 of the state at 1500 tokens), reads B turned in LDS.
+// still (split, its error grew: 6.3e-8 -> 7.5e-8 of the state at 1500 tokens), reads B turned in LDS.  An infinite C or value times a part that is 0
+// is NaN where the whole product is infinite: who stages a block marks one that holds any, and its products are taken whole (1500 tokens 64.0 -> 66.0
+// us; sums checked where they are made 65.5, but 82 -> 96 at 1000 tokens of state 256, here 84).
 // Bound: one workgroup a CU and its chain of blocks, 2.7 us each; waves 4..7 alone take 2.05 of it, waves 0..3 as long.  us, 64 heads of 64
-// dimensions, state 128 (fp32 products, waves 4..7 staging -> products in parts -> waves 0..3 staging): 1500 tokens 78 -> 67 -> 64.5, 2048
-// 102.6 -> 83.8 in all, 333 25.9 -> 21.4; outputs' error against float64 7.69e-8 -> 7.59e-8.  No gain: wave 0 preparing the step sizes, all waves
+// dimensions, state 128 (fp32 products, waves 4..7 staging -> products in parts -> waves 0..3 staging): 1500 tokens 77 -> 67 -> 64, 2048
+// 96 -> 80 in all, 333 21.3 -> 18.6; outputs' error against float64 7.69e-8 -> 7.59e-8.  No gain: wave 0 preparing the step sizes, all waves
 // staging.
 template <class T, int NTW, bool DB>
 __global__ __launch_bounds__(512, 1) void ssd_scan_kernel(const ti_ssd_args a) {
@@ -319,6 +328,7 @@ __global__ __launch_bounds__(512, 1) void ssd_scan_kernel(const ti_ssd_args a) {
   f32x4* reds = (f32x4*)(xts + 2 * 16 * XLD);                // [DB ? 2 : 1][4][4][64] the state's output shares
   // [2][5][64]: cum_t / ln 2 in two floats, dt, L(last, t) dt_t, exp(cum_t)
   float* coef = (float*)(reds + (DB ? 2 : 1) * 16 * 64);
+  __shared__ __attribute__((aligned(16))) int marks[2][4];   // S3: a wave's share of the block holds an infinity or NaN (or squares beyond fp32)
   const int h = blockIdx.y, p0 = blockIdx.x * 16, tid = threadIdx.x, lane = tid & 63, col = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), grp = h / (a.heads / a.groups);
   const bool sw = wave < 4;
@@ -371,6 +381,7 @@ __global__ __launch_bounds__(512, 1) void ssd_scan_kernel(const ti_ssd_args a) {
     for (int e = 0; e < 4; ++e) d.x[e] = x[e];
   };
   auto stage = [&](const Regs& d, int buf, int m0) {
+    float big = 0.0f;
     T* B = bc + (DB ? buf : 0) * 2 * kSsdTok * ld;
     T* C = B + kSsdTok * ld;
 #pragma unroll
@@ -378,15 +389,25 @@ __global__ __launch_bounds__(512, 1) void ssd_scan_kernel(const ti_ssd_args a) {
       if (prow_[u] < kSsdTok) {
         *(V*)(B + prow_[u] * ld + pcol_[u]) = d.b[u];
         *(V*)(C + prow_[u] * ld + pcol_[u]) = d.c[u];
+        if constexpr (S3) big = squares(d.c[u], big);
       }
     for (int i = (tid & 255) + PF * TH; i < pieces; i += TH) {   // (long states)
       const int t = i / ppr, c = (i - t * ppr) * VEC;
       const T* s = bsrc + (size_t)min(m0 + t, a.M - 1) * a.lda + c;
+      const V cv = *(const V*)(s + c_off);
       *(V*)(B + t * ld + c) = *(const V*)s;
-      *(V*)(C + t * ld + c) = *(const V*)(s + c_off);
+      *(V*)(C + t * ld + c) = cv;
+      if constexpr (S3) big = squares(cv, big);
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) xts[buf * 16 * XLD + ((tid & 3) * 4 + e) * XLD + ((tid & 255) >> 2)] = (float)d.x[e];
+    for (int e = 0; e < 4; ++e) {
+      xts[buf * 16 * XLD + ((tid & 3) * 4 + e) * XLD + ((tid & 255) >> 2)] = (float)d.x[e];
+      if constexpr (S3) big = fmaf((float)d.x[e], (float)d.x[e], big);
+    }
+    if constexpr (S3) {
+      const bool mark = __builtin_amdgcn_ballot_w64(!(big < INFINITY)) != 0;
+      if (lane == 0) marks[buf][w4] = mark;
+    }
   };
   auto steps = [&](int buf, int m0, float raw) {   // one wave: step sizes, cumulated log decays
     const float dt = m0 + lane < a.M ? softplusf(raw + bias) : 0.0f;   // (past the end: no decay, no input)
@@ -413,6 +434,9 @@ __global__ __launch_bounds__(512, 1) void ssd_scan_kernel(const ti_ssd_args a) {
                 *ec = wl + kSsdTok;
     f32x4* red = reds + (DB ? buf : 0) * 16 * 64;
     const bool more = m0 + kSsdTok < a.M;
+    int4 mark = {};
+    if constexpr (S3) mark = *(const int4*)marks[buf];
+    auto whole = [&] { return S3 && __builtin_amdgcn_readfirstlane(mark.x | mark.y | mark.z | mark.w) != 0; };
     float rdt = 0.0f;
     if (more && sw) load(reg, m0 + kSsdTok);
     if (more && wave == 4) rdt = raw_dt(m0 + kSsdTok);
@@ -425,19 +449,30 @@ __global__ __launch_bounds__(512, 1) void ssd_scan_kernel(const ti_ssd_args a) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) yi[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
       if constexpr (S3) {
+        bf16x8 c[NTW / 2][4];
 #pragma unroll
-        for (int q = 0; q < NTW; q += 2) {
-          const Split3 st(S[q], S[q + 1]);
-          bf16x8 c[4];
+        for (int q = 0; q < NTW / 2; ++q)
 #pragma unroll
           for (int t = 0; t < 4; ++t) {
-            const T* ct = Cs + (t * 16 + col) * ld + n0 + 16 * q + 4 * g;
-            c[t] = pair_of(*(const bf16x4*)ct, *(const bf16x4*)(ct + 16));
+            const T* ct = Cs + (t * 16 + col) * ld + n0 + 32 * q + 4 * g;
+            c[q][t] = pair_of(*(const bf16x4*)ct, *(const bf16x4*)(ct + 16));
           }
+        if (whole()) {
 #pragma unroll
-          for (int k = 2; k >= 0; --k)
+          for (int q = 0; q < NTW; ++q)
 #pragma unroll
-            for (int t = 0; t < 4; ++t) yi[t] = mma(st.part[k], c[t], yi[t]);
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+              for (int t = 0; t < 4; ++t) yi[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(S[q][r], (float)c[q / 2][t][q % 2 * 4 + r], yi[t], 0, 0, 0);
+        } else {
+#pragma unroll
+          for (int q = 0; q < NTW / 2; ++q) {
+            const Split3 st(S[2 * q], S[2 * q + 1]);
+#pragma unroll
+            for (int k = 2; k >= 0; --k)
+#pragma unroll
+              for (int t = 0; t < 4; ++t) yi[t] = mma(st.part[k], c[q][t], yi[t]);
+          }
         }
       } else {
         typedef T TN __attribute__((ext_vector_type(4 * NTW), aligned(4 * NTW * sizeof(T) < 16 ? 4 * NTW * sizeof(T) : 16)));
@@ -533,7 +568,7 @@ __global__ __launch_bounds__(512, 1) void ssd_scan_kernel(const ti_ssd_args a) {
             sc[i][r] = s0 + r <= tok ? sc[i][r] * (e * d[r]) : 0.0f;
           }
         }
-        if constexpr (S3) {
+        if constexpr (S3) if (!whole()) {
 #pragma unroll
           for (int i = 0; i < NS; i += 2) {
             const f32x4 x0 = *(const f32x4*)(xt + col * XLD + i * 16 + 4 * g), x1 = *(const f32x4*)(xt + col * XLD + i * 16 + 16 + 4 * g);
