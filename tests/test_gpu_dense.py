@@ -115,6 +115,46 @@ def test_rotary_blocks(ti, shape, M, N, K, dtype):
     assert (out[M] == 7).all()
 
 
+@pytest.mark.parametrize("shape,M,N,K", [((256, 256), 1100, 8640, 2048), ((128, 256), 700, 8640, 2048), ((128, 128), 1100, 2112, 8192)])
+@pytest.mark.parametrize("head_w,rot_off", [(192, 128), (96, 64), (32, 16), (64, 0)])
+@pytest.mark.parametrize("pad", [0, 4])
+def test_rotary_heads(ti, shape, M, N, K, head_w, rot_off, pad):
+    """Pieces of 64 columns without a rotated part, all of it, both, and of two heads; rows that 16 bytes fit, and not.  A column in front of the
+    rotated part is infinite: its neighbours are what they are without it.  Bound as above."""
+    N = N // head_w * head_w
+    a, w, _ = operands(M, N, K, torch.bfloat16)
+    inf = head_w + 5
+    a[:, 0] = 1.0
+    w = torch.cat([w[0], w.new_zeros(-N % 16, K)])
+    if rot_off:
+        w[inf, 0] = float("inf")
+    f = w.view(-1, 16, K // 32, 4, 8).permute(0, 2, 3, 1, 4).contiguous()
+    pairs, ldo = (head_w - rot_off) // 2, N + pad
+    pos = torch.randperm(M, device="cuda", generator=torch.Generator(device="cuda").manual_seed(2)).int()
+    ang = torch.arange(M, device="cuda")[:, None].double() * 100.0 ** (-torch.arange(pairs, device="cuda").double() / pairs)
+    cs = torch.stack([ang.cos(), ang.sin()], -1).float().contiguous()
+    out = torch.full((M + 1, ldo), 7.0, device="cuda").bfloat16()
+    d = ti.DenseArgs(w=f.data_ptr(), a=a.data_ptr(), out=out.data_ptr(), lda=K, ldo=ldo, M=M, N=N, K=K, batch=1, epi=ti.DE_ROPE, head_w=head_w,
+                     rot_off=rot_off, rope_cs=cs.data_ptr(), pos=pos.data_ptr(), dtype=ti.DT_BF16)
+    assert tile(ti, d) == shape
+    call(ti, d)
+    if rot_off:
+        w[inf, 0] = 0.0
+    y, mag = a.double() @ w[:N].double().T, K * 2.0**-24 * (a.double().abs() @ w[:N].double().abs().T)
+    y, mag = y.view(M, -1, head_w), mag.view(M, -1, head_w)
+    c, s = (cs[pos.long()].double()[:, None, :, i] for i in (0, 1))
+    e, o = y[..., rot_off::2], y[..., rot_off + 1 :: 2]
+    ref, tol = y.clone(), mag.clone()
+    ref[..., rot_off::2], ref[..., rot_off + 1 :: 2] = e * c - o * s, o * c + e * s
+    tol[..., rot_off:] = (mag[..., rot_off::2] + mag[..., rot_off + 1 :: 2]).repeat_interleave(2, -1) + 2.0**-22 * (e.abs() + o.abs()).repeat_interleave(2, -1)
+    got, ref, tol = out[:M, :N].double(), ref.reshape(M, N), tol.reshape(M, N)
+    if rot_off:
+        assert (got[:, inf] == float("inf")).all()
+        got[:, inf] = ref[:, inf]
+    assert (got - ref).abs().le(tol + 2.0**-8 * ref.abs()).all()
+    assert (out[M] == 7).all() and (out[:, N:] == 7).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("tile_rows", [128, 256])
 @pytest.mark.parametrize("N,K", [(48, 64), (264, 128), (512, 192), (250, 448)])

@@ -342,9 +342,11 @@ struct Wave64 {   // column tiles nt .. nt + 3
           const float* cs = a.rope_cs + (size_t)a.pos[live ? m : 0] * pairs * 2;
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
-            const f32x4 t = rot[j] >= 0 ? *(const f32x4*)(cs + rot[j]) : (f32x4){1.0f, 0.0f, 1.0f, 0.0f};
-            v[j] = (f32x4){v[j][0] * t[0] - v[j][1] * t[1], v[j][1] * t[0] + v[j][0] * t[1], v[j][2] * t[2] - v[j][3] * t[3],
-                           v[j][3] * t[2] + v[j][2] * t[3]};
+            const f32x4 t = *(const f32x4*)(cs + max(rot[j], 0));   // (columns in front of the rotated part are left as they are)
+            const f32x4 u = {v[j][0] * t[0] - v[j][1] * t[1], v[j][1] * t[0] + v[j][0] * t[1], v[j][2] * t[2] - v[j][3] * t[3],
+                             v[j][3] * t[2] + v[j][2] * t[3]};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[j][i] = rot[j] >= 0 ? u[i] : v[j][i];
           }
         }
       } else {
