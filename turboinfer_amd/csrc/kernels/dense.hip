@@ -607,12 +607,16 @@ inline int tile_of(const ti_dense_args& a) {
 }
 // Few 16 x 16 tiles of outputs (short prompts' narrower products, routers): a workgroup each (dense_skinny_kernel), its waves over k, where
 // blocks would leave most CUs idle.  The line is where a second round of workgroups begins, with fp32's a third.  Measured, us, blocks -> this,
-// bf16: 66 x 1024 (K 2048) 8.5 -> 5.7, 100 x 512 (1024) 6.2 -> 3.9, 1000 x 64 (2048) 8.5 -> 4.8, 2048 x 64 8.5 -> 7.3; at 512 tiles 250 x 512 (4096) 13.1 ->
+// bf16: 66 x 1024 (K 2048) 8.5 -> 5.7, 100 x 512 (1024) 6.2 -> 3.9, 1000 x 64 (2048) 8.5 -> 4.8, 2048 x 64 8.4 -> 7.8; at 512 tiles 250 x 512 (4096) 12.9 ->
 // 11.2, at 576 and 640 8.4 -> 7.8 and 13.2 -> 15.9; fp32: 100 x 1024 (2048) 22.8 -> 12.0, 2048 x 64 23.0 -> 13.3, at 1024 tiles 23.0 -> 20.6, at
-// 1216 13.2 -> 13.7.  Short k leaves the waves nothing to share (300 x 64, bf16: K 256 3.86 / 3.87, K 512 x 384 4.76 -> 3.88).
+// 1216 13.2 -> 13.7.  Short k leaves the waves nothing to share (300 x 64, bf16: K 256 3.86 / 3.87, K 512 x 384 4.76 -> 3.88).  Few columns of long k have
+// more rows at as many tiles, which every column tile reads again and which fit no L2: half as many (bf16: 1000 x 64 (8192) 22.0 -> 15.0, 1200 22.0 ->
+// 23.6, 2048 x 64 (4096) 13.0 -> 14.6, 1000 x 128 (4096) 12.9 -> 14.6, 700 x 128 (3072) 10.6 -> 10.1, 500 x 256 (8192) 22.9 -> 21.4; fp32: 2048 x 64 (8192)
+// 78.5 -> 44.4, 2048 x 128 (8192) 79.0 -> 83.7, (4096) 43.0 -> 43.5, 1000 x 256 (8192) 79.5 -> 74.9).
 inline bool few_tiles(const ti_dense_args& a) {
   const int f = a.dtype == TI_DT_F32;
-  return a.K >= (f ? 256 : 512) && (long)((a.M + 15) / 16) * ((a.N + 15) / 16) * a.batch <= (f ? 1024 : 512);
+  const bool narrow = a.N < 256 && a.K > (f ? 4096 : 3072);
+  return a.K >= (f ? 256 : 512) && (long)((a.M + 15) / 16) * ((a.N + 15) / 16) * a.batch <= (f ? 1024 : 512) >> narrow;
 }
 template <class T, int EPI>
 int tiled(const ti_dense_args& a, hipStream_t s) {
