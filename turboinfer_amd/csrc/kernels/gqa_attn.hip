@@ -6,7 +6,7 @@
 //   * gqa_decode_kernel: the query heads that share a key/value head are the MFMA columns; a workgroup
 //     takes 64-position blocks, its waves split the positions for the scores and the value dimensions for
 //     the sums; keys are split over workgroups, merged by gqa_merge_kernel.
-//   * gqa_block_kernel: larger prompt chunks of 16-bit heads of 64 or 128 dims (attn_plan.hpp), blocks of keys and values in LDS for eight waves;
+//   * gqa_block_kernel: prompt chunks of 16-bit heads of 64 or 128 dims (attn_plan.hpp), blocks of keys and values in LDS for eight waves;
 //   * gqa_prefill_kernel: other prompt chunks; a workgroup owns MQ tiles of 16 rows of one key/value head's query
 //     heads (heads of the same rows first), its waves split the key blocks.
 // Scores, softmax and sums are fp32; the denominator holds exp(sink) of the head once.

@@ -10,7 +10,7 @@
 //     workgroups (splits) and over the waves of each.
 //   * latent_prefill_kernel: prompt chunks, keys and values expanded per head into MFMA fragments
 //     (dense.hip TI_DE_KFRAG / TI_DE_VFRAG); a workgroup owns 16 or 32 query rows of one head, its waves
-//     split the keys.  latent_block_kernel: larger chunks of 16-bit heads of 64 or 128 dims (attn_plan.hpp), blocks of keys in LDS for four
+//     split the keys.  latent_block_kernel: 16-bit heads of 64 or 128 dims (attn_plan.hpp), blocks of keys in LDS for four
 //     times as many rows.
 // Scores, softmax and sums are fp32; the softmax denominator holds exp(sink) of the head once.
 #include <algorithm>
@@ -588,7 +588,7 @@ int launch_prefill(const ti_latent_prefill_args& a, hipStream_t s) {
   if constexpr (sizeof(T) == 2) {
     const bool sized = a.vdim == a.vdim_p && a.vdim == a.dim_p && (a.dim_p == 64 || a.dim_p == 128) && (a.rot_p == 32 || a.rot_p == 64) &&
                        a.ldo % 4 == 0 && ((uintptr_t)a.out & 7) == 0 && a.scale > 0.0f;
-    if (const int rows = sized ? latent_rows_a_wave(a.dim_p, a.rot_p, a.M, a.pos0, a.heads) : 0) {
+    if (const int rows = sized ? latent_rows_a_wave(a.dim_p, a.rot_p, a.M, a.heads) : 0) {
 #define TI_LB(D, R) return rows == 32 ? launch_block<2, D, R>(a, s) : launch_block<1, D, R>(a, s)
       if (a.dim_p == 128 && a.rot_p == 64) TI_LB(4, 2);
       if (a.dim_p == 128) TI_LB(4, 1);
