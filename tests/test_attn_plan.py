@@ -10,17 +10,17 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 GQA = [   # dim, rows, position, heads, kv-heads, kernel
     (128, 40, 0, 16, 4, 16),        # 8.8 / 7.5
     (128, 300, 0, 8, 2, 16),        # 12.4 / 11.2
-    (128, 64, 1000, 16, 4, 0),      # 21.9 / 22.3
-    (128, 200, 2000, 8, 2, 0),      # 34.6 / 38.5
+    (128, 64, 1000, 20, 5, 16),     # a prompt 634 / 605
     (128, 500, 0, 16, 4, 16),       # 13.5 / 13.2
     (128, 400, 0, 32, 8, 16),       # 18.1 / 13.3
-    (128, 1000, 0, 4, 1, 0),        # 19.5 / 19.9
+    (128, 600, 0, 4, 1, 16),        # a prompt 354 / 341
     (128, 1000, 0, 16, 4, 16),      # 27.1 / 21.2 / 28.6
     (128, 1300, 0, 16, 4, 32),      # 37.3 / 40.7 / 35.2
     (128, 2048, 0, 16, 4, 32),      # 59.0 / 59.3 / 46.9
     (64, 300, 0, 16, 4, 16),        # 8.1 / 7.7
     (64, 500, 0, 16, 4, 0),         # 8.7 / 9.3
     (64, 2048, 0, 4, 1, 0),         # 19.8 / 23.2
+    (64, 30, 1800, 12, 3, 0),       # a prompt 288 / 306
     (64, 256, 0, 48, 12, 16),       # 8.5 / 7.0
     (64, 500, 0, 32, 8, 16),        # 12.2 / 9.5
     (64, 2048, 0, 16, 4, 16),       # 36.1 / 29.2 / 35.6

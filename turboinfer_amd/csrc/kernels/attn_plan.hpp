@@ -10,14 +10,16 @@ namespace ti {
 // 5 %).
 
 // Grouped queries, heads of dim dims. us, own / 16 / 32 rows: dims of 128, 16 heads on 4, 40 rows 8.8 / 7.5, 500 13.5 / 13.2, 1000 27.1 / 21.2 /
-// 28.6, 1300 37.3 / 40.7 / 35.2, 2048 59.0 / 59.3 / 46.9; 8 on 2, 300 12.4 / 11.2, 1000 20.2 / 20.1, 200 behind 2000 34.6 / 38.5; dims of 64, 16 on
-// 4, 300 8.1 / 7.7, 500 8.7 / 9.3, 1000 14.1 / 14.4, 2048 36.1 / 29.2 / 35.6; 4 on 1, 2048 19.8 / 23.2; 48 on 12, 256 8.5 / 7.0, 800 32.9 / 23.1 /
-// 27.0; 32 on 8, 1300 38.8 / 30.6 / 33.5, 1600 50.6 / 40.7 / 39.8. So: waves on their own where keys are many and they are at most one workgroup a CU
-// (dims of 64: three); 32 rows a wave where 16 would be a second round (64: two workgroups a CU, a third round). Left slower than waves on their own:
-// 3000 rows of 16 heads on 4 (108 / 119, a second round that is half full).
+// 28.6, 1300 37.3 / 40.7 / 35.2, 2048 59.0 / 59.3 / 46.9; 8 on 2, 300 12.4 / 11.2, 1000 20.2 / 20.1, 200 behind 2000 34.6 / 38.5 (whole prompts of 6
+// layers, own -> 16 rows: 4 on 1, 600 354 -> 341, 20 on 5, 64 behind 1000 634 -> 605, 30 behind 1800 604 -> 572: their keys come from farther still);
+// dims of 64, 16 on 4, 300 8.1 / 7.7, 500 8.7 / 9.3, 1000 14.1 / 14.4, 2048 36.1 / 29.2 / 35.6; 4 on 1, 2048 19.8 / 23.2; 48 on 12, 256 8.5 / 7.0,
+// 800 32.9 / 23.1 / 27.0; 32 on 8, 1300 38.8 / 30.6 / 33.5, 1600 50.6 / 40.7 / 39.8 (prompts, own -> 16: 12 on 3, 30 behind 1800 288 -> 306). So:
+// heads of 64 dims' waves on their own where keys are many and they are at most three workgroups a CU; 32 rows a wave where 16 would be a second
+// round (64: two workgroups a CU, a third round). Left slower than waves on their own: 3000 rows of 16 heads on 4 of 128 (108 / 119, a second round
+// that is half full).
 constexpr int gqa_rows_a_wave(int dim, long M, long pos0, int heads, int kv_heads) {
-  const long tiles = (M + 15) / 16 * (heads / kv_heads), keys = pos0 + M;
-  if (dim == 64 ? keys > 320 && tiles * kv_heads <= 768 : keys > 512 && tiles * kv_heads <= 256) return 0;
+  const long tiles = (M + 15) / 16 * (heads / kv_heads);
+  if (dim == 64 && pos0 + M > 320 && tiles * kv_heads <= 768) return 0;
   return (tiles + 3) / 4 * kv_heads > (dim == 64 ? 768 : 256) ? 32 : 16;
 }
 
