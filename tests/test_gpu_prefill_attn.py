@@ -46,8 +46,7 @@ def _case(ti, M, nh, nkv, hd, pos, max_seq, seed):
 @pytest.fixture(params=[0, 1, 2, 3], ids=["auto", "per_wave", "shared4", "shared8"])
 def kernel(request, ti):
     """ti_attn_prefill_set_kernel: the automatic choice, the per-wave kernel, and the shared-K/V
-    kernel with 4- and 8-wave workgroups forced at any grid size (head_dim 128; other head_dims
-    take the per-wave kernel)."""
+    kernel with 4- and 8-wave workgroups forced at any grid size."""
     L = ti.lib()
     assert L.ti_attn_prefill_set_kernel(request.param) == 0
     yield request.param
@@ -64,8 +63,6 @@ def kernel(request, ti):
     (200, 8, 8, 128, 1000, 1200),   # MHA, long prefix before a chunk whose blocks straddle 16
 ])
 def test_prefill_attention_vs_oracle(ti, oracle, kernel, M, nh, nkv, hd, start, max_seq):
-    if hd != 128 and kernel > 1:
-        pytest.skip("the shared-K/V kernel is head_dim 128 only")
     pos = (start + np.arange(M)).astype(np.int32)
     q, kc, vc, got, dec = _case(ti, M, nh, nkv, hd, pos, max_seq, seed=M + nh + hd)
     assert np.all(np.isfinite(got))
@@ -84,8 +81,6 @@ def test_prefill_attention_vs_oracle(ti, oracle, kernel, M, nh, nkv, hd, start, 
 def test_prefill_attention_ragged_positions(ti, kernel, hd):
     """Positions in any order and with gaps (each row's own causal limit, blocks of mixed length)
     and the 7B chunk shape, against the decode kernel."""
-    if hd != 128 and kernel > 1:
-        pytest.skip("the shared-K/V kernel is head_dim 128 only")
     rng = np.random.RandomState(hd)
     pos = rng.permutation(900)[:333].astype(np.int32)
     _, _, _, got, dec = _case(ti, 333, 8, 2, hd, pos, 1024, seed=hd + 1)

@@ -337,16 +337,13 @@ __global__ __launch_bounds__(64, WPE) void attn_prefill_kernel(const float* __re
 #ifndef TI_PF_WG_RING
 #define TI_PF_WG_RING 6    // K / V blocks in the LDS ring (8 KiB each), 4-wave workgroups
 #endif
-#ifndef TI_PF_QK_SPLIT
-#define TI_PF_QK_SPLIT 0   // shared-K/V kernel: S = K Q^T's hi and lo products in separate chains
-#endif
 #ifndef TI_PF_WG_LATE_DMA
 #define TI_PF_WG_LATE_DMA 0   // 1: DMAs issued after the step's S = K Q^T (even, profiles/r5_prefill_wg_latedma_ab.txt)
 #endif
 #ifndef TI_PF_WG_RING2
-#define TI_PF_WG_RING2 8   // the same, 8-wave workgroups (4 blocks per iteration; 8 beat 12 and 16, profiles/r5_prefill_wg_ring_ab.txt)
+#define TI_PF_WG_RING2 8   // half of the same, 8-wave workgroups: two iterations of 8 blocks
 #endif
-// HALVES: parts of a query block's keys, a wave each (iteration = 2 HALVES blocks, part h computes blocks 2 h, 2 h + 1 of it),
+// HALVES: parts of a query block's keys, a wave each (iteration = NB HALVES blocks, part h computes blocks NB h .. of it),
 // merging their (max, sum, O) through LDS at the end: two chains per SIMD hide each other's latencies.  The step is a chain
 // of dependent latencies beside ~ 110 vector instructions, so what counts is that the SIMDs have equal work: waves w and w +
 // 4 (one SIMD) take a long and a short chain (1000 rows of 32 heads on 4, head_dim 64: 26.5 -> 23.6 us with two parts of the
@@ -456,7 +453,7 @@ __global__ __launch_bounds__(64 * QB * HALVES, HD == 64 ? 4 : 1) void attn_prefi
 #if !TI_PF_WG_LATE_DMA
     issue(kbi + R - BI);
 #endif
-    const int kb = kbi + NB * part;   // this part's pair
+    const int kb = kbi + NB * part;   // this part's blocks
 #if TI_PF_DIAG & 4   // diagnostic: the ring and its barriers alone, no math
     const bool act = false;
 #else
@@ -535,9 +532,9 @@ __global__ __launch_bounds__(64 * QB * HALVES, HD == 64 ? 4 : 1) void attn_prefi
           ps += pv[b][i];
         }
       l_run += ps;
-      // O^T += V^T P^T over both blocks in one 32-key product (16x16x32, the full-rate form): k index
-      // 8 g + e is key 4 g + e of the first block for e < 4 and of the second for e >= 4, in the
-      // A fragment (V, lane (dim r DV + t, k)) and the B fragment (P, lane (column r, k)) alike
+      // O^T += V^T P^T over two blocks at a time in one 32-key product (16x16x32, the full-rate form): k
+      // index 8 g + e is key 4 g + e of the first block for e < 4 and of the second for e >= 4, in the
+      // A fragment (V, lane (dim 16 t + r, k)) and the B fragment (P, lane (column r, k)) alike
 #pragma unroll
       for (int u = 0; u < NB; u += 2) {
         f16x8 ph, pl;
