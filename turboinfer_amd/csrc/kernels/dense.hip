@@ -334,7 +334,8 @@ struct BlockCfg {
 // k-tiles, fewer LDS reads per product than tiles of half the size.  Deeper rings than NS give nothing.  A row of a stage
 // is 64 bytes: four lanes fetch it (chunks XOR-swizzled by row against LDS bank conflicts), 2 - 10 % over a lane per row; with two
 // k-tiles a stage 128 bytes, eight lanes (us a launch inside a prompt: 1500 rows, K 2048 .. 8192, 2048 columns 45.6 -> 39.8, 2048 rows
-// 31.1 -> 29.1; alone with weights in the caches K 2048 3 - 6 % faster, K 4096 and 8192 up to 4 % slower).
+// 31.1 -> 29.1; means over 245 products of 512 .. 4096 columns, 100 .. 2048 rows, K 512 .. 8192, weights in the caches and not: bf16 32 x 64 0 - 4 %
+// faster, 64 x 64 3 - 9, 64 x 128 3 - 5, 128 x 128 1 - 5; fp32 0 - 3).
 // Measured, us, bf16, dense_tile_kernel and blocks without KG -> this: 2048 x 2048 at 100 rows 10.8 -> 8.6, 333 11.4 ->
 // 9.2, 1000 18.4 -> 15.0; 2048 x 8192 (N x K) at 333 46.5 -> 29, 1500 85.5 -> 64; 5120 x 2048 at 700 29.8 -> 22; fp32
 // 2048 x 2048 at 100 rows 45 -> 24.

@@ -101,7 +101,7 @@ __global__ __launch_bounds__(512, 2) void dense_expert_kernel(const ti_dense_arg
 #pragma unroll
       for (int c = 0; c < FN; ++c) acc[i][c] = (f32x4){0.f, 0.f, 0.f, 0.f};
     V af[R - 1], al[2], wf[2][FN];
-        auto read_a = [&](V& d, int pair, int h, int i) { d = *(const V*)(ring + pair + at_a + (((h * 4 + (lane >> 4)) ^ sw) * 16) + i * 4096); };
+    auto read_a = [&](V& d, int pair, int h, int i) { d = *(const V*)(ring + pair + at_a + (((h * 4 + (lane >> 4)) ^ sw) * 16) + i * 4096); };
     auto read_w = [&](int k, V (&d)[FN], int c) { d[c] = *(const V*)(ring + k + at_w + c * 1024); };
     wait_dma<3 * ND>();
     __builtin_amdgcn_s_barrier();

@@ -300,7 +300,7 @@ __device__ __forceinline__ bf16x8 pair_of(bf16x4 a, bf16x4 b) { return __builtin
 //   y_t = sum_{s <= t} (C_t . B_s) L(t, s) dt_s x_s + exp(cum_t) S^T C_t + D x_t
 //   S  <- exp(cum_last) S + sum_t L(last, t) dt_t B_t x_t^T
 // Waves 0..3 carry the state, 16 * NTW of its rows each, tile i holding every NTW-th from the i-th (a lane's
-// rows are 4 * NTW consecutive ones, its operands of all tiles come in one read): its share of every token's output, then
+// rows are 4 * NTW consecutive ones, its operands of all tiles come in one read; S3: 16 consecutive ones): its share of every token's output, then
 // its update.  Waves 4..7 own 16 tokens each: their scores within the block and the output.  Accumulators
 // are the operand fragments of the next product (scores, state).  Waves 0..3 also load the next block and
 // stage it at the end of this one (DB: into the other buffer); wave 4, which has the fewest scores, prepares
