@@ -170,3 +170,27 @@ def test_prefill_attention_many_rows(ti):
         ti.sync()
     assert few.isfinite().all() and few[0].abs().max() > 0 and (few == few[0]).all()
     assert (out - few[0]).abs().le(2.0**-10 * few[0].abs() + 2.0**-24).all()   # (another split of the keys: a unit in the last place)
+
+
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+@pytest.mark.parametrize("M,nh,nkv,hd,start", [(400, 32, 32, 128, 0), (360, 32, 4, 64, 64), (200, 4, 4, 128, 0)])
+def test_prefill_attention_values_behind_a_row(ti, kernel, M, nh, nkv, hd, start, bad):
+    """Values that are no numbers reach rows at most 31 keys in front of theirs (two blocks of 16 are one product, their weights
+    there are 0): all others are what they are without."""
+    rng = np.random.RandomState(M)
+    top = start + M
+    k, v = rng.standard_normal((2, nkv, top, hd)).astype(f16)
+    q, pos = rng.standard_normal((M, nh * hd)).astype(f32), (start + np.arange(M)).astype(np.int32)
+    qd_, kd, pd, out = dev(ti, q), dev(ti, k), dev(ti, pos), ti.DeviceBuffer(M * nh * hd * 2)
+    for at in (start + 32, start + 101, start + 175):
+        got = []
+        for value in (v[:, at], bad):
+            w = v.copy()
+            w[:, at] = value
+            vd = dev(ti, w)
+            ti.check(ti.lib().ti_attn_prefill_keys(qd_.ptr, kd.ptr, vd.ptr, top, pd.ptr, M, top, nh, nkv, hd, out.ptr, None))
+            ti.sync()
+            got.append(out.download(f16, (M, nh * hd)))
+        clear = at // 32 * 32 - start
+        assert np.isfinite(got[0]).all()
+        np.testing.assert_array_equal(got[0][:clear], got[1][:clear])

@@ -500,6 +500,11 @@ __global__ __launch_bounds__(64 * QB * HALVES, HD == 64 ? 4 : 1) void attn_prefi
 #pragma unroll
           for (int i = 0; i < 4; ++i)
             if (16 * b + i > lim) pv[b][i] = -INFINITY;
+#pragma unroll
+        for (int b = 2; b < NB; ++b)   // (two that none of the wave's rows sees: an infinity times a weight of 0 is NaN)
+          if (kb + (b & ~1) >= nkb_w)
+#pragma unroll
+            for (int t = 0; t < DV; ++t) vf[b][t] = (f16x4){};
       }
 #pragma unroll
       for (int b = 0; b < NB; ++b)
