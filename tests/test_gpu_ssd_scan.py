@@ -20,7 +20,8 @@ class SsdArgs(C.Structure):   # ti_ssd_args (include/ti_stack.h)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M,heads,vdim,n,groups,carry", [
     (1, 2, 16, 128, 1, True), (15, 4, 64, 128, 2, False), (64, 2, 24, 100, 1, True), (65, 2, 64, 68, 2, True), (129, 4, 40, 132, 4, True),
-    (200, 2, 64, 256, 1, True), (333, 8, 64, 128, 1, True), (70, 2, 20, 64, 1, True), (130, 2, 16, 12, 2, False)])
+    (200, 2, 64, 256, 1, True), (333, 8, 64, 128, 1, True), (70, 2, 20, 64, 1, True), (130, 2, 16, 12, 2, False), (512, 2, 16, 64, 1, True),
+    (577, 2, 20, 40, 1, True)])
 def test_ssd_scan(ti, dtype, M, heads, vdim, n, groups, carry):
     g = torch.Generator("cuda").manual_seed(M + n)
 

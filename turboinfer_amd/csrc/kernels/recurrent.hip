@@ -304,7 +304,7 @@ __device__ __forceinline__ bf16x8 pair_of(bf16x4 a, bf16x4 b) { return __builtin
 // its update.  Waves 4..7 own 16 tokens each: their scores within the block and the output.  Accumulators
 // are the operand fragments of the next product (scores, state).  Waves 0..3 also load the next block and
 // stage it at the end of this one (DB: into the other buffer); wave 4, which has the fewest scores, prepares
-// its step sizes and decays.
+// its step sizes and decays.  (!SS: waves 4..7 load and stage; launch_ssd_scan.)
 // S3 (16-bit operands, states of more than 64): the fp32 factors of a token's output -- the carried state, the decayed scores -- are
 // taken apart into three bf16 (Split3), the other factor is bf16 already: three 16x16x32 products instead of eight fp32
 // 16x16x4 ones, which hold the matrix cores 5 times as long.  Tiles then hold 16 consecutive state rows, and the state's update, on fp32 products
@@ -315,7 +315,7 @@ __device__ __forceinline__ bf16x8 pair_of(bf16x4 a, bf16x4 b) { return __builtin
 // dimensions, state 128 (fp32 products, waves 4..7 staging -> products in parts -> waves 0..3 staging): 1500 tokens 77 -> 67 -> 64, 2048
 // 96 -> 80 in all, 333 21.3 -> 18.6; outputs' error against float64 7.69e-8 -> 7.59e-8.  No gain: wave 0 preparing the step sizes, all waves
 // staging.
-template <class T, int NTW, bool DB>
+template <class T, int NTW, bool DB, bool SS = true>
 __global__ __launch_bounds__(512, 1) void ssd_scan_kernel(const ti_ssd_args a) {
   typedef typename El<T>::V V;
   constexpr int KT = El<T>::KT, VEC = El<T>::VEC, PF = NTW * 16 / VEC < 4 ? NTW * 16 / VEC : 4, XLD = kSsdTok + 4, TH = 256;
@@ -331,7 +331,7 @@ __global__ __launch_bounds__(512, 1) void ssd_scan_kernel(const ti_ssd_args a) {
   __shared__ __attribute__((aligned(16))) int marks[2][4];   // S3: a wave's share of the block holds an infinity or NaN (or squares beyond fp32)
   const int h = blockIdx.y, p0 = blockIdx.x * 16, tid = threadIdx.x, lane = tid & 63, col = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), grp = h / (a.heads / a.groups);
-  const bool sw = wave < 4;
+  const bool sw = wave < 4, stages = sw == SS;
   const int w4 = wave & 3;
   const T* src = (const T*)a.a;
   const T* bsrc = src + a.o0 + (size_t)grp * nk;
@@ -421,7 +421,7 @@ __global__ __launch_bounds__(512, 1) void ssd_scan_kernel(const ti_ssd_args a) {
     k[4 * kSsdTok + lane] = __builtin_amdgcn_exp2f(hi);
   };
   auto raw_dt = [&](int m0) { return a.dt[(size_t)min(m0 + lane, a.M - 1) * a.heads + h]; };
-  if (sw) {
+  if (stages) {
     load(reg, 0);
     stage(reg, 0, 0);
   }
@@ -438,7 +438,7 @@ __global__ __launch_bounds__(512, 1) void ssd_scan_kernel(const ti_ssd_args a) {
     if constexpr (S3) mark = *(const int4*)marks[buf];
     auto whole = [&] { return S3 && __builtin_amdgcn_readfirstlane(mark.x | mark.y | mark.z | mark.w) != 0; };
     float rdt = 0.0f;
-    if (more && sw) load(reg, m0 + kSsdTok);
+    if (more && stages) load(reg, m0 + kSsdTok);
     if (more && wave == 4) rdt = raw_dt(m0 + kSsdTok);
     const int tok = w4 * 16 + col;
     f32x4 y = {0.f, 0.f, 0.f, 0.f};
@@ -593,7 +593,7 @@ __global__ __launch_bounds__(512, 1) void ssd_scan_kernel(const ti_ssd_args a) {
       for (int r = 0; r < 4; ++r) y[r] = fmaf(D, xt[(4 * g + r) * XLD + tok], y[r]);
       if (wave == 4 && more) steps(buf ^ 1, m0 + kSsdTok, rdt);
     }
-    if (DB && more && sw) stage(reg, buf ^ 1, m0 + kSsdTok);
+    if (DB && more && stages) stage(reg, buf ^ 1, m0 + kSsdTok);
     lds_sync();
     if (!sw && m0 + tok < a.M) {   // out: this wave's tokens, dimensions 4 g + r
       f32x4 z = red[w4 * 64 + lane];
@@ -612,7 +612,7 @@ __global__ __launch_bounds__(512, 1) void ssd_scan_kernel(const ti_ssd_args a) {
       }
     }
     if (!DB && more) {
-      if (sw) stage(reg, buf ^ 1, m0 + kSsdTok);
+      if (stages) stage(reg, buf ^ 1, m0 + kSsdTok);
       lds_sync();
     }
   }
@@ -890,7 +890,11 @@ int launch_ssd_scan(const ti_ssd_args& a, hipStream_t s) {
 #define TI_SS(NTW)                                                                       \
   if (db) hipLaunchKernelGGL((ssd_scan_kernel<T, NTW, true>), grid, blk, lds, s, a);     \
   else hipLaunchKernelGGL((ssd_scan_kernel<T, NTW, false>), grid, blk, lds, s, a)
-  if (ntw == 1) TI_SS(1);
+  // Long fp32 prompts of states of up to 64: waves 4..7 stage.  us, 64 heads of 64 dimensions, state 64, waves 0..3 / 4..7: 100 tokens 9.1 / 9.7, 400
+  // 24.0 / 24.6, 577 33.4 / 32.9, 1000 52.1 / 49.9, 2000 99.8 / 95.0; 24 heads, 1000 48.9 / 49.3, 2000 98.9 / 94.4; state 16, 400 22.6 / 22.5, 1000
+  // 46.2 / 43.1.  Larger states 178.6 / 189.9 at 2000, bf16 70.5 / 74.3.
+  if (sizeof(T) == 4 && ntw == 1 && a.M > 512) hipLaunchKernelGGL((ssd_scan_kernel<float, 1, true, false>), grid, blk, lds, s, a);
+  else if (ntw == 1) TI_SS(1);
   else if (ntw == 2) TI_SS(2);
   else TI_SS(4);
 #undef TI_SS
@@ -903,7 +907,7 @@ int recurrent_prepare() {
   const void* k[] = {(const void*)ssd_scan_kernel<T, 1, true>,  (const void*)ssd_scan_kernel<T, 2, true>,
                      (const void*)ssd_scan_kernel<T, 4, true>,  (const void*)ssd_scan_kernel<T, 1, false>,
                      (const void*)ssd_scan_kernel<T, 2, false>, (const void*)ssd_scan_kernel<T, 4, false>,
-                     (const void*)ssd_norm_kernel<T>};
+                     (const void*)ssd_scan_kernel<float, 1, true, false>, (const void*)ssd_norm_kernel<T>};
   const void* step[] = {(const void*)lru_step_kernel<T, 1>, (const void*)lru_step_kernel<T, El<T>::VEC>};
   for (const void* f : k)
     TI_HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSsdLds), "recurrent kernels' LDS");
