@@ -353,8 +353,9 @@ __global__ __launch_bounds__(64, WPE) void attn_prefill_kernel(const float* __re
 // keys all in flight, its blocks' products in turn; four blocks a step (two where there are 4 parts: 64 rows 6.3 against
 // 6.1 us); values transposed by their LDS reads instead of a v_perm per fragment word; a kv-head's workgroups on one XCD,
 // whose L2 its keys reach once (512 rows of 32 heads, head_dim 128: the copies alone 13.0 -> 7.4 us).  Together, us: head_dim
-// 64, 32 heads on 4, 1000 rows 20.8 -> 16.7, 333 behind 600 keys 14.0 -> 11.9, 256 5.4 -> 5.4; head_dim 128, 32 on 32, 512 rows 15.0 -> 12.2,
-// 1024 38.2 -> 34.3, 256 8.8 -> 7.9; 32 on 8, 400 behind 500 19.9 -> 18.3.
+// 64, 32 heads on 4, 1000 rows 20.8 -> 16.7, 333 behind 600 keys 14.0 -> 12.1, 256 5.4 -> 5.5; head_dim 128, 32 on 32, 512 rows 15.0 -> 12.3,
+// 1024 38.2 -> 34.5, 256 8.8 -> 7.9; 32 on 8, 400 behind 500 19.9 -> 18.3.  Output errors against float64 are those of the exact result rounded
+// to fp16 (2.0e-4; six seeds, four shapes), with four blocks a step as with two.
 template <int HD, int QB, int HALVES, int R, int NB>
 __global__ __launch_bounds__(64 * QB * HALVES, HD == 64 ? 4 : 1) void attn_prefill_wg_kernel(const float* __restrict__ q, const uint16_t* __restrict__ kc,
                                                                  const uint16_t* __restrict__ vc, int max_seq,
